@@ -170,34 +170,34 @@ def main():
         med = xs[n // 2] if n % 2 else 0.5 * (xs[n // 2 - 1] + xs[n // 2])
         return {"median": med, "min": xs[0], "max": xs[-1], "mean": sum(xs) / n}
 
-    # ---- the timed region: exactly `steps` calls of the operator; every call records an event on the stream the
-    #      kernels run on at each stage boundary (K mean | pooling, quantisation, selection | V quantisation | attention)
-    core._stage_hook = hook
+    # ---- the timed region: exactly `steps` calls of the operator ------------------------------------------------
+    edges = [torch.cuda.Event(enable_timing=True) for _ in range(args.steps + 1)]
     torch.cuda.synchronize()
     t0 = time.perf_counter()
-    for _ in range(args.steps):
+    edges[0].record()
+    for i in range(args.steps):
         step()
+        edges[i + 1].record()
     torch.cuda.synchronize()
     t1 = time.perf_counter()
     step_s = (t1 - t0) / args.steps
-    timed_marks = len(marks)
-    # stage medians want at least 20 samples: further calls outside the timed region when `steps` is smaller
-    for _ in range(max(0, 20 - args.steps)):
+    step_stats = stats([e0.elapsed_time(e1) for e0, e1 in zip(edges[:-1], edges[1:])])
+
+    # ---- stage times: further calls, outside the timed region, that run stage by stage with an event at each boundary
+    #      (K mean | pooling, quantisation, selection | V quantisation | attention)
+    core._stage_hook = hook
+    stage_calls = max(20, args.steps)
+    for _ in range(stage_calls):
         step()
     torch.cuda.synchronize()
     core._stage_hook = None
     per_stage = {n: [] for n in names[:-1]}
-    per_step_total = []
     for i in range(0, len(marks), len(names)):
         grp = marks[i:i + len(names)]
         for (n0, e0), (_, e1) in zip(grp[:-1], grp[1:]):
             per_stage[n0].append(e0.elapsed_time(e1))
-        per_step_total.append(grp[0][1].elapsed_time(grp[-1][1]))
-    n_timed = timed_marks // len(names)
-    assert n_timed == args.steps
-    step_stats = stats(per_step_total[:n_timed])
-    attn_stats = stats(per_stage["attn"][:n_timed])
-    attn_s = attn_stats["mean"] * 1e-3          # average launch duration over the timed region (roofline denominator)
+    attn_stats = stats(per_stage["attn"])
+    attn_s = attn_stats["mean"] * 1e-3          # average launch duration (roofline denominator)
     stage_ms = {n0: stats(v)["median"] for n0, v in per_stage.items()}
     mp_serial = stats([a + b for a, b in zip(per_stage["km"], per_stage["maskpred"])])
     serial_runs = len(per_stage["km"])

@@ -168,6 +168,36 @@ int spg_block_sparse_attn_f16v(const int8_t *q8, const int8_t *k8, const void *v
                                int B, int H, int Hkv, int N, int N_kv, int D, float sm_scale, int is_causal,
                                int qk_quant_gran, int pv_threshold_mode, int32_t *pv_count, void *stream);
 
+/* ---- the whole operator in one call (spas_sage2_attn_meansim[_topk]_cuda, block_sparse_sage2_attn_cuda and, with pv_f16,
+ * spas_sage_attn_meansim[_topk]_cuda; spas_sage_attn/core.py:39-319) ---------------------------------------------------
+ * Runs the stages above with the same results, but stages that do not depend on each other share a launch, scalar
+ * hyper-parameters need no device memory, and all intermediate tensors live in one workspace of
+ * spg_sparse_attn_workspace_bytes() bytes, 256-byte aligned, that may be used again by the next call on the stream. */
+enum spg_selection { SPG_SELECT_TOPK = 0, SPG_SELECT_CDF = 1, SPG_SELECT_MASK = 2 };
+
+typedef struct spg_attn_args {
+  int B, H, Hkv, N, N_kv, D;
+  int qk_dtype, v_dtype;              /* enum spg_dtype; the output has qk_dtype */
+  int selection;                      /* enum spg_selection */
+  int pv_f16;                         /* 0: FP8 PV (spg_block_sparse_attn), 1: FP16 PV (spg_block_sparse_attn_f16v) */
+  int is_causal, attention_sink;      /* block selection */
+  int kernel_causal;                  /* token-level causal mask inside the attention kernel */
+  int qk_quant_gran, mask_kind;
+  /* hyper-parameters: (H,) float32 device pointers, or NULL and one value for all heads.  level = top-k fraction or CDF
+   * threshold.  With Hkv < H the K blocks of a head follow simthreshd1 of the first query head of its group. */
+  float level_value, simthreshd1_value, pvthreshd_value, sm_scale;
+  const float *level, *simthreshd1, *pvthreshd;
+  const void *q, *k, *v, *mask;       /* q (B,H,N,D), k and v (B,Hkv,N_kv,D); mask (B,H,nq,nk) for SPG_SELECT_MASK */
+  void *out;
+  const int64_t *q_strides, *k_strides, *v_strides, *out_strides;
+  int32_t *valid_block_num;           /* (B,H,nq), or NULL if the caller has no use for the counts */
+  void *workspace;
+  uint64_t workspace_bytes;
+} spg_attn_args;
+
+size_t spg_sparse_attn_workspace_bytes(const spg_attn_args *args);
+int spg_sparse_attn(const spg_attn_args *args, void *stream);
+
 /* ---- measurement comparator: dense FP16 flash attention on MFMA (no counterpart in the reference;
  * the "dense FP16 attention kernel built in the same run" the speed-up is quoted against).
  * q,k,out (B,H,N,D) fp16; vt = the fp16 V^T tiles spg_v_tiles_f16 writes, (B,H,ceil(N/64),D,64), chunk-swizzled,

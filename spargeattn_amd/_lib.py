@@ -41,10 +41,24 @@ SIGNATURES = {
     "spg_block_sparse_attn": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _vp, _vp]),
     "spg_v_tiles_f16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "spg_block_sparse_attn_f16v": (_i, [_vp] * 5 + [_i] + [_vp] * 5 + [_i] * 6 + [_f, _i, _i, _i, _vp, _vp]),
+    "spg_sparse_attn_workspace_bytes": (_sz, [_vp]),
+    "spg_sparse_attn": (_i, [_vp, _vp]),
     "spg_dense_attn_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _f, _i, _vp]),
     "spg_selftest_division": (_i, [_vp, _i, ctypes.c_uint, _vp]),
     "spg_selftest_fp8_pack": (_i, [_vp, _vp, _i, _i, _vp]),
 }
+
+class AttnArgs(_c.Structure):
+    """spg_attn_args of include/spargeattn_amd.h."""
+    _fields_ = ([(n, _i) for n in ("B", "H", "Hkv", "N", "N_kv", "D", "qk_dtype", "v_dtype", "selection", "pv_f16",
+                                   "is_causal", "attention_sink", "kernel_causal", "qk_quant_gran", "mask_kind")]
+                + [(n, _f) for n in ("level_value", "simthreshd1_value", "pvthreshd_value", "sm_scale")]
+                + [(n, _vp) for n in ("level", "simthreshd1", "pvthreshd", "q", "k", "v", "mask", "out", "q_strides",
+                                      "k_strides", "v_strides", "out_strides", "valid_block_num", "workspace")]
+                + [("workspace_bytes", _c.c_uint64)])
+
+
+SELECT_TOPK, SELECT_CDF, SELECT_MASK = 0, 1, 2
 
 _lib = None
 _ops = None          # torch.ops.spargeattn_amd once the extension is loaded
@@ -342,6 +356,83 @@ def block_sparse_attn(q8, k8, v8, out, lut, valid, pvthreshd, q_scale, k_scale, 
                                         _p(q_scale), _p(k_scale), _p(v_scale), B, H, Hkv, N, Nk, D, float(sm_scale),
                                         int(bool(is_causal)), qk_quant_gran, int(pv_mode), _p(pvc), _stream()))
     return pvc
+
+
+class ForwardPlan:
+    """Everything about a call of the whole operator (spg_sparse_attn) that follows from shapes, strides, dtypes and
+    options: the argument block with those fields filled in, and the workspace it needs.  Holds no data of any call."""
+
+    def __init__(self, q, k, v, out, mask, selection, pv_f16, is_causal, attention_sink, kernel_causal,
+                 qk_quant_gran, sm_scale):
+        """q, k, v: (B,H,N,D) views the kernels can read in place; out: shape and strides of the output."""
+        _dev_strided(q, k, v)
+        if not (q.device == k.device == v.device):
+            raise RuntimeError("q, k and v must be on one GPU")
+        B, H, N, D = q.shape
+        a = self.template = AttnArgs()
+        a.B, a.H, a.Hkv, a.N, a.N_kv, a.D = B, H, k.shape[1], N, k.shape[2], D
+        a.qk_dtype, a.v_dtype = _dt(q), _dt(v)
+        a.selection, a.pv_f16, a.is_causal, a.attention_sink = selection, int(pv_f16), int(bool(is_causal)), int(bool(attention_sink))
+        a.kernel_causal, a.qk_quant_gran, a.sm_scale = int(bool(kernel_causal)), qk_quant_gran, sm_scale
+        nq, nk = (N + 127) // 128, (k.shape[2] + 63) // 64
+        self.valid_shape = (B, H, nq)
+        self.nk = nk
+        if mask is not None:
+            assert mask.dim() == 4
+            assert mask.is_contiguous()
+            _dev(mask)
+            if mask.dtype not in _MASK_KIND:
+                raise RuntimeError(f"unsupported mask dtype {mask.dtype}")
+            if tuple(mask.shape) != (B, H, nq, nk):
+                raise RuntimeError(f"mask_id has shape {tuple(mask.shape)}, expected {(B, H, nq, nk)}")
+            a.mask_kind = _MASK_KIND[mask.dtype]
+        # a contiguous tensor may carry any stride in a dimension of size 1: the canonical ones are passed
+        self._strides = [(ctypes.c_int64 * 3)(*((t.shape[1] * t.shape[2] * D, t.shape[2] * D, D) if t.is_contiguous()
+                                                else t.stride()[:3])) for t in (q, k, v, out)]
+        a.q_strides, a.k_strides, a.v_strides, a.out_strides = (ctypes.addressof(s) for s in self._strides)
+        self._lib = load()
+        self.workspace_bytes = a.workspace_bytes = self._lib.spg_sparse_attn_workspace_bytes(ctypes.addressof(a))
+        if self.workspace_bytes == 0:
+            _check(SPG_ERR_INVALID)
+        self.device = q.device
+        self.device_index = q.device.index
+
+    def run(self, q, k, v, out, mask, level, simthreshd1, pvthreshd, return_valid=False):
+        """level / simthreshd1 / pvthreshd: a Python number, or a contiguous (H,) float32 tensor on the device."""
+        if _torch() is not None:
+            t = self.template
+            par = [(x, 0.0) if isinstance(x, torch.Tensor) else (None, float(x)) for x in (level, simthreshd1, pvthreshd)]
+            s = self._strides
+            valid = _ops.sparse_attn(q, k, v, out, mask, *par[0], *par[1], *par[2], [t.B, t.H, t.Hkv, t.N, t.N_kv, t.D],
+                                     list(s[0]), list(s[1]), list(s[2]), list(s[3]), t.selection, bool(t.pv_f16),
+                                     bool(t.is_causal), bool(t.attention_sink), bool(t.kernel_causal), t.qk_quant_gran, t.sm_scale)
+            return valid if return_valid else None
+        a = AttnArgs.from_buffer_copy(self.template)
+        workspace = torch.empty(self.workspace_bytes, dtype=torch.uint8, device=self.device)
+        a.q, a.k, a.v, a.out, a.workspace = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), workspace.data_ptr()
+        valid = None
+        if return_valid:
+            valid = torch.empty(self.valid_shape, dtype=torch.int32, device=self.device)
+            a.valid_block_num = valid.data_ptr()
+        if mask is not None:
+            a.mask = mask.data_ptr()
+        else:
+            if isinstance(level, torch.Tensor):
+                a.level = level.data_ptr()
+            else:
+                a.level_value = level
+            if isinstance(simthreshd1, torch.Tensor):
+                a.simthreshd1 = simthreshd1.data_ptr()
+            else:
+                a.simthreshd1_value = simthreshd1
+        if isinstance(pvthreshd, torch.Tensor):
+            a.pvthreshd = pvthreshd.data_ptr()
+        else:
+            a.pvthreshd_value = pvthreshd
+        rc = self._lib.spg_sparse_attn(ctypes.addressof(a), torch._C._cuda_getCurrentRawStream(self.device_index))
+        if rc != SPG_OK:
+            _check(rc)
+        return valid
 
 
 def v_tiles_f16_swizzled(v, stream=None):

@@ -23,6 +23,7 @@ COMMON = [
 SOURCES = {
     "maskpred.hip": ["-ffp-contract=off"],
     "vquant.hip": ["-ffp-contract=off"],
+    "forward.hip": ["-ffp-contract=off"],
     "attn.hip": [],
     "dense.hip": [],
     "capi.hip": ["-fvisibility=default"],

@@ -19,12 +19,13 @@ granularity through the LUT (the reference passes ``is_causal=False`` to its ker
 import torch
 
 from . import _lib
-from .utils import (hyperparameter_check, get_block_map_meansim_fuse_quant, get_vanilla_qk_quant,
+from .utils import (check_grouped_simthreshd1, hyperparameter_check, get_block_map_meansim_fuse_quant, get_vanilla_qk_quant,
                     block_map_lut_triton)
 
 
-# Optional callable(name) invoked at stage boundaries ("km", "maskpred", "vquant", "attn", "end");
-# bench.py installs one that records HIP events on the current stream.  None in normal use.
+# Optional callable(name) invoked at stage boundaries ("km", "maskpred", "vquant", "attn", "end").  While one is
+# installed the operators run stage by stage through the separate entry points (same results); None in normal use, where
+# the whole operator is one native call that has no such boundaries.
 _stage_hook = None
 
 
@@ -73,14 +74,13 @@ def _rows_ok(t):
     return t if ok else t.contiguous()
 
 
-def _empty_out(q):
+def _empty_out(q, meta=False):
     """Output buffer with q's shape whose MEMORY layout follows q's (an NHD view gets an NHD buffer, so that the
-    transpose back at the end is a view of contiguous memory)."""
-    if q.is_contiguous():
-        return torch.empty_like(q)
-    if q.transpose(-2, -3).is_contiguous():
-        return torch.empty_like(q.transpose(-2, -3)).transpose(-2, -3)
-    return torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    transpose back at the end is a view of contiguous memory).  meta: shape and strides only."""
+    device = "meta" if meta else q.device
+    if not q.is_contiguous() and q.transpose(-2, -3).is_contiguous():
+        return torch.empty(q.transpose(-2, -3).shape, dtype=q.dtype, device=device).transpose(-2, -3)
+    return torch.empty(q.shape, dtype=q.dtype, device=device)
 
 
 def _attention(q, k, v, q_int8, q_scale, k_int8, k_scale, lut, valid_block_num, scale, pvthreshd, kernel_causal,
@@ -112,13 +112,9 @@ def _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_deno
     return o
 
 
-def _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
-             tensor_layout, return_sparsity, kernel_causal, qk_quant_gran=1):
-    qk_quant_gran = _lib.quant_gran(qk_quant_gran)
+def _staged_meansim(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
+                    tensor_layout, return_sparsity, kernel_causal, qk_quant_gran=1):
     q, k, v = _prologue(q, k, v, tensor_layout)
-    if not smooth_k:
-        # the reference leaves `km` undefined in this case (core.py:119-126)
-        raise NameError("name 'km' is not defined")
     _mark("km")
     km = _lib.km_mean(k)
     _mark("maskpred")
@@ -130,14 +126,11 @@ def _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, topk,
     return _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_denominator=is_causal is not False)
 
 
-def _meansim_sage1(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
-                   tensor_layout, return_sparsity, qk_quant_gran=1):
+def _staged_meansim_sage1(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
+                          tensor_layout, return_sparsity, qk_quant_gran=1):
     """INT8 QK^T / FP16 PV path (spas_sage_attn/core.py:235-319): fp16 V, token-level causal masking in the kernel,
     sparsity reported against the full grid unless is_causal."""
-    qk_quant_gran = _lib.quant_gran(qk_quant_gran)
     q, k, v = _prologue(q, k, v, tensor_layout)
-    if not smooth_k:
-        raise NameError("name 'km' is not defined")           # as the reference (core.py:249-252)
     _mark("km")
     km = _lib.km_mean(k)
     _mark("maskpred")
@@ -159,50 +152,8 @@ def _meansim_sage1(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd,
     return _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_denominator=is_causal is not False)
 
 
-@torch.compiler.disable
-def spas_sage_attn_meansim_cuda(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None, smooth_k=True,
-                                simthreshd1=0.6, cdfthreshd=0.98, pvthreshd=50, attention_sink=False,
-                                tensor_layout="HND", output_dtype=torch.float16, return_sparsity=False, *,
-                                qk_quant_gran=1):
-    return _meansim_sage1(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, None, pvthreshd,
-                          attention_sink, tensor_layout, return_sparsity, qk_quant_gran)
-
-
-@torch.compiler.disable
-def spas_sage_attn_meansim_topk_cuda(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None,
-                                     smooth_k=True, simthreshd1=-0.1, cdfthreshd=None, topk=0.5, pvthreshd=50,
-                                     attention_sink=False, tensor_layout="HND", output_dtype=torch.float16,
-                                     return_sparsity=False, *, qk_quant_gran=1):
-    return _meansim_sage1(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, topk, pvthreshd,
-                          attention_sink, tensor_layout, return_sparsity, qk_quant_gran)
-
-
-@torch.compiler.disable
-def spas_sage2_attn_meansim_cuda(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None, smooth_k=True,
-                                 simthreshd1=0.6, cdfthreshd=0.98, pvthreshd=50, attention_sink=False,
-                                 tensor_layout="HND", output_dtype=torch.float16, return_sparsity=False,
-                                 kernel_causal=False, *, qk_quant_gran=1):
-    return _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, None, pvthreshd, attention_sink,
-                    tensor_layout, return_sparsity, kernel_causal, qk_quant_gran)
-
-
-@torch.compiler.disable
-def spas_sage2_attn_meansim_topk_cuda(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None,
-                                      smooth_k=True, simthreshd1=-0.1, cdfthreshd=None, topk=0.5, pvthreshd=50,
-                                      attention_sink=False, tensor_layout="HND", output_dtype=torch.float16,
-                                      return_sparsity=False, kernel_causal=False, *, qk_quant_gran=1):
-    return _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
-                    tensor_layout, return_sparsity, kernel_causal, qk_quant_gran)
-
-
-@torch.compiler.disable
-def block_sparse_sage2_attn_cuda(q, k, v, mask_id=None, dropout_p=0.0, scale=None, smooth_k=True, pvthreshd=50,
-                                 attention_sink=False, tensor_layout="HND", output_dtype=torch.float16,
-                                 return_sparsity=False, kernel_causal=False, *, qk_quant_gran=1):
-    qk_quant_gran = _lib.quant_gran(qk_quant_gran)
+def _staged_mask(q, k, v, mask_id, scale, pvthreshd, tensor_layout, return_sparsity, kernel_causal, qk_quant_gran):
     q, k, v = _prologue(q, k, v, tensor_layout)
-    if not smooth_k:
-        raise NameError("name 'km' is not defined")
     _mark("km")
     km = _lib.km_mean(k)
     _mark("maskpred")
@@ -212,3 +163,142 @@ def block_sparse_sage2_attn_cuda(q, k, v, mask_id=None, dropout_p=0.0, scale=Non
                       qk_quant_gran=qk_quant_gran)
     # the reference always reports against the causal denominator here (core.py:230)
     return _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_denominator=True)
+
+
+# ---- the whole operator in one native call (spg_sparse_attn) --------------------------------------------------------
+# What follows from shapes, strides, dtypes and options is worked out once per combination and kept (_lib.ForwardPlan
+# holds sizes, never data); a call then costs two allocations and one foreign call.  Plans are immutable and the dict
+# operations atomic, so threads may share them; the cache is emptied when a program has shown it very many shapes.
+_plans = {}
+_MAX_PLANS = 512
+
+
+def _hyper(value, H, device):
+    """A hyper-parameter as the native call takes it: one Python float for all heads, or an (H,) float32 tensor."""
+    if type(value) is float or type(value) is int:
+        return float(value)
+    if isinstance(value, torch.Tensor) and value.dim() == 0:
+        return float(value.item())
+    return hyperparameter_check(value, H, device)
+
+
+def _run(q, k, v, mask, selection, level, simthreshd1, pvthreshd, is_causal, attention_sink, kernel_causal, pv_f16,
+         scale, tensor_layout, return_sparsity, qk_quant_gran, causal_denominator):
+    key = (q.shape, k.shape, v.shape, q.stride(), k.stride(), v.stride(), q.dtype, k.dtype, v.dtype, q.device, k.device,
+           v.device, None if mask is None else (mask.shape, mask.dtype, mask.device, mask.is_contiguous()), selection,
+           bool(is_causal), bool(attention_sink), bool(kernel_causal), pv_f16, scale, tensor_layout, qk_quant_gran)
+    plan = _plans.get(key)
+    if plan is None or q.data_ptr() % 16 or k.data_ptr() % 16 or v.data_ptr() % 16:
+        given = (q, k, v)
+        q, k, v = _prologue(q, k, v, tensor_layout)
+        headdim = q.size(-1)
+        nhd = tensor_layout == 'NHD'
+        copied = any(a.data_ptr() != b.data_ptr() for a, b in zip(given, (q, k, v)))
+        if copied:
+            # some tensor had to be converted or copied: go on with what the prologue returned
+            out = _run(q, k, v, mask, selection, level, simthreshd1, pvthreshd, is_causal, attention_sink, kernel_causal,
+                       pv_f16, scale, 'HND', return_sparsity, qk_quant_gran, causal_denominator)
+            if nhd:
+                return (out[0].transpose(-2, -3),) + out[1:] if return_sparsity else out.transpose(-2, -3)
+            return out
+        assert headdim in [64, 128], "headdim should be in [64, 128]. For other headdim, you can use padding and specify the softmax scale."
+        like = _empty_out(q, meta=True)
+        plan = _lib.ForwardPlan(q, k, v, like, mask, selection, pv_f16, is_causal,
+                                attention_sink, kernel_causal, qk_quant_gran,
+                                1.0 / (headdim ** 0.5) if scale is None else scale)
+        q, k, v = given
+        plan.out = like.transpose(-2, -3) if nhd else like
+        if len(_plans) >= _MAX_PLANS:
+            _plans.clear()
+        _plans[key] = plan
+    device = plan.device
+    if torch.cuda.current_device() != plan.device_index:
+        torch.cuda.set_device(device)
+    H = plan.valid_shape[1]
+    if mask is None:
+        level = _hyper(level, H, device)
+        Hkv = plan.template.Hkv
+        if Hkv != H and isinstance(simthreshd1, torch.Tensor) and simthreshd1.dim() == 1:
+            check_grouped_simthreshd1(hyperparameter_check(simthreshd1, H, device), H, Hkv)
+        simthreshd1 = _hyper(simthreshd1, H, device)
+    pvthreshd = _hyper(pvthreshd, H, device)
+    o = torch.empty_strided(plan.out.shape, plan.out.stride(), dtype=q.dtype, device=device)
+    valid = plan.run(q, k, v, o, mask, level, simthreshd1, pvthreshd, return_sparsity)
+    if not return_sparsity:
+        return o
+    B, H, nq = plan.valid_shape
+    cols = (plan.nk + 2) // 2 if causal_denominator else plan.nk
+    qk_sparsity = 1 - valid.cpu().sum().float() / (cols * nq * B * H)
+    return o, qk_sparsity.item()
+
+
+def _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
+             tensor_layout, return_sparsity, kernel_causal, qk_quant_gran, pv_f16):
+    qk_quant_gran = _lib.quant_gran(qk_quant_gran)
+    if not smooth_k:
+        _prologue(q, k, v, tensor_layout)
+        # the reference leaves `km` undefined in this case (core.py:119-126, 249-252)
+        raise NameError("name 'km' is not defined")
+    if _stage_hook is not None:
+        if pv_f16:
+            return _staged_meansim_sage1(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, topk, pvthreshd,
+                                         attention_sink, tensor_layout, return_sparsity, qk_quant_gran)
+        return _staged_meansim(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
+                               tensor_layout, return_sparsity, kernel_causal, qk_quant_gran)
+    if (cdfthreshd is None) == (topk is None):
+        _prologue(q, k, v, tensor_layout)
+        raise AssertionError("Only one of cdfthreshd and topk can be set.")
+    selection, level = (_lib.SELECT_TOPK, topk) if topk is not None else (_lib.SELECT_CDF, cdfthreshd)
+    return _run(q, k, v, None, selection, level, simthreshd1, pvthreshd, is_causal, attention_sink, kernel_causal, pv_f16,
+                scale, tensor_layout, return_sparsity, qk_quant_gran, is_causal is not False)
+
+
+@torch.compiler.disable
+def spas_sage_attn_meansim_cuda(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None, smooth_k=True,
+                                simthreshd1=0.6, cdfthreshd=0.98, pvthreshd=50, attention_sink=False,
+                                tensor_layout="HND", output_dtype=torch.float16, return_sparsity=False, *,
+                                qk_quant_gran=1):
+    return _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, None, pvthreshd, attention_sink,
+                    tensor_layout, return_sparsity, is_causal, qk_quant_gran, True)
+
+
+@torch.compiler.disable
+def spas_sage_attn_meansim_topk_cuda(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None,
+                                     smooth_k=True, simthreshd1=-0.1, cdfthreshd=None, topk=0.5, pvthreshd=50,
+                                     attention_sink=False, tensor_layout="HND", output_dtype=torch.float16,
+                                     return_sparsity=False, *, qk_quant_gran=1):
+    return _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
+                    tensor_layout, return_sparsity, is_causal, qk_quant_gran, True)
+
+
+@torch.compiler.disable
+def spas_sage2_attn_meansim_cuda(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None, smooth_k=True,
+                                 simthreshd1=0.6, cdfthreshd=0.98, pvthreshd=50, attention_sink=False,
+                                 tensor_layout="HND", output_dtype=torch.float16, return_sparsity=False,
+                                 kernel_causal=False, *, qk_quant_gran=1):
+    return _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, None, pvthreshd, attention_sink,
+                    tensor_layout, return_sparsity, kernel_causal, qk_quant_gran, False)
+
+
+@torch.compiler.disable
+def spas_sage2_attn_meansim_topk_cuda(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None,
+                                      smooth_k=True, simthreshd1=-0.1, cdfthreshd=None, topk=0.5, pvthreshd=50,
+                                      attention_sink=False, tensor_layout="HND", output_dtype=torch.float16,
+                                      return_sparsity=False, kernel_causal=False, *, qk_quant_gran=1):
+    return _meansim(q, k, v, is_causal, scale, smooth_k, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
+                    tensor_layout, return_sparsity, kernel_causal, qk_quant_gran, False)
+
+
+@torch.compiler.disable
+def block_sparse_sage2_attn_cuda(q, k, v, mask_id=None, dropout_p=0.0, scale=None, smooth_k=True, pvthreshd=50,
+                                 attention_sink=False, tensor_layout="HND", output_dtype=torch.float16,
+                                 return_sparsity=False, kernel_causal=False, *, qk_quant_gran=1):
+    qk_quant_gran = _lib.quant_gran(qk_quant_gran)
+    if not smooth_k:
+        _prologue(q, k, v, tensor_layout)
+        raise NameError("name 'km' is not defined")
+    if _stage_hook is not None:
+        return _staged_mask(q, k, v, mask_id, scale, pvthreshd, tensor_layout, return_sparsity, kernel_causal, qk_quant_gran)
+    # the reference always reports against the causal denominator here (core.py:230)
+    return _run(q, k, v, mask_id, _lib.SELECT_MASK, 0.0, 0.0, pvthreshd, False, False, kernel_causal, False, scale,
+                tensor_layout, return_sparsity, qk_quant_gran, True)

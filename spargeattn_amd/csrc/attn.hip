@@ -55,7 +55,8 @@ struct AttnParams {
   void *out;
   Strides os;      // element strides of out (B, H, N, D), last dimension contiguous
   const int32_t *lut, *valid;
-  const float *pvthr, *q_scale, *k_scale, *v_scale;
+  Hyper pvthr;
+  const float *q_scale, *k_scale, *v_scale;
   int32_t *pv_count;
   int B, H, Hkv, N, Nk, nq, nk;   // N query rows, Nk key/value rows per head (qo_len / kv_len of sm89.cu:256-300)
   float sm_scale_log2;
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   const size_t qsi = (size_t)bh * p.nq + qb;
   const float qs = ((c_f32_t)p.q_scale)[p.q_per_warp ? qsi * 4 + wave : qsi];
   const float c = p.sm_scale_log2;
-  const float thr = ((c_f32_t)p.pvthr)[head];
+  const float thr = p.pvthr.p != nullptr ? ((c_f32_t)p.pvthr.p)[head] : p.pvthr.v;
 
   // ---- tile loader: wave w copies LDS bytes [1024*(WL*w+u), +1024) of each tile, lane l the 16-byte chunk l ----
   // K: LDS chunk position pos <-> (row = pos / CPR, slot = pos % CPR) holds global chunk slot ^ k_swz(row).
@@ -657,11 +658,11 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   }
 }
 
-hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
-                                    int out_dtype, const int32_t *lut, const int32_t *valid, const float *pvthreshd,
-                                    const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
-                                    int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
-                                    int pv_mode, int32_t *pv_count, hipStream_t st) {
+hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
+                                      int out_dtype, const int32_t *lut, const int32_t *valid, Hyper pvthreshd,
+                                      const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
+                                      int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
+                                      int pv_mode, int32_t *pv_count, hipStream_t st) {
   AttnParams p;
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.out = out; p.os = os; p.lut = lut; p.valid = valid; p.pvthr = pvthreshd;
   p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.pv_count = pv_count;
@@ -691,6 +692,15 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
     }
   }
   return hipGetLastError();
+}
+
+hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
+                                    int out_dtype, const int32_t *lut, const int32_t *valid, const float *pvthreshd,
+                                    const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
+                                    int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
+                                    int pv_mode, int32_t *pv_count, hipStream_t st) {
+  return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, Hyper{pvthreshd, 0.f}, q_scale, k_scale, v_scale, B,
+                                    H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, st);
 }
 
 }  // namespace spg

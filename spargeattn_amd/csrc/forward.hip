@@ -1,0 +1,356 @@
+// The whole operator behind one call: K mean, mask prediction + INT8 quantisation, V quantisation, block-sparse
+// attention, as four launches (three for a mask of the caller's own) on workspace the caller hands over.
+//
+// Short sequences are bound by the length of the launch chain and by kernels that cannot fill the chip, so stages that do
+// not depend on each other share a launch; which stage a workgroup belongs to follows from its number:
+//   front    partial column sums of K | partial channel maxima of V (FP16 PV: the V^T tiles, finished) | LUT rows of a
+//            user mask | pooling + quantisation of Q
+//   (final   column mean of K, channel maxima of V: only where there are too many partial results for every workgroup
+//            of the next launch to add them up for itself)
+//   back     pooling + quantisation of K | V -> e4m3 tiles and scales
+//   select   block_select_* of maskpred.hip
+//   attn     block_sparse_attn_kernel
+// Every body is the one the stage-by-stage entry points launch (stage_bodies.h): results are the same bits.
+// Compile with -ffp-contract=off.
+#include "capi_checks.h"
+#include "stage_bodies.h"
+
+namespace spg {
+
+constexpr int MASK_NKP_FRONT = 4096;    // longest mask row (padded to a power of two) whose index list fits the front LDS
+
+struct FrontParams {
+  const uint16_t *q, *k, *v;
+  Strides qs, ks, vs;
+  int H, Hkv, N, Nk, nq, nk;
+  int v_dtype, v_f16;
+  // first workgroup of each role; the roles follow one another in this order
+  int wg_v, wg_mask, wg_q;
+  int k_chunks, k_rows, v_chunks, v_rows;
+  double *km_part;
+  float *v_part;                        // [B Hkv][v_chunks][D]
+  uint16_t *v_tiles;
+  const void *mask;
+  int mask_kind, nkp;
+  int32_t *lut, *valid;
+  Hyper simthr;
+  uint16_t *pool_q;
+  uint8_t *sim_q;
+  int8_t *q8;
+  float *q_scale;
+};
+
+template <int A, int B> constexpr int max_c() { return A > B ? A : B; }
+template <int D, bool POOL> constexpr int front_lds() {
+  return max_c<max_c<km_partial_lds<D>(), v_tiles_f16_lds<D>()>(), max_c<POOL ? psq_lds<128, D>() : 16, POOL ? 16 : 4 * MASK_NKP_FRONT + 16>()>();
+}
+
+template <int D, int DT, bool POOL, int QR>
+__global__ __launch_bounds__(256) void front_kernel(const FrontParams p) {
+  __shared__ __align__(16) unsigned char smem[front_lds<D, POOL>()];
+  const int w = blockIdx.x;
+  if (w >= p.wg_q) {
+    const int id = w - p.wg_q, bh = id / p.nq;
+    float thr = 0.f;
+    if constexpr (POOL) thr = p.simthr.at(bh % p.H);
+    psq_body<128, D, DT, MEAN_NONE, POOL, QR>(p.q, p.qs, nullptr, nullptr, 0, p.pool_q, p.sim_q, p.q8, p.q_scale, thr, p.H, p.N, p.nq,
+                                              id - bh * p.nq, bh, smem);
+  } else if (w < p.wg_v) {
+    const int bh = w / p.k_chunks;
+    km_partial_body<D, DT>(p.k, p.ks, p.Hkv, p.km_part, p.Nk, p.k_rows, w - bh * p.k_chunks, p.k_chunks, bh, smem);
+  } else if (w < p.wg_mask) {
+    const int id = w - p.wg_v;
+    if (p.v_f16) {
+      const int bh = id / p.nk;
+      if (p.v_dtype == 0) v_tiles_f16_body<D, 0>(p.v, p.vs, p.Hkv, p.v_tiles, p.Nk, p.nk, id - bh * p.nk, bh, smem);
+      else v_tiles_f16_body<D, 1>(p.v, p.vs, p.Hkv, p.v_tiles, p.Nk, p.nk, id - bh * p.nk, bh, smem);
+    } else {
+      const int bh = id / p.v_chunks;
+      float *dst = p.v_part + (size_t)id * D;
+      auto store = [&](int d, float s) { dst[d] = s; };
+      if (p.v_dtype == 0) v_absmax_body<D, 0>(p.v, p.vs, p.Hkv, p.Nk, p.v_rows, id - bh * p.v_chunks, bh, smem, store);
+      else v_absmax_body<D, 1>(p.v, p.vs, p.Hkv, p.Nk, p.v_rows, id - bh * p.v_chunks, bh, smem, store);
+    }
+  } else if constexpr (!POOL) {
+    const size_t row = (size_t)(w - p.wg_mask);
+#define SPG_M2L(K_) case K_: map_to_lut_body<K_>(p.mask, p.lut, p.valid, p.nk, p.nkp, row, smem); break;
+    switch (p.mask_kind) { SPG_M2L(0) SPG_M2L(1) SPG_M2L(2) SPG_M2L(3) SPG_M2L(4) SPG_M2L(5) SPG_M2L(6) }
+#undef SPG_M2L
+  }
+}
+
+struct FinalParams {
+  const double *km_part;
+  const float *v_part;
+  uint16_t *km;
+  float *v_amax;
+  int k_chunks, v_chunks, N;            // v_chunks == 0: no V maxima
+};
+
+// blockDim = (D, 8): eight threads share a column's partial results
+template <int D, int DT>
+__global__ void final_kernel(const FinalParams p) {
+  __shared__ double s_sub[8][D];
+  __shared__ float s_max[8][D];
+  const int bh = blockIdx.x, d = threadIdx.x, y = threadIdx.y;
+  double s = 0.0;
+#pragma unroll 4
+  for (int i = y; i < p.k_chunks; i += 8) s += p.km_part[((size_t)bh * p.k_chunks + i) * D + d];
+  float m = 0.f;
+#pragma unroll 4
+  for (int i = y; i < p.v_chunks; i += 8) m = fmaxf(m, p.v_part[((size_t)bh * p.v_chunks + i) * D + d]);
+  s_sub[y][d] = s;
+  s_max[y][d] = m;
+  __syncthreads();
+  if (y == 0) {
+#pragma unroll
+    for (int u = 1; u < 8; u++) { s += s_sub[u][d]; m = fmaxf(m, s_max[u][d]); }
+    p.km[(size_t)bh * D + d] = f64_to_elem<DT>(s / (double)p.N);
+    if (p.v_chunks > 0) p.v_amax[(size_t)bh * D + d] = m;
+  }
+}
+
+struct BackParams {
+  const uint16_t *k, *v;
+  Strides ks, vs;
+  int H, Hkv, Nk, nk;                   // H: query heads (simthr has one entry per query head)
+  int v_dtype;
+  int wg_v;                             // workgroups below it quantise K, the others V
+  int k_wgs_per_head;
+  const uint16_t *km;
+  const double *km_part;
+  int k_chunks;
+  const float *v_amax, *v_part;
+  int v_chunks;
+  Hyper simthr;
+  uint16_t *pool_k;
+  uint8_t *sim_k;
+  int8_t *k8;
+  float *k_scale;
+  uint8_t *v8;
+  float *v_scale;
+};
+
+// PARTIAL: the partial results of the front kernel are combined here, by every workgroup for the head it works on
+template <int D, int DT, bool POOL, bool PARTIAL>
+__global__ __launch_bounds__(256) void back_kernel(const BackParams p) {
+  constexpr int LK = POOL ? psq_lds<64, D>() : 256 * 8 + 2 * D;
+  constexpr int LV = v_quant_lds<D>() + 1024 + 4 * D;
+  __shared__ __align__(16) unsigned char smem[max_c<LK, LV>()];
+  const int w = blockIdx.x;
+  if (w < p.wg_v) {
+    const int bh = w / p.k_wgs_per_head;
+    float thr = 0.f;
+    if constexpr (POOL) thr = p.simthr.at((bh % p.Hkv) * (p.H / p.Hkv));
+    psq_body<64, D, DT, PARTIAL ? MEAN_PARTIAL : MEAN_GIVEN, POOL>(p.k, p.ks, p.km, p.km_part, p.k_chunks, p.pool_k, p.sim_k, p.k8,
+                                                                  p.k_scale, thr, p.Hkv, p.Nk, p.nk, w - bh * p.k_wgs_per_head, bh, smem);
+  } else {
+    const int id = w - p.wg_v, bh = id / p.nk, blk = id - bh * p.nk;
+    float *s_amax = (float *)(smem + v_quant_lds<D>());
+    float *s_sub = s_amax + D;
+    const int tid = threadIdx.x;
+    if constexpr (PARTIAL) {
+      float m = 0.f;
+#pragma unroll 4
+      for (int i = tid / D; i < p.v_chunks; i += 256 / D) m = fmaxf(m, p.v_part[((size_t)bh * p.v_chunks + i) * D + tid % D]);
+      s_sub[tid] = m;
+      __syncthreads();
+      if (tid < D) {
+#pragma unroll
+        for (int u = 1; u < 256 / D; u++) m = fmaxf(m, s_sub[tid + u * D]);
+        s_amax[tid] = m;
+      }
+    } else if (tid < D) {
+      s_amax[tid] = p.v_amax[(size_t)bh * D + tid];
+    }
+    __syncthreads();
+    if (blk == 0 && tid < D) p.v_scale[(size_t)bh * D + tid] = s_amax[tid] / 2.25f;
+    auto amax_of = [&](int d) { return s_amax[d]; };
+    if (p.v_dtype == 0) v_quant_body<D, 0>(p.v, p.vs, p.Hkv, p.v8, p.Nk, p.nk, blk, bh, smem, amax_of);
+    else v_quant_body<D, 1>(p.v, p.vs, p.Hkv, p.v8, p.Nk, p.nk, blk, bh, smem, amax_of);
+  }
+}
+
+// ---- workspace ----------------------------------------------------------------------------------------------------
+// Partial column sums / maxima: `chunks` workgroups per head.  Up to 8192 rows a head has at most sixteen chunks, few
+// enough to be combined by every workgroup of the back kernel (a few KiB from L2 against a launch of about 4.5 us);
+// beyond, the final kernel combines as many as it takes to spread the read over the chip.
+struct Chunks {
+  int n, rows;
+  bool partial;
+};
+static Chunks chunks_for(int heads, int N) {
+  Chunks c;
+  c.partial = N <= 8192;
+  const int want = c.partial ? 16 : (2048 + heads - 1) / heads;
+  const int most = c.partial ? (N + 63) / 64 : (N + 255) / 256;
+  c.n = want < most ? want : most;
+  c.rows = (N + c.n - 1) / c.n;
+  c.n = (N + c.rows - 1) / c.rows;      // no chunk without rows
+  return c;
+}
+
+struct Layout {
+  size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, total;
+};
+static Layout layout_for(const spg_attn_args *a) {
+  Layout l;
+  size_t at = 0;
+  auto take = [&](size_t bytes) { const size_t r = at; at += (bytes + 255) / 256 * 256; return r; };
+  const size_t bh = (size_t)a->B * a->H, bhk = (size_t)a->B * a->Hkv, D = a->D;
+  const size_t nq = ((size_t)a->N + 127) / 128, nk = ((size_t)a->N_kv + 63) / 64;
+  const Chunks c = chunks_for((int)bhk, a->N_kv);
+  const bool pool = a->selection != SPG_SELECT_MASK;
+  l.km_part = take(bhk * c.n * D * 8);
+  l.v_part = take(a->pv_f16 ? 0 : bhk * c.n * D * 4);
+  l.km = take(bhk * D * 2);
+  l.v_amax = take(bhk * D * 4);
+  l.pool_q = take(pool ? bh * nq * D * 2 : 0);
+  l.pool_k = take(pool ? bhk * nk * D * 2 : 0);
+  l.sim_q = take(pool ? bh * nq : 0);
+  l.sim_k = take(pool ? bhk * nk : 0);
+  l.q8 = take(bh * a->N * D);
+  l.k8 = take(bhk * a->N_kv * D);
+  l.q_scale = take(bh * nq * 4 * (a->qk_quant_gran == SPG_QUANT_PER_WARP ? 4 : 1));
+  l.k_scale = take(bhk * nk * 4);
+  l.v = take(bhk * nk * 64 * D * (a->pv_f16 ? 2 : 1));
+  l.v_scale = take(bhk * D * 4);
+  l.lut = take(bh * nq * nk * 4);
+  l.valid = take(bh * nq * 4);
+  l.total = at;
+  return l;
+}
+
+template <int D, int DT>
+static hipError_t run_front_back(const spg_attn_args *a, FrontParams &f, BackParams &b, const Chunks &c, uint16_t *km, float *v_amax,
+                                 int front_wgs, int back_wgs, hipStream_t st) {
+  const bool pool = a->selection != SPG_SELECT_MASK, per_warp = a->qk_quant_gran == SPG_QUANT_PER_WARP;
+  if (pool) {
+    if (per_warp) front_kernel<D, DT, true, 32><<<front_wgs, 256, 0, st>>>(f);
+    else front_kernel<D, DT, true, 128><<<front_wgs, 256, 0, st>>>(f);
+  } else {
+    if (per_warp) front_kernel<D, DT, false, 32><<<front_wgs, 256, 0, st>>>(f);
+    else front_kernel<D, DT, false, 128><<<front_wgs, 256, 0, st>>>(f);
+  }
+  if (!c.partial) {
+    const FinalParams p = {f.km_part, f.v_part, km, v_amax, f.k_chunks, a->pv_f16 ? 0 : f.v_chunks, a->N_kv};
+    final_kernel<D, DT><<<a->B * a->Hkv, dim3(D, 8), 0, st>>>(p);
+    if (pool) back_kernel<D, DT, true, false><<<back_wgs, 256, 0, st>>>(b);
+    else back_kernel<D, DT, false, false><<<back_wgs, 256, 0, st>>>(b);
+  } else {
+    if (pool) back_kernel<D, DT, true, true><<<back_wgs, 256, 0, st>>>(b);
+    else back_kernel<D, DT, false, true><<<back_wgs, 256, 0, st>>>(b);
+  }
+  return hipGetLastError();
+}
+
+static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides &ks, const Strides &vs, const Strides &os,
+                              hipStream_t st) {
+  const Layout l = layout_for(a);
+  unsigned char *ws = (unsigned char *)a->workspace;
+  const int heads = a->B * a->H, kv_heads = a->B * a->Hkv;
+  const int nq = (a->N + 127) / 128, nk = (a->N_kv + 63) / 64;
+  const Chunks c = chunks_for(kv_heads, a->N_kv);
+  const bool pool = a->selection != SPG_SELECT_MASK;
+  const Hyper simthr = {a->simthreshd1, a->simthreshd1_value};
+  int32_t *const lut = (int32_t *)(ws + l.lut);
+  int32_t *const valid = a->valid_block_num != nullptr ? a->valid_block_num : (int32_t *)(ws + l.valid);
+  int nkp = 256;
+  while (nkp < nk) nkp <<= 1;
+  const bool mask_in_front = !pool && nkp <= MASK_NKP_FRONT;
+
+  FrontParams f = {};
+  f.q = (const uint16_t *)a->q; f.k = (const uint16_t *)a->k; f.v = (const uint16_t *)a->v;
+  f.qs = qs; f.ks = ks; f.vs = vs;
+  f.H = a->H; f.Hkv = a->Hkv; f.N = a->N; f.Nk = a->N_kv; f.nq = nq; f.nk = nk;
+  f.v_dtype = a->v_dtype; f.v_f16 = a->pv_f16;
+  f.k_chunks = f.v_chunks = c.n; f.k_rows = f.v_rows = c.rows;
+  f.wg_v = kv_heads * c.n;
+  f.wg_mask = f.wg_v + kv_heads * (a->pv_f16 ? nk : c.n);
+  f.wg_q = f.wg_mask + (mask_in_front ? heads * nq : 0);
+  f.km_part = (double *)(ws + l.km_part); f.v_part = (float *)(ws + l.v_part); f.v_tiles = (uint16_t *)(ws + l.v);
+  f.mask = a->mask; f.mask_kind = a->mask_kind; f.nkp = nkp; f.lut = lut; f.valid = valid;
+  f.simthr = simthr;
+  f.pool_q = (uint16_t *)(ws + l.pool_q); f.sim_q = ws + l.sim_q; f.q8 = (int8_t *)(ws + l.q8); f.q_scale = (float *)(ws + l.q_scale);
+
+  BackParams b = {};
+  b.k = f.k; b.v = f.v; b.ks = ks; b.vs = vs;
+  b.H = a->H; b.Hkv = a->Hkv; b.Nk = a->N_kv; b.nk = nk; b.v_dtype = a->v_dtype;
+  b.k_wgs_per_head = (a->N_kv + 127) / 128;
+  b.wg_v = kv_heads * b.k_wgs_per_head;
+  b.km = (const uint16_t *)(ws + l.km); b.km_part = f.km_part; b.k_chunks = c.n;
+  b.v_amax = (const float *)(ws + l.v_amax); b.v_part = f.v_part; b.v_chunks = c.n;
+  b.simthr = simthr;
+  b.pool_k = (uint16_t *)(ws + l.pool_k); b.sim_k = ws + l.sim_k; b.k8 = (int8_t *)(ws + l.k8); b.k_scale = (float *)(ws + l.k_scale);
+  b.v8 = ws + l.v; b.v_scale = (float *)(ws + l.v_scale);
+
+  const int front_wgs = f.wg_q + heads * nq, back_wgs = b.wg_v + (a->pv_f16 ? 0 : kv_heads * nk);
+  uint16_t *km = (uint16_t *)(ws + l.km);
+  float *v_amax = (float *)(ws + l.v_amax);
+  hipError_t e;
+  if (a->D == 64) e = a->qk_dtype == 0 ? run_front_back<64, 0>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st)
+                                       : run_front_back<64, 1>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);
+  else e = a->qk_dtype == 0 ? run_front_back<128, 0>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st)
+                            : run_front_back<128, 1>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);
+  if (e != hipSuccess) return e;
+  if (pool)
+    e = launch_block_select_h(f.pool_q, f.sim_q, b.pool_k, b.sim_k, a->selection == SPG_SELECT_TOPK, Hyper{a->level, a->level_value},
+                              a->is_causal, a->attention_sink, lut, valid, nullptr, a->B, a->H, a->Hkv, nq, nk, a->D, a->qk_dtype, st);
+  else if (!mask_in_front)
+    e = launch_map_to_lut(a->mask, a->mask_kind, lut, valid, a->B, a->H, nq, nk, st);
+  if (e != hipSuccess) return e;
+  return launch_block_sparse_attn_h(f.q8, b.k8, b.v8, a->out, os, a->qk_dtype, lut, valid, Hyper{a->pvthreshd, a->pvthreshd_value},
+                                    f.q_scale, b.k_scale, a->pv_f16 ? nullptr : b.v_scale, a->B, a->H, a->Hkv, a->N, a->N_kv, a->D,
+                                    a->sm_scale, a->kernel_causal ? 1 : 0, a->qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0,
+                                    SPG_PV_PER_BLOCK, nullptr, st);
+}
+
+static int check_args(const char *fn, const spg_attn_args *a) {
+  SPG_TRY(check_shape(fn, a->B, a->H, a->N, a->D));
+  SPG_TRY(check_shape(fn, a->B, a->Hkv > 0 ? a->Hkv : 1, a->N_kv, a->D));
+  SPG_TRY(check_kv_heads(fn, a->H, a->Hkv));
+  SPG_TRY(check_dtype(fn, a->qk_dtype));
+  SPG_TRY(check_dtype(fn, a->v_dtype));
+  SPG_TRY(check_quant_gran(fn, a->qk_quant_gran));
+  if (a->selection < SPG_SELECT_TOPK || a->selection > SPG_SELECT_MASK)
+    return fail(SPG_ERR_INVALID, "%s: selection must be 0 (top-k), 1 (CDF) or 2 (mask), got %d", fn, a->selection);
+  const int nk = (a->N_kv + 63) / 64;
+  if (a->selection == SPG_SELECT_MASK) {
+    if (a->mask_kind < SPG_MASK_I8 || a->mask_kind > SPG_MASK_F64) return fail(SPG_ERR_INVALID, "%s: bad mask_kind %d", fn, a->mask_kind);
+    if (nk > 32768) return fail(SPG_ERR_UNSUPPORTED, "%s: nk = %d exceeds the supported maximum 32768", fn, nk);
+  } else if (nk > block_select_max_nk()) {
+    return fail(SPG_ERR_UNSUPPORTED, "%s: nk = %d exceeds the supported maximum %d", fn, nk, block_select_max_nk());
+  }
+  return SPG_OK;
+}
+
+}  // namespace spg
+using namespace spg;
+
+#pragma GCC visibility push(default)
+extern "C" {
+
+size_t spg_sparse_attn_workspace_bytes(const spg_attn_args *args) {
+  if (args == nullptr || check_args("spg_sparse_attn_workspace_bytes", args) != SPG_OK) return 0;
+  return layout_for(args).total;
+}
+
+int spg_sparse_attn(const spg_attn_args *args, void *stream) {
+  const char *fn = "spg_sparse_attn";
+  SPG_NONNULL(fn, args);
+  const spg_attn_args *a = args;
+  SPG_TRY(check_args(fn, a));
+  SPG_NONNULL(fn, a->q); SPG_NONNULL(fn, a->k); SPG_NONNULL(fn, a->v); SPG_NONNULL(fn, a->out); SPG_NONNULL(fn, a->workspace);
+  if (a->selection == SPG_SELECT_MASK) SPG_NONNULL(fn, a->mask);
+  const size_t need = layout_for(a).total;
+  if (a->workspace_bytes < need) return fail(SPG_ERR_INVALID, "%s: workspace of %zu bytes, %zu needed", fn, (size_t)a->workspace_bytes, need);
+  Strides qs, ks, vs, os;
+  SPG_TRY(get_strides(fn, "q_strides", a->q_strides, a->H, a->N, a->D, &qs));
+  SPG_TRY(get_strides(fn, "k_strides", a->k_strides, a->Hkv, a->N_kv, a->D, &ks));
+  SPG_TRY(get_strides(fn, "v_strides", a->v_strides, a->Hkv, a->N_kv, a->D, &vs));
+  SPG_TRY(get_strides(fn, "out_strides", a->out_strides, a->H, a->N, a->D, &os));
+  return check_launch(fn, run_forward(a, qs, ks, vs, os, (hipStream_t)stream));
+}
+
+}  // extern "C"
+#pragma GCC visibility pop

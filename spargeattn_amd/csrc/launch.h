@@ -12,6 +12,16 @@ struct Strides {
   long long sb, sh, sn;
 };
 
+// A per-head hyper-parameter: (H,) values on the device, or one value for all heads.  The second form takes no device
+// memory and no fill kernel.
+struct Hyper {
+  const float *p;
+  float v;
+#ifdef __HIPCC__
+  __device__ float at(int h) const { return p != nullptr ? p[h] : v; }
+#endif
+};
+
 size_t km_mean_workspace_bytes(int B, int H, int N, int D);
 void launch_km_mean(const void *k, Strides ks, void *km, void *ws, int B, int H, int N, int D, int dtype, hipStream_t st);
 // size of the library-owned scratch array behind launch_km_mean_static (bytes); a shape whose
@@ -26,6 +36,10 @@ int block_select_max_nk();
 hipError_t launch_block_select(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, const float *topk,
                                const float *cdf, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
                                int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st);
+// the same with the level (top-k fraction or CDF threshold) as a Hyper
+hipError_t launch_block_select_h(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, bool by_topk,
+                                 Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
+                                 int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st);
 void launch_div_selftest(unsigned long long *counts, int n_div, uint32_t seed, hipStream_t st);
 hipError_t launch_map_to_lut(const void *mask, int kind, int32_t *lut, int32_t *valid, int B, int H, int nq, int nk,
                              hipStream_t st);
@@ -41,6 +55,11 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st);
+hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
+                                      int out_dtype, const int32_t *lut, const int32_t *valid, Hyper pvthreshd,
+                                      const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
+                                      int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
+                                      int pv_mode, int32_t *pv_count, hipStream_t st);
 void launch_fp8_pack_selftest(const float *x, uint8_t *codes, int n, int saturate, hipStream_t st);
 
 hipError_t launch_dense_attn_f16(const void *q, const void *k, const void *v, void *out, int B, int H, int N, int D,

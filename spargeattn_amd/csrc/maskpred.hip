@@ -16,11 +16,9 @@
 // (round-to-nearest-even, straight from binary64); fp32 quantisation steps use IEEE divide / sqrt; the
 // compressed softmax uses a fixed binary64 operation sequence and a fixed summation tree.  This file must be
 // compiled with -ffp-contract=off.
-#include "common.h"
-#include "launch.h"
+#include "stage_bodies.h"
 
 #include <atomic>
-#include <type_traits>
 
 namespace spg {
 
@@ -30,35 +28,8 @@ namespace spg {
 template <int D, int DT>
 __global__ __launch_bounds__(256) void km_partial_kernel(const uint16_t *__restrict__ k, const Strides ks, int H,
                                                          double *__restrict__ part, int N, int rows_per_chunk) {
-  constexpr int TPR = D / 8;      // lanes per row (16 B each)
-  constexpr int RPP = 256 / TPR;  // rows per pass of the workgroup
-  const int bh = blockIdx.y, chunk = blockIdx.x, nchunk = gridDim.x;
-  const int c = threadIdx.x % TPR, r = threadIdx.x / TPR;
-  const int row0 = chunk * rows_per_chunk;
-  const int row1 = min(N, row0 + rows_per_chunk);
-  const uint16_t *base = k + (size_t)(bh / H) * ks.sb + (size_t)(bh % H) * ks.sh + c * 8;
-  double acc[8];
-#pragma unroll
-  for (int e = 0; e < 8; e++) acc[e] = 0.0;
-#pragma unroll 4
-  for (int row = row0 + r; row < row1; row += RPP) {
-    const uint4 v = load_stream_u4(base + (size_t)row * ks.sn);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      acc[2 * e] += (double)elem_to_f32<DT>((uint16_t)(w[e] & 0xffffu));
-      acc[2 * e + 1] += (double)elem_to_f32<DT>((uint16_t)(w[e] >> 16));
-    }
-  }
-  __shared__ double sm[RPP][D];
-#pragma unroll
-  for (int e = 0; e < 8; e++) sm[r][c * 8 + e] = acc[e];
-  __syncthreads();
-  if (threadIdx.x < D) {
-    double s = 0.0;
-    for (int i = 0; i < RPP; i++) s += sm[i][threadIdx.x];
-    part[((size_t)bh * nchunk + chunk) * D + threadIdx.x] = s;
-  }
+  __shared__ __align__(16) unsigned char smem[km_partial_lds<D>()];
+  km_partial_body<D, DT>(k, ks, H, part, N, rows_per_chunk, blockIdx.x, gridDim.x, blockIdx.y, smem);
 }
 
 // One workgroup per (batch, head), blockDim = (D, 8): eight threads share a column's partial sums (exact, so the order of
@@ -79,24 +50,6 @@ __global__ void km_final_kernel(const double *__restrict__ part, uint16_t *__res
     km[(size_t)bh * D + d] = f64_to_elem<DT>(t / (double)N);
   }
 }
-
-// =============================================================================================
-// pool + sim + INT8 quantisation.  One workgroup per (block, b*h).
-// =============================================================================================
-// IEEE binary32 quotient a/b with a reciprocal shared by many numerators: r = RN(1/b) (one correctly rounded
-// division), then q = RN(a*r), one exact residual and one correction (Markstein).  div_selftest_kernel below
-// compares it with the hardware's correctly rounded division for every finite binary16/bfloat16 numerator with
-// |a| >= 2^-100 against pseudo-random divisors: the only difference is the sign of a zero quotient, which no user of
-// the result can see.
-// Valid while b stays in [2^-60, 2^60] (no scaling of the operands is done); quotients below 2^-100 in magnitude
-// may be off in the last place, far below anything the callers resolve.
-__device__ __forceinline__ float exact_rcp(float b) { return 1.0f / b; }
-__device__ __forceinline__ float div_by(float a, float b, float r) {
-  const float q = a * r;
-  const float e = __builtin_fmaf(-b, q, a);
-  return __builtin_fmaf(e, r, q);
-}
-__device__ __forceinline__ bool rcp_safe(float b) { return b >= 0x1p-60f && b <= 0x1p60f; }
 
 // Self-test of div_by: divisor number i is a hash of (seed, i) with exponent in [-40, 40); every finite 16-bit
 // numerator of both element types with |a| >= 2^-100 and 2^-100 <= |a/b| <= 2^100 is divided both ways.  counts[0] += comparisons,
@@ -126,402 +79,18 @@ __global__ __launch_bounds__(256) void div_selftest_kernel(unsigned long long *c
   atomicAdd(&counts[1], bad);
 }
 
-// binary64 -> 16-bit pattern (round to nearest even) through binary32 where that provably gives the same bits: the
-// first rounding (to 24 bits) can only change the second one when it lands exactly on a rounding tie of the 16-bit
-// format, so every other value inside the format's normal range takes two hardware conversions instead of the 64-bit
-// integer arithmetic of f64_to_elem; ties, zero-range, subnormal and overflowing values go the exact way.
-template <int DT>
-__device__ __forceinline__ uint16_t f64_to_elem_fast(double x) {
-  const float r = (float)x;                                        // v_cvt_f32_f64
-  const uint32_t b = __builtin_bit_cast(uint32_t, r);
-  const uint32_t mag = b & 0x7fffffffu;
-  constexpr uint32_t DROP = DT == 1 ? 16u : 13u;                   // binary32 mantissa bits the 16-bit format drops
-  constexpr uint32_t LOW = (1u << DROP) - 1u, TIE = 1u << (DROP - 1u);
-  constexpr uint32_t LO = DT == 1 ? 0x00800000u : 0x38800000u;     // 2^-126 / 2^-14: smallest normal of the format
-  constexpr uint32_t HI = DT == 1 ? 0x7f000000u : 0x47000000u;     // 2^127 / 2^15: well below the overflow threshold
-  const bool safe = mag == 0u || (mag >= LO && mag < HI && (b & LOW) != TIE);
-  return safe ? f32_to_elem<DT>(r) : f64_to_elem<DT>(x);
-}
-
-// Packed 16-bit helpers.  A tile is kept in registers as the 16-bit patterns it was loaded with (two per register) and
-// widened where it is used: half the registers of a binary32 copy, which is what lets enough workgroups share a CU to
-// keep HBM busy.
-typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
-}
-template <int DT> __device__ __forceinline__ void unpack2(uint32_t w, float &lo, float &hi) {
-  lo = elem_to_f32<DT>((uint16_t)(w & 0xffffu));
-  hi = elem_to_f32<DT>((uint16_t)(w >> 16));
-}
-// two binary32 values -> two 16-bit patterns, round to nearest even
-template <int DT> __device__ __forceinline__ uint32_t pack_round2(float a, float b);
-template <> __device__ __forceinline__ uint32_t pack_round2<0>(float a, float b) {
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  const f2 v = {a, b};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, h2));
-}
-template <> __device__ __forceinline__ uint32_t pack_round2<1>(float a, float b) {
-  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  const f2 v = {a, b};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf2));   // v_cvt_pk_bf16_f32
-}
-// (int)y truncated toward zero, its low 8 bits written to byte B of acc: one instruction per element (the conversion's
-// sub-dword destination select) instead of a conversion plus shifts and ors.  Byte 0 clears the other three bytes, bytes
-// 1-3 keep them, so four calls in ascending order build a packed word without an initial value.
-template <int B>
-__device__ __forceinline__ void cvt_trunc_to_byte(uint32_t &acc, float y) {
-  if constexpr (B == 0) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD" : "=v"(acc) : "v"(y));
-  else if constexpr (B == 1) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(acc) : "v"(y));
-  else if constexpr (B == 2) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(acc) : "v"(y));
-  else asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(acc) : "v"(y));
-}
-// Hides a register's value from the optimiser: placed between two passes over the packed tile, it keeps the compiler
-// from carrying the widened (binary32) copies of one pass over to the next, which would double the registers again.
-__device__ __forceinline__ void forget(uint32_t &v) { asm volatile("" : "+v"(v)); }
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, SPG_WAVE));
-  return v;
-}
-
-// One workgroup handles 128 consecutive rows of one (batch, head): one 128-row block or two 64-row blocks (SUB), so
-// that the per-block tail (column reduction, pooled mean, flag, scale) is spread over all four wavefronts in both cases.
-// QR = rows that share one INT8 scale: BS (per-block granularity, what the reference's operators use) or 32 rows of a
-// 128-row Q block (per-warp granularity: quant_per_block.py:102-148 with WARPQ = 32, one scale per 32 query rows, which
-// are the rows of one wavefront of the attention kernel).  Pooling and the similarity flag stay per block.
+// pool + sim + INT8 quantisation: one workgroup per (128 rows, b*h)
 template <int BS, int D, int DT, bool HAS_MEAN, bool WITH_POOL, int QR = BS>
 __global__ __launch_bounds__(256) void pool_sim_quant_kernel(const uint16_t *__restrict__ x, const Strides xs,
                                                              const uint16_t *__restrict__ km,
                                                              uint16_t *__restrict__ pool, uint8_t *__restrict__ sim,
                                                              int8_t *__restrict__ xq, float *__restrict__ scale,
                                                              const float *__restrict__ simthr, int H, int N, int nb) {
-  constexpr int ROWS = 128;           // rows per workgroup
-  constexpr int SUB = ROWS / BS;      // blocks per workgroup
-  constexpr int TPR = D / 8;          // lanes per row (16 B each)
-  constexpr int RPP = 256 / TPR;      // rows per pass of the workgroup
-  constexpr int NPT = ROWS / RPP;     // passes (rows per thread)
-  constexpr int NP = BS / RPP;        // passes per block
-  constexpr int WPS = D / 64;         // wavefronts that hold one block's columns in the tail (thread = block * D + column)
-  constexpr int NQG = ROWS / QR;      // quantisation groups per workgroup (1, 2 or 4)
-  constexpr int GPB = BS / QR;        // ... per block
-  constexpr int NPQ = QR / RPP;       // passes per quantisation group
-  static_assert(BS == 64 || BS == 128, "block sizes of the operators");
-  static_assert(QR == BS || (QR == 32 && BS == 128), "per-block, or 32-row groups of a Q block");
-  static_assert(RPP <= QR, "a pass of the workgroup stays inside one quantisation group");
-  static_assert(RPP <= BS && SUB * D <= 256, "thread <-> (block, column) mapping of the tail");
-  // magnitude patterns (sign bit cleared) order like the magnitudes, for both 16-bit formats
-  constexpr uint32_t ABS2 = 0x7fff7fffu;
-  constexpr uint32_t INF16 = DT == 1 ? 0x7f80u : 0x7c00u;
-  // "every element of the row is tiny": bfloat16 below 2^-63 (both top exponent bits clear), binary16 zero
-  constexpr uint32_t TINY2 = DT == 1 ? 0x60006000u : 0x7fff7fffu;
-  const int bh = blockIdx.y;
-  const int tid = threadIdx.x, c = tid % TPR, r = tid / TPR;
-  const int row_base = blockIdx.x * ROWS;
-  const int rows_here = min(ROWS, N - row_base);          // >= 1
-  const bool partial = rows_here < ROWS;                  // workgroup-uniform: only the last workgroup of a head
-  const int blk0 = blockIdx.x * SUB;
-  auto rows_valid_of = [&](int sb) { return max(0, min(BS, rows_here - sb * BS)); };
-  const uint16_t *xb = x + (size_t)(bh / H) * xs.sb + (size_t)(bh % H) * xs.sh + (size_t)row_base * xs.sn + c * 8;
-
-  float kmf[8];
-  if constexpr (HAS_MEAN) {
-    const uint4 v = *(const uint4 *)(km + (size_t)bh * D + c * 8);
-    unpack2<DT>(v.x, kmf[0], kmf[1]);
-    unpack2<DT>(v.y, kmf[2], kmf[3]);
-    unpack2<DT>(v.z, kmf[4], kmf[5]);
-    unpack2<DT>(v.w, kmf[6], kmf[7]);
-  }
-
-  // all loads of the thread are issued before the first use (rows beyond the end re-read the last row and are zeroed
-  // afterwards: no load sits behind a branch)
-  uint32_t w[NPT][4];
-  {
-    uint4 raw[NPT];
-#pragma unroll
-    for (int p = 0; p < NPT; p++) raw[p] = load_stream_u4(xb + (size_t)min(r + p * RPP, rows_here - 1) * xs.sn);
-#pragma unroll
-    for (int p = 0; p < NPT; p++) { w[p][0] = raw[p].x; w[p][1] = raw[p].y; w[p][2] = raw[p].z; w[p][3] = raw[p].w; }
-  }
-  if constexpr (HAS_MEAN) {
-    // (k - km) rounded once to the input dtype (utils.py:184-188).  The binary32 difference of two 16-bit floats is
-    // either exact or nowhere near a rounding tie of the 16-bit format, so rounding it to nearest even equals rounding
-    // the exact difference.  The tile is kept as the rounded 16-bit patterns.
-#pragma unroll
-    for (int p = 0; p < NPT; p++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        float f0, f1;
-        unpack2<DT>(w[p][j], f0, f1);
-        w[p][j] = pack_round2<DT>(f0 - kmf[2 * j], f1 - kmf[2 * j + 1]);
-      }
-  }
-  if (partial) {                                  // masked rows are zero (utils.py:188)
-#pragma unroll
-    for (int p = 0; p < NPT; p++)
-      if (r + p * RPP >= rows_here) { w[p][0] = 0; w[p][1] = 0; w[p][2] = 0; w[p][3] = 0; }
-  }
-
-  // largest magnitude of the thread's elements per quantisation group (as 16-bit patterns: group g in half g % 2 of
-  // word g / 2) and, per row, whether all of the thread's elements are tiny
-  constexpr int MW = (NQG + 1) / 2;
-  uint32_t m_thread[MW], tiny_rows = 0;
-#pragma unroll
-  for (int i = 0; i < MW; i++) m_thread[i] = 0;
-#pragma unroll
-  for (int g = 0; g < NQG; g++) {
-    uint32_t m2 = 0;
-#pragma unroll
-    for (int p = g * NPQ; p < (g + 1) * NPQ; p++) {
-      const uint32_t rm = pk_max_u16(pk_max_u16(w[p][0] & ABS2, w[p][1] & ABS2), pk_max_u16(w[p][2] & ABS2, w[p][3] & ABS2));
-      m2 = pk_max_u16(m2, rm);
-      if constexpr (WITH_POOL) tiny_rows |= ((rm & TINY2) == 0 ? 1u : 0u) << p;
-    }
-    m_thread[g / 2] |= max(m2 & 0xffffu, m2 >> 16) << (16 * (g % 2));
-  }
-  // A NaN pattern lies above the infinity pattern and wins the maxima above.  The similarity flag wants exactly that
-  // (a block with a NaN is never "similar"), the quantisation scale does not: the reference's block maximum ignores NaN
-  // (tl.max lowers to a maxnum, utils.py:140 / 206), so only the NaN elements themselves are poisoned (they quantise to
-  // 0).  m_raw keeps the maxima with NaN for the flag; a thread that met one recomputes m_thread without (rare).
-  uint32_t m_raw[MW];
-#pragma unroll
-  for (int i = 0; i < MW; i++) m_raw[i] = m_thread[i];
-  {
-    bool nan_seen = false;
-#pragma unroll
-    for (int i = 0; i < MW; i++) nan_seen |= (m_thread[i] & 0xffffu) > INF16 || (m_thread[i] >> 16) > INF16;
-    if (nan_seen) {
-#pragma unroll
-      for (int i = 0; i < MW; i++) m_thread[i] = 0;
-#pragma unroll
-      for (int g = 0; g < NQG; g++) {
-        uint32_t m1 = 0;
-#pragma unroll
-        for (int p = g * NPQ; p < (g + 1) * NPQ; p++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const uint32_t lo = w[p][j] & 0x7fffu, hi = (w[p][j] >> 16) & 0x7fffu;
-            m1 = max(m1, max(lo > INF16 ? 0u : lo, hi > INF16 ? 0u : hi));
-          }
-        m_thread[g / 2] |= m1 << (16 * (g % 2));
-      }
-    }
-  }
-  // largest magnitude pattern of block sb as this thread (or, after the reduction, the workgroup) knows it
-  auto block_max = [&](const uint32_t(&mm)[MW], int sb) -> uint32_t {
-    uint32_t m = 0;
-#pragma unroll
-    for (int g = sb * GPB; g < (sb + 1) * GPB; g++) m = max(m, (mm[g / 2] >> (16 * (g % 2))) & 0xffffu);
-    return m;
-  };
-  __shared__ uint32_t s_wmax[4][MW], s_wbad[4];
-  __shared__ long long s_wg[4];
-#pragma unroll
-  for (int i = 0; i < MW; i++) {
-    uint32_t mw = m_thread[i];                    // two groups' maxima reduced together
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) mw = pk_max_u16(mw, (uint32_t)__shfl_xor((int)mw, o, SPG_WAVE));
-    if ((tid & 63) == 0) s_wmax[tid >> 6][i] = mw;
-  }
-
-  if constexpr (WITH_POOL) {
-    // column sums of all blocks of the workgroup, one row group per line; used for the pooled mean first and, with a
-    // non-negative similarity threshold, for the normalised rows afterwards
-    __shared__ double s_red[SUB][RPP][D];
-    // column sums for the pooled mean: binary64, exact
-#pragma unroll
-    for (int sb = 0; sb < SUB; sb++) {
-      double colsum[8];
-#pragma unroll
-      for (int e = 0; e < 8; e++) colsum[e] = 0.0;
-#pragma unroll
-      for (int p = sb * NP; p < (sb + 1) * NP; p++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          float f0, f1;
-          forget(w[p][j]);
-          unpack2<DT>(w[p][j], f0, f1);
-          colsum[2 * j] += (double)f0;
-          colsum[2 * j + 1] += (double)f1;
-        }
-#pragma unroll
-      for (int e = 0; e < 8; e++) s_red[sb][r][c * 8 + e] = colsum[e];
-    }
-
-    // row norms: the TPR lanes of a row group all need sqrt(sum of squares) and its reciprocal for each of their NPT
-    // rows.  Both are computed ONCE per NPT rows - lane c of the group takes row c % NPT - and handed round with lane
-    // reads, instead of NPT times in every lane.
-    static_assert(NPT <= TPR, "one lane of the row group per row");
-    // A NEGATIVE similarity threshold (the top-k operators' default, -0.1) decides the flag without the normalised rows:
-    // the statistic is ||sum of x_hat||^2 / rows^2 >= 0 > threshold whenever every x_hat is finite.  x_hat = x / norm is
-    // non-finite exactly for rows with norm == 0 (all-zero rows such as the padding of a partial block, or rows too
-    // small for their squares) and for non-finite x; |x| <= norm (1 + 2^-23) keeps every other quotient within fp16.
-    // Only two facts about the rows are needed then: is any element non-finite, and does any row have a zero norm.  A
-    // row whose largest |x| is at least 2^-63 has a sum of squares of at least 2^-126, a positive binary32 number; rows
-    // in which every element is smaller (all-zero rows, the padding of a partial block, bfloat16 values near the bottom
-    // of the range) are decided by the exact sums below.
-    const bool sim_trivial = simthr[bh % H] < 0.f;     // workgroup-uniform
-    uint32_t bad = 0;                                  // bit sb: block sb holds a non-finite x_hat
-    float ssf_mine = 0.f;
-    bool need_norms = true;                            // wavefront-uniform
-    if (sim_trivial) {
-#pragma unroll
-      for (int sb = 0; sb < SUB; sb++)                 // inf or NaN anywhere (overflowing squares of finite values are harmless: x / inf = 0)
-        bad |= (block_max(m_raw, sb) >= INF16 ? 1u : 0u) << sb;
-      tiny_rows = group_and_u32<TPR>(tiny_rows);      // rows tiny in every lane of their group
-      need_norms = __any(tiny_rows != 0);             // rare
-    }
-    if (need_norms) {
-      // sum of squares of every row (exact in binary64), rounded to binary32 like the reference's (utils.py:194)
-#pragma unroll
-      for (int p = 0; p < NPT; p++) {
-        double ss = 0.0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          float f0, f1;
-          forget(w[p][j]);
-          unpack2<DT>(w[p][j], f0, f1);
-          const double d0 = (double)f0, d1 = (double)f1;
-          ss = __builtin_fma(d0, d0, ss);             // squares and their sum are exact in binary64
-          ss = __builtin_fma(d1, d1, ss);
-        }
-        ss = group_sum_f64<TPR>(ss);                 // the TPR lanes of this row
-        const float ssf = (float)ss;
-        ssf_mine = (c % NPT == p) ? ssf : ssf_mine;
-        if (sim_trivial) bad |= ((ssf == 0.f) ? 1u : 0u) << (p / NP);
-      }
-    }
-    __syncthreads();
-    // tail: thread = block * D + column
-    const int t_sb = tid / D, t_col = tid % D;
-    const bool t_on = tid < SUB * D;
-    const int t_rows = rows_valid_of(t_sb);
-    if (t_on && t_rows > 0) {
-      double s = 0.0;
-      for (int i = 0; i < RPP; i++) s += s_red[t_sb][i][t_col];
-      // full blocks: the row count is a power of two, so the product with its reciprocal is the exact quotient
-      const double mean = t_rows == BS ? s * (1.0 / BS) : s / (double)t_rows;
-      pool[((size_t)bh * nb + blk0 + t_sb) * D + t_col] = f64_to_elem_fast<DT>(mean);
-    }
-    long long g = 0;
-    if (!sim_trivial) {
-      __syncthreads();                                // s_red is reused
-      const float norm_mine = sqrtf(ssf_mine);
-      const float rn_mine = rcp_safe(norm_mine) ? exact_rcp(norm_mine) : 0.f;
-      const int group_lane0 = (tid & 63) & ~(TPR - 1);
-#pragma unroll
-      for (int sb = 0; sb < SUB; sb++) {
-        double colxh[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) colxh[e] = 0.0;
-#pragma unroll
-        for (int p = sb * NP; p < (sb + 1) * NP; p++) {
-          const float norm = __shfl(norm_mine, group_lane0 + p, SPG_WAVE);
-          const float rn = __shfl(rn_mine, group_lane0 + p, SPG_WAVE);
-          const bool fast = rcp_safe(norm);
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            float f0, f1;
-            forget(w[p][j]);
-            unpack2<DT>(w[p][j], f0, f1);
-            // the slow branch gives 0/0 = NaN for all-zero (masked) rows
-            const _Float16 h0 = (_Float16)(fast ? div_by(f0, norm, rn) : f0 / norm);
-            const _Float16 h1 = (_Float16)(fast ? div_by(f1, norm, rn) : f1 / norm);
-            colxh[2 * j] += (double)(float)h0;        // fp16 values: integer multiples of 2^-24, sums are exact
-            colxh[2 * j + 1] += (double)(float)h1;
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < 8; e++) s_red[sb][r][c * 8 + e] = colxh[e];
-      }
-      __syncthreads();
-      if (t_on) {
-        double sx = 0.0;
-        for (int i = 0; i < RPP; i++) sx += s_red[t_sb][i][t_col];
-        if (__builtin_isfinite(sx)) {
-          const long long si = (long long)(sx * 16777216.0);   // exact integer
-          g = si * si;
-        } else {
-          bad |= 1u << t_sb;                          // a NaN/inf x_hat anywhere in the column
-        }
-      }
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) g += shfl_xor_i64(g, o);
-      if ((tid & 63) == 0) s_wg[tid >> 6] = g;
-    }
-    // bit sb of any_bad: some thread saw a non-finite x_hat in block sb (one flag word per wavefront, combined below)
-    {
-      uint32_t wb = 0;
-#pragma unroll
-      for (int sb = 0; sb < SUB; sb++) wb |= (__any((bad >> sb) & 1u) ? 1u : 0u) << sb;
-      if ((tid & 63) == 0) s_wbad[tid >> 6] = wb;
-    }
-    __syncthreads();
-    const uint32_t any_bad = s_wbad[0] | s_wbad[1] | s_wbad[2] | s_wbad[3];
-    if (tid < SUB && rows_valid_of(tid) > 0) {
-      const int rv = rows_valid_of(tid);
-      bool similar = sim_trivial;
-      if (!sim_trivial) {
-        long long gt = 0;                             // = sum(gram) * 2^48, exact
-        for (int i = 0; i < WPS; i++) gt += s_wg[tid * WPS + i];
-        const double thr = (double)simthr[bh % H] * (double)(rv * rv) * 281474976710656.0;
-        similar = (double)gt > thr;
-      }
-      sim[(size_t)bh * nb + blk0 + tid] = (!((any_bad >> tid) & 1u) && similar) ? 1 : 0;
-    }
-  } else {
-    __syncthreads();
-  }
-
-  uint32_t m_all[MW];
-#pragma unroll
-  for (int i = 0; i < MW; i++)
-    m_all[i] = pk_max_u16(pk_max_u16(s_wmax[0][i], s_wmax[1][i]), pk_max_u16(s_wmax[2][i], s_wmax[3][i]));
-  int8_t *qb = xq + ((size_t)bh * N + row_base) * D + c * 8;
-#pragma unroll
-  for (int g = 0; g < NQG; g++) {
-    // per-block scales exist for blocks with at least one row; the 32-row groups of the last Q block all get a scale
-    // (1e-7 for a group without rows, what the reference's quantiser writes for an all-masked group)
-    if (QR == BS && rows_here - g * QR <= 0) break;     // workgroup-uniform
-    const float amax = elem_to_f32<DT>((uint16_t)(m_all[g / 2] >> (16 * (g % 2))));
-    const float s = amax / 127.0f + 1e-7f;
-    auto quantise = [&](auto divide, auto check_rows) {
-#pragma unroll
-      for (int p = g * NPQ; p < (g + 1) * NPQ; p++) {
-        const int row = r + p * RPP;
-        if (!decltype(check_rows)::value || row < rows_here) {
-          float y[8];
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            float f[2];
-            forget(w[p][j]);
-            unpack2<DT>(w[p][j], f[0], f[1]);
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-              const float t = divide(f[h]);
-              y[2 * j + h] = t + __builtin_copysignf(0.5f, t);   // +0.5 for t >= 0 (a -0 quotient truncates to 0 either way)
-            }
-          }
-          uint32_t pk0, pk1;                       // truncation toward zero, low 8 bits of element e into byte e % 4
-          cvt_trunc_to_byte<0>(pk0, y[0]); cvt_trunc_to_byte<1>(pk0, y[1]); cvt_trunc_to_byte<2>(pk0, y[2]); cvt_trunc_to_byte<3>(pk0, y[3]);
-          cvt_trunc_to_byte<0>(pk1, y[4]); cvt_trunc_to_byte<1>(pk1, y[5]); cvt_trunc_to_byte<2>(pk1, y[6]); cvt_trunc_to_byte<3>(pk1, y[7]);
-          *(uint2 *)(qb + (size_t)row * D) = make_uint2(pk0, pk1);
-        }
-      }
-    };
-    if (rcp_safe(s) && !partial) {         // workgroup-uniform; the common case carries no row test
-      const float rs = exact_rcp(s);
-      quantise([&](float v) { return div_by(v, s, rs); }, std::false_type{});
-    } else if (rcp_safe(s)) {
-      const float rs = exact_rcp(s);
-      quantise([&](float v) { return div_by(v, s, rs); }, std::true_type{});
-    } else {
-      quantise([&](float v) { return v / s; }, std::true_type{});
-    }
-    if (tid == 0) scale[((size_t)bh * nb + blk0) * GPB + g] = s;
-  }
+  __shared__ __align__(16) unsigned char smem[WITH_POOL ? psq_lds<BS, D>() : 16];
+  float thr = 0.f;
+  if constexpr (WITH_POOL) thr = simthr[blockIdx.y % H];
+  psq_body<BS, D, DT, HAS_MEAN ? MEAN_GIVEN : MEAN_NONE, WITH_POOL, QR>(x, xs, km, nullptr, 0, pool, sim, xq, scale, thr, H, N, nb,
+                                                                        blockIdx.x, blockIdx.y, smem);
 }
 
 // =============================================================================================
@@ -548,45 +117,6 @@ __device__ __forceinline__ double cexp(double t) {
   return __builtin_ldexp(p, (int)k);
 }
 
-// exclusive prefix of per-thread counts over the 256 threads of the workgroup; returns (offset, total)
-__device__ __forceinline__ int2 block_exclusive_scan_i32(int v, int *s_tmp /* >= 4 ints */) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int inc = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(inc, o, SPG_WAVE);
-    if (lane >= o) inc += t;
-  }
-  __syncthreads();                       // s_tmp may still be read from a previous call
-  if (lane == 63) s_tmp[wave] = inc;
-  __syncthreads();
-  const int w0 = s_tmp[0], w1 = s_tmp[1], w2 = s_tmp[2], w3 = s_tmp[3];
-  const int base = (wave > 0 ? w0 : 0) + (wave > 1 ? w1 : 0) + (wave > 2 ? w2 : 0);
-  return make_int2(base + inc - v, w0 + w1 + w2 + w3);
-}
-
-// flags (per column, via functor) -> ascending compact index list -> delta LUT, zero tail, valid count.
-template <class FlagFn>
-__device__ __forceinline__ void emit_lut(FlagFn flag, int nk, int nkp, int32_t *s_idx, int *s_tmp,
-                                         int32_t *__restrict__ lut_row, int32_t *__restrict__ valid_out) {
-  const int tid = threadIdx.x;
-  const int seg = nkp / 256;
-  const int j0 = tid * seg, j1 = min(nk, j0 + seg);
-  int cnt = 0;
-  for (int j = j0; j < j1; j++) cnt += flag(j) ? 1 : 0;
-  const int2 st = block_exclusive_scan_i32(cnt, s_tmp);
-  int pos = st.x;
-  for (int j = j0; j < j1; j++)
-    if (flag(j)) s_idx[pos++] = j;
-  __syncthreads();
-  for (int p = tid; p < nk; p += 256) {
-    int v = 0;
-    if (p < st.y) v = s_idx[p] - (p ? s_idx[p - 1] : 0);
-    lut_row[p] = v;
-  }
-  if (tid == 0) *valid_out = st.y;
-}
-
 // =============================================================================================
 // block_select: one workgroup per (R consecutive q block rows, b*h).
 // Phase 1 computes the R x nk pooled scores with every pooled-K row read ONCE for the R rows (one lane per
@@ -597,7 +127,7 @@ __device__ __forceinline__ void emit_lut(FlagFn flag, int nk, int nkp, int32_t *
 template <int D, int DT, int R>
 __global__ __launch_bounds__(256) void block_select_kernel(
     const uint16_t *__restrict__ pool_q, const uint8_t *__restrict__ sim_q, const uint16_t *__restrict__ pool_k,
-    const uint8_t *__restrict__ sim_k, const float *__restrict__ topk, const float *__restrict__ cdfthr, int is_causal,
+    const uint8_t *__restrict__ sim_k, const bool by_topk, const Hyper level, int is_causal,
     int sink, int32_t *__restrict__ lut, int32_t *__restrict__ valid, uint8_t *__restrict__ bmap, int H, int Hkv, int nq,
     int nk, int nkp) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -718,8 +248,8 @@ __global__ __launch_bounds__(256) void block_select_kernel(
 
     // how many to keep
     long long n;
-    if (topk != nullptr) {
-      const float t = topk[h] * (float)nk;     // binary32 product, truncated (utils.py:405)
+    if (by_topk) {
+      const float t = level.at(h) * (float)nk;     // binary32 product, truncated (utils.py:405)
       n = (long long)t;
     } else {
       // cdf[i] = T(sum_{u<=i} p_sorted[u]);  n = #{i < nk : cdf[i] <= threshold}  (utils.py:398-403)
@@ -731,7 +261,7 @@ __global__ __launch_bounds__(256) void block_select_kernel(
       __syncthreads();
       double run = 0.0;
       for (int u = 0; u < tid; u++) run += s_tsum[u];
-      const double thr = (double)cdfthr[h];
+      const double thr = (double)level.at(h);
       int cnt = 0;
       for (int u = 0; u < seg; u++) {
         run += (double)elem_to_f32<DT>((uint16_t)(skey[p0 + u] >> 16));
@@ -822,7 +352,7 @@ __device__ __forceinline__ void bitonic_sort_desc(uint32_t (&key)[EPL], int lane
 template <int D, int DT, int NW, int EPL, bool DUAL>
 __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_select_wave_kernel(
     const uint16_t *__restrict__ pool_q, const uint8_t *__restrict__ sim_q, const uint16_t *__restrict__ pool_k,
-    const uint8_t *__restrict__ sim_k, const float *__restrict__ topk, const float *__restrict__ cdfthr, int is_causal,
+    const uint8_t *__restrict__ sim_k, const bool by_topk, const Hyper level, int is_causal,
     int sink, int32_t *__restrict__ lut, int32_t *__restrict__ valid, uint8_t *__restrict__ bmap, int H, int Hkv, int nq,
     int nk) {
   constexpr int R = 16;             // rows per workgroup: phase 1 computes 16 x 16 score tiles on the matrix unit
@@ -997,8 +527,8 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
     // how many to keep, and the key of the last one kept
     long long n;
     uint32_t kth = 0u;
-    if (topk != nullptr) {
-      const float t = topk[h] * (float)nk;            // binary32 product, truncated (utils.py:405)
+    if (by_topk) {
+      const float t = level.at(h) * (float)nk;            // binary32 product, truncated (utils.py:405)
       n = (long long)t;
       if (n <= 0) n = 1;                              // utils.py:289
       if (n < nk) {
@@ -1037,7 +567,7 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
       __builtin_amdgcn_wave_barrier();
       double run = 0.0;
       for (int u = 0; u < lane; u++) run += s_lsum[u];
-      const double thr = (double)cdfthr[h];
+      const double thr = (double)level.at(h);
       int cnt = 0;
 #pragma unroll
       for (int t = 0; t < EPL; t++) {
@@ -1097,29 +627,10 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
 // user mask -> LUT
 // =============================================================================================
 template <int KIND>
-__device__ __forceinline__ bool mask_nonzero(const void *row, int j) {
-  if constexpr (KIND == 0) return ((const uint8_t *)row)[j] != 0;
-  if constexpr (KIND == 1) return ((const uint16_t *)row)[j] != 0;
-  if constexpr (KIND == 2) return ((const uint32_t *)row)[j] != 0;
-  if constexpr (KIND == 3) return ((const uint64_t *)row)[j] != 0;
-  if constexpr (KIND == 4) return (((const uint16_t *)row)[j] & 0x7fffu) != 0;            // +-0.0 is zero
-  if constexpr (KIND == 5) return (((const uint32_t *)row)[j] & 0x7fffffffu) != 0;
-  if constexpr (KIND == 6) return (((const uint64_t *)row)[j] & 0x7fffffffffffffffull) != 0;
-  return false;
-}
-constexpr int mask_elem_size(int kind) { return kind == 0 ? 1 : (kind == 1 || kind == 4) ? 2 : (kind == 2 || kind == 5) ? 4 : 8; }
-
-template <int KIND>
 __global__ __launch_bounds__(256) void map_to_lut_kernel(const void *__restrict__ mask, int32_t *__restrict__ lut,
                                                          int32_t *__restrict__ valid, int nq, int nk, int nkp) {
   extern __shared__ __align__(16) unsigned char smem[];
-  int32_t *s_idx = (int32_t *)smem;
-  __shared__ int s_tmp[256];
-  const int i = blockIdx.x, bh = blockIdx.y;
-  const size_t row_off = ((size_t)bh * nq + i) * nk;
-  const void *row = (const unsigned char *)mask + row_off * mask_elem_size(KIND);
-  auto flag = [&](int j) -> bool { return mask_nonzero<KIND>(row, j); };
-  emit_lut(flag, nk, nkp, s_idx, s_tmp, lut + row_off, valid + (size_t)bh * nq + i);
+  map_to_lut_body<KIND>(mask, lut, valid, nk, nkp, (size_t)blockIdx.y * nq + blockIdx.x, smem);
 }
 
 // =============================================================================================
@@ -1255,8 +766,8 @@ void launch_div_selftest(unsigned long long *counts, int n_div, uint32_t seed, h
 }
 
 template <int D, int DT, int R>
-static hipError_t launch_bs3(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, const float *topk,
-                             const float *cdf, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap, int B,
+static hipError_t launch_bs3(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, bool by_topk,
+                             Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap, int B,
                              int H, int Hkv, int nq, int nk, int nkp, hipStream_t st) {
   const size_t lds = (size_t)R * D * 8 + (size_t)R * nkp * 4 + 12 * (size_t)nkp;
   auto kern = block_select_kernel<D, DT, R>;
@@ -1264,14 +775,14 @@ static hipError_t launch_bs3(const void *pq, const uint8_t *sq, const void *pk, 
     hipError_t e = allow_dynamic_lds<block_select_kernel<D, DT, R>>(lds);
     if (e != hipSuccess) return e;
   }
-  kern<<<dim3((nq + R - 1) / R, B * H), 256, lds, st>>>((const uint16_t *)pq, sq, (const uint16_t *)pk, sk, topk, cdf,
+  kern<<<dim3((nq + R - 1) / R, B * H), 256, lds, st>>>((const uint16_t *)pq, sq, (const uint16_t *)pk, sk, by_topk, level,
                                                         causal, sink, lut, valid, bmap, H, Hkv, nq, nk, nkp);
   return hipSuccess;
 }
 
 template <int D, int DT>
-static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, const float *topk,
-                             const float *cdf, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap, int B,
+static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, bool by_topk,
+                             Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap, int B,
                              int H, int Hkv, int nq, int nk, hipStream_t st) {
   const int nkp = next_pow2_ge(nk, 256);
   if (nkp <= 2048) {
@@ -1284,8 +795,8 @@ static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, 
         hipError_t e = allow_dynamic_lds<block_select_wave_kernel<D, DT, NW_, EPL_, DUAL_>>(lds);                      \
         if (e != hipSuccess) return e;                                                                          \
       }                                                                                                         \
-      kern<<<dim3((nq + 15) / 16, B * H), 64 * NW_, lds, st>>>((const uint16_t *)pq, sq, (const uint16_t *)pk, sk, topk, \
-                                                               cdf, causal, sink, lut, valid, bmap, H, Hkv, nq, nk); \
+      kern<<<dim3((nq + 15) / 16, B * H), 64 * NW_, lds, st>>>((const uint16_t *)pq, sq, (const uint16_t *)pk, sk, by_topk, \
+                                                               level, causal, sink, lut, valid, bmap, H, Hkv, nq, nk); \
       return hipSuccess;                                                                                        \
     }
     // one wavefront per row (16 per workgroup) where a row's registers fit the 128 a 1024-thread workgroup leaves each
@@ -1297,26 +808,33 @@ static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, 
 #undef SPG_BSW
   }
   // rows per workgroup: reuse of the pooled-K reads against LDS footprint (scores are R*nkp floats)
-  if (nkp <= 1024) return launch_bs3<D, DT, 8>(pq, sq, pk, sk, topk, cdf, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
-  if (nkp <= 4096) return launch_bs3<D, DT, 4>(pq, sq, pk, sk, topk, cdf, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
+  if (nkp <= 1024) return launch_bs3<D, DT, 8>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
+  if (nkp <= 4096) return launch_bs3<D, DT, 4>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
   // nkp = 8192: one row per workgroup (D*8 + 16*nkp = 129 KiB; two rows would need 162 KiB, more than the 160 KiB a
   // workgroup can have)
-  return launch_bs3<D, DT, 1>(pq, sq, pk, sk, topk, cdf, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
+  return launch_bs3<D, DT, 1>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
 }
 
-hipError_t launch_block_select(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, const float *topk,
-                               const float *cdf, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
-                               int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st) {
-#define SPG_BS(D_, DT_) return launch_bs2<D_, DT_>(pq, sq, pk, sk, topk, cdf, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, st)
+hipError_t launch_block_select_h(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, bool by_topk,
+                                 Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
+                                 int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st) {
+#define SPG_BS(D_, DT_) return launch_bs2<D_, DT_>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, st)
   if (D == 64) { if (dtype == 0) SPG_BS(64, 0); else SPG_BS(64, 1); }
   else         { if (dtype == 0) SPG_BS(128, 0); else SPG_BS(128, 1); }
 #undef SPG_BS
 }
 
+hipError_t launch_block_select(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, const float *topk,
+                               const float *cdf, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
+                               int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st) {
+  return launch_block_select_h(pq, sq, pk, sk, topk != nullptr, Hyper{topk != nullptr ? topk : cdf, 0.f}, causal, sink, lut, valid,
+                               bmap, B, H, Hkv, nq, nk, D, dtype, st);
+}
+
 hipError_t launch_map_to_lut(const void *mask, int kind, int32_t *lut, int32_t *valid, int B, int H, int nq, int nk,
                              hipStream_t st) {
   const int nkp = next_pow2_ge(nk, 256);
-  const size_t lds = 4 * (size_t)nkp;
+  const size_t lds = 4 * (size_t)nkp + 16;
   const dim3 grid(nq, B * H);
 #define SPG_M2L(K_)                                                                                      \
   case K_: {                                                                                             \

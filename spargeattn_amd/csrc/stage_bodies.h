@@ -1,0 +1,723 @@
+// Device code of the stages in front of the attention kernel, as bodies that more than one kernel is built from: the
+// stage-by-stage entry points launch one body per kernel (maskpred.hip, vquant.hip), the whole-operator entry point
+// launches several independent ones side by side in one kernel (forward.hip).  A body takes its place in the problem
+// (block, head) as arguments and its LDS as a pointer, so that bodies sharing a kernel share one allocation.
+//
+// Include only in translation units compiled with -ffp-contract=off (see the arithmetic contract in maskpred.hip).
+#pragma once
+#include "common.h"
+#include "launch.h"
+
+#include <type_traits>
+
+namespace spg {
+
+// =============================================================================================
+// K column mean
+// =============================================================================================
+template <int D> constexpr int km_partial_lds() { return 256 / (D / 8) * D * 8; }
+template <int D, int DT>
+__device__ __forceinline__ void km_partial_body(const uint16_t *__restrict__ k, const Strides &ks, int H,
+                                                double *__restrict__ part, int N, int rows_per_chunk, int chunk, int nchunk,
+                                                int bh, unsigned char *smem) {
+  constexpr int TPR = D / 8;      // lanes per row (16 B each)
+  constexpr int RPP = 256 / TPR;  // rows per pass of the workgroup
+  const int c = threadIdx.x % TPR, r = threadIdx.x / TPR;
+  const int row0 = chunk * rows_per_chunk;
+  const int row1 = min(N, row0 + rows_per_chunk);
+  const uint16_t *base = k + (size_t)(bh / H) * ks.sb + (size_t)(bh % H) * ks.sh + c * 8;
+  double acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) acc[e] = 0.0;
+#pragma unroll 4
+  for (int row = row0 + r; row < row1; row += RPP) {
+    const uint4 v = load_stream_u4(base + (size_t)row * ks.sn);
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      acc[2 * e] += (double)elem_to_f32<DT>((uint16_t)(w[e] & 0xffffu));
+      acc[2 * e + 1] += (double)elem_to_f32<DT>((uint16_t)(w[e] >> 16));
+    }
+  }
+  double(*sm)[D] = (double(*)[D])smem;
+#pragma unroll
+  for (int e = 0; e < 8; e++) sm[r][c * 8 + e] = acc[e];
+  __syncthreads();
+  if (threadIdx.x < D) {
+    double s = 0.0;
+    for (int i = 0; i < RPP; i++) s += sm[i][threadIdx.x];
+    part[((size_t)bh * nchunk + chunk) * D + threadIdx.x] = s;
+  }
+}
+
+// =============================================================================================
+// pool + sim + INT8 quantisation.  One workgroup per (block, b*h).
+// =============================================================================================
+// IEEE binary32 quotient a/b with a reciprocal shared by many numerators: r = RN(1/b) (one correctly rounded
+// division), then q = RN(a*r), one exact residual and one correction (Markstein).  div_selftest_kernel below
+// compares it with the hardware's correctly rounded division for every finite binary16/bfloat16 numerator with
+// |a| >= 2^-100 against pseudo-random divisors: the only difference is the sign of a zero quotient, which no user of
+// the result can see.
+// Valid while b stays in [2^-60, 2^60] (no scaling of the operands is done); quotients below 2^-100 in magnitude
+// may be off in the last place, far below anything the callers resolve.
+__device__ __forceinline__ float exact_rcp(float b) { return 1.0f / b; }
+__device__ __forceinline__ float div_by(float a, float b, float r) {
+  const float q = a * r;
+  const float e = __builtin_fmaf(-b, q, a);
+  return __builtin_fmaf(e, r, q);
+}
+__device__ __forceinline__ bool rcp_safe(float b) { return b >= 0x1p-60f && b <= 0x1p60f; }
+
+// binary64 -> 16-bit pattern (round to nearest even) through binary32 where that provably gives the same bits: the
+// first rounding (to 24 bits) can only change the second one when it lands exactly on a rounding tie of the 16-bit
+// format, so every other value inside the format's normal range takes two hardware conversions instead of the 64-bit
+// integer arithmetic of f64_to_elem; ties, zero-range, subnormal and overflowing values go the exact way.
+template <int DT>
+__device__ __forceinline__ uint16_t f64_to_elem_fast(double x) {
+  const float r = (float)x;                                        // v_cvt_f32_f64
+  const uint32_t b = __builtin_bit_cast(uint32_t, r);
+  const uint32_t mag = b & 0x7fffffffu;
+  constexpr uint32_t DROP = DT == 1 ? 16u : 13u;                   // binary32 mantissa bits the 16-bit format drops
+  constexpr uint32_t LOW = (1u << DROP) - 1u, TIE = 1u << (DROP - 1u);
+  constexpr uint32_t LO = DT == 1 ? 0x00800000u : 0x38800000u;     // 2^-126 / 2^-14: smallest normal of the format
+  constexpr uint32_t HI = DT == 1 ? 0x7f000000u : 0x47000000u;     // 2^127 / 2^15: well below the overflow threshold
+  const bool safe = mag == 0u || (mag >= LO && mag < HI && (b & LOW) != TIE);
+  return safe ? f32_to_elem<DT>(r) : f64_to_elem<DT>(x);
+}
+
+// Packed 16-bit helpers.  A tile is kept in registers as the 16-bit patterns it was loaded with (two per register) and
+// widened where it is used: half the registers of a binary32 copy, which is what lets enough workgroups share a CU to
+// keep HBM busy.
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
+}
+template <int DT> __device__ __forceinline__ void unpack2(uint32_t w, float &lo, float &hi) {
+  lo = elem_to_f32<DT>((uint16_t)(w & 0xffffu));
+  hi = elem_to_f32<DT>((uint16_t)(w >> 16));
+}
+// two binary32 values -> two 16-bit patterns, round to nearest even
+template <int DT> __device__ __forceinline__ uint32_t pack_round2(float a, float b);
+template <> __device__ __forceinline__ uint32_t pack_round2<0>(float a, float b) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  const f2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, h2));
+}
+template <> __device__ __forceinline__ uint32_t pack_round2<1>(float a, float b) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  const f2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf2));   // v_cvt_pk_bf16_f32
+}
+// (int)y truncated toward zero, its low 8 bits written to byte B of acc: one instruction per element (the conversion's
+// sub-dword destination select) instead of a conversion plus shifts and ors.  Byte 0 clears the other three bytes, bytes
+// 1-3 keep them, so four calls in ascending order build a packed word without an initial value.
+template <int B>
+__device__ __forceinline__ void cvt_trunc_to_byte(uint32_t &acc, float y) {
+  if constexpr (B == 0) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD" : "=v"(acc) : "v"(y));
+  else if constexpr (B == 1) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(acc) : "v"(y));
+  else if constexpr (B == 2) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(acc) : "v"(y));
+  else asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(acc) : "v"(y));
+}
+// Hides a register's value from the optimiser: placed between two passes over the packed tile, it keeps the compiler
+// from carrying the widened (binary32) copies of one pass over to the next, which would double the registers again.
+__device__ __forceinline__ void forget(uint32_t &v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, SPG_WAVE));
+  return v;
+}
+
+// One workgroup handles 128 consecutive rows of one (batch, head): one 128-row block or two 64-row blocks (SUB), so
+// that the per-block tail (column reduction, pooled mean, flag, scale) is spread over all four wavefronts in both cases.
+// QR = rows that share one INT8 scale: BS (per-block granularity, what the reference's operators use) or 32 rows of a
+// 128-row Q block (per-warp granularity: quant_per_block.py:102-148 with WARPQ = 32, one scale per 32 query rows, which
+// are the rows of one wavefront of the attention kernel).  Pooling and the similarity flag stay per block.
+// MEAN: 0 no mean (Q), 1 the finished column mean `km`, 2 the partial column sums km_part (km_chunks per head) that
+// km_partial_body wrote - every workgroup adds them up for itself, which takes the small kernel in between out of the
+// launch chain and pays while there are few chunks.
+enum { MEAN_NONE = 0, MEAN_GIVEN = 1, MEAN_PARTIAL = 2 };
+template <int BS, int D> constexpr int psq_lds() { return 128 / BS * (256 / (D / 8)) * D * 8; }
+template <int BS, int D, int DT, int MEAN, bool WITH_POOL, int QR = BS>
+__device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const Strides &xs,
+                                         const uint16_t *__restrict__ km, const double *__restrict__ km_part, int km_chunks,
+                                         uint16_t *__restrict__ pool, uint8_t *__restrict__ sim,
+                                         int8_t *__restrict__ xq, float *__restrict__ scale,
+                                         const float simthr, int H, int N, int nb, int wg, int bh, unsigned char *smem) {
+  constexpr int ROWS = 128;           // rows per workgroup
+  constexpr int SUB = ROWS / BS;      // blocks per workgroup
+  constexpr int TPR = D / 8;          // lanes per row (16 B each)
+  constexpr int RPP = 256 / TPR;      // rows per pass of the workgroup
+  constexpr int NPT = ROWS / RPP;     // passes (rows per thread)
+  constexpr int NP = BS / RPP;        // passes per block
+  constexpr int WPS = D / 64;         // wavefronts that hold one block's columns in the tail (thread = block * D + column)
+  constexpr int NQG = ROWS / QR;      // quantisation groups per workgroup (1, 2 or 4)
+  constexpr int GPB = BS / QR;        // ... per block
+  constexpr int NPQ = QR / RPP;       // passes per quantisation group
+  static_assert(BS == 64 || BS == 128, "block sizes of the operators");
+  static_assert(QR == BS || (QR == 32 && BS == 128), "per-block, or 32-row groups of a Q block");
+  static_assert(RPP <= QR, "a pass of the workgroup stays inside one quantisation group");
+  static_assert(RPP <= BS && SUB * D <= 256, "thread <-> (block, column) mapping of the tail");
+  // magnitude patterns (sign bit cleared) order like the magnitudes, for both 16-bit formats
+  constexpr uint32_t ABS2 = 0x7fff7fffu;
+  constexpr uint32_t INF16 = DT == 1 ? 0x7f80u : 0x7c00u;
+  // "every element of the row is tiny": bfloat16 below 2^-63 (both top exponent bits clear), binary16 zero
+  constexpr uint32_t TINY2 = DT == 1 ? 0x60006000u : 0x7fff7fffu;
+  constexpr bool HAS_MEAN = MEAN != MEAN_NONE;
+  const int tid = threadIdx.x, c = tid % TPR, r = tid / TPR;
+  const int row_base = wg * ROWS;
+  const int rows_here = min(ROWS, N - row_base);          // >= 1
+  const bool partial = rows_here < ROWS;                  // workgroup-uniform: only the last workgroup of a head
+  const int blk0 = wg * SUB;
+  auto rows_valid_of = [&](int sb) { return max(0, min(BS, rows_here - sb * BS)); };
+  const uint16_t *xb = x + (size_t)(bh / H) * xs.sb + (size_t)(bh % H) * xs.sh + (size_t)row_base * xs.sn + c * 8;
+
+  // all loads of the thread are issued before the first use (rows beyond the end re-read the last row and are zeroed
+  // afterwards: no load sits behind a branch)
+  uint32_t w[NPT][4];
+  {
+    uint4 raw[NPT];
+#pragma unroll
+    for (int p = 0; p < NPT; p++) raw[p] = load_stream_u4(xb + (size_t)min(r + p * RPP, rows_here - 1) * xs.sn);
+#pragma unroll
+    for (int p = 0; p < NPT; p++) { w[p][0] = raw[p].x; w[p][1] = raw[p].y; w[p][2] = raw[p].z; w[p][3] = raw[p].w; }
+  }
+  if constexpr (HAS_MEAN) {
+    float kmf[8];
+    uint4 v;
+    if constexpr (MEAN == MEAN_GIVEN) {
+      v = *(const uint4 *)(km + (size_t)bh * D + c * 8);
+    } else {
+      // (the sums are exact in binary64: their order is free)
+      constexpr int G = 256 / D;
+      double *s_sub = (double *)smem;
+      uint16_t *s_km = (uint16_t *)(smem + 256 * 8);
+      double s = 0.0;
+#pragma unroll 4
+      for (int i = tid / D; i < km_chunks; i += G) s += km_part[((size_t)bh * km_chunks + i) * D + tid % D];
+      s_sub[tid] = s;
+      __syncthreads();
+      if (tid < D) {
+        double t = s_sub[tid];
+#pragma unroll
+        for (int u = 1; u < G; u++) t += s_sub[tid + u * D];
+        s_km[tid] = f64_to_elem<DT>(t / (double)N);
+      }
+      __syncthreads();
+      v = *(const uint4 *)(s_km + c * 8);
+      __syncthreads();                                // the LDS is used again below
+    }
+    unpack2<DT>(v.x, kmf[0], kmf[1]);
+    unpack2<DT>(v.y, kmf[2], kmf[3]);
+    unpack2<DT>(v.z, kmf[4], kmf[5]);
+    unpack2<DT>(v.w, kmf[6], kmf[7]);
+    // (k - km) rounded once to the input dtype (utils.py:184-188).  The binary32 difference of two 16-bit floats is
+    // either exact or nowhere near a rounding tie of the 16-bit format, so rounding it to nearest even equals rounding
+    // the exact difference.  The tile is kept as the rounded 16-bit patterns.
+#pragma unroll
+    for (int p = 0; p < NPT; p++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        float f0, f1;
+        unpack2<DT>(w[p][j], f0, f1);
+        w[p][j] = pack_round2<DT>(f0 - kmf[2 * j], f1 - kmf[2 * j + 1]);
+      }
+  }
+  if (partial) {                                  // masked rows are zero (utils.py:188)
+#pragma unroll
+    for (int p = 0; p < NPT; p++)
+      if (r + p * RPP >= rows_here) { w[p][0] = 0; w[p][1] = 0; w[p][2] = 0; w[p][3] = 0; }
+  }
+
+  // largest magnitude of the thread's elements per quantisation group (as 16-bit patterns: group g in half g % 2 of
+  // word g / 2) and, per row, whether all of the thread's elements are tiny
+  constexpr int MW = (NQG + 1) / 2;
+  uint32_t m_thread[MW], tiny_rows = 0;
+#pragma unroll
+  for (int i = 0; i < MW; i++) m_thread[i] = 0;
+#pragma unroll
+  for (int g = 0; g < NQG; g++) {
+    uint32_t m2 = 0;
+#pragma unroll
+    for (int p = g * NPQ; p < (g + 1) * NPQ; p++) {
+      const uint32_t rm = pk_max_u16(pk_max_u16(w[p][0] & ABS2, w[p][1] & ABS2), pk_max_u16(w[p][2] & ABS2, w[p][3] & ABS2));
+      m2 = pk_max_u16(m2, rm);
+      if constexpr (WITH_POOL) tiny_rows |= ((rm & TINY2) == 0 ? 1u : 0u) << p;
+    }
+    m_thread[g / 2] |= max(m2 & 0xffffu, m2 >> 16) << (16 * (g % 2));
+  }
+  // A NaN pattern lies above the infinity pattern and wins the maxima above.  The similarity flag wants exactly that
+  // (a block with a NaN is never "similar"), the quantisation scale does not: the reference's block maximum ignores NaN
+  // (tl.max lowers to a maxnum, utils.py:140 / 206), so only the NaN elements themselves are poisoned (they quantise to
+  // 0).  m_raw keeps the maxima with NaN for the flag; a thread that met one recomputes m_thread without (rare).
+  uint32_t m_raw[MW];
+#pragma unroll
+  for (int i = 0; i < MW; i++) m_raw[i] = m_thread[i];
+  {
+    bool nan_seen = false;
+#pragma unroll
+    for (int i = 0; i < MW; i++) nan_seen |= (m_thread[i] & 0xffffu) > INF16 || (m_thread[i] >> 16) > INF16;
+    if (nan_seen) {
+#pragma unroll
+      for (int i = 0; i < MW; i++) m_thread[i] = 0;
+#pragma unroll
+      for (int g = 0; g < NQG; g++) {
+        uint32_t m1 = 0;
+#pragma unroll
+        for (int p = g * NPQ; p < (g + 1) * NPQ; p++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const uint32_t lo = w[p][j] & 0x7fffu, hi = (w[p][j] >> 16) & 0x7fffu;
+            m1 = max(m1, max(lo > INF16 ? 0u : lo, hi > INF16 ? 0u : hi));
+          }
+        m_thread[g / 2] |= m1 << (16 * (g % 2));
+      }
+    }
+  }
+  // largest magnitude pattern of block sb as this thread (or, after the reduction, the workgroup) knows it
+  auto block_max = [&](const uint32_t(&mm)[MW], int sb) -> uint32_t {
+    uint32_t m = 0;
+#pragma unroll
+    for (int g = sb * GPB; g < (sb + 1) * GPB; g++) m = max(m, (mm[g / 2] >> (16 * (g % 2))) & 0xffffu);
+    return m;
+  };
+  __shared__ uint32_t s_wmax[4][MW], s_wbad[4];
+  __shared__ long long s_wg[4];
+#pragma unroll
+  for (int i = 0; i < MW; i++) {
+    uint32_t mw = m_thread[i];                    // two groups' maxima reduced together
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) mw = pk_max_u16(mw, (uint32_t)__shfl_xor((int)mw, o, SPG_WAVE));
+    if ((tid & 63) == 0) s_wmax[tid >> 6][i] = mw;
+  }
+
+  if constexpr (WITH_POOL) {
+    // column sums of all blocks of the workgroup, one row group per line; used for the pooled mean first and, with a
+    // non-negative similarity threshold, for the normalised rows afterwards
+    double(*s_red)[RPP][D] = (double(*)[RPP][D])smem;
+    // column sums for the pooled mean: binary64, exact
+#pragma unroll
+    for (int sb = 0; sb < SUB; sb++) {
+      double colsum[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) colsum[e] = 0.0;
+#pragma unroll
+      for (int p = sb * NP; p < (sb + 1) * NP; p++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          float f0, f1;
+          forget(w[p][j]);
+          unpack2<DT>(w[p][j], f0, f1);
+          colsum[2 * j] += (double)f0;
+          colsum[2 * j + 1] += (double)f1;
+        }
+#pragma unroll
+      for (int e = 0; e < 8; e++) s_red[sb][r][c * 8 + e] = colsum[e];
+    }
+
+    // row norms: the TPR lanes of a row group all need sqrt(sum of squares) and its reciprocal for each of their NPT
+    // rows.  Both are computed ONCE per NPT rows - lane c of the group takes row c % NPT - and handed round with lane
+    // reads, instead of NPT times in every lane.
+    static_assert(NPT <= TPR, "one lane of the row group per row");
+    // A NEGATIVE similarity threshold (the top-k operators' default, -0.1) decides the flag without the normalised rows:
+    // the statistic is ||sum of x_hat||^2 / rows^2 >= 0 > threshold whenever every x_hat is finite.  x_hat = x / norm is
+    // non-finite exactly for rows with norm == 0 (all-zero rows such as the padding of a partial block, or rows too
+    // small for their squares) and for non-finite x; |x| <= norm (1 + 2^-23) keeps every other quotient within fp16.
+    // Only two facts about the rows are needed then: is any element non-finite, and does any row have a zero norm.  A
+    // row whose largest |x| is at least 2^-63 has a sum of squares of at least 2^-126, a positive binary32 number; rows
+    // in which every element is smaller (all-zero rows, the padding of a partial block, bfloat16 values near the bottom
+    // of the range) are decided by the exact sums below.
+    const bool sim_trivial = simthr < 0.f;     // workgroup-uniform
+    uint32_t bad = 0;                                  // bit sb: block sb holds a non-finite x_hat
+    float ssf_mine = 0.f;
+    bool need_norms = true;                            // wavefront-uniform
+    if (sim_trivial) {
+#pragma unroll
+      for (int sb = 0; sb < SUB; sb++)                 // inf or NaN anywhere (overflowing squares of finite values are harmless: x / inf = 0)
+        bad |= (block_max(m_raw, sb) >= INF16 ? 1u : 0u) << sb;
+      tiny_rows = group_and_u32<TPR>(tiny_rows);      // rows tiny in every lane of their group
+      need_norms = __any(tiny_rows != 0);             // rare
+    }
+    if (need_norms) {
+      // sum of squares of every row (exact in binary64), rounded to binary32 like the reference's (utils.py:194)
+#pragma unroll
+      for (int p = 0; p < NPT; p++) {
+        double ss = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          float f0, f1;
+          forget(w[p][j]);
+          unpack2<DT>(w[p][j], f0, f1);
+          const double d0 = (double)f0, d1 = (double)f1;
+          ss = __builtin_fma(d0, d0, ss);             // squares and their sum are exact in binary64
+          ss = __builtin_fma(d1, d1, ss);
+        }
+        ss = group_sum_f64<TPR>(ss);                 // the TPR lanes of this row
+        const float ssf = (float)ss;
+        ssf_mine = (c % NPT == p) ? ssf : ssf_mine;
+        if (sim_trivial) bad |= ((ssf == 0.f) ? 1u : 0u) << (p / NP);
+      }
+    }
+    __syncthreads();
+    // tail: thread = block * D + column
+    const int t_sb = tid / D, t_col = tid % D;
+    const bool t_on = tid < SUB * D;
+    const int t_rows = rows_valid_of(t_sb);
+    if (t_on && t_rows > 0) {
+      double s = 0.0;
+      for (int i = 0; i < RPP; i++) s += s_red[t_sb][i][t_col];
+      // full blocks: the row count is a power of two, so the product with its reciprocal is the exact quotient
+      const double mean = t_rows == BS ? s * (1.0 / BS) : s / (double)t_rows;
+      pool[((size_t)bh * nb + blk0 + t_sb) * D + t_col] = f64_to_elem_fast<DT>(mean);
+    }
+    long long g = 0;
+    if (!sim_trivial) {
+      __syncthreads();                                // s_red is reused
+      const float norm_mine = sqrtf(ssf_mine);
+      const float rn_mine = rcp_safe(norm_mine) ? exact_rcp(norm_mine) : 0.f;
+      const int group_lane0 = (tid & 63) & ~(TPR - 1);
+#pragma unroll
+      for (int sb = 0; sb < SUB; sb++) {
+        double colxh[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) colxh[e] = 0.0;
+#pragma unroll
+        for (int p = sb * NP; p < (sb + 1) * NP; p++) {
+          const float norm = __shfl(norm_mine, group_lane0 + p, SPG_WAVE);
+          const float rn = __shfl(rn_mine, group_lane0 + p, SPG_WAVE);
+          const bool fast = rcp_safe(norm);
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            float f0, f1;
+            forget(w[p][j]);
+            unpack2<DT>(w[p][j], f0, f1);
+            // the slow branch gives 0/0 = NaN for all-zero (masked) rows
+            const _Float16 h0 = (_Float16)(fast ? div_by(f0, norm, rn) : f0 / norm);
+            const _Float16 h1 = (_Float16)(fast ? div_by(f1, norm, rn) : f1 / norm);
+            colxh[2 * j] += (double)(float)h0;        // fp16 values: integer multiples of 2^-24, sums are exact
+            colxh[2 * j + 1] += (double)(float)h1;
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) s_red[sb][r][c * 8 + e] = colxh[e];
+      }
+      __syncthreads();
+      if (t_on) {
+        double sx = 0.0;
+        for (int i = 0; i < RPP; i++) sx += s_red[t_sb][i][t_col];
+        if (__builtin_isfinite(sx)) {
+          const long long si = (long long)(sx * 16777216.0);   // exact integer
+          g = si * si;
+        } else {
+          bad |= 1u << t_sb;                          // a NaN/inf x_hat anywhere in the column
+        }
+      }
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) g += shfl_xor_i64(g, o);
+      if ((tid & 63) == 0) s_wg[tid >> 6] = g;
+    }
+    // bit sb of any_bad: some thread saw a non-finite x_hat in block sb (one flag word per wavefront, combined below)
+    {
+      uint32_t wb = 0;
+#pragma unroll
+      for (int sb = 0; sb < SUB; sb++) wb |= (__any((bad >> sb) & 1u) ? 1u : 0u) << sb;
+      if ((tid & 63) == 0) s_wbad[tid >> 6] = wb;
+    }
+    __syncthreads();
+    const uint32_t any_bad = s_wbad[0] | s_wbad[1] | s_wbad[2] | s_wbad[3];
+    if (tid < SUB && rows_valid_of(tid) > 0) {
+      const int rv = rows_valid_of(tid);
+      bool similar = sim_trivial;
+      if (!sim_trivial) {
+        long long gt = 0;                             // = sum(gram) * 2^48, exact
+        for (int i = 0; i < WPS; i++) gt += s_wg[tid * WPS + i];
+        const double thr = (double)simthr * (double)(rv * rv) * 281474976710656.0;
+        similar = (double)gt > thr;
+      }
+      sim[(size_t)bh * nb + blk0 + tid] = (!((any_bad >> tid) & 1u) && similar) ? 1 : 0;
+    }
+  } else {
+    __syncthreads();
+  }
+
+  uint32_t m_all[MW];
+#pragma unroll
+  for (int i = 0; i < MW; i++)
+    m_all[i] = pk_max_u16(pk_max_u16(s_wmax[0][i], s_wmax[1][i]), pk_max_u16(s_wmax[2][i], s_wmax[3][i]));
+  int8_t *qb = xq + ((size_t)bh * N + row_base) * D + c * 8;
+#pragma unroll
+  for (int g = 0; g < NQG; g++) {
+    // per-block scales exist for blocks with at least one row; the 32-row groups of the last Q block all get a scale
+    // (1e-7 for a group without rows, what the reference's quantiser writes for an all-masked group)
+    if (QR == BS && rows_here - g * QR <= 0) break;     // workgroup-uniform
+    const float amax = elem_to_f32<DT>((uint16_t)(m_all[g / 2] >> (16 * (g % 2))));
+    const float s = amax / 127.0f + 1e-7f;
+    auto quantise = [&](auto divide, auto check_rows) {
+#pragma unroll
+      for (int p = g * NPQ; p < (g + 1) * NPQ; p++) {
+        const int row = r + p * RPP;
+        if (!decltype(check_rows)::value || row < rows_here) {
+          float y[8];
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            float f[2];
+            forget(w[p][j]);
+            unpack2<DT>(w[p][j], f[0], f[1]);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+              const float t = divide(f[h]);
+              y[2 * j + h] = t + __builtin_copysignf(0.5f, t);   // +0.5 for t >= 0 (a -0 quotient truncates to 0 either way)
+            }
+          }
+          uint32_t pk0, pk1;                       // truncation toward zero, low 8 bits of element e into byte e % 4
+          cvt_trunc_to_byte<0>(pk0, y[0]); cvt_trunc_to_byte<1>(pk0, y[1]); cvt_trunc_to_byte<2>(pk0, y[2]); cvt_trunc_to_byte<3>(pk0, y[3]);
+          cvt_trunc_to_byte<0>(pk1, y[4]); cvt_trunc_to_byte<1>(pk1, y[5]); cvt_trunc_to_byte<2>(pk1, y[6]); cvt_trunc_to_byte<3>(pk1, y[7]);
+          *(uint2 *)(qb + (size_t)row * D) = make_uint2(pk0, pk1);
+        }
+      }
+    };
+    if (rcp_safe(s) && !partial) {         // workgroup-uniform; the common case carries no row test
+      const float rs = exact_rcp(s);
+      quantise([&](float v) { return div_by(v, s, rs); }, std::false_type{});
+    } else if (rcp_safe(s)) {
+      const float rs = exact_rcp(s);
+      quantise([&](float v) { return div_by(v, s, rs); }, std::true_type{});
+    } else {
+      quantise([&](float v) { return v / s; }, std::true_type{});
+    }
+    if (tid == 0) scale[((size_t)bh * nb + blk0) * GPB + g] = s;
+  }
+}
+
+// exclusive prefix of per-thread counts over the 256 threads of the workgroup; returns (offset, total)
+__device__ __forceinline__ int2 block_exclusive_scan_i32(int v, int *s_tmp /* >= 4 ints */) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int inc = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(inc, o, SPG_WAVE);
+    if (lane >= o) inc += t;
+  }
+  __syncthreads();                       // s_tmp may still be read from a previous call
+  if (lane == 63) s_tmp[wave] = inc;
+  __syncthreads();
+  const int w0 = s_tmp[0], w1 = s_tmp[1], w2 = s_tmp[2], w3 = s_tmp[3];
+  const int base = (wave > 0 ? w0 : 0) + (wave > 1 ? w1 : 0) + (wave > 2 ? w2 : 0);
+  return make_int2(base + inc - v, w0 + w1 + w2 + w3);
+}
+
+// flags (per column, via functor) -> ascending compact index list -> delta LUT, zero tail, valid count.
+template <class FlagFn>
+__device__ __forceinline__ void emit_lut(FlagFn flag, int nk, int nkp, int32_t *s_idx, int *s_tmp,
+                                         int32_t *__restrict__ lut_row, int32_t *__restrict__ valid_out) {
+  const int tid = threadIdx.x;
+  const int seg = nkp / 256;
+  const int j0 = tid * seg, j1 = min(nk, j0 + seg);
+  int cnt = 0;
+  for (int j = j0; j < j1; j++) cnt += flag(j) ? 1 : 0;
+  const int2 st = block_exclusive_scan_i32(cnt, s_tmp);
+  int pos = st.x;
+  for (int j = j0; j < j1; j++)
+    if (flag(j)) s_idx[pos++] = j;
+  __syncthreads();
+  for (int p = tid; p < nk; p += 256) {
+    int v = 0;
+    if (p < st.y) v = s_idx[p] - (p ? s_idx[p - 1] : 0);
+    lut_row[p] = v;
+  }
+  if (tid == 0) *valid_out = st.y;
+}
+
+// =============================================================================================
+// user mask -> LUT
+// =============================================================================================
+template <int KIND>
+__device__ __forceinline__ bool mask_nonzero(const void *row, int j) {
+  if constexpr (KIND == 0) return ((const uint8_t *)row)[j] != 0;
+  if constexpr (KIND == 1) return ((const uint16_t *)row)[j] != 0;
+  if constexpr (KIND == 2) return ((const uint32_t *)row)[j] != 0;
+  if constexpr (KIND == 3) return ((const uint64_t *)row)[j] != 0;
+  if constexpr (KIND == 4) return (((const uint16_t *)row)[j] & 0x7fffu) != 0;            // +-0.0 is zero
+  if constexpr (KIND == 5) return (((const uint32_t *)row)[j] & 0x7fffffffu) != 0;
+  if constexpr (KIND == 6) return (((const uint64_t *)row)[j] & 0x7fffffffffffffffull) != 0;
+  return false;
+}
+constexpr int mask_elem_size(int kind) { return kind == 0 ? 1 : (kind == 1 || kind == 4) ? 2 : (kind == 2 || kind == 5) ? 4 : 8; }
+
+// one row of a user mask -> LUT row; LDS: 4 * nkp bytes for the index list, 16 for the scan
+template <int KIND>
+__device__ __forceinline__ void map_to_lut_body(const void *__restrict__ mask, int32_t *__restrict__ lut,
+                                                int32_t *__restrict__ valid, int nk, int nkp, size_t row_id,
+                                                unsigned char *smem) {
+  int32_t *s_idx = (int32_t *)(smem + 16);
+  const size_t row_off = row_id * nk;
+  const void *row = (const unsigned char *)mask + row_off * mask_elem_size(KIND);
+  auto flag = [&](int j) -> bool { return mask_nonzero<KIND>(row, j); };
+  emit_lut(flag, nk, nkp, s_idx, (int *)smem, lut + row_off, valid + row_id);
+}
+
+// =============================================================================================
+// V path
+// =============================================================================================
+template <int DT>
+__device__ __forceinline__ float elem_to_f16_f32(uint16_t b) {
+  // value of the element after the cast to fp16 the reference applies to V (core.py:117)
+  if constexpr (DT == 0) return elem_to_f32<0>(b);
+  const _Float16 h = (_Float16)elem_to_f32<1>(b);
+  return (float)h;
+}
+
+// Largest |fp16(v)| of every channel over one chunk of rows.  store(d, value) receives the result of channel d.
+template <int D> constexpr int v_absmax_lds() { return 256 / (D / 8) * D * 4; }
+template <int D, int DT, class Store>
+__device__ __forceinline__ void v_absmax_body(const uint16_t *__restrict__ v, const Strides &vs, int H, int N,
+                                              int rows_per_chunk, int chunk, int bh, unsigned char *smem, Store store) {
+  constexpr int TPR = D / 8;
+  constexpr int RPP = 256 / TPR;
+  const int c = threadIdx.x % TPR, r = threadIdx.x / TPR;
+  const int row0 = chunk * rows_per_chunk;
+  const int row1 = min(N, row0 + rows_per_chunk);
+  const uint16_t *base = v + (size_t)(bh / H) * vs.sb + (size_t)(bh % H) * vs.sh + c * 8;
+  // The cast to fp16 is monotonic in the magnitude, so the largest |fp16(v)| is the cast of the largest |v|: the maximum
+  // is taken on the 16-bit magnitude patterns (which order like the magnitudes), two per instruction, and only the
+  // result is converted.
+  typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+  constexpr uint32_t INF16 = DT == 1 ? 0x7f80u : 0x7c00u;
+  uint32_t mp[4] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int row = row0 + r; row < row1; row += RPP) {
+    const uint4 q = load_stream_u4(base + (size_t)row * vs.sn);
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      mp[j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, mp[j]),
+                                                                      __builtin_bit_cast(u16x2_t, w[j] & 0x7fff7fffu)));
+  }
+  // A NaN pattern lies above the infinity pattern and would win the maximum, whereas the reference's fmaxf / fminf
+  // (fused.cu:120-123) ignore NaN: only the NaN elements themselves are poisoned, not their channel's scale.  The
+  // common case pays one test; a thread that met a NaN goes over its rows again with the NaN patterns taken as zero.
+  if (max(max(mp[0] & 0xffffu, mp[0] >> 16), max(mp[1] & 0xffffu, mp[1] >> 16)) > INF16 ||
+      max(max(mp[2] & 0xffffu, mp[2] >> 16), max(mp[3] & 0xffffu, mp[3] >> 16)) > INF16) {
+    mp[0] = mp[1] = mp[2] = mp[3] = 0;
+    for (int row = row0 + r; row < row1; row += RPP) {
+      const uint4 q = *(const uint4 *)(base + (size_t)row * vs.sn);
+      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        uint32_t lo = w[j] & 0x7fffu, hi = (w[j] >> 16) & 0x7fffu;
+        lo = lo > INF16 ? 0u : lo;
+        hi = hi > INF16 ? 0u : hi;
+        mp[j] = max(mp[j] & 0xffffu, lo) | (max(mp[j] >> 16, hi) << 16);
+      }
+    }
+  }
+  float m[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++)
+    m[e] = elem_to_f16_f32<DT>((uint16_t)((e & 1) ? (mp[e >> 1] >> 16) : (mp[e >> 1] & 0xffffu)));
+  float(*sm)[D] = (float(*)[D])smem;
+#pragma unroll
+  for (int e = 0; e < 8; e++) sm[r][c * 8 + e] = m[e];
+  __syncthreads();
+  if (threadIdx.x < D) {
+    float s = 0.f;
+    for (int i = 0; i < RPP; i++) s = fmaxf(s, sm[i][threadIdx.x]);
+    store((int)threadIdx.x, s);
+  }
+}
+
+// One workgroup per 64-key tile.  LDS holds the transposed tile [D][64] bytes.
+// amax_of(d): the channel maximum (a whole-head value, from wherever the kernel has it).
+template <int D> constexpr int v_quant_lds() { return D * (64 + 4); }
+template <int D, int DT, class Amax>
+__device__ __forceinline__ void v_quant_body(const uint16_t *__restrict__ v, const Strides &vs, int H,
+                                             uint8_t *__restrict__ v8, int N, int nk, int blk, int bh, unsigned char *smem,
+                                             Amax amax_of) {
+  constexpr int TPR = D / 8;
+  constexpr int RPP = 256 / TPR;
+  constexpr int NP = 64 / RPP;
+  constexpr int LDW = 64 + 4;  // padded row (bytes) of the transposed tile
+  uint8_t *tile = smem;
+  const int tid = threadIdx.x;
+  const int c = tid % TPR, r = tid / TPR;
+  const uint16_t *base = v + (size_t)(bh / H) * vs.sb + (size_t)(bh % H) * vs.sh + (size_t)blk * 64 * vs.sn + c * 8;
+  const int last_row = min(63, N - 1 - blk * 64);
+  uint4 raw[NP];                     // every load is issued before the first use; rows beyond N re-read the last row
+#pragma unroll
+  for (int p = 0; p < NP; p++) raw[p] = load_stream_u4(base + (size_t)min(r + p * RPP, last_row) * vs.sn);
+  float recp[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) recp[e] = 2.25f / amax_of(c * 8 + e);
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    const int row = r + p * RPP;
+    const bool ok = row <= last_row;
+    const uint4 q = raw[p];
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const float a = elem_to_f16_f32<DT>((uint16_t)(w[e >> 1] & 0xffffu)) * recp[e];
+      const float b = elem_to_f16_f32<DT>((uint16_t)(w[e >> 1] >> 16)) * recp[e + 1];
+      const int pk = ok ? __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) : 0;   // rows beyond N are zero
+      tile[(c * 8 + e) * LDW + row] = (uint8_t)(pk & 0xff);
+      tile[(c * 8 + e + 1) * LDW + row] = (uint8_t)((pk >> 8) & 0xff);
+    }
+  }
+  __syncthreads();
+  uint8_t *out = v8 + ((size_t)bh * nk + blk) * (size_t)(D * 64);
+  for (int i = tid; i < D * 4; i += 256) {   // 16-byte pieces: D rows x 4 slots
+    const int d = i >> 2, slot = i & 3;
+    const int kc = slot ^ ((d >> 2) & 3);      // key chunk stored in this slot
+    const uint32_t *src = (const uint32_t *)(tile + d * LDW + kc * 16);
+    *(uint4 *)(out + d * 64 + slot * 16) = make_uint4(src[0], src[1], src[2], src[3]);
+  }
+}
+
+// V -> fp16 -> V^T tiles [nk][D][64] fp16 for the fp16-PV attention variant.  Inside a 128-byte tile row (one channel,
+// 64 keys) the eight 8-key chunks are stored at slot = chunk ^ ((d >> 1) & 7) (the LDS swizzle of the attention kernel).
+// Keys at or beyond N are zero.  One workgroup per 64-key tile.
+template <int D> constexpr int v_tiles_f16_lds() { return D * (64 + 2) * 2; }
+template <int D, int DT>
+__device__ __forceinline__ void v_tiles_f16_body(const uint16_t *__restrict__ v, const Strides &vs, int H,
+                                                 uint16_t *__restrict__ vt, int N, int nk, int blk, int bh,
+                                                 unsigned char *smem) {
+  constexpr int TPR = D / 8;
+  constexpr int RPP = 256 / TPR;
+  constexpr int NP = 64 / RPP;
+  constexpr int LDW = 64 + 2;  // padded row (halves) of the transposed tile
+  uint16_t *tile = (uint16_t *)smem;
+  const int tid = threadIdx.x;
+  const int c = tid % TPR, r = tid / TPR;
+  const uint16_t *base = v + (size_t)(bh / H) * vs.sb + (size_t)(bh % H) * vs.sh + (size_t)blk * 64 * vs.sn + c * 8;
+  const int last_row = min(63, N - 1 - blk * 64);
+  uint4 raw[NP];
+#pragma unroll
+  for (int p = 0; p < NP; p++) raw[p] = load_stream_u4(base + (size_t)min(r + p * RPP, last_row) * vs.sn);
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    const int row = r + p * RPP;
+    const uint4 q = row <= last_row ? raw[p] : make_uint4(0, 0, 0, 0);
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const uint16_t b = (uint16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu));
+      uint16_t h = b;
+      if constexpr (DT == 1) h = f32_to_elem<0>(elem_to_f32<1>(b));     // bf16 -> fp16, one rounding
+      tile[(c * 8 + e) * LDW + row] = h;
+    }
+  }
+  __syncthreads();
+  uint16_t *out = vt + ((size_t)bh * nk + blk) * (size_t)(D * 64);
+  for (int i = tid; i < D * 8; i += 256) {   // 16-byte pieces: D rows x 8 slots
+    const int d = i >> 3, slot = i & 7;
+    const int kc = slot ^ ((d >> 1) & 7);      // key chunk stored in this slot
+    const uint16_t *src = tile + d * LDW + kc * 8;
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] = (uint32_t)src[2 * e] | ((uint32_t)src[2 * e + 1] << 16);
+    *(uint4 *)(out + d * 64 + slot * 8) = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
+}  // namespace spg

@@ -296,6 +296,66 @@ Tensor block_sparse_attn_f16v_meta(const Tensor &q8, const Tensor &, const Tenso
   return pv_count_alloc(q8, return_pv_count);
 }
 
+// ---- the whole operator ------------------------------------------------------------------------------------------
+// q, k, v and out are handed over in the caller's own layout: sizes = {B, H, Hkv, N, N_kv, D}, the stride lists are
+// {batch, head, row}.  Returns valid_block_num (B,H,nq).
+Tensor sparse_attn(const Tensor &q, const Tensor &k, const Tensor &v, Tensor out, const c10::optional<Tensor> &mask,
+                   const c10::optional<Tensor> &level, double level_value, const c10::optional<Tensor> &simthreshd1,
+                   double simthreshd1_value, const c10::optional<Tensor> &pvthreshd, double pvthreshd_value, at::IntArrayRef sizes,
+                   at::IntArrayRef q_strides, at::IntArrayRef k_strides, at::IntArrayRef v_strides, at::IntArrayRef out_strides,
+                   int64_t selection, bool pv_f16, bool is_causal, bool attention_sink, bool kernel_causal, int64_t qk_quant_gran,
+                   double sm_scale) {
+  CHECK_GPU(q); CHECK_GPU(k); CHECK_GPU(v); CHECK_GPU(out);
+  TORCH_CHECK(sizes.size() == 6 && q_strides.size() == 3 && k_strides.size() == 3 && v_strides.size() == 3 && out_strides.size() == 3,
+              "sizes must be {B, H, Hkv, N, N_kv, D} and strides {batch, head, row}");
+  TORCH_CHECK(k.scalar_type() == q.scalar_type() && out.scalar_type() == q.scalar_type(), "q, k and out must have one dtype");
+  const DeviceGuard guard(q.device());
+  spg_attn_args a = {};
+  a.B = sizes[0]; a.H = sizes[1]; a.Hkv = sizes[2]; a.N = sizes[3]; a.N_kv = sizes[4]; a.D = sizes[5];
+  a.qk_dtype = dtype_of(q); a.v_dtype = dtype_of(v);
+  a.selection = selection; a.pv_f16 = pv_f16; a.is_causal = is_causal; a.attention_sink = attention_sink;
+  a.kernel_causal = kernel_causal; a.qk_quant_gran = qk_quant_gran;
+  for (const auto *t : {&level, &simthreshd1, &pvthreshd})
+    if (t->has_value()) {
+      CHECK_GPU(**t); CHECK_CONTIGUOUS(**t); CHECK_DTYPE(**t, at::kFloat);
+      TORCH_CHECK((*t)->numel() == a.H, "per-head hyper-parameter has ", (*t)->numel(), " entries, expected ", a.H);
+    }
+  a.level = (const float *)opt_ptr(level); a.level_value = level_value;
+  a.simthreshd1 = (const float *)opt_ptr(simthreshd1); a.simthreshd1_value = simthreshd1_value;
+  a.pvthreshd = (const float *)opt_ptr(pvthreshd); a.pvthreshd_value = pvthreshd_value;
+  a.sm_scale = sm_scale;
+  // the last element a (size, stride) pair reaches has to lie inside the tensor's storage
+  auto fits = [&](const Tensor &t, at::IntArrayRef st, int64_t h, int64_t n, const char *name) {
+    TORCH_CHECK(st[0] >= 0 && st[1] >= 0 && st[2] >= 0 && t.storage_offset() + (sizes[0] - 1) * st[0] + (h - 1) * st[1] + (n - 1) * st[2] + a.D <=
+                (int64_t)(t.storage().nbytes() / t.element_size()), "Tensor ", name, ": sizes and strides reach beyond its storage");
+    TORCH_CHECK((uintptr_t)t.data_ptr() % 16 == 0, "Tensor ", name, " must be 16-byte aligned");
+  };
+  fits(q, q_strides, a.H, a.N, "q"); fits(k, k_strides, a.Hkv, a.N_kv, "k"); fits(v, v_strides, a.Hkv, a.N_kv, "v");
+  fits(out, out_strides, a.H, a.N, "out");
+  const int64_t nq = (a.N + 127) / 128, nk = (a.N_kv + 63) / 64;
+  if (mask.has_value()) {
+    CHECK_GPU(*mask); CHECK_CONTIGUOUS(*mask);
+    CHECK_SHAPE(*mask, a.B, a.H, nq, nk);
+    a.mask = mask->data_ptr(); a.mask_kind = mask_kind_of(*mask);
+  }
+  a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.out = out.data_ptr();
+  a.q_strides = q_strides.data(); a.k_strides = k_strides.data(); a.v_strides = v_strides.data(); a.out_strides = out_strides.data();
+  Tensor valid = at::empty({a.B, a.H, nq}, q.options().dtype(at::kInt));
+  a.valid_block_num = (int32_t *)valid.data_ptr();
+  a.workspace_bytes = spg_sparse_attn_workspace_bytes(&a);
+  if (a.workspace_bytes == 0) check(SPG_ERR_INVALID);
+  Tensor ws = at::empty({(int64_t)a.workspace_bytes}, q.options().dtype(at::kByte));
+  a.workspace = ws.data_ptr();
+  check(spg_sparse_attn(&a, stream_of(q)));
+  return valid;
+}
+Tensor sparse_attn_meta(const Tensor &q, const Tensor &, const Tensor &, Tensor, const c10::optional<Tensor> &,
+                        const c10::optional<Tensor> &, double, const c10::optional<Tensor> &, double, const c10::optional<Tensor> &,
+                        double, at::IntArrayRef sizes, at::IntArrayRef, at::IntArrayRef, at::IntArrayRef, at::IntArrayRef, int64_t,
+                        bool, bool, bool, bool, int64_t, double) {
+  return at::empty({sizes[0], sizes[1], (sizes[3] + 127) / 128}, q.options().dtype(at::kInt));
+}
+
 // ---- measurement comparator and self tests ------------------------------------------------------------------------
 Tensor dense_attn_f16(const Tensor &q, const Tensor &k, const Tensor &vt, Tensor out, double sm_scale, bool is_causal) {
   CHECK_GPU(q); CHECK_GPU(k); CHECK_GPU(vt); CHECK_GPU(out);
@@ -340,6 +400,7 @@ TORCH_LIBRARY(spargeattn_amd, m) {
   m.def("v_tiles_f16(Tensor v) -> Tensor");
   m.def("block_sparse_attn(Tensor q8, Tensor k8, Tensor v8, Tensor(a!) out, Tensor lut, Tensor valid_block_num, Tensor pvthreshd, Tensor q_scale, Tensor k_scale, Tensor v_scale, float sm_scale, bool is_causal, int qk_quant_gran, int pv_threshold_mode, bool return_pv_count) -> Tensor");
   m.def("block_sparse_attn_f16v(Tensor q8, Tensor k8, Tensor vt, Tensor(a!) out, Tensor lut, Tensor valid_block_num, Tensor pvthreshd, Tensor q_scale, Tensor k_scale, float sm_scale, bool is_causal, int qk_quant_gran, int pv_threshold_mode, bool return_pv_count) -> Tensor");
+  m.def("sparse_attn(Tensor q, Tensor k, Tensor v, Tensor(a!) out, Tensor? mask, Tensor? level, float level_value, Tensor? simthreshd1, float simthreshd1_value, Tensor? pvthreshd, float pvthreshd_value, int[] sizes, int[] q_strides, int[] k_strides, int[] v_strides, int[] out_strides, int selection, bool pv_f16, bool is_causal, bool attention_sink, bool kernel_causal, int qk_quant_gran, float sm_scale) -> Tensor");
   m.def("dense_attn_f16(Tensor q, Tensor k, Tensor vt, Tensor(a!) out, float sm_scale, bool is_causal) -> Tensor(a!)");
   m.def("selftest_fp8_pack(Tensor x, bool saturate) -> Tensor");
   m.def("selftest_division(Tensor(a!) counts, int n_divisors, int seed) -> Tensor(a!)");
@@ -355,6 +416,7 @@ TORCH_LIBRARY_IMPL(spargeattn_amd, CUDA, m) {
   m.impl("v_tiles_f16", &v_tiles_f16);
   m.impl("block_sparse_attn", &block_sparse_attn);
   m.impl("block_sparse_attn_f16v", &block_sparse_attn_f16v);
+  m.impl("sparse_attn", &sparse_attn);
   m.impl("dense_attn_f16", &dense_attn_f16);
   m.impl("selftest_fp8_pack", &selftest_fp8_pack);
   m.impl("selftest_division", &selftest_division);
@@ -369,6 +431,7 @@ TORCH_LIBRARY_IMPL(spargeattn_amd, Meta, m) {
   m.impl("v_tiles_f16", &v_tiles_f16_meta);
   m.impl("block_sparse_attn", &block_sparse_attn_meta);
   m.impl("block_sparse_attn_f16v", &block_sparse_attn_f16v_meta);
+  m.impl("sparse_attn", &sparse_attn_meta);
   m.impl("dense_attn_f16", &dense_attn_f16_meta);
   m.impl("selftest_fp8_pack", &selftest_fp8_pack_meta);
   m.impl("selftest_division", &selftest_division_meta);

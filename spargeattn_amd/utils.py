@@ -90,6 +90,14 @@ def block_map_lut_triton(block_map):
 block_map_lut = block_map_lut_triton
 
 
+def check_grouped_simthreshd1(simthreshd1, H, Hkv):
+    """Raises if a per-head similarity threshold differs inside a group of query heads that share a K/V head."""
+    grouped = simthreshd1.view(Hkv, H // Hkv)
+    if not bool((grouped == grouped[:, :1]).all()):
+        raise ValueError("simthreshd1 must be equal for the query heads that share a K/V head "
+                         f"({H} query heads, {Hkv} K/V heads): K is pooled once per K/V head")
+
+
 def get_block_map_meansim_fuse_quant(q, k, km=None, is_causal=False, BLKQ=128, BLKK=64, simthreshd1=0.1,
                                      cdfthreshd=0.9, topk=None, is_sparse=True, return_lut=False,
                                      attention_sink=False, qk_quant_gran=1):
@@ -118,10 +126,7 @@ def get_block_map_meansim_fuse_quant(q, k, km=None, is_causal=False, BLKQ=128, B
     # to its first entry); every query head of the group is scored against those pooled blocks with its own topk /
     # cdfthreshd.
     if Hkv != H and per_head_sim:
-        grouped = simthreshd1.view(Hkv, H // Hkv)
-        if not bool((grouped == grouped[:, :1]).all()):
-            raise ValueError("simthreshd1 must be equal for the query heads that share a K/V head "
-                             f"({H} query heads, {Hkv} K/V heads): K is pooled once per K/V head")
+        check_grouped_simthreshd1(simthreshd1, H, Hkv)
     simthreshd1_k = simthreshd1 if Hkv == H else simthreshd1[::H // Hkv].contiguous()
     pool_k, sim_k, k_int8, k_scale = _lib.pool_sim_quant(k, km, BLKK, simthreshd1_k)
     lut, valid, bmap = _lib.block_select(pool_q, sim_q, pool_k, sim_k, topk=topk, cdfthreshd=cdfthreshd,

@@ -1,0 +1,73 @@
+"""The whole operator in one native call (spg_sparse_attn) against the same stages launched one by one: same bits.
+
+The stages are checked against the oracle elsewhere; what can go wrong here is which workgroup does what - chunk and role
+boundaries, the combination of partial sums, workspace offsets, strides, and where the hyper-parameters come from."""
+import pytest
+import torch
+
+import spargeattn_amd as sa
+from spargeattn_amd import core
+from gpu_common import rand_T
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(fn):
+    whole = fn()
+    core._stage_hook = lambda name: None
+    try:
+        staged = fn()
+    finally:
+        core._stage_hook = None
+    return whole, staged
+
+
+def _bits(t):
+    return t.view(torch.int16)
+
+
+# key/value lengths: one block, the edges of a 64- and a 128-row workgroup, one row more than sixteen full chunks of 64,
+# the last length whose partial results every workgroup combines for itself (8192) and the first beyond it
+@pytest.mark.parametrize("Nk", [64, 65, 127, 129, 1025, 8192, 8193])
+@pytest.mark.parametrize("D,dtype,vdtype", [(128, torch.bfloat16, torch.bfloat16), (64, torch.float16, torch.float16),
+                                            (128, torch.float16, torch.bfloat16)])
+def test_one_call_equals_the_stages(Nk, D, dtype, vdtype):
+    B, H, Hkv, N = 2, 4, 2, 257
+    q, k = rand_T((B, H, N, D), dtype, 1), rand_T((B, Hkv, Nk, D), dtype, 2, shift=0.4)
+    v = rand_T((B, Hkv, Nk, D), vdtype, 3)
+    sim = torch.tensor([0.3, 0.3, -0.1, -0.1], device="cuda")
+    level, pv = torch.linspace(0.3, 0.9, H, device="cuda"), torch.tensor([50.0, 3.0, 10.0, 50.0], device="cuda")
+    for fn in (lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.5, return_sparsity=True),
+               lambda: sa.spas_sage2_attn_meansim_cuda(q, k, v, cdfthreshd=level, simthreshd1=sim, pvthreshd=pv, is_causal=True,
+                                                       attention_sink=True, qk_quant_gran=2, return_sparsity=True),
+               lambda: sa.spas_sage_attn_meansim_topk_cuda(q, k, v, topk=level, simthreshd1=0.2, return_sparsity=True),
+               lambda: sa.spas_sage_attn_meansim_cuda(q, k, v, cdfthreshd=0.9, is_causal=Nk == 257, return_sparsity=True)):
+        (o, s), (o2, s2) = _both(fn)
+        assert torch.equal(_bits(o), _bits(o2)) and s == s2
+
+
+@pytest.mark.parametrize("nk", [4, 256, 257, 4097])
+@pytest.mark.parametrize("kind", [torch.bool, torch.int32, torch.bfloat16])
+def test_own_mask_in_one_call(nk, kind):
+    """Mask rows up to 4096 blocks are turned into the LUT beside the quantisation, longer ones in a launch of their own."""
+    H, N, D = 2, 200, 64
+    q, k, v = (rand_T((1, H, n, D), torch.bfloat16, 5 + i) for i, n in enumerate((N, 64 * nk - 3, 64 * nk - 3)))
+    mask = (torch.rand((1, H, 2, nk), generator=torch.Generator().manual_seed(nk)) < 0.3).cuda()
+    mask[..., 0] = True
+    o, o2 = _both(lambda: sa.block_sparse_sage2_attn_cuda(q, k, v, mask_id=mask.to(kind), return_sparsity=True))
+    assert torch.equal(_bits(o[0]), _bits(o2[0])) and o[1] == o2[1]
+
+
+def test_layouts_and_copied_inputs():
+    """(B,N,H,D) tensors, slices of a fused QKV tensor, broadcast heads and float32 inputs give what contiguous copies give,
+    in the memory layout the stages give it; a second call with the same shapes and other data is independent of the first."""
+    B, H, N, D = 1, 3, 300, 64
+    fused = rand_T((B, N, 3, H, D), torch.float16, 9)
+    q, k, v = (fused[:, :, i] for i in range(3))
+    for args in ((q, k, v), (q.contiguous(), k.contiguous(), v.contiguous()), (q.float(), k.float(), v.float()),
+                 (q, k[:, :, :1].expand(B, N, H, D), v)):
+        o, o2 = _both(lambda: sa.spas_sage2_attn_meansim_topk_cuda(*args, topk=0.4, tensor_layout="NHD"))
+        assert o.stride() == o2.stride() and o.dtype == o2.dtype and torch.equal(_bits(o), _bits(o2))
+    other = tuple(t.contiguous() * 0.5 for t in (q, k, v))
+    o, o2 = _both(lambda: sa.spas_sage2_attn_meansim_topk_cuda(*other, topk=0.4, tensor_layout="NHD"))
+    assert torch.equal(_bits(o), _bits(o2))
