@@ -153,6 +153,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   // thresholds in use), and only a wavefront that voted "skip" itself has to read the others' slots.  Two sets of slots,
   // used alternately: a wavefront can be at most one barrier ahead of the slowest one.
   __shared__ int sSkipAt[2][4];
+  __shared__ __align__(16) float sVscale[PV16 ? 4 : D];   // fetched at the start, read in the epilogue
   unsigned char *const sKr = smem;
   unsigned char *const sVr = smem + NBUF * TILE;
   const uint32_t lds_k0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)smem;   // LDS byte address
@@ -167,15 +168,28 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   const int head = bh % p.H;
   // grouped-query attention: H / Hkv consecutive query heads share one K/V head (sm89.cuh:118, head_id / num_kv_groups)
   const int bhk = (bh / p.H) * p.Hkv + head / (p.H / p.Hkv);
-  const int nv = p.valid[(size_t)bh * p.nq + qb];
-  if (nv == 0) return;                                       // output rows stay unwritten (sm89.cuh:232-235)
-  const int32_t *lut_row = p.lut + ((size_t)bh * p.nq + qb) * p.nk;
 
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: everything derived from it stays scalar
   const int N = p.N, Nk = p.Nk;
   const int q_row = qb * 128 + wave * 32 + r;
   if constexpr (!PV16) fp8_saturation_on();
+
+  // Everything whose address follows from the launch arguments is requested before the first wait: the count, the first
+  // four LUT entries (indices clamped to the row, unused ones ignored), the scales, Q.  A chain of dependent scalar loads
+  // costs a short row more than its first block.
+  // LUT and K scales are read through the constant address space: uniform addresses become scalar loads (SMEM),
+  // which never touch the vector-memory counter the tile ring is synchronised with.
+  typedef const __attribute__((address_space(4))) int32_t *c_i32_t;
+  typedef const __attribute__((address_space(4))) float *c_f32_t;
+  const size_t row_id = (size_t)bh * p.nq + qb;
+  const c_i32_t lutc = (c_i32_t)(p.lut + row_id * p.nk);
+  const int last_col = p.nk - 1;
+  const int nv = ((c_i32_t)p.valid)[row_id];
+  const int l0 = lutc[0], l1 = lutc[min(1, last_col)], l2 = lutc[min(2, last_col)], l3 = lutc[min(3, last_col)];
+  // per-warp granularity: the 32 query rows of a wavefront are one quantisation group, so the scale stays a scalar
+  const float qs = ((c_f32_t)p.q_scale)[p.q_per_warp ? row_id * 4 + wave : row_id];
+  const float thr = p.pvthr.p != nullptr ? ((c_f32_t)p.pvthr.p)[head] : p.pvthr.v;
 
   // ---- Q fragment: B operand of S^T = K.Q^T, resident for the whole loop -------------------------------
   v4i qreg[KS];
@@ -184,20 +198,12 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     qreg[ks] = (v4i){0, 0, 0, 0};
     if (q_row < N) qreg[ks] = *(const v4i *)(p.q8 + ((size_t)bh * N + q_row) * D + 32 * ks + 16 * hh);
   }
+  if (nv == 0) return;                                       // output rows stay unwritten (sm89.cuh:232-235)
 
   const int8_t *kbase = p.k8 + (size_t)bhk * Nk * D;
   const uint8_t *vbase = p.v8 + (size_t)bhk * p.nk * (size_t)VTILE;
-  // LUT and K scales are read through the constant address space: uniform addresses become scalar loads (SMEM),
-  // which never touch the vector-memory counter the tile ring is synchronised with.
-  typedef const __attribute__((address_space(4))) int32_t *c_i32_t;
-  typedef const __attribute__((address_space(4))) float *c_f32_t;
-  const c_i32_t lutc = (c_i32_t)(p.lut + ((size_t)bh * p.nq + qb) * p.nk);
   const c_f32_t kscale = (c_f32_t)(p.k_scale + (size_t)bhk * p.nk);
-  // per-warp granularity: the 32 query rows of a wavefront are one quantisation group, so the scale stays a scalar
-  const size_t qsi = (size_t)bh * p.nq + qb;
-  const float qs = ((c_f32_t)p.q_scale)[p.q_per_warp ? qsi * 4 + wave : qsi];
   const float c = p.sm_scale_log2;
-  const float thr = p.pvthr.p != nullptr ? ((c_f32_t)p.pvthr.p)[head] : p.pvthr.v;
 
   // ---- tile loader: wave w copies LDS bytes [1024*(WL*w+u), +1024) of each tile, lane l the 16-byte chunk l ----
   // K: LDS chunk position pos <-> (row = pos / CPR, slot = pos % CPR) holds global chunk slot ^ k_swz(row).
@@ -284,10 +290,10 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
 
   // block ids: blk = block of iteration it, blk1 = it+1, blk2 = it+2 (tiles in flight); d3 = LUT delta of it+3.
   // K scales are fetched one iteration ahead as well.
-  int blk = lutc[0];
-  int blk1 = blk + (nv > 1 ? lutc[1] : 0);
-  int blk2 = blk1 + (nv > 2 ? lutc[2] : 0);
-  int d3 = nv > 3 ? lutc[3] : 0;
+  int blk = l0;
+  int blk1 = blk + (nv > 1 ? l1 : 0);
+  int blk2 = blk1 + (nv > 2 ? l2 : 0);
+  int d3 = nv > 3 ? l3 : 0;
   float ksc = kscale[blk], ksc1 = kscale[blk1];
   if constexpr (PV16) {
     SPG_LOAD_K(blk, 0);
@@ -296,6 +302,10 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   } else {
     SPG_LOAD_TILES(blk, 0);
     if (nv > 1) SPG_LOAD_TILES(blk1, TILE);
+  }
+  if constexpr (!PV16) {
+    if (wave < D / 64)
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(p.v_scale + (size_t)bhk * D + wave * 64 + lane), (lds_ptr_t)(sVscale + wave * 64), 4, 0, 0);
   }
   uint32_t bufoff = 0;                     // LDS ring offset of block it
 
@@ -443,10 +453,17 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     if constexpr (!TAIL) {
       // max over rows of (diff) + thr > 0  <=>  some row has diff + thr > 0 (fp32 addition is monotonic)
       vote = __any(diff + thr > 0.f);
-      if (vote == 0 && lane == 0) sSkipAt[it & 1][wave] = it;
+      if (vote == 0) {                    // wavefront-uniform
+        if (lane == 0) sSkipAt[it & 1][wave] = it;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's share of block it+1's tiles has landed in LDS
-    __syncthreads();   // block it+1's tiles are complete; the votes are visible; ring slot of block it-1 is free
+    // block it+1's tiles are complete; the votes are visible; ring slot of block it-1 is free.  (A bare barrier: the fence
+    // of __syncthreads() would also wait for the scalar loads above.)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     bool compute = true;
     if constexpr (!TAIL) {   // workgroup-uniform in the per-block mode (sm89.cuh:318-353), wavefront-uniform otherwise
       compute = p.pv_mode == 0 || vote != 0;
@@ -638,23 +655,38 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   // ---- epilogue: O / d * v_scale -> out dtype -----------------------------------------------------------
   const float dtot = half_swap_sum_f32(dsum);
   const float inv = __builtin_amdgcn_rcpf(dtot);
-  if (q_row < N) {
-    uint16_t *orow = (uint16_t *)p.out + (size_t)(bh / p.H) * p.os.sb + (size_t)head * p.os.sh + (size_t)q_row * p.os.sn;
-    const float *vs = p.v_scale + (size_t)bhk * D;
+  // A lane holds four channels of one row per group: stored from here, an instruction would touch 32 rows with 16 bytes
+  // each.  The rows of a wavefront go through LDS instead (the tile ring is free once every wavefront is past its last
+  // P.V product) and leave as whole rows, 16 bytes per lane.
+  constexpr int OROW = 2 * D + 16;                           // padded row: the 8-byte writes of 32 rows spread over the banks
+  static_assert(4 * 32 * OROW <= NBUF * (TILE + VTILE), "output rows of four wavefronts fit the tile ring");
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  unsigned char *const orow_lds = smem + wave * (32 * OROW);
 #pragma unroll
-    for (int dt = 0; dt < NDT; dt++) {
+  for (int dt = 0; dt < NDT; dt++) {
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const int d0 = 32 * dt + 8 * g + 4 * hh;
-        float4 sc = make_float4(1.f, 1.f, 1.f, 1.f);
-        if constexpr (!PV16) sc = *(const float4 *)(vs + d0);
-        const uint16_t o0 = f32_to_elem<ODT>(O[dt][4 * g + 0] * inv * sc.x);
-        const uint16_t o1 = f32_to_elem<ODT>(O[dt][4 * g + 1] * inv * sc.y);
-        const uint16_t o2 = f32_to_elem<ODT>(O[dt][4 * g + 2] * inv * sc.z);
-        const uint16_t o3 = f32_to_elem<ODT>(O[dt][4 * g + 3] * inv * sc.w);
-        *(uint2 *)(orow + d0) = make_uint2((uint32_t)o0 | ((uint32_t)o1 << 16), (uint32_t)o2 | ((uint32_t)o3 << 16));
-      }
+    for (int g = 0; g < 4; g++) {
+      const int d0 = 32 * dt + 8 * g + 4 * hh;
+      float4 sc = make_float4(1.f, 1.f, 1.f, 1.f);
+      if constexpr (!PV16) sc = *(const float4 *)(sVscale + d0);
+      const uint16_t o0 = f32_to_elem<ODT>(O[dt][4 * g + 0] * inv * sc.x);
+      const uint16_t o1 = f32_to_elem<ODT>(O[dt][4 * g + 1] * inv * sc.y);
+      const uint16_t o2 = f32_to_elem<ODT>(O[dt][4 * g + 2] * inv * sc.z);
+      const uint16_t o3 = f32_to_elem<ODT>(O[dt][4 * g + 3] * inv * sc.w);
+      *(uint2 *)(orow_lds + r * OROW + d0 * 2) = make_uint2((uint32_t)o0 | ((uint32_t)o1 << 16), (uint32_t)o2 | ((uint32_t)o3 << 16));
     }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  constexpr int LPR = D / 8, RPI = 64 / LPR;                 // lanes per row, rows per store instruction
+  uint16_t *obase = (uint16_t *)p.out + (size_t)(bh / p.H) * p.os.sb + (size_t)head * p.os.sh + (lane % LPR) * 8;
+#pragma unroll
+  for (int i = 0; i < 32 / RPI; i++) {
+    const int row = i * RPI + lane / LPR, grow = qb * 128 + wave * 32 + row;
+    const uint4 t = *(const uint4 *)(orow_lds + row * OROW + (lane % LPR) * 16);
+    if (grow < N) *(uint4 *)(obase + (size_t)grow * p.os.sn) = t;
   }
 }
 
