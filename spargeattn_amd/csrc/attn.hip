@@ -33,6 +33,7 @@
 #include "common.h"
 #include "launch.h"
 #include "lds_asm.h"
+#include "select_row.h"
 
 #include <type_traits>
 
@@ -64,6 +65,7 @@ struct AttnParams {
   int pv_mode;     // PVThresholdMode of the reference (attn_utils.cuh:58-62): 0 none, 1 per block, 2 per wavefront of 32 rows
   int q_per_warp;  // QuantGranularity of Q (sm89.cuh:106-121): 0 one scale per 128-row block, 1 one per 32 rows (B,H,nq*4)
   int total_wg, wg_per_xcd;
+  RowSelect sel;   // selection inside the kernel (template argument SEL); lut is unused then
 };
 
 // v_max_f32 as one instruction: fmaxf() on a value the compiler cannot prove to be a quiet number (a loop-carried
@@ -133,7 +135,10 @@ __device__ __forceinline__ int v_swz(int row) { return (row >> 2) & 3; }
 //               sum on the tensor cores computes, qk_int_sv_f16_cuda_sm80.cuh:339-368, attn_utils.cuh:599-626).  The PV product is
 //               accumulated in fp32; the reference accumulates each 64-key block in fp16 before adding it to its fp32
 //               accumulator (attn_utils.cuh:683-751), a rounding this kernel does not reproduce.
-template <int D, int ODT, bool PV16>
+// SEL: rows of at most 64 blocks are selected here, by the workgroup that then works on them, instead of by a kernel in
+// front that writes a LUT: the row's map is one 64-bit scalar, and the next block is its next set bit.  Takes a launch
+// (about 4.5 us) and the selection kernel's 7-15 us out of the chain and puts about 3 us in.
+template <int D, int ODT, bool PV16, bool SEL>
 __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnParams p) {
   constexpr int KS = D / 32;        // k-steps of the int8 MFMA
   constexpr int NDT = D / 32;       // 32-channel output tiles
@@ -183,10 +188,13 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   typedef const __attribute__((address_space(4))) int32_t *c_i32_t;
   typedef const __attribute__((address_space(4))) float *c_f32_t;
   const size_t row_id = (size_t)bh * p.nq + qb;
-  const c_i32_t lutc = (c_i32_t)(p.lut + row_id * p.nk);
+  const c_i32_t lutc = (c_i32_t)(p.lut + (SEL ? 0 : row_id * p.nk));
   const int last_col = p.nk - 1;
-  const int nv = ((c_i32_t)p.valid)[row_id];
-  const int l0 = lutc[0], l1 = lutc[min(1, last_col)], l2 = lutc[min(2, last_col)], l3 = lutc[min(3, last_col)];
+  int nv, l0, l1, l2, l3;
+  if constexpr (!SEL) {
+    nv = ((c_i32_t)p.valid)[row_id];
+    l0 = lutc[0]; l1 = lutc[min(1, last_col)]; l2 = lutc[min(2, last_col)]; l3 = lutc[min(3, last_col)];
+  }
   // per-warp granularity: the 32 query rows of a wavefront are one quantisation group, so the scale stays a scalar
   const float qs = ((c_f32_t)p.q_scale)[p.q_per_warp ? row_id * 4 + wave : row_id];
   const float thr = p.pvthr.p != nullptr ? ((c_f32_t)p.pvthr.p)[head] : p.pvthr.v;
@@ -198,6 +206,28 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     qreg[ks] = (v4i){0, 0, 0, 0};
     if (q_row < N) qreg[ks] = *(const v4i *)(p.q8 + ((size_t)bh * N + q_row) * D + 32 * ks + 16 * hh);
   }
+  uint64_t map = 0;                        // SEL: blocks not fetched yet
+  if constexpr (SEL) {
+    __shared__ uint16_t sScore[64];
+    const uint8_t *simk = p.sel.sim_k + (size_t)bhk * p.nk;
+    const bool row_forced = p.sel.sim_q[row_id] == 0;
+    const bool k_dead = simk[min(lane, last_col)] == 0;
+    const int col = tid >> 2;
+    const uint16_t s16 = pooled_score_4lanes<D, ODT>(p.sel.pool_q + row_id * D, p.sel.pool_k + ((size_t)bhk * p.nk + min(col, last_col)) * D, tid & 3);
+    if ((tid & 3) == 0) sScore[col] = s16;
+    __syncthreads();
+    const int causal_lim = p.sel.is_causal ? min(p.nk, 2 * (qb + 1)) : p.nk;
+    const float sc = (lane >= causal_lim || k_dead) ? -INFINITY : elem_to_f32<ODT>(sScore[lane]);
+    map = select_row64<ODT>(sc, k_dead, p.sel.by_topk, p.sel.level.at(head), p.nk, causal_lim, row_forced, p.sel.sink, lane);
+    nv = __builtin_popcountll(map);
+    if (p.sel.valid_out != nullptr && tid == 0) p.sel.valid_out[row_id] = nv;
+  }
+  // SEL: takes the next block out of the map; beyond the last one it repeats `prev`
+  auto next_block = [&](int prev) __attribute__((always_inline)) {
+    const int b = map != 0 ? __builtin_ctzll(map) : prev;
+    map &= map - 1;
+    return b;
+  };
   if (nv == 0) return;                                       // output rows stay unwritten (sm89.cuh:232-235)
 
   const int8_t *kbase = p.k8 + (size_t)bhk * Nk * D;
@@ -290,10 +320,17 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
 
   // block ids: blk = block of iteration it, blk1 = it+1, blk2 = it+2 (tiles in flight); d3 = LUT delta of it+3.
   // K scales are fetched one iteration ahead as well.
-  int blk = l0;
-  int blk1 = blk + (nv > 1 ? l1 : 0);
-  int blk2 = blk1 + (nv > 2 ? l2 : 0);
-  int d3 = nv > 3 ? l3 : 0;
+  int blk, blk1, blk2, d3 = 0;
+  if constexpr (SEL) {
+    blk = next_block(0);
+    blk1 = next_block(blk);
+    blk2 = next_block(blk1);
+  } else {
+    blk = l0;
+    blk1 = blk + (nv > 1 ? l1 : 0);
+    blk2 = blk1 + (nv > 2 ? l2 : 0);
+    d3 = nv > 3 ? l3 : 0;
+  }
   float ksc = kscale[blk], ksc1 = kscale[blk1];
   if constexpr (PV16) {
     SPG_LOAD_K(blk, 0);
@@ -398,7 +435,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     int d4 = 0;
     if constexpr (!TAIL) {
       ksc2 = kscale[blk2];
-      d4 = it + 4 < nv ? lutc[it + 4] : 0;
+      if constexpr (!SEL) d4 = it + 4 < nv ? lutc[it + 4] : 0;
     }
     __builtin_amdgcn_sched_barrier(0);
     const float dq = qs * ksc;                     // used by the tail blocks only
@@ -622,7 +659,9 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
       }   // !PV16
     }
     // advance the block pipeline and the ring
-    blk = blk1; blk1 = blk2; blk2 = blk2 + d3; d3 = d4;
+    blk = blk1; blk1 = blk2;
+    if constexpr (SEL) blk2 = next_block(blk2);
+    else { blk2 = blk2 + d3; d3 = d4; }
     ksc = ksc1; ksc1 = ksc2;
     if constexpr (!CS) bufoff = bufoff == (NBUF - 1) * TILE ? 0 : bufoff + TILE;
   };
@@ -690,40 +729,48 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   }
 }
 
+template <bool SEL>
+static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, hipStream_t st) {
+  p.nq = (p.N + 127) / 128; p.nk = (p.Nk + 63) / 64;
+  p.total_wg = p.nq * p.H * p.B;
+  p.wg_per_xcd = (p.total_wg + 7) / 8;
+  const int grid = p.wg_per_xcd * 8;
+  if (p.v_scale != nullptr) {
+    if (D == 64) {
+      if (out_dtype == 0) block_sparse_attn_kernel<64, 0, false, SEL><<<grid, 256, 0, st>>>(p);
+      else block_sparse_attn_kernel<64, 1, false, SEL><<<grid, 256, 0, st>>>(p);
+    } else {
+      if (out_dtype == 0) block_sparse_attn_kernel<128, 0, false, SEL><<<grid, 256, 0, st>>>(p);
+      else block_sparse_attn_kernel<128, 1, false, SEL><<<grid, 256, 0, st>>>(p);
+    }
+  } else {   // fp16 V^T tiles, no V scale
+    if (D == 64) {
+      if (out_dtype == 0) block_sparse_attn_kernel<64, 0, true, SEL><<<grid, 256, 0, st>>>(p);
+      else block_sparse_attn_kernel<64, 1, true, SEL><<<grid, 256, 0, st>>>(p);
+    } else {
+      if (out_dtype == 0) block_sparse_attn_kernel<128, 0, true, SEL><<<grid, 256, 0, st>>>(p);
+      else block_sparse_attn_kernel<128, 1, true, SEL><<<grid, 256, 0, st>>>(p);
+    }
+  }
+  return hipGetLastError();
+}
+
 hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
-                                      int out_dtype, const int32_t *lut, const int32_t *valid, Hyper pvthreshd,
-                                      const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
-                                      int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
-                                      int pv_mode, int32_t *pv_count, hipStream_t st) {
-  AttnParams p;
+                                      int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel,
+                                      Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
+                                      int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
+                                      int q_per_warp, int pv_mode, int32_t *pv_count, hipStream_t st) {
+  AttnParams p = {};
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.out = out; p.os = os; p.lut = lut; p.valid = valid; p.pvthr = pvthreshd;
   p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.pv_count = pv_count;
-  p.B = B; p.H = H; p.Hkv = Hkv; p.N = N; p.Nk = Nk; p.nq = (N + 127) / 128; p.nk = (Nk + 63) / 64;
+  p.B = B; p.H = H; p.Hkv = Hkv; p.N = N; p.Nk = Nk;
   p.sm_scale_log2 = sm_scale * SPG_LOG2E;
   p.is_causal = is_causal;
   p.pv_mode = pv_mode;
   p.q_per_warp = q_per_warp;
-  p.total_wg = p.nq * H * B;
-  p.wg_per_xcd = (p.total_wg + 7) / 8;
-  const int grid = p.wg_per_xcd * 8;
-  if (v_scale != nullptr) {
-    if (D == 64) {
-      if (out_dtype == 0) block_sparse_attn_kernel<64, 0, false><<<grid, 256, 0, st>>>(p);
-      else block_sparse_attn_kernel<64, 1, false><<<grid, 256, 0, st>>>(p);
-    } else {
-      if (out_dtype == 0) block_sparse_attn_kernel<128, 0, false><<<grid, 256, 0, st>>>(p);
-      else block_sparse_attn_kernel<128, 1, false><<<grid, 256, 0, st>>>(p);
-    }
-  } else {   // fp16 V^T tiles, no V scale
-    if (D == 64) {
-      if (out_dtype == 0) block_sparse_attn_kernel<64, 0, true><<<grid, 256, 0, st>>>(p);
-      else block_sparse_attn_kernel<64, 1, true><<<grid, 256, 0, st>>>(p);
-    } else {
-      if (out_dtype == 0) block_sparse_attn_kernel<128, 0, true><<<grid, 256, 0, st>>>(p);
-      else block_sparse_attn_kernel<128, 1, true><<<grid, 256, 0, st>>>(p);
-    }
-  }
-  return hipGetLastError();
+  if (sel == nullptr) return launch_attn<false>(p, D, out_dtype, st);
+  p.sel = *sel;
+  return launch_attn<true>(p, D, out_dtype, st);
 }
 
 hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
@@ -731,8 +778,8 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st) {
-  return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, Hyper{pvthreshd, 0.f}, q_scale, k_scale, v_scale, B,
-                                    H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, st);
+  return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, nullptr, Hyper{pvthreshd, 0.f}, q_scale, k_scale,
+                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, st);
 }
 
 }  // namespace spg

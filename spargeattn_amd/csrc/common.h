@@ -59,6 +59,23 @@ template <> __device__ __forceinline__ uint16_t f32_to_elem<1>(float x) {
   return __builtin_bit_cast(uint16_t, (__bf16)x);   // v_cvt_pk_bf16_f32: round to nearest even in hardware
 }
 
+// binary64 -> 16-bit pattern (round to nearest even) through binary32 where that provably gives the same bits: the
+// first rounding (to 24 bits) can only change the second one when it lands exactly on a rounding tie of the 16-bit
+// format, so every other value inside the format's normal range takes two hardware conversions instead of the 64-bit
+// integer arithmetic of f64_to_elem; ties, zero-range, subnormal and overflowing values go the exact way.
+template <int DT>
+__device__ __forceinline__ uint16_t f64_to_elem_fast(double x) {
+  const float r = (float)x;                                        // v_cvt_f32_f64
+  const uint32_t b = __builtin_bit_cast(uint32_t, r);
+  const uint32_t mag = b & 0x7fffffffu;
+  constexpr uint32_t DROP = DT == 1 ? 16u : 13u;                   // binary32 mantissa bits the 16-bit format drops
+  constexpr uint32_t LOW = (1u << DROP) - 1u, TIE = 1u << (DROP - 1u);
+  constexpr uint32_t LO = DT == 1 ? 0x00800000u : 0x38800000u;     // 2^-126 / 2^-14: smallest normal of the format
+  constexpr uint32_t HI = DT == 1 ? 0x7f000000u : 0x47000000u;     // 2^127 / 2^15: well below the overflow threshold
+  const bool safe = mag == 0u || (mag >= LO && mag < HI && (b & LOW) != TIE);
+  return safe ? f32_to_elem<DT>(r) : f64_to_elem<DT>(x);
+}
+
 // Round two binary32 values to the 16-bit element type and widen them again (one packed conversion for bfloat16).
 template <int DT> __device__ __forceinline__ void round2_through_elem(float &a, float &b);
 template <> __device__ __forceinline__ void round2_through_elem<0>(float &a, float &b) {

@@ -1,5 +1,5 @@
 // The whole operator behind one call: K mean, mask prediction + INT8 quantisation, V quantisation, block-sparse
-// attention, as four launches (three for a mask of the caller's own) on workspace the caller hands over.
+// attention, as three or four launches on workspace the caller hands over.
 //
 // Short sequences are bound by the length of the launch chain and by kernels that cannot fill the chip, so stages that do
 // not depend on each other share a launch; which stage a workgroup belongs to follows from its number:
@@ -8,7 +8,7 @@
 //   (final   column mean of K, channel maxima of V: only where there are too many partial results for every workgroup
 //            of the next launch to add them up for itself)
 //   back     pooling + quantisation of K | V -> e4m3 tiles and scales
-//   select   block_select_* of maskpred.hip
+//   select   block_select_* of maskpred.hip (rows of more than 64 blocks; shorter ones are selected inside the next launch)
 //   attn     block_sparse_attn_kernel
 // Every body is the one the stage-by-stage entry points launch (stage_bodies.h): results are the same bits.
 // Compile with -ffp-contract=off.
@@ -293,13 +293,19 @@ static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const S
   else e = a->qk_dtype == 0 ? run_front_back<128, 0>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st)
                             : run_front_back<128, 1>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);
   if (e != hipSuccess) return e;
-  if (pool)
+  const bool sel_in_attn = pool && nk <= SPG_SELECT_IN_ATTN_NK;
+  RowSelect sel = {};
+  if (sel_in_attn)
+    sel = {f.pool_q, b.pool_k, f.sim_q, b.sim_k, Hyper{a->level, a->level_value}, a->selection == SPG_SELECT_TOPK, a->is_causal,
+           a->attention_sink, a->valid_block_num};
+  else if (pool)
     e = launch_block_select_h(f.pool_q, f.sim_q, b.pool_k, b.sim_k, a->selection == SPG_SELECT_TOPK, Hyper{a->level, a->level_value},
                               a->is_causal, a->attention_sink, lut, valid, nullptr, a->B, a->H, a->Hkv, nq, nk, a->D, a->qk_dtype, st);
   else if (!mask_in_front)
     e = launch_map_to_lut(a->mask, a->mask_kind, lut, valid, a->B, a->H, nq, nk, st);
   if (e != hipSuccess) return e;
-  return launch_block_sparse_attn_h(f.q8, b.k8, b.v8, a->out, os, a->qk_dtype, lut, valid, Hyper{a->pvthreshd, a->pvthreshd_value},
+  return launch_block_sparse_attn_h(f.q8, b.k8, b.v8, a->out, os, a->qk_dtype, lut, valid, sel_in_attn ? &sel : nullptr,
+                                    Hyper{a->pvthreshd, a->pvthreshd_value},
                                     f.q_scale, b.k_scale, a->pv_f16 ? nullptr : b.v_scale, a->B, a->H, a->Hkv, a->N, a->N_kv, a->D,
                                     a->sm_scale, a->kernel_causal ? 1 : 0, a->qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0,
                                     SPG_PV_PER_BLOCK, nullptr, st);

@@ -55,11 +55,22 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st);
+// What the attention kernel needs to select a row's blocks by itself (rows of at most SPG_SELECT_IN_ATTN_NK blocks):
+// the arguments of launch_block_select_h
+#define SPG_SELECT_IN_ATTN_NK 64
+struct RowSelect {
+  const uint16_t *pool_q, *pool_k;
+  const uint8_t *sim_q, *sim_k;
+  Hyper level;
+  int by_topk, is_causal, sink;
+  int32_t *valid_out;               // counts for the caller, or NULL
+};
+// sel == NULL: blocks come from lut / valid; otherwise they are selected in place and lut / valid are not read
 hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
-                                      int out_dtype, const int32_t *lut, const int32_t *valid, Hyper pvthreshd,
-                                      const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
-                                      int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
-                                      int pv_mode, int32_t *pv_count, hipStream_t st);
+                                      int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel,
+                                      Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
+                                      int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
+                                      int q_per_warp, int pv_mode, int32_t *pv_count, hipStream_t st);
 void launch_fp8_pack_selftest(const float *x, uint8_t *codes, int n, int saturate, hipStream_t st);
 
 hipError_t launch_dense_attn_f16(const void *q, const void *k, const void *v, void *out, int B, int H, int N, int D,

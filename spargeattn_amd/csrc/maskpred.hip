@@ -16,6 +16,7 @@
 // (round-to-nearest-even, straight from binary64); fp32 quantisation steps use IEEE divide / sqrt; the
 // compressed softmax uses a fixed binary64 operation sequence and a fixed summation tree.  This file must be
 // compiled with -ffp-contract=off.
+#include "select_row.h"
 #include "stage_bodies.h"
 
 #include <atomic>
@@ -91,30 +92,6 @@ __global__ __launch_bounds__(256) void pool_sim_quant_kernel(const uint16_t *__r
   if constexpr (WITH_POOL) thr = simthr[blockIdx.y % H];
   psq_body<BS, D, DT, HAS_MEAN ? MEAN_GIVEN : MEAN_NONE, WITH_POOL, QR>(x, xs, km, nullptr, 0, pool, sim, xq, scale, thr, H, N, nb,
                                                                         blockIdx.x, blockIdx.y, smem);
-}
-
-// =============================================================================================
-// canonical exp: a fixed sequence of binary64 mul / add (no fma), t <= 0.
-// =============================================================================================
-__device__ __forceinline__ double cexp(double t) {
-  if (!(t >= -700.0)) return 0.0;
-  const double k = __builtin_rint(t * 1.4426950408889634);
-  const double r = (t - k * 0.6931471803691238) - k * 1.9082149292705877e-10;
-  double p = 1.0 / 6227020800.0;
-  p = p * r; p = p + 1.0 / 479001600.0;
-  p = p * r; p = p + 1.0 / 39916800.0;
-  p = p * r; p = p + 1.0 / 3628800.0;
-  p = p * r; p = p + 1.0 / 362880.0;
-  p = p * r; p = p + 1.0 / 40320.0;
-  p = p * r; p = p + 1.0 / 5040.0;
-  p = p * r; p = p + 1.0 / 720.0;
-  p = p * r; p = p + 1.0 / 120.0;
-  p = p * r; p = p + 1.0 / 24.0;
-  p = p * r; p = p + 1.0 / 6.0;
-  p = p * r; p = p + 1.0 / 2.0;
-  p = p * r; p = p + 1.0;
-  p = p * r; p = p + 1.0;
-  return __builtin_ldexp(p, (int)k);
 }
 
 // =============================================================================================
@@ -304,51 +281,6 @@ __global__ __launch_bounds__(256) void block_select_kernel(
 // whose short-distance steps are register-local and whose long-distance steps are lane exchanges.
 // dynamic LDS: 16*nkp*2 (scores) + 4*nkp*4 (per-wave index list) + 4*64*8 (lane sums).
 // =============================================================================================
-template <int EPL, int K, int J>
-__device__ __forceinline__ void bitonic_step(uint32_t (&key)[EPL], int lane) {
-  constexpr int NKP = 64 * EPL;
-  // element v = lane * EPL + t; a step compares v with v ^ J inside blocks of size K (descending where (v & K) == 0)
-  if constexpr (J >= EPL) {
-    constexpr int DL = J / EPL;                                     // partner lane = lane ^ DL
-    const bool lower = (lane & DL) == 0;
-    const bool desc = (K >= NKP) ? true : ((lane & (K / EPL)) == 0);
-    const bool want_max = lower == desc;
-#pragma unroll
-    for (int t = 0; t < EPL; t++) {
-      const uint32_t o = (uint32_t)__shfl_xor((int)key[t], DL, SPG_WAVE);
-      const uint32_t mx = key[t] > o ? key[t] : o, mn = key[t] > o ? o : key[t];
-      key[t] = want_max ? mx : mn;
-    }
-  } else {
-#pragma unroll
-    for (int t = 0; t < EPL; t++) {
-      if ((t & J) == 0) {
-        const uint32_t a = key[t], b = key[t | J];
-        const uint32_t mx = a > b ? a : b, mn = a > b ? b : a;
-        if constexpr (K < EPL) {
-          const bool desc = (t & K) == 0;                           // compile-time
-          key[t] = desc ? mx : mn;
-          key[t | J] = desc ? mn : mx;
-        } else {
-          const bool desc = (K >= NKP) ? true : ((lane & (K / EPL)) == 0);
-          key[t] = desc ? mx : mn;
-          key[t | J] = desc ? mn : mx;
-        }
-      }
-    }
-  }
-}
-template <int EPL, int K, int J>
-__device__ __forceinline__ void bitonic_inner(uint32_t (&key)[EPL], int lane) {
-  bitonic_step<EPL, K, J>(key, lane);
-  if constexpr (J > 1) bitonic_inner<EPL, K, J / 2>(key, lane);
-}
-template <int EPL, int K>
-__device__ __forceinline__ void bitonic_sort_desc(uint32_t (&key)[EPL], int lane) {
-  bitonic_inner<EPL, K, K / 2>(key, lane);
-  if constexpr (K < 64 * EPL) bitonic_sort_desc<EPL, K * 2>(key, lane);
-}
-
 template <int D, int DT, int NW, int EPL, bool DUAL>
 __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_select_wave_kernel(
     const uint16_t *__restrict__ pool_q, const uint8_t *__restrict__ sim_q, const uint16_t *__restrict__ pool_k,

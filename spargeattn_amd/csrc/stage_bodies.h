@@ -68,23 +68,6 @@ __device__ __forceinline__ float div_by(float a, float b, float r) {
 }
 __device__ __forceinline__ bool rcp_safe(float b) { return b >= 0x1p-60f && b <= 0x1p60f; }
 
-// binary64 -> 16-bit pattern (round to nearest even) through binary32 where that provably gives the same bits: the
-// first rounding (to 24 bits) can only change the second one when it lands exactly on a rounding tie of the 16-bit
-// format, so every other value inside the format's normal range takes two hardware conversions instead of the 64-bit
-// integer arithmetic of f64_to_elem; ties, zero-range, subnormal and overflowing values go the exact way.
-template <int DT>
-__device__ __forceinline__ uint16_t f64_to_elem_fast(double x) {
-  const float r = (float)x;                                        // v_cvt_f32_f64
-  const uint32_t b = __builtin_bit_cast(uint32_t, r);
-  const uint32_t mag = b & 0x7fffffffu;
-  constexpr uint32_t DROP = DT == 1 ? 16u : 13u;                   // binary32 mantissa bits the 16-bit format drops
-  constexpr uint32_t LOW = (1u << DROP) - 1u, TIE = 1u << (DROP - 1u);
-  constexpr uint32_t LO = DT == 1 ? 0x00800000u : 0x38800000u;     // 2^-126 / 2^-14: smallest normal of the format
-  constexpr uint32_t HI = DT == 1 ? 0x7f000000u : 0x47000000u;     // 2^127 / 2^15: well below the overflow threshold
-  const bool safe = mag == 0u || (mag >= LO && mag < HI && (b & LOW) != TIE);
-  return safe ? f32_to_elem<DT>(r) : f64_to_elem<DT>(x);
-}
-
 // Packed 16-bit helpers.  A tile is kept in registers as the 16-bit patterns it was loaded with (two per register) and
 // widened where it is used: half the registers of a binary32 copy, which is what lets enough workgroups share a CU to
 // keep HBM busy.

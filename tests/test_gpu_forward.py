@@ -26,9 +26,26 @@ def _bits(t):
     return t.view(torch.int16)
 
 
+@pytest.mark.parametrize("Nk", [300, 4096])
+def test_ties_and_extreme_levels_in_place(Nk):
+    """Equal probabilities (the lower column wins), levels that keep one block, all of them, or nothing but dissimilar ones."""
+    q = rand_T((1, 2, 256, 64), torch.float16, 1)
+    k = rand_T((1, 2, 1, 64), torch.float16, 2).expand(1, 2, Nk, 64).contiguous()
+    k[:, :, 130:200] = rand_T((1, 2, 70, 64), torch.float16, 4)
+    v = rand_T((1, 2, Nk, 64), torch.float16, 3)
+    for kw in (dict(topk=0.0), dict(topk=1.0), dict(topk=0.5), dict(topk=0.37, is_causal=True), dict(topk=5.0),
+               dict(topk=0.2, simthreshd1=0.9)):
+        (o, s), (o2, s2) = _both(lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, return_sparsity=True, **kw))
+        assert torch.equal(_bits(o), _bits(o2)) and s == s2, kw
+    for cdf in (0.0, 0.5, 1.0):
+        (o, s), (o2, s2) = _both(lambda: sa.spas_sage2_attn_meansim_cuda(q, k, v, cdfthreshd=cdf, simthreshd1=0.5, return_sparsity=True))
+        assert torch.equal(_bits(o), _bits(o2)) and s == s2, cdf
+
+
 # key/value lengths: one block, the edges of a 64- and a 128-row workgroup, one row more than sixteen full chunks of 64,
-# the last length whose partial results every workgroup combines for itself (8192) and the first beyond it
-@pytest.mark.parametrize("Nk", [64, 65, 127, 129, 1025, 8192, 8193])
+# the last length whose rows the attention kernel selects by itself (4096) and the first beyond it, the last whose partial
+# results every workgroup combines for itself (8192) and the first beyond it
+@pytest.mark.parametrize("Nk", [64, 65, 127, 129, 1025, 4096, 4097, 8192, 8193])
 @pytest.mark.parametrize("D,dtype,vdtype", [(128, torch.bfloat16, torch.bfloat16), (64, torch.float16, torch.float16),
                                             (128, torch.float16, torch.bfloat16)])
 def test_one_call_equals_the_stages(Nk, D, dtype, vdtype):
