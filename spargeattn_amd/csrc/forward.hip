@@ -41,39 +41,39 @@ struct FrontParams {
 };
 
 template <int A, int B> constexpr int max_c() { return A > B ? A : B; }
-template <int D, bool POOL> constexpr int front_lds() {
-  return max_c<max_c<km_partial_lds<D>(), v_tiles_f16_lds<D>()>(), max_c<POOL ? psq_lds<128, D>() : 16, POOL ? 16 : 4 * MASK_NKP_FRONT + 16>()>();
+template <int D, bool POOL, int NT> constexpr int front_lds() {
+  return max_c<max_c<km_partial_lds<D, NT>(), v_tiles_f16_lds<D>()>(), max_c<POOL ? psq_lds<128, D, NT>() : 16, POOL ? 16 : 4 * MASK_NKP_FRONT + 64>()>();
 }
 
-template <int D, int DT, bool POOL, int QR>
-__global__ __launch_bounds__(256) void front_kernel(const FrontParams p) {
-  __shared__ __align__(16) unsigned char smem[front_lds<D, POOL>()];
+template <int D, int DT, bool POOL, int QR, int NT>
+__global__ __launch_bounds__(NT) void front_kernel(const FrontParams p) {
+  __shared__ __align__(16) unsigned char smem[front_lds<D, POOL, NT>()];
   const int w = blockIdx.x;
   if (w >= p.wg_q) {
     const int id = w - p.wg_q, bh = id / p.nq;
     float thr = 0.f;
     if constexpr (POOL) thr = p.simthr.at(bh % p.H);
-    psq_body<128, D, DT, MEAN_NONE, POOL, QR>(p.q, p.qs, nullptr, nullptr, 0, p.pool_q, p.sim_q, p.q8, p.q_scale, thr, p.H, p.N, p.nq,
+    psq_body<128, D, DT, MEAN_NONE, POOL, QR, NT>(p.q, p.qs, nullptr, nullptr, 0, p.pool_q, p.sim_q, p.q8, p.q_scale, thr, p.H, p.N, p.nq,
                                               id - bh * p.nq, bh, smem);
   } else if (w < p.wg_v) {
     const int bh = w / p.k_chunks;
-    km_partial_body<D, DT>(p.k, p.ks, p.Hkv, p.km_part, p.Nk, p.k_rows, w - bh * p.k_chunks, p.k_chunks, bh, smem);
+    km_partial_body<D, DT, NT>(p.k, p.ks, p.Hkv, p.km_part, p.Nk, p.k_rows, w - bh * p.k_chunks, p.k_chunks, bh, smem);
   } else if (w < p.wg_mask) {
     const int id = w - p.wg_v;
     if (p.v_f16) {
       const int bh = id / p.nk;
-      if (p.v_dtype == 0) v_tiles_f16_body<D, 0>(p.v, p.vs, p.Hkv, p.v_tiles, p.Nk, p.nk, id - bh * p.nk, bh, smem);
-      else v_tiles_f16_body<D, 1>(p.v, p.vs, p.Hkv, p.v_tiles, p.Nk, p.nk, id - bh * p.nk, bh, smem);
+      if (p.v_dtype == 0) v_tiles_f16_body<D, 0, NT>(p.v, p.vs, p.Hkv, p.v_tiles, p.Nk, p.nk, id - bh * p.nk, bh, smem);
+      else v_tiles_f16_body<D, 1, NT>(p.v, p.vs, p.Hkv, p.v_tiles, p.Nk, p.nk, id - bh * p.nk, bh, smem);
     } else {
       const int bh = id / p.v_chunks;
       float *dst = p.v_part + (size_t)id * D;
       auto store = [&](int d, float s) { dst[d] = s; };
-      if (p.v_dtype == 0) v_absmax_body<D, 0>(p.v, p.vs, p.Hkv, p.Nk, p.v_rows, id - bh * p.v_chunks, bh, smem, store);
-      else v_absmax_body<D, 1>(p.v, p.vs, p.Hkv, p.Nk, p.v_rows, id - bh * p.v_chunks, bh, smem, store);
+      if (p.v_dtype == 0) v_absmax_body<D, 0, NT>(p.v, p.vs, p.Hkv, p.Nk, p.v_rows, id - bh * p.v_chunks, bh, smem, store);
+      else v_absmax_body<D, 1, NT>(p.v, p.vs, p.Hkv, p.Nk, p.v_rows, id - bh * p.v_chunks, bh, smem, store);
     }
   } else if constexpr (!POOL) {
     const size_t row = (size_t)(w - p.wg_mask);
-#define SPG_M2L(K_) case K_: map_to_lut_body<K_>(p.mask, p.lut, p.valid, p.nk, p.nkp, row, smem); break;
+#define SPG_M2L(K_) case K_: map_to_lut_body<K_, NT>(p.mask, p.lut, p.valid, p.nk, p.nkp, row, smem); break;
     switch (p.mask_kind) { SPG_M2L(0) SPG_M2L(1) SPG_M2L(2) SPG_M2L(3) SPG_M2L(4) SPG_M2L(5) SPG_M2L(6) }
 #undef SPG_M2L
   }
@@ -110,6 +110,9 @@ __global__ void final_kernel(const FinalParams p) {
   }
 }
 
+// rows of K per workgroup of the back kernel
+constexpr int k_rows_per_wg(int nt) { return nt == 256 ? 128 : 64; }
+
 struct BackParams {
   const uint16_t *k, *v;
   Strides ks, vs;
@@ -132,17 +135,18 @@ struct BackParams {
 };
 
 // PARTIAL: the partial results of the front kernel are combined here, by every workgroup for the head it works on
-template <int D, int DT, bool POOL, bool PARTIAL>
-__global__ __launch_bounds__(256) void back_kernel(const BackParams p) {
-  constexpr int LK = POOL ? psq_lds<64, D>() : 256 * 8 + 2 * D;
-  constexpr int LV = v_quant_lds<D>() + 1024 + 4 * D;
+template <int D, int DT, bool POOL, bool PARTIAL, int NT>
+__global__ __launch_bounds__(NT) void back_kernel(const BackParams p) {
+  constexpr int ROWS = k_rows_per_wg(NT);
+  constexpr int LK = max_c<POOL ? psq_lds<64, D, NT, ROWS>() : 16, NT * 8 + 2 * D>();
+  constexpr int LV = v_quant_lds<D>() + 4 * NT + 4 * D;
   __shared__ __align__(16) unsigned char smem[max_c<LK, LV>()];
   const int w = blockIdx.x;
   if (w < p.wg_v) {
     const int bh = w / p.k_wgs_per_head;
     float thr = 0.f;
     if constexpr (POOL) thr = p.simthr.at((bh % p.Hkv) * (p.H / p.Hkv));
-    psq_body<64, D, DT, PARTIAL ? MEAN_PARTIAL : MEAN_GIVEN, POOL>(p.k, p.ks, p.km, p.km_part, p.k_chunks, p.pool_k, p.sim_k, p.k8,
+    psq_body<64, D, DT, PARTIAL ? MEAN_PARTIAL : MEAN_GIVEN, POOL, 64, NT, ROWS>(p.k, p.ks, p.km, p.km_part, p.k_chunks, p.pool_k, p.sim_k, p.k8,
                                                                   p.k_scale, thr, p.Hkv, p.Nk, p.nk, w - bh * p.k_wgs_per_head, bh, smem);
   } else {
     const int id = w - p.wg_v, bh = id / p.nk, blk = id - bh * p.nk;
@@ -152,12 +156,12 @@ __global__ __launch_bounds__(256) void back_kernel(const BackParams p) {
     if constexpr (PARTIAL) {
       float m = 0.f;
 #pragma unroll 4
-      for (int i = tid / D; i < p.v_chunks; i += 256 / D) m = fmaxf(m, p.v_part[((size_t)bh * p.v_chunks + i) * D + tid % D]);
+      for (int i = tid / D; i < p.v_chunks; i += NT / D) m = fmaxf(m, p.v_part[((size_t)bh * p.v_chunks + i) * D + tid % D]);
       s_sub[tid] = m;
       __syncthreads();
       if (tid < D) {
 #pragma unroll
-        for (int u = 1; u < 256 / D; u++) m = fmaxf(m, s_sub[tid + u * D]);
+        for (int u = 1; u < NT / D; u++) m = fmaxf(m, s_sub[tid + u * D]);
         s_amax[tid] = m;
       }
     } else if (tid < D) {
@@ -166,8 +170,8 @@ __global__ __launch_bounds__(256) void back_kernel(const BackParams p) {
     __syncthreads();
     if (blk == 0 && tid < D) p.v_scale[(size_t)bh * D + tid] = s_amax[tid] / 2.25f;
     auto amax_of = [&](int d) { return s_amax[d]; };
-    if (p.v_dtype == 0) v_quant_body<D, 0>(p.v, p.vs, p.Hkv, p.v8, p.Nk, p.nk, blk, bh, smem, amax_of);
-    else v_quant_body<D, 1>(p.v, p.vs, p.Hkv, p.v8, p.Nk, p.nk, blk, bh, smem, amax_of);
+    if (p.v_dtype == 0) v_quant_body<D, 0, NT>(p.v, p.vs, p.Hkv, p.v8, p.Nk, p.nk, blk, bh, smem, amax_of);
+    else v_quant_body<D, 1, NT>(p.v, p.vs, p.Hkv, p.v8, p.Nk, p.nk, blk, bh, smem, amax_of);
   }
 }
 
@@ -221,27 +225,30 @@ static Layout layout_for(const spg_attn_args *a) {
   return l;
 }
 
-template <int D, int DT>
-static hipError_t run_front_back(const spg_attn_args *a, FrontParams &f, BackParams &b, const Chunks &c, uint16_t *km, float *v_amax,
-                                 int front_wgs, int back_wgs, hipStream_t st) {
+template <int D, int DT, int NT>
+static void run_front_back(const spg_attn_args *a, const FrontParams &f, const BackParams &b, const Chunks &c, uint16_t *km, float *v_amax,
+                           int front_wgs, int back_wgs, hipStream_t st) {
   const bool pool = a->selection != SPG_SELECT_MASK, per_warp = a->qk_quant_gran == SPG_QUANT_PER_WARP;
-  if (pool) {
-    if (per_warp) front_kernel<D, DT, true, 32><<<front_wgs, 256, 0, st>>>(f);
-    else front_kernel<D, DT, true, 128><<<front_wgs, 256, 0, st>>>(f);
-  } else {
-    if (per_warp) front_kernel<D, DT, false, 32><<<front_wgs, 256, 0, st>>>(f);
-    else front_kernel<D, DT, false, 128><<<front_wgs, 256, 0, st>>>(f);
+  // (a pass of the workgroup stays inside one 32-row quantisation group: the wide form needs D = 128 for it)
+  if constexpr (NT == 256 || D == 128) {
+    if (per_warp) {
+      if (pool) front_kernel<D, DT, true, 32, NT><<<front_wgs, NT, 0, st>>>(f);
+      else front_kernel<D, DT, false, 32, NT><<<front_wgs, NT, 0, st>>>(f);
+    }
+  }
+  if (!per_warp) {
+    if (pool) front_kernel<D, DT, true, 128, NT><<<front_wgs, NT, 0, st>>>(f);
+    else front_kernel<D, DT, false, 128, NT><<<front_wgs, NT, 0, st>>>(f);
   }
   if (!c.partial) {
     const FinalParams p = {f.km_part, f.v_part, km, v_amax, f.k_chunks, a->pv_f16 ? 0 : f.v_chunks, a->N_kv};
     final_kernel<D, DT><<<a->B * a->Hkv, dim3(D, 8), 0, st>>>(p);
-    if (pool) back_kernel<D, DT, true, false><<<back_wgs, 256, 0, st>>>(b);
-    else back_kernel<D, DT, false, false><<<back_wgs, 256, 0, st>>>(b);
+    if (pool) back_kernel<D, DT, true, false, NT><<<back_wgs, NT, 0, st>>>(b);
+    else back_kernel<D, DT, false, false, NT><<<back_wgs, NT, 0, st>>>(b);
   } else {
-    if (pool) back_kernel<D, DT, true, true><<<back_wgs, 256, 0, st>>>(b);
-    else back_kernel<D, DT, false, true><<<back_wgs, 256, 0, st>>>(b);
+    if (pool) back_kernel<D, DT, true, true, NT><<<back_wgs, NT, 0, st>>>(b);
+    else back_kernel<D, DT, false, true, NT><<<back_wgs, NT, 0, st>>>(b);
   }
-  return hipGetLastError();
 }
 
 static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides &ks, const Strides &vs, const Strides &os,
@@ -255,8 +262,12 @@ static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const S
   const Hyper simthr = {a->simthreshd1, a->simthreshd1_value};
   int32_t *const lut = (int32_t *)(ws + l.lut);
   int32_t *const valid = a->valid_block_num != nullptr ? a->valid_block_num : (int32_t *)(ws + l.valid);
+  // Fewer than two workgroups of 256 threads per CU leave the stages bound by the length of one thread's work (9.8 and
+  // 13.0 us for the two launches at B2 H3 N1025 D128 with a similarity threshold): twice the threads take half of it.
+  const int wgs256 = heads * nq + kv_heads * 2 * c.n;
+  const int nt = wgs256 <= 512 && !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP) ? 512 : 256;
   int nkp = 256;
-  while (nkp < nk) nkp <<= 1;
+  while (nkp < nk || nkp < nt) nkp <<= 1;
   const bool mask_in_front = !pool && nkp <= MASK_NKP_FRONT;
 
   FrontParams f = {};
@@ -276,7 +287,7 @@ static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const S
   BackParams b = {};
   b.k = f.k; b.v = f.v; b.ks = ks; b.vs = vs;
   b.H = a->H; b.Hkv = a->Hkv; b.Nk = a->N_kv; b.nk = nk; b.v_dtype = a->v_dtype;
-  b.k_wgs_per_head = (a->N_kv + 127) / 128;
+  b.k_wgs_per_head = (a->N_kv + k_rows_per_wg(nt) - 1) / k_rows_per_wg(nt);
   b.wg_v = kv_heads * b.k_wgs_per_head;
   b.km = (const uint16_t *)(ws + l.km); b.km_part = f.km_part; b.k_chunks = c.n;
   b.v_amax = (const float *)(ws + l.v_amax); b.v_part = f.v_part; b.v_chunks = c.n;
@@ -287,11 +298,15 @@ static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const S
   const int front_wgs = f.wg_q + heads * nq, back_wgs = b.wg_v + (a->pv_f16 ? 0 : kv_heads * nk);
   uint16_t *km = (uint16_t *)(ws + l.km);
   float *v_amax = (float *)(ws + l.v_amax);
-  hipError_t e;
-  if (a->D == 64) e = a->qk_dtype == 0 ? run_front_back<64, 0>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st)
-                                       : run_front_back<64, 1>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);
-  else e = a->qk_dtype == 0 ? run_front_back<128, 0>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st)
-                            : run_front_back<128, 1>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);
+#define SPG_RUN(D_, DT_)                                                                                    \
+  {                                                                                                         \
+    if (nt == 512) run_front_back<D_, DT_, 512>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);            \
+    else run_front_back<D_, DT_, 256>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);                      \
+  }
+  if (a->D == 64) { if (a->qk_dtype == 0) SPG_RUN(64, 0) else SPG_RUN(64, 1) }
+  else            { if (a->qk_dtype == 0) SPG_RUN(128, 0) else SPG_RUN(128, 1) }
+#undef SPG_RUN
+  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const bool sel_in_attn = pool && nk <= SPG_SELECT_IN_ATTN_NK;
   RowSelect sel = {};

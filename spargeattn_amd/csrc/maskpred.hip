@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void block_select_kernel(
     const size_t row_off = ((size_t)bh * nq + i) * nk;
     if (bmap != nullptr)
       for (int j = tid; j < nk; j += 256) bmap[row_off + j] = flag(j) ? 1 : 0;
-    emit_lut(flag, nk, nkp, s_idx, s_tmp, lut + row_off, valid + (size_t)bh * nq + i);
+    emit_lut<256>(flag, nk, nkp, s_idx, s_tmp, lut + row_off, valid + (size_t)bh * nq + i);
     __syncthreads();                                // the work area is reused by the next row
   }
 }
@@ -766,7 +766,7 @@ hipError_t launch_block_select(const void *pq, const uint8_t *sq, const void *pk
 hipError_t launch_map_to_lut(const void *mask, int kind, int32_t *lut, int32_t *valid, int B, int H, int nq, int nk,
                              hipStream_t st) {
   const int nkp = next_pow2_ge(nk, 256);
-  const size_t lds = 4 * (size_t)nkp + 16;
+  const size_t lds = 4 * (size_t)nkp + 64;
   const dim3 grid(nq, B * H);
 #define SPG_M2L(K_)                                                                                      \
   case K_: {                                                                                             \

@@ -15,13 +15,13 @@ namespace spg {
 // =============================================================================================
 // K column mean
 // =============================================================================================
-template <int D> constexpr int km_partial_lds() { return 256 / (D / 8) * D * 8; }
-template <int D, int DT>
+template <int D, int NT = 256> constexpr int km_partial_lds() { return NT / (D / 8) * D * 8; }
+template <int D, int DT, int NT = 256>
 __device__ __forceinline__ void km_partial_body(const uint16_t *__restrict__ k, const Strides &ks, int H,
                                                 double *__restrict__ part, int N, int rows_per_chunk, int chunk, int nchunk,
                                                 int bh, unsigned char *smem) {
   constexpr int TPR = D / 8;      // lanes per row (16 B each)
-  constexpr int RPP = 256 / TPR;  // rows per pass of the workgroup
+  constexpr int RPP = NT / TPR;   // rows per pass of the workgroup
   const int c = threadIdx.x % TPR, r = threadIdx.x / TPR;
   const int row0 = chunk * rows_per_chunk;
   const int row1 = min(N, row0 + rows_per_chunk);
@@ -112,7 +112,7 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return v;
 }
 
-// One workgroup handles 128 consecutive rows of one (batch, head): one 128-row block or two 64-row blocks (SUB), so
+// One workgroup handles ROWS consecutive rows of one (batch, head), by default 128: one 128-row block or two 64-row blocks (SUB), so
 // that the per-block tail (column reduction, pooled mean, flag, scale) is spread over all four wavefronts in both cases.
 // QR = rows that share one INT8 scale: BS (per-block granularity, what the reference's operators use) or 32 rows of a
 // 128-row Q block (per-warp granularity: quant_per_block.py:102-148 with WARPQ = 32, one scale per 32 query rows, which
@@ -121,17 +121,19 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 // km_partial_body wrote - every workgroup adds them up for itself, which takes the small kernel in between out of the
 // launch chain and pays while there are few chunks.
 enum { MEAN_NONE = 0, MEAN_GIVEN = 1, MEAN_PARTIAL = 2 };
-template <int BS, int D> constexpr int psq_lds() { return 128 / BS * (256 / (D / 8)) * D * 8; }
-template <int BS, int D, int DT, int MEAN, bool WITH_POOL, int QR = BS>
+// NT threads work on ROWS rows: 256 on 128 where there are enough workgroups to fill the chip, more threads on fewer rows
+// where there are not and the time is the length of one thread's work.
+template <int BS, int D, int NT = 256, int ROWS = 128> constexpr int psq_lds() { return ROWS / BS * (NT / (D / 8)) * D * 8; }
+template <int BS, int D, int DT, int MEAN, bool WITH_POOL, int QR = BS, int NT = 256, int ROWS = 128>
 __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const Strides &xs,
                                          const uint16_t *__restrict__ km, const double *__restrict__ km_part, int km_chunks,
                                          uint16_t *__restrict__ pool, uint8_t *__restrict__ sim,
                                          int8_t *__restrict__ xq, float *__restrict__ scale,
                                          const float simthr, int H, int N, int nb, int wg, int bh, unsigned char *smem) {
-  constexpr int ROWS = 128;           // rows per workgroup
   constexpr int SUB = ROWS / BS;      // blocks per workgroup
   constexpr int TPR = D / 8;          // lanes per row (16 B each)
-  constexpr int RPP = 256 / TPR;      // rows per pass of the workgroup
+  constexpr int RPP = NT / TPR;       // rows per pass of the workgroup
+  constexpr int NWV = NT / 64;        // wavefronts
   constexpr int NPT = ROWS / RPP;     // passes (rows per thread)
   constexpr int NP = BS / RPP;        // passes per block
   constexpr int WPS = D / 64;         // wavefronts that hold one block's columns in the tail (thread = block * D + column)
@@ -141,7 +143,7 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
   static_assert(BS == 64 || BS == 128, "block sizes of the operators");
   static_assert(QR == BS || (QR == 32 && BS == 128), "per-block, or 32-row groups of a Q block");
   static_assert(RPP <= QR, "a pass of the workgroup stays inside one quantisation group");
-  static_assert(RPP <= BS && SUB * D <= 256, "thread <-> (block, column) mapping of the tail");
+  static_assert(RPP <= BS && SUB >= 1 && SUB * D <= NT, "thread <-> (block, column) mapping of the tail");
   // magnitude patterns (sign bit cleared) order like the magnitudes, for both 16-bit formats
   constexpr uint32_t ABS2 = 0x7fff7fffu;
   constexpr uint32_t INF16 = DT == 1 ? 0x7f80u : 0x7c00u;
@@ -173,9 +175,9 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
       v = *(const uint4 *)(km + (size_t)bh * D + c * 8);
     } else {
       // (the sums are exact in binary64: their order is free)
-      constexpr int G = 256 / D;
+      constexpr int G = NT / D;
       double *s_sub = (double *)smem;
-      uint16_t *s_km = (uint16_t *)(smem + 256 * 8);
+      uint16_t *s_km = (uint16_t *)(smem + NT * 8);
       double s = 0.0;
 #pragma unroll 4
       for (int i = tid / D; i < km_chunks; i += G) s += km_part[((size_t)bh * km_chunks + i) * D + tid % D];
@@ -265,8 +267,8 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
     for (int g = sb * GPB; g < (sb + 1) * GPB; g++) m = max(m, (mm[g / 2] >> (16 * (g % 2))) & 0xffffu);
     return m;
   };
-  __shared__ uint32_t s_wmax[4][MW], s_wbad[4];
-  __shared__ long long s_wg[4];
+  __shared__ uint32_t s_wmax[NWV][MW], s_wbad[NWV];
+  __shared__ long long s_wg[NWV];
 #pragma unroll
   for (int i = 0; i < MW; i++) {
     uint32_t mw = m_thread[i];                    // two groups' maxima reduced together
@@ -408,7 +410,9 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
       if ((tid & 63) == 0) s_wbad[tid >> 6] = wb;
     }
     __syncthreads();
-    const uint32_t any_bad = s_wbad[0] | s_wbad[1] | s_wbad[2] | s_wbad[3];
+    uint32_t any_bad = 0;
+#pragma unroll
+    for (int i = 0; i < NWV; i++) any_bad |= s_wbad[i];
     if (tid < SUB && rows_valid_of(tid) > 0) {
       const int rv = rows_valid_of(tid);
       bool similar = sim_trivial;
@@ -426,8 +430,11 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
 
   uint32_t m_all[MW];
 #pragma unroll
-  for (int i = 0; i < MW; i++)
-    m_all[i] = pk_max_u16(pk_max_u16(s_wmax[0][i], s_wmax[1][i]), pk_max_u16(s_wmax[2][i], s_wmax[3][i]));
+  for (int i = 0; i < MW; i++) {
+    m_all[i] = s_wmax[0][i];
+#pragma unroll
+    for (int wv = 1; wv < NWV; wv++) m_all[i] = pk_max_u16(m_all[i], s_wmax[wv][i]);
+  }
   int8_t *qb = xq + ((size_t)bh * N + row_base) * D + c * 8;
 #pragma unroll
   for (int g = 0; g < NQG; g++) {
@@ -473,8 +480,9 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
   }
 }
 
-// exclusive prefix of per-thread counts over the 256 threads of the workgroup; returns (offset, total)
-__device__ __forceinline__ int2 block_exclusive_scan_i32(int v, int *s_tmp /* >= 4 ints */) {
+// exclusive prefix of per-thread counts over the NT threads of the workgroup; returns (offset, total)
+template <int NT>
+__device__ __forceinline__ int2 block_exclusive_scan_i32(int v, int *s_tmp /* >= NT / 64 ints */) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int inc = v;
 #pragma unroll
@@ -485,26 +493,31 @@ __device__ __forceinline__ int2 block_exclusive_scan_i32(int v, int *s_tmp /* >=
   __syncthreads();                       // s_tmp may still be read from a previous call
   if (lane == 63) s_tmp[wave] = inc;
   __syncthreads();
-  const int w0 = s_tmp[0], w1 = s_tmp[1], w2 = s_tmp[2], w3 = s_tmp[3];
-  const int base = (wave > 0 ? w0 : 0) + (wave > 1 ? w1 : 0) + (wave > 2 ? w2 : 0);
-  return make_int2(base + inc - v, w0 + w1 + w2 + w3);
+  int base = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; w++) {
+    const int t = s_tmp[w];
+    if (w < wave) base += t;
+    total += t;
+  }
+  return make_int2(base + inc - v, total);
 }
 
 // flags (per column, via functor) -> ascending compact index list -> delta LUT, zero tail, valid count.
-template <class FlagFn>
+template <int NT, class FlagFn>
 __device__ __forceinline__ void emit_lut(FlagFn flag, int nk, int nkp, int32_t *s_idx, int *s_tmp,
                                          int32_t *__restrict__ lut_row, int32_t *__restrict__ valid_out) {
   const int tid = threadIdx.x;
-  const int seg = nkp / 256;
+  const int seg = nkp / NT;
   const int j0 = tid * seg, j1 = min(nk, j0 + seg);
   int cnt = 0;
   for (int j = j0; j < j1; j++) cnt += flag(j) ? 1 : 0;
-  const int2 st = block_exclusive_scan_i32(cnt, s_tmp);
+  const int2 st = block_exclusive_scan_i32<NT>(cnt, s_tmp);
   int pos = st.x;
   for (int j = j0; j < j1; j++)
     if (flag(j)) s_idx[pos++] = j;
   __syncthreads();
-  for (int p = tid; p < nk; p += 256) {
+  for (int p = tid; p < nk; p += NT) {
     int v = 0;
     if (p < st.y) v = s_idx[p] - (p ? s_idx[p - 1] : 0);
     lut_row[p] = v;
@@ -528,16 +541,16 @@ __device__ __forceinline__ bool mask_nonzero(const void *row, int j) {
 }
 constexpr int mask_elem_size(int kind) { return kind == 0 ? 1 : (kind == 1 || kind == 4) ? 2 : (kind == 2 || kind == 5) ? 4 : 8; }
 
-// one row of a user mask -> LUT row; LDS: 4 * nkp bytes for the index list, 16 for the scan
-template <int KIND>
+// one row of a user mask -> LUT row; LDS: 4 * nkp bytes for the index list, 64 for the scan; nkp is a multiple of NT
+template <int KIND, int NT = 256>
 __device__ __forceinline__ void map_to_lut_body(const void *__restrict__ mask, int32_t *__restrict__ lut,
                                                 int32_t *__restrict__ valid, int nk, int nkp, size_t row_id,
                                                 unsigned char *smem) {
-  int32_t *s_idx = (int32_t *)(smem + 16);
+  int32_t *s_idx = (int32_t *)(smem + 64);
   const size_t row_off = row_id * nk;
   const void *row = (const unsigned char *)mask + row_off * mask_elem_size(KIND);
   auto flag = [&](int j) -> bool { return mask_nonzero<KIND>(row, j); };
-  emit_lut(flag, nk, nkp, s_idx, (int *)smem, lut + row_off, valid + row_id);
+  emit_lut<NT>(flag, nk, nkp, s_idx, (int *)smem, lut + row_off, valid + row_id);
 }
 
 // =============================================================================================
@@ -552,12 +565,12 @@ __device__ __forceinline__ float elem_to_f16_f32(uint16_t b) {
 }
 
 // Largest |fp16(v)| of every channel over one chunk of rows.  store(d, value) receives the result of channel d.
-template <int D> constexpr int v_absmax_lds() { return 256 / (D / 8) * D * 4; }
-template <int D, int DT, class Store>
+template <int D, int NT = 256> constexpr int v_absmax_lds() { return NT / (D / 8) * D * 4; }
+template <int D, int DT, int NT = 256, class Store>
 __device__ __forceinline__ void v_absmax_body(const uint16_t *__restrict__ v, const Strides &vs, int H, int N,
                                               int rows_per_chunk, int chunk, int bh, unsigned char *smem, Store store) {
   constexpr int TPR = D / 8;
-  constexpr int RPP = 256 / TPR;
+  constexpr int RPP = NT / TPR;
   const int c = threadIdx.x % TPR, r = threadIdx.x / TPR;
   const int row0 = chunk * rows_per_chunk;
   const int row1 = min(N, row0 + rows_per_chunk);
@@ -613,12 +626,12 @@ __device__ __forceinline__ void v_absmax_body(const uint16_t *__restrict__ v, co
 // One workgroup per 64-key tile.  LDS holds the transposed tile [D][64] bytes.
 // amax_of(d): the channel maximum (a whole-head value, from wherever the kernel has it).
 template <int D> constexpr int v_quant_lds() { return D * (64 + 4); }
-template <int D, int DT, class Amax>
+template <int D, int DT, int NT = 256, class Amax>
 __device__ __forceinline__ void v_quant_body(const uint16_t *__restrict__ v, const Strides &vs, int H,
                                              uint8_t *__restrict__ v8, int N, int nk, int blk, int bh, unsigned char *smem,
                                              Amax amax_of) {
   constexpr int TPR = D / 8;
-  constexpr int RPP = 256 / TPR;
+  constexpr int RPP = NT / TPR;
   constexpr int NP = 64 / RPP;
   constexpr int LDW = 64 + 4;  // padded row (bytes) of the transposed tile
   uint8_t *tile = smem;
@@ -649,7 +662,7 @@ __device__ __forceinline__ void v_quant_body(const uint16_t *__restrict__ v, con
   }
   __syncthreads();
   uint8_t *out = v8 + ((size_t)bh * nk + blk) * (size_t)(D * 64);
-  for (int i = tid; i < D * 4; i += 256) {   // 16-byte pieces: D rows x 4 slots
+  for (int i = tid; i < D * 4; i += NT) {   // 16-byte pieces: D rows x 4 slots
     const int d = i >> 2, slot = i & 3;
     const int kc = slot ^ ((d >> 2) & 3);      // key chunk stored in this slot
     const uint32_t *src = (const uint32_t *)(tile + d * LDW + kc * 16);
@@ -661,12 +674,12 @@ __device__ __forceinline__ void v_quant_body(const uint16_t *__restrict__ v, con
 // 64 keys) the eight 8-key chunks are stored at slot = chunk ^ ((d >> 1) & 7) (the LDS swizzle of the attention kernel).
 // Keys at or beyond N are zero.  One workgroup per 64-key tile.
 template <int D> constexpr int v_tiles_f16_lds() { return D * (64 + 2) * 2; }
-template <int D, int DT>
+template <int D, int DT, int NT = 256>
 __device__ __forceinline__ void v_tiles_f16_body(const uint16_t *__restrict__ v, const Strides &vs, int H,
                                                  uint16_t *__restrict__ vt, int N, int nk, int blk, int bh,
                                                  unsigned char *smem) {
   constexpr int TPR = D / 8;
-  constexpr int RPP = 256 / TPR;
+  constexpr int RPP = NT / TPR;
   constexpr int NP = 64 / RPP;
   constexpr int LDW = 64 + 2;  // padded row (halves) of the transposed tile
   uint16_t *tile = (uint16_t *)smem;
@@ -692,7 +705,7 @@ __device__ __forceinline__ void v_tiles_f16_body(const uint16_t *__restrict__ v,
   }
   __syncthreads();
   uint16_t *out = vt + ((size_t)bh * nk + blk) * (size_t)(D * 64);
-  for (int i = tid; i < D * 8; i += 256) {   // 16-byte pieces: D rows x 8 slots
+  for (int i = tid; i < D * 8; i += NT) {   // 16-byte pieces: D rows x 8 slots
     const int d = i >> 3, slot = i & 7;
     const int kc = slot ^ ((d >> 1) & 7);      // key chunk stored in this slot
     const uint16_t *src = tile + d * LDW + kc * 8;
