@@ -257,11 +257,11 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   const int last_partial_blk = (Nk % 64) ? p.nk - 1 : -1;   // the only block with rows beyond Nk
   typedef __attribute__((address_space(3))) void *lds_ptr_t;
   typedef const __attribute__((address_space(1))) void *glb_ptr_t;
-#define SPG_LOAD_K_(BLK, KOFF)   /* inside a scope that holds SPG_LANE_OFFSETS() */                            \
+#define SPG_LOAD_K_(BLK, KOFF, CHK)   /* inside a scope that holds SPG_LANE_OFFSETS() */                            \
   {                                                                                                           \
-    const int8_t *kb_ = kbase + (size_t)(BLK) * TILE;                                                         \
+    const int8_t *kb_ = kbase + (size_t)((uint32_t)(BLK) * (uint32_t)TILE);                                                         \
     unsigned char *lk_ = sKr + (KOFF) + WL * wave * 1024;                                                     \
-    if ((BLK) != last_partial_blk) {                                                                          \
+    if (CHK == 0 || (BLK) != last_partial_blk) {                                                              \
       /* the loads of one tile back to back: they share the LDS base register (M0) */                          \
       __builtin_amdgcn_global_load_lds((glb_ptr_t)(kb_ + k_lane), (lds_ptr_t)lk_, 16, 0, 0);                  \
       if constexpr (WL == 2)                                                                                  \
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   }
 #define SPG_LOAD_V_(BLK, VOFF)                                                                                \
   {                                                                                                           \
-    const uint8_t *vb_ = vbase + (size_t)(BLK) * VTILE;                                                       \
+    const uint8_t *vb_ = vbase + (size_t)((uint32_t)(BLK) * (uint32_t)VTILE);                                                       \
     unsigned char *lv_ = sVr + (VOFF) + WLV * wave * 1024;                                                    \
     __builtin_amdgcn_global_load_lds((glb_ptr_t)(vb_ + v_lane), (lds_ptr_t)lv_, 16, 0, 0);                    \
     if constexpr (WLV >= 2)                                                                                   \
@@ -289,10 +289,10 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
       __builtin_amdgcn_global_load_lds((glb_ptr_t)(vb_ + v_lane), (lds_ptr_t)lv_, 16, 3072, 0);               \
     }                                                                                                         \
   }
-#define SPG_LOAD_K(BLK, KOFF) { SPG_LANE_OFFSETS() (void)v_lane; SPG_LOAD_K_(BLK, KOFF) }
+#define SPG_LOAD_K(BLK, KOFF) { SPG_LANE_OFFSETS() (void)v_lane; SPG_LOAD_K_(BLK, KOFF, 1) }
 #define SPG_LOAD_V(BLK, VOFF) { SPG_LANE_OFFSETS() (void)k_lane; (void)pos0; SPG_LOAD_V_(BLK, VOFF) }
 // FP8 PV: both tiles of one block into ring slot offset BUFOFF (in K-tile units)
-#define SPG_LOAD_TILES(BLK, BUFOFF) { SPG_LANE_OFFSETS() SPG_LOAD_K_(BLK, BUFOFF) SPG_LOAD_V_(BLK, BUFOFF) }
+#define SPG_LOAD_TILES(BLK, BUFOFF, CHK) { SPG_LANE_OFFSETS() SPG_LOAD_K_(BLK, BUFOFF, CHK) SPG_LOAD_V_(BLK, BUFOFF) }
 
   // MFMA row i of key tile kt carries key 32*((i>>2)&1) + 16*kt + 4*(i>>3) + (i&3); rows krow0 and krow0+16 have
   // the same swizzle, so tile 1's operand sits 16 rows (16*D bytes) after tile 0's.
@@ -337,8 +337,8 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     SPG_LOAD_V(blk, 0);
     if (nv > 1) SPG_LOAD_K(blk1, TILE);           // the V^T tile of block 1 follows behind the first barrier
   } else {
-    SPG_LOAD_TILES(blk, 0);
-    if (nv > 1) SPG_LOAD_TILES(blk1, TILE);
+    SPG_LOAD_TILES(blk, 0, 1);
+    if (nv > 1) SPG_LOAD_TILES(blk1, TILE, 1);
   }
   if constexpr (!PV16) {
     if (wave < D / 64)
@@ -434,8 +434,8 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     float ksc2 = 0.f;
     int d4 = 0;
     if constexpr (!TAIL) {
-      ksc2 = kscale[blk2];
-      if constexpr (!SEL) d4 = it + 4 < nv ? lutc[it + 4] : 0;
+      ksc2 = kscale[(uint32_t)blk2];
+      if constexpr (!SEL) d4 = it + 4 < nv ? lutc[(uint32_t)(it + 4)] : 0;
     }
     __builtin_amdgcn_sched_barrier(0);
     const float dq = qs * ksc;                     // used by the tail blocks only
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
       // max over rows of (diff) + thr > 0  <=>  some row has diff + thr > 0 (fp32 addition is monotonic)
       vote = __any(diff + thr > 0.f);
       if (vote == 0) {                    // wavefront-uniform
-        if (lane == 0) sSkipAt[it & 1][wave] = it;
+        sSkipAt[it & 1][wave] = it;       // every lane: a branch on the lane would make the body's control flow divergent
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       }
     }
@@ -515,14 +515,14 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
       // (it + 1) % 2 (the previous block's P.V product)
       SPG_LANE_OFFSETS()
       (void)pos0;
-      if (!TAIL || it + 2 < nv) SPG_LOAD_K_(blk2, bufoff);
+      if (!TAIL || it + 2 < nv) SPG_LOAD_K_(blk2, bufoff, (TAIL || SLOT < 0));
       if (!TAIL || it + 1 < nv) SPG_LOAD_V_(blk1, 2 * (bufoff ^ (uint32_t)TILE));
     } else if (!TAIL || it + 2 < nv) {
       if constexpr (CS) {
-        SPG_LOAD_TILES(blk2, ((SLOT + 2) % 3) * TILE);
+        SPG_LOAD_TILES(blk2, ((SLOT + 2) % 3) * TILE, 0);
       } else {
         const uint32_t b2 = bufoff == 0 ? 2 * TILE : bufoff - TILE;   // slot (it+2) % 3
-        SPG_LOAD_TILES(blk2, b2);
+        SPG_LOAD_TILES(blk2, b2, 1);
       }
     }
     // the running maximum of some query rose: rescale (exp2(0) = 1 exactly, so the other iterations need neither the
@@ -535,7 +535,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
 #pragma unroll
         for (int e = 0; e < 16; e++) O[dt][e] *= osc;
     }
-    if (compute) {
+    if (__builtin_expect(compute, 1)) {
       cnt++;
       const float neg0 = PV16 ? -m : -m + SPG_FP8_OFFSET;
       float ps;
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
       if (!masked) {
         // three passes kept apart for the scheduler: a multiply-add feeding the exponential of the same element directly,
         // and the exponential feeding the running sum, would issue as one long chain of dependent instructions
-        if (!precise) {
+        if (__builtin_expect(!precise, 1)) {
           const float neg = __builtin_fmaf(-acc_c, a26, neg0);   // takes the accumulator constant out: one rounding per row
 #pragma unroll
           for (int e = 0; e < 32; e++) x[e] = __builtin_fmaf(__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]), a26, neg);
@@ -560,9 +560,15 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
         for (int e = 0; e < 32; e++) x[e] = __builtin_amdgcn_exp2f(x[e]);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!PV16) {
-          ps = x[0];
+          // (four chains at D = 64, whose two P.V matrix instructions do not cover one chain of 31 dependent additions)
+          constexpr int NC = D == 64 ? 4 : 1;
+          float pc[NC];
 #pragma unroll
-          for (int e = 1; e < 32; e++) ps += x[e];
+          for (int e = 0; e < NC; e++) pc[e] = x[e];
+#pragma unroll
+          for (int e = NC; e < 32; e++) pc[e % NC] += x[e];
+          ps = pc[0];
+          if constexpr (NC == 4) ps = (pc[0] + pc[1]) + (pc[2] + pc[3]);
         }
       } else {
         ps = 0.f;
@@ -658,6 +664,12 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
       }
       }   // !PV16
     }
+    // the scalar prefetches are taken over here, where no LDS read is in flight: a first use behind the next K reads
+    // would wait for those as well (one counter)
+    if constexpr (!TAIL) {
+      if constexpr (SEL) asm volatile("" : "+s"(ksc2));
+      else asm volatile("" : "+s"(ksc2), "+s"(d4));
+    }
     // advance the block pipeline and the ring
     blk = blk1; blk1 = blk2;
     if constexpr (SEL) blk2 = next_block(blk2);
@@ -670,7 +682,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     // the common loop, three blocks per trip (ring slots 0, 1, 2); `bufoff` stays 0 throughout where the slots are
     // compile-time constants, and three run-time steps bring it back to 0 where they are not
 #pragma unroll 1
-    for (; it + 3 <= nv - 2; it += 3) {
+    for (; it + 3 <= nv - 3; it += 3) {
       step(std::false_type{}, std::integral_constant<int, 0>{}, it);
       step(std::false_type{}, std::integral_constant<int, 1>{}, it + 1);
       step(std::false_type{}, std::integral_constant<int, 2>{}, it + 2);
