@@ -48,6 +48,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define SPG_FP8_OFFSET 8.807f       // csrc/qattn/attn_utils.cuh:28
 #define SPG_ACC_C_BITS 0x3E22F983    // the float 1/(2 pi), an inline constant of the instruction set: initial accumulator
 #define SPG_ACC_SCALE 67108864.0f    // 2^26: one unit of the integer dot product is 2^-26 in the binade [1/8, 1/4)
+#define SPG_ROW_MAJOR_MAX 512       // workgroups per XCD up to which causal rows are ordered by length across heads
 #define SPG_LOG2E 1.44269504088896340736f
 
 struct AttnParams {
@@ -65,8 +66,57 @@ struct AttnParams {
   int pv_mode;     // PVThresholdMode of the reference (attn_utils.cuh:58-62): 0 none, 1 per block, 2 per wavefront of 32 rows
   int q_per_warp;  // QuantGranularity of Q (sm89.cuh:106-121): 0 one scale per 128-row block, 1 one per 32 rows (B,H,nq*4)
   int total_wg, wg_per_xcd;
+  int rows_first;  // so many of the longest rows of every head come before the rest (place_workgroup)
   RowSelect sel;   // selection inside the kernel (template argument SEL); lut is unused then
 };
+
+// Workgroup -> (batch*head, q block).  Ids are dealt round-robin over the 8 XCDs; each XCD (one L2) gets a contiguous
+// range of (head, row) pairs, rows from the last one down: causal rows get longer with the row index, and a partial last
+// Q block is never "similar", so all its blocks are kept.
+// Within the range the order is head by head, so that the resident workgroups share K/V tiles - except that the first
+// `rows_first` rows of ALL heads of the range come first: a long row that starts when the rest of the chip is about to
+// finish runs on alone.  (Measured with head-by-head order: H30 N17776 D64, whose partial last rows are twice as long as the
+// others, last workgroup at 1150 us with the median CU done at 1034; causal H32 N4096, 101 us against 81.)
+__device__ __forceinline__ bool place_workgroup(const AttnParams &p, int w, int &bh, int &qb) {
+  const int L0 = (w & 7) * p.wg_per_xcd, L1 = min(L0 + p.wg_per_xcd, p.total_wg);
+  int j = w >> 3;
+  if (L0 + j >= L1) return false;
+  const int nq = p.nq, T = p.rows_first;
+  // the range is rows a.. of head h0 (if a > 0), all rows of F heads from hf on, rows ..b-1 of head h1 (if b > 0)
+  const int h0 = L0 / nq, a = L0 - h0 * nq, h1 = L1 / nq, b = L1 - h1 * nq;
+  const int hf = h0 + (a > 0 ? 1 : 0), F = h1 - hf;
+  int h, t;
+  if (T == 0 || F < 0) {
+    h = (L0 + j) / nq;
+    t = L0 + j - h * nq;
+  } else {
+    auto upto = [&](int rows) { return F * rows + (a > 0 ? max(0, rows - a) : 0) + min(rows, b); };   // pairs with row < rows
+    if (j < upto(T)) {
+      int lo = 0, hi = T - 1;                        // largest row with upto(row) <= j
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (upto(mid) <= j) lo = mid; else hi = mid - 1;
+      }
+      t = lo;
+      int i = j - upto(t);
+      const int first = a > 0 && t >= a ? 1 : 0;
+      h = i < first ? h0 : hf + (i - first);         // the partial last head h1 = hf + F follows the full ones
+    } else {
+      j -= upto(T);
+      const int n0 = a > 0 ? nq - max(a, T) : 0, per = nq - T;
+      if (j < n0) { h = h0; t = max(a, T) + j; }
+      else {
+        j -= n0;
+        const int i = per > 0 ? j / per : 0;
+        h = hf + min(i, F);
+        t = T + j - min(i, F) * per;
+      }
+    }
+  }
+  bh = h;
+  qb = nq - 1 - t;
+  return true;
+}
 
 // v_max_f32 as one instruction: fmaxf() on a value the compiler cannot prove to be a quiet number (a loop-carried
 // maximum, the output of a lane exchange) costs a canonicalising self-maximum per operand first.  The operands here are
@@ -164,12 +214,8 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   const uint32_t lds_k0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)smem;   // LDS byte address
   const uint32_t lds_v0 = lds_k0 + NBUF * TILE;
 
-  // ---- workgroup -> (batch*head, q block): one XCD per head at a time, heavy (late) rows first ----------
-  const int w = blockIdx.x;
-  const int L = (w & 7) * p.wg_per_xcd + (w >> 3);
-  if (L >= p.total_wg) return;
-  const int bh = L / p.nq;
-  const int qb = p.nq - 1 - (L % p.nq);
+  int bh, qb;
+  if (!place_workgroup(p, blockIdx.x, bh, qb)) return;
   const int head = bh % p.H;
   // grouped-query attention: H / Hkv consecutive query heads share one K/V head (sm89.cuh:118, head_id / num_kv_groups)
   const int bhk = (bh / p.H) * p.Hkv + head / (p.H / p.Hkv);
@@ -742,11 +788,14 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
 }
 
 template <bool SEL>
-static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, hipStream_t st) {
+static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_rows, hipStream_t st) {
   p.nq = (p.N + 127) / 128; p.nk = (p.Nk + 63) / 64;
   p.total_wg = p.nq * p.H * p.B;
   p.wg_per_xcd = (p.total_wg + 7) / 8;
   const int grid = p.wg_per_xcd * 8;
+  // Causal rows differ in length throughout: all rows by length while the heads an XCD works on at once share its L2
+  // anyway (grids of a few rounds), head by head beyond.  Otherwise only a partial last Q block stands out.
+  p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
   if (p.v_scale != nullptr) {
     if (D == 64) {
       if (out_dtype == 0) block_sparse_attn_kernel<64, 0, false, SEL><<<grid, 256, 0, st>>>(p);
@@ -771,7 +820,7 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
                                       int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel,
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
-                                      int q_per_warp, int pv_mode, int32_t *pv_count, hipStream_t st) {
+                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, hipStream_t st) {
   AttnParams p = {};
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.out = out; p.os = os; p.lut = lut; p.valid = valid; p.pvthr = pvthreshd;
   p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.pv_count = pv_count;
@@ -780,9 +829,9 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
   p.is_causal = is_causal;
   p.pv_mode = pv_mode;
   p.q_per_warp = q_per_warp;
-  if (sel == nullptr) return launch_attn<false>(p, D, out_dtype, st);
+  if (sel == nullptr) return launch_attn<false>(p, D, out_dtype, causal_rows || is_causal, st);
   p.sel = *sel;
-  return launch_attn<true>(p, D, out_dtype, st);
+  return launch_attn<true>(p, D, out_dtype, causal_rows || is_causal, st);
 }
 
 hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
@@ -791,7 +840,7 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st) {
   return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, nullptr, Hyper{pvthreshd, 0.f}, q_scale, k_scale,
-                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, st);
+                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, false, st);
 }
 
 }  // namespace spg

@@ -323,7 +323,7 @@ static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const S
                                     Hyper{a->pvthreshd, a->pvthreshd_value},
                                     f.q_scale, b.k_scale, a->pv_f16 ? nullptr : b.v_scale, a->B, a->H, a->Hkv, a->N, a->N_kv, a->D,
                                     a->sm_scale, a->kernel_causal ? 1 : 0, a->qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0,
-                                    SPG_PV_PER_BLOCK, nullptr, st);
+                                    SPG_PV_PER_BLOCK, nullptr, pool && a->is_causal, st);
 }
 
 static int check_args(const char *fn, const spg_attn_args *a) {
