@@ -49,6 +49,8 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define SPG_ACC_C_BITS 0x3E22F983    // the float 1/(2 pi), an inline constant of the instruction set: initial accumulator
 #define SPG_ACC_SCALE 67108864.0f    // 2^26: one unit of the integer dot product is 2^-26 in the binade [1/8, 1/4)
 #define SPG_ROW_MAJOR_MAX 512       // workgroups per XCD up to which causal rows are ordered by length across heads
+#define SPG_QUEUE_MIN 384           // workgroups per XCD from which the queue pays: four rounds of 32 CUs x 3
+#define SPG_QUEUE_EXTRA 12          // one workgroup in so many is launched on top
 #define SPG_LOG2E 1.44269504088896340736f
 
 struct AttnParams {
@@ -66,6 +68,7 @@ struct AttnParams {
   int pv_mode;     // PVThresholdMode of the reference (attn_utils.cuh:58-62): 0 none, 1 per block, 2 per wavefront of 32 rows
   int q_per_warp;  // QuantGranularity of Q (sm89.cuh:106-121): 0 one scale per 128-row block, 1 one per 32 rows (B,H,nq*4)
   int total_wg, wg_per_xcd;
+  int *queue;      // NULL, or 8 counters, zero at the start (take_item)
   int rows_first;  // so many of the longest rows of every head come before the rest (place_workgroup)
   RowSelect sel;   // selection inside the kernel (template argument SEL); lut is unused then
 };
@@ -77,9 +80,8 @@ struct AttnParams {
 // `rows_first` rows of ALL heads of the range come first: a long row that starts when the rest of the chip is about to
 // finish runs on alone.  (Measured with head-by-head order: H30 N17776 D64, whose partial last rows are twice as long as the
 // others, last workgroup at 1150 us with the median CU done at 1034; causal H32 N4096, 101 us against 81.)
-__device__ __forceinline__ bool place_workgroup(const AttnParams &p, int w, int &bh, int &qb) {
-  const int L0 = (w & 7) * p.wg_per_xcd, L1 = min(L0 + p.wg_per_xcd, p.total_wg);
-  int j = w >> 3;
+__device__ __forceinline__ bool place_workgroup(const AttnParams &p, int xcd, int j, int &bh, int &qb) {
+  const int L0 = xcd * p.wg_per_xcd, L1 = min(L0 + p.wg_per_xcd, p.total_wg);
   if (L0 + j >= L1) return false;
   const int nq = p.nq, T = p.rows_first;
   // the range is rows a.. of head h0 (if a > 0), all rows of F heads from hf on, rows ..b-1 of head h1 (if b > 0)
@@ -116,6 +118,21 @@ __device__ __forceinline__ bool place_workgroup(const AttnParams &p, int w, int 
   bh = h;
   qb = nq - 1 - t;
   return true;
+}
+
+// With a queue the j-th place of a range goes to whoever asks for it next, and a workgroup whose own XCD has nothing left
+// asks the others: the XCDs do not run at one speed (the fastest and the slowest differ by 5 to 6 % in the time they take for
+// equal shares of a long grid, the same ones on every launch), and a fixed share each leaves the fast ones idle at the end.
+// The grid holds SPG_QUEUE_EXTRA more workgroups than places, so that a fast XCD is dealt enough of them; one that finds
+// nothing ends.  Called by one thread.
+__device__ __forceinline__ int take_item(const AttnParams &p, int w) {
+  for (int i = 0; i < 8; i++) {
+    const int x = (w + i) & 7;
+    const int size = min(p.wg_per_xcd, p.total_wg - x * p.wg_per_xcd);
+    const int j = size > 0 ? __hip_atomic_fetch_add(p.queue + x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    if (j < size) return (j << 3) | x;
+  }
+  return -1;
 }
 
 // v_max_f32 as one instruction: fmaxf() on a value the compiler cannot prove to be a quiet number (a loop-carried
@@ -214,8 +231,17 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   const uint32_t lds_k0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)smem;   // LDS byte address
   const uint32_t lds_v0 = lds_k0 + NBUF * TILE;
 
-  int bh, qb;
-  if (!place_workgroup(p, blockIdx.x, bh, qb)) return;
+  int bh, qb, item = blockIdx.x;
+  if constexpr (!SEL) {                    // (short rows: the grid is over before the XCDs drift apart)
+    if (p.queue != nullptr) {
+      __shared__ int sItem;
+      if (threadIdx.x == 0) sItem = take_item(p, item);
+      __syncthreads();
+      item = __builtin_amdgcn_readfirstlane(sItem);
+      if (item < 0) return;
+    }
+  }
+  if (!place_workgroup(p, item & 7, item >> 3, bh, qb)) return;
   const int head = bh % p.H;
   // grouped-query attention: H / Hkv consecutive query heads share one K/V head (sm89.cuh:118, head_id / num_kv_groups)
   const int bhk = (bh / p.H) * p.Hkv + head / (p.H / p.Hkv);
@@ -792,7 +818,8 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   p.nq = (p.N + 127) / 128; p.nk = (p.Nk + 63) / 64;
   p.total_wg = p.nq * p.H * p.B;
   p.wg_per_xcd = (p.total_wg + 7) / 8;
-  const int grid = p.wg_per_xcd * 8;
+  if (SEL || p.wg_per_xcd < SPG_QUEUE_MIN) p.queue = nullptr;
+  const int grid = 8 * (p.queue != nullptr ? p.wg_per_xcd + p.wg_per_xcd / SPG_QUEUE_EXTRA : p.wg_per_xcd);
   // Causal rows differ in length throughout: all rows by length while the heads an XCD works on at once share its L2
   // anyway (grids of a few rounds), head by head beyond.  Otherwise only a partial last Q block stands out.
   p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
@@ -820,8 +847,9 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
                                       int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel,
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
-                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, hipStream_t st) {
+                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue, hipStream_t st) {
   AttnParams p = {};
+  p.queue = queue;
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.out = out; p.os = os; p.lut = lut; p.valid = valid; p.pvthr = pvthreshd;
   p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.pv_count = pv_count;
   p.B = B; p.H = H; p.Hkv = Hkv; p.N = N; p.Nk = Nk;
@@ -840,7 +868,7 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st) {
   return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, nullptr, Hyper{pvthreshd, 0.f}, q_scale, k_scale,
-                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, false, st);
+                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, false, nullptr, st);
 }
 
 }  // namespace spg

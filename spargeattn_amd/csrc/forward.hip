@@ -38,6 +38,7 @@ struct FrontParams {
   uint8_t *sim_q;
   int8_t *q8;
   float *q_scale;
+  int *queue;                           // cleared here for the attention kernel
 };
 
 template <int A, int B> constexpr int max_c() { return A > B ? A : B; }
@@ -49,6 +50,7 @@ template <int D, int DT, bool POOL, int QR, int NT>
 __global__ __launch_bounds__(NT) void front_kernel(const FrontParams p) {
   __shared__ __align__(16) unsigned char smem[front_lds<D, POOL, NT>()];
   const int w = blockIdx.x;
+  if (w == 0 && threadIdx.x < 8 && (!POOL || p.nk > SPG_SELECT_IN_ATTN_NK)) p.queue[threadIdx.x] = 0;
   if (w >= p.wg_q) {
     const int id = w - p.wg_q, bh = id / p.nq;
     float thr = 0.f;
@@ -195,7 +197,7 @@ static Chunks chunks_for(int heads, int N) {
 }
 
 struct Layout {
-  size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, total;
+  size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, queue, total;
 };
 static Layout layout_for(const spg_attn_args *a) {
   Layout l;
@@ -221,6 +223,7 @@ static Layout layout_for(const spg_attn_args *a) {
   l.v_scale = take(bhk * D * 4);
   l.lut = take(bh * nq * nk * 4);
   l.valid = take(bh * nq * 4);
+  l.queue = take(8 * sizeof(int));
   l.total = at;
   return l;
 }
@@ -283,6 +286,7 @@ static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const S
   f.mask = a->mask; f.mask_kind = a->mask_kind; f.nkp = nkp; f.lut = lut; f.valid = valid;
   f.simthr = simthr;
   f.pool_q = (uint16_t *)(ws + l.pool_q); f.sim_q = ws + l.sim_q; f.q8 = (int8_t *)(ws + l.q8); f.q_scale = (float *)(ws + l.q_scale);
+  f.queue = (int *)(ws + l.queue);
 
   BackParams b = {};
   b.k = f.k; b.v = f.v; b.ks = ks; b.vs = vs;
@@ -323,7 +327,7 @@ static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const S
                                     Hyper{a->pvthreshd, a->pvthreshd_value},
                                     f.q_scale, b.k_scale, a->pv_f16 ? nullptr : b.v_scale, a->B, a->H, a->Hkv, a->N, a->N_kv, a->D,
                                     a->sm_scale, a->kernel_causal ? 1 : 0, a->qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0,
-                                    SPG_PV_PER_BLOCK, nullptr, pool && a->is_causal, st);
+                                    SPG_PV_PER_BLOCK, nullptr, pool && a->is_causal, f.queue, st);
 }
 
 static int check_args(const char *fn, const spg_attn_args *a) {

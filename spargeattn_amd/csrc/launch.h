@@ -66,12 +66,14 @@ struct RowSelect {
   int32_t *valid_out;               // counts for the caller, or NULL
 };
 // sel == NULL: blocks come from lut / valid; otherwise they are selected in place and lut / valid are not read.
+// queue: 8 device ints, zero when the kernel starts, for handing out rows across the XCDs, or NULL for a fixed share each.
 // causal_rows: the selection is causal, so rows get longer with their index (order of the workgroups only).
 hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
                                       int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel,
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
-                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, hipStream_t st);
+                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue,
+                                      hipStream_t st);
 void launch_fp8_pack_selftest(const float *x, uint8_t *codes, int n, int saturate, hipStream_t st);
 
 hipError_t launch_dense_attn_f16(const void *q, const void *k, const void *v, void *out, int B, int H, int N, int D,
