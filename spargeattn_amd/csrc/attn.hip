@@ -51,6 +51,8 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define SPG_ROW_MAJOR_MAX 512       // workgroups per XCD up to which causal rows are ordered by length across heads
 #define SPG_QUEUE_MIN 384           // workgroups per XCD from which the queue pays: four rounds of 32 CUs x 3
 #define SPG_QUEUE_EXTRA 12          // one workgroup in so many is launched on top
+#define SPG_GROUPS_MAX_WG 256       // rows up to which ...
+#define SPG_GROUPS_MIN_NK 12        // ... and K blocks from which a row gets groups of wavefronts
 #define SPG_LOG2E 1.44269504088896340736f
 
 struct AttnParams {
@@ -205,8 +207,15 @@ __device__ __forceinline__ int v_swz(int row) { return (row >> 2) & 3; }
 // SEL: rows of at most 64 blocks are selected here, by the workgroup that then works on them, instead of by a kernel in
 // front that writes a LUT: the row's map is one 64-bit scalar, and the next block is its next set bit.  Takes a launch
 // (about 4.5 us) and the selection kernel's 7-15 us out of the chain and puts about 3 us in.
-template <int D, int ODT, bool PV16, bool SEL>
-__global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnParams p) {
+// G: groups of four wavefronts that share one Q block.  G = 1 is the general kernel.  G > 1 is for grids that leave a row
+// alone on its CU (launch_attn): one wavefront per SIMD then waits out every latency of the chain scores - maximum -
+// exponentials - product by itself.  The groups take the blocks of the row in turn (group g: places g, g + G, ... of the
+// list), each with its own tile rings; what keeps the arithmetic that of the sequential walk is that P is rounded against the
+// running maximum of the blocks BEFORE it in the list, so the groups exchange their block maxima through LDS once per round
+// of G blocks (at the barrier that the rings need anyway), and so the PV-skip test sees the same differences.  O and the
+// denominator are per group and meet in the epilogue.
+template <int D, int ODT, bool PV16, bool SEL, int G>
+__global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_kernel(const AttnParams p) {
   constexpr int KS = D / 32;        // k-steps of the int8 MFMA
   constexpr int NDT = D / 32;       // 32-channel output tiles
   constexpr int TILE = 64 * D;      // bytes of one K tile
@@ -217,18 +226,24 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   // Tile rings.  FP8 PV: three slots each, the tiles of block it+2 are requested while block it is computed.
   // FP16 PV (tiles twice as large): two slots each, so that three workgroups still share a CU (48 KiB): the K tile of
   // block it+2 goes to the slot block it's K tile just left, the V^T tile of block it+1 to the slot of block it-1.
-  constexpr int NBUF = PV16 ? 2 : 3;
-  // LDS: K ring [NBUF][TILE] | V^T ring [NBUF][VTILE] | votes
-  __shared__ __align__(1024) unsigned char smem[NBUF * (TILE + VTILE)];
+  // With groups the CU holds one workgroup only, and three slots each fit for both.
+  constexpr int NBUF = PV16 && G == 1 ? 2 : 3;
+  // LDS: per group K ring [NBUF][TILE] | V^T ring [NBUF][VTILE]; votes
+  __shared__ __align__(1024) unsigned char smem[G * NBUF * (TILE + VTILE)];
   // PV-skip vote of the per-block mode: a wavefront that votes "skip" stamps the iteration number into its slot; a slot
   // that does not hold the current iteration number means "compute".  Only "skip" votes are written (they are rare at the
   // thresholds in use), and only a wavefront that voted "skip" itself has to read the others' slots.  Two sets of slots,
   // used alternately: a wavefront can be at most one barrier ahead of the slowest one.
   __shared__ int sSkipAt[2][4];
   __shared__ __align__(16) float sVscale[PV16 ? 4 : D];   // fetched at the start, read in the epilogue
-  unsigned char *const sKr = smem;
-  unsigned char *const sVr = smem + NBUF * TILE;
-  const uint32_t lds_k0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)smem;   // LDS byte address
+  // Groups: block maxima of a round and the running maximum in front of it, one value per query, two sets used alternately.
+  __shared__ float sFm[2][G > 1 ? G + 1 : 1][G > 1 ? 128 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(G == 1 ? tid >> 6 : (tid >> 6) & 3);   // uniform: everything derived from it stays scalar
+  const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  unsigned char *const sKr = smem + grp * (NBUF * (TILE + VTILE));
+  unsigned char *const sVr = sKr + NBUF * TILE;
+  const uint32_t lds_k0 = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)smem + (uint32_t)(grp * (NBUF * (TILE + VTILE)));   // LDS byte address
   const uint32_t lds_v0 = lds_k0 + NBUF * TILE;
 
   int bh, qb, item = blockIdx.x;
@@ -246,8 +261,6 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   // grouped-query attention: H / Hkv consecutive query heads share one K/V head (sm89.cuh:118, head_id / num_kv_groups)
   const int bhk = (bh / p.H) * p.Hkv + head / (p.H / p.Hkv);
 
-  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: everything derived from it stays scalar
   const int N = p.N, Nk = p.Nk;
   const int q_row = qb * 128 + wave * 32 + r;
   if constexpr (!PV16) fp8_saturation_on();
@@ -263,7 +276,8 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   const c_i32_t lutc = (c_i32_t)(p.lut + (SEL ? 0 : row_id * p.nk));
   const int last_col = p.nk - 1;
   int nv, l0, l1, l2, l3;
-  if constexpr (!SEL) {
+  if constexpr (!SEL && G > 1) nv = ((c_i32_t)p.valid)[row_id];
+  if constexpr (!SEL && G == 1) {
     nv = ((c_i32_t)p.valid)[row_id];
     l0 = lutc[0]; l1 = lutc[min(1, last_col)]; l2 = lutc[min(2, last_col)]; l3 = lutc[min(3, last_col)];
   }
@@ -284,9 +298,11 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     const uint8_t *simk = p.sel.sim_k + (size_t)bhk * p.nk;
     const bool row_forced = p.sel.sim_q[row_id] == 0;
     const bool k_dead = simk[min(lane, last_col)] == 0;
-    const int col = tid >> 2;
-    const uint16_t s16 = pooled_score_4lanes<D, ODT>(p.sel.pool_q + row_id * D, p.sel.pool_k + ((size_t)bhk * p.nk + min(col, last_col)) * D, tid & 3);
-    if ((tid & 3) == 0) sScore[col] = s16;
+    if (grp == 0) {
+      const int col = tid >> 2;
+      const uint16_t s16 = pooled_score_4lanes<D, ODT>(p.sel.pool_q + row_id * D, p.sel.pool_k + ((size_t)bhk * p.nk + min(col, last_col)) * D, tid & 3);
+      if ((tid & 3) == 0) sScore[col] = s16;
+    }
     __syncthreads();
     const int causal_lim = p.sel.is_causal ? min(p.nk, 2 * (qb + 1)) : p.nk;
     const float sc = (lane >= causal_lim || k_dead) ? -INFINITY : elem_to_f32<ODT>(sScore[lane]);
@@ -294,12 +310,15 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     nv = __builtin_popcountll(map);
     if (p.sel.valid_out != nullptr && tid == 0) p.sel.valid_out[row_id] = nv;
   }
-  // SEL: takes the next block out of the map; beyond the last one it repeats `prev`
+  // SEL: takes the next block (of this group) out of the map; beyond the last one it repeats `prev`
   auto next_block = [&](int prev) __attribute__((always_inline)) {
     const int b = map != 0 ? __builtin_ctzll(map) : prev;
-    map &= map - 1;
+#pragma unroll
+    for (int i = 0; i < G; i++) map &= map - 1;
     return b;
   };
+  if constexpr (SEL && G > 1)
+    for (int i = 0; i < grp; i++) map &= map - 1;
   if (nv == 0) return;                                       // output rows stay unwritten (sm89.cuh:232-235)
 
   const int8_t *kbase = p.k8 + (size_t)bhk * Nk * D;
@@ -363,8 +382,8 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   }
 #define SPG_LOAD_K(BLK, KOFF) { SPG_LANE_OFFSETS() (void)v_lane; SPG_LOAD_K_(BLK, KOFF, 1) }
 #define SPG_LOAD_V(BLK, VOFF) { SPG_LANE_OFFSETS() (void)k_lane; (void)pos0; SPG_LOAD_V_(BLK, VOFF) }
-// FP8 PV: both tiles of one block into ring slot offset BUFOFF (in K-tile units)
-#define SPG_LOAD_TILES(BLK, BUFOFF, CHK) { SPG_LANE_OFFSETS() SPG_LOAD_K_(BLK, BUFOFF, CHK) SPG_LOAD_V_(BLK, BUFOFF) }
+// rings of three slots: both tiles of one block into ring slot offset BUFOFF (in K-tile units)
+#define SPG_LOAD_TILES(BLK, BUFOFF, CHK) { SPG_LANE_OFFSETS() SPG_LOAD_K_(BLK, BUFOFF, CHK) SPG_LOAD_V_(BLK, (VTILE / TILE) * (BUFOFF)) }
 
   // MFMA row i of key tile kt carries key 32*((i>>2)&1) + 16*kt + 4*(i>>3) + (i&3); rows krow0 and krow0+16 have
   // the same swizzle, so tile 1's operand sits 16 rows (16*D bytes) after tile 0's.
@@ -382,7 +401,8 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
 
   float m = SPG_NEG_BIG;
   // d = 1.0 initially (sm89.cuh:172).  Each half-lane sums its own 32 keys, so only one of the two starts at 1.
-  float dsum = hh == 0 ? 1.0f : 0.0f;
+  float dsum = hh == 0 && grp == 0 ? 1.0f : 0.0f;
+  float m_own = SPG_NEG_BIG;               // groups: the maximum that this group's O and dsum refer to
   v16f O[NDT];
 #pragma unroll
   for (int dt = 0; dt < NDT; dt++)
@@ -391,9 +411,25 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   int cnt = 0;
 
   // block ids: blk = block of iteration it, blk1 = it+1, blk2 = it+2 (tiles in flight); d3 = LUT delta of it+3.
-  // K scales are fetched one iteration ahead as well.
+  // K scales are fetched one iteration ahead as well.  With groups an iteration is a round: place it * G + grp of the list.
   int blk, blk1, blk2, d3 = 0;
-  if constexpr (SEL) {
+  if constexpr (!SEL && G > 1) {
+    // the LUT holds differences: running sums of its first entries, unused ones read as 0
+    int at = 0, acc = 0;
+    auto advance = [&](int upto) __attribute__((always_inline)) {
+      int l[G];
+#pragma unroll
+      for (int i = 0; i < G; i++) l[i] = lutc[min(at + i, last_col)];
+#pragma unroll
+      for (int i = 0; i < G; i++) acc += at + i < min(nv, upto) ? l[i] : 0;
+      at = upto;
+    };
+    advance(grp + 1); blk = acc;
+    advance(grp + 1 + G); blk1 = acc;
+    advance(grp + 1 + 2 * G); blk2 = acc;
+    acc = 0;
+    advance(grp + 1 + 3 * G); d3 = acc;
+  } else if constexpr (SEL) {
     blk = next_block(0);
     blk1 = next_block(blk);
     blk2 = next_block(blk1);
@@ -404,16 +440,16 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     d3 = nv > 3 ? l3 : 0;
   }
   float ksc = kscale[blk], ksc1 = kscale[blk1];
-  if constexpr (PV16) {
+  if constexpr (PV16 && G == 1) {
     SPG_LOAD_K(blk, 0);
     SPG_LOAD_V(blk, 0);
     if (nv > 1) SPG_LOAD_K(blk1, TILE);           // the V^T tile of block 1 follows behind the first barrier
   } else {
     SPG_LOAD_TILES(blk, 0, 1);
-    if (nv > 1) SPG_LOAD_TILES(blk1, TILE, 1);
+    if (nv > grp + G) SPG_LOAD_TILES(blk1, TILE, 1);
   }
   if constexpr (!PV16) {
-    if (wave < D / 64)
+    if (wave < D / 64 && grp == 0)
       __builtin_amdgcn_global_load_lds((glb_ptr_t)(p.v_scale + (size_t)bhk * D + wave * 64 + lane), (lds_ptr_t)(sVscale + wave * 64), 4, 0, 0);
   }
   uint32_t bufoff = 0;                     // LDS ring offset of block it
@@ -447,6 +483,9 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     constexpr bool TAIL = decltype(tail_tag)::value;
     constexpr int SLOT = decltype(slot_tag)::value;
     constexpr bool CS = SLOT >= 0 && !PV16;         // compile-time ring slot
+    const int place = G == 1 ? it : it * G + grp;   // in the row's list of blocks
+    // groups: a round at the end can hold ordinary blocks, the last two and places beyond the list side by side
+    const bool tail = TAIL && (G == 1 || place >= nv - 2), active = !TAIL || G == 1 || place < nv;
     // ---- S^T = K . Q^T ---------------------------------------------------------------------------------
     v16i S0, S1;
     {
@@ -504,10 +543,14 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     // K operands; from here its latency runs under the MFMAs and the max reduction.
     __builtin_amdgcn_sched_barrier(0);
     float ksc2 = 0.f;
-    int d4 = 0;
-    if constexpr (!TAIL) {
+    int d4 = 0, d4g[G] = {};
+    if constexpr (!TAIL || G > 1) {
       ksc2 = kscale[(uint32_t)blk2];
-      if constexpr (!SEL) d4 = it + 4 < nv ? lutc[(uint32_t)(it + 4)] : 0;
+      if constexpr (!SEL && G == 1) d4 = it + 4 < nv ? lutc[(uint32_t)(it + 4)] : 0;
+      if constexpr (!SEL && G > 1) {
+#pragma unroll
+        for (int i = 0; i < G; i++) d4g[i] = place + 3 * G + 1 + i < nv ? lutc[(uint32_t)(place + 3 * G + 1 + i)] : 0;
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
     const float dq = qs * ksc;                     // used by the tail blocks only
@@ -531,8 +574,8 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
       // slot e of this lane is key 64*blk + 32*hh + e; keys beyond `lim` are masked
       const int key0 = blk * 64 + 32 * hh;
       if (p.is_causal) lim = q_row - key0;                       // key > query (attn_utils.cuh:334-361)
-      if (it == nv - 1) lim = min(lim, Nk - 1 - key0);           // key >= kv_len (attn_utils.cuh:363-389)
-      masked = __any(lim < 31);
+      if (place == nv - 1) lim = min(lim, Nk - 1 - key0);        // key >= kv_len (attn_utils.cuh:363-389)
+      masked = tail && __any(lim < 31);
     }
     if (!masked) {
       int imax = S0[0];
@@ -554,12 +597,20 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
       fm = fm * c;
     }
     fm = half_swap_max_raw(fm);
-    const float diff = fm - m;
-    const float m_new = max_raw(m, fm);
-    const float m_old = m;
-    m = m_new;
+    float diff, m_new, m_old;
+    if constexpr (G == 1) {
+      diff = fm - m;
+      m_new = max_raw(m, fm);
+      m_old = m;
+      m = m_new;
+    } else {
+      if (!active) fm = -INFINITY;
+      sFm[it & 1][grp][wave * 32 + r] = fm;                      // (both halves hold the same value)
+      if (grp == 0) sFm[it & 1][G][wave * 32 + r] = m;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
     int vote = 1;
-    if constexpr (!TAIL) {
+    if constexpr (!TAIL && G == 1) {
       // max over rows of (diff) + thr > 0  <=>  some row has diff + thr > 0 (fp32 addition is monotonic)
       vote = __any(diff + thr > 0.f);
       if (vote == 0) {                    // wavefront-uniform
@@ -574,7 +625,37 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     bool compute = true;
-    if constexpr (!TAIL) {   // workgroup-uniform in the per-block mode (sm89.cuh:318-353), wavefront-uniform otherwise
+    if constexpr (G > 1) {
+      float before = m, after = -INFINITY;                       // maxima of the round's earlier / later blocks
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        const float v = sFm[it & 1][g][wave * 32 + r];
+        if (g < grp) before = max_raw(before, v);
+        if (g > grp) after = max_raw(after, v);
+      }
+      diff = fm - before;
+      m_old = m_own;
+      m_new = max_raw(before, fm);
+      m = max_raw(m_new, after);
+      m_own = m_new;
+      if (!TAIL || (active && !tail)) {
+        // a wavefront that votes "skip" looks at the other queries of the Q block: their maxima are all here
+        if (!__any(diff + thr > 0.f)) {
+          bool some = false;
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            const int q = lane + 64 * u;
+            float b = sFm[it & 1][G][q];
+#pragma unroll
+            for (int g = 0; g < G - 1; g++) b = g < grp ? fmaxf(b, sFm[it & 1][g][q]) : b;
+            some |= sFm[it & 1][grp][q] - b + thr > 0.f;
+          }
+          compute = __any(some);
+        }
+      }
+      if (TAIL) compute = compute && active;
+    }
+    if constexpr (!TAIL && G == 1) {   // workgroup-uniform in the per-block mode (sm89.cuh:318-353), wavefront-uniform otherwise
       compute = p.pv_mode == 0 || vote != 0;
       // per-block mode: a wavefront whose own vote is set knows the OR already; only one that voted "skip" has to read
       // what the others wrote (an LDS round trip that the common case does without)
@@ -582,14 +663,14 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
         compute = !(sSkipAt[it & 1][0] == it && sSkipAt[it & 1][1] == it && sSkipAt[it & 1][2] == it &&
                     sSkipAt[it & 1][3] == it);
     }
-    if constexpr (PV16) {
+    if constexpr (PV16 && G == 1) {
       // two-slot rings: every wavefront is past its reads of K slot it % 2 (this block's scores) and of V^T slot
       // (it + 1) % 2 (the previous block's P.V product)
       SPG_LANE_OFFSETS()
       (void)pos0;
       if (!TAIL || it + 2 < nv) SPG_LOAD_K_(blk2, bufoff, (TAIL || SLOT < 0));
       if (!TAIL || it + 1 < nv) SPG_LOAD_V_(blk1, 2 * (bufoff ^ (uint32_t)TILE));
-    } else if (!TAIL || it + 2 < nv) {
+    } else if (!TAIL || place + 2 * G < nv) {
       if constexpr (CS) {
         SPG_LOAD_TILES(blk2, ((SLOT + 2) % 3) * TILE, 0);
       } else {
@@ -599,7 +680,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     }
     // the running maximum of some query rose: rescale (exp2(0) = 1 exactly, so the other iterations need neither the
     // exponential nor the products)
-    if (__any(diff > 0.f)) {
+    if (__any(G == 1 ? diff > 0.f : m_new > m_old)) {
       const float osc = __builtin_amdgcn_exp2f(m_old - m_new);
       dsum *= osc;
 #pragma unroll
@@ -609,7 +690,7 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     }
     if (__builtin_expect(compute, 1)) {
       cnt++;
-      const float neg0 = PV16 ? -m : -m + SPG_FP8_OFFSET;
+      const float neg0 = PV16 ? -m_new : -m_new + SPG_FP8_OFFSET;
       float ps;
       float x[32];
       if (!masked) {
@@ -738,7 +819,11 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
     }
     // the scalar prefetches are taken over here, where no LDS read is in flight: a first use behind the next K reads
     // would wait for those as well (one counter)
-    if constexpr (!TAIL) {
+    if constexpr (G > 1) {
+      asm volatile("" : "+s"(ksc2));
+#pragma unroll
+      for (int i = 0; i < G; i++) d4 += d4g[i];
+    } else if constexpr (!TAIL) {
       if constexpr (SEL) asm volatile("" : "+s"(ksc2));
       else asm volatile("" : "+s"(ksc2), "+s"(d4));
     }
@@ -751,18 +836,21 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   };
   {
     int it = 0;
+    // rounds whose successor's successor ends in front of the last block (no partial tile to load); rounds in front of the
+    // last two blocks; all rounds
+    const int n_fast = G == 1 ? nv - 3 : (nv - 1) / G - 2, n_common = G == 1 ? nv - 2 : (nv - 2) / G, n_all = (nv + G - 1) / G;
     // the common loop, three blocks per trip (ring slots 0, 1, 2); `bufoff` stays 0 throughout where the slots are
     // compile-time constants, and three run-time steps bring it back to 0 where they are not
 #pragma unroll 1
-    for (; it + 3 <= nv - 3; it += 3) {
+    for (; it + 3 <= n_fast; it += 3) {
       step(std::false_type{}, std::integral_constant<int, 0>{}, it);
       step(std::false_type{}, std::integral_constant<int, 1>{}, it + 1);
       step(std::false_type{}, std::integral_constant<int, 2>{}, it + 2);
     }
 #pragma unroll 1
-    for (; it < nv - 2; it++) step(std::false_type{}, std::integral_constant<int, -1>{}, it);
+    for (; it < n_common; it++) step(std::false_type{}, std::integral_constant<int, -1>{}, it);
 #pragma unroll 1
-    for (; it < nv; it++) step(std::true_type{}, std::integral_constant<int, -1>{}, it);
+    for (; it < n_all; it++) step(std::true_type{}, std::integral_constant<int, -1>{}, it);
   }
 #undef SPG_LOAD_TILES
 #undef SPG_LOAD_K
@@ -776,16 +864,48 @@ __global__ __launch_bounds__(256, 3) void block_sparse_attn_kernel(const AttnPar
   if (p.pv_count != nullptr && lane == 0) p.pv_count[((size_t)bh * p.nq + qb) * 4 + wave] = cnt;
 
   // ---- epilogue: O / d * v_scale -> out dtype -----------------------------------------------------------
-  const float dtot = half_swap_sum_f32(dsum);
+  float dtot = half_swap_sum_f32(dsum);
+  if constexpr (G > 1) {
+    // the groups' sums, relative to the row's final maximum, meet in the (free) tile rings; group 0 goes on alone
+    constexpr int GBYTES = 4 * 64 * NDT * 64;                // of one group's O
+    static_assert((G - 1) * GBYTES <= (int)sizeof(smem), "O of the other groups fits the tile rings");
+    const float f = __builtin_amdgcn_exp2f(m_own - m);
+    dtot *= f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) O[dt][e] *= f;
+    __syncthreads();
+    float4 *const so = (float4 *)smem + (wave * NDT * 4) * 64 + lane;
+    if (grp > 0) {
+      sFm[0][grp][wave * 32 + r] = dtot;
+#pragma unroll
+      for (int i = 0; i < NDT * 4; i++)
+        so[(grp - 1) * (GBYTES / 16) + i * 64] = make_float4(O[i / 4][4 * (i % 4)], O[i / 4][4 * (i % 4) + 1], O[i / 4][4 * (i % 4) + 2], O[i / 4][4 * (i % 4) + 3]);
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int g = 1; g < G; g++) {
+        dtot += sFm[0][g][wave * 32 + r];
+#pragma unroll
+        for (int i = 0; i < NDT * 4; i++) {
+          const float4 t = so[(g - 1) * (GBYTES / 16) + i * 64];
+          O[i / 4][4 * (i % 4)] += t.x; O[i / 4][4 * (i % 4) + 1] += t.y; O[i / 4][4 * (i % 4) + 2] += t.z; O[i / 4][4 * (i % 4) + 3] += t.w;
+        }
+      }
+    }
+  }
   const float inv = __builtin_amdgcn_rcpf(dtot);
   // A lane holds four channels of one row per group: stored from here, an instruction would touch 32 rows with 16 bytes
   // each.  The rows of a wavefront go through LDS instead (the tile ring is free once every wavefront is past its last
   // P.V product) and leave as whole rows, 16 bytes per lane.
   constexpr int OROW = 2 * D + 16;                           // padded row: the 8-byte writes of 32 rows spread over the banks
-  static_assert(4 * 32 * OROW <= NBUF * (TILE + VTILE), "output rows of four wavefronts fit the tile ring");
+  static_assert(4 * 32 * OROW <= G * NBUF * (TILE + VTILE), "output rows of four wavefronts fit the tile ring");
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
+  if (grp > 0) return;
   unsigned char *const orow_lds = smem + wave * (32 * OROW);
 #pragma unroll
   for (int dt = 0; dt < NDT; dt++) {
@@ -823,23 +943,28 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   // Causal rows differ in length throughout: all rows by length while the heads an XCD works on at once share its L2
   // anyway (grids of a few rounds), head by head beyond.  Otherwise only a partial last Q block stands out.
   p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
-  if (p.v_scale != nullptr) {
-    if (D == 64) {
-      if (out_dtype == 0) block_sparse_attn_kernel<64, 0, false, SEL><<<grid, 256, 0, st>>>(p);
-      else block_sparse_attn_kernel<64, 1, false, SEL><<<grid, 256, 0, st>>>(p);
-    } else {
-      if (out_dtype == 0) block_sparse_attn_kernel<128, 0, false, SEL><<<grid, 256, 0, st>>>(p);
-      else block_sparse_attn_kernel<128, 1, false, SEL><<<grid, 256, 0, st>>>(p);
-    }
-  } else {   // fp16 V^T tiles, no V scale
-    if (D == 64) {
-      if (out_dtype == 0) block_sparse_attn_kernel<64, 0, true, SEL><<<grid, 256, 0, st>>>(p);
-      else block_sparse_attn_kernel<64, 1, true, SEL><<<grid, 256, 0, st>>>(p);
-    } else {
-      if (out_dtype == 0) block_sparse_attn_kernel<128, 0, true, SEL><<<grid, 256, 0, st>>>(p);
-      else block_sparse_attn_kernel<128, 1, true, SEL><<<grid, 256, 0, st>>>(p);
-    }
+  // A row alone on its CU: its blocks go over groups of wavefronts (kernel comment).  Three groups where registers allow and
+  // rows are long, two otherwise.  us per call with 1 / 2 / 3 groups: one head N17776 D64 281 / 236 / 225, H2 N16384 D64 131 /
+  // 111 / 105, D128 161 / 140 / -, FP16 PV D128 188 / 164 / -, H8 N4096 D64 45 / 41 / 41, D128 59 / 54 / -, H1 N2048 D64 28.3 / 26.7 /
+  // 27.2; H2 N256 18.0 / 18.6 / 19.9 (too few rounds for the exchange and the final sum).  Beyond one row per CU the rows fill
+  // each other's gaps: H10 N4096 unchanged without groups.
+  const bool groups = p.total_wg <= SPG_GROUPS_MAX_WG && p.nk >= SPG_GROUPS_MIN_NK && p.pv_mode == 1 && p.pv_count == nullptr;
+  const int n_groups = !groups ? 1 : D == 64 && p.nk > SPG_SELECT_IN_ATTN_NK ? 3 : 2;
+#define SPG_ATTN(D_, PV16_, G_)                                                                             \
+  {                                                                                                         \
+    if (out_dtype == 0) block_sparse_attn_kernel<D_, 0, PV16_, SEL, G_><<<grid, 256 * G_, 0, st>>>(p);       \
+    else block_sparse_attn_kernel<D_, 1, PV16_, SEL, G_><<<grid, 256 * G_, 0, st>>>(p);                      \
   }
+#define SPG_ATTN_G(D_, PV16_)                                                                               \
+  {                                                                                                         \
+    if (n_groups == 1) SPG_ATTN(D_, PV16_, 1)                                                                \
+    else if (n_groups == 2) SPG_ATTN(D_, PV16_, 2)                                                           \
+    else if constexpr (D_ == 64 && !SEL) SPG_ATTN(D_, PV16_, 3)                                              \
+  }
+  if (p.v_scale != nullptr) { if (D == 64) SPG_ATTN_G(64, false) else SPG_ATTN_G(128, false) }
+  else { if (D == 64) SPG_ATTN_G(64, true) else SPG_ATTN_G(128, true) }   // fp16 V^T tiles, no V scale
+#undef SPG_ATTN_G
+#undef SPG_ATTN
   return hipGetLastError();
 }
 
