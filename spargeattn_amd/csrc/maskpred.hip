@@ -276,18 +276,20 @@ __global__ __launch_bounds__(256) void block_select_kernel(
 // block_select, wavefront-per-row variant (nk <= 2048).
 // Phase 1 computes the scores of 16 pooled-Q rows against all pooled-K rows on the matrix unit in binary64
 // (v_mfma_f64_16x16x4_f64: operands are delivered once per 1024 multiply-adds instead of once per multiply-add) and
-// leaves them in LDS as 16-bit patterns.  Phase 2 gives each of the four wavefronts its own rows and keeps a whole row
+// leaves them in LDS as 16-bit patterns.  Phase 2 gives each of the eight wavefronts its own rows (one of R = 8, two of
+// R = 16) and keeps a whole row
 // in registers (EPL = nkp / 64 columns per lane): no workgroup barrier, the stable descending sort is a bitonic network
 // whose short-distance steps are register-local and whose long-distance steps are lane exchanges.
-// dynamic LDS: 16*nkp*2 (scores) + 4*nkp*4 (per-wave index list) + 4*64*8 (lane sums).
+// dynamic LDS: R*nkp*2 (scores) + 8*nkp*2 (per-wave index list) + 8*64*8 (lane sums).
 // =============================================================================================
-template <int D, int DT, int NW, int EPL, bool DUAL>
+template <int D, int DT, int NW, int EPL, bool DUAL, int R>
 __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_select_wave_kernel(
     const uint16_t *__restrict__ pool_q, const uint8_t *__restrict__ sim_q, const uint16_t *__restrict__ pool_k,
     const uint8_t *__restrict__ sim_k, const bool by_topk, const Hyper level, int is_causal,
     int sink, int32_t *__restrict__ lut, int32_t *__restrict__ valid, uint8_t *__restrict__ bmap, int H, int Hkv, int nq,
     int nk) {
-  constexpr int R = 16;             // rows per workgroup: phase 1 computes 16 x 16 score tiles on the matrix unit
+  // R rows per workgroup; phase 1 computes 16 x 16 score tiles on the matrix unit, of which R = 8 uses the first 8 rows
+  static_assert(R == 16 || R == 8, "rows per workgroup");
   constexpr int NKP = 64 * EPL;
   static_assert(NW == 8 || NW == 16, "wavefronts per workgroup");
   extern __shared__ __align__(16) unsigned char smem[];
@@ -347,7 +349,7 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
       const int j = 16 * ct + c;
       const bool dead = j >= nk || simk[min(j, nk - 1)] == 0;
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
+      for (int v = 0; v < R / 4; v++) {
         const int row = g + 4 * v;
         const float a1 = elem_to_f32<DT>(f64_to_elem_fast<DT>(acc[v]));
         uint16_t a2 = f64_to_elem_fast<DT>((double)a1 * (double)sm_scale);
@@ -397,7 +399,7 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
     for (int t2 = live_tiles + wave; t2 < n_tiles; t2 += NW) {
       const int j = 16 * t2 + c;
 #pragma unroll
-      for (int v = 0; v < 4; v++) s_scores[(size_t)(g + 4 * v) * NKP + j] = NEG_INF;
+      for (int v = 0; v < R / 4; v++) s_scores[(size_t)(g + 4 * v) * NKP + j] = NEG_INF;
     }
   }
   __syncthreads();
@@ -719,24 +721,27 @@ static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, 
   const int nkp = next_pow2_ge(nk, 256);
   if (nkp <= 2048) {
     // a whole row fits the registers of one wavefront
-#define SPG_BSW(NW_, EPL_, DUAL_)                                                                                    \
+#define SPG_BSW(NW_, EPL_, DUAL_, R_)                                                                                    \
     {                                                                                                           \
-      const size_t lds = (size_t)16 * nkp * 2 + (size_t)NW_ * nkp * 2 + NW_ * 64 * 8;                           \
-      auto kern = block_select_wave_kernel<D, DT, NW_, EPL_, DUAL_>;                                                   \
+      const size_t lds = (size_t)R_ * nkp * 2 + (size_t)NW_ * nkp * 2 + NW_ * 64 * 8;                           \
+      auto kern = block_select_wave_kernel<D, DT, NW_, EPL_, DUAL_, R_>;                                                   \
       {                                                                                                         \
-        hipError_t e = allow_dynamic_lds<block_select_wave_kernel<D, DT, NW_, EPL_, DUAL_>>(lds);                      \
+        hipError_t e = allow_dynamic_lds<block_select_wave_kernel<D, DT, NW_, EPL_, DUAL_, R_>>(lds);                      \
         if (e != hipSuccess) return e;                                                                          \
       }                                                                                                         \
-      kern<<<dim3((nq + 15) / 16, B * H), 64 * NW_, lds, st>>>((const uint16_t *)pq, sq, (const uint16_t *)pk, sk, by_topk, \
+      kern<<<dim3((nq + R_ - 1) / R_, B * H), 64 * NW_, lds, st>>>((const uint16_t *)pq, sq, (const uint16_t *)pk, sk, by_topk, \
                                                                level, causal, sink, lut, valid, bmap, H, Hkv, nq, nk); \
       return hipSuccess;                                                                                        \
     }
-    // one wavefront per row (16 per workgroup) where a row's registers fit the 128 a 1024-thread workgroup leaves each
-    // lane, two rows per wavefront beyond
-    if (nkp == 256) SPG_BSW(8, 4, false)
-    if (nkp == 512) SPG_BSW(8, 8, false)
-    if (nkp == 1024) SPG_BSW(8, 16, false)
-    SPG_BSW(8, 32, true)
+    // Eight rows instead of sixteen per workgroup, one per wavefront, where sixteen leave a CU with little more than one
+    // workgroup: the time is then that of one wavefront's rows, and the half-empty score tiles cost less than the second row.
+    // us with 16 / 8: 9 workgroups D=64 nk=278 CDF 28.0 / 18.1, 96 D=128 nk=128 15.3 / 10.4, 128 D=128 nk=256 25.4 / 16.9, 192 D=64
+    // nk=256 21.5 / 18.2, 270 D=64 nk=278 44.0 / 35.7, 49 D=128 nk=1563 130 / 85; 512 D=128 nk=512 46.6 / 64.1.
+    const bool few = (nq + 15) / 16 * B * H <= (D == 64 ? 384 : 256);
+    if (nkp == 256) { if (few) SPG_BSW(8, 4, false, 8) else SPG_BSW(8, 4, false, 16) }
+    if (nkp == 512) { if (few) SPG_BSW(8, 8, false, 8) else SPG_BSW(8, 8, false, 16) }
+    if (nkp == 1024) { if (few) SPG_BSW(8, 16, false, 8) else SPG_BSW(8, 16, false, 16) }
+    if (few) SPG_BSW(8, 32, true, 8) else SPG_BSW(8, 32, true, 16)
 #undef SPG_BSW
   }
   // rows per workgroup: reuse of the pooled-K reads against LDS footprint (scores are R*nkp floats)

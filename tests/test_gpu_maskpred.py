@@ -84,6 +84,22 @@ def test_block_select(dtype, nq, nk, D, mode):
     assert np.array_equal(valid.cpu().numpy(), ref_valid)
     assert np.array_equal(lut.cpu().numpy(), ref_lut)
 
+@pytest.mark.parametrize("nq,nk,D", [(20, 40, 64), (17, 300, 128), (8, 700, 64), (25, 1100, 128)])
+@pytest.mark.parametrize("by_topk", [True, False])
+def test_block_select_many_heads_equal_few(nq, nk, D, by_topk):
+    """Grids of many workgroups give a workgroup sixteen rows, small ones eight: the same rows come out the same."""
+    H = 400 // ((nq + 15) // 16)
+    pq, sq, pk, sk = _pools(1, H, nq, nk, D, torch.bfloat16, 60 + nq)
+    level = torch.linspace(0.2, 0.95, H, device="cuda")
+    kw = dict(topk=level) if by_topk else dict(cdfthreshd=level)
+    many = _lib.block_select(pq, sq, pk, sk, return_map=True, **kw)
+    few = 10
+    for h in range(0, H - few + 1, few * 13):
+        c = slice(h, h + few)
+        part = _lib.block_select(pq[:, c].contiguous(), sq[:, c].contiguous(), pk[:, c].contiguous(), sk[:, c].contiguous(),
+                                 return_map=True, **{k: v[c].contiguous() for k, v in kw.items()})
+        assert all(torch.equal(a[:, c], b) for a, b in zip(many, part))
+
 
 def test_block_select_rejects_bad_arguments():
     pq, sq, pk, sk = _pools(1, 1, 4, 8, 64, torch.float16, 5)
