@@ -55,6 +55,20 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define SPG_GROUPS_MIN_NK 12        // ... and K blocks from which a row gets groups of wavefronts
 #define SPG_LOG2E 1.44269504088896340736f
 
+// n / d for 0 <= n < 2^31 as a multiplication and a shift: m = ceil(2^(31+s) / d) with 2^(s-1) < d <= 2^s is a 32-bit number, and
+// m d - 2^(31+s) < d <= 2^s keeps the truncated product exact.  (A division by a launch argument is some 40 dependent
+// instructions; a workgroup needs six of them before it can ask for its data.)
+struct FastDiv {
+  uint32_t m, s;
+  static FastDiv of(int d) {
+    FastDiv f = {0, 0};
+    while ((1ll << f.s) < d) f.s++;
+    f.m = (uint32_t)(((1ull << (31 + f.s)) + (unsigned)d - 1) / (unsigned)d);
+    return f;
+  }
+  __device__ __forceinline__ int operator()(int n) const { return (int)(__umulhi((uint32_t)n << 1, m) >> s); }
+};
+
 struct AttnParams {
   const int8_t *q8, *k8;
   const uint8_t *v8;
@@ -71,6 +85,7 @@ struct AttnParams {
   int q_per_warp;  // QuantGranularity of Q (sm89.cuh:106-121): 0 one scale per 128-row block, 1 one per 32 rows (B,H,nq*4)
   int total_wg, wg_per_xcd;
   int *queue;      // NULL, or 8 counters, zero at the start (take_item)
+  FastDiv by_nq, by_rest, by_H, by_group;   // nq, nq - rows_first, H, H / Hkv
   int rows_first;  // so many of the longest rows of every head come before the rest (place_workgroup)
   RowSelect sel;   // selection inside the kernel (template argument SEL); lut is unused then
 };
@@ -87,11 +102,11 @@ __device__ __forceinline__ bool place_workgroup(const AttnParams &p, int xcd, in
   if (L0 + j >= L1) return false;
   const int nq = p.nq, T = p.rows_first;
   // the range is rows a.. of head h0 (if a > 0), all rows of F heads from hf on, rows ..b-1 of head h1 (if b > 0)
-  const int h0 = L0 / nq, a = L0 - h0 * nq, h1 = L1 / nq, b = L1 - h1 * nq;
+  const int h0 = p.by_nq(L0), a = L0 - h0 * nq, h1 = p.by_nq(L1), b = L1 - h1 * nq;
   const int hf = h0 + (a > 0 ? 1 : 0), F = h1 - hf;
   int h, t;
   if (T == 0 || F < 0) {
-    h = (L0 + j) / nq;
+    h = p.by_nq(L0 + j);
     t = L0 + j - h * nq;
   } else {
     auto upto = [&](int rows) { return F * rows + (a > 0 ? max(0, rows - a) : 0) + min(rows, b); };   // pairs with row < rows
@@ -111,7 +126,7 @@ __device__ __forceinline__ bool place_workgroup(const AttnParams &p, int xcd, in
       if (j < n0) { h = h0; t = max(a, T) + j; }
       else {
         j -= n0;
-        const int i = per > 0 ? j / per : 0;
+        const int i = per > 0 ? p.by_rest(j) : 0;
         h = hf + min(i, F);
         t = T + j - min(i, F) * per;
       }
@@ -257,9 +272,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     }
   }
   if (!place_workgroup(p, item & 7, item >> 3, bh, qb)) return;
-  const int head = bh % p.H;
+  const int batch = p.by_H(bh), head = bh - batch * p.H;
   // grouped-query attention: H / Hkv consecutive query heads share one K/V head (sm89.cuh:118, head_id / num_kv_groups)
-  const int bhk = (bh / p.H) * p.Hkv + head / (p.H / p.Hkv);
+  const int bhk = batch * p.Hkv + p.by_group(head);
 
   const int N = p.N, Nk = p.Nk;
   const int q_row = qb * 128 + wave * 32 + r;
@@ -924,7 +939,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   constexpr int LPR = D / 8, RPI = 64 / LPR;                 // lanes per row, rows per store instruction
-  uint16_t *obase = (uint16_t *)p.out + (size_t)(bh / p.H) * p.os.sb + (size_t)head * p.os.sh + (lane % LPR) * 8;
+  uint16_t *obase = (uint16_t *)p.out + (size_t)batch * p.os.sb + (size_t)head * p.os.sh + (lane % LPR) * 8;
 #pragma unroll
   for (int i = 0; i < 32 / RPI; i++) {
     const int row = i * RPI + lane / LPR, grow = qb * 128 + wave * 32 + row;
@@ -943,6 +958,8 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   // Causal rows differ in length throughout: all rows by length while the heads an XCD works on at once share its L2
   // anyway (grids of a few rounds), head by head beyond.  Otherwise only a partial last Q block stands out.
   p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
+  p.by_nq = FastDiv::of(p.nq); p.by_rest = FastDiv::of(p.nq > p.rows_first ? p.nq - p.rows_first : 1);
+  p.by_H = FastDiv::of(p.H); p.by_group = FastDiv::of(p.H / p.Hkv);
   // A row alone on its CU: its blocks go over groups of wavefronts (kernel comment).  Three groups where registers allow and
   // rows are long, two otherwise.  us per call with 1 / 2 / 3 groups: one head N17776 D64 281 / 236 / 225, H2 N16384 D64 131 /
   // 111 / 105, D128 161 / 140 / -, FP16 PV D128 188 / 164 / -, H8 N4096 D64 45 / 41 / 41, D128 59 / 54 / -, H1 N2048 D64 28.3 / 26.7 /

@@ -102,13 +102,6 @@ __device__ __forceinline__ uint4 load_stream_u4(const void *p) {
 // ---------------------------------------------------------------------------------------------
 // wavefront shuffles for 64-bit values
 // ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ double shfl_xor_f64(double v, int mask) {
-  uint64_t u = __builtin_bit_cast(uint64_t, v);
-  uint32_t lo = (uint32_t)u, hi = (uint32_t)(u >> 32);
-  lo = __shfl_xor(lo, mask, SPG_WAVE);
-  hi = __shfl_xor(hi, mask, SPG_WAVE);
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
 __device__ __forceinline__ long long shfl_xor_i64(long long v, int mask) {
   uint64_t u = (uint64_t)v;
   uint32_t lo = (uint32_t)u, hi = (uint32_t)(u >> 32);
@@ -166,15 +159,66 @@ __device__ __forceinline__ uint32_t group_and_u32(uint32_t v) {
   return v;
 }
 
+// Exchanges over the 64 lanes at VALU rate.  A __shfl_xor is an LDS round trip of 100 clocks and more, and the reductions
+// below are chains of six: they stand in the start-up of every row of the attention kernel.
+// Lane l receives the value of lane l ^ M.
+template <int M>
+__device__ __forceinline__ uint32_t lane_xor_u32(uint32_t v) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8, "inside a row of 16 lanes");
+  constexpr int CTRL = M == 1 ? 0xB1 : M == 2 ? 0x4E : M == 4 ? 0x141 : 0x128;   // quad permutes, half-row mirror (l ^ 7), rotate by 8
+  const int t = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+  return (uint32_t)(M == 4 ? __builtin_amdgcn_update_dpp(0, t, 0x1B, 0xf, 0xf, true) : t);        // ... and l ^ 3
+}
+// a = the value of the lane of the pair (l, l ^ M) whose bit M is clear, b = the other's, in both lanes
+template <int M>
+__device__ __forceinline__ void pair_of_u32(uint32_t v, uint32_t &a, uint32_t &b) {
+  static_assert(M == 16 || M == 32, "rows of 16 lanes");
+  a = v;
+  b = v;
+  if constexpr (M == 32) asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  else asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+template <int M>
+__device__ __forceinline__ double pair_sum_f64(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  uint32_t al, bl, ah, bh;
+  pair_of_u32<M>((uint32_t)u, al, bl);
+  pair_of_u32<M>((uint32_t)(u >> 32), ah, bh);
+  return __builtin_bit_cast(double, ((uint64_t)ah << 32) | al) + __builtin_bit_cast(double, ((uint64_t)bh << 32) | bl);
+}
+// v + (v of lane l ^ 32), then of l ^ 16, 8, 4, 2, 1: the fixed summation tree of the compressed softmax.  (Once the sums agree
+// across l ^ 8, a rotation by 4 reaches the value of lane l ^ 4.)
+__device__ __forceinline__ double wave_tree_sum_f64(double v) {
+  v = pair_sum_f64<32>(v);
+  v = pair_sum_f64<16>(v);
+  v += dpp_f64<0x128>(v);
+  v += dpp_f64<0x124>(v);
+  v += dpp_f64<0x4E>(v);
+  v += dpp_f64<0xB1>(v);
+  return v;
+}
 __device__ __forceinline__ float wave_max_f32(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, SPG_WAVE));
+  uint32_t a, b;
+  pair_of_u32<32>(__builtin_bit_cast(uint32_t, v), a, b);
+  v = fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+  pair_of_u32<16>(__builtin_bit_cast(uint32_t, v), a, b);
+  v = fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+  v = fmaxf(v, __builtin_bit_cast(float, lane_xor_u32<8>(__builtin_bit_cast(uint32_t, v))));
+  v = fmaxf(v, __builtin_bit_cast(float, lane_xor_u32<4>(__builtin_bit_cast(uint32_t, v))));
+  v = fmaxf(v, __builtin_bit_cast(float, lane_xor_u32<2>(__builtin_bit_cast(uint32_t, v))));
+  v = fmaxf(v, __builtin_bit_cast(float, lane_xor_u32<1>(__builtin_bit_cast(uint32_t, v))));
   return v;
 }
 __device__ __forceinline__ int wave_sum_i32(int v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, SPG_WAVE);
-  return v;
+  uint32_t a, b;
+  pair_of_u32<32>((uint32_t)v, a, b);
+  pair_of_u32<16>(a + b, a, b);
+  uint32_t s = a + b;
+  s += lane_xor_u32<8>(s);
+  s += lane_xor_u32<4>(s);
+  s += lane_xor_u32<2>(s);
+  s += lane_xor_u32<1>(s);
+  return (int)s;
 }
 
 }  // namespace spg

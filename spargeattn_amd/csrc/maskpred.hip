@@ -190,8 +190,7 @@ __global__ __launch_bounds__(256) void block_select_kernel(
     if (tid < 64) {
       double part = 0.0;
       for (int j = tid; j < nk; j += 64) part = part + e_buf[j];
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) part = part + shfl_xor_f64(part, o);
+      part = wave_tree_sum_f64(part);
       if (tid == 0) s_wsum[0] = part;
     }
     __syncthreads();
@@ -429,8 +428,7 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
       ev[t] = (sc[t] == -INFINITY) ? 0.0 : cexp((double)sc[t] - (double)mx);
       part = part + ev[t];
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) part = part + shfl_xor_f64(part, o);
+    part = wave_tree_sum_f64(part);
     const double total = part;
 
     // probabilities -> sortable keys (value bits, then lower column first).  The 16-bit pattern of e / total is taken

@@ -43,8 +43,10 @@ __device__ __forceinline__ void bitonic_step(uint32_t (&key)[EPL], int lane) {
     const bool want_max = lower == desc;
 #pragma unroll
     for (int t = 0; t < EPL; t++) {
-      const uint32_t o = (uint32_t)__shfl_xor((int)key[t], DL, SPG_WAVE);
-      const uint32_t mx = key[t] > o ? key[t] : o, mn = key[t] > o ? o : key[t];
+      uint32_t o, own = key[t];
+      if constexpr (DL >= 16) pair_of_u32<DL>(own, own, o);        // (the maximum and the minimum do not ask which is whose)
+      else o = lane_xor_u32<DL>(own);
+      const uint32_t mx = own > o ? own : o, mn = own > o ? o : own;
       key[t] = want_max ? mx : mn;
     }
   } else {
@@ -117,9 +119,7 @@ __device__ __forceinline__ uint64_t select_row64(float sc, bool k_dead, bool by_
 #pragma clang fp contract(off)
   const float mx = wave_max_f32(sc);
   const double ev = (sc == -INFINITY) ? 0.0 : cexp((double)sc - (double)mx);
-  double total = ev;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) total = total + shfl_xor_f64(total, o);
+  const double total = wave_tree_sum_f64(ev);
   double p = ev / total;
   if (!__builtin_isfinite(p)) p = 0.0;
   const uint32_t okey = lane < nk ? (((uint32_t)f64_to_elem_fast<DT>(p) << 16) | (0xffffu - (uint32_t)lane)) : 0u;
