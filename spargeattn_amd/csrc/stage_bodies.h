@@ -112,6 +112,25 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return v;
 }
 
+// Sums of eight columns over the four 16-lane rows of a wavefront (bits 4 and 5 of the lane): half the columns change places
+// with the other half's lanes, the two add up, and again.  Lane l ends with columns 4 * bit 5 + 2 * bit 4 + {0, 1}: a quarter
+// of the LDS space and of its writes and reads for the rest of the column sum.  (With the full set in LDS, 32 KiB held a CU
+// to four workgroups of the back kernel: 30 heads N17776 D64 55.8 us, with 10 KiB and word-wide V tile writes 44.0 us.)
+template <int M>
+__device__ __forceinline__ double swap_add_f64(double a, double b) {
+  const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+  uint32_t al = (uint32_t)ua, ah = (uint32_t)(ua >> 32), bl = (uint32_t)ub, bh = (uint32_t)(ub >> 32);
+  if constexpr (M == 32) asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_permlane32_swap_b32 %2, %3" : "+v"(al), "+v"(bl), "+v"(ah), "+v"(bh));
+  else asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3" : "+v"(al), "+v"(bl), "+v"(ah), "+v"(bh));
+  return __builtin_bit_cast(double, ((uint64_t)ah << 32) | al) + __builtin_bit_cast(double, ((uint64_t)bh << 32) | bl);
+}
+__device__ __forceinline__ double2 fold_columns(const double (&x)[8]) {
+  double y[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) y[i] = swap_add_f64<32>(x[i], x[i + 4]);
+  return make_double2(swap_add_f64<16>(y[0], y[2]), swap_add_f64<16>(y[1], y[3]));
+}
+
 // One workgroup handles ROWS consecutive rows of one (batch, head), by default 128: one 128-row block or two 64-row blocks (SUB), so
 // that the per-block tail (column reduction, pooled mean, flag, scale) is spread over all four wavefronts in both cases.
 // QR = rows that share one INT8 scale: BS (per-block granularity, what the reference's operators use) or 32 rows of a
@@ -123,7 +142,7 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 enum { MEAN_NONE = 0, MEAN_GIVEN = 1, MEAN_PARTIAL = 2 };
 // NT threads work on ROWS rows: 256 on 128 where there are enough workgroups to fill the chip, more threads on fewer rows
 // where there are not and the time is the length of one thread's work.
-template <int BS, int D, int NT = 256, int ROWS = 128> constexpr int psq_lds() { return ROWS / BS * (NT / (D / 8)) * D * 8; }
+template <int BS, int D, int NT = 256, int ROWS = 128> constexpr int psq_lds() { return ROWS / BS * (NT / 64 * 128 / D) * D * 8; }
 template <int BS, int D, int DT, int MEAN, bool WITH_POOL, int QR = BS, int NT = 256, int ROWS = 128>
 __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const Strides &xs,
                                          const uint16_t *__restrict__ km, const double *__restrict__ km_part, int km_chunks,
@@ -278,9 +297,12 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
   }
 
   if constexpr (WITH_POOL) {
-    // column sums of all blocks of the workgroup, one row group per line; used for the pooled mean first and, with a
+    // column sums of all blocks of the workgroup, one line per wavefront (two at D = 64: fold_columns); used for the pooled mean first and, with a
     // non-negative similarity threshold, for the normalised rows afterwards
-    double(*s_red)[RPP][D] = (double(*)[RPP][D])smem;
+    constexpr int RG = NWV * 128 / D;
+    double(*s_red)[RG][D] = (double(*)[RG][D])smem;
+    const int rg = D == 128 ? tid >> 6 : tid >> 6 << 1 | (tid >> 3 & 1);
+    const int rg_col = c * 8 + (tid >> 5 & 1) * 4 + (tid >> 4 & 1) * 2;
     // column sums for the pooled mean: binary64, exact
 #pragma unroll
     for (int sb = 0; sb < SUB; sb++) {
@@ -297,8 +319,7 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
           colsum[2 * j] += (double)f0;
           colsum[2 * j + 1] += (double)f1;
         }
-#pragma unroll
-      for (int e = 0; e < 8; e++) s_red[sb][r][c * 8 + e] = colsum[e];
+      *(double2 *)&s_red[sb][rg][rg_col] = fold_columns(colsum);
     }
 
     // row norms: the TPR lanes of a row group all need sqrt(sum of squares) and its reciprocal for each of their NPT
@@ -351,7 +372,8 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
     const int t_rows = rows_valid_of(t_sb);
     if (t_on && t_rows > 0) {
       double s = 0.0;
-      for (int i = 0; i < RPP; i++) s += s_red[t_sb][i][t_col];
+      #pragma unroll
+      for (int i = 0; i < RG; i++) s += s_red[t_sb][i][t_col];
       // full blocks: the row count is a power of two, so the product with its reciprocal is the exact quotient
       const double mean = t_rows == BS ? s * (1.0 / BS) : s / (double)t_rows;
       pool[((size_t)bh * nb + blk0 + t_sb) * D + t_col] = f64_to_elem_fast<DT>(mean);
@@ -384,13 +406,13 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
             colxh[2 * j + 1] += (double)(float)h1;
           }
         }
-#pragma unroll
-        for (int e = 0; e < 8; e++) s_red[sb][r][c * 8 + e] = colxh[e];
+        *(double2 *)&s_red[sb][rg][rg_col] = fold_columns(colxh);
       }
       __syncthreads();
       if (t_on) {
         double sx = 0.0;
-        for (int i = 0; i < RPP; i++) sx += s_red[t_sb][i][t_col];
+        #pragma unroll
+        for (int i = 0; i < RG; i++) sx += s_red[t_sb][i][t_col];
         if (__builtin_isfinite(sx)) {
           const long long si = (long long)(sx * 16777216.0);   // exact integer
           g = si * si;
@@ -633,32 +655,38 @@ __device__ __forceinline__ void v_quant_body(const uint16_t *__restrict__ v, con
   constexpr int TPR = D / 8;
   constexpr int RPP = NT / TPR;
   constexpr int NP = 64 / RPP;
+  static_assert(NP == 1 || NP == 2 || NP == 4, "rows per thread");
   constexpr int LDW = 64 + 4;  // padded row (bytes) of the transposed tile
   uint8_t *tile = smem;
   const int tid = threadIdx.x;
   const int c = tid % TPR, r = tid / TPR;
   const uint16_t *base = v + (size_t)(bh / H) * vs.sb + (size_t)(bh % H) * vs.sh + (size_t)blk * 64 * vs.sn + c * 8;
   const int last_row = min(63, N - 1 - blk * 64);
+  // A thread takes NP neighbouring rows, so that their codes of one channel leave as one LDS word.
   uint4 raw[NP];                     // every load is issued before the first use; rows beyond N re-read the last row
 #pragma unroll
-  for (int p = 0; p < NP; p++) raw[p] = load_stream_u4(base + (size_t)min(r + p * RPP, last_row) * vs.sn);
+  for (int p = 0; p < NP; p++) raw[p] = load_stream_u4(base + (size_t)min(r * NP + p, last_row) * vs.sn);
   float recp[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) recp[e] = 2.25f / amax_of(c * 8 + e);
 #pragma unroll
-  for (int p = 0; p < NP; p++) {
-    const int row = r + p * RPP;
-    const bool ok = row <= last_row;
-    const uint4 q = raw[p];
-    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+  for (int e = 0; e < 8; e++) {
+    float x[4];
 #pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      const float a = elem_to_f16_f32<DT>((uint16_t)(w[e >> 1] & 0xffffu)) * recp[e];
-      const float b = elem_to_f16_f32<DT>((uint16_t)(w[e >> 1] >> 16)) * recp[e + 1];
-      const int pk = ok ? __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) : 0;   // rows beyond N are zero
-      tile[(c * 8 + e) * LDW + row] = (uint8_t)(pk & 0xff);
-      tile[(c * 8 + e + 1) * LDW + row] = (uint8_t)((pk >> 8) & 0xff);
+    for (int p = 0; p < 4; p++) {
+      x[p] = 0.f;
+      if (p < NP) {
+        const uint32_t w[4] = {raw[p % NP].x, raw[p % NP].y, raw[p % NP].z, raw[p % NP].w};
+        x[p] = elem_to_f16_f32<DT>((uint16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu))) * recp[e];
+        if (r * NP + p > last_row) x[p] = 0.f;                        // rows beyond N are zero
+      }
     }
+    int pk = __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false);
+    if constexpr (NP == 4) pk = __builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], pk, true);
+    uint8_t *const dst = tile + (c * 8 + e) * LDW + r * NP;
+    if constexpr (NP == 4) *(uint32_t *)dst = (uint32_t)pk;
+    else if constexpr (NP == 2) *(uint16_t *)dst = (uint16_t)pk;
+    else *dst = (uint8_t)pk;
   }
   __syncthreads();
   uint8_t *out = v8 + ((size_t)bh * nk + blk) * (size_t)(D * 64);
