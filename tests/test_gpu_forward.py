@@ -101,3 +101,15 @@ def test_every_row_is_placed_once(H, N):
         o, o2 = _both(lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.6, is_causal=causal))
         assert torch.equal(_bits(o), _bits(o2))
         assert torch.isfinite(o.float()).all() and (o != 0).any(-1).all()
+
+
+@pytest.mark.parametrize("Nk", [8193, 12288, 12289])
+@pytest.mark.parametrize("D", [64, 128])
+def test_few_long_heads_combine_partial_sums(D, Nk):
+    """Up to 24576 key/value rows in all, longer heads get 32 chunks that every workgroup adds up (here up to 12288 rows of two
+    heads); one row more goes through the launch in between."""
+    q = rand_T((1, 2, 130, D), torch.bfloat16, 31)
+    k, v = rand_T((1, 2, Nk, D), torch.bfloat16, 32, shift=0.3), rand_T((1, 2, Nk, D), torch.float16, 33)
+    for fn in (sa.spas_sage2_attn_meansim_topk_cuda, sa.spas_sage_attn_meansim_topk_cuda):
+        o, o2 = _both(lambda: fn(q, k, v, topk=0.3, simthreshd1=0.1))
+        assert torch.equal(_bits(o), _bits(o2))
