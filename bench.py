@@ -29,8 +29,8 @@ PEAK_HBM = 8.0e12
 # was measured on AND for the kernel source it was measured with: the entry carries the SHA-256 of csrc/attn.hip at
 # the time of the measurement, and the bench line reports the figure only while the source still has that digest.
 MEASURED_ATTN_TRAFFIC = {
-    "cfg4": {"bytes": int((1.894 + 0.250) * 2 ** 30), "attn_hip_sha256": "9d3835bafde519dec8ed5b1f64fe12aa40221642b738c159112c255c267f55b1",
-             "profile": "profiles/cfg4_attn_kernel_pmc.md"},
+    "cfg4": {"bytes": int((2.236 + 0.250) * 2 ** 30), "attn_hip_sha256": "f2f2db4f8aec43ccc60ddd51b4cf40bf2e451ad7907cbb7074ac46e1bec4e8fc",
+             "profile": "profiles/operator_kernel_trace.md"},
 }
 
 
