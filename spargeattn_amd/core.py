@@ -184,6 +184,8 @@ def _hyper(value, H, device):
 
 def _run(q, k, v, mask, selection, level, simthreshd1, pvthreshd, is_causal, attention_sink, kernel_causal, pv_f16,
          scale, tensor_layout, return_sparsity, qk_quant_gran, causal_denominator):
+    # the key and the plan hold the scale's value at this call: a tensor would compare by identity, an array not at all
+    scale = None if scale is None else float(scale)
     key = (q.shape, k.shape, v.shape, q.stride(), k.stride(), v.stride(), q.dtype, k.dtype, v.dtype, q.device, k.device,
            v.device, None if mask is None else (mask.shape, mask.dtype, mask.device, mask.is_contiguous()), selection,
            bool(is_causal), bool(attention_sink), bool(kernel_causal), pv_f16, scale, tensor_layout, qk_quant_gran)

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from spargeattn_amd import utils, workloads as W
+from spargeattn_amd import _lib, utils, workloads as W
 import spargeattn_amd as sa
 
 
@@ -59,7 +59,6 @@ def test_workload_generators_shapes_and_determinism():
 
 def test_attention_wrapper_rejects_inconsistent_shapes_before_any_launch():
     """The kernels index K, V, the LUT and the scales with ceil(kv_len/64): shapes that disagree must raise on the host."""
-    from spargeattn_amd import _lib
     B, H, N, Nk, D = 1, 2, 256, 320, 64
     nq, nk = 2, 5
     q8 = torch.zeros((B, H, N, D), dtype=torch.int8)
@@ -120,3 +119,50 @@ def test_build_names_the_compiler_it_was_validated_with(monkeypatch):
     monkeypatch.delenv("SPARGEATTN_AMD_ALLOW_UNVALIDATED_COMPILER", raising=False)
     with pytest.raises(RuntimeError, match="not a validated version"):
         b.build(verbose=False)
+
+
+class _StandInPlan:
+    """Takes the place of _lib.ForwardPlan where no GPU is needed to see what a call would hand over: each run records the
+    plan's softmax scale."""
+    ran = []
+
+    def __init__(self, q, k, v, out, mask, selection, pv_f16, is_causal, attention_sink, kernel_causal, qk_quant_gran, sm_scale):
+        self.sm_scale = _lib.AttnArgs(sm_scale=sm_scale).sm_scale       # the argument block holds a number
+        self.device, self.device_index = q.device, 0
+        self.nk, self.valid_shape = (k.shape[2] + 63) // 64, (q.shape[0], q.shape[1], (q.shape[2] + 127) // 128)
+        self.template = type("Template", (), {"Hkv": k.shape[1]})
+
+    def run(self, q, k, v, out, mask, level, simthreshd1, pvthreshd, return_valid=False):
+        self.ran.append(self.sm_scale)
+
+
+@pytest.fixture
+def stand_in_plans(monkeypatch):
+    from spargeattn_amd import core
+    monkeypatch.setattr(core, "_prologue", lambda q, k, v, layout: (q, k, v))
+    monkeypatch.setattr(core, "_plans", {})
+    monkeypatch.setattr(_lib, "ForwardPlan", _StandInPlan)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(_StandInPlan, "ran", [])
+    return core._plans
+
+
+def test_softmax_scale_is_read_on_every_call(stand_in_plans):
+    """A scale that is a tensor or an array counts with the value it has at the call (a learned temperature is updated in
+    place); a number, a 0-d tensor and a 0-d array of one value share a plan."""
+    import numpy as np
+    q = torch.zeros(1, 2, 128, 64, dtype=torch.float16)
+    scale = torch.tensor(0.125)
+    sa.spas_sage2_attn_meansim_topk_cuda(q, q, q, scale=scale)
+    scale.fill_(0.25)
+    sa.spas_sage2_attn_meansim_topk_cuda(q, q, q, scale=scale)
+    assert _StandInPlan.ran == [0.125, 0.25]
+    array = np.array(0.5)
+    for s in (array, 0.5, torch.tensor(0.5), torch.tensor([0.5])):
+        sa.spas_sage2_attn_meansim_topk_cuda(q, q, q, scale=s)
+    array.fill(2.0)
+    sa.block_sparse_sage2_attn_cuda(q, q, q, mask_id=torch.ones(1, 2, 1, 2), scale=array)
+    sa.spas_sage_attn_meansim_cuda(q, q, q)
+    assert _StandInPlan.ran[2:] == [0.5] * 4 + [2.0, 0.125]
+    assert len(stand_in_plans) == 5
+    assert not any(isinstance(part, (torch.Tensor, np.ndarray)) for key in stand_in_plans for part in key)
