@@ -345,6 +345,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   // K: LDS chunk position pos <-> (row = pos / CPR, slot = pos % CPR) holds global chunk slot ^ k_swz(row).
   // A tile's global address is (uniform base of the block) + (per-lane 32-bit offset) + u*1024, and the same
   // u*1024 is the LDS offset: it rides in the instruction's immediate (applied to both addresses).
+  // The base is a 64-bit shift of the block number: the tiles of one head may span more than 4 GiB.
   // (the two per-lane offsets are recomputed from the thread id where they are used: cheaper than keeping them
   //  in registers across the loop, where the register file is the scarce resource)
   // Split into a part that depends on the lane only (recomputed with three or four vector instructions where it is
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   typedef const __attribute__((address_space(1))) void *glb_ptr_t;
 #define SPG_LOAD_K_(BLK, KOFF, CHK)   /* inside a scope that holds SPG_LANE_OFFSETS() */                            \
   {                                                                                                           \
-    const int8_t *kb_ = kbase + (size_t)((uint32_t)(BLK) * (uint32_t)TILE);                                                         \
+    const int8_t *kb_ = kbase + (size_t)(uint32_t)(BLK) * TILE;                                                 \
     unsigned char *lk_ = sKr + (KOFF) + WL * wave * 1024;                                                     \
     if (CHK == 0 || (BLK) != last_partial_blk) {                                                              \
       /* the loads of one tile back to back: they share the LDS base register (M0) */                          \
@@ -385,7 +386,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   }
 #define SPG_LOAD_V_(BLK, VOFF)                                                                                \
   {                                                                                                           \
-    const uint8_t *vb_ = vbase + (size_t)((uint32_t)(BLK) * (uint32_t)VTILE);                                                       \
+    const uint8_t *vb_ = vbase + (size_t)(uint32_t)(BLK) * VTILE;                                               \
     unsigned char *lv_ = sVr + (VOFF) + WLV * wave * 1024;                                                    \
     __builtin_amdgcn_global_load_lds((glb_ptr_t)(vb_ + v_lane), (lds_ptr_t)lv_, 16, 0, 0);                    \
     if constexpr (WLV >= 2)                                                                                   \

@@ -458,6 +458,50 @@ def test_query_and_key_lengths_differ():
         sa.spas_sage2_attn_meansim_topk_cuda(q, k, v[:, :, :128])
 
 
+@pytest.mark.parametrize("count", [False, True])
+@pytest.mark.parametrize("fp16v", [False, True])
+def test_tiles_of_a_head_beyond_four_gib(fp16v, count):
+    """A row that keeps the first and the last blocks of a head whose V^T tiles (FP8 PV: K tiles as well) span a little more
+    than 2^32 bytes: the same bits as over those blocks alone, in the general kernel (PV counts asked for) and with groups."""
+    D, nk = 128, (1 << (18 if fp16v else 19)) + 12
+    cols = torch.cat([torch.arange(12), torch.arange(nk - 24, nk)])
+    g = torch.Generator().manual_seed(11)
+    n = len(cols)
+    k_few = torch.randint(-127, 128, (n, 64, D), generator=g, dtype=torch.int8).cuda()
+    if fp16v:
+        v_few = torch.randn((n, D, 64), generator=g).to(torch.float16).cuda()
+    else:
+        v_few = (torch.randint(0, 0x70, (n, D, 64), generator=g) + 128 * torch.randint(0, 2, (n, D, 64), generator=g)).to(torch.uint8).cuda()
+    ks_few = (1e-3 * (1 + torch.rand(n, generator=g))).cuda()
+    N = 200
+    q8 = torch.randint(-127, 128, (1, 1, N, D), generator=g, dtype=torch.int8).cuda()
+    qs = torch.full((1, 1, 2), 0.02, device="cuda")
+    thr, vs = torch.full((1,), 50.0, device="cuda"), torch.ones((1, 1, D), device="cuda")
+
+    def run(total, where):
+        k8 = torch.zeros((1, 1, total * 64, D), dtype=torch.int8, device="cuda")
+        vt = torch.zeros((1, 1, total, D, 64), dtype=v_few.dtype, device="cuda")
+        ks = torch.full((1, 1, total), 1e-3, device="cuda")
+        at = where.cuda()
+        k8.view(total, 64, D)[at], vt[0, 0, at], ks[0, 0, at] = k_few, v_few, ks_few
+        lut = torch.zeros((1, 1, 2, total), dtype=torch.int32, device="cuda")
+        lut[..., :n] = torch.diff(where, prepend=torch.zeros(1, dtype=where.dtype)).to(torch.int32).cuda()
+        valid = torch.full((1, 1, 2), n, dtype=torch.int32, device="cuda")
+        o = torch.empty((1, 1, N, D), dtype=torch.bfloat16, device="cuda")
+        k8 = k8[:, :, :total * 64 - 9]                 # a partial last block (the slice of one head stays contiguous)
+        if fp16v:
+            pvc = _lib.block_sparse_attn_f16v(q8, k8, vt, o, lut, valid, thr, qs, ks, D ** -0.5, return_pv_count=count)
+        else:
+            pvc = _lib.block_sparse_attn(q8, k8, vt, o, lut, valid, thr, qs, ks, vs, D ** -0.5, return_pv_count=count)
+        return o, pvc
+
+    far, far_count = run(nk, cols)
+    near, near_count = run(n, torch.arange(n))
+    assert torch.isfinite(near.float()).all() and (near != 0).any()
+    assert torch.equal(far.view(torch.int16), near.view(torch.int16))
+    assert not count or torch.equal(far_count, near_count)
+
+
 def test_fp8_denominator_and_offset_construction():
     """The kernel on the closed-form construction that separates "fp32 P in the denominator, e4m3(P) in the numerator,
     offset 8.807" from "rounded P in the denominator" and from "no offset" (see tests/gpu_common.py)."""
