@@ -2,6 +2,7 @@
 // stream.  No allocation, no synchronisation; the only state is the thread-local error string and, behind
 // spg_km_mean_static, a library-owned device array per GPU with its cached address.
 #include "capi_checks.h"
+#include "forward_plan.h"
 
 #include <cstdarg>
 #include <cstdio>
@@ -191,6 +192,47 @@ int spg_block_sparse_attn_f16v(const int8_t *q8, const int8_t *k8, const void *v
                                                         pvthreshd, q_scale, k_scale, nullptr, B, H, Hkv, N, N_kv, D, sm_scale,
                                                         is_causal ? 1 : 0, qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0,
                                                         pv_threshold_mode, pv_count, (hipStream_t)stream));
+}
+
+static int check_forward(const char *fn, const spg_attn_args *a) {
+  SPG_TRY(check_shape(fn, a->B, a->H, a->N, a->D));
+  SPG_TRY(check_shape(fn, a->B, a->Hkv > 0 ? a->Hkv : 1, a->N_kv, a->D));
+  SPG_TRY(check_kv_heads(fn, a->H, a->Hkv));
+  SPG_TRY(check_dtype(fn, a->qk_dtype));
+  SPG_TRY(check_dtype(fn, a->v_dtype));
+  SPG_TRY(check_quant_gran(fn, a->qk_quant_gran));
+  if (a->selection < SPG_SELECT_TOPK || a->selection > SPG_SELECT_MASK)
+    return fail(SPG_ERR_INVALID, "%s: selection must be 0 (top-k), 1 (CDF) or 2 (mask), got %d", fn, a->selection);
+  const int nk = (a->N_kv + 63) / 64;
+  if (a->selection == SPG_SELECT_MASK) {
+    if (a->mask_kind < SPG_MASK_I8 || a->mask_kind > SPG_MASK_F64) return fail(SPG_ERR_INVALID, "%s: bad mask_kind %d", fn, a->mask_kind);
+    if (nk > 32768) return fail(SPG_ERR_UNSUPPORTED, "%s: nk = %d exceeds the supported maximum 32768", fn, nk);
+  } else if (nk > spg::block_select_max_nk()) {
+    return fail(SPG_ERR_UNSUPPORTED, "%s: nk = %d exceeds the supported maximum %d", fn, nk, spg::block_select_max_nk());
+  }
+  return SPG_OK;
+}
+
+size_t spg_sparse_attn_workspace_bytes(const spg_attn_args *args) {
+  if (args == nullptr || check_forward("spg_sparse_attn_workspace_bytes", args) != SPG_OK) return 0;
+  return layout_for(args).total;
+}
+
+int spg_sparse_attn(const spg_attn_args *args, void *stream) {
+  const char *fn = "spg_sparse_attn";
+  SPG_NONNULL(fn, args);
+  const spg_attn_args *a = args;
+  SPG_TRY(check_forward(fn, a));
+  SPG_NONNULL(fn, a->q); SPG_NONNULL(fn, a->k); SPG_NONNULL(fn, a->v); SPG_NONNULL(fn, a->out); SPG_NONNULL(fn, a->workspace);
+  if (a->selection == SPG_SELECT_MASK) SPG_NONNULL(fn, a->mask);
+  const size_t need = layout_for(a).total;
+  if (a->workspace_bytes < need) return fail(SPG_ERR_INVALID, "%s: workspace of %zu bytes, %zu needed", fn, (size_t)a->workspace_bytes, need);
+  Strides qs, ks, vs, os;
+  SPG_TRY(get_strides(fn, "q_strides", a->q_strides, a->H, a->N, a->D, &qs));
+  SPG_TRY(get_strides(fn, "k_strides", a->k_strides, a->Hkv, a->N_kv, a->D, &ks));
+  SPG_TRY(get_strides(fn, "v_strides", a->v_strides, a->Hkv, a->N_kv, a->D, &vs));
+  SPG_TRY(get_strides(fn, "out_strides", a->out_strides, a->H, a->N, a->D, &os));
+  return check_launch(fn, run_forward(a, qs, ks, vs, os, (hipStream_t)stream));
 }
 
 int spg_dense_attn_f16(const void *q, const void *k, const void *v, void *out, int B, int H, int N, int D,

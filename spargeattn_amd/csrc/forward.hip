@@ -11,8 +11,9 @@
 //   select   block_select_* of maskpred.hip (rows of more than 64 blocks; shorter ones are selected inside the next launch)
 //   attn     block_sparse_attn_kernel
 // Every body is the one the stage-by-stage entry points launch (stage_bodies.h): results are the same bits.
+// The extern "C" entry points and their argument checks are in capi.hip, the workspace layout in forward_plan.h.
 // Compile with -ffp-contract=off.
-#include "capi_checks.h"
+#include "forward_plan.h"
 #include "stage_bodies.h"
 
 namespace spg {
@@ -177,60 +178,6 @@ __global__ __launch_bounds__(NT) void back_kernel(const BackParams p) {
   }
 }
 
-// ---- workspace ----------------------------------------------------------------------------------------------------
-// Partial column sums / maxima: `chunks` workgroups per head.  Up to 8192 rows a head has at most sixteen chunks, few
-// enough to be combined by every workgroup of the back kernel (a few KiB from L2 against a launch of about 4.5 us);
-// beyond, the final kernel combines as many as it takes to spread the read over the chip - unless the heads are so few that
-// the back kernel's workgroups can read 32 chunks each for less than the launch (up to 24576 rows in all: at most 768
-// workgroups, 13 MB from L2 in one head N17776 D64, 205.2 us per call with the final kernel, 201.8 without).
-struct Chunks {
-  int n, rows;
-  bool partial;
-};
-static Chunks chunks_for(int heads, int N) {
-  Chunks c;
-  const bool few = (long long)heads * N <= 24576;
-  c.partial = N <= 8192 || few;
-  const int want = N <= 8192 ? 16 : few ? 32 : (2048 + heads - 1) / heads;
-  const int most = N <= 8192 ? (N + 63) / 64 : (N + 255) / 256;
-  c.n = want < most ? want : most;
-  c.rows = (N + c.n - 1) / c.n;
-  c.n = (N + c.rows - 1) / c.rows;      // no chunk without rows
-  return c;
-}
-
-struct Layout {
-  size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, queue, total;
-};
-static Layout layout_for(const spg_attn_args *a) {
-  Layout l;
-  size_t at = 0;
-  auto take = [&](size_t bytes) { const size_t r = at; at += (bytes + 255) / 256 * 256; return r; };
-  const size_t bh = (size_t)a->B * a->H, bhk = (size_t)a->B * a->Hkv, D = a->D;
-  const size_t nq = ((size_t)a->N + 127) / 128, nk = ((size_t)a->N_kv + 63) / 64;
-  const Chunks c = chunks_for((int)bhk, a->N_kv);
-  const bool pool = a->selection != SPG_SELECT_MASK;
-  l.km_part = take(bhk * c.n * D * 8);
-  l.v_part = take(a->pv_f16 ? 0 : bhk * c.n * D * 4);
-  l.km = take(bhk * D * 2);
-  l.v_amax = take(bhk * D * 4);
-  l.pool_q = take(pool ? bh * nq * D * 2 : 0);
-  l.pool_k = take(pool ? bhk * nk * D * 2 : 0);
-  l.sim_q = take(pool ? bh * nq : 0);
-  l.sim_k = take(pool ? bhk * nk : 0);
-  l.q8 = take(bh * a->N * D);
-  l.k8 = take(bhk * a->N_kv * D);
-  l.q_scale = take(bh * nq * 4 * (a->qk_quant_gran == SPG_QUANT_PER_WARP ? 4 : 1));
-  l.k_scale = take(bhk * nk * 4);
-  l.v = take(bhk * nk * 64 * D * (a->pv_f16 ? 2 : 1));
-  l.v_scale = take(bhk * D * 4);
-  l.lut = take(bh * nq * nk * 4);
-  l.valid = take(bh * nq * 4);
-  l.queue = take(8 * sizeof(int));
-  l.total = at;
-  return l;
-}
-
 template <int D, int DT, int NT>
 static void run_front_back(const spg_attn_args *a, const FrontParams &f, const BackParams &b, const Chunks &c, uint16_t *km, float *v_amax,
                            int front_wgs, int back_wgs, hipStream_t st) {
@@ -257,7 +204,7 @@ static void run_front_back(const spg_attn_args *a, const FrontParams &f, const B
   }
 }
 
-static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides &ks, const Strides &vs, const Strides &os,
+hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides &ks, const Strides &vs, const Strides &os,
                               hipStream_t st) {
   const Layout l = layout_for(a);
   unsigned char *ws = (unsigned char *)a->workspace;
@@ -333,52 +280,4 @@ static hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const S
                                     SPG_PV_PER_BLOCK, nullptr, pool && a->is_causal, f.queue, st);
 }
 
-static int check_args(const char *fn, const spg_attn_args *a) {
-  SPG_TRY(check_shape(fn, a->B, a->H, a->N, a->D));
-  SPG_TRY(check_shape(fn, a->B, a->Hkv > 0 ? a->Hkv : 1, a->N_kv, a->D));
-  SPG_TRY(check_kv_heads(fn, a->H, a->Hkv));
-  SPG_TRY(check_dtype(fn, a->qk_dtype));
-  SPG_TRY(check_dtype(fn, a->v_dtype));
-  SPG_TRY(check_quant_gran(fn, a->qk_quant_gran));
-  if (a->selection < SPG_SELECT_TOPK || a->selection > SPG_SELECT_MASK)
-    return fail(SPG_ERR_INVALID, "%s: selection must be 0 (top-k), 1 (CDF) or 2 (mask), got %d", fn, a->selection);
-  const int nk = (a->N_kv + 63) / 64;
-  if (a->selection == SPG_SELECT_MASK) {
-    if (a->mask_kind < SPG_MASK_I8 || a->mask_kind > SPG_MASK_F64) return fail(SPG_ERR_INVALID, "%s: bad mask_kind %d", fn, a->mask_kind);
-    if (nk > 32768) return fail(SPG_ERR_UNSUPPORTED, "%s: nk = %d exceeds the supported maximum 32768", fn, nk);
-  } else if (nk > block_select_max_nk()) {
-    return fail(SPG_ERR_UNSUPPORTED, "%s: nk = %d exceeds the supported maximum %d", fn, nk, block_select_max_nk());
-  }
-  return SPG_OK;
-}
-
 }  // namespace spg
-using namespace spg;
-
-#pragma GCC visibility push(default)
-extern "C" {
-
-size_t spg_sparse_attn_workspace_bytes(const spg_attn_args *args) {
-  if (args == nullptr || check_args("spg_sparse_attn_workspace_bytes", args) != SPG_OK) return 0;
-  return layout_for(args).total;
-}
-
-int spg_sparse_attn(const spg_attn_args *args, void *stream) {
-  const char *fn = "spg_sparse_attn";
-  SPG_NONNULL(fn, args);
-  const spg_attn_args *a = args;
-  SPG_TRY(check_args(fn, a));
-  SPG_NONNULL(fn, a->q); SPG_NONNULL(fn, a->k); SPG_NONNULL(fn, a->v); SPG_NONNULL(fn, a->out); SPG_NONNULL(fn, a->workspace);
-  if (a->selection == SPG_SELECT_MASK) SPG_NONNULL(fn, a->mask);
-  const size_t need = layout_for(a).total;
-  if (a->workspace_bytes < need) return fail(SPG_ERR_INVALID, "%s: workspace of %zu bytes, %zu needed", fn, (size_t)a->workspace_bytes, need);
-  Strides qs, ks, vs, os;
-  SPG_TRY(get_strides(fn, "q_strides", a->q_strides, a->H, a->N, a->D, &qs));
-  SPG_TRY(get_strides(fn, "k_strides", a->k_strides, a->Hkv, a->N_kv, a->D, &ks));
-  SPG_TRY(get_strides(fn, "v_strides", a->v_strides, a->Hkv, a->N_kv, a->D, &vs));
-  SPG_TRY(get_strides(fn, "out_strides", a->out_strides, a->H, a->N, a->D, &os));
-  return check_launch(fn, run_forward(a, qs, ks, vs, os, (hipStream_t)stream));
-}
-
-}  // extern "C"
-#pragma GCC visibility pop

@@ -1,6 +1,7 @@
 // Host-only stand-ins for the kernel launchers declared in spargeattn_amd/csrc/launch.h, so that the argument
 // validation of capi.hip can be linked and run under AddressSanitizer / UBSan on a machine without a GPU.
 // Every function records that it was reached: the checks in check.cpp only make calls that must be refused before.
+#include "forward_plan.h"
 #include "launch.h"
 
 namespace spg {
@@ -24,4 +25,5 @@ hipError_t launch_block_sparse_attn(const int8_t *, const int8_t *, const uint8_
 void launch_fp8_pack_selftest(const float *, uint8_t *, int, int, hipStream_t) { g_launches++; }
 hipError_t launch_dense_attn_f16(const void *, const void *, const void *, void *, int, int, int, int, float, int,
                                  hipStream_t) { g_launches++; return hipSuccess; }
+hipError_t run_forward(const spg_attn_args *, const Strides &, const Strides &, const Strides &, const Strides &, hipStream_t) { g_launches++; return hipSuccess; }
 }  // namespace spg

@@ -1,6 +1,7 @@
 """The argument validation of the C ABI under AddressSanitizer and UndefinedBehaviorSanitizer, on the host only.
 
-capi.hip is compiled for the host (no device pass), linked with stand-ins for the kernel launchers
+capi.hip - every extern "C" entry point, with the workspace layout of the whole-operator call (forward_plan.h) - is
+compiled for the host (no device pass), linked with stand-ins for the kernel launchers
 (tests/capi_host/stubs.cpp) and driven by tests/capi_host/check.cpp with bad arguments of every kind; a sanitizer report
 or a wrong status / message fails the test.  Nothing here touches a GPU, and no GPU code is ever built with a sanitizer.
 """
