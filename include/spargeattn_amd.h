@@ -172,7 +172,8 @@ int spg_block_sparse_attn_f16v(const int8_t *q8, const int8_t *k8, const void *v
  * spas_sage_attn_meansim[_topk]_cuda; spas_sage_attn/core.py:39-319) ---------------------------------------------------
  * Runs the stages above with the same results, but stages that do not depend on each other share a launch, scalar
  * hyper-parameters need no device memory, and all intermediate tensors live in one workspace of
- * spg_sparse_attn_workspace_bytes() bytes, 256-byte aligned, that may be used again by the next call on the stream. */
+ * spg_sparse_attn_workspace_bytes() bytes, 256-byte aligned (SPG_ERR_INVALID otherwise), that may be used again by the next
+ * call on the stream. */
 enum spg_selection { SPG_SELECT_TOPK = 0, SPG_SELECT_CDF = 1, SPG_SELECT_MASK = 2 };
 
 typedef struct spg_attn_args {

@@ -227,6 +227,8 @@ int spg_sparse_attn(const spg_attn_args *args, void *stream) {
   if (a->selection == SPG_SELECT_MASK) SPG_NONNULL(fn, a->mask);
   const size_t need = layout_for(a).total;
   if (a->workspace_bytes < need) return fail(SPG_ERR_INVALID, "%s: workspace of %zu bytes, %zu needed", fn, (size_t)a->workspace_bytes, need);
+  // every part of the workspace starts at a multiple of 256 bytes and is read and written in pieces of up to 16
+  if ((uintptr_t)a->workspace % 256 != 0) return fail(SPG_ERR_INVALID, "%s: workspace must be 256-byte aligned (got %p)", fn, a->workspace);
   Strides qs, ks, vs, os;
   SPG_TRY(get_strides(fn, "q_strides", a->q_strides, a->H, a->N, a->D, &qs));
   SPG_TRY(get_strides(fn, "k_strides", a->k_strides, a->Hkv, a->N_kv, a->D, &ks));

@@ -138,6 +138,7 @@ int main() {
   REFUSED(a.out = nullptr, "a->out is NULL")
   REFUSED(a.workspace = nullptr, "a->workspace is NULL")
   REFUSED((a.selection = SPG_SELECT_MASK, a.mask = nullptr), "a->mask is NULL")
+  REFUSED((a.workspace = (char *)p + 128, a.workspace_bytes += 128), "256-byte aligned")
   REFUSED(a.workspace_bytes -= 1, "needed")
   REFUSED((a.pv_f16 = 1), "needed")                       // FP16 tiles take more than the workspace of the FP8 form
   REFUSED(a.q_strides = bad_mult, "q_strides[2]")
