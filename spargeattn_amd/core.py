@@ -16,6 +16,8 @@ granularity through the LUT (the reference passes ``is_causal=False`` to its ker
 (csrc/qattn/attn_cuda.h:61-76): 1 / "per_block", or 2 / "per_warp" - one Q scale per 32 query rows
 (spas_sage_attn/quant_per_block.py:102-148), which lowers the quantisation error at no cost in time.
 """
+import threading
+
 import torch
 
 from . import _lib
@@ -167,10 +169,11 @@ def _staged_mask(q, k, v, mask_id, scale, pvthreshd, tensor_layout, return_spars
 
 # ---- the whole operator in one native call (spg_sparse_attn) --------------------------------------------------------
 # What follows from shapes, strides, dtypes and options is worked out once per combination and kept (_lib.ForwardPlan
-# holds sizes, never data); a call then costs two allocations and one foreign call.  Plans are immutable and the dict
-# operations atomic, so threads may share them; the cache is emptied when a program has shown it very many shapes.
+# holds sizes, never data); a call then costs two allocations and one foreign call.  Plans are immutable and a lookup is one
+# dict operation, so threads may share them.  At most _MAX_PLANS are kept: a new one then takes the place of the oldest.
 _plans = {}
 _MAX_PLANS = 512
+_plans_lock = threading.Lock()          # for additions
 
 
 def _hyper(value, H, device):
@@ -210,9 +213,10 @@ def _run(q, k, v, mask, selection, level, simthreshd1, pvthreshd, is_causal, att
                                 1.0 / (headdim ** 0.5) if scale is None else scale)
         q, k, v = given
         plan.out = like.transpose(-2, -3) if nhd else like
-        if len(_plans) >= _MAX_PLANS:
-            _plans.clear()
-        _plans[key] = plan
+        with _plans_lock:
+            while len(_plans) >= _MAX_PLANS:
+                del _plans[next(iter(_plans))]
+            _plans[key] = plan
     device = plan.device
     if torch.cuda.current_device() != plan.device_index:
         torch.cuda.set_device(device)

@@ -166,3 +166,17 @@ def test_softmax_scale_is_read_on_every_call(stand_in_plans):
     assert _StandInPlan.ran[2:] == [0.5] * 4 + [2.0, 0.125]
     assert len(stand_in_plans) == 5
     assert not any(isinstance(part, (torch.Tensor, np.ndarray)) for key in stand_in_plans for part in key)
+
+
+def test_plans_beyond_the_bound_replace_the_oldest(stand_in_plans, monkeypatch):
+    """The newest shapes stay planned, one at a time leaves; a shape that left is planned anew."""
+    from spargeattn_amd import core
+    monkeypatch.setattr(core, "_MAX_PLANS", 4)
+    made = []
+    monkeypatch.setattr(_lib, "ForwardPlan", lambda q, *rest: made.append(q.shape[2]) or _StandInPlan(q, *rest))
+    for n in (128, 129, 130, 131, 132, 133, 130, 133, 128):
+        x = torch.zeros(1, 1, n, 64, dtype=torch.float16)
+        sa.spas_sage2_attn_meansim_topk_cuda(x, x, x)
+        assert len(stand_in_plans) <= 4
+    assert made == [128, 129, 130, 131, 132, 133, 128]
+    assert sorted(key[0][2] for key in stand_in_plans) == [128, 131, 132, 133]
