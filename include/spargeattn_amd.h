@@ -145,7 +145,10 @@ int spg_v_quant_fp8(const void *v, const int64_t *v_strides, uint8_t *v8, float 
  * sm89.cu:310-314, sm89.cuh:118); Hkv = H is plain multi-head attention; pv_count (B,H,nq*4) int32 or NULL: number of K blocks
  * whose PV was computed, one entry per 32 query rows as in the reference (sm89.cu:331-334); entries of Q blocks with
  * valid_block_num == 0 are left untouched.
- * Row blocks with valid_block_num == 0 are left unwritten, as in the reference (sm89.cuh:232-235). */
+ * Row blocks with valid_block_num == 0 are left unwritten, as in the reference (sm89.cuh:232-235).
+ * Asking for counts can change the last bits of out: on small grids (up to 256 Q blocks in all, nk >= 12, mode
+ * SPG_PV_PER_BLOCK) a call with pv_count == NULL splits a row over groups of wavefronts, which sum O and the denominator in
+ * another order than the block-by-block walk that counts.  P, its rounding and the skipped blocks are the same. */
 int spg_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, const int64_t *out_strides,
                           int out_dtype, const int32_t *lut, const int32_t *valid_block_num, const float *pvthreshd,
                           const float *q_scale, const float *k_scale, const float *v_scale,
@@ -157,7 +160,7 @@ int spg_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8,
  * kernel csrc/qattn/qk_int_sv_f16_cuda_sm80.cuh:42-671) as called by spas_sage_attn_meansim[_topk]_cuda
  * (spas_sage_attn/core.py:235-319): P is rounded to fp16, the denominator sums the rounded P, the output is O / d
  * with no V scale, is_causal masks at token level.  PV is accumulated in fp32 throughout (the reference rounds each
- * 64-key partial product to fp16 first).
+ * 64-key partial product to fp16 first).  pv_count and the last bits of out: as for spg_block_sparse_attn.
  * spg_v_tiles_f16 prepares the V operand: v (B,H,N,D) fp16|bf16 -> vt (B,H,ceil(N/64),D,64) fp16, the V^T of each
  * 64-key block (bf16 is rounded to fp16 as core.py:247 does), 8-key chunks of a row stored at slot chunk ^ ((d >> 1) & 7),
  * zero beyond N.  It takes the place of the kernel's transposing shared-memory reads (ldmatrix.trans). */

@@ -1,5 +1,5 @@
 // The whole operator behind one call: K mean, mask prediction + INT8 quantisation, V quantisation, block-sparse
-// attention, as three or four launches on workspace the caller hands over.
+// attention, as three to five launches on workspace the caller hands over.
 //
 // Short sequences are bound by the length of the launch chain and by kernels that cannot fill the chip, so stages that do
 // not depend on each other share a launch; which stage a workgroup belongs to follows from its number:
