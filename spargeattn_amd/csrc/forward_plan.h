@@ -11,14 +11,17 @@ namespace spg {
 // enough to be combined by every workgroup of the back kernel (a few KiB from L2 against a launch of about 4.5 us);
 // beyond, the final kernel combines as many as it takes to spread the read over the chip - unless the heads are so few that
 // the back kernel's workgroups can read 32 chunks each for less than the launch (up to 24576 rows in all: at most 768
-// workgroups, 13 MB from L2 in one head N17776 D64, 205.2 us per call with the final kernel, 201.8 without).
+// workgroups, 13 MB from L2 in one head N17776 D64) and a head so short that reading its 32 chunks does not become the
+// length of the front kernel (below 3 MiB of K).  us per call without / with the final kernel: one head D64 N12288 55.2 / 57.2,
+// N17776 166.4 / 168.9, N20480 83.8 / 84.4, N24000 215.1 / 215.2, N24576 97.0 / 96.0; D128 N8448 59.9 / 61.5, N11000 145.8 / 146.9,
+// N12000 157.9 / 157.8, N16384 94.6 / 93.5, N24576 132.0 / 126.3; two heads D128 N12288 80.9 / 80.9, with FP16 PV 88.9 / 88.3.
 struct Chunks {
   int n, rows;
   bool partial;
 };
-inline Chunks chunks_for(int heads, int N) {
+inline Chunks chunks_for(int heads, int N, int D) {
   Chunks c;
-  const bool few = (long long)heads * N <= 24576;
+  const bool few = (long long)heads * N <= 24576 && (long long)N * D < 3 << 19;
   c.partial = N <= 8192 || few;
   const int want = N <= 8192 ? 16 : few ? 32 : (2048 + heads - 1) / heads;
   const int most = N <= 8192 ? (N + 63) / 64 : (N + 255) / 256;
@@ -37,7 +40,7 @@ inline Layout layout_for(const spg_attn_args *a) {
   auto take = [&](size_t bytes) { const size_t r = at; at += (bytes + 255) / 256 * 256; return r; };
   const size_t bh = (size_t)a->B * a->H, bhk = (size_t)a->B * a->Hkv, D = a->D;
   const size_t nq = ((size_t)a->N + 127) / 128, nk = ((size_t)a->N_kv + 63) / 64;
-  const Chunks c = chunks_for((int)bhk, a->N_kv);
+  const Chunks c = chunks_for((int)bhk, a->N_kv, a->D);
   const bool pool = a->selection != SPG_SELECT_MASK;
   l.km_part = take(bhk * c.n * D * 8);
   l.v_part = take(a->pv_f16 ? 0 : bhk * c.n * D * 4);

@@ -107,9 +107,20 @@ def test_every_row_is_placed_once(H, N):
 @pytest.mark.parametrize("D", [64, 128])
 def test_few_long_heads_combine_partial_sums(D, Nk):
     """Up to 24576 key/value rows in all, longer heads get 32 chunks that every workgroup adds up (here up to 12288 rows of two
-    heads); one row more goes through the launch in between."""
+    heads, at D = 64); one row more goes through the launch in between."""
     q = rand_T((1, 2, 130, D), torch.bfloat16, 31)
     k, v = rand_T((1, 2, Nk, D), torch.bfloat16, 32, shift=0.3), rand_T((1, 2, Nk, D), torch.float16, 33)
+    for fn in (sa.spas_sage2_attn_meansim_topk_cuda, sa.spas_sage_attn_meansim_topk_cuda):
+        o, o2 = _both(lambda: fn(q, k, v, topk=0.3, simthreshd1=0.1))
+        assert torch.equal(_bits(o), _bits(o2))
+
+
+@pytest.mark.parametrize("H,Nk,D", [(1, 24575, 64), (1, 24576, 64), (2, 12287, 128), (1, 12288, 128)])
+def test_long_heads_go_through_the_launch_in_between(H, Nk, D):
+    """The other end of the same rule: the last length of a head whose partial sums every workgroup adds up (24575 at D = 64,
+    12287 at D = 128) and the first beyond it."""
+    q = rand_T((1, H, 130, D), torch.float16, 34)
+    k, v = rand_T((1, H, Nk, D), torch.float16, 35, shift=0.3), rand_T((1, H, Nk, D), torch.bfloat16, 36)
     for fn in (sa.spas_sage2_attn_meansim_topk_cuda, sa.spas_sage_attn_meansim_topk_cuda):
         o, o2 = _both(lambda: fn(q, k, v, topk=0.3, simthreshd1=0.1))
         assert torch.equal(_bits(o), _bits(o2))
