@@ -49,7 +49,8 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define SPG_ACC_C_BITS 0x3E22F983    // the float 1/(2 pi), an inline constant of the instruction set: initial accumulator
 #define SPG_ACC_SCALE 67108864.0f    // 2^26: one unit of the integer dot product is 2^-26 in the binade [1/8, 1/4)
 #define SPG_ROW_MAJOR_MAX 512       // workgroups per XCD up to which causal rows are ordered by length across heads
-#define SPG_QUEUE_MIN 384           // workgroups per XCD from which the queue pays: four rounds of 32 CUs x 3
+#define SPG_QUEUE_MIN 384           // workgroups per XCD (four rounds of 32 CUs x 3) and ...
+#define SPG_QUEUE_MIN_ROW 16384     // ... length of a row, in channels of K blocks, beyond which the queue pays (launch_attn)
 #define SPG_QUEUE_EXTRA 12          // one workgroup in so many is launched on top
 #define SPG_GROUPS_MAX_WG 256       // rows up to which ...
 #define SPG_GROUPS_MIN_NK 12        // ... and K blocks from which a row gets groups of wavefronts
@@ -954,7 +955,15 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   p.nq = (p.N + 127) / 128; p.nk = (p.Nk + 63) / 64;
   p.total_wg = p.nq * p.H * p.B;
   p.wg_per_xcd = (p.total_wg + 7) / 8;
-  if (SEL || p.wg_per_xcd < SPG_QUEUE_MIN) p.queue = nullptr;
+  // The queue costs a row an atomic round trip before it can start and gains it a share of its time: it takes rows long enough,
+  // and several rounds of them.  A row is nk blocks of D channels, half of that on average where the selection is causal.  us per
+  // call with / without, N or H x N, top-k 0.3 to 0.5: D64 96 x 6000 450 / 431, 32 x 16384 941 / 932, 24 x 16448 677 / 677, 23 x 17000
+  // 789 / 796, 48 x 32768 5095 / 5180; D128 96 x 6000 659 / 652, 96 x 8192 1046 / 1051, 48 x 12288 1047 / 1060; causal D64 40 x 16384
+  // 976 / 952, 32 x 32768 2681 / 2670, 28 x 40000 3755 / 3755, 12 x 65536 4334 / 4422; causal D128 96 x 8192 1057 / 1043, 32 x 16384
+  // 1138 / 1134, 48 x 24576 3624 / 3650, 12 x 65536 6161 / 6330, 11 x 90000 10188 / 10864.  Fewer rows per XCD: D64 8 x 16384 278 / 269,
+  // 20 x 16384 628 / 618, 18 x 17000 647 / 641, D128 8 x 16384 396 / 389, 18 x 17000 894 / 901; causal D128 18 x 17000 724 / 714.
+  const long long row = ((long long)p.nk * D) >> (causal_rows ? 1 : 0);
+  if (SEL || p.wg_per_xcd < SPG_QUEUE_MIN || row <= SPG_QUEUE_MIN_ROW) p.queue = nullptr;
   const int grid = 8 * (p.queue != nullptr ? p.wg_per_xcd + p.wg_per_xcd / SPG_QUEUE_EXTRA : p.wg_per_xcd);
   // Causal rows differ in length throughout: all rows by length while the heads an XCD works on at once share its L2
   // anyway (grids of a few rounds), head by head beyond.  Otherwise only a partial last Q block stands out.

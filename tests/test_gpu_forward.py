@@ -103,6 +103,23 @@ def test_every_row_is_placed_once(H, N):
         assert torch.isfinite(o.float()).all() and (o != 0).any(-1).all()
 
 
+@pytest.mark.parametrize("op,H,N,D,causal", [("topk", 31, 16500, 64, False), ("topk", 48, 16384, 64, False), ("topk16", 49, 8300, 128, False),
+                                             ("topk", 25, 16500, 128, True), ("topk16", 25, 16384, 128, True), ("mask", 31, 16500, 64, False)])
+def test_long_grids_place_every_row_once(op, H, N, D, causal):
+    """Grids whose rows are handed out from counters (384 rows per XCD and more, of more than 16384 K-block channels), with counts
+    that do and do not divide by eight, and beside the line: the same bits as the stages, whose rows have fixed places."""
+    q, k, v = (rand_T((1, 1, N, D), torch.bfloat16, 40 + i).expand(1, H, N, D) * (1 + torch.arange(H, device="cuda").view(1, H, 1, 1) / H).bfloat16()
+               for i in range(3))
+    mask = (torch.rand((1, H, (N + 127) // 128, (N + 63) // 64), generator=torch.Generator().manual_seed(1)) < 0.1).cuda()
+    mask[..., 0] = True
+    fn = {"topk": lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.2, is_causal=causal),
+          "topk16": lambda: sa.spas_sage_attn_meansim_topk_cuda(q, k, v, topk=0.2, is_causal=causal),
+          "mask": lambda: sa.block_sparse_sage2_attn_cuda(q, k, v, mask_id=mask)}[op]
+    torch.full_like(q, float("nan"))                     # an output row that is missed would not keep the value of an earlier call
+    o, o2 = _both(fn)
+    assert torch.isfinite(o.float()).all() and torch.equal(_bits(o), _bits(o2))
+
+
 @pytest.mark.parametrize("Nk", [8193, 12288, 12289])
 @pytest.mark.parametrize("D", [64, 128])
 def test_few_long_heads_combine_partial_sums(D, Nk):
