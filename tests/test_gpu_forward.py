@@ -90,6 +90,20 @@ def test_layouts_and_copied_inputs():
     assert torch.equal(_bits(o), _bits(o2))
 
 
+@pytest.mark.parametrize("H,N,Nk", [(2, 700, 4300), (3, 400, 4200), (9, 4200, 4200), (7, 1000, 1500), (5, 300, 3000)])
+def test_reported_sparsity_has_the_same_bits(H, N, Nk):
+    """Block counts that are not powers of two: the quotient and the product with the reciprocal differ in the last bit."""
+    q, k, v = rand_T((1, H, N, 64), torch.bfloat16, 1), rand_T((1, H, Nk, 64), torch.bfloat16, 2, shift=0.3), rand_T((1, H, Nk, 64), torch.bfloat16, 3)
+    mask = (torch.rand((1, H, (N + 127) // 128, (Nk + 63) // 64), generator=torch.Generator().manual_seed(4)) < 0.4).cuda()
+    fns = [lambda: sa.block_sparse_sage2_attn_cuda(q, k, v, mask_id=mask, return_sparsity=True)]
+    for topk in (0.1, 0.3, 0.5, 0.6):
+        fns.append(lambda topk=topk: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=topk, return_sparsity=True))
+        fns.append(lambda topk=topk: sa.spas_sage_attn_meansim_topk_cuda(q, k, v, topk=topk, is_causal=N == Nk, return_sparsity=True))
+    for fn in fns:
+        (_, s), (_, s2) = _both(fn)
+        assert s == s2
+
+
 @pytest.mark.parametrize("H", [1, 3, 8, 9, 17])
 @pytest.mark.parametrize("N", [128, 200, 640, 1100])
 def test_every_row_is_placed_once(H, N):
