@@ -362,7 +362,17 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   const uint32_t v_lane = v_wave + lane_ * 16u;                                                               \
   const uint32_t kswz_lane = D == 128 ? ((lane_ >> 4) & 3u) : ((lane_ >> 4) & 1u);                            \
   const uint32_t k_lane = k_wave + (((lane_ ^ kswz_lane) << 4) ^ kswz_wave16);   /* row * D + (slot ^ swz) * 16 */
-  const int last_partial_blk = (Nk % 64) ? p.nk - 1 : -1;   // the only block with rows beyond Nk
+  // FP8 PV, D = 128 or groups: a wavefront copies half of ONE of the two tiles instead of a quarter of each - wavefronts 0 and 1
+  // the K tile, 2 and 3 the V^T tile: one base address, one LDS base and one resident lane offset for all its loads of a block.
+  // us per call, quarters / halves: H32 N32768 D128 causal 3926 / 3895, one head N17776 D64 (three groups) 170.2 / 168.9; but a mask
+  // over H48 N16384 D64 904 / 918, where a wavefront has two loads per block only.
+  constexpr bool HALF_LOADS = !PV16 && (D == 128 || G > 1);
+  constexpr int HALF = TILE / 2;
+  const uint32_t half_swz = wave >= 2 ? 0u : D == 128 ? ((lane >> 4) & 3u) | ((uint32_t)wave << 2) : ((lane >> 4) & 1u) | ((uint32_t)wave << 1);
+  const uint32_t half_lane = ((uint32_t)lane ^ half_swz) << 4;
+  const uint8_t *const half_base = (wave >= 2 ? vbase : (const uint8_t *)kbase) + (wave & 1) * HALF;
+  unsigned char *const half_lds = (wave >= 2 ? sVr : sKr) + (wave & 1) * HALF;
+  const int last_partial_blk = (Nk % 64) && (!HALF_LOADS || wave < 2) ? p.nk - 1 : -1;   // the only block with rows beyond Nk
   typedef __attribute__((address_space(3))) void *lds_ptr_t;
   typedef const __attribute__((address_space(1))) void *glb_ptr_t;
 #define SPG_LOAD_K_(BLK, KOFF, CHK)   /* inside a scope that holds SPG_LANE_OFFSETS() */                            \
@@ -400,7 +410,35 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
 #define SPG_LOAD_K(BLK, KOFF) { SPG_LANE_OFFSETS() (void)v_lane; SPG_LOAD_K_(BLK, KOFF, 1) }
 #define SPG_LOAD_V(BLK, VOFF) { SPG_LANE_OFFSETS() (void)k_lane; (void)pos0; SPG_LOAD_V_(BLK, VOFF) }
 // rings of three slots: both tiles of one block into ring slot offset BUFOFF (in K-tile units)
-#define SPG_LOAD_TILES(BLK, BUFOFF, CHK) { SPG_LANE_OFFSETS() SPG_LOAD_K_(BLK, BUFOFF, CHK) SPG_LOAD_V_(BLK, (VTILE / TILE) * (BUFOFF)) }
+#define SPG_LOAD_QUARTERS(BLK, BUFOFF, CHK) { SPG_LANE_OFFSETS() SPG_LOAD_K_(BLK, BUFOFF, CHK) SPG_LOAD_V_(BLK, (VTILE / TILE) * (BUFOFF)) }
+  auto load_tiles = [&](int b, uint32_t boff, auto chk) __attribute__((always_inline)) {
+    if constexpr (!HALF_LOADS) { SPG_LOAD_QUARTERS(b, boff, decltype(chk)::value) }
+    else {
+      const uint8_t *const tb = half_base + (size_t)(uint32_t)b * TILE;
+      unsigned char *const tl = half_lds + boff;
+      if (!decltype(chk)::value || b != last_partial_blk) {
+        __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + half_lane), (lds_ptr_t)tl, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + half_lane), (lds_ptr_t)tl, 16, 1024, 0);
+        if constexpr (D == 128) {
+          __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + half_lane), (lds_ptr_t)tl, 16, 2048, 0);
+          __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + half_lane), (lds_ptr_t)tl, 16, 3072, 0);
+        }
+      } else {
+        // K rows beyond Nk are clamped to row Nk-1: their scores are masked, their V rows are zero
+        const uint8_t *const kb = (const uint8_t *)kbase + (size_t)(uint32_t)b * TILE;
+        const uint32_t last_row = (uint32_t)(Nk - 1 - b * 64);
+        uint32_t lane_off = half_lane;
+        asm volatile("" : "+v"(lane_off));           // keeps these offsets out of the registers of the loop
+#pragma unroll
+        for (int u = 0; u < HALF / 1024; u++) {
+          const uint32_t row = (uint32_t)((wave & 1) * 32 + u * (64 / CPR)) + (lane_off / D);   // the swizzle stays within a row
+          const uint32_t off = min(row, last_row) * D + (lane_off & (D - 1));
+          __builtin_amdgcn_global_load_lds((glb_ptr_t)(kb + off), (lds_ptr_t)(tl + u * 1024), 16, 0, 0);
+        }
+      }
+    }
+  };
+#define SPG_LOAD_TILES(BLK, BUFOFF, CHK) load_tiles(BLK, BUFOFF, std::integral_constant<int, CHK>{})
 
   // MFMA row i of key tile kt carries key 32*((i>>2)&1) + 16*kt + 4*(i>>3) + (i&3); rows krow0 and krow0+16 have
   // the same swizzle, so tile 1's operand sits 16 rows (16*D bytes) after tile 0's.
@@ -562,7 +600,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     float ksc2 = 0.f;
     int d4 = 0, d4g[G] = {};
     if constexpr (!TAIL || G > 1) {
-      ksc2 = kscale[(uint32_t)blk2];
+      ksc2 = *(c_f32_t)((const __attribute__((address_space(4))) char *)kscale + (uint32_t)(blk2 << 2));
       if constexpr (!SEL && G == 1) d4 = it + 4 < nv ? lutc[(uint32_t)(it + 4)] : 0;
       if constexpr (!SEL && G > 1) {
 #pragma unroll
@@ -572,9 +610,10 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     __builtin_amdgcn_sched_barrier(0);
     const float dq = qs * ksc;                     // used by the tail blocks only
     // S0/S1 are never rewritten (no copies at the join of the two paths): slot e < 16 is S0[e], slot e >= 16 is S1[e - 16]
-    // multiplier of the accumulator read as a float: a * 2^26.  Wavefront-uniform, so it is moved to a scalar register:
-    // the 32 multiply-adds below then read two vector registers each instead of three
-    const float a26 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, cq26 * ksc)));
+    // multiplier of the accumulator read as a float: a * 2^26.  Wavefront-uniform, but kept in a vector register: with two or
+    // more wavefronts per SIMD a multiply-add of three vector registers issues in 2.6 clocks, one that reads a scalar register
+    // in 4.3 (128 of them per wavefront, three wavefronts: 138 against 233 ns)
+    const float a26 = cq26 * ksc;
     // The constant 1/(2 pi) leaves the exponent through ONE additive term, -(1/(2 pi) a 2^26 + m) (+ 8.807), whose rounding
     // error is half an ulp of 1.07e7 a.  Below 2^14 that is at most 2^-11 in the exponent (3e-4 relative in P, and the
     // row maximum's P stays below 448.2).  At or above it (large |q| |k| or a large softmax scale; uniform for the
@@ -629,8 +668,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     int vote = 1;
     if constexpr (!TAIL && G == 1) {
       // max over rows of (diff) + thr > 0  <=>  some row has diff + thr > 0 (fp32 addition is monotonic)
-      vote = __any(diff + thr > 0.f);
-      if (vote == 0) {                    // wavefront-uniform
+      vote = __any(diff > -thr);          // (the sign of a binary32 sum is exact)
+      if (__builtin_expect(vote == 0, 0)) {                    // wavefront-uniform
         sSkipAt[it & 1][wave] = it;       // every lane: a branch on the lane would make the body's control flow divergent
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       }
@@ -673,12 +712,12 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       if (TAIL) compute = compute && active;
     }
     if constexpr (!TAIL && G == 1) {   // workgroup-uniform in the per-block mode (sm89.cuh:318-353), wavefront-uniform otherwise
-      compute = p.pv_mode == 0 || vote != 0;
       // per-block mode: a wavefront whose own vote is set knows the OR already; only one that voted "skip" has to read
       // what the others wrote (an LDS round trip that the common case does without)
-      if (p.pv_mode == 1 && !compute)
-        compute = !(sSkipAt[it & 1][0] == it && sSkipAt[it & 1][1] == it && sSkipAt[it & 1][2] == it &&
-                    sSkipAt[it & 1][3] == it);
+      if (__builtin_expect(vote == 0, 0)) {
+        compute = p.pv_mode == 0;
+        if (p.pv_mode == 1) compute = !__builtin_amdgcn_readfirstlane(sSkipAt[it & 1][0] == it && sSkipAt[it & 1][1] == it && sSkipAt[it & 1][2] == it && sSkipAt[it & 1][3] == it);
+      }
     }
     if constexpr (PV16 && G == 1) {
       // two-slot rings: every wavefront is past its reads of K slot it % 2 (this block's scores) and of V^T slot
@@ -696,8 +735,10 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       }
     }
     // the running maximum of some query rose: rescale (exp2(0) = 1 exactly, so the other iterations need neither the
-    // exponential nor the products)
-    if (__any(G == 1 ? diff > 0.f : m_new > m_old)) {
+    // exponential nor the products).  Only the lanes of such a query take part - mostly one or two of the 32: the clock under
+    // this kernel is set by its power, and idle lanes draw none (H32 N32768 D128 causal 3918 -> 3895 us, a mask over H48
+    // N16384 D128 1371 -> 1358)
+    if (G == 1 ? diff > 0.f : m_new > m_old) {
       const float osc = __builtin_amdgcn_exp2f(m_old - m_new);
       dsum *= osc;
 #pragma unroll
@@ -713,18 +754,20 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       if (!masked) {
         // three passes kept apart for the scheduler: a multiply-add feeding the exponential of the same element directly,
         // and the exponential feeding the running sum, would issue as one long chain of dependent instructions
-        if (__builtin_expect(!precise, 1)) {
-          const float neg = __builtin_fmaf(-acc_c, a26, neg0);   // takes the accumulator constant out: one rounding per row
-#pragma unroll
-          for (int e = 0; e < 32; e++) x[e] = __builtin_fmaf(__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]), a26, neg);
-        } else {
+        float neg = __builtin_fmaf(-acc_c, a26, neg0);   // takes the accumulator constant out: one rounding per row
+        if (__builtin_expect(precise, 0)) {
           // (S - S_max,lane) a + (S_max,lane a - m + offset): what the reference's fma(S, a, -m + offset) computes
           // (attn_utils.cuh:391-415), with the rounding of m as the only error
-          const float c0 = __builtin_fmaf(mloc - acc_c, a26, neg0);
+          neg = __builtin_fmaf(mloc - acc_c, a26, neg0);
 #pragma unroll
-          for (int e = 0; e < 32; e++)
-            x[e] = __builtin_fmaf(__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]) - mloc, a26, c0);
+          for (int e = 0; e < 16; e++) {
+            const int s0 = S0[e], s1 = S1[e];
+            S0[e] = __builtin_bit_cast(int, __builtin_bit_cast(float, s0) - mloc);
+            S1[e] = __builtin_bit_cast(int, __builtin_bit_cast(float, s1) - mloc);
+          }
         }
+#pragma unroll
+        for (int e = 0; e < 32; e++) x[e] = __builtin_fmaf(__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]), a26, neg);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int e = 0; e < 32; e++) x[e] = __builtin_amdgcn_exp2f(x[e]);
@@ -870,6 +913,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     for (; it < n_all; it++) step(std::true_type{}, std::integral_constant<int, -1>{}, it);
   }
 #undef SPG_LOAD_TILES
+#undef SPG_LOAD_QUARTERS
 #undef SPG_LOAD_K
 #undef SPG_LOAD_V
 #undef SPG_LOAD_K_
