@@ -52,6 +52,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define SPG_QUEUE_MIN 384           // workgroups per XCD (four rounds of 32 CUs x 3) and ...
 #define SPG_QUEUE_MIN_ROW 16384     // ... length of a row, in channels of K blocks, beyond which the queue pays (launch_attn)
 #define SPG_QUEUE_EXTRA 12          // one workgroup in so many is launched on top
+#define SPG_PLACES 96               // rows that an XCD works on at a time: 32 CUs x 3
 #define SPG_GROUPS_MAX_WG 256       // rows up to which ...
 #define SPG_GROUPS_MIN_NK 12        // ... and K blocks from which a row gets groups of wavefronts
 #define SPG_LOG2E 1.44269504088896340736f
@@ -901,8 +902,29 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     const int n_fast = G == 1 ? nv - 3 : (nv - 1) / G - 2, n_common = G == 1 ? nv - 2 : (nv - 2) / G, n_all = (nv + G - 1) / G;
     // the common loop, three blocks per trip (ring slots 0, 1, 2); `bufoff` stays 0 throughout where the slots are
     // compile-time constants, and three run-time steps bring it back to 0 where they are not
+    // The wavefronts of a SIMD are served oldest first: of the three rows on a CU the first runs at almost the speed it would
+    // have alone, the last gets what is left and ends alone, at less than half the rate of three (three rows of 32 blocks ended
+    // at 50, 67 and 83 us).  While other rows wait for a place that is welcome.  The rows of an XCD that none wait for lower
+    // their priority as they near their end, so that those with more to do catch up and all end together.  us per call
+    // without / with, H x N top-k 0.5: D128 6 x 8192 124 / 118, 13 x 8192 214 / 201, 20 x 8192 272 / 263, 26 x 8192 354 / 342, causal 28 x
+    // 4096 118 / 116, D64 14 x 8192 156 / 144, 30 x 17776 1035 / 1016, FP16 PV 6 x 16384 379 / 367.  (The last 64 or 80 rows
+    // instead of the places of an XCD: 13 x 8192 205 / 200, 20 x 8192 266 / 267; steps at thirds of the row: 205, 265.)
+    int drop_at = 0x7fffffff;
+    if constexpr (G == 1) {
+      __builtin_amdgcn_s_setprio(3);
+      if ((item >> 3) >= p.wg_per_xcd - SPG_PLACES) drop_at = nv >> 1;
+    }
 #pragma unroll 1
     for (; it + 3 <= n_fast; it += 3) {
+      if constexpr (G == 1) {
+        if (it >= drop_at) {
+          const int d2 = nv - (nv >> 2), d3 = nv - (nv >> 3);
+          __builtin_amdgcn_s_setprio(2);
+          if (it >= d2) __builtin_amdgcn_s_setprio(1);
+          if (it >= d3) __builtin_amdgcn_s_setprio(0);
+          drop_at = it >= d3 ? 0x7fffffff : it >= d2 ? d3 : d2;
+        }
+      }
       step(std::false_type{}, std::integral_constant<int, 0>{}, it);
       step(std::false_type{}, std::integral_constant<int, 1>{}, it + 1);
       step(std::false_type{}, std::integral_constant<int, 2>{}, it + 2);
