@@ -552,6 +552,22 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
         if constexpr (CS) lds_read_2x128<(SLOT < 0 ? 0 : SLOT) * TILE, (SLOT < 0 ? 0 : SLOT) * TILE + 16 * D>(a0[ks], a1[ks], kaddr_c[ks]);
         else lds_read_2x128<0, 16 * D>(a0[ks], a1[ks], kaddr_c[ks] + bufoff);
       };
+      // FP16 PV: two k-steps in registers, each replaced by the one after next as soon as its products are issued
+      if constexpr (PV16) {
+        read_k(0); read_k(1);
+        lds_wait_but<2>(a0[0], a1[0]);
+        asm volatile("v_mfma_i32_32x32x32_i8 %0, %2, %4, 0.15915494\n\tv_mfma_i32_32x32x32_i8 %1, %3, %4, 0.15915494"
+                     : "=&v"(S0), "=&v"(S1)
+                     : "v"(a0[0]), "v"(a1[0]), "v"(qreg[0]));
+#pragma unroll
+        for (int ks = 1; ks < KS; ks++) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (ks + 1 < KS) { read_k(ks + 1); lds_wait_but<2>(a0[ks], a1[ks]); }
+          else lds_wait_but<0>(a0[ks], a1[ks]);
+          S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0[ks], qreg[ks], S0, 0, 0, 0);
+          S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1[ks], qreg[ks], S1, 0, 0, 0);
+        }
+      } else {
       // first group: nothing to overlap with, the reads carry their wait
       {
         constexpr int SO = CS ? SLOT * TILE : 0;
@@ -559,12 +575,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
         if constexpr (HK == 2) lds_read_4x128_wait<SO, SO + 16 * D>(a0[0], a1[0], a0[1], a1[1], kaddr_c[0] + bo, kaddr_c[1] + bo);
         else lds_read_2x128_wait<SO, SO + 16 * D>(a0[0], a1[0], kaddr_c[0] + bo, kaddr_c[0] + bo);
       }
-      // second group: in flight under the first group's products (FP8 PV); the FP16-PV variant reads it afterwards, into
-      // the first group's registers, which is what lets it keep three wavefronts per SIMD
-      if constexpr (!PV16) {
+      // second group: in flight under the first group's products
 #pragma unroll
-        for (int ks = HK; ks < KS; ks++) read_k(ks);
-      }
+      for (int ks = HK; ks < KS; ks++) read_k(ks);
       // the first product of each chain, with the inline constant as its C operand (the compiler would otherwise keep
       // the constant in sixteen registers); the products that follow accumulate onto these and are ordinary builtins,
       // which the other chain's product always separates from their predecessor
@@ -576,21 +589,12 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
         S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0[ks], qreg[ks], S0, 0, 0, 0);
         S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1[ks], qreg[ks], S1, 0, 0, 0);
       }
-      if constexpr (PV16) {
-        if constexpr (HK == 2) lds_read_4x128_wait<0, 16 * D>(a0[0], a1[0], a0[1], a1[1], kaddr_c[2] + bufoff, kaddr_c[3] + bufoff);
-        else lds_read_2x128_wait<0, 16 * D>(a0[0], a1[0], kaddr_c[1] + bufoff, kaddr_c[1] + bufoff);
+      if constexpr (HK == 2) lds_wait4(a0[2], a1[2], a0[3], a1[3]); else lds_wait2(a0[1], a1[1]);
 #pragma unroll
-        for (int ks = HK; ks < KS; ks++) {
-          S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0[ks - HK], qreg[ks], S0, 0, 0, 0);
-          S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1[ks - HK], qreg[ks], S1, 0, 0, 0);
-        }
-      } else {
-        if constexpr (HK == 2) lds_wait4(a0[2], a1[2], a0[3], a1[3]); else lds_wait2(a0[1], a1[1]);
-#pragma unroll
-        for (int ks = HK; ks < KS; ks++) {
-          S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0[ks], qreg[ks], S0, 0, 0, 0);
-          S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1[ks], qreg[ks], S1, 0, 0, 0);
-        }
+      for (int ks = HK; ks < KS; ks++) {
+        S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0[ks], qreg[ks], S0, 0, 0, 0);
+        S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1[ks], qreg[ks], S1, 0, 0, 0);
+      }
       }
     }
 
@@ -827,22 +831,28 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
             }
           dsum += rs;
         }
-        // V^T operands in two halves of two 16-key steps each, through ONE set of registers (the budget of three
-        // wavefronts per SIMD); every read carries its wait
+        // V^T operands: two 16-key steps in registers, each replaced by the one after next as soon as its products are issued.
+        // (Two halves of two steps, every read waited for at once: H24 N8192 D128 causal 334 us, so 332; 4 heads N8192, two groups, 98.9 / 97.7.)
         const uint32_t va = lds_v0 + 2 * bufoff + v_rd16;
+        v4i t[4][NDT];
+        auto read_v = [&](int st) __attribute__((always_inline)) {
+          const uint32_t a_ = va ^ (uint32_t)(16 * st);
+          if constexpr (NDT == 4) lds_read_4x128<0, 4096, 8192, 12288>(t[st][0], t[st][1], t[st][2], t[st][3], a_);
+          else lds_read_2x128<0, 4096>(t[st][0], t[st][1], a_);
+        };
+        auto wait_v = [&](int st, auto but) __attribute__((always_inline)) {
+          if constexpr (NDT == 4) lds_wait_but<decltype(but)::value>(t[st][0], t[st][1], t[st][2], t[st][3]);
+          else lds_wait_but<decltype(but)::value>(t[st][0], t[st][1]);
+        };
+        read_v(0); read_v(1);
 #pragma unroll
-        for (int half = 0; half < 2; half++) {
-          v4i t[2][NDT];
-          const uint32_t va0 = va ^ (uint32_t)(32 * half), va1 = va0 ^ 16u;
-          if constexpr (NDT == 4)
-            lds_read_8x128_wait<0, 4096, 8192, 12288>(t[0][0], t[0][1], t[0][2], t[0][3], t[1][0], t[1][1], t[1][2], t[1][3], va0, va1);
-          else
-            lds_read_4x128_wait<0, 4096>(t[0][0], t[0][1], t[1][0], t[1][1], va0, va1);
+        for (int st = 0; st < 4; st++) {
+          if (st < 3) wait_v(st, std::integral_constant<int, NDT>{}); else wait_v(st, std::integral_constant<int, 0>{});
 #pragma unroll
-          for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int dt = 0; dt < NDT; dt++)
-              O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, t[u][dt]), pb16[2 * half + u], O[dt], 0, 0, 0);
+          for (int dt = 0; dt < NDT; dt++)
+            O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, t[st][dt]), pb16[st], O[dt], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (st < 2) read_v(st + 2);
         }
       } else {
       dsum += ps;

@@ -37,18 +37,6 @@ __device__ __forceinline__ void lds_read_4x128_wait(v4i &a, v4i &b, v4i &c, v4i 
                : "v"(addr0), "v"(addr1), "n"(O0), "n"(O1)
                : "memory");
 }
-// a, b, c, d <- addr0 + O0 .. O3; e, f, g, h <- addr1 + O0 .. O3
-template <int O0, int O1, int O2, int O3>
-__device__ __forceinline__ void lds_read_8x128_wait(v4i &a, v4i &b, v4i &c, v4i &d, v4i &e, v4i &f, v4i &g, v4i &h,
-                                                    uint32_t addr0, uint32_t addr1) {
-  asm volatile("ds_read_b128 %0, %8 offset:%10\n\tds_read_b128 %1, %8 offset:%11\n\t"
-               "ds_read_b128 %2, %8 offset:%12\n\tds_read_b128 %3, %8 offset:%13\n\t"
-               "ds_read_b128 %4, %9 offset:%10\n\tds_read_b128 %5, %9 offset:%11\n\t"
-               "ds_read_b128 %6, %9 offset:%12\n\tds_read_b128 %7, %9 offset:%13\n\ts_waitcnt lgkmcnt(0)"
-               : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d), "=&v"(e), "=&v"(f), "=&v"(g), "=&v"(h)
-               : "v"(addr0), "v"(addr1), "n"(O0), "n"(O1), "n"(O2), "n"(O3)
-               : "memory");
-}
 // a <- addr0 + O0, b <- addr1 + O1
 template <int O0, int O1>
 __device__ __forceinline__ void lds_read_2x128_wait(v4i &a, v4i &b, uint32_t addr0, uint32_t addr1) {
@@ -61,6 +49,22 @@ __device__ __forceinline__ void lds_read_2x128_wait(v4i &a, v4i &b, uint32_t add
 // Between such a read and its wait the destination registers are "written" as far as the compiler knows: the kernels
 // that use them are built with a check that nothing is spilled, and the build records the compiler version the
 // generated code was inspected with.
+// a, b, c, d <- addr + O0 .. O3
+template <int O0, int O1, int O2, int O3>
+__device__ __forceinline__ void lds_read_4x128(v4i &a, v4i &b, v4i &c, v4i &d, uint32_t addr) {
+  asm volatile("ds_read_b128 %0, %4 offset:%5\n\tds_read_b128 %1, %4 offset:%6\n\t"
+               "ds_read_b128 %2, %4 offset:%7\n\tds_read_b128 %3, %4 offset:%8"
+               : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d)
+               : "v"(addr), "n"(O0), "n"(O1), "n"(O2), "n"(O3)
+               : "memory");
+}
+// wait for all LDS reads but the last N (they return in order; a scalar load still under way only makes the wait longer)
+template <int N> __device__ __forceinline__ void lds_wait_but(v4i &a, v4i &b) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "n"(N));
+}
+template <int N> __device__ __forceinline__ void lds_wait_but(v4i &a, v4i &b, v4i &c, v4i &d) {
+  asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "n"(N));
+}
 // wait for all outstanding LDS reads; the operands tie the wait to the registers it makes valid
 __device__ __forceinline__ void lds_wait4(v4i &a, v4i &b, v4i &c, v4i &d) {
   asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
