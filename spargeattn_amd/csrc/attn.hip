@@ -417,19 +417,19 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     else {
       const uint8_t *const tb = half_base + (size_t)(uint32_t)b * TILE;
       unsigned char *const tl = half_lds + boff;
+      uint32_t lane_off = half_lane;
+      if constexpr (decltype(chk)::value || G > 1) asm volatile("" : "+v"(lane_off));   // keeps address arithmetic out of the registers of the loop
       if (!decltype(chk)::value || b != last_partial_blk) {
-        __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + half_lane), (lds_ptr_t)tl, 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + half_lane), (lds_ptr_t)tl, 16, 1024, 0);
+        __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + lane_off), (lds_ptr_t)tl, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + lane_off), (lds_ptr_t)tl, 16, 1024, 0);
         if constexpr (D == 128) {
-          __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + half_lane), (lds_ptr_t)tl, 16, 2048, 0);
-          __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + half_lane), (lds_ptr_t)tl, 16, 3072, 0);
+          __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + lane_off), (lds_ptr_t)tl, 16, 2048, 0);
+          __builtin_amdgcn_global_load_lds((glb_ptr_t)(tb + lane_off), (lds_ptr_t)tl, 16, 3072, 0);
         }
       } else {
         // K rows beyond Nk are clamped to row Nk-1: their scores are masked, their V rows are zero
         const uint8_t *const kb = (const uint8_t *)kbase + (size_t)(uint32_t)b * TILE;
         const uint32_t last_row = (uint32_t)(Nk - 1 - b * 64);
-        uint32_t lane_off = half_lane;
-        asm volatile("" : "+v"(lane_off));           // keeps these offsets out of the registers of the loop
 #pragma unroll
         for (int u = 0; u < HALF / 1024; u++) {
           const uint32_t row = (uint32_t)((wave & 1) * 32 + u * (64 / CPR)) + (lane_off / D);   // the swizzle stays within a row
@@ -633,8 +633,10 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     bool masked = false;                             // wavefront-uniform
     if constexpr (TAIL) {
       // slot e of this lane is key 64*blk + 32*hh + e; keys beyond `lim` are masked
-      const int key0 = blk * 64 + 32 * hh;
-      if (p.is_causal) lim = q_row - key0;                       // key > query (attn_utils.cuh:334-361)
+      uint32_t t = threadIdx.x;                                  // (the lane is worked out here: no register holds it across the loop)
+      asm volatile("" : "+v"(t));
+      const int key0 = blk * 64 + (int)(t & 32u), row = qb * 128 + wave * 32 + (int)(t & 31u);
+      if (p.is_causal) lim = row - key0;                         // key > query (attn_utils.cuh:334-361)
       if (place == nv - 1) lim = min(lim, Nk - 1 - key0);        // key >= kv_len (attn_utils.cuh:363-389)
       masked = tail && __any(lim < 31);
     }
@@ -654,6 +656,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
         float v = (__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]) - acc_c) * dq26;
         v = e > lim ? SPG_NEG_BIG : v;
         fm = fmaxf(fm, v);
+        if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // (one group after the other: the scheduler would spread them over registers that the loop does not have)
       }
       fm = fm * c;
     }
@@ -772,34 +775,38 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
           }
         }
 #pragma unroll
-        for (int e = 0; e < 32; e++) x[e] = __builtin_fmaf(__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]), a26, neg);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int e = 0; e < 32; e++) x[e] = __builtin_amdgcn_exp2f(x[e]);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (!PV16) {
-          // (four chains at D = 64, whose two P.V matrix instructions do not cover one chain of 31 dependent additions)
-          constexpr int NC = D == 64 ? 4 : 1;
-          float pc[NC];
-#pragma unroll
-          for (int e = 0; e < NC; e++) pc[e] = x[e];
-#pragma unroll
-          for (int e = NC; e < 32; e++) pc[e % NC] += x[e];
-          ps = pc[0];
-          if constexpr (NC == 4) ps = (pc[0] + pc[1]) + (pc[2] + pc[3]);
+        for (int e = 0; e < 16; e++) {
+          const int s0 = S0[e], s1 = S1[e];
+          S0[e] = __builtin_bit_cast(int, __builtin_fmaf(__builtin_bit_cast(float, s0), a26, neg));
+          S1[e] = __builtin_bit_cast(int, __builtin_fmaf(__builtin_bit_cast(float, s1), a26, neg));
         }
       } else {
-        ps = 0.f;
         const float masked = __builtin_fmaf(SPG_NEG_BIG, c, neg0);   // what the sentinel score turns into
         const float dq26 = dq * SPG_ACC_SCALE;
+        // de-quantised score first, then the softmax scale, as the reference's masked branch does (sm89.cuh:467-648)
 #pragma unroll
-        for (int e = 0; e < 32; e++) {
-          // de-quantised score first, then the softmax scale, as the reference's masked branch does (sm89.cuh:467-648)
-          const float sv = (__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]) - acc_c) * dq26;
-          const float t = __builtin_fmaf(sv, c, neg0);
-          x[e] = __builtin_amdgcn_exp2f(e > lim ? masked : t);
-          if constexpr (!PV16) ps += x[e];
+        for (int e = 0; e < 16; e++) {
+          const int s0 = S0[e], s1 = S1[e];
+          const float t0 = __builtin_fmaf((__builtin_bit_cast(float, s0) - acc_c) * dq26, c, neg0);
+          const float t1 = __builtin_fmaf((__builtin_bit_cast(float, s1) - acc_c) * dq26, c, neg0);
+          S0[e] = __builtin_bit_cast(int, e > lim ? masked : t0);
+          S1[e] = __builtin_bit_cast(int, e + 16 > lim ? masked : t1);
         }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 32; e++) x[e] = __builtin_amdgcn_exp2f(__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]));
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!PV16) {
+        // (four chains at D = 64, whose two P.V matrix instructions do not cover one chain of 31 dependent additions)
+        constexpr int NC = D == 64 ? 4 : 1;
+        float pc[NC];
+#pragma unroll
+        for (int e = 0; e < NC; e++) pc[e] = x[e];
+#pragma unroll
+        for (int e = NC; e < 32; e++) pc[e % NC] += x[e];
+        ps = pc[0];
+        if constexpr (NC == 4) ps = (pc[0] + pc[1]) + (pc[2] + pc[3]);
       }
       if constexpr (PV16) {
         typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -989,6 +996,10 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       }
     }
   }
+  // (computed again: no register holds them across the loop)
+  uint32_t lane_e = threadIdx.x & 63u;
+  asm volatile("" : "+v"(lane_e));
+  const int r_e = (int)lane_e & 31, hh_e = (int)lane_e >> 5;
   const float inv = __builtin_amdgcn_rcpf(dtot);
   // A lane holds four channels of one row per group: stored from here, an instruction would touch 32 rows with 16 bytes
   // each.  The rows of a wavefront go through LDS instead (the tile ring is free once every wavefront is past its last
@@ -1004,24 +1015,24 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   for (int dt = 0; dt < NDT; dt++) {
 #pragma unroll
     for (int g = 0; g < 4; g++) {
-      const int d0 = 32 * dt + 8 * g + 4 * hh;
+      const int d0 = 32 * dt + 8 * g + 4 * hh_e;
       float4 sc = make_float4(1.f, 1.f, 1.f, 1.f);
       if constexpr (!PV16) sc = *(const float4 *)(sVscale + d0);
       const uint16_t o0 = f32_to_elem<ODT>(O[dt][4 * g + 0] * inv * sc.x);
       const uint16_t o1 = f32_to_elem<ODT>(O[dt][4 * g + 1] * inv * sc.y);
       const uint16_t o2 = f32_to_elem<ODT>(O[dt][4 * g + 2] * inv * sc.z);
       const uint16_t o3 = f32_to_elem<ODT>(O[dt][4 * g + 3] * inv * sc.w);
-      *(uint2 *)(orow_lds + r * OROW + d0 * 2) = make_uint2((uint32_t)o0 | ((uint32_t)o1 << 16), (uint32_t)o2 | ((uint32_t)o3 << 16));
+      *(uint2 *)(orow_lds + r_e * OROW + d0 * 2) = make_uint2((uint32_t)o0 | ((uint32_t)o1 << 16), (uint32_t)o2 | ((uint32_t)o3 << 16));
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   constexpr int LPR = D / 8, RPI = 64 / LPR;                 // lanes per row, rows per store instruction
-  uint16_t *obase = (uint16_t *)p.out + (size_t)batch * p.os.sb + (size_t)head * p.os.sh + (lane % LPR) * 8;
+  uint16_t *obase = (uint16_t *)p.out + (size_t)batch * p.os.sb + (size_t)head * p.os.sh + ((int)lane_e % LPR) * 8;
 #pragma unroll
   for (int i = 0; i < 32 / RPI; i++) {
-    const int row = i * RPI + lane / LPR, grow = qb * 128 + wave * 32 + row;
-    const uint4 t = *(const uint4 *)(orow_lds + row * OROW + (lane % LPR) * 16);
+    const int row = i * RPI + (int)lane_e / LPR, grow = qb * 128 + wave * 32 + row;
+    const uint4 t = *(const uint4 *)(orow_lds + row * OROW + ((int)lane_e % LPR) * 16);
     if (grow < N) *(uint4 *)(obase + (size_t)grow * p.os.sn) = t;
   }
 }
@@ -1046,13 +1057,17 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
   p.by_nq = FastDiv::of(p.nq); p.by_rest = FastDiv::of(p.nq > p.rows_first ? p.nq - p.rows_first : 1);
   p.by_H = FastDiv::of(p.H); p.by_group = FastDiv::of(p.H / p.Hkv);
-  // A row alone on its CU: its blocks go over groups of wavefronts (kernel comment).  Three groups where registers allow and
-  // rows are long, two otherwise.  us per call with 1 / 2 / 3 groups: one head N17776 D64 281 / 236 / 225, H2 N16384 D64 131 /
-  // 111 / 105, D128 161 / 140 / -, FP16 PV D128 188 / 164 / -, H8 N4096 D64 45 / 41 / 41, D128 59 / 54 / -, H1 N2048 D64 28.3 / 26.7 /
-  // 27.2; H2 N256 18.0 / 18.6 / 19.9 (too few rounds for the exchange and the final sum).  Beyond one row per CU the rows fill
-  // each other's gaps: H10 N4096 unchanged without groups.
+  // A row alone on its CU: its blocks go over groups of wavefronts (kernel comment).  As many groups as registers and LDS
+  // allow where rows are long, two up to 64 blocks, where the exchange and the final sum weigh more.  us per call with 1 / 2 / 3 / 4
+  // groups, D64: one head N17776 281 / 236 / 169 / 163.5 (the last two of a later build), H2 N16384 131 / 111 / 98.4 / 96.2, H2 N12000
+  // CDF - / - / 123.5 / 120.7; H8 N4096 45 / 39.2 / 39.0 / 39.8, H2 N2048 - / 25.8 / 26.3 / 27.2; H2 N256 18.0 / 18.6 / 19.9.  D128: one head
+  // N17776 - / 227 / 214, H2 N16384 161 / 131 / 127, H2 N12000 causal - / 166 / 157.5; H8 N4096 59 / 53.5 / 54.0, H4 N3584 - / 42.4 /
+  // 43.1, H2 N2304 - / 32.6 / 33.4, H2 N1024 - / 25.2 / 26.6.  FP16 PV D128 H2 N16384 188 / 164 (two fit the LDS).  At D128 a grid of
+  // fewer than eight rows keeps two for every nk, so that a list has the same bits whatever the length of the head around it.
+  // Beyond one row per CU the rows fill each other's gaps: H10 N4096 unchanged without groups.
   const bool groups = p.total_wg <= SPG_GROUPS_MAX_WG && p.nk >= SPG_GROUPS_MIN_NK && p.pv_mode == 1 && p.pv_count == nullptr;
-  const int n_groups = !groups ? 1 : D == 64 && p.nk > SPG_SELECT_IN_ATTN_NK ? 3 : 2;
+  const int most = D == 64 ? 4 : p.v_scale != nullptr && p.total_wg >= 8 ? 3 : 2;
+  const int n_groups = !groups ? 1 : p.nk > SPG_SELECT_IN_ATTN_NK ? most : 2;
 #define SPG_ATTN(D_, PV16_, G_)                                                                             \
   {                                                                                                         \
     if (out_dtype == 0) block_sparse_attn_kernel<D_, 0, PV16_, SEL, G_><<<grid, 256 * G_, 0, st>>>(p);       \
@@ -1060,9 +1075,10 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   }
 #define SPG_ATTN_G(D_, PV16_)                                                                               \
   {                                                                                                         \
+    constexpr int GMAX = SEL ? 2 : D_ == 64 ? 4 : PV16_ ? 2 : 3;                                              \
     if (n_groups == 1) SPG_ATTN(D_, PV16_, 1)                                                                \
     else if (n_groups == 2) SPG_ATTN(D_, PV16_, 2)                                                           \
-    else if constexpr (D_ == 64 && !SEL) SPG_ATTN(D_, PV16_, 3)                                              \
+    else if constexpr (GMAX > 2) SPG_ATTN(D_, PV16_, GMAX)                                                   \
   }
   if (p.v_scale != nullptr) { if (D == 64) SPG_ATTN_G(64, false) else SPG_ATTN_G(128, false) }
   else { if (D == 64) SPG_ATTN_G(64, true) else SPG_ATTN_G(128, true) }   // fp16 V^T tiles, no V scale
