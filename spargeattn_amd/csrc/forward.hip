@@ -1,8 +1,10 @@
 // The whole operator behind one call: K mean, mask prediction + INT8 quantisation, V quantisation, block-sparse
-// attention, as three to five launches on workspace the caller hands over.
+// attention, as two to five launches on workspace the caller hands over.
 //
 // Short sequences are bound by the length of the launch chain and by kernels that cannot fill the chip, so stages that do
 // not depend on each other share a launch; which stage a workgroup belongs to follows from its number:
+//   short    (short heads) everything up to the selection: blocks of K and V, whose workgroups sum and search their whole head for
+//            themselves | mask rows | pooling + quantisation of Q.  Otherwise:
 //   front    partial column sums of K | partial channel maxima of V (FP16 PV: the V^T tiles, finished) | LUT rows of a
 //            user mask | pooling + quantisation of Q
 //   (final   column mean of K, channel maxima of V: only where there are too many partial results for every workgroup
@@ -178,6 +180,87 @@ __global__ __launch_bounds__(NT) void back_kernel(const BackParams p) {
   }
 }
 
+// Short heads: front and back in one launch.  Every workgroup that quantises a block of K sums the columns of its whole head for
+// itself, every one that quantises a block of V takes the maxima of its whole head; the rest are the front kernel's mask rows and Q
+// blocks.  Bound by the chain of one workgroup - its head from L2 (at most 256 KiB), the sums, then the block - which is shorter than
+// the two launches.
+struct ShortParams {
+  FrontParams f;
+  BackParams b;
+  int wg_v, wg_mask, wg_q;              // first workgroup of each role behind the blocks of K
+};
+template <int D, int DT, bool POOL, int QR>
+__global__ __launch_bounds__(512) void short_kernel(const ShortParams p) {
+  constexpr int NT = 512, ROWS = k_rows_per_wg(NT);
+  constexpr int LK = max_c<POOL ? psq_lds<64, D, NT, ROWS>() : 16, NT / 64 * 128 * 8 + 2 * D>();
+  constexpr int LV = max_c<max_c<v_quant_lds<D>(), v_absmax_lds<D, NT>()>() + 4 * D, v_tiles_f16_lds<D>()>();
+  constexpr int LQ = max_c<POOL ? psq_lds<128, D, NT>() : 16, POOL ? 16 : 4 * MASK_NKP_FRONT + 64>();
+  __shared__ __align__(16) unsigned char smem[max_c<max_c<LK, LV>(), LQ>()];
+  const int w = blockIdx.x;
+  const FrontParams &f = p.f;
+  const BackParams &b = p.b;
+  if (w == 0 && threadIdx.x < 8 && !POOL) f.queue[threadIdx.x] = 0;
+  if (w < p.wg_v) {
+    const int bh = w / b.k_wgs_per_head;
+    float thr = 0.f;
+    if constexpr (POOL) thr = b.simthr.at((bh % b.Hkv) * (b.H / b.Hkv));
+    psq_body<64, D, DT, MEAN_HERE, POOL, 64, NT, ROWS>(b.k, b.ks, nullptr, nullptr, 0, b.pool_k, b.sim_k, b.k8, b.k_scale, thr, b.Hkv, b.Nk, b.nk,
+                                                       w - bh * b.k_wgs_per_head, bh, smem);
+  } else if (w < p.wg_mask) {
+    const int id = w - p.wg_v, bh = id / b.nk, blk = id - bh * b.nk;
+    if (f.v_f16) {
+      if (f.v_dtype == 0) v_tiles_f16_body<D, 0, NT>(f.v, f.vs, f.Hkv, f.v_tiles, f.Nk, f.nk, blk, bh, smem);
+      else v_tiles_f16_body<D, 1, NT>(f.v, f.vs, f.Hkv, f.v_tiles, f.Nk, f.nk, blk, bh, smem);
+    } else {
+      float *const s_amax = (float *)(smem + max_c<v_quant_lds<D>(), v_absmax_lds<D, NT>()>());
+      auto store = [&](int d, float s) { s_amax[d] = s; };
+      if (b.v_dtype == 0) v_absmax_body<D, 0, NT>(b.v, b.vs, b.Hkv, b.Nk, b.Nk, 0, bh, smem, store);
+      else v_absmax_body<D, 1, NT>(b.v, b.vs, b.Hkv, b.Nk, b.Nk, 0, bh, smem, store);
+      __syncthreads();
+      if (blk == 0 && threadIdx.x < D) b.v_scale[(size_t)bh * D + threadIdx.x] = s_amax[threadIdx.x] / 2.25f;
+      auto amax_of = [&](int d) { return s_amax[d]; };
+      if (b.v_dtype == 0) v_quant_body<D, 0, NT>(b.v, b.vs, b.Hkv, b.v8, b.Nk, b.nk, blk, bh, smem, amax_of);
+      else v_quant_body<D, 1, NT>(b.v, b.vs, b.Hkv, b.v8, b.Nk, b.nk, blk, bh, smem, amax_of);
+    }
+  } else if (w >= p.wg_q) {
+    const int id = w - p.wg_q, bh = id / f.nq;
+    float thr = 0.f;
+    if constexpr (POOL) thr = f.simthr.at(bh % f.H);
+    psq_body<128, D, DT, MEAN_NONE, POOL, QR, NT>(f.q, f.qs, nullptr, nullptr, 0, f.pool_q, f.sim_q, f.q8, f.q_scale, thr, f.H, f.N, f.nq,
+                                                  id - bh * f.nq, bh, smem);
+  } else if constexpr (!POOL) {
+    const size_t row = (size_t)(w - p.wg_mask);
+#define SPG_M2L(K_) case K_: map_to_lut_body<K_, NT>(f.mask, f.lut, f.valid, f.nk, f.nkp, row, smem); break;
+    switch (f.mask_kind) { SPG_M2L(0) SPG_M2L(1) SPG_M2L(2) SPG_M2L(3) SPG_M2L(4) SPG_M2L(5) SPG_M2L(6) }
+#undef SPG_M2L
+  }
+}
+// One launch instead of front and back: a workgroup reads its whole head, so the head has to be short, and all of them together
+// read it once per block.  us per call with two launches / one, top-k H x N: D64 16 x 512 18.7 / 15.5, 2 x 1024 21.2 / 18.1, 8 x 1024 21.8 /
+// 19.0, 2 x 1500 30.0 / 28.9, 1 x 2048 25.4 / 24.4, 1 x 2500 38.2 / 38.7, 40 x 400 22.3 / 22.8; D128 8 x 128 18.3 / 14.1, 8 x 512 22.2 / 18.8, 4 x
+// 1024 25.2 / 23.9, 2 x 1200 32.2 / 31.7, 1 x 1500 35.5 / 36.0, 12 x 640 24.1 / 21.9, 30 x 512 25.8 / 27.0, 16 x 1024 30.6 / 34.7.  FP16 PV, whose V^T tiles need
+// no maxima: D128 30 x 512 27.1 / 23.8, 16 x 1024 32.0 / 28.5, 40 x 400 30.7 / 26.6, 2 x 1500 38.0 / 38.7.  With a similarity threshold, whose
+// work on a block outweighs the sums: D128 8 x 700 33.3 / 28.2, 20 x 700 41.1 / 38.5, 2 x 1500 40.1 / 38.0, 1 x 2048 45.1 / 44.6.
+static bool short_heads(const spg_attn_args *a, int kv_heads, int nk) {
+  const long long head = (long long)a->N_kv * a->D, all = head * kv_heads * nk;
+  const bool sim = a->selection != SPG_SELECT_MASK && (a->simthreshd1 != nullptr || a->simthreshd1_value >= 0.f);
+  return head <= (sim ? 262144 : 155648) && all <= (a->pv_f16 ? 34 << 20 : sim ? 20 << 20 : 12 << 20) &&
+         (long long)kv_heads * nk <= (a->pv_f16 ? 320 : 256);
+}
+template <int D, int DT>
+static void run_short(const spg_attn_args *a, const ShortParams &p, int wgs, hipStream_t st) {
+  const bool pool = a->selection != SPG_SELECT_MASK;
+  if constexpr (D == 128) {
+    if (a->qk_quant_gran == SPG_QUANT_PER_WARP) {
+      if (pool) short_kernel<D, DT, true, 32><<<wgs, 512, 0, st>>>(p);
+      else short_kernel<D, DT, false, 32><<<wgs, 512, 0, st>>>(p);
+      return;
+    }
+  }
+  if (pool) short_kernel<D, DT, true, 128><<<wgs, 512, 0, st>>>(p);
+  else short_kernel<D, DT, false, 128><<<wgs, 512, 0, st>>>(p);
+}
+
 template <int D, int DT, int NT>
 static void run_front_back(const spg_attn_args *a, const FrontParams &f, const BackParams &b, const Chunks &c, uint16_t *km, float *v_amax,
                            int front_wgs, int back_wgs, hipStream_t st) {
@@ -218,7 +301,9 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   // Fewer than two workgroups of 256 threads per CU leave the stages bound by the length of one thread's work (9.8 and
   // 13.0 us for the two launches at B2 H3 N1025 D128 with a similarity threshold): twice the threads take half of it.
   const int wgs256 = heads * nq + kv_heads * 2 * c.n;
-  const int nt = wgs256 <= 512 && !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP) ? 512 : 256;
+  const bool wide = !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP);
+  const bool one_launch = wide && short_heads(a, kv_heads, nk);
+  const int nt = one_launch || (wgs256 <= 512 && wide) ? 512 : 256;
   int nkp = 256;
   while (nkp < nk || nkp < nt) nkp <<= 1;
   const bool mask_in_front = !pool && nkp <= MASK_NKP_FRONT;
@@ -249,6 +334,15 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   b.pool_k = (uint16_t *)(ws + l.pool_k); b.sim_k = ws + l.sim_k; b.k8 = (int8_t *)(ws + l.k8); b.k_scale = (float *)(ws + l.k_scale);
   b.v8 = ws + l.v; b.v_scale = (float *)(ws + l.v_scale);
 
+  if (one_launch) {
+    ShortParams s = {f, b, 0, 0, 0};
+    s.wg_v = b.wg_v;
+    s.wg_mask = s.wg_v + kv_heads * nk;
+    s.wg_q = s.wg_mask + (mask_in_front ? heads * nq : 0);
+    const int wgs = s.wg_q + heads * nq;
+    if (a->D == 64) { if (a->qk_dtype == 0) run_short<64, 0>(a, s, wgs, st); else run_short<64, 1>(a, s, wgs, st); }
+    else            { if (a->qk_dtype == 0) run_short<128, 0>(a, s, wgs, st); else run_short<128, 1>(a, s, wgs, st); }
+  }
   const int front_wgs = f.wg_q + heads * nq, back_wgs = b.wg_v + (a->pv_f16 ? 0 : kv_heads * nk);
   uint16_t *km = (uint16_t *)(ws + l.km);
   float *v_amax = (float *)(ws + l.v_amax);
@@ -257,8 +351,9 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
     if (nt == 512) run_front_back<D_, DT_, 512>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);            \
     else run_front_back<D_, DT_, 256>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);                      \
   }
-  if (a->D == 64) { if (a->qk_dtype == 0) SPG_RUN(64, 0) else SPG_RUN(64, 1) }
-  else            { if (a->qk_dtype == 0) SPG_RUN(128, 0) else SPG_RUN(128, 1) }
+  if (one_launch) {}
+  else if (a->D == 64) { if (a->qk_dtype == 0) SPG_RUN(64, 0) else SPG_RUN(64, 1) }
+  else                 { if (a->qk_dtype == 0) SPG_RUN(128, 0) else SPG_RUN(128, 1) }
 #undef SPG_RUN
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

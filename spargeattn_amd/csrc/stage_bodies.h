@@ -138,8 +138,8 @@ __device__ __forceinline__ double2 fold_columns(const double (&x)[8]) {
 // are the rows of one wavefront of the attention kernel).  Pooling and the similarity flag stay per block.
 // MEAN: 0 no mean (Q), 1 the finished column mean `km`, 2 the partial column sums km_part (km_chunks per head) that
 // km_partial_body wrote - every workgroup adds them up for itself, which takes the small kernel in between out of the
-// launch chain and pays while there are few chunks.
-enum { MEAN_NONE = 0, MEAN_GIVEN = 1, MEAN_PARTIAL = 2 };
+// launch chain and pays while there are few chunks - 3 nothing but x: every workgroup sums the columns of its whole head.
+enum { MEAN_NONE = 0, MEAN_GIVEN = 1, MEAN_PARTIAL = 2, MEAN_HERE = 3 };
 // NT threads work on ROWS rows: 256 on 128 where there are enough workgroups to fill the chip, more threads on fewer rows
 // where there are not and the time is the length of one thread's work.
 template <int BS, int D, int NT = 256, int ROWS = 128> constexpr int psq_lds() { return ROWS / BS * (NT / 64 * 128 / D) * D * 8; }
@@ -192,6 +192,39 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
     uint4 v;
     if constexpr (MEAN == MEAN_GIVEN) {
       v = *(const uint4 *)(km + (size_t)bh * D + c * 8);
+    } else if constexpr (MEAN == MEAN_HERE) {
+      // (the sums are exact in binary64: their order is free)
+      constexpr int SG = NWV * 128 / D;                // partial sums per column (fold_columns)
+      double(*s_part)[D] = (double(*)[D])smem;
+      uint16_t *s_km = (uint16_t *)(smem + SG * D * 8);
+      const uint16_t *hb = x + (size_t)(bh / H) * xs.sb + (size_t)(bh % H) * xs.sh + c * 8;
+      double acc[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) acc[e] = 0.0;
+#pragma unroll 8
+      for (int row = r; row < N; row += RPP) {
+        const uint4 q = *(const uint4 *)(hb + (size_t)row * xs.sn);
+        const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          float f0, f1;
+          unpack2<DT>(qw[j], f0, f1);
+          acc[2 * j] += (double)f0;
+          acc[2 * j + 1] += (double)f1;
+        }
+      }
+      const int sg = D == 128 ? tid >> 6 : tid >> 6 << 1 | (tid >> 3 & 1);
+      *(double2 *)&s_part[sg][c * 8 + (tid >> 5 & 1) * 4 + (tid >> 4 & 1) * 2] = fold_columns(acc);
+      __syncthreads();
+      if (tid < D) {
+        double t = 0.0;
+#pragma unroll
+        for (int u = 0; u < SG; u++) t += s_part[u][tid];
+        s_km[tid] = f64_to_elem<DT>(t / (double)N);
+      }
+      __syncthreads();
+      v = *(const uint4 *)(s_km + c * 8);
+      __syncthreads();                                // the LDS is used again below
     } else {
       // (the sums are exact in binary64: their order is free)
       constexpr int G = NT / D;

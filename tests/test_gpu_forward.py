@@ -155,3 +155,23 @@ def test_long_heads_go_through_the_launch_in_between(H, Nk, D):
     for fn in (sa.spas_sage2_attn_meansim_topk_cuda, sa.spas_sage_attn_meansim_topk_cuda):
         o, o2 = _both(lambda: fn(q, k, v, topk=0.3, simthreshd1=0.1))
         assert torch.equal(_bits(o), _bits(o2))
+
+
+@pytest.mark.parametrize("Nk,D,Hkv", [(1, 64, 1), (1216, 128, 2), (1217, 128, 2), (2432, 64, 2), (2433, 64, 2), (2048, 128, 1), (2049, 128, 1),
+                                      (4096, 64, 2), (4097, 64, 2), (250, 64, 40), (250, 64, 42), (700, 128, 16)])
+def test_short_heads_in_one_launch(Nk, D, Hkv):
+    """Heads of up to 155648 elements (262144 with a similarity threshold) go from the inputs to the selection in one launch whose
+    workgroups sum and search the whole head; one row or one head more takes two.  Both sides of each line against the stages, with
+    non-finite elements in K and V, strided inputs, and a mask of the caller's own."""
+    N, Nk = 140, max(Nk, 128)
+    q, k, v = (rand_T((1, n, Hkv, D), torch.bfloat16, 50 + i, shift=0.2).transpose(1, 2) for i, n in enumerate((N, Nk, Nk)))
+    k[0, 0, Nk // 2, 3], v[0, 0, Nk - 1, 5], v[0, Hkv - 1, 0, 7] = float("nan"), float("nan"), float("inf")
+    mask = (torch.rand((1, Hkv, 2, (Nk + 63) // 64), generator=torch.Generator().manual_seed(Nk)) < 0.5).cuda()
+    mask[..., 0] = True
+    for fn in (lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.4, return_sparsity=True),
+               lambda: sa.spas_sage2_attn_meansim_cuda(q, k, v, cdfthreshd=0.8, simthreshd1=0.1, return_sparsity=True,
+                                                       qk_quant_gran=2 if D == 128 else 1),
+               lambda: sa.spas_sage_attn_meansim_topk_cuda(q, k, v, topk=0.6, return_sparsity=True),
+               lambda: sa.block_sparse_sage2_attn_cuda(q, k, v, mask_id=mask, return_sparsity=True)):
+        (o, s), (o2, s2) = _both(fn)
+        assert torch.equal(_bits(o), _bits(o2)) and s == s2
