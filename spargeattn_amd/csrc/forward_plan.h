@@ -15,6 +15,11 @@ namespace spg {
 // length of the front kernel (below 3 MiB of K).  us per call without / with the final kernel: one head D64 N12288 55.2 / 57.2,
 // N17776 166.4 / 168.9, N20480 83.8 / 84.4, N24000 215.1 / 215.2, N24576 97.0 / 96.0; D128 N8448 59.9 / 61.5, N11000 145.8 / 146.9,
 // N12000 157.9 / 157.8, N16384 94.6 / 93.5, N24576 132.0 / 126.3; two heads D128 N12288 80.9 / 80.9, with FP16 PV 88.9 / 88.3.
+// Many heads: sixteen chunks each already spread the read over the chip, and the rest of the front kernel (Q, and the other
+// heads) is long enough to hide that a chunk of up to 2048 rows takes its time - from about ten heads on, whatever N is.  us per call
+// with / without the final kernel: 30 heads D64 N17776 1031 / 1026, 48 heads N16384 908 / 891, 32 heads N10000 425 / 408, 10 heads N24000
+// 661 / 658; D128 12 heads N12000 385 / 380, 24 heads N9000 386.8 / 385.4, 32 heads N32768 causal 3913 / 3905; but 8 heads D64 N12000 193 /
+// 202, 6 heads D128 N16384 288 / 290.
 struct Chunks {
   int n, rows;
   bool partial;
@@ -22,8 +27,9 @@ struct Chunks {
 inline Chunks chunks_for(int heads, int N, int D) {
   Chunks c;
   const bool few = (long long)heads * N <= 24576 && (long long)N * D < 3 << 19;
-  c.partial = N <= 8192 || few;
-  const int want = N <= 8192 ? 16 : few ? 32 : (2048 + heads - 1) / heads;
+  const bool many = heads >= 12 && N <= 32768;
+  c.partial = N <= 8192 || few || many;
+  const int want = N <= 8192 || many ? 16 : few ? 32 : (2048 + heads - 1) / heads;
   const int most = N <= 8192 ? (N + 63) / 64 : (N + 255) / 256;
   c.n = want < most ? want : most;
   c.rows = (N + c.n - 1) / c.n;

@@ -175,3 +175,13 @@ def test_short_heads_in_one_launch(Nk, D, Hkv):
                lambda: sa.block_sparse_sage2_attn_cuda(q, k, v, mask_id=mask, return_sparsity=True)):
         (o, s), (o2, s2) = _both(fn)
         assert torch.equal(_bits(o), _bits(o2)) and s == s2
+
+
+@pytest.mark.parametrize("H,Nk,D", [(11, 8200, 128), (12, 8200, 128), (12, 32768, 64), (12, 32769, 64)])
+def test_many_heads_combine_partial_sums(H, Nk, D):
+    """From twelve heads on and up to 32768 rows a head has sixteen chunks that every workgroup adds up; both sides of either line."""
+    q = rand_T((1, H, 130, D), torch.bfloat16, 61)
+    k, v = rand_T((1, H, Nk, D), torch.bfloat16, 62, shift=0.3), rand_T((1, H, Nk, D), torch.float16, 63)
+    for fn in (sa.spas_sage2_attn_meansim_topk_cuda, sa.spas_sage_attn_meansim_topk_cuda):
+        o, o2 = _both(lambda: fn(q, k, v, topk=0.3, simthreshd1=0.1))
+        assert torch.equal(_bits(o), _bits(o2))
