@@ -221,9 +221,9 @@ __device__ __forceinline__ int v_swz(int row) { return (row >> 2) & 3; }
 //               sum on the tensor cores computes, qk_int_sv_f16_cuda_sm80.cuh:339-368, attn_utils.cuh:599-626).  The PV product is
 //               accumulated in fp32; the reference accumulates each 64-key block in fp16 before adding it to its fp32
 //               accumulator (attn_utils.cuh:683-751), a rounding this kernel does not reproduce.
-// SEL: rows of at most 64 blocks are selected here, by the workgroup that then works on them, instead of by a kernel in
-// front that writes a LUT: the row's map is one 64-bit scalar, and the next block is its next set bit.  Takes a launch
-// (about 4.5 us) and the selection kernel's 7-15 us out of the chain and puts about 3 us in.
+// SEL: rows of at most 64 SEL blocks are selected here, by the workgroup that then works on them, instead of by a kernel in
+// front that writes a LUT: the row's map is one or two 64-bit scalars, and the next block is its next set bit.  Takes a launch
+// (about 4.5 us) and the selection kernel's 7-15 us out of the chain and puts about 3 us in (SPG_SELECT_IN_ATTN_NK: where the line lies).
 // G: groups of four wavefronts that share one Q block.  G = 1 is the general kernel.  G > 1 is for grids that leave a row
 // alone on its CU (launch_attn): one wavefront per SIMD then waits out every latency of the chain scores - maximum -
 // exponentials - product by itself.  The groups take the blocks of the row in turn (group g: places g, g + G, ... of the
@@ -231,7 +231,7 @@ __device__ __forceinline__ int v_swz(int row) { return (row >> 2) & 3; }
 // running maximum of the blocks BEFORE it in the list, so the groups exchange their block maxima through LDS once per round
 // of G blocks (at the barrier that the rings need anyway), and so the PV-skip test sees the same differences.  O and the
 // denominator are per group and meet in the epilogue.
-template <int D, int ODT, bool PV16, bool SEL, int G>
+template <int D, int ODT, bool PV16, int SEL, int G>
 __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_kernel(const AttnParams p) {
   constexpr int KS = D / 32;        // k-steps of the int8 MFMA
   constexpr int NDT = D / 32;       // 32-channel output tiles
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   const uint32_t lds_v0 = lds_k0 + NBUF * TILE;
 
   int bh, qb, item = blockIdx.x;
-  if constexpr (!SEL) {                    // (short rows: the grid is over before the XCDs drift apart)
+  if constexpr (SEL == 0) {                    // (short rows: the grid is over before the XCDs drift apart)
     if (p.queue != nullptr) {
       __shared__ int sItem;
       if (threadIdx.x == 0) sItem = take_item(p, item);
@@ -290,11 +290,11 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   typedef const __attribute__((address_space(4))) int32_t *c_i32_t;
   typedef const __attribute__((address_space(4))) float *c_f32_t;
   const size_t row_id = (size_t)bh * p.nq + qb;
-  const c_i32_t lutc = (c_i32_t)(p.lut + (SEL ? 0 : row_id * p.nk));
+  const c_i32_t lutc = (c_i32_t)(p.lut + (SEL > 0 ? 0 : row_id * p.nk));
   const int last_col = p.nk - 1;
   int nv, l0, l1, l2, l3;
-  if constexpr (!SEL && G > 1) nv = ((c_i32_t)p.valid)[row_id];
-  if constexpr (!SEL && G == 1) {
+  if constexpr (SEL == 0 && G > 1) nv = ((c_i32_t)p.valid)[row_id];
+  if constexpr (SEL == 0 && G == 1) {
     nv = ((c_i32_t)p.valid)[row_id];
     l0 = lutc[0]; l1 = lutc[min(1, last_col)]; l2 = lutc[min(2, last_col)]; l3 = lutc[min(3, last_col)];
   }
@@ -309,33 +309,55 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     qreg[ks] = (v4i){0, 0, 0, 0};
     if (q_row < N) qreg[ks] = *(const v4i *)(p.q8 + ((size_t)bh * N + q_row) * D + 32 * ks + 16 * hh);
   }
-  uint64_t map = 0;                        // SEL: blocks not fetched yet
-  if constexpr (SEL) {
-    __shared__ uint16_t sScore[64];
+  constexpr int W = SEL > 0 ? SEL : 1;
+  uint64_t map[W] = {};                    // SEL: blocks not fetched yet
+  if constexpr (SEL > 0) {
+    __shared__ uint16_t sScore[64 * W];
     const uint8_t *simk = p.sel.sim_k + (size_t)bhk * p.nk;
     const bool row_forced = p.sel.sim_q[row_id] == 0;
-    const bool k_dead = simk[min(lane, last_col)] == 0;
-    if (grp == 0) {
-      const int col = tid >> 2;
-      const uint16_t s16 = pooled_score_4lanes<D, ODT>(p.sel.pool_q + row_id * D, p.sel.pool_k + ((size_t)bhk * p.nk + min(col, last_col)) * D, tid & 3);
-      if ((tid & 3) == 0) sScore[col] = s16;
+    bool k_dead[W];
+#pragma unroll
+    for (int t = 0; t < W; t++) k_dead[t] = simk[min(64 * t + lane, last_col)] == 0;
+    // 64 columns a turn, the groups take turns
+#pragma unroll
+    for (int t = 0; t < W; t++) {
+      if (G == 1 || t % G == grp) {
+        const int col = 64 * t + ((tid & 255) >> 2);
+        const uint16_t s16 = pooled_score_4lanes<D, ODT>(p.sel.pool_q + row_id * D, p.sel.pool_k + ((size_t)bhk * p.nk + min(col, last_col)) * D, tid & 3);
+        if ((tid & 3) == 0) sScore[col] = s16;
+      }
     }
     __syncthreads();
     const int causal_lim = p.sel.is_causal ? min(p.nk, 2 * (qb + 1)) : p.nk;
-    const float sc = (lane >= causal_lim || k_dead) ? -INFINITY : elem_to_f32<ODT>(sScore[lane]);
-    map = select_row64<ODT>(sc, k_dead, p.sel.by_topk, p.sel.level.at(head), p.nk, causal_lim, row_forced, p.sel.sink, lane);
-    nv = __builtin_popcountll(map);
+    float sc[W];
+#pragma unroll
+    for (int t = 0; t < W; t++) sc[t] = (64 * t + lane >= causal_lim || k_dead[t]) ? -INFINITY : elem_to_f32<ODT>(sScore[64 * t + lane]);
+    select_row<ODT, W>(map, sc, k_dead, p.sel.by_topk, p.sel.level.at(head), p.nk, causal_lim, row_forced, p.sel.sink, lane);
+    nv = 0;
+#pragma unroll
+    for (int t = 0; t < W; t++) nv += __builtin_popcountll(map[t]);
     if (p.sel.valid_out != nullptr && tid == 0) p.sel.valid_out[row_id] = nv;
   }
+  auto drop_lowest = [&]() __attribute__((always_inline)) {
+    bool below = true;                     // no lower word holds a block
+#pragma unroll
+    for (int t = 0; t < W; t++) {
+      const uint64_t w = map[t];
+      map[t] = below ? w & (w - 1) : w;    // (0 stays 0)
+      below = below && w == 0;
+    }
+  };
   // SEL: takes the next block (of this group) out of the map; beyond the last one it repeats `prev`
   auto next_block = [&](int prev) __attribute__((always_inline)) {
-    const int b = map != 0 ? __builtin_ctzll(map) : prev;
+    int b = prev;
 #pragma unroll
-    for (int i = 0; i < G; i++) map &= map - 1;
+    for (int t = W - 1; t >= 0; t--) b = map[t] != 0 ? 64 * t + __builtin_ctzll(map[t]) : b;
+#pragma unroll
+    for (int i = 0; i < G; i++) drop_lowest();
     return b;
   };
-  if constexpr (SEL && G > 1)
-    for (int i = 0; i < grp; i++) map &= map - 1;
+  if constexpr (SEL > 0 && G > 1)
+    for (int i = 0; i < grp; i++) drop_lowest();
   if (nv == 0) return;                                       // output rows stay unwritten (sm89.cuh:232-235)
 
   const int8_t *kbase = p.k8 + (size_t)bhk * Nk * D;
@@ -469,7 +491,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   // block ids: blk = block of iteration it, blk1 = it+1, blk2 = it+2 (tiles in flight); d3 = LUT delta of it+3.
   // K scales are fetched one iteration ahead as well.  With groups an iteration is a round: place it * G + grp of the list.
   int blk, blk1, blk2, d3 = 0;
-  if constexpr (!SEL && G > 1) {
+  if constexpr (SEL == 0 && G > 1) {
     // the LUT holds differences: running sums of its first entries, unused ones read as 0
     int at = 0, acc = 0;
     auto advance = [&](int upto) __attribute__((always_inline)) {
@@ -485,7 +507,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     advance(grp + 1 + 2 * G); blk2 = acc;
     acc = 0;
     advance(grp + 1 + 3 * G); d3 = acc;
-  } else if constexpr (SEL) {
+  } else if constexpr (SEL > 0) {
     blk = next_block(0);
     blk1 = next_block(blk);
     blk2 = next_block(blk1);
@@ -606,8 +628,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     int d4 = 0, d4g[G] = {};
     if constexpr (!TAIL || G > 1) {
       ksc2 = *(c_f32_t)((const __attribute__((address_space(4))) char *)kscale + (uint32_t)(blk2 << 2));
-      if constexpr (!SEL && G == 1) d4 = it + 4 < nv ? lutc[(uint32_t)(it + 4)] : 0;
-      if constexpr (!SEL && G > 1) {
+      if constexpr (SEL == 0 && G == 1) d4 = it + 4 < nv ? lutc[(uint32_t)(it + 4)] : 0;
+      if constexpr (SEL == 0 && G > 1) {
 #pragma unroll
         for (int i = 0; i < G; i++) d4g[i] = place + 3 * G + 1 + i < nv ? lutc[(uint32_t)(place + 3 * G + 1 + i)] : 0;
       }
@@ -902,12 +924,12 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
 #pragma unroll
       for (int i = 0; i < G; i++) d4 += d4g[i];
     } else if constexpr (!TAIL) {
-      if constexpr (SEL) asm volatile("" : "+s"(ksc2));
+      if constexpr (SEL > 0) asm volatile("" : "+s"(ksc2));
       else asm volatile("" : "+s"(ksc2), "+s"(d4));
     }
     // advance the block pipeline and the ring
     blk = blk1; blk1 = blk2;
-    if constexpr (SEL) blk2 = next_block(blk2);
+    if constexpr (SEL > 0) blk2 = next_block(blk2);
     else { blk2 = blk2 + d3; d3 = d4; }
     ksc = ksc1; ksc1 = ksc2;
     if constexpr (!CS) bufoff = bufoff == (NBUF - 1) * TILE ? 0 : bufoff + TILE;
@@ -1037,7 +1059,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   }
 }
 
-template <bool SEL>
+template <int SEL>
 static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_rows, hipStream_t st) {
   p.nq = (p.N + 127) / 128; p.nk = (p.Nk + 63) / 64;
   p.total_wg = p.nq * p.H * p.B;
@@ -1050,7 +1072,7 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   // 1138 / 1134, 48 x 24576 3624 / 3650, 12 x 65536 6161 / 6330, 11 x 90000 10188 / 10864.  Fewer rows per XCD: D64 8 x 16384 278 / 269,
   // 20 x 16384 628 / 618, 18 x 17000 647 / 641, D128 8 x 16384 396 / 389, 18 x 17000 894 / 901; causal D128 18 x 17000 724 / 714.
   const long long row = ((long long)p.nk * D) >> (causal_rows ? 1 : 0);
-  if (SEL || p.wg_per_xcd < SPG_QUEUE_MIN || row <= SPG_QUEUE_MIN_ROW) p.queue = nullptr;
+  if (SEL > 0 || p.wg_per_xcd < SPG_QUEUE_MIN || row <= SPG_QUEUE_MIN_ROW) p.queue = nullptr;
   const int grid = 8 * (p.queue != nullptr ? p.wg_per_xcd + p.wg_per_xcd / SPG_QUEUE_EXTRA : p.wg_per_xcd);
   // Causal rows differ in length throughout: all rows by length while the heads an XCD works on at once share its L2
   // anyway (grids of a few rounds), head by head beyond.  Otherwise only a partial last Q block stands out.
@@ -1067,7 +1089,7 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   // Beyond one row per CU the rows fill each other's gaps: H10 N4096 unchanged without groups.
   const bool groups = p.total_wg <= SPG_GROUPS_MAX_WG && p.nk >= SPG_GROUPS_MIN_NK && p.pv_mode == 1 && p.pv_count == nullptr;
   const int most = D == 64 ? 4 : p.v_scale != nullptr && p.total_wg >= 8 ? 3 : 2;
-  const int n_groups = !groups ? 1 : p.nk > SPG_SELECT_IN_ATTN_NK ? most : 2;
+  const int n_groups = !groups ? 1 : p.nk > 64 ? most : 2;
 #define SPG_ATTN(D_, PV16_, G_)                                                                             \
   {                                                                                                         \
     if (out_dtype == 0) block_sparse_attn_kernel<D_, 0, PV16_, SEL, G_><<<grid, 256 * G_, 0, st>>>(p);       \
@@ -1075,7 +1097,7 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   }
 #define SPG_ATTN_G(D_, PV16_)                                                                               \
   {                                                                                                         \
-    constexpr int GMAX = SEL ? 2 : D_ == 64 ? 4 : PV16_ ? 2 : 3;                                              \
+    constexpr int GMAX = SEL == 1 ? 2 : D_ == 64 ? 4 : PV16_ ? 2 : 3;                                              \
     if (n_groups == 1) SPG_ATTN(D_, PV16_, 1)                                                                \
     else if (n_groups == 2) SPG_ATTN(D_, PV16_, 2)                                                           \
     else if constexpr (GMAX > 2) SPG_ATTN(D_, PV16_, GMAX)                                                   \
@@ -1101,9 +1123,10 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
   p.is_causal = is_causal;
   p.pv_mode = pv_mode;
   p.q_per_warp = q_per_warp;
-  if (sel == nullptr) return launch_attn<false>(p, D, out_dtype, causal_rows || is_causal, st);
+  if (sel == nullptr) return launch_attn<0>(p, D, out_dtype, causal_rows || is_causal, st);
   p.sel = *sel;
-  return launch_attn<true>(p, D, out_dtype, causal_rows || is_causal, st);
+  if (Nk <= 64 * 64) return launch_attn<1>(p, D, out_dtype, causal_rows || is_causal, st);
+  return launch_attn<2>(p, D, out_dtype, causal_rows || is_causal, st);
 }
 
 hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,

@@ -10,7 +10,7 @@
 //   (final   column mean of K, channel maxima of V: only where there are too many partial results for every workgroup
 //            of the next launch to add them up for itself)
 //   back     pooling + quantisation of K | V -> e4m3 tiles and scales
-//   select   block_select_* of maskpred.hip (rows of more than 64 blocks; shorter ones are selected inside the next launch)
+//   select   block_select_* of maskpred.hip (rows of more than 128 blocks; shorter ones are selected inside the next launch)
 //   attn     block_sparse_attn_kernel
 // Every body is the one the stage-by-stage entry points launch (stage_bodies.h): results are the same bits.
 // The extern "C" entry points and their argument checks are in capi.hip, the workspace layout in forward_plan.h.

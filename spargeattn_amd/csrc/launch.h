@@ -56,8 +56,11 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st);
 // What the attention kernel needs to select a row's blocks by itself (rows of at most SPG_SELECT_IN_ATTN_NK blocks):
-// the arguments of launch_block_select_h
-#define SPG_SELECT_IN_ATTN_NK 64
+// the arguments of launch_block_select_h.  us per call with a selection kernel / in place, 65 to 128 blocks: D128 H1 N8192 76.6 / 71.1,
+// H8 127.3 / 120.5, H24 310 / 305, FP16 PV H24 causal 326 / 320, CDF H20 N7000 386 / 381; D64 H4 62.4 / 59.2, H40 337.5 / 337.8.  129 to
+// 256 blocks would gain at D128 (H8 N9000 190.3 / 186.7, H1 119.0 / 119.6) and lose at D64 (H2 N16384 95.8 / 105.4, H20 N16000 570 / 580),
+// FP16 PV (H10 N12000 380 / 387) and on long grids (H16 N16000 671 / 679).
+#define SPG_SELECT_IN_ATTN_NK 128
 struct RowSelect {
   const uint16_t *pool_q, *pool_k;
   const uint8_t *sim_q, *sim_k;

@@ -80,8 +80,8 @@ __device__ __forceinline__ void bitonic_sort_desc(uint32_t (&key)[EPL], int lane
 }
 
 // =============================================================================================
-// A whole row of at most 64 columns in one wavefront: lane = column.  Same arithmetic as block_select_wave_kernel with one
-// column per lane, and the result stays a 64-bit map: bit j = column j is kept.
+// A whole row of at most 64 W columns in one wavefront: lane l holds columns l, l + 64, ...  Same arithmetic as
+// block_select_wave_kernel with W columns per lane, and the result stays a map of W 64-bit words: bit j = column j is kept.
 // =============================================================================================
 // Pooled score of row `qrow` (D elements) against a pooled K row, by the four lanes of a group: lane `part` takes the
 // 16-byte pieces part, part + 4, ...  Products of two 16-bit floats and their sums are exact in binary64, so the order of
@@ -111,49 +111,71 @@ __device__ __forceinline__ uint16_t pooled_score_4lanes(const uint16_t *__restri
   return f64_to_elem_fast<DT>((double)s1 * (double)sm_scale);
 }
 
-// sc: the score of column `lane`, -inf where the column is masked (beyond nk, dissimilar K block, causal).
-// k_dead: column `lane` is a dissimilar K block (kept in every row).
-template <int DT>
-__device__ __forceinline__ uint64_t select_row64(float sc, bool k_dead, bool by_topk, float level, int nk, int causal_lim,
-                                                 bool row_forced, bool sink, int lane) {
+// sc[t]: the score of column 64 t + lane, -inf where the column is masked (beyond nk, dissimilar K block, causal).
+// k_dead[t]: that column is a dissimilar K block (kept in every row).
+template <int DT, int W>
+__device__ __forceinline__ void select_row(uint64_t (&map)[W], const float (&sc)[W], const bool (&k_dead)[W], bool by_topk, float level,
+                                           int nk, int causal_lim, bool row_forced, bool sink, int lane) {
 #pragma clang fp contract(off)
-  const float mx = wave_max_f32(sc);
-  const double ev = (sc == -INFINITY) ? 0.0 : cexp((double)sc - (double)mx);
-  const double total = wave_tree_sum_f64(ev);
-  double p = ev / total;
-  if (!__builtin_isfinite(p)) p = 0.0;
-  const uint32_t okey = lane < nk ? (((uint32_t)f64_to_elem_fast<DT>(p) << 16) | (0xffffu - (uint32_t)lane)) : 0u;
+  constexpr int LOW = W == 1 ? 6 : 7;                   // log2(64 W)
+  static_assert(W == 1 || W == 2, "columns per lane");
+  float lmax = sc[0];
+#pragma unroll
+  for (int t = 1; t < W; t++) lmax = fmaxf(lmax, sc[t]);
+  const float mx = wave_max_f32(lmax);
+  double ev[W], part = 0.0;
+#pragma unroll
+  for (int t = 0; t < W; t++) {
+    ev[t] = (sc[t] == -INFINITY) ? 0.0 : cexp((double)sc[t] - (double)mx);
+    part = part + ev[t];
+  }
+  const double total = wave_tree_sum_f64(part);
+  uint32_t okey[W];
+#pragma unroll
+  for (int t = 0; t < W; t++) {
+    double p = ev[t] / total;
+    if (!__builtin_isfinite(p)) p = 0.0;
+    const int j = 64 * t + lane;
+    okey[t] = j < nk ? (((uint32_t)f64_to_elem_fast<DT>(p) << 16) | (0xffffu - (uint32_t)j)) : 0u;
+  }
   int n;
   uint32_t kth = 0u;
   if (by_topk) {
     const float t = level * (float)nk;                  // binary32 product, truncated (utils.py:405)
-    n = (int)fminf(fmaxf(t, 0.f), 64.f);
+    n = (int)fminf(fmaxf(t, 0.f), 64.f * W);
     if (n <= 0) n = 1;                                  // utils.py:289
     if (n < nk) {
-      // n-th largest key, bit by bit (bits 31 and 30 are clear, 15..6 are set in every real key); a candidate that exactly
+      // n-th largest key, bit by bit (bits 31 and 30 are clear, 15..LOW are set in every real key); a candidate that exactly
       // n keys reach selects the same set
       uint32_t T = 0u;
       bool exact = false;
       auto try_bit = [&](int bit) {
         const uint32_t cand = T | (1u << bit);
-        const int cnt = __builtin_popcountll(__ballot(okey >= cand));
+        int cnt = 0;
+#pragma unroll
+        for (int t = 0; t < W; t++) cnt += __builtin_popcountll(__ballot(okey[t] >= cand));
         if (cnt >= n) T = cand;
         exact = cnt == n;
       };
 #pragma unroll 1
       for (int bit = 29; bit >= 16 && !exact; bit--) try_bit(bit);
       if (!exact) {
-        T |= 0xffc0u;
+        T |= 0xffffu & ~((1u << LOW) - 1u);
 #pragma unroll 1
-        for (int bit = 5; bit >= 0 && !exact; bit--) try_bit(bit);
+        for (int bit = LOW - 1; bit >= 0 && !exact; bit--) try_bit(bit);
       }
       kth = T;
     }
   } else {
-    uint32_t key[1] = {okey};
-    bitonic_sort_desc<1, 2>(key, lane);
-    // cdf[v] = T(sum_{u<=v} p_sorted[u]);  n = #{v < nk : cdf[v] <= threshold}  (utils.py:398-403)
-    double run = (double)elem_to_f32<DT>((uint16_t)(key[0] >> 16));
+    uint32_t key[W];
+#pragma unroll
+    for (int t = 0; t < W; t++) key[t] = okey[t];
+    bitonic_sort_desc<W, 2>(key, lane);                 // sorted position of key[t] is lane * W + t
+    // cdf[v] = T(sum_{u<=v} p_sorted[u]);  n = #{v < nk : cdf[v] <= threshold}  (utils.py:398-403); the sums are exact
+    double own = 0.0;
+#pragma unroll
+    for (int t = 0; t < W; t++) own += (double)elem_to_f32<DT>((uint16_t)(key[t] >> 16));
+    double run = own;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const uint64_t u = __builtin_bit_cast(uint64_t, run);
@@ -161,18 +183,33 @@ __device__ __forceinline__ uint64_t select_row64(float sc, bool k_dead, bool by_
       const double before = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
       run = lane >= o ? run + before : run;
     }
-    const float cdfv = elem_to_f32<DT>(f64_to_elem<DT>(run));
-    n = __builtin_popcountll(__ballot(lane < nk && (double)cdfv <= (double)level));
+    n = 0;
+    if constexpr (W > 1) run -= own;                    // of the lanes before this one
+#pragma unroll
+    for (int t = 0; t < W; t++) {
+      if constexpr (W > 1) run += (double)elem_to_f32<DT>((uint16_t)(key[t] >> 16));
+      const float cdfv = elem_to_f32<DT>(f64_to_elem<DT>(run));
+      n += __builtin_popcountll(__ballot(lane * W + t < nk && (double)cdfv <= (double)level));
+    }
     if (n <= 0) n = 1;                                  // utils.py:289
-    if (n < nk) kth = (uint32_t)__shfl((int)key[0], n - 1, SPG_WAVE);
+    if (n < nk) {                                       // wavefront-uniform
+      uint32_t mine = key[0];
+#pragma unroll
+      for (int t = 1; t < W; t++) mine = (n - 1) % W == t ? key[t] : mine;
+      kth = (uint32_t)__shfl((int)mine, (n - 1) / W, SPG_WAVE);
+    }
   }
-  bool f = false;
-  if (lane < nk) {
-    f = row_forced || okey >= kth || k_dead;
-    if (lane >= causal_lim) f = false;
-    if (sink && lane == 0) f = true;
+#pragma unroll
+  for (int t = 0; t < W; t++) {
+    const int j = 64 * t + lane;
+    bool f = false;
+    if (j < nk) {
+      f = row_forced || okey[t] >= kth || k_dead[t];
+      if (j >= causal_lim) f = false;
+      if (sink && j == 0) f = true;
+    }
+    map[t] = __ballot(f);
   }
-  return __ballot(f);
 }
 
 }  // namespace spg

@@ -185,3 +185,22 @@ def test_many_heads_combine_partial_sums(H, Nk, D):
     for fn in (sa.spas_sage2_attn_meansim_topk_cuda, sa.spas_sage_attn_meansim_topk_cuda):
         o, o2 = _both(lambda: fn(q, k, v, topk=0.3, simthreshd1=0.1))
         assert torch.equal(_bits(o), _bits(o2))
+
+
+@pytest.mark.parametrize("Nk", [4097, 6000, 8192])
+@pytest.mark.parametrize("D", [64, 128])
+def test_two_columns_per_lane_in_place(Nk, D):
+    """Rows of 65 to 128 blocks are selected by the attention kernel with two columns per lane: equal probabilities on both sides of
+    column 64, levels that keep one block, all of them, or nothing but dissimilar ones, in the general kernel and with groups."""
+    for H in (2, 130):
+        q = rand_T((1, H, 256, D), torch.bfloat16, 71)
+        k = rand_T((1, H, 1, D), torch.bfloat16, 72).expand(1, H, Nk, D).contiguous()
+        k[:, :, 130:200], k[:, :, 4000:4160] = rand_T((1, H, 70, D), torch.bfloat16, 74), rand_T((1, H, 160, D), torch.bfloat16, 75)
+        v = rand_T((1, H, Nk, D), torch.bfloat16, 73)
+        for kw in (dict(topk=0.0), dict(topk=1.0), dict(topk=0.5), dict(topk=0.37, is_causal=True), dict(topk=0.2, simthreshd1=0.9),
+                   dict(topk=0.3, attention_sink=True)):
+            (o, s), (o2, s2) = _both(lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, return_sparsity=True, **kw))
+            assert torch.equal(_bits(o), _bits(o2)) and s == s2, (H, kw)
+        for cdf in (0.0, 0.5, 0.97, 1.0):
+            (o, s), (o2, s2) = _both(lambda: sa.spas_sage2_attn_meansim_cuda(q, k, v, cdfthreshd=cdf, simthreshd1=0.5, return_sparsity=True))
+            assert torch.equal(_bits(o), _bits(o2)) and s == s2, (H, cdf)
