@@ -195,7 +195,7 @@ def test_two_columns_per_lane_in_place(Nk, D):
     for H in (2, 130):
         q = rand_T((1, H, 256, D), torch.bfloat16, 71)
         k = rand_T((1, H, 1, D), torch.bfloat16, 72).expand(1, H, Nk, D).contiguous()
-        k[:, :, 130:200], k[:, :, 4000:4160] = rand_T((1, H, 70, D), torch.bfloat16, 74), rand_T((1, H, 160, D), torch.bfloat16, 75)
+        k[:, :, 130:200], k[:, :, 4000:4160] = rand_T((1, H, 70, D), torch.bfloat16, 74), rand_T((1, H, 160, D), torch.bfloat16, 75)[:, :, :Nk - 4000]
         v = rand_T((1, H, Nk, D), torch.bfloat16, 73)
         for kw in (dict(topk=0.0), dict(topk=1.0), dict(topk=0.5), dict(topk=0.37, is_causal=True), dict(topk=0.2, simthreshd1=0.9),
                    dict(topk=0.3, attention_sink=True)):
