@@ -547,9 +547,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   // TAIL = true: the last two blocks - token-causal and out-of-bound masks where a score needs them, no skip
   // (sm89.cuh:467-648).  The two are
   // separate loops so that the common one carries none of the tail's predicates.
-  // SLOT = 0, 1, 2: the ring slot of the block is a compile-time constant (the common loop is unrolled three times), so
+  // SLOT = 0, 1, 2: the ring slot of the block is a compile-time constant (the common loop is unrolled over the ring), so
   // every LDS address of the iteration is a loop-invariant register plus an immediate offset; SLOT = -1: the slot is the
-  // run-time value `bufoff` (the up to two left-over blocks of the common loop and the two tail blocks).
+  // run-time value `bufoff` (the left-over blocks of the common loop and the two tail blocks).
   uint32_t kaddr_c[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) kaddr_c[ks] = lds_k0 + k_rd_base + ((uint32_t)(32 * ks) ^ k_rd_x);
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   auto step = [&](auto tail_tag, auto slot_tag, const int it) __attribute__((always_inline)) {
     constexpr bool TAIL = decltype(tail_tag)::value;
     constexpr int SLOT = decltype(slot_tag)::value;
-    constexpr bool CS = SLOT >= 0 && !PV16;         // compile-time ring slot
+    constexpr bool CS = SLOT >= 0;                  // compile-time ring slot
     const int place = G == 1 ? it : it * G + grp;   // in the row's list of blocks
     // groups: a round at the end can hold ordinary blocks, the last two and places beyond the list side by side
     const bool tail = TAIL && (G == 1 || place >= nv - 2), active = !TAIL || G == 1 || place < nv;
@@ -754,8 +754,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       // (it + 1) % 2 (the previous block's P.V product)
       SPG_LANE_OFFSETS()
       (void)pos0;
-      if (!TAIL || it + 2 < nv) SPG_LOAD_K_(blk2, bufoff, (TAIL || SLOT < 0));
-      if (!TAIL || it + 1 < nv) SPG_LOAD_V_(blk1, 2 * (bufoff ^ (uint32_t)TILE));
+      const uint32_t here = CS ? (uint32_t)(SLOT * TILE) : bufoff;
+      if (!TAIL || it + 2 < nv) SPG_LOAD_K_(blk2, here, (TAIL || SLOT < 0));
+      if (!TAIL || it + 1 < nv) SPG_LOAD_V_(blk1, 2 * (here ^ (uint32_t)TILE));
     } else if (!TAIL || place + 2 * G < nv) {
       if constexpr (CS) {
         SPG_LOAD_TILES(blk2, ((SLOT + 2) % 3) * TILE, 0);
@@ -862,12 +863,13 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
         }
         // V^T operands: two 16-key steps in registers, each replaced by the one after next as soon as its products are issued.
         // (Two halves of two steps, every read waited for at once: H24 N8192 D128 causal 334 us, so 332; 4 heads N8192, two groups, 98.9 / 97.7.)
-        const uint32_t va = lds_v0 + 2 * bufoff + v_rd16;
+        constexpr int SB = CS ? SLOT * VTILE : 0;    // ring slot as an immediate, or in the address register
+        const uint32_t va = lds_v0 + v_rd16 + (CS ? 0u : 2 * bufoff);
         v4i t[4][NDT];
         auto read_v = [&](int st) __attribute__((always_inline)) {
           const uint32_t a_ = va ^ (uint32_t)(16 * st);
-          if constexpr (NDT == 4) lds_read_4x128<0, 4096, 8192, 12288>(t[st][0], t[st][1], t[st][2], t[st][3], a_);
-          else lds_read_2x128<0, 4096>(t[st][0], t[st][1], a_);
+          if constexpr (NDT == 4) lds_read_4x128<SB, SB + 4096, SB + 8192, SB + 12288>(t[st][0], t[st][1], t[st][2], t[st][3], a_);
+          else lds_read_2x128<SB, SB + 4096>(t[st][0], t[st][1], a_);
         };
         auto wait_v = [&](int st, auto but) __attribute__((always_inline)) {
           if constexpr (NDT == 4) lds_wait_but<decltype(but)::value>(t[st][0], t[st][1], t[st][2], t[st][3]);
@@ -939,8 +941,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     // rounds whose successor's successor ends in front of the last block (no partial tile to load); rounds in front of the
     // last two blocks; all rounds
     const int n_fast = G == 1 ? nv - 3 : (nv - 1) / G - 2, n_common = G == 1 ? nv - 2 : (nv - 2) / G, n_all = (nv + G - 1) / G;
-    // the common loop, three blocks per trip (ring slots 0, 1, 2); `bufoff` stays 0 throughout where the slots are
-    // compile-time constants, and three run-time steps bring it back to 0 where they are not
+    // the common loop, one block per ring slot and trip; the slots are compile-time constants and `bufoff` stays 0.  (FP16 PV with
+    // run-time slots: H24 N8192 D128 causal 333 us, so 329; H6 N16384 381 / 377, H10 N5000 122 / 120, H1 N12000 D64 121 / 119.)
     // The wavefronts of a SIMD are served oldest first: of the three rows on a CU the first runs at almost the speed it would
     // have alone, the last gets what is left and ends alone, at less than half the rate of three (three rows of 32 blocks ended
     // at 50, 67 and 83 us).  While other rows wait for a place that is welcome.  The rows of an XCD that none wait for lower
@@ -954,7 +956,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       if ((item >> 3) >= p.wg_per_xcd - SPG_PLACES) drop_at = nv >> 1;
     }
 #pragma unroll 1
-    for (; it + 3 <= n_fast; it += 3) {
+    for (; it + NBUF <= n_fast; it += NBUF) {
       if constexpr (G == 1) {
         if (it >= drop_at) {
           const int d2 = nv - (nv >> 2), d3 = nv - (nv >> 3);
@@ -966,7 +968,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       }
       step(std::false_type{}, std::integral_constant<int, 0>{}, it);
       step(std::false_type{}, std::integral_constant<int, 1>{}, it + 1);
-      step(std::false_type{}, std::integral_constant<int, 2>{}, it + 2);
+      if constexpr (NBUF == 3) step(std::false_type{}, std::integral_constant<int, 2>{}, it + 2);
     }
 #pragma unroll 1
     for (; it < n_common; it++) step(std::false_type{}, std::integral_constant<int, -1>{}, it);
