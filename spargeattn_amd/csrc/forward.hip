@@ -235,18 +235,6 @@ __global__ __launch_bounds__(512) void short_kernel(const ShortParams p) {
 #undef SPG_M2L
   }
 }
-// One launch instead of front and back: a workgroup reads its whole head, so the head has to be short, and all of them together
-// read it once per block.  us per call with two launches / one, top-k H x N: D64 16 x 512 18.7 / 15.5, 2 x 1024 21.2 / 18.1, 8 x 1024 21.8 /
-// 19.0, 2 x 1500 30.0 / 28.9, 1 x 2048 25.4 / 24.4, 1 x 2500 38.2 / 38.7, 40 x 400 22.3 / 22.8; D128 8 x 128 18.3 / 14.1, 8 x 512 22.2 / 18.8, 4 x
-// 1024 25.2 / 23.9, 2 x 1200 32.2 / 31.7, 1 x 1500 35.5 / 36.0, 12 x 640 24.1 / 21.9, 30 x 512 25.8 / 27.0, 16 x 1024 30.6 / 34.7.  FP16 PV, whose V^T tiles need
-// no maxima: D128 30 x 512 27.1 / 23.8, 16 x 1024 32.0 / 28.5, 40 x 400 30.7 / 26.6, 2 x 1500 38.0 / 38.7.  With a similarity threshold, whose
-// work on a block outweighs the sums: D128 8 x 700 33.3 / 28.2, 20 x 700 41.1 / 38.5, 2 x 1500 40.1 / 38.0, 1 x 2048 45.1 / 44.6.
-static bool short_heads(const spg_attn_args *a, int kv_heads, int nk) {
-  const long long head = (long long)a->N_kv * a->D, all = head * kv_heads * nk;
-  const bool sim = a->selection != SPG_SELECT_MASK && (a->simthreshd1 != nullptr || a->simthreshd1_value >= 0.f);
-  return head <= (sim ? 262144 : 155648) && all <= (a->pv_f16 ? 34 << 20 : sim ? 20 << 20 : 12 << 20) &&
-         (long long)kv_heads * nk <= (a->pv_f16 ? 320 : 256);
-}
 template <int D, int DT>
 static void run_short(const spg_attn_args *a, const ShortParams &p, int wgs, hipStream_t st) {
   const bool pool = a->selection != SPG_SELECT_MASK;
@@ -302,7 +290,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   // 13.0 us for the two launches at B2 H3 N1025 D128 with a similarity threshold): twice the threads take half of it.
   const int wgs256 = heads * nq + kv_heads * 2 * c.n;
   const bool wide = !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP);
-  const bool one_launch = wide && short_heads(a, kv_heads, nk);
+  const bool one_launch = wide && short_heads(a);
   const int nt = one_launch || (wgs256 <= 512 && wide) ? 512 : 256;
   int nkp = 256;
   while (nkp < nk || nkp < nt) nkp <<= 1;

@@ -1,5 +1,5 @@
-// Host side of the whole-operator call, free of device code: how the partial sums are split, where everything lies in the
-// workspace.  Shared by the entry points (capi.hip) and the launches (forward.hip).
+// Host side of the whole-operator call, free of device code: which launches it takes, how the partial sums are split, where
+// everything lies in the workspace.  Shared by the entry points (capi.hip) and the launches (forward.hip).
 #pragma once
 #include "../../include/spargeattn_amd.h"
 #include "launch.h"
@@ -35,6 +35,25 @@ inline Chunks chunks_for(int heads, int N, int D) {
   c.rows = (N + c.n - 1) / c.n;
   c.n = (N + c.rows - 1) / c.rows;      // no chunk without rows
   return c;
+}
+
+// One launch instead of front and back (short_kernel): a workgroup reads its whole head, so the head has to be short, and all of
+// them together read it once per block.  us per call with two launches / one, top-k H x N: D64 16 x 512 18.7 / 15.5, 2 x 1024 21.2 /
+// 18.1, 8 x 1024 21.8 / 19.0, 2 x 1500 30.0 / 28.9, 1 x 2048 25.4 / 24.4, 1 x 2500 38.2 / 38.7, 40 x 400 22.3 / 22.8; D128 8 x 128 18.3 /
+// 14.1, 8 x 512 22.2 / 18.8, 4 x 1024 25.2 / 23.9, 2 x 1200 32.2 / 31.7, 1 x 1500 35.5 / 36.0, 12 x 640 24.1 / 21.9, 30 x 512 25.8 / 27.0, 16 x
+// 1024 30.6 / 34.7.  FP16 PV, whose V^T tiles need no maxima: D128 30 x 512 27.1 / 23.8, 16 x 1024 32.0 / 28.5, 40 x 400 30.7 / 26.6, 2 x 1500
+// 38.0 / 38.7.  With a similarity threshold, whose work on a block outweighs the sums: D128 8 x 700 33.3 / 28.2, 20 x 700 41.1 / 38.5, 2 x
+// 1500 40.1 / 38.0, 1 x 2048 45.1 / 44.6.
+// Many queries over short heads: beyond about 1024 Q blocks the blocks of Q are most of the launch, and those go faster through the
+// front kernel's 256 threads than through 512.  H, Nk, Q blocks: D128 8 x 512 1024 46.8 / 43.4, 24 x 512 768 40.3 / 40.5, 1536 58.6 / 60.5,
+// 6144 172.6 / 183.5, 40 x 256 1280 47.0 / 45.8, 2560 72.2 / 73.9; D64 16 x 512 1024 35.5 / 32.6, 2048 50.8 / 52.7, 36 x 400 1152 42.9 / 42.5, 4608
+// 92.5 / 106.0; FP16 PV 16 x 1024 1024 62.1 / 61.4, 30 x 512 1920 73.0 / 75.3; similarity 8 x 700 1024 76.1 / 72.1, 20 x 700 1280 88.3 / 89.2.
+inline bool short_heads(const spg_attn_args *a) {
+  const long long nq = (a->N + 127) / 128, nk = (a->N_kv + 63) / 64, kv_heads = (long long)a->B * a->Hkv;
+  const long long head = (long long)a->N_kv * a->D, all = head * kv_heads * nk;
+  const bool sim = a->selection != SPG_SELECT_MASK && (a->simthreshd1 != nullptr || a->simthreshd1_value >= 0.f);
+  return head <= (sim ? 262144 : 155648) && all <= (a->pv_f16 ? 34 << 20 : sim ? 20 << 20 : 12 << 20) &&
+         kv_heads * nk <= (a->pv_f16 ? 320 : 256) && (long long)a->B * a->H * nq <= 1024;
 }
 
 struct Layout {

@@ -1,0 +1,14 @@
+// Prints the route of whole-operator calls, one line per call read from standard input:
+//   B H Hkv N N_kv D selection pv_f16 simthreshd1  ->  one_launch
+// The rules are host code (spargeattn_amd/csrc/forward_plan.h); nothing is launched.
+#include "forward_plan.h"
+
+#include <cstdio>
+
+int main() {
+  spg_attn_args a = {};
+  a.qk_quant_gran = SPG_QUANT_PER_BLOCK;
+  while (std::scanf("%d %d %d %d %d %d %d %d %f", &a.B, &a.H, &a.Hkv, &a.N, &a.N_kv, &a.D, &a.selection, &a.pv_f16, &a.simthreshd1_value) == 9)
+    std::printf("%d\n", (int)spg::short_heads(&a));
+  return 0;
+}

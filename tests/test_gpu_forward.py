@@ -204,3 +204,15 @@ def test_two_columns_per_lane_in_place(Nk, D):
         for cdf in (0.0, 0.5, 0.97, 1.0):
             (o, s), (o2, s2) = _both(lambda: sa.spas_sage2_attn_meansim_cuda(q, k, v, cdfthreshd=cdf, simthreshd1=0.5, return_sparsity=True))
             assert torch.equal(_bits(o), _bits(o2)) and s == s2, (H, cdf)
+
+
+@pytest.mark.parametrize("N", [16384, 16385])
+@pytest.mark.parametrize("D", [64, 128])
+def test_many_queries_over_short_heads(N, D):
+    """1024 Q blocks over short heads are the last that go through one launch in front of the attention; one row more takes two."""
+    q = rand_T((1, 8, N, D), torch.bfloat16, 81)
+    k, v = rand_T((1, 8, 500, D), torch.bfloat16, 82, shift=0.3), rand_T((1, 8, 500, D), torch.float16, 83)
+    for fn in (lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.3, return_sparsity=True),
+               lambda: sa.spas_sage_attn_meansim_cuda(q, k, v, cdfthreshd=0.8, simthreshd1=0.1, return_sparsity=True)):
+        (o, s), (o2, s2) = _both(fn)
+        assert torch.equal(_bits(o), _bits(o2)) and s == s2
