@@ -281,7 +281,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   unsigned char *ws = (unsigned char *)a->workspace;
   const int heads = a->B * a->H, kv_heads = a->B * a->Hkv;
   const int nq = (a->N + 127) / 128, nk = (a->N_kv + 63) / 64;
-  const Chunks c = chunks_for(kv_heads, a->N_kv, a->D);
+  const Chunks c = chunks_for(a);
   const bool pool = a->selection != SPG_SELECT_MASK;
   const Hyper simthr = {a->simthreshd1, a->simthreshd1_value};
   int32_t *const lut = (int32_t *)(ws + l.lut);

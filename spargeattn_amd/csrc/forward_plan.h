@@ -15,19 +15,28 @@ namespace spg {
 // length of the front kernel (below 3 MiB of K).  us per call without / with the final kernel: one head D64 N12288 55.2 / 57.2,
 // N17776 166.4 / 168.9, N20480 83.8 / 84.4, N24000 215.1 / 215.2, N24576 97.0 / 96.0; D128 N8448 59.9 / 61.5, N11000 145.8 / 146.9,
 // N12000 157.9 / 157.8, N16384 94.6 / 93.5, N24576 132.0 / 126.3; two heads D128 N12288 80.9 / 80.9, with FP16 PV 88.9 / 88.3.
-// Many heads: sixteen chunks each already spread the read over the chip, and the rest of the front kernel (Q, and the other
-// heads) is long enough to hide that a chunk of up to 2048 rows takes its time - from about ten heads on, whatever N is.  us per call
-// with / without the final kernel: 30 heads D64 N17776 1031 / 1026, 48 heads N16384 908 / 891, 32 heads N10000 425 / 408, 10 heads N24000
-// 661 / 658; D128 12 heads N12000 385 / 380, 24 heads N9000 386.8 / 385.4, 32 heads N32768 causal 3913 / 3905; but 8 heads D64 N12000 193 /
-// 202, 6 heads D128 N16384 288 / 290.
+// Many heads: sixteen chunks each already spread the read over the chip.  What takes its time then is a chunk of N / 16 rows, which
+// needs something beside it, and the reading of sixteen chunks by every workgroup of the back kernel, which grows with all rows of
+// K.  So at D = 128 the front grid has to be large enough for 256 threads per workgroup (more than 512 workgroups; below, the chunks
+// are all there is) and the rows of all heads few; at D = 64 the blocks of Q have to be many, and a head short.  A mask takes the
+// work of pooling off the blocks of Q, and with it what the chunks hide behind.  us per call with / without the final kernel, heads,
+// queries, keys: D128 12 x 1024 x 8200 53.5 / 57.2, 12 x 2560 x 8200 57.9 / 55.4, 12 x 1024 x 20000 94.3 / 104.7, 13 x 1024 x 20000 100.8 / 95.1, 16 x
+// 128 x 8200 62.1 / 57.9, 16 x 16384 138.0 / 139.8, 18 x 2560 x 16384 102.5 / 105.3, 20 x 32768 412 / 424, 24 x 10000 225.8 / 225.8, 24 x
+// 32768 483 / 493, 48 x 512 x 17776 208.6 / 214.6, 32 x 32768 causal 3900 / 3901; D64 16 x 2048 x 10000 (256 blocks) 1.7 slower, 16 x 10000
+// 157.7 / 156.9, 32 x 2048 x 8200 63.2 / 62.1, 48 x 2048 x 8200 81.8 / 77.5, 48 x 12288 146.3 / 145.8, 16 x 16384 87.0 / 90.5, 24 x 32768 310.6 /
+// 321.9, 40 x 24000 563 / 572, 12 x 10000 0.9 slower; masks D128 12 x 17776 122 / 138, 16 x 12288 105.6 / 114.4, 24 x 9000 113.0 / 114.3.
 struct Chunks {
   int n, rows;
   bool partial;
 };
-inline Chunks chunks_for(int heads, int N, int D) {
+inline Chunks chunks_for(const spg_attn_args *a) {
   Chunks c;
-  const bool few = (long long)heads * N <= 24576 && (long long)N * D < 3 << 19;
-  const bool many = heads >= 12 && N <= 32768;
+  const int N = a->N_kv, heads = a->B * a->Hkv;
+  const long long all = (long long)heads * N, q_blocks = (long long)a->B * a->H * ((a->N + 127) / 128);
+  const bool few = all <= 24576 && (long long)N * a->D < 3 << 19;
+  const bool many = a->selection != SPG_SELECT_MASK &&
+                    (a->D == 128 ? heads >= 12 && q_blocks + 32ll * heads > 512 && all <= 262144
+                                 : heads >= 16 && q_blocks >= 512 && N <= 12288 && all <= 524288);
   c.partial = N <= 8192 || few || many;
   const int want = N <= 8192 || many ? 16 : few ? 32 : (2048 + heads - 1) / heads;
   const int most = N <= 8192 ? (N + 63) / 64 : (N + 255) / 256;
@@ -65,7 +74,7 @@ inline Layout layout_for(const spg_attn_args *a) {
   auto take = [&](size_t bytes) { const size_t r = at; at += (bytes + 255) / 256 * 256; return r; };
   const size_t bh = (size_t)a->B * a->H, bhk = (size_t)a->B * a->Hkv, D = a->D;
   const size_t nq = ((size_t)a->N + 127) / 128, nk = ((size_t)a->N_kv + 63) / 64;
-  const Chunks c = chunks_for((int)bhk, a->N_kv, a->D);
+  const Chunks c = chunks_for(a);
   const bool pool = a->selection != SPG_SELECT_MASK;
   l.km_part = take(bhk * c.n * D * 8);
   l.v_part = take(a->pv_f16 ? 0 : bhk * c.n * D * 4);

@@ -216,3 +216,14 @@ def test_many_queries_over_short_heads(N, D):
                lambda: sa.spas_sage_attn_meansim_cuda(q, k, v, cdfthreshd=0.8, simthreshd1=0.1, return_sparsity=True)):
         (o, s), (o2, s2) = _both(fn)
         assert torch.equal(_bits(o), _bits(o2)) and s == s2
+
+
+@pytest.mark.parametrize("H,N,Nk,D", [(12, 1280, 8300, 128), (12, 1281, 8300, 128), (12, 1281, 21845, 128), (12, 1281, 21846, 128), (16, 3968, 8300, 64),
+                                      (16, 3969, 8300, 64), (16, 3969, 12288, 64), (16, 3969, 12289, 64)])
+def test_many_heads_with_queries_beside_them(H, N, Nk, D):
+    """Both sides of the lines from which on sixteen chunks a head are combined by every workgroup of the back kernel."""
+    q = rand_T((1, H, N, D), torch.bfloat16, 91)
+    k, v = rand_T((1, H, Nk, D), torch.bfloat16, 92, shift=0.3), rand_T((1, H, Nk, D), torch.float16, 93)
+    for fn in (sa.spas_sage2_attn_meansim_topk_cuda, sa.spas_sage_attn_meansim_topk_cuda):
+        o, o2 = _both(lambda: fn(q, k, v, topk=0.1))
+        assert torch.equal(_bits(o), _bits(o2))
