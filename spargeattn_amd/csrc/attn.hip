@@ -53,8 +53,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define SPG_QUEUE_MIN_ROW 16384     // ... length of a row, in channels of K blocks, beyond which the queue pays (launch_attn)
 #define SPG_QUEUE_EXTRA 12          // one workgroup in so many is launched on top
 #define SPG_PLACES 96               // rows that an XCD works on at a time: 32 CUs x 3
-#define SPG_GROUPS_MAX_WG 256       // rows up to which ...
-#define SPG_GROUPS_MIN_NK 12        // ... and K blocks from which a row gets groups of wavefronts
 #define SPG_LOG2E 1.44269504088896340736f
 
 // n / d for 0 <= n < 2^31 as a multiplication and a shift: m = ceil(2^(31+s) / d) with 2^(s-1) < d <= 2^s is a 32-bit number, and
@@ -1081,17 +1079,7 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
   p.by_nq = FastDiv::of(p.nq); p.by_rest = FastDiv::of(p.nq > p.rows_first ? p.nq - p.rows_first : 1);
   p.by_H = FastDiv::of(p.H); p.by_group = FastDiv::of(p.H / p.Hkv);
-  // A row alone on its CU: its blocks go over groups of wavefronts (kernel comment).  As many groups as registers and LDS
-  // allow where rows are long, two up to 64 blocks, where the exchange and the final sum weigh more.  us per call with 1 / 2 / 3 / 4
-  // groups, D64: one head N17776 281 / 236 / 169 / 163.5 (the last two of a later build), H2 N16384 131 / 111 / 98.4 / 96.2, H2 N12000
-  // CDF - / - / 123.5 / 120.7; H8 N4096 45 / 39.2 / 39.0 / 39.8, H2 N2048 - / 25.8 / 26.3 / 27.2; H2 N256 18.0 / 18.6 / 19.9.  D128: one head
-  // N17776 - / 227 / 214, H2 N16384 161 / 131 / 127, H2 N12000 causal - / 166 / 157.5; H8 N4096 59 / 53.5 / 54.0, H4 N3584 - / 42.4 /
-  // 43.1, H2 N2304 - / 32.6 / 33.4, H2 N1024 - / 25.2 / 26.6.  FP16 PV D128 H2 N16384 188 / 164 (two fit the LDS).  At D128 a grid of
-  // fewer than eight rows keeps two for every nk, so that a list has the same bits whatever the length of the head around it.
-  // Beyond one row per CU the rows fill each other's gaps: H10 N4096 unchanged without groups.
-  const bool groups = p.total_wg <= SPG_GROUPS_MAX_WG && p.nk >= SPG_GROUPS_MIN_NK && p.pv_mode == 1 && p.pv_count == nullptr;
-  const int most = D == 64 ? 4 : p.v_scale != nullptr && p.total_wg >= 8 ? 3 : 2;
-  const int n_groups = !groups ? 1 : p.nk > 64 ? most : 2;
+  const int n_groups = p.pv_mode == 1 && p.pv_count == nullptr ? attn_groups(p.total_wg, p.nk, D, p.v_scale == nullptr) : 1;
 #define SPG_ATTN(D_, PV16_, G_)                                                                             \
   {                                                                                                         \
     if (out_dtype == 0) block_sparse_attn_kernel<D_, 0, PV16_, SEL, G_><<<grid, 256 * G_, 0, st>>>(p);       \

@@ -7,6 +7,7 @@ rounding to the output type, which may fall on the other side (one unit in the l
 import pytest
 import torch
 
+import spargeattn_amd as sa
 from spargeattn_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +56,16 @@ def test_groups_equal_the_sequential_walk(D, dtype, f16v, Nk, causal):
     ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
     assert ((o - w).abs() <= ulp * w.abs() + 1e-5 * w.abs().max()).all()
     assert (o - w).norm() <= 3e-4 * w.norm() * (1 if dtype == torch.float16 else 8)
+
+
+@pytest.mark.parametrize("nk", [96, 97, 128, 129])
+def test_long_rows_at_both_sides_of_the_line(nk):
+    """D = 128 takes three groups beyond 96 blocks; a row's bits do not depend on how many others the grid holds."""
+    test_groups_equal_the_sequential_walk(128, torch.bfloat16, False, 64 * nk - 3, False)
+    g = torch.Generator().manual_seed(nk)
+    Nk, D = 64 * nk - 3, 128
+    q, k, v = (torch.randn((1, 12, n, D), generator=g).bfloat16().cuda() for n in (130, Nk, Nk))
+    many = sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.7)
+    for h in (0, 11):
+        few = sa.spas_sage2_attn_meansim_topk_cuda(*(t[:, h:h + 1].contiguous() for t in (q, k, v)), topk=0.7)
+        assert torch.equal(few.view(torch.int16), many[:, h:h + 1].view(torch.int16))
