@@ -17,14 +17,17 @@ namespace spg {
 // N12000 157.9 / 157.8, N16384 94.6 / 93.5, N24576 132.0 / 126.3; two heads D128 N12288 80.9 / 80.9, with FP16 PV 88.9 / 88.3.
 // Many heads: sixteen chunks each already spread the read over the chip.  What takes its time then is a chunk of N / 16 rows, which
 // needs something beside it, and the reading of sixteen chunks by every workgroup of the back kernel, which grows with all rows of
-// K.  So at D = 128 the front grid has to be large enough for 256 threads per workgroup (more than 512 workgroups; below, the chunks
-// are all there is) and the rows of all heads few; at D = 64 the blocks of Q have to be many, and a head short.  A mask takes the
-// work of pooling off the blocks of Q, and with it what the chunks hide behind.  us per call with / without the final kernel, heads,
-// queries, keys: D128 12 x 1024 x 8200 53.5 / 57.2, 12 x 2560 x 8200 57.9 / 55.4, 12 x 1024 x 20000 94.3 / 104.7, 13 x 1024 x 20000 100.8 / 95.1, 16 x
-// 128 x 8200 62.1 / 57.9, 16 x 16384 138.0 / 139.8, 18 x 2560 x 16384 102.5 / 105.3, 20 x 32768 412 / 424, 24 x 10000 225.8 / 225.8, 24 x
-// 32768 483 / 493, 48 x 512 x 17776 208.6 / 214.6, 32 x 32768 causal 3900 / 3901; D64 16 x 2048 x 10000 (256 blocks) 1.7 slower, 16 x 10000
-// 157.7 / 156.9, 32 x 2048 x 8200 63.2 / 62.1, 48 x 2048 x 8200 81.8 / 77.5, 48 x 12288 146.3 / 145.8, 16 x 16384 87.0 / 90.5, 24 x 32768 310.6 /
-// 321.9, 40 x 24000 563 / 572, 12 x 10000 0.9 slower; masks D128 12 x 17776 122 / 138, 16 x 12288 105.6 / 114.4, 24 x 9000 113.0 / 114.3.
+// K.  At D = 128 that something is a front grid large enough for 256 threads per workgroup (more than 512 workgroups; below, the chunks
+// are all there is) and the gain ends early; a mask takes the work of pooling off the blocks of Q, and with it what the chunks hide
+// behind.  At D = 64, half the bytes in a row, it is 512 blocks of Q (1280 for fewer than sixteen heads), or none over short heads.
+// us per call with sixteen chunks / with the final kernel, top-k 0.4, heads x queries x keys (steady runs over three sets of inputs;
+// calls of the two forms in turn mislead here, their workspaces differ):
+// D128 16 x 1024 x 8200 92 / 97, 12 x 4096 x 12288 151 / 156, 16 x 256 x 16384 145 / 148, 24 x 4096 x 8200 175 / 176, 12 x 8192 186 / 189, 32 x 1024 x
+// 8200 124 / 126; 12 x 1024 x 8200 89 / 85, 12 x 256 x 32768 265 / 243, 10 x 1024 x 16384 140 / 132, 48 x 1024 x 16384 314 / 309, 24 x 16384 883 / 878;
+// masks 16 x 1024 x 8200 94 / 90, 12 x 16384 468 / 455, 24 x 4096 x 16384 306 / 295, 48 x 16384 1770 / 1756.
+// D64 48 x 256 x 8200 94 / 96, 24 x 4096 x 8200 118 / 122, 24 x 12288 359 / 372, 16 x 16384 405 / 422, 24 x 4096 x 20480 252 / 258, 16 x 8192 x 32768
+// 429 / 440, 12 x 20480 475 / 490; 16 x 1024 x 12288 90 / 87, 12 x 4096 x 16384 149 / 143, 10 x 256 x 32768 187 / 164, 24 x 1024 x 32768 226 / 220, 32 x
+// 4096 x 32768 486 / 480, 48 x 20480 equal; masks 16 x 16384 412 / 441, 12 x 20480 471 / 500, 32 x 4096 x 8200 150 / 158, 16 x 1024 x 32768 187 / 182.
 struct Chunks {
   int n, rows;
   bool partial;
@@ -34,9 +37,8 @@ inline Chunks chunks_for(const spg_attn_args *a) {
   const int N = a->N_kv, heads = a->B * a->Hkv;
   const long long all = (long long)heads * N, q_blocks = (long long)a->B * a->H * ((a->N + 127) / 128);
   const bool few = all <= 24576 && (long long)N * a->D < 3 << 19;
-  const bool many = a->selection != SPG_SELECT_MASK &&
-                    (a->D == 128 ? heads >= 12 && q_blocks + 32ll * heads > 512 && all <= 262144
-                                 : heads >= 16 && q_blocks >= 512 && N <= 12288 && all <= 524288);
+  const bool many = a->D == 128 ? a->selection != SPG_SELECT_MASK && heads >= 12 && q_blocks + 32ll * heads > 512 && all <= 294912
+                                : (heads >= 16 && N <= 9216) || (heads >= 12 && q_blocks >= (heads >= 16 ? 512 : 1280) && N <= 32768 && all <= 786432);
   c.partial = N <= 8192 || few || many;
   const int want = N <= 8192 || many ? 16 : few ? 32 : (2048 + heads - 1) / heads;
   const int most = N <= 8192 ? (N + 63) / 64 : (N + 255) / 256;

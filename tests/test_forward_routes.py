@@ -43,11 +43,12 @@ def test_short_heads_take_one_launch_up_to_1024_q_blocks(routes, kw):
 # of Q beside them, and the rows of all heads, which read them, have to be few.  Both sides of each line.
 @pytest.mark.parametrize("H,N,Nk,D,kw,combined", [
     (12, 130, 32768, 128, {}, 0), (12, 1280, 20000, 128, {}, 0), (12, 1281, 20000, 128, {}, 1), (11, 20000, 20000, 128, {}, 0),
-    (16, 16384, 16384, 128, {}, 1), (16, 16385, 16385, 128, {}, 0), (32, 32768, 32768, 128, {}, 0), (16, 12288, 12288, 128, dict(selection=MASK), 0),
+    (18, 16384, 16384, 128, {}, 1), (18, 16385, 16385, 128, {}, 0), (32, 32768, 32768, 128, {}, 0), (16, 12288, 12288, 128, dict(selection=MASK), 0),
     (16, 128, 8200, 128, {}, 1), (24, 10000, 10000, 128, dict(pv_f16=1), 1), (2, 130, 12287, 128, {}, 1), (40, 130, 8192, 128, {}, 1),
-    (16, 3968, 8200, 64, {}, 0), (16, 3969, 8200, 64, {}, 1), (15, 12288, 12288, 64, {}, 0), (16, 12288, 12288, 64, {}, 1),
-    (16, 12289, 12289, 64, {}, 0), (30, 17776, 17776, 64, {}, 0), (12, 32768, 32768, 64, {}, 0), (43, 12288, 12288, 64, {}, 0),
-    (64, 12288, 12288, 64, dict(Hkv=16), 1)])
+    (16, 128, 9216, 64, {}, 1), (15, 128, 9216, 64, {}, 0), (16, 128, 9217, 64, {}, 0), (16, 3968, 9217, 64, {}, 0), (16, 3969, 9217, 64, {}, 1),
+    (12, 12288, 12288, 64, {}, 0), (12, 16384, 16384, 64, {}, 1), (24, 4096, 32768, 64, dict(selection=MASK), 1), (24, 4096, 32769, 64, {}, 0),
+    (25, 4096, 32768, 64, {}, 0), (12, 130, 32768, 64, {}, 0), (30, 17776, 17776, 64, {}, 1), (64, 12288, 12288, 64, dict(Hkv=16), 1),
+    (64, 12288, 12288, 64, dict(Hkv=8), 0)])
 def test_sixteen_chunks_need_queries_beside_them(routes, H, N, Nk, D, kw, combined):
     assert routes(H=H, N=N, Nk=Nk, D=D, **kw)[2] == combined
 

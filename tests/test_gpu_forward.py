@@ -218,8 +218,8 @@ def test_many_queries_over_short_heads(N, D):
         assert torch.equal(_bits(o), _bits(o2)) and s == s2
 
 
-@pytest.mark.parametrize("H,N,Nk,D", [(12, 1280, 8300, 128), (12, 1281, 8300, 128), (12, 1281, 21845, 128), (12, 1281, 21846, 128), (16, 3968, 8300, 64),
-                                      (16, 3969, 8300, 64), (16, 3969, 12288, 64), (16, 3969, 12289, 64)])
+@pytest.mark.parametrize("H,N,Nk,D", [(12, 1280, 8300, 128), (12, 1281, 8300, 128), (12, 1281, 24576, 128), (12, 1281, 24577, 128), (16, 130, 9216, 64),
+                                      (16, 130, 9217, 64), (16, 3968, 9300, 64), (16, 3969, 9300, 64), (24, 2700, 32768, 64), (24, 2700, 32769, 64)])
 def test_many_heads_with_queries_beside_them(H, N, Nk, D):
     """Both sides of the lines from which on sixteen chunks a head are combined by every workgroup of the back kernel."""
     q = rand_T((1, H, N, D), torch.bfloat16, 91)
