@@ -52,7 +52,8 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define SPG_QUEUE_MIN 384           // workgroups per XCD (four rounds of 32 CUs x 3) and ...
 #define SPG_QUEUE_MIN_ROW 16384     // ... length of a row, in channels of K blocks, beyond which the queue pays (launch_attn)
 #define SPG_QUEUE_EXTRA 12          // one workgroup in so many is launched on top
-#define SPG_PLACES 96               // rows that an XCD works on at a time: 32 CUs x 3
+#define SPG_PLACES 96               // last rows of an XCD that lower their priority: 32 CUs x 3, the rows it works on at a time at D = 128.  D = 64
+                                    // fits four workgroups per CU (124 registers, 25 KB): 112 and 128 make no difference there, one number for both
 #define SPG_LOG2E 1.44269504088896340736f
 
 // n / d for 0 <= n < 2^31 as a multiplication and a shift: m = ceil(2^(31+s) / d) with 2^(s-1) < d <= 2^s is a 32-bit number, and
@@ -948,6 +949,11 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     // without / with, H x N top-k 0.5: D128 6 x 8192 124 / 118, 13 x 8192 214 / 201, 20 x 8192 272 / 263, 26 x 8192 354 / 342, causal 28 x
     // 4096 118 / 116, D64 14 x 8192 156 / 144, 30 x 17776 1035 / 1016, FP16 PV 6 x 16384 379 / 367.  (The last 64 or 80 rows
     // instead of the places of an XCD: 13 x 8192 205 / 200, 20 x 8192 266 / 267; steps at thirds of the row: 205, 265.)
+    // The priority counts against every wavefront of the SIMD, those of other streams' kernels among them, as long as a row runs.  Raised for
+    // the last 192 rows of an XCD only, which alone meet the ones that lower theirs, calls are slower (30 x 17776 D64 top-k 1026 / 1048, CDF
+    // 1851 / 1915), and what else runs gains nothing by it: three wavefronts of 168 registers leave no room on a SIMD, and beside D64 48 x 16384
+    // small kernels of another stream take as long either way (an addition over a million floats 54.6, 51.5 with priority and 50.5, 51.4
+    // without, 4.5 us alone).
     int drop_at = 0x7fffffff;
     if constexpr (G == 1) {
       __builtin_amdgcn_s_setprio(3);

@@ -171,7 +171,10 @@ __device__ __forceinline__ void select_row(uint64_t (&map)[W], const float (&sc)
 #pragma unroll
     for (int t = 0; t < W; t++) key[t] = okey[t];
     bitonic_sort_desc<W, 2>(key, lane);                 // sorted position of key[t] is lane * W + t
-    // cdf[v] = T(sum_{u<=v} p_sorted[u]);  n = #{v < nk : cdf[v] <= threshold}  (utils.py:398-403); the sums are exact
+    // cdf[v] = T(sum_{u<=v} p_sorted[u]);  n = #{v < nk : cdf[v] <= threshold}  (utils.py:398-403).  fp16 probabilities are multiples of
+    // 2^-24, so their sums are exact in any order.  bf16 ones reach further down than binary64 holds beside 1: probabilities below about
+    // 2^-45 of the sum can be rounded, here and in the selection kernel in another order (with two columns per lane `run - own`, too).
+    // That shows only if it carries the sum across a rounding tie of T that sits at the threshold.
     double own = 0.0;
 #pragma unroll
     for (int t = 0; t < W; t++) own += (double)elem_to_f32<DT>((uint16_t)(key[t] >> 16));
