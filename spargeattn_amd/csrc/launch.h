@@ -74,15 +74,16 @@ struct RowSelect {
 // N12000 CDF - / - / 123.5 / 120.7; H8 N4096 45 / 39.2 / 39.0 / 39.8, H2 N2048 - / 25.8 / 26.3 / 27.2; H2 N256 18.0 / 18.6 / 19.9.  D128: one head
 // N17776 - / 227 / 214, H2 N16384 161 / 131 / 127, H2 N12000 causal - / 166 / 157.5; H8 N4096 59 / 53.5 / 54.0, H4 N3584 - / 42.4 / 43.1, H2
 // N2304 - / 32.6 / 33.4, H2 N1024 - / 25.2 / 26.6.  FP16 PV D128 H2 N16384 188 / 164 (two fit the LDS).
-// D128 with two / three groups around the line, top-k 0.3 and 0.6: H2 N5120 41.0 / 42.4 and 57.4 / 57.6, N6144 46.7 / 48.2 and 66.7 / 65.8,
-// N7168 51.9 / 52.3 and 74.9 / 74.2; 8 rows of Nk 6144 51.9 / 53.0 and 72.8 / 71.8, 128 rows 122.0 / 123.1 and 142.1 / 140.7.  The number of rows
+// D128 with two / three groups around the line: rows that keep all blocks (the partial last row of a head does) H2 N4500 69.0 / 67.5,
+// H2 N6100 90.6 / 88.4, one head 130 x 4200 60.6 / 59.3, 500 x 6100 87.8 / 85.6; whole rows with top-k 0.3 and 0.6 lose a little or gain: H2
+// N5120 41.0 / 42.4 and 57.4 / 57.6, N6144 46.7 / 48.2 and 66.7 / 65.8, 8 rows of Nk 6144 51.9 / 53.0 and 72.8 / 71.8.  The number of rows
 // makes no difference: one row of Nk 17776 134.1 / 128.4, 32768 216 / 205, 300000 1781 / 1659; 4 rows of 8200 73.8 / 71.5, 7 rows of 12000 98.5 / 95.0.
 // Beyond one row per CU the rows fill each other's gaps: H10 N4096 unchanged without groups.  Lists of the caller's own in a head
 // longer than the operators take (32768 blocks) say nothing of their length by nk: two, as over a short head.
 inline int attn_groups(int rows, int nk, int D, bool pv_f16) {
   if (rows > 256 || nk < 12) return 1;
-  if (D == 64) return nk > 64 ? 4 : 2;
-  return !pv_f16 && nk > 96 && nk <= 32768 ? 3 : 2;
+  if (nk <= 64) return 2;
+  return D == 64 ? 4 : !pv_f16 && nk <= 32768 ? 3 : 2;
 }
 // sel == NULL: blocks come from lut / valid; otherwise they are selected in place and lut / valid are not read.
 // queue: 8 device ints, zero when the kernel starts, for handing out rows across the XCDs, or NULL for a fixed share each.

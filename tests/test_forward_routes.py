@@ -63,8 +63,7 @@ def test_chunks_hold_every_row_of_a_head(routes):
 @pytest.mark.parametrize("H,N", [(1, 1), (1, 128), (3, 200), (7, 128), (8, 128), (2, 16384)])
 @pytest.mark.parametrize("D,pv_f16,long", [(64, 0, 4), (64, 1, 4), (128, 0, 3), (128, 1, 2)])
 def test_groups_follow_the_row_not_the_number_of_rows(routes, H, N, D, pv_f16, long):
-    line = 96 if D == 128 else 64
-    groups = [routes(H=H, N=N, Nk=64 * nk, D=D, pv_f16=pv_f16)[3] for nk in (11, 12, line, line + 1, 8192)]
+    groups = [routes(H=H, N=N, Nk=64 * nk, D=D, pv_f16=pv_f16)[3] for nk in (11, 12, 64, 65, 8192)]
     assert groups == [1, 2, 2, long, long]
 
 

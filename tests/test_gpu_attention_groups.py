@@ -58,9 +58,9 @@ def test_groups_equal_the_sequential_walk(D, dtype, f16v, Nk, causal):
     assert (o - w).norm() <= 3e-4 * w.norm() * (1 if dtype == torch.float16 else 8)
 
 
-@pytest.mark.parametrize("nk", [96, 97, 128, 129])
+@pytest.mark.parametrize("nk", [64, 65, 128, 129])
 def test_long_rows_at_both_sides_of_the_line(nk):
-    """D = 128 takes three groups beyond 96 blocks; a row's bits do not depend on how many others the grid holds."""
+    """D = 128 takes three groups beyond 64 blocks; a row's bits do not depend on how many others the grid holds."""
     test_groups_equal_the_sequential_walk(128, torch.bfloat16, False, 64 * nk - 3, False)
     g = torch.Generator().manual_seed(nk)
     Nk, D = 64 * nk - 3, 128
