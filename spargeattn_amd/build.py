@@ -37,7 +37,7 @@ RESOURCE_REMARKS = "-Rpass-analysis=kernel-resource-usage"
 # The same kernels issue some LDS reads through inline asm and wait for them in a LATER asm statement (the reads run
 # under matrix instructions).  In between, the compiler believes the destination registers are already written; the
 # generated code of this compiler version was inspected for copies or live-range splits inside those windows and has
-# none: in all 60 attention kernels (FP8 PV, where a window is half of the operands; FP16 PV, where it is a step of two or four
+# none: in all 72 attention kernels (FP8 PV, where a window is half of the operands; FP16 PV, where it is a step of two or four
 # reads behind a partial wait) and both dense ones, no instruction names a register of such a read before the wait that
 # covers it, and no label or branch lies in between.  Another compiler may schedule differently: the build then says so,
 # loudly, and asks for the check to be redone (SPARGEATTN_AMD_ALLOW_UNVALIDATED_COMPILER=1 silences the failure, not the warning).

@@ -29,11 +29,13 @@
 //    no int-to-float conversion; the constant is folded into the additive term of the fma that feeds exp2;
 //  * only "skip" votes of the PV threshold reach LDS, and the rescale factor of O is computed only in iterations in which
 //    a running maximum rose;
-//  * workgroup ids are remapped so that one XCD (one L2) works on one head at a time, heaviest rows first.
+//  * workgroup ids are remapped so that one XCD (one L2) works on one head at a time, heaviest rows first;
+//  * on large grids at D = 128 a workgroup quantises its own Q block before it starts (FQ; q_in_front has the line and the figures).
 #include "common.h"
 #include "launch.h"
 #include "lds_asm.h"
 #include "select_row.h"
+#include "stage_bodies.h"
 
 #include <type_traits>
 
@@ -43,6 +45,27 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v8i_a16 __attribute__((ext_vector_type(8), aligned(16)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+
+// Results of psq_core for one Q block in LDS.  A code row of D bytes has its 16-byte chunks at chunk ^ swz(row): the Q operand is read by 32
+// lanes of as many rows, which spreads them over the sixteen slots of a 256-byte line.
+template <int D>
+struct PsqToLds {
+  static constexpr bool ALL_ROWS = true;
+  uint16_t *pool_at;
+  uint32_t *sim_at;
+  float *scale_at;
+  unsigned char *lo, *hi;             // rows 0-63 and 64-127
+  bool one;
+  static_assert(D == 128, "two rows to a line");
+  static __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
+  __device__ __forceinline__ bool one_scale() const { return one; }
+  __device__ __forceinline__ void pool(int, int col, uint16_t v) const { pool_at[col] = v; }
+  __device__ __forceinline__ void sim(int, bool v) const { *sim_at = v ? 1 : 0; }
+  __device__ __forceinline__ void codes(int row, int c, uint2 v) const {
+    *(uint2 *)((row < 64 ? lo : hi) + (row & 63) * D + ((c >> 1) ^ swz(row)) * 16 + (c & 1) * 8) = v;
+  }
+  __device__ __forceinline__ void scale(int g, float v) const { scale_at[g] = v; }
+};
 
 #define SPG_NEG_BIG (-5000000.0f)   // csrc/qattn/attn_utils.cuh:350, qk_int_sv_f8_cuda_sm89.cuh:171
 #define SPG_FP8_OFFSET 8.807f       // csrc/qattn/attn_utils.cuh:28
@@ -89,6 +112,7 @@ struct AttnParams {
   FastDiv by_nq, by_rest, by_H, by_group;   // nq, nq - rows_first, H, H / Hkv
   int rows_first;  // so many of the longest rows of every head come before the rest (place_workgroup)
   RowSelect sel;   // selection inside the kernel (template argument SEL); lut is unused then
+  RawQ q;          // Q as the caller has it (template argument FQ); q8, q_scale, sel.pool_q and sel.sim_q are unused then
 };
 
 // Workgroup -> (batch*head, q block).  Ids are dealt round-robin over the 8 XCDs; each XCD (one L2) gets a contiguous
@@ -230,7 +254,10 @@ __device__ __forceinline__ int v_swz(int row) { return (row >> 2) & 3; }
 // running maximum of the blocks BEFORE it in the list, so the groups exchange their block maxima through LDS once per round
 // of G blocks (at the barrier that the rings need anyway), and so the PV-skip test sees the same differences.  O and the
 // denominator are per group and meet in the epilogue.
-template <int D, int ODT, bool PV16, int SEL, int G>
+// FQ: 0 Q comes as INT8 codes and scales; 1 the workgroup quantises its Q block itself; 2 it pools it, too, and works out its similarity
+// flag, for a selection in place (SEL).  Codes, pooled row and flag stay in LDS: what a kernel in front would write (half of Q's bytes
+// and more) and this one read again.
+template <int D, int ODT, bool PV16, int SEL, int G, int FQ>
 __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_kernel(const AttnParams p) {
   constexpr int KS = D / 32;        // k-steps of the int8 MFMA
   constexpr int NDT = D / 32;       // 32-channel output tiles
@@ -281,8 +308,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   const int bhk = batch * p.Hkv + p.by_group(head);
 
   const int N = p.N, Nk = p.Nk;
-  const int q_row = qb * 128 + wave * 32 + r;
-  if constexpr (!PV16) fp8_saturation_on();
+  if constexpr (!PV16 && FQ == 0) fp8_saturation_on();
 
   // Everything whose address follows from the launch arguments is requested before the first wait: the count, the first
   // four LUT entries (indices clamped to the row, unused ones ignored), the scales, Q.  A chain of dependent scalar loads
@@ -301,22 +327,51 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     l0 = lutc[0]; l1 = lutc[min(1, last_col)]; l2 = lutc[min(2, last_col)]; l3 = lutc[min(3, last_col)];
   }
   // per-warp granularity: the 32 query rows of a wavefront are one quantisation group, so the scale stays a scalar
-  const float qs = ((c_f32_t)p.q_scale)[p.q_per_warp ? row_id * 4 + wave : row_id];
+  float qs;
+  if constexpr (FQ == 0) qs = ((c_f32_t)p.q_scale)[p.q_per_warp ? row_id * 4 + wave : row_id];
   const float thr = p.pvthr.p != nullptr ? ((c_f32_t)p.pvthr.p)[head] : p.pvthr.v;
 
   // ---- Q fragment: B operand of S^T = K.Q^T, resident for the whole loop -------------------------------
   v4i qreg[KS];
+  if constexpr (FQ == 0) {
+    const int q_row = qb * 128 + wave * 32 + r;
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) {
-    qreg[ks] = (v4i){0, 0, 0, 0};
-    if (q_row < N) qreg[ks] = *(const v4i *)(p.q8 + ((size_t)bh * N + q_row) * D + 32 * ks + 16 * hh);
+    for (int ks = 0; ks < KS; ks++) {
+      qreg[ks] = (v4i){0, 0, 0, 0};
+      if (q_row < N) qreg[ks] = *(const v4i *)(p.q8 + ((size_t)bh * N + q_row) * D + 32 * ks + 16 * hh);
+    }
   }
+  // Q from the caller's tensor: codes through the ring slot that the first tiles leave free, 64 rows in its K and 64 in its V^T tile (FP16
+  // PV: all in a V^T tile)
+  static_assert(FQ == 0 || (G == 1 && D == 128), "where it pays (q_in_front)");
+  __shared__ float sQscale[FQ > 0 ? 4 : 1];
+  __shared__ __align__(16) uint16_t sPoolQ[FQ == 2 ? D : 8];
+  __shared__ uint32_t sSimQ;
+  auto quantise_q = [&]() __attribute__((always_inline)) {
+    if constexpr (FQ > 0) {
+      unsigned char *const lo = NBUF == 3 ? sKr + 2 * TILE : sVr + VTILE, *const hi = NBUF == 3 ? sVr + 2 * VTILE : sVr + VTILE + TILE;
+      const PsqToLds<D> to = {sPoolQ, &sSimQ, sQscale, lo, hi, p.q_per_warp == 0};
+      float simthr = 0.f;
+      if constexpr (FQ == 2) simthr = p.q.simthr.at(head);
+      psq_core<128, D, ODT, MEAN_NONE, FQ == 2, 32, 256, 128>(p.q.x + (size_t)batch * p.q.st.sb + (size_t)head * p.q.st.sh, p.q.st.sn, nullptr, nullptr, 0,
+                                                              simthr, N, qb, bh, sKr, tid, to);
+      __syncthreads();
+      const unsigned char *const half = (wave < 2 ? lo : hi) + ((wave & 1) * 32 + r) * D;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) qreg[ks] = *(const v4i *)(half + (((2 * ks + hh) ^ PsqToLds<D>::swz(r)) * 16));
+      qs = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, sQscale[wave])));
+    }
+  };
+  if constexpr (FQ == 2) quantise_q();
   constexpr int W = SEL > 0 ? SEL : 1;
   uint64_t map[W] = {};                    // SEL: blocks not fetched yet
   if constexpr (SEL > 0) {
     __shared__ uint16_t sScore[64 * W];
     const uint8_t *simk = p.sel.sim_k + (size_t)bhk * p.nk;
-    const bool row_forced = p.sel.sim_q[row_id] == 0;
+    bool row_forced;
+    const uint16_t *pool_q;
+    if constexpr (FQ == 2) { row_forced = sSimQ == 0; pool_q = sPoolQ; }
+    else { row_forced = p.sel.sim_q[row_id] == 0; pool_q = p.sel.pool_q + row_id * D; }
     bool k_dead[W];
 #pragma unroll
     for (int t = 0; t < W; t++) k_dead[t] = simk[min(64 * t + lane, last_col)] == 0;
@@ -325,7 +380,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     for (int t = 0; t < W; t++) {
       if (G == 1 || t % G == grp) {
         const int col = 64 * t + ((tid & 255) >> 2);
-        const uint16_t s16 = pooled_score_4lanes<D, ODT>(p.sel.pool_q + row_id * D, p.sel.pool_k + ((size_t)bhk * p.nk + min(col, last_col)) * D, tid & 3);
+        const uint16_t s16 = pooled_score_4lanes<D, ODT>(pool_q, p.sel.pool_k + ((size_t)bhk * p.nk + min(col, last_col)) * D, tid & 3);
         if ((tid & 3) == 0) sScore[col] = s16;
       }
     }
@@ -546,6 +601,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     if (wave < D / 64 && grp == 0)
       __builtin_amdgcn_global_load_lds((glb_ptr_t)(p.v_scale + (size_t)bhk * D + wave * 64 + lane), (lds_ptr_t)(sVscale + wave * 64), 4, 0, 0);
   }
+  if constexpr (FQ == 1) quantise_q();
+  if constexpr (!PV16 && FQ > 0) fp8_saturation_on();   // (behind the conversions of Q, whose overflows stay infinite)
   uint32_t bufoff = 0;                     // LDS ring offset of block it
 
   // The INT8 accumulators do not start at zero but at the bit pattern 0x3E22F983 - the float 1/(2 pi), which the
@@ -1082,7 +1139,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   }
 }
 
-template <int SEL>
+template <int SEL, int FQ>
 static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_rows, hipStream_t st) {
   p.nq = (p.N + 127) / 128; p.nk = (p.Nk + 63) / 64;
   p.total_wg = p.nq * p.H * p.B;
@@ -1102,16 +1159,19 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
   p.by_nq = FastDiv::of(p.nq); p.by_rest = FastDiv::of(p.nq > p.rows_first ? p.nq - p.rows_first : 1);
   p.by_H = FastDiv::of(p.H); p.by_group = FastDiv::of(p.H / p.Hkv);
-  const int n_groups = p.pv_mode == 1 && p.pv_count == nullptr ? attn_groups(p.total_wg, p.nk, D, p.v_scale == nullptr) : 1;
+  const int n_groups = FQ == 0 && p.pv_mode == 1 && p.pv_count == nullptr ? attn_groups(p.total_wg, p.nk, D, p.v_scale == nullptr) : 1;
 #define SPG_ATTN(D_, PV16_, G_)                                                                             \
   {                                                                                                         \
-    if (out_dtype == 0) block_sparse_attn_kernel<D_, 0, PV16_, SEL, G_><<<grid, 256 * G_, 0, st>>>(p);       \
-    else block_sparse_attn_kernel<D_, 1, PV16_, SEL, G_><<<grid, 256 * G_, 0, st>>>(p);                      \
+    if (out_dtype == 0) block_sparse_attn_kernel<D_, 0, PV16_, SEL, G_, FQ><<<grid, 256 * G_, 0, st>>>(p);  \
+    else block_sparse_attn_kernel<D_, 1, PV16_, SEL, G_, FQ><<<grid, 256 * G_, 0, st>>>(p);                 \
   }
 #define SPG_ATTN_G(D_, PV16_)                                                                               \
   {                                                                                                         \
     constexpr int GMAX = SEL == 1 ? 2 : D_ == 64 ? 4 : PV16_ ? 2 : 3;                                              \
-    if (n_groups == 1) SPG_ATTN(D_, PV16_, 1)                                                                \
+    if constexpr (FQ > 0) {                                                                                 \
+      if constexpr (D_ == 128) SPG_ATTN(D_, PV16_, 1)                                                        \
+      else return hipErrorInvalidValue;                                                                     \
+    } else if (n_groups == 1) SPG_ATTN(D_, PV16_, 1)                                                         \
     else if (n_groups == 2) SPG_ATTN(D_, PV16_, 2)                                                           \
     else if constexpr (GMAX > 2) SPG_ATTN(D_, PV16_, GMAX)                                                   \
   }
@@ -1123,7 +1183,7 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
 }
 
 hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
-                                      int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel,
+                                      int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel, const RawQ *q,
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
                                       int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue, hipStream_t st) {
@@ -1136,10 +1196,12 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
   p.is_causal = is_causal;
   p.pv_mode = pv_mode;
   p.q_per_warp = q_per_warp;
-  if (sel == nullptr) return launch_attn<0>(p, D, out_dtype, causal_rows || is_causal, st);
+  if (q != nullptr) p.q = *q;
+  const bool causal = causal_rows || is_causal;
+  if (sel == nullptr) return q != nullptr ? launch_attn<0, 1>(p, D, out_dtype, causal, st) : launch_attn<0, 0>(p, D, out_dtype, causal, st);
   p.sel = *sel;
-  if (Nk <= 64 * 64) return launch_attn<1>(p, D, out_dtype, causal_rows || is_causal, st);
-  return launch_attn<2>(p, D, out_dtype, causal_rows || is_causal, st);
+  if (Nk <= 64 * 64) return q != nullptr ? launch_attn<1, 2>(p, D, out_dtype, causal, st) : launch_attn<1, 0>(p, D, out_dtype, causal, st);
+  return q != nullptr ? launch_attn<2, 2>(p, D, out_dtype, causal, st) : launch_attn<2, 0>(p, D, out_dtype, causal, st);
 }
 
 hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
@@ -1147,7 +1209,7 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     const float *q_scale, const float *k_scale, const float *v_scale, int B, int H,
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st) {
-  return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, nullptr, Hyper{pvthreshd, 0.f}, q_scale, k_scale,
+  return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, nullptr, nullptr, Hyper{pvthreshd, 0.f}, q_scale, k_scale,
                                     v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, false, nullptr, st);
 }
 

@@ -6,7 +6,7 @@
 //   short    (short heads) everything up to the selection: blocks of K and V, whose workgroups sum and search their whole head for
 //            themselves | mask rows | pooling + quantisation of Q.  Otherwise:
 //   front    partial column sums of K | partial channel maxima of V (FP16 PV: the V^T tiles, finished) | LUT rows of a
-//            user mask | pooling + quantisation of Q
+//            user mask | pooling + quantisation of Q (unless the attention kernel does that in place: q_in_front)
 //   (final   column mean of K, channel maxima of V: only where there are too many partial results for every workgroup
 //            of the next launch to add them up for itself)
 //   back     pooling + quantisation of K | V -> e4m3 tiles and scales
@@ -250,29 +250,40 @@ static void run_short(const spg_attn_args *a, const ShortParams &p, int wgs, hip
 }
 
 template <int D, int DT, int NT>
-static void run_front_back(const spg_attn_args *a, const FrontParams &f, const BackParams &b, const Chunks &c, uint16_t *km, float *v_amax,
-                           int front_wgs, int back_wgs, hipStream_t st) {
-  const bool pool = a->selection != SPG_SELECT_MASK, per_warp = a->qk_quant_gran == SPG_QUANT_PER_WARP;
+static void run_front(bool pool, bool per_warp, const FrontParams &f, int wgs, hipStream_t st) {
   // (a pass of the workgroup stays inside one 32-row quantisation group: the wide form needs D = 128 for it)
   if constexpr (NT == 256 || D == 128) {
     if (per_warp) {
-      if (pool) front_kernel<D, DT, true, 32, NT><<<front_wgs, NT, 0, st>>>(f);
-      else front_kernel<D, DT, false, 32, NT><<<front_wgs, NT, 0, st>>>(f);
+      if (pool) front_kernel<D, DT, true, 32, NT><<<wgs, NT, 0, st>>>(f);
+      else front_kernel<D, DT, false, 32, NT><<<wgs, NT, 0, st>>>(f);
+      return;
     }
   }
-  if (!per_warp) {
-    if (pool) front_kernel<D, DT, true, 128, NT><<<front_wgs, NT, 0, st>>>(f);
-    else front_kernel<D, DT, false, 128, NT><<<front_wgs, NT, 0, st>>>(f);
+  if (pool) front_kernel<D, DT, true, 128, NT><<<wgs, NT, 0, st>>>(f);
+  else front_kernel<D, DT, false, 128, NT><<<wgs, NT, 0, st>>>(f);
+}
+template <int D, int DT, int NT>
+static void run_back(bool pool, bool partial, const BackParams &b, int wgs, hipStream_t st) {
+  if (partial) {
+    if (pool) back_kernel<D, DT, true, true, NT><<<wgs, NT, 0, st>>>(b);
+    else back_kernel<D, DT, false, true, NT><<<wgs, NT, 0, st>>>(b);
+  } else {
+    if (pool) back_kernel<D, DT, true, false, NT><<<wgs, NT, 0, st>>>(b);
+    else back_kernel<D, DT, false, false, NT><<<wgs, NT, 0, st>>>(b);
   }
+}
+template <int D, int DT>
+static void run_front_back(const spg_attn_args *a, const FrontParams &f, const BackParams &b, const Chunks &c, uint16_t *km, float *v_amax,
+                           int front_nt, int front_wgs, int back_nt, int back_wgs, hipStream_t st) {
+  const bool pool = a->selection != SPG_SELECT_MASK, per_warp = a->qk_quant_gran == SPG_QUANT_PER_WARP;
+  if (front_nt == 512) run_front<D, DT, 512>(pool, per_warp, f, front_wgs, st);
+  else run_front<D, DT, 256>(pool, per_warp, f, front_wgs, st);
   if (!c.partial) {
     const FinalParams p = {f.km_part, f.v_part, km, v_amax, f.k_chunks, a->pv_f16 ? 0 : f.v_chunks, a->N_kv};
     final_kernel<D, DT><<<a->B * a->Hkv, dim3(D, 8), 0, st>>>(p);
-    if (pool) back_kernel<D, DT, true, false, NT><<<back_wgs, NT, 0, st>>>(b);
-    else back_kernel<D, DT, false, false, NT><<<back_wgs, NT, 0, st>>>(b);
-  } else {
-    if (pool) back_kernel<D, DT, true, true, NT><<<back_wgs, NT, 0, st>>>(b);
-    else back_kernel<D, DT, false, true, NT><<<back_wgs, NT, 0, st>>>(b);
   }
+  if (back_nt == 512) run_back<D, DT, 512>(pool, c.partial, b, back_wgs, st);
+  else run_back<D, DT, 256>(pool, c.partial, b, back_wgs, st);
 }
 
 hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides &ks, const Strides &vs, const Strides &os,
@@ -288,12 +299,13 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   int32_t *const valid = a->valid_block_num != nullptr ? a->valid_block_num : (int32_t *)(ws + l.valid);
   // Fewer than two workgroups of 256 threads per CU leave the stages bound by the length of one thread's work (9.8 and
   // 13.0 us for the two launches at B2 H3 N1025 D128 with a similarity threshold): twice the threads take half of it.
-  const int wgs256 = heads * nq + kv_heads * 2 * c.n;
-  const bool wide = !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP);
-  const bool one_launch = wide && short_heads(a);
-  const int nt = one_launch || (wgs256 <= 512 && wide) ? 512 : 256;
+  const bool in_one = one_launch(a), sel_in_attn = pool && nk <= SPG_SELECT_IN_ATTN_NK, front_q = q_in_front(a);
+  const int q_wgs = front_q ? heads * nq : 0;
+  const bool can_wide = !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP);
+  const int front_nt = in_one || (q_wgs + kv_heads * 2 * c.n <= 512 && (can_wide || !front_q)) ? 512 : 256;
+  const int back_nt = in_one || (heads * nq + kv_heads * 2 * c.n <= 512 && can_wide) ? 512 : 256;
   int nkp = 256;
-  while (nkp < nk || nkp < nt) nkp <<= 1;
+  while (nkp < nk || nkp < front_nt) nkp <<= 1;
   const bool mask_in_front = !pool && nkp <= MASK_NKP_FRONT;
 
   FrontParams f = {};
@@ -314,7 +326,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   BackParams b = {};
   b.k = f.k; b.v = f.v; b.ks = ks; b.vs = vs;
   b.H = a->H; b.Hkv = a->Hkv; b.Nk = a->N_kv; b.nk = nk; b.v_dtype = a->v_dtype;
-  b.k_wgs_per_head = (a->N_kv + k_rows_per_wg(nt) - 1) / k_rows_per_wg(nt);
+  b.k_wgs_per_head = (a->N_kv + k_rows_per_wg(back_nt) - 1) / k_rows_per_wg(back_nt);
   b.wg_v = kv_heads * b.k_wgs_per_head;
   b.km = (const uint16_t *)(ws + l.km); b.km_part = f.km_part; b.k_chunks = c.n;
   b.v_amax = (const float *)(ws + l.v_amax); b.v_part = f.v_part; b.v_chunks = c.n;
@@ -322,7 +334,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   b.pool_k = (uint16_t *)(ws + l.pool_k); b.sim_k = ws + l.sim_k; b.k8 = (int8_t *)(ws + l.k8); b.k_scale = (float *)(ws + l.k_scale);
   b.v8 = ws + l.v; b.v_scale = (float *)(ws + l.v_scale);
 
-  if (one_launch) {
+  if (in_one) {
     ShortParams s = {f, b, 0, 0, 0};
     s.wg_v = b.wg_v;
     s.wg_mask = s.wg_v + kv_heads * nk;
@@ -330,22 +342,17 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
     const int wgs = s.wg_q + heads * nq;
     if (a->D == 64) { if (a->qk_dtype == 0) run_short<64, 0>(a, s, wgs, st); else run_short<64, 1>(a, s, wgs, st); }
     else            { if (a->qk_dtype == 0) run_short<128, 0>(a, s, wgs, st); else run_short<128, 1>(a, s, wgs, st); }
-  }
-  const int front_wgs = f.wg_q + heads * nq, back_wgs = b.wg_v + (a->pv_f16 ? 0 : kv_heads * nk);
-  uint16_t *km = (uint16_t *)(ws + l.km);
-  float *v_amax = (float *)(ws + l.v_amax);
-#define SPG_RUN(D_, DT_)                                                                                    \
-  {                                                                                                         \
-    if (nt == 512) run_front_back<D_, DT_, 512>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);            \
-    else run_front_back<D_, DT_, 256>(a, f, b, c, km, v_amax, front_wgs, back_wgs, st);                      \
-  }
-  if (one_launch) {}
-  else if (a->D == 64) { if (a->qk_dtype == 0) SPG_RUN(64, 0) else SPG_RUN(64, 1) }
-  else                 { if (a->qk_dtype == 0) SPG_RUN(128, 0) else SPG_RUN(128, 1) }
+  } else {
+    const int front_wgs = f.wg_q + q_wgs, back_wgs = b.wg_v + (a->pv_f16 ? 0 : kv_heads * nk);
+    uint16_t *km = (uint16_t *)(ws + l.km);
+    float *v_amax = (float *)(ws + l.v_amax);
+#define SPG_RUN(D_, DT_) run_front_back<D_, DT_>(a, f, b, c, km, v_amax, front_nt, front_wgs, back_nt, back_wgs, st)
+    if (a->D == 64) { if (a->qk_dtype == 0) SPG_RUN(64, 0); else SPG_RUN(64, 1); }
+    else            { if (a->qk_dtype == 0) SPG_RUN(128, 0); else SPG_RUN(128, 1); }
 #undef SPG_RUN
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const bool sel_in_attn = pool && nk <= SPG_SELECT_IN_ATTN_NK;
   RowSelect sel = {};
   if (sel_in_attn)
     sel = {f.pool_q, b.pool_k, f.sim_q, b.sim_k, Hyper{a->level, a->level_value}, a->selection == SPG_SELECT_TOPK, a->is_causal,
@@ -356,7 +363,8 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   else if (!mask_in_front)
     e = launch_map_to_lut(a->mask, a->mask_kind, lut, valid, a->B, a->H, nq, nk, st);
   if (e != hipSuccess) return e;
-  return launch_block_sparse_attn_h(f.q8, b.k8, b.v8, a->out, os, a->qk_dtype, lut, valid, sel_in_attn ? &sel : nullptr,
+  const RawQ raw = {f.q, qs, simthr};
+  return launch_block_sparse_attn_h(f.q8, b.k8, b.v8, a->out, os, a->qk_dtype, lut, valid, sel_in_attn ? &sel : nullptr, front_q ? nullptr : &raw,
                                     Hyper{a->pvthreshd, a->pvthreshd_value},
                                     f.q_scale, b.k_scale, a->pv_f16 ? nullptr : b.v_scale, a->B, a->H, a->Hkv, a->N, a->N_kv, a->D,
                                     a->sm_scale, a->kernel_causal ? 1 : 0, a->qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0,

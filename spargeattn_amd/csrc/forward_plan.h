@@ -67,6 +67,26 @@ inline bool short_heads(const spg_attn_args *a) {
          kv_heads * nk <= (a->pv_f16 ? 320 : 256) && (long long)a->B * a->H * nq <= 1024;
 }
 
+// (a pass of 512 threads over 64 channels covers two 32-row groups of Q scales)
+inline bool one_launch(const spg_attn_args *a) { return !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP) && short_heads(a); }
+
+// Whether Q is quantised (and pooled) in front of the attention kernel, or in place by its workgroups.  In place Q is read once, its codes never
+// reach memory (half of Q's bytes written and read again), and the front kernel is left with K and V; but a row starts some 3 us later
+// and its vector instructions are taken from the loops beside it.  That pays at D = 128 (twice the work per row of the list at the same
+// cost) once rows beside each other cover the start, from about two per CU, and earlier for a caller's mask, which needs no pooling.  us
+// per call in front / in place, H x N, top-k 0.5 unless noted: 10 x 3840 66.7 / 70.1, 13 x 3900 85.5 / 89.3, 16 x 3900 89.7 / 92.4, 8 x 8192 118.0 /
+// 119.3, 20 x 3840 91.9 / 89.7, 25 x 3840 101.4 / 99.0, 20 x 5120 143.4 / 142.8, 30 x 3840 122.7 / 121.2, GQA 32/8 x 4096 causal 103.0 / 98.4, 48
+// x 8192 x 400 100.2 / 96.5, CDF with similarity 32 x 8000 697 / 689, 20 x 5120 239.3 / 240.5, FP16 PV 20 x 3840 106.5 / 105.5, 32 x 8000
+// 487 / 482; masks 5 x 7680 84.3 / 87.9, 40 x 1024 41.2 / 43.3, 7 x 7300 91.1 / 87.2, 8 x 8000 101.1 / 95.5, 14 x 7300 139.8 / 132.8, 48 x 16384 1342 /
+// 1318, 48 x 16384 x 1000 193.4 / 177.9.  D = 64: 14 x 6400 95.5 / 96.5, 22 x 6400 140.2 / 143.3, 30 x 8192 265.6 / 266.4, CDF 40 x 8000 585 /
+// 605; masks 12 x 7500 83.9 / 84.8, 20 x 10240 124.1 / 125.7, 16 x 16384 325.7 / 325.3, 48 x 16384 657 / 650.  Where a selection kernel
+// wants Q pooled, the front kernel reads Q anyway: H32 N32768 causal 3953 / 3952, H30 N17776 D64 1007 / 1012.
+inline bool q_in_front(const spg_attn_args *a) {
+  const long long rows = (long long)a->B * a->H * ((a->N + 127) / 128);
+  if (a->D == 64 || one_launch(a)) return true;
+  return a->selection == SPG_SELECT_MASK ? rows <= 352 : a->N_kv > 64 * SPG_SELECT_IN_ATTN_NK || rows <= 576;
+}
+
 struct Layout {
   size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, queue, total;
 };
@@ -77,18 +97,18 @@ inline Layout layout_for(const spg_attn_args *a) {
   const size_t bh = (size_t)a->B * a->H, bhk = (size_t)a->B * a->Hkv, D = a->D;
   const size_t nq = ((size_t)a->N + 127) / 128, nk = ((size_t)a->N_kv + 63) / 64;
   const Chunks c = chunks_for(a);
-  const bool pool = a->selection != SPG_SELECT_MASK;
+  const bool pool = a->selection != SPG_SELECT_MASK, front_q = q_in_front(a);
   l.km_part = take(bhk * c.n * D * 8);
   l.v_part = take(a->pv_f16 ? 0 : bhk * c.n * D * 4);
   l.km = take(bhk * D * 2);
   l.v_amax = take(bhk * D * 4);
-  l.pool_q = take(pool ? bh * nq * D * 2 : 0);
+  l.pool_q = take(pool && front_q ? bh * nq * D * 2 : 0);
   l.pool_k = take(pool ? bhk * nk * D * 2 : 0);
-  l.sim_q = take(pool ? bh * nq : 0);
+  l.sim_q = take(pool && front_q ? bh * nq : 0);
   l.sim_k = take(pool ? bhk * nk : 0);
-  l.q8 = take(bh * a->N * D);
+  l.q8 = take(front_q ? bh * a->N * D : 0);
   l.k8 = take(bhk * a->N_kv * D);
-  l.q_scale = take(bh * nq * 4 * (a->qk_quant_gran == SPG_QUANT_PER_WARP ? 4 : 1));
+  l.q_scale = take(front_q ? bh * nq * 4 * (a->qk_quant_gran == SPG_QUANT_PER_WARP ? 4 : 1) : 0);
   l.k_scale = take(bhk * nk * 4);
   l.v = take(bhk * nk * 64 * D * (a->pv_f16 ? 2 : 1));
   l.v_scale = take(bhk * D * 4);

@@ -68,6 +68,13 @@ struct RowSelect {
   int by_topk, is_causal, sink;
   int32_t *valid_out;               // counts for the caller, or NULL
 };
+// Q as the caller has it, for an attention kernel that quantises it (and pools it, with a RowSelect) in place: one scale per block or per 32 rows
+// as q_per_warp says, simthr as psq_core takes it.
+struct RawQ {
+  const uint16_t *x;
+  Strides st;
+  Hyper simthr;
+};
 // Groups of wavefronts per row (attn.hip, template argument G).  A row alone on its CU: its blocks go over groups.  As many groups
 // as registers and LDS allow where rows are long, two for shorter ones, where the exchange and the final sum weigh more.  us per call
 // with 1 / 2 / 3 / 4 groups, D64: one head N17776 281 / 236 / 169 / 163.5 (the last two of a later build), H2 N16384 131 / 111 / 98.4 / 96.2, H2
@@ -86,10 +93,11 @@ inline int attn_groups(int rows, int nk, int D, bool pv_f16) {
   return D == 64 ? 4 : !pv_f16 && nk <= 32768 ? 3 : 2;
 }
 // sel == NULL: blocks come from lut / valid; otherwise they are selected in place and lut / valid are not read.
+// q == NULL: Q comes as q8 / q_scale (and pooled in sel); otherwise from the caller's tensor, and those are not read.
 // queue: 8 device ints, zero when the kernel starts, for handing out rows across the XCDs, or NULL for a fixed share each.
 // causal_rows: the selection is causal, so rows get longer with their index (order of the workgroups only).
 hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, Strides os,
-                                      int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel,
+                                      int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel, const RawQ *q,
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
                                       int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue,

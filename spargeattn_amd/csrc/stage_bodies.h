@@ -170,12 +170,30 @@ enum { MEAN_NONE = 0, MEAN_GIVEN = 1, MEAN_PARTIAL = 2, MEAN_HERE = 3 };
 // NT threads work on ROWS rows: 256 on 128 where there are enough workgroups to fill the chip, more threads on fewer rows
 // where there are not and the time is the length of one thread's work.
 template <int BS, int D, int NT = 256, int ROWS = 128> constexpr int psq_lds() { return ROWS / BS * (NT / 64 * 128 / D) * D * 8; }
-template <int BS, int D, int DT, int MEAN, bool WITH_POOL, int QR = BS, int NT = 256, int ROWS = 128>
-__device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const Strides &xs,
-                                         const uint16_t *__restrict__ km, const double *__restrict__ km_part, int km_chunks,
-                                         uint16_t *__restrict__ pool, uint8_t *__restrict__ sim,
-                                         int8_t *__restrict__ xq, float *__restrict__ scale,
-                                         const float simthr, int H, int N, int nb, int wg, int bh, unsigned char *smem) {
+// Where the results go: device memory as the stages hand it on (PsqStore), or the attention kernel's LDS (attn.hip).
+// ALL_ROWS: rows beyond the end are written, too (as zeros).  one_scale(): the groups of QR rows
+// share the scale of their block after all, so that one instantiation serves both granularities.
+template <int D>
+struct PsqStore {
+  static constexpr bool ALL_ROWS = false;
+  uint16_t *pool_at;                  // of the workgroup's first block, row and group
+  uint8_t *sim_at;
+  int8_t *xq_at;
+  float *scale_at;
+  __device__ __forceinline__ bool one_scale() const { return false; }
+  __device__ __forceinline__ void pool(int sb, int col, uint16_t v) const { pool_at[sb * D + col] = v; }
+  __device__ __forceinline__ void sim(int sb, bool v) const { sim_at[sb] = v ? 1 : 0; }
+  __device__ __forceinline__ void codes(int row, int c, uint2 v) const { *(uint2 *)(xq_at + (size_t)row * D + c * 8) = v; }
+  __device__ __forceinline__ void scale(int g, float v) const { scale_at[g] = v; }
+};
+
+// xh: first row of the (batch, head), sn: elements from row to row, wg: number of the ROWS rows, tid: thread among NT (a workgroup of
+// more threads runs the body once per NT threads, with the same results)
+template <int BS, int D, int DT, int MEAN, bool WITH_POOL, int QR, int NT, int ROWS, class Out>
+__device__ __forceinline__ void psq_core(const uint16_t *__restrict__ xh, long long sn, const uint16_t *__restrict__ km,
+                                         const double *__restrict__ km_part, int km_chunks, const float simthr, int N, int wg, int bh,
+                                         unsigned char *smem, int tid, const Out &out) {
+#pragma clang fp contract(off)
   constexpr int SUB = ROWS / BS;      // blocks per workgroup
   constexpr int TPR = D / 8;          // lanes per row (16 B each)
   constexpr int RPP = NT / TPR;       // rows per pass of the workgroup
@@ -196,13 +214,12 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
   // "every element of the row is tiny": bfloat16 below 2^-63 (both top exponent bits clear), binary16 zero
   constexpr uint32_t TINY2 = DT == 1 ? 0x60006000u : 0x7fff7fffu;
   constexpr bool HAS_MEAN = MEAN != MEAN_NONE;
-  const int tid = threadIdx.x, c = tid % TPR, r = tid / TPR;
+  const int c = tid % TPR, r = tid / TPR;
   const int row_base = wg * ROWS;
   const int rows_here = min(ROWS, N - row_base);          // >= 1
   const bool partial = rows_here < ROWS;                  // workgroup-uniform: only the last workgroup of a head
-  const int blk0 = wg * SUB;
   auto rows_valid_of = [&](int sb) { return max(0, min(BS, rows_here - sb * BS)); };
-  const uint16_t *xb = x + (size_t)(bh / H) * xs.sb + (size_t)(bh % H) * xs.sh + (size_t)row_base * xs.sn + c * 8;
+  const uint16_t *xb = xh + (size_t)row_base * sn + c * 8;
 
   // all loads of the thread are issued before the first use (rows beyond the end re-read the last row and are zeroed
   // afterwards: no load sits behind a branch)
@@ -210,7 +227,7 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
   {
     uint4 raw[NPT];
 #pragma unroll
-    for (int p = 0; p < NPT; p++) raw[p] = load_stream_u4(xb + (size_t)min(r + p * RPP, rows_here - 1) * xs.sn);
+    for (int p = 0; p < NPT; p++) raw[p] = load_stream_u4(xb + (size_t)min(r + p * RPP, rows_here - 1) * sn);
 #pragma unroll
     for (int p = 0; p < NPT; p++) { w[p][0] = raw[p].x; w[p][1] = raw[p].y; w[p][2] = raw[p].z; w[p][3] = raw[p].w; }
   }
@@ -224,13 +241,13 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
       constexpr int SG = NWV * 128 / D;                // partial sums per column (fold_columns)
       double(*s_part)[D] = (double(*)[D])smem;
       uint16_t *s_km = (uint16_t *)(smem + SG * D * 8);
-      const uint16_t *hb = x + (size_t)(bh / H) * xs.sb + (size_t)(bh % H) * xs.sh + c * 8;
+      const uint16_t *hb = xh + c * 8;
       double acc[8];
 #pragma unroll
       for (int e = 0; e < 8; e++) acc[e] = 0.0;
 #pragma unroll 8
       for (int row = r; row < N; row += RPP) {
-        const uint4 q = *(const uint4 *)(hb + (size_t)row * xs.sn);
+        const uint4 q = *(const uint4 *)(hb + (size_t)row * sn);
         const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -436,7 +453,7 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
       for (int i = 0; i < RG; i++) s += s_red[t_sb][i][t_col];
       // full blocks: the row count is a power of two, so the product with its reciprocal is the exact quotient
       const double mean = t_rows == BS ? s * (1.0 / BS) : s / (double)t_rows;
-      pool[((size_t)bh * nb + blk0 + t_sb) * D + t_col] = f64_to_elem_fast<DT>(mean);
+      out.pool(t_sb, t_col, f64_to_elem_fast<DT>(mean));
     }
     long long g = 0;
     if (!sim_trivial) {
@@ -504,7 +521,7 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
         const double thr = (double)simthr * (double)(rv * rv) * 281474976710656.0;
         similar = (double)gt > thr;
       }
-      sim[(size_t)bh * nb + blk0 + tid] = (!((any_bad >> tid) & 1u) && similar) ? 1 : 0;
+      out.sim(tid, !((any_bad >> tid) & 1u) && similar);
     }
   } else {
     __syncthreads();
@@ -517,7 +534,14 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
 #pragma unroll
     for (int wv = 1; wv < NWV; wv++) m_all[i] = pk_max_u16(m_all[i], s_wmax[wv][i]);
   }
-  int8_t *qb = xq + ((size_t)bh * N + row_base) * D + c * 8;
+  if (NQG > 1 && out.one_scale()) {
+    static_assert(NQG <= 4, "two words of maxima");
+    uint32_t m = m_all[0];
+    if constexpr (MW == 2) m = pk_max_u16(m, m_all[1]);
+    m = max(m & 0xffffu, m >> 16);
+#pragma unroll
+    for (int i = 0; i < MW; i++) m_all[i] = m | (m << 16);
+  }
 #pragma unroll
   for (int g = 0; g < NQG; g++) {
     // per-block scales exist for blocks with at least one row; the 32-row groups of the last Q block all get a scale
@@ -529,7 +553,7 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
 #pragma unroll
       for (int p = g * NPQ; p < (g + 1) * NPQ; p++) {
         const int row = r + p * RPP;
-        if (!decltype(check_rows)::value || row < rows_here) {
+        if (!decltype(check_rows)::value || Out::ALL_ROWS || row < rows_here) {
           float f[8];
 #pragma unroll
           for (int j = 0; j < 4; j++) {
@@ -537,7 +561,7 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
             unpack2<DT>(w[p][j], f[2 * j], f[2 * j + 1]);
           }
           const uint32_t pk0 = code4(f[0], f[1], f[2], f[3]), pk1 = code4(f[4], f[5], f[6], f[7]);
-          *(uint2 *)(qb + (size_t)row * D) = make_uint2(pk0, pk1);
+          out.codes(row, c, make_uint2(pk0, pk1));
         }
       }
     };
@@ -563,8 +587,23 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
     } else {
       quantise(divided([&](float v) { return v / s; }), std::true_type{});
     }
-    if (tid == 0) scale[((size_t)bh * nb + blk0) * GPB + g] = s;
+    if (tid == 0) out.scale(g, s);
   }
+}
+template <int BS, int D, int DT, int MEAN, bool WITH_POOL, int QR = BS, int NT = 256, int ROWS = 128>
+__device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const Strides &xs,
+                                         const uint16_t *__restrict__ km, const double *__restrict__ km_part, int km_chunks,
+                                         uint16_t *__restrict__ pool, uint8_t *__restrict__ sim,
+                                         int8_t *__restrict__ xq, float *__restrict__ scale,
+                                         const float simthr, int H, int N, int nb, int wg, int bh, unsigned char *smem) {
+  const size_t blk0 = (size_t)bh * nb + wg * (ROWS / BS);
+  PsqStore<D> out;
+  out.pool_at = pool + blk0 * D;
+  out.sim_at = sim + blk0;
+  out.xq_at = xq + ((size_t)bh * N + (size_t)wg * ROWS) * D;
+  out.scale_at = scale + blk0 * (BS / QR);
+  psq_core<BS, D, DT, MEAN, WITH_POOL, QR, NT, ROWS>(x + (size_t)(bh / H) * xs.sb + (size_t)(bh % H) * xs.sh, xs.sn, km, km_part, km_chunks,
+                                                     simthr, N, wg, bh, smem, (int)threadIdx.x, out);
 }
 
 // exclusive prefix of per-thread counts over the NT threads of the workgroup; returns (offset, total)

@@ -1,0 +1,70 @@
+"""Q quantised, and pooled for a selection in place, by the attention kernel's own workgroups: same bits as the stages one by one.
+
+Grids around the line where the route changes, partial last Q blocks of one row, 32-row groups without rows, tensors that are read through
+strides, thresholds that need the normalised rows, blocks with zero rows, NaN and infinities."""
+import pytest
+import torch
+
+import spargeattn_amd as sa
+from test_gpu_forward import _both, _bits
+from gpu_common import rand_T
+
+pytestmark = pytest.mark.gpu
+
+
+def _qkv(H, Hkv, N, Nk, D, dtype, nhd, seed):
+    q, k, v = rand_T((1, H, N, D), dtype, seed), rand_T((1, Hkv, Nk, D), dtype, seed + 1, shift=0.4), rand_T((1, Hkv, Nk, D), dtype, seed + 2)
+    q = q * torch.linspace(0.01, 2.0, N, device="cuda")[:, None].to(dtype)          # 32-row groups of different magnitude
+    q[:, :, N // 2:N // 2 + 130] = (q[:, :, :1] + 0.05 * q[:, :, N // 2:N // 2 + 130]).to(dtype)      # similar blocks
+    if H > 3 and N > 300:
+        q[:, 1, 5] = 0.0
+        q[:, 2, 140, 3] = float("nan")
+        q[:, 3, 270, 7] = float("inf")
+    return [t.transpose(1, 2).contiguous() if nhd else t for t in (q, k, v)]
+
+
+# D = 128, more than 576 rows of Q blocks; the first has exactly as many and is quantised in front
+@pytest.mark.parametrize("H,N,Nk,D", [(36, 2048, 700, 128), (48, 1537, 64, 128), (34, 2049, 1000, 128), (74, 1024, 4096, 128), (54, 1313, 4097, 128),
+                                      (64, 2049, 300, 64)])
+@pytest.mark.parametrize("dtype,gran,nhd", [(torch.bfloat16, 1, False), (torch.float16, 2, True)])
+def test_selection_in_place(H, N, Nk, D, dtype, gran, nhd):
+    q, k, v = _qkv(H, H // 2, N, Nk, D, dtype, nhd, N)
+    kw = dict(qk_quant_gran=gran, tensor_layout="NHD" if nhd else "HND", return_sparsity=True)
+    sim = torch.tensor([0.3, -0.1], device="cuda").repeat_interleave(2).repeat((H + 3) // 4)[:H].contiguous()
+    for fn in (lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.4, **kw),
+               lambda: sa.spas_sage2_attn_meansim_cuda(q, k, v, cdfthreshd=0.8, simthreshd1=0.4, attention_sink=True, **kw),
+               lambda: sa.spas_sage2_attn_meansim_cuda(q, k, v, cdfthreshd=0.9, simthreshd1=sim, **kw),
+               lambda: sa.spas_sage_attn_meansim_topk_cuda(q, k, v, topk=0.3, **kw)):
+        (o, s), (o2, s2) = _both(fn)
+        assert torch.equal(_bits(o), _bits(o2)) and s == s2
+
+
+@pytest.mark.parametrize("H,N,Nk,D", [(11, 4096, 700, 128), (11, 4097, 700, 128), (45, 1024, 9000, 128), (3, 16400, 64, 128)])     # 352 rows and more
+@pytest.mark.parametrize("dtype,gran,nhd", [(torch.bfloat16, 2, False), (torch.float16, 1, True)])
+def test_own_mask(H, N, Nk, D, dtype, gran, nhd):
+    q, k, v = _qkv(H, H, N, Nk, D, dtype, nhd, N)
+    nq, nk = -(-N // 128), -(-Nk // 64)
+    mask = (torch.rand((1, H, nq, nk), generator=torch.Generator().manual_seed(N)) < 0.4).cuda()
+    mask[..., 0] = True
+    o, o2 = _both(lambda: sa.block_sparse_sage2_attn_cuda(q, k, v, mask_id=mask, qk_quant_gran=gran, tensor_layout="NHD" if nhd else "HND"))
+    assert torch.equal(_bits(o), _bits(o2))
+
+
+def test_in_place_under_capture():
+    """The route has no state of its own: a captured call replays with other inputs in the same buffers."""
+    H, N, Nk, D = 40, 2049, 1000, 128
+    q, k, v = _qkv(H, H, N, Nk, D, torch.bfloat16, False, 1)
+    call = lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.4)       # noqa: E731
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for seed in (1, 11, 21):
+        for dst, src in zip((q, k, v), _qkv(H, H, N, Nk, D, torch.bfloat16, False, seed)):
+            dst.copy_(src)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(_bits(out), _bits(call()))

@@ -1,0 +1,22 @@
+"""Where Q is quantised: the rule on the host (tests/capi_host/routes.cpp).  The groups of wavefronts and the selection kernel take Q as codes,
+so the calls that have them keep Q in front."""
+import pytest
+
+from test_forward_routes import CDF, MASK, TOPK, pytestmark, routes  # noqa: F401
+
+
+@pytest.mark.parametrize("kw,in_front", [
+    (dict(H=36, N=2048, Nk=4096), 1), (dict(H=37, N=2048, Nk=4096), 0), (dict(H=577, N=1, Nk=3000), 0), (dict(H=577, N=128, Nk=8192, selection=CDF), 0),
+    (dict(H=577, N=128, Nk=8193, selection=CDF), 1), (dict(H=32, Hkv=8, N=4096), 0), (dict(H=577, N=128, Nk=3000, pv_f16=1), 0),
+    (dict(H=11, N=4096, selection=MASK), 1), (dict(H=11, N=4097, selection=MASK), 0), (dict(H=48, N=16384, selection=MASK), 0),
+    (dict(H=48, N=16384, D=64), 1), (dict(H=48, N=16384, D=64, selection=MASK), 1), (dict(H=48, N=8192, D=64), 1), (dict(H=700, N=128, Nk=256), 0)])
+def test_where_q_is_quantised(routes, kw, in_front):  # noqa: F811
+    assert routes(**kw)[4] == in_front
+
+
+def test_groups_never_meet_q_in_place(routes):  # noqa: F811
+    for H, N in ((1, 32768), (2, 16384), (256, 128), (4, 8192)):
+        for sel in (TOPK, CDF, MASK):
+            for Nk in (64, 800, 4096, 8192, 20000):
+                r = routes(H=H, N=N, Nk=Nk, selection=sel)
+                assert r[3] == 1 or r[4] == 1
