@@ -97,18 +97,20 @@ inline Layout layout_for(const spg_attn_args *a) {
   const size_t bh = (size_t)a->B * a->H, bhk = (size_t)a->B * a->Hkv, D = a->D;
   const size_t nq = ((size_t)a->N + 127) / 128, nk = ((size_t)a->N_kv + 63) / 64;
   const Chunks c = chunks_for(a);
-  const bool pool = a->selection != SPG_SELECT_MASK, front_q = q_in_front(a);
+  const bool pool = a->selection != SPG_SELECT_MASK;
+  // (the parts that an attention kernel which quantises Q itself does not use are there all the same: the size follows from shapes and options
+  // alone, whatever hyper-parameters a later call on the same workspace brings)
   l.km_part = take(bhk * c.n * D * 8);
   l.v_part = take(a->pv_f16 ? 0 : bhk * c.n * D * 4);
   l.km = take(bhk * D * 2);
   l.v_amax = take(bhk * D * 4);
-  l.pool_q = take(pool && front_q ? bh * nq * D * 2 : 0);
+  l.pool_q = take(pool ? bh * nq * D * 2 : 0);
   l.pool_k = take(pool ? bhk * nk * D * 2 : 0);
-  l.sim_q = take(pool && front_q ? bh * nq : 0);
+  l.sim_q = take(pool ? bh * nq : 0);
   l.sim_k = take(pool ? bhk * nk : 0);
-  l.q8 = take(front_q ? bh * a->N * D : 0);
+  l.q8 = take(bh * a->N * D);
   l.k8 = take(bhk * a->N_kv * D);
-  l.q_scale = take(front_q ? bh * nq * 4 * (a->qk_quant_gran == SPG_QUANT_PER_WARP ? 4 : 1) : 0);
+  l.q_scale = take(bh * nq * 4 * (a->qk_quant_gran == SPG_QUANT_PER_WARP ? 4 : 1));
   l.k_scale = take(bhk * nk * 4);
   l.v = take(bhk * nk * 64 * D * (a->pv_f16 ? 2 : 1));
   l.v_scale = take(bhk * D * 4);

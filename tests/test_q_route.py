@@ -20,3 +20,10 @@ def test_groups_never_meet_q_in_place(routes):  # noqa: F811
             for Nk in (64, 800, 4096, 8192, 20000):
                 r = routes(H=H, N=N, Nk=Nk, selection=sel)
                 assert r[3] == 1 or r[4] == 1
+
+
+@pytest.mark.parametrize("kw", [dict(H=24, N=3200, Nk=640), dict(H=24, N=3200, Nk=640, selection=CDF), dict(H=32, Hkv=8, N=2688, Nk=1024)])
+def test_the_workspace_serves_every_similarity_threshold(routes, kw):  # noqa: F811
+    """A workspace is sized once for a shape; with a similarity threshold short heads take another route."""
+    a, b = routes(sim=-0.1, **kw), routes(sim=0.3, **kw)
+    assert a[4] != b[4] and a[5] == b[5]
