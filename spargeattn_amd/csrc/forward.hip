@@ -299,7 +299,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   int32_t *const valid = a->valid_block_num != nullptr ? a->valid_block_num : (int32_t *)(ws + l.valid);
   // Fewer than two workgroups of 256 threads per CU leave the stages bound by the length of one thread's work (9.8 and
   // 13.0 us for the two launches at B2 H3 N1025 D128 with a similarity threshold): twice the threads take half of it.
-  const bool in_one = one_launch(a), sel_in_attn = pool && nk <= SPG_SELECT_IN_ATTN_NK, front_q = q_in_front(a);
+  const bool in_one = one_launch(a), sel_in_attn = pool && nk <= SPG_SELECT_IN_ATTN_NK, front_q = q_in_front(a) || q_overwritten(a, qs, os);
   const int q_wgs = front_q ? heads * nq : 0;
   const bool can_wide = !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP);
   const int front_nt = in_one || (q_wgs + kv_heads * 2 * c.n <= 512 && (can_wide || !front_q)) ? 512 : 256;

@@ -87,6 +87,14 @@ inline bool q_in_front(const spg_attn_args *a) {
   return a->selection == SPG_SELECT_MASK ? rows <= 352 : a->N_kv > 64 * SPG_SELECT_IN_ATTN_NK || rows <= 576;
 }
 
+// In place a workgroup reads its Q block when others have stored their output already: `out` may be q itself, row on row, or lie apart.
+inline bool q_overwritten(const spg_attn_args *a, const Strides &qs, const Strides &os) {
+  if (a->q == a->out && qs.sb == os.sb && qs.sh == os.sh && qs.sn == os.sn) return false;
+  auto bytes = [&](const Strides &s) { return (uintptr_t)(2 * ((a->B - 1) * s.sb + (a->H - 1) * s.sh + (a->N - 1) * s.sn + a->D)); };
+  const uintptr_t q = (uintptr_t)a->q, out = (uintptr_t)a->out;
+  return q < out + bytes(os) && out < q + bytes(qs);
+}
+
 struct Layout {
   size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, queue, total;
 };

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import spargeattn_amd as sa
+from spargeattn_amd import _lib
 from test_gpu_forward import _both, _bits
 from gpu_common import rand_T
 
@@ -68,3 +69,23 @@ def test_in_place_under_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(_bits(out), _bits(call()))
+
+
+@pytest.mark.parametrize("alias", ["rows", "shifted", "other_layout"])
+@pytest.mark.parametrize("selection", [_lib.SELECT_TOPK, _lib.SELECT_MASK])
+def test_output_over_q(alias, selection):
+    """Every Q block is read before another's output lands on it: the output may lie over q in any way."""
+    H, N, Nk, D = 40, 2048, 512, 128
+    buf = rand_T((H * N * D + 64 * D,), torch.bfloat16, 5)
+    q = buf[:H * N * D].view(1, H, N, D)
+    k, v = rand_T((1, H, Nk, D), torch.bfloat16, 6), rand_T((1, H, Nk, D), torch.bfloat16, 7)
+    out = {"rows": q, "shifted": buf[64 * D:].view(1, H, N, D), "other_layout": q.view(1, N, H, D).transpose(1, 2)}[alias]
+    mask = torch.ones((1, H, N // 128, Nk // 64), dtype=torch.int8, device="cuda") if selection == _lib.SELECT_MASK else None
+
+    def call(q, out):
+        plan = _lib.ForwardPlan(q, k, v, out, mask, selection, False, False, False, False, 1, D ** -0.5)
+        plan.run(q, k, v, out, mask, 0.5, -0.1, 50.0)
+        return out
+
+    want = call(q.clone(), torch.empty_like(q))
+    assert torch.equal(_bits(call(q, out).contiguous()), _bits(want))
