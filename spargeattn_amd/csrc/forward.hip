@@ -5,11 +5,11 @@
 // not depend on each other share a launch; which stage a workgroup belongs to follows from its number:
 //   short    (short heads) everything up to the selection: blocks of K and V, whose workgroups sum and search their whole head for
 //            themselves | mask rows | pooling + quantisation of Q.  Otherwise:
-//   front    partial column sums of K | partial channel maxima of V (FP16 PV: the V^T tiles, finished) | LUT rows of a
+//   front    partial column sums of K | partial channel maxima of V (FP16 PV, few blocks: the V^T tiles, finished) | LUT rows of a
 //            user mask | pooling + quantisation of Q (unless the attention kernel does that in place: q_in_front)
 //   (final   column mean of K, channel maxima of V: only where there are too many partial results for every workgroup
 //            of the next launch to add them up for itself)
-//   back     pooling + quantisation of K | V -> e4m3 tiles and scales
+//   back     pooling + quantisation of K | V -> e4m3 tiles and scales (FP16 PV, many blocks: V^T tiles)
 //   select   block_select_* of maskpred.hip (rows of more than 128 blocks; shorter ones are selected inside the next launch)
 //   attn     block_sparse_attn_kernel
 // Every body is the one the stage-by-stage entry points launch (stage_bodies.h): results are the same bits.
@@ -130,6 +130,7 @@ struct BackParams {
   int k_chunks;
   const float *v_amax, *v_part;
   int v_chunks;
+  uint16_t *v_tiles;                    // V16
   Hyper simthr;
   uint16_t *pool_k;
   uint8_t *sim_k;
@@ -140,11 +141,12 @@ struct BackParams {
 };
 
 // PARTIAL: the partial results of the front kernel are combined here, by every workgroup for the head it works on
-template <int D, int DT, bool POOL, bool PARTIAL, int NT>
+// V16: V goes to FP16 tiles (f16_tiles_in_back)
+template <int D, int DT, bool POOL, bool PARTIAL, bool V16, int NT>
 __global__ __launch_bounds__(NT) void back_kernel(const BackParams p) {
   constexpr int ROWS = k_rows_per_wg(NT);
   constexpr int LK = max_c<POOL ? psq_lds<64, D, NT, ROWS>() : 16, NT * 8 + 2 * D>();
-  constexpr int LV = v_quant_lds<D>() + 4 * NT + 4 * D;
+  constexpr int LV = V16 ? v_tiles_f16_lds<D>() : v_quant_lds<D>() + 4 * NT + 4 * D;
   __shared__ __align__(16) unsigned char smem[max_c<LK, LV>()];
   const int w = blockIdx.x;
   if (w < p.wg_v) {
@@ -153,6 +155,10 @@ __global__ __launch_bounds__(NT) void back_kernel(const BackParams p) {
     if constexpr (POOL) thr = p.simthr.at((bh % p.Hkv) * (p.H / p.Hkv));
     psq_body<64, D, DT, PARTIAL ? MEAN_PARTIAL : MEAN_GIVEN, POOL, 64, NT, ROWS>(p.k, p.ks, p.km, p.km_part, p.k_chunks, p.pool_k, p.sim_k, p.k8,
                                                                   p.k_scale, thr, p.Hkv, p.Nk, p.nk, w - bh * p.k_wgs_per_head, bh, smem);
+  } else if constexpr (V16) {
+    const int id = w - p.wg_v, bh = id / p.nk, blk = id - bh * p.nk;
+    if (p.v_dtype == 0) v_tiles_f16_body<D, 0, NT>(p.v, p.vs, p.Hkv, p.v_tiles, p.Nk, p.nk, blk, bh, smem);
+    else v_tiles_f16_body<D, 1, NT>(p.v, p.vs, p.Hkv, p.v_tiles, p.Nk, p.nk, blk, bh, smem);
   } else {
     const int id = w - p.wg_v, bh = id / p.nk, blk = id - bh * p.nk;
     float *s_amax = (float *)(smem + v_quant_lds<D>());
@@ -209,8 +215,8 @@ __global__ __launch_bounds__(512) void short_kernel(const ShortParams p) {
   } else if (w < p.wg_mask) {
     const int id = w - p.wg_v, bh = id / b.nk, blk = id - bh * b.nk;
     if (f.v_f16) {
-      if (f.v_dtype == 0) v_tiles_f16_body<D, 0, NT>(f.v, f.vs, f.Hkv, f.v_tiles, f.Nk, f.nk, blk, bh, smem);
-      else v_tiles_f16_body<D, 1, NT>(f.v, f.vs, f.Hkv, f.v_tiles, f.Nk, f.nk, blk, bh, smem);
+      if (b.v_dtype == 0) v_tiles_f16_body<D, 0, NT>(b.v, b.vs, b.Hkv, b.v_tiles, b.Nk, b.nk, blk, bh, smem);
+      else v_tiles_f16_body<D, 1, NT>(b.v, b.vs, b.Hkv, b.v_tiles, b.Nk, b.nk, blk, bh, smem);
     } else {
       float *const s_amax = (float *)(smem + max_c<v_quant_lds<D>(), v_absmax_lds<D, NT>()>());
       auto store = [&](int d, float s) { s_amax[d] = s; };
@@ -263,14 +269,15 @@ static void run_front(bool pool, bool per_warp, const FrontParams &f, int wgs, h
   else front_kernel<D, DT, false, 128, NT><<<wgs, NT, 0, st>>>(f);
 }
 template <int D, int DT, int NT>
-static void run_back(bool pool, bool partial, const BackParams &b, int wgs, hipStream_t st) {
-  if (partial) {
-    if (pool) back_kernel<D, DT, true, true, NT><<<wgs, NT, 0, st>>>(b);
-    else back_kernel<D, DT, false, true, NT><<<wgs, NT, 0, st>>>(b);
-  } else {
-    if (pool) back_kernel<D, DT, true, false, NT><<<wgs, NT, 0, st>>>(b);
-    else back_kernel<D, DT, false, false, NT><<<wgs, NT, 0, st>>>(b);
+static void run_back(bool pool, bool partial, bool v16, const BackParams &b, int wgs, hipStream_t st) {
+#define SPG_BACK(POOL_, PARTIAL_)                                                          \
+  {                                                                                        \
+    if (v16) back_kernel<D, DT, POOL_, PARTIAL_, true, NT><<<wgs, NT, 0, st>>>(b);          \
+    else back_kernel<D, DT, POOL_, PARTIAL_, false, NT><<<wgs, NT, 0, st>>>(b);             \
   }
+  if (partial) { if (pool) SPG_BACK(true, true) else SPG_BACK(false, true) }
+  else         { if (pool) SPG_BACK(true, false) else SPG_BACK(false, false) }
+#undef SPG_BACK
 }
 template <int D, int DT>
 static void run_front_back(const spg_attn_args *a, const FrontParams &f, const BackParams &b, const Chunks &c, uint16_t *km, float *v_amax,
@@ -282,8 +289,8 @@ static void run_front_back(const spg_attn_args *a, const FrontParams &f, const B
     const FinalParams p = {f.km_part, f.v_part, km, v_amax, f.k_chunks, a->pv_f16 ? 0 : f.v_chunks, a->N_kv};
     final_kernel<D, DT><<<a->B * a->Hkv, dim3(D, 8), 0, st>>>(p);
   }
-  if (back_nt == 512) run_back<D, DT, 512>(pool, c.partial, b, back_wgs, st);
-  else run_back<D, DT, 256>(pool, c.partial, b, back_wgs, st);
+  if (back_nt == 512) run_back<D, DT, 512>(pool, c.partial, f16_tiles_in_back(a), b, back_wgs, st);
+  else run_back<D, DT, 256>(pool, c.partial, f16_tiles_in_back(a), b, back_wgs, st);
 }
 
 hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides &ks, const Strides &vs, const Strides &os,
@@ -302,7 +309,9 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   const bool in_one = one_launch(a), sel_in_attn = pool && nk <= SPG_SELECT_IN_ATTN_NK, front_q = q_in_front(a) || q_overwritten(a, qs, os);
   const int q_wgs = front_q ? heads * nq : 0;
   const bool can_wide = !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP);
-  const int front_nt = in_one || (q_wgs + kv_heads * 2 * c.n <= 512 && (can_wide || !front_q)) ? 512 : 256;
+  const bool tiles_in_back = f16_tiles_in_back(a);
+  const int v_front = a->pv_f16 ? tiles_in_back ? 0 : kv_heads * nk : kv_heads * c.n;
+  const int front_nt = in_one || (q_wgs + kv_heads * (tiles_in_back ? 1 : 2) * c.n <= 512 && (can_wide || !front_q)) ? 512 : 256;
   const int back_nt = in_one || (heads * nq + kv_heads * 2 * c.n <= 512 && can_wide) ? 512 : 256;
   int nkp = 256;
   while (nkp < nk || nkp < front_nt) nkp <<= 1;
@@ -315,7 +324,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   f.v_dtype = a->v_dtype; f.v_f16 = a->pv_f16;
   f.k_chunks = f.v_chunks = c.n; f.k_rows = f.v_rows = c.rows;
   f.wg_v = kv_heads * c.n;
-  f.wg_mask = f.wg_v + kv_heads * (a->pv_f16 ? nk : c.n);
+  f.wg_mask = f.wg_v + v_front;
   f.wg_q = f.wg_mask + (mask_in_front ? heads * nq : 0);
   f.km_part = (double *)(ws + l.km_part); f.v_part = (float *)(ws + l.v_part); f.v_tiles = (uint16_t *)(ws + l.v);
   f.mask = a->mask; f.mask_kind = a->mask_kind; f.nkp = nkp; f.lut = lut; f.valid = valid;
@@ -332,7 +341,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   b.v_amax = (const float *)(ws + l.v_amax); b.v_part = f.v_part; b.v_chunks = c.n;
   b.simthr = simthr;
   b.pool_k = (uint16_t *)(ws + l.pool_k); b.sim_k = ws + l.sim_k; b.k8 = (int8_t *)(ws + l.k8); b.k_scale = (float *)(ws + l.k_scale);
-  b.v8 = ws + l.v; b.v_scale = (float *)(ws + l.v_scale);
+  b.v8 = ws + l.v; b.v_tiles = f.v_tiles; b.v_scale = (float *)(ws + l.v_scale);
 
   if (in_one) {
     ShortParams s = {f, b, 0, 0, 0};
@@ -343,7 +352,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
     if (a->D == 64) { if (a->qk_dtype == 0) run_short<64, 0>(a, s, wgs, st); else run_short<64, 1>(a, s, wgs, st); }
     else            { if (a->qk_dtype == 0) run_short<128, 0>(a, s, wgs, st); else run_short<128, 1>(a, s, wgs, st); }
   } else {
-    const int front_wgs = f.wg_q + q_wgs, back_wgs = b.wg_v + (a->pv_f16 ? 0 : kv_heads * nk);
+    const int front_wgs = f.wg_q + q_wgs, back_wgs = b.wg_v + (a->pv_f16 && !tiles_in_back ? 0 : kv_heads * nk);
     uint16_t *km = (uint16_t *)(ws + l.km);
     float *v_amax = (float *)(ws + l.v_amax);
 #define SPG_RUN(D_, DT_) run_front_back<D_, DT_>(a, f, b, c, km, v_amax, front_nt, front_wgs, back_nt, back_wgs, st)

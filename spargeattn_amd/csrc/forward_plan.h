@@ -70,6 +70,16 @@ inline bool short_heads(const spg_attn_args *a) {
 // (a pass of 512 threads over 64 channels covers two 32-row groups of Q scales)
 inline bool one_launch(const spg_attn_args *a) { return !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP) && short_heads(a); }
 
+// FP16 PV: where V's tiles are written.  They depend on nothing and are bound by memory.  In the back kernel they stand beside blocks of K, which
+// are bound by their vector instructions, and the front kernel is left with the sums of K; with no more blocks than CUs (of 128
+// channels) both kernels are chains of latencies, and only the front one has places free under it.  us per call in front / in the back
+// kernel, H x N (x Nk): D128 8 x 4096 CDF with similarity 92.0 / 88.2, 20 x 3840 103.8 / 99.5, 30 x 4096 x 1000 64.8 / 63.6, 40 x 700 41.1 / 39.8, 12 x
+// 1024 x 8000 89.2 / 87.5, 32 x 1024 x 8200 138.0 / 133.7, 24 x 8192 causal 304.4 / 302.5, 24 x 16384 755.3 / 753.1; 1 x 2500 49.4 / 49.9, 2 x 4096 45.35
+// / 45.46, 2 x 300 x 8000 121.3 / 121.6.  D64 30 x 8192 292.3 / 290.8, 16 x 1024 x 12288 95.7 / 93.9, 32 x 4096 x 8200 equal; 4 x 6000 71.9 / 72.2.
+inline bool f16_tiles_in_back(const spg_attn_args *a) {
+  return a->pv_f16 && (long long)a->B * a->Hkv * ((a->N_kv + 63) / 64) * a->D > 256 * 128 && !one_launch(a);
+}
+
 // Whether Q is quantised (and pooled) in front of the attention kernel, or in place by its workgroups.  In place Q is read once, its codes never
 // reach memory (half of Q's bytes written and read again), and the front kernel is left with K and V; but a row starts some 3 us later
 // and its vector instructions are taken from the loops beside it.  That pays at D = 128 (twice the work per row of the list at the same

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import spargeattn_amd as sa
-from spargeattn_amd import core
+from spargeattn_amd import _lib, core
 from gpu_common import rand_T
 
 pytestmark = pytest.mark.gpu
@@ -227,3 +227,18 @@ def test_many_heads_with_queries_beside_them(H, N, Nk, D):
     for fn in (sa.spas_sage2_attn_meansim_topk_cuda, sa.spas_sage_attn_meansim_topk_cuda):
         o, o2 = _both(lambda: fn(q, k, v, topk=0.1))
         assert torch.equal(_bits(o), _bits(o2))
+
+
+# partial sums combined by the back kernel, and by a launch of their own; a tail of one row, an odd number of blocks; 512 and 256 threads
+@pytest.mark.parametrize("H,N,Nk,D", [(2, 200, 3000, 128), (4, 300, 8321, 128), (30, 2049, 1601, 128), (3, 200, 3009, 64), (26, 1300, 8260, 64)])
+@pytest.mark.parametrize("vdtype", [torch.float16, torch.bfloat16])
+def test_fp16_tiles_beside_the_blocks_of_k(H, N, Nk, D, vdtype):
+    """V^T tiles come from the launch that quantises K, with a selection and with a mask: the stages' bits, and the same for all blocks."""
+    q, k, v = rand_T((1, H, N, D), vdtype, 50), rand_T((1, H, Nk, D), vdtype, 51, shift=0.4), rand_T((1, H, Nk, D), vdtype, 52)
+    o, o2 = _both(lambda: sa.spas_sage_attn_meansim_topk_cuda(q, k, v, topk=1.0))
+    assert torch.equal(_bits(o), _bits(o2))
+    mask = torch.ones((1, H, (N + 127) // 128, (Nk + 63) // 64), dtype=torch.bool, device="cuda")
+    got = torch.empty_like(q)
+    plan = _lib.ForwardPlan(q, k, v, got, mask, _lib.SELECT_MASK, True, False, False, False, 1, D ** -0.5)
+    plan.run(q, k, v, got, mask, 0.0, 0.0, 50.0)
+    assert torch.equal(_bits(got), _bits(o))
