@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       float simthr = 0.f;
       if constexpr (FQ == 2) simthr = p.q.simthr.at(head);
       psq_core<128, D, ODT, MEAN_NONE, FQ == 2, 32, 256, 128>(p.q.x + (size_t)batch * p.q.st.sb + (size_t)head * p.q.st.sh, p.q.st.sn, nullptr, nullptr, 0,
-                                                              simthr, N, qb, bh, sKr, tid, to);
+                                                              simthr, N, qb, bh, sKr, to);
       __syncthreads();
       const unsigned char *const half = (wave < 2 ? lo : hi) + ((wave & 1) * 32 + r) * D;
 #pragma unroll

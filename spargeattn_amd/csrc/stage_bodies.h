@@ -66,27 +66,36 @@ __device__ __forceinline__ float div_by(float a, float b, float r) {
   const float e = __builtin_fmaf(-b, q, a);
   return __builtin_fmaf(e, r, q);
 }
-// The INT8 code of an element a under scale s is trunc(RN(RN(a / s) + 0.5)) with the sign of a: the quotient to the nearest integer, unless it
-// comes so close to n + 1/2 that one of the roundings decides.  The quotient is off by at most 2^-24 of itself, the sum by 2^-24 (n + 1), so
-// that takes |a / s - (n + 1/2)| <= 3 2^-24 (n + 1/2).  Rounding a * RN(1 / s), off by 2^-24, once to an integer (an fma onto 1.5 2^23) gives
-// the same code for every other a.  The elements are 16-bit floats: whether any of them comes that close to (n + 1/2) s for some n is decided
-// for all of them at once, two n per lane.  t = RN((n + 1/2) s) is off by 2^-24 of itself, its difference from a 16-bit float that close is exact:
-// 2^-22 and a little for the product's own rounding covers both.  About 1 % of the blocks of bfloat16 and 9 % of binary16 have such an
-// element and take the division.  The stages in front are bound by their vector instructions as much as by memory: 2.75 instructions per element
-// for its code instead of 7 take H16 Nq8190 Nk2500 fp16 with per-warp scales from 107.2 to 104.5 us per call, H2 N4096 D128 from 44.8 to
-// 42.5, H24 N8192 with FP16 PV from 315.3 to 312.6.
-template <int DT> __device__ __forceinline__ bool no_code_near_tie(float s) {
+constexpr float CODE_MAGIC = 12582912.0f;   // 1.5 * 2^23
+// The INT8 code of an element a under scale s is trunc(RN(RN(a / s) + 0.5)) with the sign of a.
+__device__ __forceinline__ float away_from_zero(float quotient) { return quotient + __builtin_copysignf(0.5f, quotient); }
+// That is the quotient to the nearest integer, unless it comes so close to n + 1/2 that one of the roundings decides: the quotient is off by at
+// most 2^-24 of itself, the sum by 2^-24 (n + 1).  Rounding a * m once to an integer (an fma onto 1.5 2^23), with m = r = RN(1 / s), off by 2^-24,
+// or the float above it, off by 3 2^-24 at most, gives the same code for every a with |a / s - (n + 1/2)| > 3 2^-24 (n + 1/2) for all n.  The
+// others lie within 2^-22 and a little of t = RN((n + 1/2) s), and 16-bit floats are 2^-11 of themselves or more apart: of the elements up
+// to the block's maximum, for which n ends at 126, one for each n can be in doubt, the one next to t.  So all of them are decided at
+// once, two n per lane, by working out both codes of that element.  Returns an m that gives the codes of the division, or 0 if neither does.
+//
+// Counted over every maximum from 10^-3 to the formats' top: r gives the codes for 99 to 100 % of those below 100.  Above, where the 1e-7 in s
+// is lost, half the maximum is a tie, 63.5 s, that the rounding of r decides: r gives them for 55 to 65 % of the maxima, the float above it for 86
+// to 96, one of the two for 98 to 99 %.  The stages in front are bound by their vector instructions as much as by memory: 2.75
+// instructions per element for its code instead of 7.  us per call with divisions / as here, maxima of Q and K of 50 to 100: mask H48 N16384 Nk1000
+// 184.8 / 172.9, FP16 PV H24 N8192 causal 287.0 / 280.8, H16 Nq8190 Nk2500 fp16 with per-warp scales 106.5 / 102.5, GQA 32/8 N4096 100.2 /
+// 97.6, H30 N8192 D64 279.9 / 275.0, H2 N4096 43.3 / 42.7; of 400 to 800 186.3 / 173.5, 283.2 / 278.2, 107.4 / 103.3, 100.1 / 97.7, 276.7 / 273.3, 43.4 / 42.9.
+template <int DT> __device__ __forceinline__ float code_multiplier(float s, float r) {
 #pragma clang fp contract(off)
-  bool near = false;
+  const float above = __builtin_bit_cast(float, __builtin_bit_cast(int, r) + 1);
+  bool no_r = false, no_above = false;
 #pragma unroll
   for (int i = 0; i < 2; i++) {
-    const float t = ((float)(int)(64 * i + (threadIdx.x & 63)) + 0.5f) * s;
+    const float t = ((float)min(64 * i + (int)(threadIdx.x & 63), 126) + 0.5f) * s;
     const float a = elem_to_f32<DT>(f32_to_elem<DT>(t));   // the element next to t
-    near |= __builtin_fabsf(a - t) <= t * 0x1.04p-22f;
+    const float code = CODE_MAGIC + __builtin_truncf(away_from_zero(div_by(a, s, r)));
+    no_r |= __builtin_fmaf(a, r, CODE_MAGIC) != code;
+    no_above |= __builtin_fmaf(a, above, CODE_MAGIC) != code;
   }
-  return !__any(near);
+  return !__any(no_r) ? r : !__any(no_above) ? above : 0.f;
 }
-constexpr float CODE_MAGIC = 12582912.0f;   // 1.5 * 2^23
 // four floats CODE_MAGIC + code -> the four codes
 __device__ __forceinline__ uint32_t pack_codes(float v0, float v1, float v2, float v3) {
   const uint32_t b0 = __builtin_bit_cast(uint32_t, v0), b1 = __builtin_bit_cast(uint32_t, v1);
@@ -187,12 +196,11 @@ struct PsqStore {
   __device__ __forceinline__ void scale(int g, float v) const { scale_at[g] = v; }
 };
 
-// xh: first row of the (batch, head), sn: elements from row to row, wg: number of the ROWS rows, tid: thread among NT (a workgroup of
-// more threads runs the body once per NT threads, with the same results)
+// xh: first row of the (batch, head), sn: elements from row to row, wg: number of the ROWS rows; NT: threads of the workgroup
 template <int BS, int D, int DT, int MEAN, bool WITH_POOL, int QR, int NT, int ROWS, class Out>
 __device__ __forceinline__ void psq_core(const uint16_t *__restrict__ xh, long long sn, const uint16_t *__restrict__ km,
                                          const double *__restrict__ km_part, int km_chunks, const float simthr, int N, int wg, int bh,
-                                         unsigned char *smem, int tid, const Out &out) {
+                                         unsigned char *smem, const Out &out) {
 #pragma clang fp contract(off)
   constexpr int SUB = ROWS / BS;      // blocks per workgroup
   constexpr int TPR = D / 8;          // lanes per row (16 B each)
@@ -214,7 +222,7 @@ __device__ __forceinline__ void psq_core(const uint16_t *__restrict__ xh, long l
   // "every element of the row is tiny": bfloat16 below 2^-63 (both top exponent bits clear), binary16 zero
   constexpr uint32_t TINY2 = DT == 1 ? 0x60006000u : 0x7fff7fffu;
   constexpr bool HAS_MEAN = MEAN != MEAN_NONE;
-  const int c = tid % TPR, r = tid / TPR;
+  const int tid = threadIdx.x, c = tid % TPR, r = tid / TPR;
   const int row_base = wg * ROWS;
   const int rows_here = min(ROWS, N - row_base);          // >= 1
   const bool partial = rows_here < ROWS;                  // workgroup-uniform: only the last workgroup of a head
@@ -542,13 +550,18 @@ __device__ __forceinline__ void psq_core(const uint16_t *__restrict__ xh, long l
 #pragma unroll
     for (int i = 0; i < MW; i++) m_all[i] = m | (m << 16);
   }
+  float s, rs, m;
 #pragma unroll
   for (int g = 0; g < NQG; g++) {
     // per-block scales exist for blocks with at least one row; the 32-row groups of the last Q block all get a scale
     // (1e-7 for a group without rows, what the reference's quantiser writes for an all-masked group)
     if (QR == BS && rows_here - g * QR <= 0) break;     // workgroup-uniform
-    const float amax = elem_to_f32<DT>((uint16_t)(m_all[g / 2] >> (16 * (g % 2))));
-    const float s = amax / 127.0f + 1e-7f;
+    if (g == 0 || !out.one_scale()) {
+      const float amax = elem_to_f32<DT>((uint16_t)(m_all[g / 2] >> (16 * (g % 2))));
+      s = amax / 127.0f + 1e-7f;
+      rs = exact_rcp(s);
+      m = rcp_safe(s) ? code_multiplier<DT>(s, rs) : 0.f;
+    }
     auto quantise = [&](auto code4, auto check_rows) {
 #pragma unroll
       for (int p = g * NPQ; p < (g + 1) * NPQ; p++) {
@@ -565,28 +578,29 @@ __device__ __forceinline__ void psq_core(const uint16_t *__restrict__ xh, long l
         }
       }
     };
-    // one fma and three quarters of a permute per element where no quotient is near a tie, otherwise the division and its rounding:
-    // truncation toward zero, low 8 bits of element e into byte e % 4 (+0.5 for t >= 0: a -0 quotient truncates to 0 either way)
-    const float rs = exact_rcp(s);
-    auto nearest = [&](float f0, float f1, float f2, float f3) {
-      return pack_codes(__builtin_fmaf(f0, rs, CODE_MAGIC), __builtin_fmaf(f1, rs, CODE_MAGIC), __builtin_fmaf(f2, rs, CODE_MAGIC), __builtin_fmaf(f3, rs, CODE_MAGIC));
+    auto all_rows = [&](auto code4) {
+      if (Out::ALL_ROWS || !partial) quantise(code4, std::false_type{});     // (the common case carries no row test)
+      else quantise(code4, std::true_type{});
+    };
+    // One fma and three quarters of a permute per element where a multiplier gives the codes (a NaN, which the maximum leaves out,
+    // passes through the fma with a zero low byte: the low mantissa bits of a widened 16-bit float are zero), otherwise the division:
+    // truncation toward zero, low 8 bits of element e into byte e % 4 (a -0 quotient truncates to 0 either way, a NaN, too).
+    auto product = [&](float f0, float f1, float f2, float f3) {
+      return pack_codes(__builtin_fmaf(f0, m, CODE_MAGIC), __builtin_fmaf(f1, m, CODE_MAGIC), __builtin_fmaf(f2, m, CODE_MAGIC), __builtin_fmaf(f3, m, CODE_MAGIC));
     };
     auto divided = [&](auto divide) {
       return [&, divide](float f0, float f1, float f2, float f3) {
-        auto away = [&](float f) { const float t = divide(f); return t + __builtin_copysignf(0.5f, t); };
         uint32_t pk;
-        cvt_trunc_to_byte<0>(pk, away(f0)); cvt_trunc_to_byte<1>(pk, away(f1)); cvt_trunc_to_byte<2>(pk, away(f2)); cvt_trunc_to_byte<3>(pk, away(f3));
+        cvt_trunc_to_byte<0>(pk, away_from_zero(divide(f0)));
+        cvt_trunc_to_byte<1>(pk, away_from_zero(divide(f1)));
+        cvt_trunc_to_byte<2>(pk, away_from_zero(divide(f2)));
+        cvt_trunc_to_byte<3>(pk, away_from_zero(divide(f3)));
         return pk;
       };
     };
-    if (rcp_safe(s) && no_code_near_tie<DT>(s)) {          // workgroup-uniform
-      if (!partial) quantise(nearest, std::false_type{});    // (the common case carries no row test)
-      else quantise(nearest, std::true_type{});
-    } else if (rcp_safe(s)) {
-      quantise(divided([&](float v) { return div_by(v, s, rs); }), std::true_type{});
-    } else {
-      quantise(divided([&](float v) { return v / s; }), std::true_type{});
-    }
+    if (m != 0.f) all_rows(product);                       // workgroup-uniform
+    else if (rcp_safe(s)) all_rows(divided([&](float v) { return div_by(v, s, rs); }));
+    else quantise(divided([&](float v) { return v / s; }), std::true_type{});
     if (tid == 0) out.scale(g, s);
   }
 }
@@ -603,7 +617,7 @@ __device__ __forceinline__ void psq_body(const uint16_t *__restrict__ x, const S
   out.xq_at = xq + ((size_t)bh * N + (size_t)wg * ROWS) * D;
   out.scale_at = scale + blk0 * (BS / QR);
   psq_core<BS, D, DT, MEAN, WITH_POOL, QR, NT, ROWS>(x + (size_t)(bh / H) * xs.sb + (size_t)(bh % H) * xs.sh, xs.sn, km, km_part, km_chunks,
-                                                     simthr, N, wg, bh, smem, (int)threadIdx.x, out);
+                                                     simthr, N, wg, bh, smem, out);
 }
 
 // exclusive prefix of per-thread counts over the NT threads of the workgroup; returns (offset, total)
