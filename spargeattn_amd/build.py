@@ -36,11 +36,11 @@ NO_SPILL = {"attn.hip", "dense.hip"}
 RESOURCE_REMARKS = "-Rpass-analysis=kernel-resource-usage"
 # The same kernels issue some LDS reads through inline asm and wait for them in a LATER asm statement (the reads run
 # under matrix instructions).  In between, the compiler believes the destination registers are already written; the
-# generated code of this compiler version was inspected for copies or live-range splits inside those windows and has
-# none: in all 72 attention kernels (FP8 PV, where a window is half of the operands; FP16 PV, where it is a step of two or four
-# reads behind a partial wait) and both dense ones, no instruction names a register of such a read before the wait that
-# covers it, and no label or branch lies in between.  Another compiler may schedule differently: the build then says so,
-# loudly, and asks for the check to be redone (SPARGEATTN_AMD_ALLOW_UNVALIDATED_COMPILER=1 silences the failure, not the warning).
+# generated code has to be free of copies or live-range splits inside those windows.  tests/test_lds_read_windows.py
+# disassembles the built kernels and follows every path through them: no instruction names a register of an LDS read
+# before the wait that covers it, in any of the 72 attention kernels or the two dense ones.  Another compiler
+# may schedule differently: the build then says so, loudly, and asks for that test
+# (SPARGEATTN_AMD_ALLOW_UNVALIDATED_COMPILER=1 silences the failure, not the warning).
 VALIDATED_COMPILERS = ("roc-7.2.0",)
 
 
@@ -91,8 +91,8 @@ def build(verbose=True):
     if not ok:
         msg = ("spargeattn_amd.build: hipcc is not a validated version (" + ", ".join(VALIDATED_COMPILERS) + "):\n  "
                + version.replace("\n", "\n  ") + "\nattn.hip / dense.hip read LDS through inline asm whose waits come "
-               "later; re-inspect the generated code around those windows (or run the GPU parity tests) before trusting "
-               "this build.")
+               "later; build with SPARGEATTN_AMD_ALLOW_UNVALIDATED_COMPILER=1 and run tests/test_lds_read_windows.py before "
+               "trusting this build.")
         print("WARNING: " + msg, file=sys.stderr)
         if os.environ.get("SPARGEATTN_AMD_ALLOW_UNVALIDATED_COMPILER") != "1":
             raise RuntimeError(msg + "\nSet SPARGEATTN_AMD_ALLOW_UNVALIDATED_COMPILER=1 to build anyway.")
