@@ -311,7 +311,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   const bool can_wide = !(a->D == 64 && a->qk_quant_gran == SPG_QUANT_PER_WARP);
   const bool tiles_in_back = f16_tiles_in_back(a);
   const int v_front = a->pv_f16 ? tiles_in_back ? 0 : kv_heads * nk : kv_heads * c.n;
-  const int front_nt = in_one || (q_wgs + kv_heads * (tiles_in_back ? 1 : 2) * c.n <= 512 && (can_wide || !front_q)) ? 512 : 256;
+  const int front_nt = in_one || (q_wgs + front_chunk_wgs(a) <= 512 && (can_wide || !front_q)) ? 512 : 256;
   const int back_nt = in_one || (heads * nq + kv_heads * 2 * c.n <= 512 && can_wide) ? 512 : 256;
   int nkp = 256;
   while (nkp < nk || nkp < front_nt) nkp <<= 1;

@@ -80,21 +80,39 @@ inline bool f16_tiles_in_back(const spg_attn_args *a) {
   return a->pv_f16 && (long long)a->B * a->Hkv * ((a->N_kv + 63) / 64) * a->D > 256 * 128 && !one_launch(a);
 }
 
+// Heads of K and V that the front kernel reads in chunks, and the workgroups that this takes.  Up to 512 of them, blocks of Q among them,
+// have 512 threads each.
+inline long long front_chunk_heads(const spg_attn_args *a) { return (long long)a->B * a->Hkv * (f16_tiles_in_back(a) ? 1 : 2); }
+inline long long front_chunk_wgs(const spg_attn_args *a) { return front_chunk_heads(a) * chunks_for(a).n; }
+
 // Whether Q is quantised (and pooled) in front of the attention kernel, or in place by its workgroups.  In place Q is read once, its codes never
 // reach memory (half of Q's bytes written and read again), and the front kernel is left with K and V; but a row starts some 3 us later
 // and its vector instructions are taken from the loops beside it.  That pays at D = 128 (twice the work per row of the list at the same
-// cost) once rows beside each other cover the start, from about two per CU, and earlier for a caller's mask, which needs no pooling.  us
-// per call in front / in place, H x N, top-k 0.5 unless noted: 10 x 3840 66.7 / 70.1, 13 x 3900 85.5 / 89.3, 16 x 3900 89.7 / 92.4, 8 x 8192 118.0 /
-// 119.3, 20 x 3840 91.9 / 89.7, 25 x 3840 101.4 / 99.0, 20 x 5120 143.4 / 142.8, 30 x 3840 122.7 / 121.2, GQA 32/8 x 4096 causal 103.0 / 98.4, 48
-// x 8192 x 400 100.2 / 96.5, CDF with similarity 32 x 8000 697 / 689, 20 x 5120 239.3 / 240.5, FP16 PV 20 x 3840 106.5 / 105.5, 32 x 8000
-// 487 / 482; masks 5 x 7680 84.3 / 87.9, 40 x 1024 41.2 / 43.3, 7 x 7300 91.1 / 87.2, 8 x 8000 101.1 / 95.5, 14 x 7300 139.8 / 132.8, 48 x 16384 1342 /
-// 1318, 48 x 16384 x 1000 193.4 / 177.9.  D = 64: 14 x 6400 95.5 / 96.5, 22 x 6400 140.2 / 143.3, 30 x 8192 265.6 / 266.4, CDF 40 x 8000 585 /
-// 605; masks 12 x 7500 83.9 / 84.8, 20 x 10240 124.1 / 125.7, 16 x 16384 325.7 / 325.3, 48 x 16384 657 / 650.  Where a selection kernel
-// wants Q pooled, the front kernel reads Q anyway: H32 N32768 causal 3953 / 3952, H30 N17776 D64 1007 / 1012.
+// cost) once rows beside each other cover the start.  us per call in front / in place, H x N (x Nk), two processes a side in turn:
+// * with a selection from about two rows per CU, with a similarity threshold or without (of 144 shapes of 588 to 1300 rows and 400 to 2500 keys
+//   each, top-k gains 2.0 % on average, CDF with similarity 1.4, FP16 PV 2.1; the largest losses are 2 %, just past the 768 rows that the chip holds at
+//   once, 2.6 % with 400 keys).  Top-k 0.5: 10 x 5760 89.9 / 93.0, 16 x 4096 76.4 / 77.3, 20 x 3840 91.9 / 89.2, 40 x 2048 70.4 / 68.3, 80 x 1024 61.5 / 59.8, 24 x
+//   4096 causal 97.5 / 93.9, 128 x 1024 83.0 / 82.5, 40 x 2560 x 700 53.7 / 54.6; CDF with similarity 16 x 3584 109.2 / 112.0, 10 x 8192 251 / 253, 20 x 3840 146.4 /
+//   144.1, 24 x 4096 170 / 165, 20 x 5120 239.5 / 240.7, 32 x 8000 686 / 681, 40 x 2048 106.8 / 102.3, 24 x 8192 x 1000 115.9 / 111.9, 48 x 2176 x 400 67.5 / 69.3;
+//   FP16 PV 80 x 1024 61.0 / 57.5, 20 x 3840 99.7 / 99.1, 16 x 8192 causal 217.2 / 214.4.
+// * with a caller's mask, which needs no pooling, from 352 rows, if what is left to the front kernel is few enough workgroups to have 512 threads
+//   each, which is most of that gain: 5 x 7680 82.8 / 85.8, 7 x 6528 83.3 / 80.8, 7 x 8192 99.3 / 94.2, 10 x 5120 74.6 / 72.8, 14 x 3712 63.9 / 63.8, 14 x
+//   5248 89.3 / 85.2, GQA 32/8 x 1664 41.8 / 39.7, 28/4 x 2304 47.8 / 45.3.
+// * with a mask and more heads of K, once the front kernel is bound by what it reads, from about 50 MB of Q, K and V (in a smaller one Q is
+//   quantised beside chains of sums that take as long without it) and 480 rows: 20 x 2560 54.4 / 57.4, 28 x 2048 52.4 / 53.7, 36 x 2048 60.8 / 61.2, 48 x 1024
+//   42.3 / 43.9, 80 x 640 39.8 / 41.8, 20 x 3712 77.3 / 77.5, 28 x 2944 73.6 / 72.5, 60 x 2048 85.8 / 82.2, 80 x 1024 57.9 / 55.7, 48 x 16384 1342 / 1318; 28 x 2688 x 1000
+//   43.1 / 45.7, 36 x 2048 x 800 40.7 / 43.2, 44 x 2048 x 500 37.6 / 38.8, 22 x 4608 x 800 43.0 / 45.3, 28 x 3712 x 1500 57.9 / 57.8, 44 x 2944 x 800 54.9 / 53.9, 36 x 4608 x 1500
+//   76.2 / 71.2, 48 x 16384 x 1000 193.4 / 177.9; 7 x 6528 x 12000 119.0 / 120.6, 7 x 9344 x 12000 equal.  Of 377 masks the rule is 0.1 % on average behind
+//   the better side of each; 352 rows for all of them were 1 % and up to 7 %.
+// D = 64: 14 x 6400 95.5 / 96.5, 22 x 6400 140.2 / 143.3, 30 x 8192 265.6 / 266.4, CDF 40 x 8000 585 / 605; masks 12 x 7500 83.9 / 84.8, 20 x 10240 124.1 /
+// 125.7, 16 x 16384 325.7 / 325.3, 48 x 16384 657 / 650.  Where a selection kernel wants Q pooled, the front kernel reads Q anyway: H32 N32768
+// causal 3953 / 3952, H30 N17776 D64 1007 / 1012.
 inline bool q_in_front(const spg_attn_args *a) {
   const long long rows = (long long)a->B * a->H * ((a->N + 127) / 128);
   if (a->D == 64 || one_launch(a)) return true;
-  return a->selection == SPG_SELECT_MASK ? rows <= 352 : a->N_kv > 64 * SPG_SELECT_IN_ATTN_NK || rows <= 576;
+  if (a->selection != SPG_SELECT_MASK) return a->N_kv > 64 * SPG_SELECT_IN_ATTN_NK || rows <= 576;
+  if (front_chunk_wgs(a) <= 512) return rows <= 352;
+  return rows <= 480 || rows * 128 + front_chunk_heads(a) * a->N_kv <= 196608;   // (16-bit rows of 128 channels)
 }
 
 // In place a workgroup reads its Q block when others have stored their output already: `out` may be q itself, row on row, or lie apart.

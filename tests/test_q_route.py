@@ -14,6 +14,15 @@ def test_where_q_is_quantised(routes, kw, in_front):  # noqa: F811
     assert routes(**kw)[4] == in_front
 
 
+@pytest.mark.parametrize("kw,in_front", [
+    (dict(H=24, N=2048), 1), (dict(H=28, N=2304), 1), (dict(H=28, N=2432), 0), (dict(H=48, N=1024), 1), (dict(H=80, N=1024), 0),
+    (dict(H=44, N=2048, Nk=500), 1), (dict(H=28, N=2688, Nk=1000), 1), (dict(H=36, N=4608, Nk=800), 0), (dict(H=60, N=1024, Nk=9000), 1),
+    (dict(H=61, N=1024, Nk=9000), 0), (dict(H=32, Hkv=8, N=1408), 1), (dict(H=32, Hkv=8, N=1409), 0)])
+def test_masks_over_many_heads_keep_q_in_front_of_small_grids(routes, kw, in_front):  # noqa: F811
+    """In front of a grid that its reads do not fill, the blocks of Q cost nothing: 24 heads N2048 took 49.8 us a call, 53.0 in place."""
+    assert routes(selection=MASK, **kw)[4] == in_front
+
+
 def test_groups_never_meet_q_in_place(routes):  # noqa: F811
     for H, N in ((1, 32768), (2, 16384), (256, 128), (4, 8192)):
         for sel in (TOPK, CDF, MASK):
