@@ -127,3 +127,29 @@ def test_codes_of_blocks_of_every_route(dtype, D):
         want = mp.pool_sim_quant(to_np(t), None, bs, np.zeros(H, F), tag_of(dtype), **kw)
         assert np.array_equal(got[2].cpu().numpy(), want["q"])
         assert np.array_equal(got[3].cpu().numpy().view(np.uint32), want["scale"].view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_groups_of_different_routes_in_one_block(dtype, D):
+    """The four 32-row groups of a block have routes and scales of their own, in every order; the last block has 40 rows."""
+    from spargeattn_amd import _lib
+    rng = np.random.default_rng(3)
+    all_max = _finite(dtype, 48.0, 6e4)
+    routes = _route(all_max, dtype)
+    H, N = 6, 128 * 4 + 40
+    x = np.zeros((1, H, N, D), F)
+    for h in range(H):
+        for g in range(0, N, 32):
+            amax = rng.choice(all_max[routes == rng.integers(3)])
+            near = _next_to_ties(_scale(amax), dtype).view(torch.int16)
+            rows = np.minimum(np.concatenate([(near + d).view(dtype).float().numpy() for d in (0, 1, -1)]), amax)
+            part = np.concatenate([[amax], rows, -rows]).astype(F)
+            n = min(32, N - g) * D
+            x[0, h, g:g + 32].flat[:min(n, part.size)] = part[:n]
+    t = torch.from_numpy(x).to(dtype).cuda()
+    got = _lib.pool_sim_quant(t, None, 128, torch.zeros(H, device="cuda"), quant_rows=32)
+    want = mp.pool_sim_quant(to_np(t), None, 128, np.zeros(H, F), tag_of(dtype), quant_rows=32)
+    assert np.array_equal(got[2].cpu().numpy(), want["q"])
+    assert np.array_equal(got[3].cpu().numpy().view(np.uint32), want["scale"].view(np.uint32))
