@@ -51,6 +51,41 @@ def test_own_mask(H, N, Nk, D, dtype, gran, nhd):
     assert torch.equal(_bits(o), _bits(o2))
 
 
+# B, H, Hkv, N, Nk, causal: two batch entries and grouped heads, one and two columns per lane of the selection, partial last blocks on both sides
+BATCHED = [(2, 24, 8, 1600, 1600, True), (2, 5, 5, 8000, 8000, True), (2, 10, 2, 4200, 4200, True), (2, 26, 13, 1537, 2500, False), (2, 9, 3, 4225, 6000, False)]
+
+
+@pytest.mark.parametrize("B,H,Hkv,N,Nk,causal", BATCHED)
+@pytest.mark.parametrize("dtype,gran,nhd", [(torch.bfloat16, 1, True), (torch.float16, 2, False)])
+def test_batched_and_causal(B, H, Hkv, N, Nk, causal, dtype, gran, nhd):
+    parts = [_qkv(H, Hkv, N, Nk, 128, dtype, nhd, 17 * b + N) for b in range(B)]
+    q, k, v = (torch.cat(t) for t in zip(*parts))
+    kw = dict(qk_quant_gran=gran, tensor_layout="NHD" if nhd else "HND", return_sparsity=True, is_causal=causal)
+    for kernel_causal in ((False, True) if causal else (False,)):
+        for fn in (lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, topk=0.4, kernel_causal=kernel_causal, **kw),
+                   lambda: sa.spas_sage2_attn_meansim_cuda(q, k, v, cdfthreshd=0.8, simthreshd1=0.4, kernel_causal=kernel_causal, **kw)):
+            (o, s), (o2, s2) = _both(fn)
+            assert torch.equal(_bits(o), _bits(o2)) and s == s2
+    (o, s), (o2, s2) = _both(lambda: sa.spas_sage_attn_meansim_topk_cuda(q, k, v, topk=0.3, **kw))
+    assert torch.equal(_bits(o), _bits(o2)) and s == s2
+
+
+# B, H, Hkv, N, Nk: few heads of K, and many of them
+MASKS = [(1, 11, 11, 4097, 1100), (2, 4, 4, 6017, 2000), (1, 3, 3, 16400, 1300), (2, 32, 16, 1537, 2000), (1, 62, 62, 1024, 9000)]
+
+
+@pytest.mark.parametrize("B,H,Hkv,N,Nk", MASKS)
+@pytest.mark.parametrize("dtype,gran,nhd", [(torch.bfloat16, 2, False), (torch.float16, 1, True)])
+def test_batched_masks(B, H, Hkv, N, Nk, dtype, gran, nhd):
+    parts = [_qkv(H, Hkv, N, Nk, 128, dtype, nhd, 19 * b + N) for b in range(B)]
+    q, k, v = (torch.cat(t) for t in zip(*parts))
+    mask = torch.rand((B, H, -(-N // 128), -(-Nk // 64)), generator=torch.Generator().manual_seed(N)) < 0.4
+    mask[..., 0] = True
+    mask = mask.cuda()
+    o, o2 = _both(lambda: sa.block_sparse_sage2_attn_cuda(q, k, v, mask_id=mask, qk_quant_gran=gran, tensor_layout="NHD" if nhd else "HND"))
+    assert torch.equal(_bits(o), _bits(o2))
+
+
 def test_in_place_under_capture():
     """The route has no state of its own: a captured call replays with other inputs in the same buffers."""
     H, N, Nk, D = 40, 2049, 1000, 128
@@ -71,11 +106,8 @@ def test_in_place_under_capture():
         assert torch.equal(_bits(out), _bits(call()))
 
 
-@pytest.mark.parametrize("alias", ["rows", "shifted", "other_layout"])
-@pytest.mark.parametrize("selection", [_lib.SELECT_TOPK, _lib.SELECT_MASK])
-def test_output_over_q(alias, selection):
-    """Every Q block is read before another's output lands on it: the output may lie over q in any way."""
-    H, N, Nk, D = 40, 2048, 512, 128
+def _output_over_q(alias, selection, N):
+    H, Nk, D = 40, 512, 128
     buf = rand_T((H * N * D + 64 * D,), torch.bfloat16, 5)
     q = buf[:H * N * D].view(1, H, N, D)
     k, v = rand_T((1, H, Nk, D), torch.bfloat16, 6), rand_T((1, H, Nk, D), torch.bfloat16, 7)
@@ -89,3 +121,15 @@ def test_output_over_q(alias, selection):
 
     want = call(q.clone(), torch.empty_like(q))
     assert torch.equal(_bits(call(q, out).contiguous()), _bits(want))
+
+
+@pytest.mark.parametrize("alias", ["rows", "shifted", "other_layout"])
+@pytest.mark.parametrize("selection", [_lib.SELECT_TOPK, _lib.SELECT_MASK])
+def test_output_over_q(alias, selection):
+    """Every Q block is read before another's output lands on it: the output may lie over q in any way."""
+    _output_over_q(alias, selection, 2048)
+
+
+@pytest.mark.parametrize("alias", ["rows", "shifted", "other_layout"])
+def test_output_over_q_with_a_mask_in_place(alias):
+    _output_over_q(alias, _lib.SELECT_MASK, 4608)

@@ -2,6 +2,7 @@
 so the calls that have them keep Q in front."""
 import pytest
 
+from test_gpu_q_in_place import BATCHED, MASKS
 from test_forward_routes import CDF, MASK, TOPK, pytestmark, routes  # noqa: F401
 
 
@@ -36,3 +37,12 @@ def test_the_workspace_serves_every_similarity_threshold(routes, kw):  # noqa: F
     """A workspace is sized once for a shape; with a similarity threshold short heads take another route."""
     a, b = routes(sim=-0.1, **kw), routes(sim=0.3, **kw)
     assert a[4] != b[4] and a[5] == b[5]
+
+
+def test_the_tests_of_q_in_place_reach_it(routes):  # noqa: F811
+    for B, H, Hkv, N, Nk, _ in BATCHED:
+        for kw in (dict(selection=TOPK), dict(selection=CDF, sim=0.4), dict(selection=TOPK, pv_f16=1)):
+            assert routes(B=B, H=H, Hkv=Hkv, N=N, Nk=Nk, **kw)[4] == 0
+    for B, H, Hkv, N, Nk in MASKS:
+        assert routes(B=B, H=H, Hkv=Hkv, N=N, Nk=Nk, selection=MASK)[4] == 0
+    assert routes(H=40, N=4608, Nk=512, selection=MASK)[4] == 0          # (output over q)
