@@ -290,7 +290,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   const uint32_t lds_v0 = lds_k0 + NBUF * TILE;
 
   // A row that is not in its loop yet leaves the matrix units idle: at the loop's own priority its selection takes half as long beside two
-  // other rows (8.8 us, 4.3), 30 heads N17776 D64 go from 1023 to 1013 us per call.
+  // other rows (8.8 us, 4.3).  us per call with the priority from the loop on / from here, medians of five processes a side: CDF with similarity
+  // 32 x 4096 224.0 / 215.6, GQA 32/8 x 4096 causal 100.5 / 99.7, 16 x 8190 x 2500 102.7 / 101.9, top-k 48 x 4096 188.1 / 187.6, 32 x 8192 392.9 / 391.1; 24 x 4096
+  // CDF, FP16 PV, masks and D = 64 equal, 30 x 17776 D64 with a LUT from a selection kernel 1010 / 1008.
   if constexpr (G == 1) __builtin_amdgcn_s_setprio(3);
   int bh, qb, item = blockIdx.x;
   if constexpr (SEL == 0) {                    // (short rows: the grid is over before the XCDs drift apart)
@@ -1029,10 +1031,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     // small kernels of another stream take as long either way (an addition over a million floats 54.6, 51.5 with priority and 50.5, 51.4
     // without, 4.5 us alone).
     int drop_at = 0x7fffffff;
-    if constexpr (G == 1) {
-      __builtin_amdgcn_s_setprio(3);
+    if constexpr (G == 1)
       if ((item >> 3) >= p.wg_per_xcd - SPG_PLACES) drop_at = nv >> 1;
-    }
 #pragma unroll 1
     for (; it + NBUF <= n_fast; it += NBUF) {
       if constexpr (G == 1) {
