@@ -74,7 +74,8 @@ __device__ __forceinline__ float away_from_zero(float quotient) { return quotien
 // or the float above it, off by 3 2^-24 at most, gives the same code for every a with |a / s - (n + 1/2)| > 3 2^-24 (n + 1/2) for all n.  The
 // others lie within 2^-22 and a little of t = RN((n + 1/2) s), and 16-bit floats are 2^-11 of themselves or more apart: of the elements up
 // to the block's maximum, for which n ends at 126, one for each n can be in doubt, the one next to t.  So all of them are decided at
-// once, two n per lane, by working out both codes of that element.  Returns an m that gives the codes of the division, or 0 if neither does.
+// once, two n per lane, by working out both codes of that element.  Returns an m that gives the codes of the division, r where it does, or 0 if
+// neither does.
 //
 // Counted over every maximum from 10^-3 to the formats' top: r gives the codes for 99 to 100 % of those below 100.  Above, where the 1e-7 in s
 // is lost, half the maximum is a tie, 63.5 s, that the rounding of r decides: r gives them for 55 to 65 % of the maxima, the float above it for 86
@@ -84,17 +85,21 @@ __device__ __forceinline__ float away_from_zero(float quotient) { return quotien
 // 97.6, H30 N8192 D64 279.9 / 275.0, H2 N4096 43.3 / 42.7; of 400 to 800 186.3 / 173.5, 283.2 / 278.2, 107.4 / 103.3, 100.1 / 97.7, 276.7 / 273.3, 43.4 / 42.9.
 template <int DT> __device__ __forceinline__ float code_multiplier(float s, float r) {
 #pragma clang fp contract(off)
-  const float above = __builtin_bit_cast(float, __builtin_bit_cast(int, r) + 1);
-  bool no_r = false, no_above = false;
+  const float n0 = (float)(threadIdx.x & 63) + 0.5f;
+  auto differs = [&](float m) {
+    bool any = false;
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const float t = ((float)min(64 * i + (int)(threadIdx.x & 63), 126) + 0.5f) * s;
-    const float a = elem_to_f32<DT>(f32_to_elem<DT>(t));   // the element next to t
-    const float code = CODE_MAGIC + __builtin_truncf(away_from_zero(div_by(a, s, r)));
-    no_r |= __builtin_fmaf(a, r, CODE_MAGIC) != code;
-    no_above |= __builtin_fmaf(a, above, CODE_MAGIC) != code;
-  }
-  return !__any(no_r) ? r : !__any(no_above) ? above : 0.f;
+    for (int i = 0; i < 2; i++) {
+      const float t = (i == 0 ? n0 : fminf(n0 + 64.f, 126.5f)) * s;
+      const float a = elem_to_f32<DT>(f32_to_elem<DT>(t));   // the element next to t
+      const uint16_t code = (uint16_t)(uint32_t)(div_by(a, s, r) + 0.5f);
+      any |= (uint16_t)__builtin_bit_cast(uint32_t, __builtin_fmaf(a, m, CODE_MAGIC)) != code;   // (CODE_MAGIC ends in 22 zero bits)
+    }
+    return __any(any) != 0;
+  };
+  if (!differs(r)) return r;
+  const float above = __builtin_bit_cast(float, __builtin_bit_cast(int, r) + 1);
+  return !differs(above) ? above : 0.f;
 }
 // four floats CODE_MAGIC + code -> the four codes
 __device__ __forceinline__ uint32_t pack_codes(float v0, float v1, float v2, float v3) {
