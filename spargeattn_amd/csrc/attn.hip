@@ -77,6 +77,7 @@ struct PsqToLds {
 #define SPG_QUEUE_EXTRA 12          // one workgroup in so many is launched on top
 #define SPG_PLACES 96               // last rows of an XCD that lower their priority: 32 CUs x 3, the rows it works on at a time at D = 128.  D = 64
                                     // fits four workgroups per CU (124 registers, 25 KB): 112 and 128 make no difference there, one number for both
+#define SPG_START_PRIO_MAX 1024     // workgroups, beyond the places for them, up to which rows that select in place start at the loop's priority
 #define SPG_LOG2E 1.44269504088896340736f
 
 // n / d for 0 <= n < 2^31 as a multiplication and a shift: m = ceil(2^(31+s) / d) with 2^(s-1) < d <= 2^s is a 32-bit number, and
@@ -290,10 +291,16 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   const uint32_t lds_v0 = lds_k0 + NBUF * TILE;
 
   // A row that is not in its loop yet leaves the matrix units idle: at the loop's own priority its selection takes half as long beside two
-  // other rows (8.8 us, 4.3).  us per call with the priority from the loop on / from here, medians of five processes a side: CDF with similarity
-  // 32 x 4096 224.0 / 215.6, GQA 32/8 x 4096 causal 100.5 / 99.7, 16 x 8190 x 2500 102.7 / 101.9, top-k 48 x 4096 188.1 / 187.6, 32 x 8192 392.9 / 391.1; 24 x 4096
-  // CDF, FP16 PV, masks and D = 64 equal, 30 x 17776 D64 with a LUT from a selection kernel 1010 / 1008.
-  if constexpr (G == 1) __builtin_amdgcn_s_setprio(3);
+  // other rows (8.8 us, 4.3), at the expense of those.  That pays with a LUT, where the start is short, on any grid, and with a selection in
+  // place where a few rows more than there are places start when little else runs.  Where all rows start at once there is nothing to gain (24 x
+  // 2351 71.0 / 71.2); on larger grids gains and losses are even, but for those of up to two rounds with a partial last Q block: its rows keep all
+  // their blocks, begin first and end last, and every row that starts beside them makes them later.  us per call with the priority from
+  // the loop on / from here, top-k at D = 128 unless noted, H x N: CDF with similarity 32 x 4096 224.0 / 215.6, GQA 32/8 x 4096 causal 100.5 / 99.7,
+  // 16 x 8190 x 2500 102.7 / 101.9, 24 x 4480 125.3 / 117.5, 24 x 4401 129.6 / 125.8, 48 x 2560 99.3 / 95.3; 32 x 4608 147.3 / 146.0, 24 x 7424 232.2 / 232.3, 24 x
+  // 5553 166.1 / 170.6, 24 x 7345 254.7 / 263.6, 32 x 5553 203.3 / 217.5, 48 x 3633 158.2 / 167.6, FP16 PV 24 x 5414 239.6 / 250.3; LUT 30 x 17776 D64 1010 /
+  // 1008, 16 x 11000 D64 195.9 / 189.9, D128 294.7 / 292.6.
+  if constexpr (G == 1)
+    if (SEL == 0 || (p.total_wg > 8 * SPG_PLACES && p.total_wg <= SPG_START_PRIO_MAX)) __builtin_amdgcn_s_setprio(3);
   int bh, qb, item = blockIdx.x;
   if constexpr (SEL == 0) {                    // (short rows: the grid is over before the XCDs drift apart)
     if (p.queue != nullptr) {
@@ -1031,8 +1038,10 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     // small kernels of another stream take as long either way (an addition over a million floats 54.6, 51.5 with priority and 50.5, 51.4
     // without, 4.5 us alone).
     int drop_at = 0x7fffffff;
-    if constexpr (G == 1)
+    if constexpr (G == 1) {
+      __builtin_amdgcn_s_setprio(3);
       if ((item >> 3) >= p.wg_per_xcd - SPG_PLACES) drop_at = nv >> 1;
+    }
 #pragma unroll 1
     for (; it + NBUF <= n_fast; it += NBUF) {
       if constexpr (G == 1) {
