@@ -41,6 +41,8 @@ SIGNATURES = {
     "spg_block_sparse_attn": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _vp, _vp]),
     "spg_v_tiles_f16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "spg_block_sparse_attn_f16v": (_i, [_vp] * 5 + [_i] + [_vp] * 5 + [_i] * 6 + [_f, _i, _i, _i, _vp, _vp]),
+    "spg_block_sparse_attn_chunks_bytes": (_sz, [_i] * 6 + [_f, _i]),
+    "spg_block_sparse_attn_chunks": (_i, [_vp] * 5 + [_i] + [_vp] * 6 + [_i] * 6 + [_f, _i, _i, _vp, _c.c_uint64, _vp]),
     "spg_sparse_attn_workspace_bytes": (_sz, [_vp]),
     "spg_sparse_attn": (_i, [_vp, _vp]),
     "spg_dense_attn_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _f, _i, _vp]),
@@ -339,14 +341,33 @@ def _check_attn_shapes(q8, k8, vt, lut, valid, q_scale, k_scale, v_scale=None, q
     return B, H, Hkv, N, Nk, D
 
 
+def _in_chunks(q8, k8, v, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, sm_scale, is_causal, qk_quant_gran, selected):
+    """Few long rows, as the whole-operator call takes them (spg_block_sparse_attn_chunks).  selected: (selection, top-k fraction or
+    None, causal) of the lists.  False where a row has one workgroup."""
+    (B, H, N, D), (Hkv, Nk) = q8.shape, k8.shape[1:3]
+    selection, share, causal = selected
+    # (0.0 stays 0.0: a negative share means that nothing is known)
+    size = load().spg_block_sparse_attn_chunks_bytes(B, H, N, Nk, D, selection, -1.0 if share is None else max(float(share), 0.0), int(bool(causal)))
+    if size == 0:
+        return False
+    workspace = torch.empty(size, dtype=torch.uint8, device=q8.device)
+    _check(load().spg_block_sparse_attn_chunks(_p(q8), _p(k8), _p(v), _p(out), _st(out), _dt(out), _p(lut), _p(valid), _p(pvthreshd), _p(q_scale),
+                                               _p(k_scale), _p(v_scale), B, H, Hkv, N, Nk, D, float(sm_scale), int(bool(is_causal)),
+                                               qk_quant_gran, _p(workspace), size, _stream()))
+    return True
+
+
 def block_sparse_attn(q8, k8, v8, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, sm_scale,
-                      is_causal=False, return_pv_count=False, pv_mode=PV_PER_BLOCK, qk_quant_gran=QUANT_PER_BLOCK):
+                      is_causal=False, return_pv_count=False, pv_mode=PV_PER_BLOCK, qk_quant_gran=QUANT_PER_BLOCK, selected=None):
     _dev(q8, k8, v8, lut, valid, pvthreshd, q_scale, k_scale, v_scale)
     _dev_strided(out)
     qk_quant_gran = quant_gran(qk_quant_gran)
     B, H, Hkv, N, Nk, D = _check_attn_shapes(q8, k8, v8, lut, valid, q_scale, k_scale, v_scale, qk_quant_gran)
     if tuple(out.shape) != (B, H, N, D) or pvthreshd.numel() != H:
         raise RuntimeError("out must have q's shape and pvthreshd one entry per query head")
+    if selected is not None and not return_pv_count and pv_mode == PV_PER_BLOCK and \
+            _in_chunks(q8, k8, v8, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, sm_scale, is_causal, qk_quant_gran, selected):
+        return None
     if _torch() is not None:
         pvc = _ops.block_sparse_attn(q8, k8, v8, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, float(sm_scale),
                                      bool(is_causal), qk_quant_gran, int(pv_mode), bool(return_pv_count))
@@ -459,13 +480,16 @@ def v_tiles_f16_to_natural(vt):
 
 
 def block_sparse_attn_f16v(q8, k8, vt, out, lut, valid, pvthreshd, q_scale, k_scale, sm_scale, is_causal=False,
-                           return_pv_count=False, pv_mode=PV_PER_BLOCK, qk_quant_gran=QUANT_PER_BLOCK):
+                           return_pv_count=False, pv_mode=PV_PER_BLOCK, qk_quant_gran=QUANT_PER_BLOCK, selected=None):
     _dev(q8, k8, vt, lut, valid, pvthreshd, q_scale, k_scale)
     _dev_strided(out)
     qk_quant_gran = quant_gran(qk_quant_gran)
     B, H, Hkv, N, Nk, D = _check_attn_shapes(q8, k8, vt, lut, valid, q_scale, k_scale, None, qk_quant_gran)
     if tuple(out.shape) != (B, H, N, D) or pvthreshd.numel() != H:
         raise RuntimeError("out must have q's shape and pvthreshd one entry per query head")
+    if selected is not None and not return_pv_count and pv_mode == PV_PER_BLOCK and \
+            _in_chunks(q8, k8, vt, out, lut, valid, pvthreshd, q_scale, k_scale, None, sm_scale, is_causal, qk_quant_gran, selected):
+        return None
     if _torch() is not None:
         pvc = _ops.block_sparse_attn_f16v(q8, k8, vt, out, lut, valid, pvthreshd, q_scale, k_scale, float(sm_scale),
                                           bool(is_causal), qk_quant_gran, int(pv_mode), bool(return_pv_count))

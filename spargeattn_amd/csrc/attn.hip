@@ -114,7 +114,42 @@ struct AttnParams {
   int rows_first;  // so many of the longest rows of every head come before the rest (place_workgroup)
   RowSelect sel;   // selection inside the kernel (template argument SEL); lut is unused then
   RawQ q;          // Q as the caller has it (template argument FQ); q8, q_scale, sel.pool_q and sel.sim_q are unused then
+  RowSplit split;  // rows in chunks (template argument SPLIT)
+  FastDiv by_chunks;    // (rows + 7) / 8 (place_part)
 };
+
+// The chunks of a row with `nv` blocks: as few as hold at most `split.per` of them each, of equal length; chunk c is places begin(c) to
+// begin(c + 1) - 1 of the list.  A row's last two blocks are in its last chunk.
+struct RowChunks {
+  uint32_t nv, n;
+  __device__ __forceinline__ RowChunks(int nv_, const RowSplit &split)
+      : nv((uint32_t)nv_), n((uint32_t)max(1, min(split.chunks, (nv_ + split.per - 1) / split.per))) {}
+  __device__ __forceinline__ int begin(int c) const { return (int)((uint32_t)c * nv / n); }
+  // Rows start at different chunks: workgroups that start together would else ask for the same tiles at the same time.  us per call, one
+  // head N17776, all rows from their first / in turn: D64 top-k 0.5 100.3 / 96.6, all blocks kept 139.8 / 135.0; D128 2 x 14000 145.0 / 141.9.
+  __device__ __forceinline__ int turned(int part, int row) const { return (int)((uint32_t)(part + row) % n); }
+};
+// Workgroup -> (row, part of it).  An XCD works on consecutive rows of a head, from the last one down; the first parts of all its rows
+// come first, so that parts which shorter rows do not have leave no gaps among those that are there.
+__device__ __forceinline__ bool place_part(const AttnParams &p, int id, int &bh, int &qb, int &part) {
+  const int x = id & 7, j = id >> 3, first = x * p.split.rows >> 3, rows = ((x + 1) * p.split.rows >> 3) - first;
+  part = p.by_chunks(j);
+  const int i = j - part * ((p.split.rows + 7) >> 3);
+  if (i >= rows) return false;
+  bh = p.by_nq(first + i);
+  qb = p.nq - 1 - (first + i - bh * p.nq);
+  return true;
+}
+// inclusive prefix sums over a wavefront (DPP: shifts within rows of sixteen, then the last lane of a row to those behind it)
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
 
 // Workgroup -> (batch*head, q block).  Ids are dealt round-robin over the 8 XCDs; each XCD (one L2) gets a contiguous
 // range of (head, row) pairs, rows from the last one down: causal rows get longer with the row index, and a partial last
@@ -224,6 +259,40 @@ void launch_fp8_pack_selftest(const float *x, uint8_t *codes, int n, int saturat
   fp8_pack_selftest_kernel<<<(n4 + 255) / 256, 256, 0, st>>>(x, (uint32_t *)codes, n4, saturate);
 }
 
+// Output rows of one wavefront, O / d * v_scale rounded to the output type: through LDS (`orow_lds`, 32 rows) and out as whole rows,
+// 16 bytes per lane.
+constexpr int orow_bytes(int D) { return 2 * D + 16; }      // padded row: the 8-byte writes of 32 rows spread over the banks
+template <int D, int ODT, bool PV16>
+__device__ __forceinline__ void store_rows(const v16f (&O)[D / 32], float inv, unsigned char *orow_lds, const float *v_scale, const AttnParams &p,
+                                           int batch, int head, int row0, uint32_t lane) {
+  constexpr int NDT = D / 32, OROW = orow_bytes(D);
+  const int r_e = (int)lane & 31, hh_e = (int)lane >> 5;
+#pragma unroll
+  for (int dt = 0; dt < NDT; dt++) {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const int d0 = 32 * dt + 8 * g + 4 * hh_e;
+      float4 sc = make_float4(1.f, 1.f, 1.f, 1.f);
+      if constexpr (!PV16) sc = *(const float4 *)(v_scale + d0);
+      const uint16_t o0 = f32_to_elem<ODT>(O[dt][4 * g + 0] * inv * sc.x);
+      const uint16_t o1 = f32_to_elem<ODT>(O[dt][4 * g + 1] * inv * sc.y);
+      const uint16_t o2 = f32_to_elem<ODT>(O[dt][4 * g + 2] * inv * sc.z);
+      const uint16_t o3 = f32_to_elem<ODT>(O[dt][4 * g + 3] * inv * sc.w);
+      *(uint2 *)(orow_lds + r_e * OROW + d0 * 2) = make_uint2((uint32_t)o0 | ((uint32_t)o1 << 16), (uint32_t)o2 | ((uint32_t)o3 << 16));
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  constexpr int LPR = D / 8, RPI = 64 / LPR;                 // lanes per row, rows per store instruction
+  uint16_t *obase = (uint16_t *)p.out + (size_t)batch * p.os.sb + (size_t)head * p.os.sh + ((int)lane % LPR) * 8;
+#pragma unroll
+  for (int i = 0; i < 32 / RPI; i++) {
+    const int row = i * RPI + (int)lane / LPR, grow = row0 + row;
+    const uint4 t = *(const uint4 *)(orow_lds + row * OROW + ((int)lane % LPR) * 16);
+    if (grow < p.N) *(uint4 *)(obase + (size_t)grow * p.os.sn) = t;
+  }
+}
+
 // 16-byte-chunk swizzles.  K tile row = key (D bytes, D/16 chunks); V^T tile row = channel (64 bytes, 4 chunks).
 // The LDS serves a ds_read_b128 one half-wavefront (32 lanes) at a time and needs two clocks for it when the 32
 // addresses fall evenly on the sixteen 16-byte slots of a 256-byte line (two lanes per slot); a slot that is hit 2k
@@ -258,7 +327,8 @@ __device__ __forceinline__ int v_swz(int row) { return (row >> 2) & 3; }
 // FQ: 0 Q comes as INT8 codes and scales; 1 the workgroup quantises its Q block itself; 2 it pools it, too, and works out its similarity
 // flag, for a selection in place (SEL).  Codes, pooled row and flag stay in LDS: what a kernel in front would write (half of Q's bytes
 // and more) and this one read again.
-template <int D, int ODT, bool PV16, int SEL, int G, int FQ>
+// SPLIT: a row's blocks go over several workgroups, each with a stretch of its list (launch_row_maxima has the why).
+template <int D, int ODT, bool PV16, int SEL, int G, int FQ, bool SPLIT>
 __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_kernel(const AttnParams p) {
   constexpr int KS = D / 32;        // k-steps of the int8 MFMA
   constexpr int NDT = D / 32;       // 32-channel output tiles
@@ -302,7 +372,12 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   if constexpr (G == 1)
     if (SEL == 0 || (p.total_wg > 8 * SPG_PLACES && p.total_wg <= SPG_START_PRIO_MAX)) __builtin_amdgcn_s_setprio(3);
   int bh, qb, item = blockIdx.x;
-  if constexpr (SEL == 0) {                    // (short rows: the grid is over before the XCDs drift apart)
+  static_assert(!SPLIT || (SEL == 0 && G == 1 && FQ == 0), "rows in chunks come with a list and with codes of Q");
+  int chunk = 0;
+  int chunks = 1, chunk_begin = 0, chunk_end = 0;
+  if constexpr (SPLIT) {
+    if (!place_part(p, item, bh, qb, chunk)) return;
+  } else if constexpr (SEL == 0) {                    // (short rows: the grid is over before the XCDs drift apart)
     if (p.queue != nullptr) {
       __shared__ int sItem;
       if (threadIdx.x == 0) sItem = take_item(p, item);
@@ -311,7 +386,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       if (item < 0) return;
     }
   }
-  if (!place_workgroup(p, item & 7, item >> 3, bh, qb)) return;
+  if constexpr (!SPLIT)
+    if (!place_workgroup(p, item & 7, item >> 3, bh, qb)) return;
   const int batch = p.by_H(bh), head = bh - batch * p.H;
   // grouped-query attention: H / Hkv consecutive query heads share one K/V head (sm89.cuh:118, head_id / num_kv_groups)
   const int bhk = batch * p.Hkv + p.by_group(head);
@@ -327,13 +403,25 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   typedef const __attribute__((address_space(4))) int32_t *c_i32_t;
   typedef const __attribute__((address_space(4))) float *c_f32_t;
   const size_t row_id = (size_t)bh * p.nq + qb;
-  const c_i32_t lutc = (c_i32_t)(p.lut + (SEL > 0 ? 0 : row_id * p.nk));
-  const int last_col = p.nk - 1;
+  const int32_t *list = p.lut + (SEL > 0 ? 0 : row_id * p.nk);
+  int last_col = p.nk - 1, chunk_first = 0;
+  if constexpr (SPLIT) {
+    const RowChunks c(((c_i32_t)p.valid)[row_id], p.split);
+    if (chunk >= (int)c.n) return;
+    chunk = c.turned(chunk, qb);
+    chunks = (int)c.n;
+    chunk_begin = c.begin(chunk);
+    chunk_end = c.begin(chunk + 1);
+    chunk_first = chunk > 0 ? ((c_i32_t)p.split.first)[row_id * p.split.chunks + chunk] : ((c_i32_t)list)[0];
+    list += chunk_begin;
+    last_col -= chunk_begin;
+  }
+  const c_i32_t lutc = (c_i32_t)list;
   int nv, l0, l1, l2, l3;
   if constexpr (SEL == 0 && G > 1) nv = ((c_i32_t)p.valid)[row_id];
   if constexpr (SEL == 0 && G == 1) {
-    nv = ((c_i32_t)p.valid)[row_id];
-    l0 = lutc[0]; l1 = lutc[min(1, last_col)]; l2 = lutc[min(2, last_col)]; l3 = lutc[min(3, last_col)];
+    nv = SPLIT ? chunk_end - chunk_begin : ((c_i32_t)p.valid)[row_id];
+    l0 = SPLIT ? chunk_first : lutc[0]; l1 = lutc[min(1, last_col)]; l2 = lutc[min(2, last_col)]; l3 = lutc[min(3, last_col)];
   }
   // per-warp granularity: the 32 query rows of a wavefront are one quantisation group, so the scale stays a scalar
   float qs;
@@ -558,8 +646,14 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   const uint32_t v_rd16 = (uint32_t)(r * 128 + (((4 * hh) ^ ((r >> 1) & 7)) * 16));
 
   float m = SPG_NEG_BIG;
+  if constexpr (SPLIT) {
+    // the running maximum in front of the chunk's first block
+    const float *cm = p.split.maxima + row_id * p.split.chunks * 128 + wave * 32 + r;
+#pragma unroll 4
+    for (int i = 0; i < chunk; i++) m = fmaxf(m, cm[i * 128]);
+  }
   // d = 1.0 initially (sm89.cuh:172).  Each half-lane sums its own 32 keys, so only one of the two starts at 1.
-  float dsum = hh == 0 && grp == 0 ? 1.0f : 0.0f;
+  float dsum = hh == 0 && grp == 0 && chunk == 0 ? 1.0f : 0.0f;
   float m_own = SPG_NEG_BIG;               // groups: the maximum that this group's O and dsum refer to
   v16f O[NDT];
 #pragma unroll
@@ -837,9 +931,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
       SPG_LANE_OFFSETS()
       (void)pos0;
       const uint32_t here = CS ? (uint32_t)(SLOT * TILE) : bufoff;
-      if (!TAIL || it + 2 < nv) SPG_LOAD_K_(blk2, here, (TAIL || SLOT < 0));
-      if (!TAIL || it + 1 < nv) SPG_LOAD_V_(blk1, 2 * (here ^ (uint32_t)TILE));
-    } else if (!TAIL || place + 2 * G < nv) {
+      if ((!TAIL && !(SPLIT && !CS)) || it + 2 < nv) SPG_LOAD_K_(blk2, here, (TAIL || SLOT < 0));
+      if ((!TAIL && !(SPLIT && !CS)) || it + 1 < nv) SPG_LOAD_V_(blk1, 2 * (here ^ (uint32_t)TILE));
+    } else if ((!TAIL && !(SPLIT && !CS)) || place + 2 * G < nv) {
       if constexpr (CS) {
         SPG_LOAD_TILES(blk2, ((SLOT + 2) % 3) * TILE, 0);
       } else {
@@ -1022,7 +1116,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     int it = 0;
     // rounds whose successor's successor ends in front of the last block (no partial tile to load); rounds in front of the
     // last two blocks; all rounds
-    const int n_fast = G == 1 ? nv - 3 : (nv - 1) / G - 2, n_common = G == 1 ? nv - 2 : (nv - 2) / G, n_all = (nv + G - 1) / G;
+    const int n_fast = G == 1 ? nv - 3 : (nv - 1) / G - 2, n_all = (nv + G - 1) / G;
+    const int n_common = G > 1 ? (nv - 2) / G : SPLIT && chunk < chunks - 1 ? nv : nv - 2;   // (only a row's last two blocks are masked)
     // the common loop, one block per ring slot and trip; the slots are compile-time constants and `bufoff` stays 0.  (FP16 PV with
     // run-time slots: H24 N8192 D128 causal 333 us, so 329; H6 N16384 381 / 377, H10 N5000 122 / 120, H1 N12000 D64 121 / 119.)
     // The wavefronts of a SIMD are served oldest first: of the three rows on a CU the first runs at almost the speed it would
@@ -1075,6 +1170,30 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   if (p.pv_count != nullptr && lane == 0) p.pv_count[((size_t)bh * p.nq + qb) * 4 + wave] = cnt;
 
   // ---- epilogue: O / d * v_scale -> out dtype -----------------------------------------------------------
+  if constexpr (SPLIT) {
+    // (worked out again: no register holds them across the loop)
+    int id = blockIdx.x;
+    asm volatile("" : "+s"(id));
+    const size_t row_id = (size_t)bh * p.nq + qb;
+    const RowChunks c(((c_i32_t)p.valid)[row_id], p.split);
+    const int chunk = c.turned(p.by_chunks(id >> 3), qb);
+    if (c.n > 1) {                         // sums of the chunk, relative to its maximum; combine_chunks_kernel goes on
+      const size_t at = row_id * p.split.chunks + chunk;
+      const float d_chunk = half_swap_sum_f32(dsum);
+      uint32_t l = threadIdx.x & 63u;
+      asm volatile("" : "+v"(l));
+      const uint32_t q = wave * 32 + (l & 31u);
+      float4 *const so = (float4 *)p.split.o + (at * 4 + wave) * (NDT * 4 * 64) + l;
+#pragma unroll
+      for (int i = 0; i < NDT * 4; i++)
+        so[i * 64] = make_float4(O[i / 4][4 * (i % 4)], O[i / 4][4 * (i % 4) + 1], O[i / 4][4 * (i % 4) + 2], O[i / 4][4 * (i % 4) + 3]);
+      if (l < 32) {
+        p.split.md[at * 256 + q] = m;
+        p.split.md[at * 256 + 128 + q] = d_chunk;
+      }
+      return;
+    }
+  }
   float dtot = half_swap_sum_f32(dsum);
   if constexpr (G > 1) {
     // the groups' sums, relative to the row's final maximum, meet in the (free) tile rings; group 0 goes on alone
@@ -1110,42 +1229,222 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   // (computed again: no register holds them across the loop)
   uint32_t lane_e = threadIdx.x & 63u;
   asm volatile("" : "+v"(lane_e));
-  const int r_e = (int)lane_e & 31, hh_e = (int)lane_e >> 5;
   const float inv = __builtin_amdgcn_rcpf(dtot);
   // A lane holds four channels of one row per group: stored from here, an instruction would touch 32 rows with 16 bytes
   // each.  The rows of a wavefront go through LDS instead (the tile ring is free once every wavefront is past its last
   // P.V product) and leave as whole rows, 16 bytes per lane.
-  constexpr int OROW = 2 * D + 16;                           // padded row: the 8-byte writes of 32 rows spread over the banks
+  constexpr int OROW = orow_bytes(D);
   static_assert(4 * 32 * OROW <= G * NBUF * (TILE + VTILE), "output rows of four wavefronts fit the tile ring");
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   if (grp > 0) return;
-  unsigned char *const orow_lds = smem + wave * (32 * OROW);
+  store_rows<D, ODT, PV16>(O, inv, smem + wave * (32 * OROW), sVscale, p, batch, head, qb * 128 + wave * 32, lane_e);
+}
+
+// ---- rows in chunks ------------------------------------------------------------------------------------------------
+// Maxima of the chunks of a row but the last, per query, over the scores as block_sparse_attn_kernel sees them: its running maximum
+// in front of a chunk is the largest of those before it, to the bit, since it takes the same products in binary32.
+// A wavefront holds all 128 queries and takes every fourth block of the chunk, with a tile of its own in LDS: nothing is read twice and
+// nothing waits for another wavefront until the end.  (Operands straight from memory, 32 rows to an instruction, are bound by the lines that
+// those touch: 35 us instead of 27 for 15 400 blocks at D = 128.)  Bound by its chain - count, list, Q block, tiles - and the rounding up to
+// whole workgroups per CU: the matrix instructions of those 15 400 blocks take 7 us.
+template <int D>
+__global__ __launch_bounds__(256, D == 64 ? 4 : 3) void row_maxima_kernel(const AttnParams p) {
+  constexpr int KS = D / 32;
+  __shared__ __align__(1024) unsigned char s_tile[4][64 * D];   // of one wavefront each
+  __shared__ __align__(1024) unsigned char s_q[128 * D];
+  __shared__ int s_id[256], s_sum[2][4];
+  __shared__ float s_max[4][128];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int bh, qb, chunk;
+  if (!place_part(p, blockIdx.x, bh, qb, chunk)) return;
+  const int batch = p.by_H(bh), head = bh - batch * p.H, bhk = batch * p.Hkv + p.by_group(head);
+  const size_t row_id = (size_t)bh * p.nq + qb;
+  const RowChunks chunks(p.valid[row_id], p.split);
+  if (chunk >= (int)chunks.n - 1) return;            // (the maximum of a row's last chunk is nobody's)
+  const int begin = chunks.begin(chunk), total = chunks.begin(chunk + 1) - begin;
+  const int32_t *const list = p.lut + row_id * p.nk;
+  int before = 0;                                    // sum of the differences in front
+#pragma unroll 4
+  for (int i = tid; i < begin; i += 256) before += list[i];
+  int diff = tid < total ? list[begin + tid] : 0;
+  const int behind = list[begin + total];
+  typedef __attribute__((address_space(3))) void *lds_ptr_t;
+  typedef const __attribute__((address_space(1))) void *glb_ptr_t;
+  {
+    // Q block to LDS, rows beyond N as the last one: chunks of 16 bytes swizzled as a K tile's
+    const int8_t *qb8 = p.q8 + ((size_t)bh * p.N + qb * 128) * D;
+    constexpr int CPR = D / 16;
 #pragma unroll
-  for (int dt = 0; dt < NDT; dt++) {
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-      const int d0 = 32 * dt + 8 * g + 4 * hh_e;
-      float4 sc = make_float4(1.f, 1.f, 1.f, 1.f);
-      if constexpr (!PV16) sc = *(const float4 *)(sVscale + d0);
-      const uint16_t o0 = f32_to_elem<ODT>(O[dt][4 * g + 0] * inv * sc.x);
-      const uint16_t o1 = f32_to_elem<ODT>(O[dt][4 * g + 1] * inv * sc.y);
-      const uint16_t o2 = f32_to_elem<ODT>(O[dt][4 * g + 2] * inv * sc.z);
-      const uint16_t o3 = f32_to_elem<ODT>(O[dt][4 * g + 3] * inv * sc.w);
-      *(uint2 *)(orow_lds + r_e * OROW + d0 * 2) = make_uint2((uint32_t)o0 | ((uint32_t)o1 << 16), (uint32_t)o2 | ((uint32_t)o3 << 16));
+    for (int u = 0; u < D / 32; u++) {
+      const uint32_t pos = (uint32_t)((wave * (D / 32) + u) * 64 + lane), row_ = pos / CPR, slot = pos % CPR;
+      const uint32_t off = min(row_, (uint32_t)(p.N - 1 - qb * 128)) * D + (slot ^ k_swz<D>(row_ & 63)) * 16u;
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(qb8 + off), (lds_ptr_t)(s_q + (wave * (D / 32) + u) * 1024), 16, 0, 0);
     }
   }
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  constexpr int LPR = D / 8, RPI = 64 / LPR;                 // lanes per row, rows per store instruction
-  uint16_t *obase = (uint16_t *)p.out + (size_t)batch * p.os.sb + (size_t)head * p.os.sh + ((int)lane_e % LPR) * 8;
+  float cq26[4], m[4];
 #pragma unroll
-  for (int i = 0; i < 32 / RPI; i++) {
-    const int row = i * RPI + (int)lane_e / LPR, grow = qb * 128 + wave * 32 + row;
-    const uint4 t = *(const uint4 *)(orow_lds + row * OROW + ((int)lane_e % LPR) * 16);
-    if (grow < N) *(uint4 *)(obase + (size_t)grow * p.os.sn) = t;
+  for (int s = 0; s < 4; s++) {
+    cq26[s] = p.sm_scale_log2 * p.q_scale[p.q_per_warp ? row_id * 4 + s : row_id] * SPG_ACC_SCALE;
+    m[s] = SPG_NEG_BIG;
   }
+  // a tile to LDS, one wavefront on its own: chunks of 16 bytes swizzled as block_sparse_attn_kernel has them
+  constexpr int TILE = 64 * D;
+  const int8_t *kbase = p.k8 + (size_t)bhk * p.Nk * D;
+  const uint32_t lane_off = ((uint32_t)lane ^ (D == 128 ? (lane >> 4) & 3u : (lane >> 4) & 1u)) << 4;
+  unsigned char *const tile = s_tile[wave];
+  auto fetch = [&](int blk) __attribute__((always_inline)) {
+    const int8_t *kb = kbase + (size_t)(uint32_t)blk * TILE;
+#pragma unroll
+    for (int u = 0; u < TILE / 1024; u++)       // rows from 32 on: one more bit of the swizzle
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(kb + u * 1024 + (lane_off ^ (u >= TILE / 2048 ? (D == 128 ? 64u : 32u) : 0u))),
+                                       (lds_ptr_t)(tile + u * 1024), 16, 0, 0);
+  };
+  const int krow0 = 32 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3), ksw = k_swz<D>(krow0);
+  const uint32_t k_rd = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)tile + (uint32_t)(krow0 * D + ((hh ^ ksw) & 1) * 16);
+  uint32_t kaddr[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) kaddr[ks] = k_rd + ((uint32_t)(32 * ks) ^ (uint32_t)((ksw & 6) * 16));
+  const float *kscale = p.k_scale + (size_t)bhk * p.nk;
+  before = wave_prefix_sum(before);
+  if (lane == 63) s_sum[1][wave] = before;
+  int base = 0;
+  v4i q[4][KS];
+  for (int t0 = 0; t0 < total; t0 += 256) {
+    // ids of up to 256 blocks: running sums of the differences
+    const int n = min(256, total - t0);
+    if (t0 > 0) diff = tid < n ? list[begin + t0 + tid] : 0;
+    int s = wave_prefix_sum(diff);
+    if (lane == 63) s_sum[0][wave] = s;
+    __builtin_amdgcn_s_waitcnt(0x0F70);        // vmcnt(0): this wavefront's share of the Q block
+    __syncthreads();
+    if (t0 == 0) {
+      base = s_sum[1][0] + s_sum[1][1] + s_sum[1][2] + s_sum[1][3];
+#pragma unroll
+      for (int s4 = 0; s4 < 4; s4++) {
+        // query 32 s4 + r, chunk 2 ks + hh
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+          q[s4][ks] = *(const v4i *)(s_q + (32 * s4 + r) * D + (((2 * ks + hh) ^ k_swz<D>((32 * s4 + r) & 63)) * 16));
+          if (qb * 128 + 32 * s4 + r >= p.N) q[s4][ks] = (v4i){0, 0, 0, 0};
+        }
+      }
+    }
+    s += base;
+    for (int w = 0; w < wave; w++) s += s_sum[0][w];
+    base += s_sum[0][0] + s_sum[0][1] + s_sum[0][2] + s_sum[0][3];
+    s_id[tid] = s;
+    __syncthreads();
+    const int ids = s_id[min(wave + 4 * lane, n - 1)];         // of this wavefront: in a register
+    const int mine = wave < n ? (n - wave + 3) / 4 : 0;
+    int blk = __builtin_amdgcn_readlane(ids, 0);
+    if (mine > 0) fetch(blk);
+    float ksc = kscale[blk];
+#pragma unroll 1
+    for (int i = 0; i < mine; i++) {
+      v4i a[2][KS];
+      __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): the tile has arrived
+      asm volatile("" ::: "memory");
+      lds_read_4x128_wait<0, 16 * D>(a[0][0], a[1][0], a[0][1], a[1][1], kaddr[0], kaddr[1]);
+      if constexpr (KS == 4) lds_read_4x128_wait<0, 16 * D>(a[0][2], a[1][2], a[0][3], a[1][3], kaddr[2], kaddr[3]);
+      blk = __builtin_amdgcn_readlane(ids, min(i + 1, 63));
+      if (i + 1 < mine) fetch(blk);            // under the products; the operands are in registers
+      const float ksc1 = kscale[blk];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s4 = 0; s4 < 4; s4++) {
+        v16i S0, S1;
+        // (both chains beside each other: left to itself the compiler puts them one behind the other into the same registers)
+        asm volatile("v_mfma_i32_32x32x32_i8 %0, %2, %4, 0\n\tv_mfma_i32_32x32x32_i8 %1, %3, %4, 0"
+                     : "=&v"(S0), "=&v"(S1)
+                     : "v"(a[0][0]), "v"(a[1][0]), "v"(q[s4][0]));
+#pragma unroll
+        for (int ks = 1; ks < KS; ks++) {
+          S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[0][ks], q[s4][ks], S0, 0, 0, 0);
+          S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[1][ks], q[s4][ks], S1, 0, 0, 0);
+        }
+        int imax = S0[0];
+#pragma unroll
+        for (int e = 1; e < 16; e++) imax = max(imax, S0[e]);
+#pragma unroll
+        for (int e = 0; e < 16; e++) imax = max(imax, S1[e]);
+        // 2^-26 imax is what the attention kernel reads off its accumulator
+        m[s4] = fmaxf(m[s4], ((float)imax * (1.0f / SPG_ACC_SCALE)) * (cq26[s4] * ksc));
+      }
+      ksc = ksc1;
+    }
+    __syncthreads();
+  }
+  if (tid == 0) p.split.first[row_id * p.split.chunks + chunk + 1] = base + behind;   // where the next chunk starts
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const float v = half_swap_max_f32(m[s]);
+    if (lane < 32) s_max[wave][s * 32 + r] = v;
+  }
+  __syncthreads();
+  if (tid < 128)
+    p.split.maxima[(row_id * p.split.chunks + chunk) * 128 + tid] = fmaxf(fmaxf(s_max[0][tid], s_max[1][tid]), fmaxf(s_max[2][tid], s_max[3][tid]));
+}
+
+// The chunks of a row, each relative to its own maximum, brought to the row's (that of the last chunk) and added up in their order.
+// A workgroup takes 32 channels of a row, as the lanes of the attention kernel hold them.
+template <int D, int ODT, bool PV16>
+__global__ __launch_bounds__(256) void combine_chunks_kernel(const AttnParams p) {
+  constexpr int NDT = D / 32;
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int bh, qb, dt;
+  if (!place_part(p, blockIdx.x, bh, qb, dt)) return;
+  const int batch = p.by_H(bh), head = bh - batch * p.H, bhk = batch * p.Hkv + p.by_group(head);
+  const size_t row_id = (size_t)bh * p.nq + qb;
+  const int chunks = (int)RowChunks(p.valid[row_id], p.split).n;
+  if (chunks == 1) return;                 // the row is finished
+  const float *md = p.split.md + row_id * p.split.chunks * 256 + wave * 32 + r;
+  const float4 *so = (const float4 *)p.split.o + (row_id * p.split.chunks * 4 + wave) * (NDT * 4 * 64) + dt * (4 * 64) + lane;
+  const float m = md[(chunks - 1) * 256];
+  float d = 0.f;
+  float4 O[4];
+#pragma unroll
+  for (int g = 0; g < 4; g++) O[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+  for (int c = 0; c < chunks; c++) {
+    const float f = __builtin_amdgcn_exp2f(md[c * 256] - m);
+    d += md[c * 256 + 128] * f;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const float4 t = so[(size_t)c * (4 * NDT * 4 * 64) + g * 64];
+      O[g].x += t.x * f; O[g].y += t.y * f; O[g].z += t.z * f; O[g].w += t.w * f;
+    }
+  }
+  const float inv = __builtin_amdgcn_rcpf(d);
+  const int q_row = qb * 128 + wave * 32 + r;
+  if (q_row >= p.N) return;
+  uint16_t *const out = (uint16_t *)p.out + (size_t)batch * p.os.sb + (size_t)head * p.os.sh + (size_t)q_row * p.os.sn;
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    const int d0 = 32 * dt + 8 * g + 4 * hh;
+    float4 sc = make_float4(1.f, 1.f, 1.f, 1.f);
+    if constexpr (!PV16) sc = *(const float4 *)(p.v_scale + (size_t)bhk * D + d0);
+    const uint16_t o0 = f32_to_elem<ODT>(O[g].x * inv * sc.x), o1 = f32_to_elem<ODT>(O[g].y * inv * sc.y);
+    const uint16_t o2 = f32_to_elem<ODT>(O[g].z * inv * sc.z), o3 = f32_to_elem<ODT>(O[g].w * inv * sc.w);
+    *(uint2 *)(out + d0) = make_uint2((uint32_t)o0 | ((uint32_t)o1 << 16), (uint32_t)o2 | ((uint32_t)o3 << 16));
+  }
+}
+
+// Few long rows: each over several workgroups (rows_in_chunks has the line).  One workgroup per row leaves CUs idle, ends when the longest
+// row ends, and has its groups of wavefronts meet at a barrier for every round of blocks; what stands against cutting the row is that P is
+// rounded against the running maximum.  Scores and maxima alone need no order and are a third of the work: a launch in front takes the maxima of
+// the chunks, after which the chunks are independent.  One head N17776 D64 with every block kept: 133 us in groups; 24 + 78 + 11 in chunks.
+template <int D, int ODT, bool PV16>
+static void launch_split(AttnParams &p, hipStream_t st) {
+  const int per_xcd = (p.total_wg + 7) / 8;
+  p.split.rows = p.total_wg;
+  p.by_chunks = FastDiv::of(per_xcd);
+  row_maxima_kernel<D><<<8 * per_xcd * (p.split.chunks - 1), 256, 0, st>>>(p);
+  block_sparse_attn_kernel<D, ODT, PV16, 0, 1, 0, true><<<8 * per_xcd * p.split.chunks, 256, 0, st>>>(p);
+  combine_chunks_kernel<D, ODT, PV16><<<8 * per_xcd * (D / 32), 256, 0, st>>>(p);
 }
 
 template <int SEL, int FQ>
@@ -1168,11 +1467,21 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
   p.by_nq = FastDiv::of(p.nq); p.by_rest = FastDiv::of(p.nq > p.rows_first ? p.nq - p.rows_first : 1);
   p.by_H = FastDiv::of(p.H); p.by_group = FastDiv::of(p.H / p.Hkv);
+  if constexpr (SEL == 0 && FQ == 0) {
+    if (p.split.chunks > 1) {
+      p.queue = nullptr;
+#define SPG_SPLIT(D_, PV16_) { if (out_dtype == 0) launch_split<D_, 0, PV16_>(p, st); else launch_split<D_, 1, PV16_>(p, st); }
+      if (p.v_scale != nullptr) { if (D == 64) SPG_SPLIT(64, false) else SPG_SPLIT(128, false) }
+      else { if (D == 64) SPG_SPLIT(64, true) else SPG_SPLIT(128, true) }
+#undef SPG_SPLIT
+      return hipGetLastError();
+    }
+  }
   const int n_groups = FQ == 0 && p.pv_mode == 1 && p.pv_count == nullptr ? attn_groups(p.total_wg, p.nk, D, p.v_scale == nullptr) : 1;
 #define SPG_ATTN(D_, PV16_, G_)                                                                             \
   {                                                                                                         \
-    if (out_dtype == 0) block_sparse_attn_kernel<D_, 0, PV16_, SEL, G_, FQ><<<grid, 256 * G_, 0, st>>>(p);  \
-    else block_sparse_attn_kernel<D_, 1, PV16_, SEL, G_, FQ><<<grid, 256 * G_, 0, st>>>(p);                 \
+    if (out_dtype == 0) block_sparse_attn_kernel<D_, 0, PV16_, SEL, G_, FQ, false><<<grid, 256 * G_, 0, st>>>(p);  \
+    else block_sparse_attn_kernel<D_, 1, PV16_, SEL, G_, FQ, false><<<grid, 256 * G_, 0, st>>>(p);                 \
   }
 #define SPG_ATTN_G(D_, PV16_)                                                                               \
   {                                                                                                         \
@@ -1195,9 +1504,11 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
                                       int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel, const RawQ *q,
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
-                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue, hipStream_t st) {
+                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue, const RowSplit *split,
+                                      hipStream_t st) {
   AttnParams p = {};
   p.queue = queue;
+  if (split != nullptr) p.split = *split;
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.out = out; p.os = os; p.lut = lut; p.valid = valid; p.pvthr = pvthreshd;
   p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.pv_count = pv_count;
   p.B = B; p.H = H; p.Hkv = Hkv; p.N = N; p.Nk = Nk;
@@ -1219,7 +1530,7 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st) {
   return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, nullptr, nullptr, Hyper{pvthreshd, 0.f}, q_scale, k_scale,
-                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, false, nullptr, st);
+                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, false, nullptr, nullptr, st);
 }
 
 }  // namespace spg

@@ -1,5 +1,5 @@
 // The whole operator behind one call: K mean, mask prediction + INT8 quantisation, V quantisation, block-sparse
-// attention, as two to five launches on workspace the caller hands over.
+// attention, as two to seven launches on workspace the caller hands over.
 //
 // Short sequences are bound by the length of the launch chain and by kernels that cannot fill the chip, so stages that do
 // not depend on each other share a launch; which stage a workgroup belongs to follows from its number:
@@ -11,7 +11,7 @@
 //            of the next launch to add them up for itself)
 //   back     pooling + quantisation of K | V -> e4m3 tiles and scales (FP16 PV, many blocks: V^T tiles)
 //   select   block_select_* of maskpred.hip (rows of more than 128 blocks; shorter ones are selected inside the next launch)
-//   attn     block_sparse_attn_kernel
+//   attn     block_sparse_attn_kernel (few long rows: in chunks, with a launch in front for their maxima and one behind)
 // Every body is the one the stage-by-stage entry points launch (stage_bodies.h): results are the same bits.
 // The extern "C" entry points and their argument checks are in capi.hip, the workspace layout in forward_plan.h.
 // Compile with -ffp-contract=off.
@@ -372,12 +372,14 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   else if (!mask_in_front)
     e = launch_map_to_lut(a->mask, a->mask_kind, lut, valid, a->B, a->H, nq, nk, st);
   if (e != hipSuccess) return e;
+  RowSplit split = {};
+  if (rows_in_chunks(a)) split = row_split(chunk_plan(a->B, a->H, a->N, a->N_kv, a->D), ws + l.split);
   const RawQ raw = {f.q, qs, simthr};
   return launch_block_sparse_attn_h(f.q8, b.k8, b.v8, a->out, os, a->qk_dtype, lut, valid, sel_in_attn ? &sel : nullptr, front_q ? nullptr : &raw,
                                     Hyper{a->pvthreshd, a->pvthreshd_value},
                                     f.q_scale, b.k_scale, a->pv_f16 ? nullptr : b.v_scale, a->B, a->H, a->Hkv, a->N, a->N_kv, a->D,
                                     a->sm_scale, a->kernel_causal ? 1 : 0, a->qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0,
-                                    SPG_PV_PER_BLOCK, nullptr, pool && a->is_causal, f.queue, st);
+                                    SPG_PV_PER_BLOCK, nullptr, pool && a->is_causal, f.queue, &split, st);
 }
 
 }  // namespace spg

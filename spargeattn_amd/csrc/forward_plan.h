@@ -123,8 +123,62 @@ inline bool q_overwritten(const spg_attn_args *a, const Strides &qs, const Strid
   return q < out + bytes(os) && out < q + bytes(qs);
 }
 
+
+inline int split_env(const char *n, int d) { const char *e = getenv(n); return e ? atoi(e) : d; }
+// ---- rows in chunks (RowSplit) --------------------------------------------------------------------------------------
+// Blocks of a chunk, and where the scratch for it lies.  About two rounds of workgroups if every block is kept (D = 64 fits four to a CU, D =
+// 128 three), so that one round or more is left with half of them.  us per call with 512 / 768 / 1024 / 1536 / 2048 workgroups in all: one head
+// N17776 D64 top-k 0.5 117 / 109 / 98 / 97 / 105, 2 x 10000 80 / 79 / 81 / 75 / 83; D128 160 / 140 / 133 / 140 / 143, 2 x 10000 106 / 101 / 96 / 103 / 108, with
+// every block kept 186 / 194 / 191 / 194 / 197.  (8 and 24 blocks instead of 16 at least: 8300 x 8300 D64 55.5 / 53.4 / 57.6, D128 68.5 / 67.7 / 74.5.)
+struct ChunkPlan {
+  int chunks, per;                  // 1, 0: a row has one workgroup, whatever it keeps
+  size_t first, maxima, md, o, bytes;
+};
+inline ChunkPlan chunk_plan(int B, int H, int N, int N_kv, int D) {
+  ChunkPlan c = {1, 0, 0, 0, 0, 0, 0};
+  const long long rows = (long long)B * H * ((N + 127) / 128), nk = (N_kv + 63) / 64;
+  if (rows > 256 || nk <= 36 || nk > 32768) return c;
+  const long long wgs = D == 64 ? 1536 : 1024, spread = (rows * nk + wgs - 1) / wgs, most = (nk + 63) / 64;   // (64 chunks: those of a row are added up one by one)
+  c.per = (int)(spread > most ? spread : most);
+  if (c.per < 16) c.per = 16;
+  c.chunks = (int)((nk + c.per - 1) / c.per);
+  auto take = [&](size_t bytes) { const size_t r = c.bytes; c.bytes += (bytes + 255) / 256 * 256; return r; };
+  const size_t all = (size_t)rows * c.chunks;
+  c.first = take(all * 4);
+  c.maxima = take(all * 128 * 4);
+  c.md = take(all * 256 * 4);
+  c.o = take(all * 128 * D * 4);
+  return c;
+}
+inline RowSplit row_split(const ChunkPlan &c, void *scratch) {
+  unsigned char *const at = (unsigned char *)scratch;
+  return {c.chunks, c.per, 0, (int *)(at + c.first), (float *)(at + c.maxima), (float *)(at + c.md), (float *)(at + c.o)};
+}
+// Whether they pay: with a workgroup per row the call takes as long as its longest row, 0.45 us per block at D = 64 and 0.6 at D = 128 (0.76
+// with FP16 PV); in chunks all blocks count, 2.05, 3.25 and 4.2 ns each, and the two launches more take 16 us.  A row is expected to keep the
+// blocks that top-k names (share; below 0: nothing on the host says, and half is taken); a partial last Q block is never similar and keeps all.
+// us per call, workgroup per row / chunks, 8 to 176 whole rows, nk, top-k: D64 8 x 132 0.2 46.5 / 48.9, 0.35 56.0 / 51.9, 1.0 95.8 / 54.4; 64 x 132 0.35 59.9
+// / 57.8, 64 x 288 0.2 80.5 / 72.1, 1.0 183 / 111; 128 x 192 0.35 76.2 / 74.6, 0.5 90.4 / 82.0, 128 x 512 0.2 115.5 / 113.5, 1.0 303 / 218; 176 x 288 0.35 100 / 105,
+// 1.0 182 / 175; 224 x 512 1.0 321 / 332.  D128 8 x 132 0.2 58.5 / 63.6, 0.35 72.3 / 66.8; 64 x 512 0.1 128.7 / 133.4, 0.5 251 / 169; 128 x 288 0.35 134 /
+// 132, 0.5 161 / 143; 176 x 512 1.0 405 / 423; FP16 PV 64 x 288 0.2 107.5 / 95.3, 160 x 288 0.5 184 / 175, 256 x 288 0.5 198 / 217.  With a partial last
+// block: N24000, 188 rows, top-k 0.5 D64 207 / 145, D128 265 / 190, causal 207 / 140; N28000 D128 310 / 231; one head N17776 CDF 171 / 136.
+inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, int selection, float share, bool causal) {
+  const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
+  if (chunk_plan(B, H, N, N_kv, D).chunks == 1 || (selection != SPG_SELECT_MASK && nk <= SPG_SELECT_IN_ATTN_NK)) return false;
+  share = share < 0.f ? 0.5f : share < 1.f ? share : 1.f;
+  const float kept = share * nk;
+  const bool partial = N % 128 != 0 && selection != SPG_SELECT_MASK;
+  const float longest = partial ? (float)nk : kept;
+  const float all = (float)(B * H) * (nq * kept * (causal ? 1.f - 0.5f * share : 1.f) + (partial ? nk - kept : 0.f));
+  return longest - all / 180.f > 36.f;
+}
+inline bool rows_in_chunks(const spg_attn_args *a) {
+  const float share = a->selection == SPG_SELECT_TOPK && a->level == nullptr ? (a->level_value > 0.f ? a->level_value : 0.f) : -1.f;
+  return rows_in_chunks(a->B, a->H, a->N, a->N_kv, a->D, a->selection, share, a->is_causal != 0);
+}
+
 struct Layout {
-  size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, queue, total;
+  size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, queue, split, total;
 };
 inline Layout layout_for(const spg_attn_args *a) {
   Layout l;
@@ -153,6 +207,7 @@ inline Layout layout_for(const spg_attn_args *a) {
   l.lut = take(bh * nq * nk * 4);
   l.valid = take(bh * nq * 4);
   l.queue = take(8 * sizeof(int));
+  l.split = take(!pool || nk > SPG_SELECT_IN_ATTN_NK ? chunk_plan(a->B, a->H, a->N, a->N_kv, a->D).bytes : 0);
   l.total = at;
   return l;
 }

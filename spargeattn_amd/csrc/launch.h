@@ -92,6 +92,17 @@ inline int attn_groups(int rows, int nk, int D, bool pv_f16) {
   if (nk <= 64) return 2;
   return D == 64 ? 4 : !pv_f16 && nk <= 32768 ? 3 : 2;
 }
+// A row's blocks over several workgroups, and scratch for what these leave behind.
+struct RowSplit {
+  int chunks;                       // workgroups of a row at most; 0 or 1: one
+  int per;                          // blocks of a workgroup at most
+  int rows;                         // (set at the launch)
+  int *first;                       // [rows][chunks]            first block of a chunk
+  float *maxima;                    // [rows][chunks][128]       largest score of a chunk
+  float *md;                        // [rows][chunks][2][128]    running maximum at its end, denominator
+  float *o;                         // [rows][chunks][128 x D]   sums, as the lanes hold them
+};
+// split: with sel == NULL, q == NULL, pv_count == NULL and the per-block PV threshold only.
 // sel == NULL: blocks come from lut / valid; otherwise they are selected in place and lut / valid are not read.
 // q == NULL: Q comes as q8 / q_scale (and pooled in sel); otherwise from the caller's tensor, and those are not read.
 // queue: 8 device ints, zero when the kernel starts, for handing out rows across the XCDs, or NULL for a fixed share each.
@@ -101,7 +112,7 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
                                       int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue,
-                                      hipStream_t st);
+                                      const RowSplit *split, hipStream_t st);
 void launch_fp8_pack_selftest(const float *x, uint8_t *codes, int n, int saturate, hipStream_t st);
 
 hipError_t launch_dense_attn_f16(const void *q, const void *k, const void *v, void *out, int B, int H, int N, int D,

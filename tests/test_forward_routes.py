@@ -20,8 +20,8 @@ def routes(tmp_path_factory):
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-4000:]
 
-    def route(B=1, H=1, Hkv=0, N=128, Nk=0, D=128, selection=TOPK, pv_f16=0, sim=-0.1):
-        line = f"{B} {H} {Hkv or H} {N} {Nk or N} {D} {selection} {pv_f16} {sim}\n"
+    def route(B=1, H=1, Hkv=0, N=128, Nk=0, D=128, selection=TOPK, pv_f16=0, sim=-0.1, level=0.5, causal=0):
+        line = f"{B} {H} {Hkv or H} {N} {Nk or N} {D} {selection} {pv_f16} {sim} {level} {causal}\n"
         out = subprocess.run([exe], input=line, capture_output=True, text=True, timeout=60)
         assert out.returncode == 0
         return [int(x) for x in out.stdout.split()]
@@ -69,3 +69,27 @@ def test_groups_follow_the_row_not_the_number_of_rows(routes, H, N, D, pv_f16, l
 
 def test_grids_beyond_one_row_per_cu_have_no_groups(routes):
     assert [routes(H=2, N=n, Nk=20000, D=64)[3] for n in (16384, 16385)] == [4, 1]
+
+
+# rows x nk, share of the blocks -> in chunks.  Whole rows: the longest is what top-k keeps; a partial last Q block keeps everything.
+@pytest.mark.parametrize("kw,chunks", [
+    (dict(H=8, N=128, Nk=64 * 132, level=0.2), 0), (dict(H=8, N=128, Nk=64 * 132, level=0.35), 1), (dict(H=8, N=1024, Nk=64 * 132, level=0.5), 1),
+    (dict(H=8, N=2048, Nk=64 * 288, level=0.2), 0), (dict(H=8, N=2048, Nk=64 * 288, level=0.5), 1), (dict(H=8, N=22 * 128, Nk=64 * 512, level=1.0), 0),
+    (dict(H=8, N=32 * 128, Nk=64 * 512, level=0.5), 0), (dict(N=17776, D=64, selection=CDF), 1), (dict(N=17776, level=0.5), 1), (dict(N=24000, causal=1), 1),
+    (dict(N=64 * 257, Nk=64 * 600, level=0.3), 1), (dict(N=8192 * 4, level=0.5), 0), (dict(N=128 * 256 + 1, level=0.5), 0),
+    (dict(H=8, N=128, Nk=64 * 128, level=1.0), 0), (dict(H=8, N=128, Nk=64 * 128, selection=MASK), 1), (dict(H=2, N=128, Nk=64 * 36, selection=MASK), 0)])
+def test_few_long_rows_go_over_several_workgroups(routes, kw, chunks):
+    assert routes(**kw)[7] == chunks
+
+
+def test_workspace_does_not_depend_on_the_level(routes):
+    for kw in (dict(H=8, N=128, Nk=64 * 132), dict(N=17776, D=64), dict(H=8, N=2048, Nk=64 * 288, pv_f16=1)):
+        assert len({routes(level=level, **kw)[5] for level in (0.05, 0.5, 1.0)}) == 1
+
+
+@pytest.mark.parametrize("D,most", [(64, 1536), (128, 1024)])
+def test_chunks_of_a_row_are_bounded(routes, D, most):
+    for H, N, nk in ((1, 1, 8192), (1, 128, 37), (8, 128, 2048), (1, 17776, 278), (2, 16384, 8192)):
+        rows, n = H * -(-N // 128), routes(H=H, N=N, Nk=64 * nk, D=D, selection=MASK)[6]
+        assert 1 < n <= 64 and n <= -(-nk // 16) and rows * (n - 1) <= most
+    assert routes(H=2, N=16385, Nk=64 * 512, D=D)[6] == 1
