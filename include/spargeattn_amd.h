@@ -209,11 +209,15 @@ typedef struct spg_attn_args {
   const void *q, *k, *v, *mask;       /* q (B,H,N,D), k and v (B,Hkv,N_kv,D); mask (B,H,nq,nk) for SPG_SELECT_MASK */
   void *out;
   const int64_t *q_strides, *k_strides, *v_strides, *out_strides;
-  int32_t *valid_block_num;           /* (B,H,nq), or NULL if the caller has no use for the counts */
+  int32_t *valid_block_num;           /* (B,H,nq), or NULL if the caller has no use for the counts.  With a selection they are written once
+                                         and not read: pinned host memory will do, see spg_wait_counts */
   void *workspace;
   uint64_t workspace_bytes;
 } spg_attn_args;
 
+/* Host only.  Waits until none of n counts is negative any more and returns their sum, or -1 after `seconds`: for counts in pinned host
+ * memory, filled with -1 before the call.  They arrive with the selection, before the attention has run. */
+int64_t spg_wait_counts(const int32_t *counts, int64_t n, double seconds);
 size_t spg_sparse_attn_workspace_bytes(const spg_attn_args *args);
 int spg_sparse_attn(const spg_attn_args *args, void *stream);
 

@@ -43,6 +43,7 @@ SIGNATURES = {
     "spg_block_sparse_attn_f16v": (_i, [_vp] * 5 + [_i] + [_vp] * 5 + [_i] * 6 + [_f, _i, _i, _i, _vp, _vp]),
     "spg_block_sparse_attn_chunks_bytes": (_sz, [_i] * 6 + [_f, _i]),
     "spg_block_sparse_attn_chunks": (_i, [_vp] * 5 + [_i] + [_vp] * 6 + [_i] * 6 + [_f, _i, _i, _vp, _c.c_uint64, _vp]),
+    "spg_wait_counts": (_c.c_int64, [_vp, _c.c_int64, _c.c_double]),
     "spg_sparse_attn_workspace_bytes": (_sz, [_vp]),
     "spg_sparse_attn": (_i, [_vp, _vp]),
     "spg_dense_attn_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _f, _i, _vp]),
@@ -419,7 +420,8 @@ class ForwardPlan:
         self.device_index = q.device.index
 
     def run(self, q, k, v, out, mask, level, simthreshd1, pvthreshd, return_valid=False):
-        """level / simthreshd1 / pvthreshd: a Python number, or a contiguous (H,) float32 tensor on the device."""
+        """level / simthreshd1 / pvthreshd: a Python number, or a contiguous (H,) float32 tensor on the device.
+        return_valid: returns how many blocks are kept in all."""
         if _torch() is not None:
             t = self.template
             par = [(x, 0.0) if isinstance(x, torch.Tensor) else (None, float(x)) for x in (level, simthreshd1, pvthreshd)]
@@ -427,13 +429,20 @@ class ForwardPlan:
             valid = _ops.sparse_attn(q, k, v, out, mask, *par[0], *par[1], *par[2], [t.B, t.H, t.Hkv, t.N, t.N_kv, t.D],
                                      list(s[0]), list(s[1]), list(s[2]), list(s[3]), t.selection, bool(t.pv_f16),
                                      bool(t.is_causal), bool(t.attention_sink), bool(t.kernel_causal), t.qk_quant_gran, t.sm_scale)
-            return valid if return_valid else None
+            return int(valid.cpu().sum()) if return_valid else None
         a = AttnArgs.from_buffer_copy(self.template)
         workspace = torch.empty(self.workspace_bytes, dtype=torch.uint8, device=self.device)
         a.q, a.k, a.v, a.out, a.workspace = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), workspace.data_ptr()
         valid = None
+        # The counts of a selection are stored straight to pinned host memory, where they are seen before the attention has run: no
+        # copy and no wait for it (one head of 17776, D = 64, 167.6 us per call with both, 136.7 so).  A caller's mask is read by the attention through its
+        # counts, and a capture refuses the copy.
+        early = return_valid and mask is None and not torch.cuda.is_current_stream_capturing()
         if return_valid:
-            valid = torch.empty(self.valid_shape, dtype=torch.int32, device=self.device)
+            if early:
+                valid = torch.full(self.valid_shape, -1, dtype=torch.int32, pin_memory=True)
+            else:
+                valid = torch.empty(self.valid_shape, dtype=torch.int32, device=self.device)
             a.valid_block_num = valid.data_ptr()
         if mask is not None:
             a.mask = mask.data_ptr()
@@ -453,7 +462,14 @@ class ForwardPlan:
         rc = self._lib.spg_sparse_attn(ctypes.addressof(a), torch._C._cuda_getCurrentRawStream(self.device_index))
         if rc != SPG_OK:
             _check(rc)
-        return valid
+        if not return_valid:
+            return None
+        if early:
+            kept = self._lib.spg_wait_counts(valid.data_ptr(), valid.numel(), 2e-3)
+            if kept >= 0:
+                return kept
+            torch.cuda.current_stream(self.device).synchronize()
+        return int(valid.cpu().sum())
 
 
 def v_tiles_f16_swizzled(v, stream=None):

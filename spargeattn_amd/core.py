@@ -238,14 +238,14 @@ def _run(q, k, v, mask, selection, level, simthreshd1, pvthreshd, is_causal, att
         simthreshd1 = _hyper(simthreshd1, H, device)
     pvthreshd = _hyper(pvthreshd, H, device)
     o = torch.empty_strided(plan.out.shape, plan.out.stride(), dtype=q.dtype, device=device)
-    valid = plan.run(q, k, v, o, mask, level, simthreshd1, pvthreshd, return_sparsity)
+    kept = plan.run(q, k, v, o, mask, level, simthreshd1, pvthreshd, return_sparsity)
     if not return_sparsity:
         return o
     B, H, nq = plan.valid_shape
     cols = (plan.nk + 2) // 2 if causal_denominator else plan.nk
     # bit for bit what _finish computes on the GPU, where a division by a number is a product with its binary32 reciprocal
     per_block = torch.tensor(cols * nq * B * H, dtype=torch.float32).reciprocal()
-    qk_sparsity = 1 - valid.cpu().sum().float() * per_block
+    qk_sparsity = 1 - torch.tensor(kept).float() * per_block
     return o, qk_sparsity.item()
 
 

@@ -4,6 +4,7 @@
 #include "capi_checks.h"
 #include "forward_plan.h"
 
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 
@@ -242,6 +243,17 @@ static int check_forward(const char *fn, const spg_attn_args *a) {
     return fail(SPG_ERR_UNSUPPORTED, "%s: nk = %d exceeds the supported maximum %d", fn, nk, spg::block_select_max_nk());
   }
   return SPG_OK;
+}
+
+int64_t spg_wait_counts(const int32_t *counts, int64_t n, double seconds) {
+  if (counts == nullptr || n < 0) return -1;
+  const auto start = std::chrono::steady_clock::now();
+  int64_t sum = 0, i = 0;
+  for (unsigned spin = 0;; spin++) {
+    for (int v; i < n && (v = __atomic_load_n(counts + i, __ATOMIC_ACQUIRE)) >= 0; i++) sum += v;
+    if (i == n) return sum;
+    if (spin % 64 == 63 && std::chrono::duration<double>(std::chrono::steady_clock::now() - start).count() > seconds) return -1;
+  }
 }
 
 size_t spg_sparse_attn_workspace_bytes(const spg_attn_args *args) {

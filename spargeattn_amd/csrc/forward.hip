@@ -303,7 +303,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
   const bool pool = a->selection != SPG_SELECT_MASK;
   const Hyper simthr = {a->simthreshd1, a->simthreshd1_value};
   int32_t *const lut = (int32_t *)(ws + l.lut);
-  int32_t *const valid = a->valid_block_num != nullptr ? a->valid_block_num : (int32_t *)(ws + l.valid);
+  int32_t *const valid = !pool && a->valid_block_num != nullptr ? a->valid_block_num : (int32_t *)(ws + l.valid);
   // Fewer than two workgroups of 256 threads per CU leave the stages bound by the length of one thread's work (9.8 and
   // 13.0 us for the two launches at B2 H3 N1025 D128 with a similarity threshold): twice the threads take half of it.
   const bool in_one = one_launch(a), sel_in_attn = pool && nk <= SPG_SELECT_IN_ATTN_NK, front_q = q_in_front(a) || q_overwritten(a, qs, os);
@@ -368,7 +368,7 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
            a->attention_sink, a->valid_block_num};
   else if (pool)
     e = launch_block_select_h(f.pool_q, f.sim_q, b.pool_k, b.sim_k, a->selection == SPG_SELECT_TOPK, Hyper{a->level, a->level_value},
-                              a->is_causal, a->attention_sink, lut, valid, nullptr, a->B, a->H, a->Hkv, nq, nk, a->D, a->qk_dtype, st);
+                              a->is_causal, a->attention_sink, lut, valid, a->valid_block_num, nullptr, a->B, a->H, a->Hkv, nq, nk, a->D, a->qk_dtype, st);
   else if (!mask_in_front)
     e = launch_map_to_lut(a->mask, a->mask_kind, lut, valid, a->B, a->H, nq, nk, st);
   if (e != hipSuccess) return e;

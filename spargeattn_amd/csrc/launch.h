@@ -36,9 +36,9 @@ int block_select_max_nk();
 hipError_t launch_block_select(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, const float *topk,
                                const float *cdf, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
                                int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st);
-// the same with the level (top-k fraction or CDF threshold) as a Hyper
+// the same with the level (top-k fraction or CDF threshold) as a Hyper; valid_out: the counts once more, where the host can see them, or NULL
 hipError_t launch_block_select_h(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, bool by_topk,
-                                 Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
+                                 Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, int32_t *valid_out, uint8_t *bmap,
                                  int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st);
 void launch_div_selftest(unsigned long long *counts, int n_div, uint32_t seed, hipStream_t st);
 hipError_t launch_map_to_lut(const void *mask, int kind, int32_t *lut, int32_t *valid, int B, int H, int nq, int nk,

@@ -105,7 +105,7 @@ template <int D, int DT, int R>
 __global__ __launch_bounds__(256) void block_select_kernel(
     const uint16_t *__restrict__ pool_q, const uint8_t *__restrict__ sim_q, const uint16_t *__restrict__ pool_k,
     const uint8_t *__restrict__ sim_k, const bool by_topk, const Hyper level, int is_causal,
-    int sink, int32_t *__restrict__ lut, int32_t *__restrict__ valid, uint8_t *__restrict__ bmap, int H, int Hkv, int nq,
+    int sink, int32_t *__restrict__ lut, int32_t *__restrict__ valid, int32_t *__restrict__ valid_out, uint8_t *__restrict__ bmap, int H, int Hkv, int nq,
     int nk, int nkp) {
   extern __shared__ __align__(16) unsigned char smem[];
   double *s_pq = (double *)smem;                                   // [R][D]
@@ -268,6 +268,7 @@ __global__ __launch_bounds__(256) void block_select_kernel(
       for (int j = tid; j < nk; j += 256) bmap[row_off + j] = flag(j) ? 1 : 0;
     emit_lut<256>(flag, nk, nkp, s_idx, s_tmp, lut + row_off, valid + (size_t)bh * nq + i);
     __syncthreads();                                // the work area is reused by the next row
+    if (valid_out != nullptr && tid == 0) valid_out[(size_t)bh * nq + i] = valid[(size_t)bh * nq + i];
   }
 }
 
@@ -285,7 +286,7 @@ template <int D, int DT, int NW, int EPL, bool DUAL, int R>
 __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_select_wave_kernel(
     const uint16_t *__restrict__ pool_q, const uint8_t *__restrict__ sim_q, const uint16_t *__restrict__ pool_k,
     const uint8_t *__restrict__ sim_k, const bool by_topk, const Hyper level, int is_causal,
-    int sink, int32_t *__restrict__ lut, int32_t *__restrict__ valid, uint8_t *__restrict__ bmap, int H, int Hkv, int nq,
+    int sink, int32_t *__restrict__ lut, int32_t *__restrict__ valid, int32_t *__restrict__ valid_out, uint8_t *__restrict__ bmap, int H, int Hkv, int nq,
     int nk) {
   // R rows per workgroup; phase 1 computes 16 x 16 score tiles on the matrix unit, of which R = 8 uses the first 8 rows
   static_assert(R == 16 || R == 8, "rows per workgroup");
@@ -549,7 +550,10 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
         lut[row_off + pidx] = v;
       }
     }
-    if (lane == 0) valid[(size_t)bh * nq + i] = base;
+    if (lane == 0) {
+      valid[(size_t)bh * nq + i] = base;
+      if (valid_out != nullptr) valid_out[(size_t)bh * nq + i] = base;
+    }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();                  // the index list is reused by this wavefront's next row
   }
@@ -699,7 +703,7 @@ void launch_div_selftest(unsigned long long *counts, int n_div, uint32_t seed, h
 
 template <int D, int DT, int R>
 static hipError_t launch_bs3(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, bool by_topk,
-                             Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap, int B,
+                             Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, int32_t *valid_out, uint8_t *bmap, int B,
                              int H, int Hkv, int nq, int nk, int nkp, hipStream_t st) {
   const size_t lds = (size_t)R * D * 8 + (size_t)R * nkp * 4 + 12 * (size_t)nkp;
   auto kern = block_select_kernel<D, DT, R>;
@@ -708,13 +712,13 @@ static hipError_t launch_bs3(const void *pq, const uint8_t *sq, const void *pk, 
     if (e != hipSuccess) return e;
   }
   kern<<<dim3((nq + R - 1) / R, B * H), 256, lds, st>>>((const uint16_t *)pq, sq, (const uint16_t *)pk, sk, by_topk, level,
-                                                        causal, sink, lut, valid, bmap, H, Hkv, nq, nk, nkp);
+                                                        causal, sink, lut, valid, valid_out, bmap, H, Hkv, nq, nk, nkp);
   return hipSuccess;
 }
 
 template <int D, int DT>
 static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, bool by_topk,
-                             Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap, int B,
+                             Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, int32_t *valid_out, uint8_t *bmap, int B,
                              int H, int Hkv, int nq, int nk, hipStream_t st) {
   const int nkp = next_pow2_ge(nk, 256);
   if (nkp <= 2048) {
@@ -728,7 +732,7 @@ static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, 
         if (e != hipSuccess) return e;                                                                          \
       }                                                                                                         \
       kern<<<dim3((nq + R_ - 1) / R_, B * H), 64 * NW_, lds, st>>>((const uint16_t *)pq, sq, (const uint16_t *)pk, sk, by_topk, \
-                                                               level, causal, sink, lut, valid, bmap, H, Hkv, nq, nk); \
+                                                               level, causal, sink, lut, valid, valid_out, bmap, H, Hkv, nq, nk); \
       return hipSuccess;                                                                                        \
     }
     // Eight rows instead of sixteen per workgroup, one per wavefront, where sixteen leave a CU with little more than one
@@ -743,17 +747,17 @@ static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, 
 #undef SPG_BSW
   }
   // rows per workgroup: reuse of the pooled-K reads against LDS footprint (scores are R*nkp floats)
-  if (nkp <= 1024) return launch_bs3<D, DT, 8>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
-  if (nkp <= 4096) return launch_bs3<D, DT, 4>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
+  if (nkp <= 1024) return launch_bs3<D, DT, 8>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, valid_out, bmap, B, H, Hkv, nq, nk, nkp, st);
+  if (nkp <= 4096) return launch_bs3<D, DT, 4>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, valid_out, bmap, B, H, Hkv, nq, nk, nkp, st);
   // nkp = 8192: one row per workgroup (D*8 + 16*nkp = 129 KiB; two rows would need 162 KiB, more than the 160 KiB a
   // workgroup can have)
-  return launch_bs3<D, DT, 1>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, nkp, st);
+  return launch_bs3<D, DT, 1>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, valid_out, bmap, B, H, Hkv, nq, nk, nkp, st);
 }
 
 hipError_t launch_block_select_h(const void *pq, const uint8_t *sq, const void *pk, const uint8_t *sk, bool by_topk,
-                                 Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
+                                 Hyper level, int causal, int sink, int32_t *lut, int32_t *valid, int32_t *valid_out, uint8_t *bmap,
                                  int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st) {
-#define SPG_BS(D_, DT_) return launch_bs2<D_, DT_>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, bmap, B, H, Hkv, nq, nk, st)
+#define SPG_BS(D_, DT_) return launch_bs2<D_, DT_>(pq, sq, pk, sk, by_topk, level, causal, sink, lut, valid, valid_out, bmap, B, H, Hkv, nq, nk, st)
   if (D == 64) { if (dtype == 0) SPG_BS(64, 0); else SPG_BS(64, 1); }
   else         { if (dtype == 0) SPG_BS(128, 0); else SPG_BS(128, 1); }
 #undef SPG_BS
@@ -763,7 +767,7 @@ hipError_t launch_block_select(const void *pq, const uint8_t *sq, const void *pk
                                const float *cdf, int causal, int sink, int32_t *lut, int32_t *valid, uint8_t *bmap,
                                int B, int H, int Hkv, int nq, int nk, int D, int dtype, hipStream_t st) {
   return launch_block_select_h(pq, sq, pk, sk, topk != nullptr, Hyper{topk != nullptr ? topk : cdf, 0.f}, causal, sink, lut, valid,
-                               bmap, B, H, Hkv, nq, nk, D, dtype, st);
+                               nullptr, bmap, B, H, Hkv, nq, nk, D, dtype, st);
 }
 
 hipError_t launch_map_to_lut(const void *mask, int kind, int32_t *lut, int32_t *valid, int B, int H, int nq, int nk,
