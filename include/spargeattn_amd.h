@@ -171,20 +171,22 @@ int spg_block_sparse_attn_f16v(const int8_t *q8, const int8_t *k8, const void *v
                                int B, int H, int Hkv, int N, int N_kv, int D, float sm_scale, int is_causal,
                                int qk_quant_gran, int pv_threshold_mode, int32_t *pv_count, void *stream);
 
-/* ---- the two above with the blocks of a row spread over several workgroups: few long rows.
- * spg_block_sparse_attn_chunks_bytes says how much device scratch that takes, or 0 where the whole-operator call below gives every row one
- * workgroup: at most 256 Q blocks in all, and rows long enough to pay for two more launches.  selection as in spg_attn_args, share the
- * top-k fraction or a negative number if there is none, is_causal the selection's.
- * spg_block_sparse_attn_chunks: v and v_scale as for spg_block_sparse_attn, or, with v_scale == NULL, v as for
- * spg_block_sparse_attn_f16v; the PV threshold is per block.  The running maxima that P is rounded against and the skipped blocks are those of the
- * block-by-block walk; O and the denominator are summed chunk by chunk.  Results are those of the whole-operator call, bit for bit.
- * workspace 256-byte aligned. */
-size_t spg_block_sparse_attn_chunks_bytes(int B, int H, int N, int N_kv, int D, int selection, float share, int is_causal);
-int spg_block_sparse_attn_chunks(const int8_t *q8, const int8_t *k8, const void *v, void *out, const int64_t *out_strides,
-                                 int out_dtype, const int32_t *lut, const int32_t *valid_block_num, const float *pvthreshd,
-                                 const float *q_scale, const float *k_scale, const float *v_scale,
-                                 int B, int H, int Hkv, int N, int N_kv, int D, float sm_scale, int is_causal,
-                                 int qk_quant_gran, void *workspace, uint64_t workspace_bytes, void *stream);
+/* ---- the two above for few rows (up to 256 Q blocks in all), whose work is spread over several workgroups to a row.
+ * spg_few_rows_route says how the whole-operator call below takes such a call: every row in one workgroup (the functions above), by its
+ * queries (short rows), or by its blocks (long ones; *workspace_bytes of device scratch).  selection as in spg_attn_args, share the top-k
+ * fraction or a negative number if there is none, is_causal the selection's, pvthreshd the threshold if it is one number for all heads, else 0.
+ * spg_block_sparse_attn_few_rows: v and v_scale as for spg_block_sparse_attn, or, with v_scale == NULL, v as for spg_block_sparse_attn_f16v;
+ * the PV threshold is per block, and by queries it is taken to be 45 or more, at which it leaves every bit as it is.  The running maxima that
+ * P is rounded against and the skipped blocks are those of the block-by-block walk, O and the denominator are summed in another order.  Results are
+ * those of the whole-operator call, bit for bit.  workspace 256-byte aligned. */
+enum spg_rows { SPG_ROWS_ONE_WORKGROUP = 0, SPG_ROWS_BY_QUERIES = 1, SPG_ROWS_BY_BLOCKS = 2 };
+int spg_few_rows_route(int B, int H, int N, int N_kv, int D, int pv_f16, int selection, float share, int is_causal, float pvthreshd,
+                       uint64_t *workspace_bytes);
+int spg_block_sparse_attn_few_rows(const int8_t *q8, const int8_t *k8, const void *v, void *out, const int64_t *out_strides,
+                                   int out_dtype, const int32_t *lut, const int32_t *valid_block_num, const float *pvthreshd,
+                                   const float *q_scale, const float *k_scale, const float *v_scale,
+                                   int B, int H, int Hkv, int N, int N_kv, int D, float sm_scale, int is_causal,
+                                   int qk_quant_gran, int route, void *workspace, uint64_t workspace_bytes, void *stream);
 
 /* ---- the whole operator in one call (spas_sage2_attn_meansim[_topk]_cuda, block_sparse_sage2_attn_cuda and, with pv_f16,
  * spas_sage_attn_meansim[_topk]_cuda; spas_sage_attn/core.py:39-319) ---------------------------------------------------

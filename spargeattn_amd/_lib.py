@@ -41,8 +41,8 @@ SIGNATURES = {
     "spg_block_sparse_attn": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _vp, _vp]),
     "spg_v_tiles_f16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "spg_block_sparse_attn_f16v": (_i, [_vp] * 5 + [_i] + [_vp] * 5 + [_i] * 6 + [_f, _i, _i, _i, _vp, _vp]),
-    "spg_block_sparse_attn_chunks_bytes": (_sz, [_i] * 6 + [_f, _i]),
-    "spg_block_sparse_attn_chunks": (_i, [_vp] * 5 + [_i] + [_vp] * 6 + [_i] * 6 + [_f, _i, _i, _vp, _c.c_uint64, _vp]),
+    "spg_few_rows_route": (_i, [_i] * 7 + [_f, _i, _f, _vp]),
+    "spg_block_sparse_attn_few_rows": (_i, [_vp] * 5 + [_i] + [_vp] * 6 + [_i] * 6 + [_f, _i, _i, _i, _vp, _c.c_uint64, _vp]),
     "spg_wait_counts": (_c.c_int64, [_vp, _c.c_int64, _c.c_double]),
     "spg_sparse_attn_workspace_bytes": (_sz, [_vp]),
     "spg_sparse_attn": (_i, [_vp, _vp]),
@@ -62,6 +62,7 @@ class AttnArgs(_c.Structure):
 
 
 SELECT_TOPK, SELECT_CDF, SELECT_MASK = 0, 1, 2
+ROWS_ONE_WORKGROUP, ROWS_BY_QUERIES, ROWS_BY_BLOCKS = 0, 1, 2
 
 _lib = None
 _ops = None          # torch.ops.spargeattn_amd once the extension is loaded
@@ -342,19 +343,27 @@ def _check_attn_shapes(q8, k8, vt, lut, valid, q_scale, k_scale, v_scale=None, q
     return B, H, Hkv, N, Nk, D
 
 
-def _in_chunks(q8, k8, v, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, sm_scale, is_causal, qk_quant_gran, selected):
-    """Few long rows, as the whole-operator call takes them (spg_block_sparse_attn_chunks).  selected: (selection, top-k fraction or
-    None, causal) of the lists.  False where a row has one workgroup."""
+def few_rows_route(shape, Nk, pv_f16, selected):
+    """(route, scratch bytes) of spg_few_rows_route.  selected: (selection, top-k fraction or None, causal, PV threshold or None)."""
+    B, H, N, D = shape
+    selection, share, causal, pvthreshd = selected
+    size = ctypes.c_uint64(0)
+    # (a negative share means that nothing is known, so 0 stays 0)
+    route = load().spg_few_rows_route(B, H, N, Nk, D, int(pv_f16), selection, -1.0 if share is None else max(float(share), 0.0), int(bool(causal)),
+                                      0.0 if pvthreshd is None else float(pvthreshd), ctypes.addressof(size))
+    return route, size.value
+
+
+def _few_rows(q8, k8, v, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, sm_scale, is_causal, qk_quant_gran, selected):
+    """Few rows, as the whole-operator call takes them (spg_block_sparse_attn_few_rows).  False where a row has one workgroup."""
     (B, H, N, D), (Hkv, Nk) = q8.shape, k8.shape[1:3]
-    selection, share, causal = selected
-    # (0.0 stays 0.0: a negative share means that nothing is known)
-    size = load().spg_block_sparse_attn_chunks_bytes(B, H, N, Nk, D, selection, -1.0 if share is None else max(float(share), 0.0), int(bool(causal)))
-    if size == 0:
+    route, size = few_rows_route(q8.shape, Nk, v_scale is None, selected)
+    if route == ROWS_ONE_WORKGROUP:
         return False
-    workspace = torch.empty(size, dtype=torch.uint8, device=q8.device)
-    _check(load().spg_block_sparse_attn_chunks(_p(q8), _p(k8), _p(v), _p(out), _st(out), _dt(out), _p(lut), _p(valid), _p(pvthreshd), _p(q_scale),
-                                               _p(k_scale), _p(v_scale), B, H, Hkv, N, Nk, D, float(sm_scale), int(bool(is_causal)),
-                                               qk_quant_gran, _p(workspace), size, _stream()))
+    workspace = torch.empty(size, dtype=torch.uint8, device=q8.device) if size else None
+    _check(load().spg_block_sparse_attn_few_rows(_p(q8), _p(k8), _p(v), _p(out), _st(out), _dt(out), _p(lut), _p(valid), _p(pvthreshd), _p(q_scale),
+                                                 _p(k_scale), _p(v_scale), B, H, Hkv, N, Nk, D, float(sm_scale), int(bool(is_causal)),
+                                                 qk_quant_gran, route, _p(workspace), size, _stream()))
     return True
 
 
@@ -367,7 +376,7 @@ def block_sparse_attn(q8, k8, v8, out, lut, valid, pvthreshd, q_scale, k_scale, 
     if tuple(out.shape) != (B, H, N, D) or pvthreshd.numel() != H:
         raise RuntimeError("out must have q's shape and pvthreshd one entry per query head")
     if selected is not None and not return_pv_count and pv_mode == PV_PER_BLOCK and \
-            _in_chunks(q8, k8, v8, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, sm_scale, is_causal, qk_quant_gran, selected):
+            _few_rows(q8, k8, v8, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, sm_scale, is_causal, qk_quant_gran, selected):
         return None
     if _torch() is not None:
         pvc = _ops.block_sparse_attn(q8, k8, v8, out, lut, valid, pvthreshd, q_scale, k_scale, v_scale, float(sm_scale),
@@ -504,7 +513,7 @@ def block_sparse_attn_f16v(q8, k8, vt, out, lut, valid, pvthreshd, q_scale, k_sc
     if tuple(out.shape) != (B, H, N, D) or pvthreshd.numel() != H:
         raise RuntimeError("out must have q's shape and pvthreshd one entry per query head")
     if selected is not None and not return_pv_count and pv_mode == PV_PER_BLOCK and \
-            _in_chunks(q8, k8, vt, out, lut, valid, pvthreshd, q_scale, k_scale, None, sm_scale, is_causal, qk_quant_gran, selected):
+            _few_rows(q8, k8, vt, out, lut, valid, pvthreshd, q_scale, k_scale, None, sm_scale, is_causal, qk_quant_gran, selected):
         return None
     if _torch() is not None:
         pvc = _ops.block_sparse_attn_f16v(q8, k8, vt, out, lut, valid, pvthreshd, q_scale, k_scale, float(sm_scale),

@@ -114,13 +114,14 @@ def _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_deno
     return o
 
 
-def _selected(cdfthreshd, topk, is_causal):
-    """What _lib.block_sparse_attn wants to know of the selection: how many blocks a row may be expected to keep."""
-    if topk is None:
-        return _lib.SELECT_CDF, None, is_causal
-    # a number as _hyper takes it; per-head values stay on the device
-    known = type(topk) in (float, int) or (isinstance(topk, torch.Tensor) and topk.dim() == 0)
-    return _lib.SELECT_TOPK, float(topk) if known else None, is_causal
+def _number(value):
+    """A hyper-parameter that _hyper hands over as a number, or None: per-head values stay on the device."""
+    return float(value) if type(value) in (float, int) or (isinstance(value, torch.Tensor) and value.dim() == 0) else None
+
+
+def _selected(cdfthreshd, topk, is_causal, pvthreshd):
+    """What _lib.block_sparse_attn wants to know of the call to take its rows as the whole-operator call does."""
+    return (_lib.SELECT_CDF, None, is_causal, _number(pvthreshd)) if topk is None else (_lib.SELECT_TOPK, _number(topk), is_causal, _number(pvthreshd))
 
 
 def _staged_meansim(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
@@ -133,7 +134,7 @@ def _staged_meansim(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, topk, pv
         q, k, km, is_causal=is_causal, simthreshd1=simthreshd1, cdfthreshd=cdfthreshd, topk=topk, return_lut=True,
         attention_sink=attention_sink, BLKQ=128, BLKK=64, qk_quant_gran=qk_quant_gran)
     o, _ = _attention(q, k, v, q_int8, q_scale, k_int8, k_scale, lut, valid_block_num, scale, pvthreshd, kernel_causal,
-                      qk_quant_gran=qk_quant_gran, selected=_selected(cdfthreshd, topk, is_causal))
+                      qk_quant_gran=qk_quant_gran, selected=_selected(cdfthreshd, topk, is_causal, pvthreshd))
     return _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_denominator=is_causal is not False)
 
 
@@ -152,13 +153,14 @@ def _staged_meansim_sage1(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, to
     if scale is None:
         scale = 1.0 / (headdim ** 0.5)
     assert headdim in [64, 128], "headdim should be in [64, 128]. For other headdim, you can use padding and specify the softmax scale."
+    selected = _selected(cdfthreshd, topk, is_causal, pvthreshd)
     pvthreshd = hyperparameter_check(pvthreshd, q.size(-3), q.device)
     o = _empty_out(q)
     _mark("vquant")
     vt = _lib.v_tiles_f16_swizzled(v)
     _mark("attn")
     _lib.block_sparse_attn_f16v(q_int8, k_int8, vt, o, lut, valid_block_num, pvthreshd, q_scale, k_scale, scale,
-                                is_causal=bool(is_causal), qk_quant_gran=qk_quant_gran, selected=_selected(cdfthreshd, topk, is_causal))
+                                is_causal=bool(is_causal), qk_quant_gran=qk_quant_gran, selected=selected)
     _mark("end")
     return _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_denominator=is_causal is not False)
 
@@ -171,7 +173,7 @@ def _staged_mask(q, k, v, mask_id, scale, pvthreshd, tensor_layout, return_spars
     q_int8, q_scale, k_int8, k_scale = get_vanilla_qk_quant(q, k, km, 128, 64, qk_quant_gran=qk_quant_gran)
     lut, valid_block_num = block_map_lut_triton(block_map=mask_id)
     o, _ = _attention(q, k, v, q_int8, q_scale, k_int8, k_scale, lut, valid_block_num, scale, pvthreshd, kernel_causal,
-                      qk_quant_gran=qk_quant_gran, selected=(_lib.SELECT_MASK, None, False))
+                      qk_quant_gran=qk_quant_gran, selected=(_lib.SELECT_MASK, None, False, _number(pvthreshd)))
     # the reference always reports against the causal denominator here (core.py:230)
     return _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_denominator=True)
 

@@ -114,6 +114,7 @@ struct AttnParams {
   int rows_first;  // so many of the longest rows of every head come before the rest (place_workgroup)
   RowSelect sel;   // selection inside the kernel (template argument SEL); lut is unused then
   RawQ q;          // Q as the caller has it (template argument FQ); q8, q_scale, sel.pool_q and sel.sim_q are unused then
+  int few;         // workgroups to a row (few_rows_attn_kernel), or 0
   RowSplit split;  // rows in chunks (template argument SPLIT)
   FastDiv by_chunks;    // (rows + 7) / 8 (place_part)
 };
@@ -1242,6 +1243,336 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
   store_rows<D, ODT, PV16>(O, inv, smem + wave * (32 * OROW), sVscale, p, batch, head, qb * 128 + wave * 32, lane_e);
 }
 
+// ---- few short rows -------------------------------------------------------------------------------------------------
+// A workgroup takes 32 QW queries of a row, a quarter or a half of it, and G wavefronts for each 32 of them, which take the row's blocks in
+// turn, place rd G + grp of the list in round rd: several CUs to a row instead of one, and a row of up to G blocks in one round.  Each wavefront has tiles of its own and the next ones
+// are requested as soon as the operands of the present ones are in registers; it meets the others once per round, to learn the
+// running maximum in front of its block (P is rounded against it), and at the end, where O and the denominators are added up in the order
+// of the groups.  No wavefront sees the votes of the row's other workgroups: for thresholds at which a skipped block leaves
+// every bit as it is (few_rows).  Arithmetic and masks are those of block_sparse_attn_kernel; at most 128 blocks to a row.
+template <int D, int ODT, bool PV16, int SEL, int QW, int G>
+__global__ __launch_bounds__(64 * QW * G, 2) void few_rows_attn_kernel(const AttnParams p) {
+  constexpr int KS = D / 32, NDT = D / 32, TILE = 64 * D, VTILE = PV16 ? 2 * TILE : TILE, NKL = TILE / 1024, NVL = VTILE / 1024, W = SEL > 0 ? SEL : 1;
+  constexpr int NI = NDT * 4, NW = QW * G, PARTS = 4 / QW;   // float4s of O per lane, wavefronts, workgroups to a row
+  static_assert(NI * 1024 <= TILE + VTILE, "O of a wavefront fits its tiles");
+  __shared__ __align__(1024) unsigned char smem[NW * (TILE + VTILE)];
+  __shared__ float s_fm[2][G][QW * 32], s_d[G][QW * 32];
+  __shared__ int s_ids[128];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave % G, qw = wave / G;
+  int bh, qb;
+  const int item = blockIdx.x, wg = (item >> 3) % PARTS;
+  if (!place_workgroup(p, item & 7, (item >> 3) / PARTS, bh, qb)) return;
+  const int first_row = qb * 128 + wg * (QW * 32), row0 = first_row + qw * 32;
+  if (first_row >= p.N) return;
+  const int batch = p.by_H(bh), head = bh - batch * p.H, bhk = batch * p.Hkv + p.by_group(head);
+  const size_t row_id = (size_t)bh * p.nq + qb;
+  const int Nk = p.Nk, last_col = p.nk - 1;
+  if constexpr (!PV16) fp8_saturation_on();
+  typedef const __attribute__((address_space(4))) int32_t *c_i32_t;
+  typedef const __attribute__((address_space(4))) float *c_f32_t;
+  const float qs = ((c_f32_t)p.q_scale)[p.q_per_warp ? row_id * 4 + wg * QW + qw : row_id];
+  v4i qreg[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    qreg[ks] = (v4i){0, 0, 0, 0};
+    if (row0 + r < p.N) qreg[ks] = *(const v4i *)(p.q8 + ((size_t)bh * p.N + row0 + r) * D + 32 * ks + 16 * hh);
+  }
+  // the row's blocks, in a register each of places 0-63 and 64-127
+  int nv, ids[2];
+  if constexpr (SEL > 0) {
+    __shared__ uint16_t s_score[64 * W];
+    __shared__ int s_nv;
+    const uint8_t *simk = p.sel.sim_k + (size_t)bhk * p.nk;
+    const bool row_forced = p.sel.sim_q[row_id] == 0;
+    bool k_dead[W];
+#pragma unroll
+    for (int t = 0; t < W; t++) k_dead[t] = simk[min(64 * t + lane, last_col)] == 0;
+#pragma unroll
+    for (int c0 = 0; c0 < 64 * W; c0 += 16 * NW) {
+      const int col = c0 + (tid >> 2);
+      if (64 * W % (16 * NW) == 0 || col < 64 * W) {
+        const uint16_t s16 = pooled_score_4lanes<D, ODT>(p.sel.pool_q + row_id * D, p.sel.pool_k + ((size_t)bhk * p.nk + min(col, last_col)) * D, tid & 3);
+        if ((tid & 3) == 0) s_score[col] = s16;
+      }
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const int causal_lim = p.sel.is_causal ? min(p.nk, 2 * (qb + 1)) : p.nk;
+      uint64_t map[W] = {};
+      float sc[W];
+#pragma unroll
+      for (int t = 0; t < W; t++) sc[t] = (64 * t + lane >= causal_lim || k_dead[t]) ? -INFINITY : elem_to_f32<ODT>(s_score[64 * t + lane]);
+      select_row<ODT, W>(map, sc, k_dead, p.sel.by_topk, p.sel.level.at(head), p.nk, causal_lim, row_forced, p.sel.sink, lane);
+      int before = 0;
+#pragma unroll
+      for (int t = 0; t < W; t++) {
+        const int rank = before + __builtin_popcountll(map[t] & ((1ull << lane) - 1));
+        if ((map[t] >> lane) & 1) s_ids[rank] = 64 * t + lane;
+        before += __builtin_popcountll(map[t]);
+      }
+      if (lane == 0) s_nv = before;
+    }
+    __syncthreads();
+    nv = __builtin_amdgcn_readfirstlane(s_nv);
+    ids[0] = s_ids[lane];
+    ids[1] = W > 1 ? s_ids[64 + lane] : 0;
+    if (p.sel.valid_out != nullptr && tid == 0 && wg == 0) p.sel.valid_out[row_id] = nv;
+  } else {
+    nv = ((c_i32_t)p.valid)[row_id];
+    const int32_t *list = p.lut + row_id * p.nk;
+    const int d0 = list[min(lane, last_col)], d1 = list[min(64 + lane, last_col)];
+    ids[0] = wave_prefix_sum(lane < nv ? d0 : 0);
+    ids[1] = __builtin_amdgcn_readlane(ids[0], 63) + wave_prefix_sum(64 + lane < nv ? d1 : 0);
+  }
+  if (nv == 0) return;                                       // output rows stay unwritten (sm89.cuh:232-235)
+  auto block_of = [&](int place) __attribute__((always_inline)) {
+    return place < 64 ? __builtin_amdgcn_readlane(ids[0], place) : __builtin_amdgcn_readlane(ids[1], place - 64);
+  };
+
+  // tiles of this wavefront, laid out as block_sparse_attn_kernel has them
+  typedef __attribute__((address_space(3))) void *lds_ptr_t;
+  typedef const __attribute__((address_space(1))) void *glb_ptr_t;
+  unsigned char *const sk = smem + wave * (TILE + VTILE), *const sv = sk + TILE;
+  const uint32_t lds_k = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)smem + (uint32_t)(wave * (TILE + VTILE)), lds_v = lds_k + TILE;
+  const int8_t *kbase = p.k8 + (size_t)bhk * Nk * D;
+  const uint8_t *vbase = p.v8 + (size_t)bhk * p.nk * (size_t)VTILE;
+  const c_f32_t kscale = (c_f32_t)(p.k_scale + (size_t)bhk * p.nk);
+  const uint32_t lane_off = ((uint32_t)lane ^ (D == 128 ? (lane >> 4) & 3u : (lane >> 4) & 1u)) << 4;
+  auto load_k = [&](int b) __attribute__((always_inline)) {
+    const int8_t *kb = kbase + (size_t)(uint32_t)b * TILE;
+    const uint32_t last_row = (uint32_t)min(Nk - 1 - b * 64, 63);   // rows beyond Nk as that one: their scores are masked, their V rows are zero
+#pragma unroll
+    for (int u = 0; u < NKL; u++) {
+      const uint32_t off = lane_off ^ (u >= NKL / 2 ? (D == 128 ? 64u : 32u) : 0u), row = (uint32_t)(u * (1024 / D)) + off / D;
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(kb + min(row, last_row) * D + (off & (D - 1))), (lds_ptr_t)(sk + u * 1024), 16, 0, 0);
+    }
+  };
+  auto load_v = [&](int b) __attribute__((always_inline)) {
+    const uint8_t *vb = vbase + (size_t)(uint32_t)b * VTILE + lane * 16;
+#pragma unroll
+    for (int u = 0; u < NVL; u++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(vb + u * 1024), (lds_ptr_t)(sv + u * 1024), 16, 0, 0);
+  };
+  int blk = block_of(min(grp, nv - 1));
+  __builtin_amdgcn_s_waitcnt(0x0F70);                        // vmcnt(0): from here on it counts tiles only
+  asm volatile("" ::: "memory");
+  if (grp < nv) { load_k(blk); load_v(blk); }
+  float ksc = kscale[blk];
+  const int krow0 = 32 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3), ksw = k_swz<D>(krow0);
+  uint32_t kaddr[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) kaddr[ks] = lds_k + (uint32_t)(krow0 * D + ((hh ^ ksw) & 1) * 16) + ((uint32_t)(32 * ks) ^ (uint32_t)((ksw & 6) * 16));
+  const uint32_t va_lo = lds_v + (uint32_t)(r * 64 + (((2 * hh) ^ v_swz(r)) * 16)), va_hi = va_lo ^ 16u;
+  const uint32_t va16 = lds_v + (uint32_t)(r * 128 + (((4 * hh) ^ ((r >> 1) & 7)) * 16));
+  const float c = p.sm_scale_log2, cq26 = c * qs * SPG_ACC_SCALE, acc_c = __builtin_bit_cast(float, (int)SPG_ACC_C_BITS);
+  const int kscale_precise_bits = __builtin_bit_cast(int, 16384.0f / (acc_c * cq26));
+  float m = SPG_NEG_BIG, m_own = SPG_NEG_BIG, dsum = hh == 0 && grp == 0 ? 1.0f : 0.0f;
+  v16f O[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) O[dt][e] = 0.f;
+  const int rounds = (nv + G - 1) / G;
+#pragma unroll 1
+  for (int rd = 0; rd < rounds; rd++) {
+    const int place = rd * G + grp;
+    const bool active = place < nv, more = place + G < nv;
+    float fm = -INFINITY, mloc = acc_c;
+    const float dq = qs * ksc, a26 = cq26 * ksc;
+    const bool precise = __builtin_bit_cast(int, ksc) >= kscale_precise_bits;
+    int lim = 0x7fffffff, blk1 = blk;
+    float ksc1 = ksc;
+    bool masked = false;
+    v16i S0, S1;
+    if (active) {
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (NVL & 15) | ((NVL >> 4) << 14));   // K has arrived, V is under way
+      asm volatile("" ::: "memory");
+      v4i a0[KS], a1[KS];
+      lds_read_4x128_wait<0, 16 * D>(a0[0], a1[0], a0[1], a1[1], kaddr[0], kaddr[1]);
+      if constexpr (KS == 4) lds_read_4x128_wait<0, 16 * D>(a0[2], a1[2], a0[3], a1[3], kaddr[2], kaddr[3]);
+      if (more) {
+        blk1 = block_of(place + G);
+        load_k(blk1);
+        ksc1 = kscale[blk1];
+      }
+      asm volatile("v_mfma_i32_32x32x32_i8 %0, %2, %4, 0.15915494\n\tv_mfma_i32_32x32x32_i8 %1, %3, %4, 0.15915494"
+                   : "=&v"(S0), "=&v"(S1)
+                   : "v"(a0[0]), "v"(a1[0]), "v"(qreg[0]));
+#pragma unroll
+      for (int ks = 1; ks < KS; ks++) {
+        S0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0[ks], qreg[ks], S0, 0, 0, 0);
+        S1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1[ks], qreg[ks], S1, 0, 0, 0);
+      }
+      const int key0 = blk * 64 + 32 * hh;
+      if (p.is_causal) lim = row0 + r - key0;                    // key > query (attn_utils.cuh:334-361)
+      if (place == nv - 1) lim = min(lim, Nk - 1 - key0);        // key >= kv_len (attn_utils.cuh:363-389)
+      masked = place >= nv - 2 && __any(lim < 31);
+      if (!masked) {
+        int imax = S0[0];
+#pragma unroll
+        for (int e = 1; e < 16; e++) imax = max(imax, S0[e]);
+#pragma unroll
+        for (int e = 0; e < 16; e++) imax = max(imax, S1[e]);
+        mloc = __builtin_bit_cast(float, imax);
+        fm = (mloc - acc_c) * a26;
+      } else {
+        fm = SPG_NEG_BIG;
+        const float dq26 = dq * SPG_ACC_SCALE;
+#pragma unroll
+        for (int e = 0; e < 32; e++) {
+          float v = (__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]) - acc_c) * dq26;
+          v = e > lim ? SPG_NEG_BIG : v;
+          fm = fmaxf(fm, v);
+        }
+        fm = fm * c;
+      }
+      fm = half_swap_max_raw(fm);
+    }
+    s_fm[rd & 1][grp][qw * 32 + r] = fm;                         // (both halves hold the same value)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    float before = m, after = -INFINITY, fms[G];
+    lds_read_column<QW * 32>(fms, (uint32_t)(size_t)(__attribute__((address_space(3))) float *)&s_fm[rd & 1][0][qw * 32 + r]);
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      if (g < grp) before = max_raw(before, fms[g]);
+      if (g > grp) after = max_raw(after, fms[g]);
+    }
+    const float m_old = m_own, m_new = max_raw(before, fm);
+    m = max_raw(m_new, after);
+    if (active) {
+      m_own = m_new;
+      if (m_new > m_old) {
+        const float osc = __builtin_amdgcn_exp2f(m_old - m_new);
+        dsum *= osc;
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) O[dt][e] *= osc;
+      }
+      const float neg0 = PV16 ? -m_new : -m_new + SPG_FP8_OFFSET;
+      float x[32];
+      if (!masked) {
+        float neg = __builtin_fmaf(-acc_c, a26, neg0), base = 0.f;
+        if (__builtin_expect(precise, 0)) { neg = __builtin_fmaf(mloc - acc_c, a26, neg0); base = mloc; }   // (x - 0 is x)
+#pragma unroll
+        for (int e = 0; e < 32; e++) x[e] = __builtin_fmaf(__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]) - base, a26, neg);
+      } else {
+        const float out = __builtin_fmaf(SPG_NEG_BIG, c, neg0), dq26 = dq * SPG_ACC_SCALE;
+#pragma unroll
+        for (int e = 0; e < 32; e++) {
+          const float t = __builtin_fmaf((__builtin_bit_cast(float, e < 16 ? S0[e] : S1[e - 16]) - acc_c) * dq26, c, neg0);
+          x[e] = e > lim ? out : t;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 32; e++) x[e] = __builtin_amdgcn_exp2f(x[e]);
+      // V: behind it only the next K may be under way
+      if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | (NKL & 15) | ((NKL >> 4) << 14));
+      else __builtin_amdgcn_s_waitcnt(0x0F70);
+      asm volatile("" ::: "memory");
+      if constexpr (PV16) {
+        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        h8 pb16[4];
+        const h2 ones2 = {(_Float16)1, (_Float16)1};
+        float rs = 0.f;
+#pragma unroll
+        for (int s4 = 0; s4 < 4; s4++)
+#pragma unroll
+          for (int j = 0; j < 8; j += 2) {
+            const f2 pr = {x[8 * s4 + j], x[8 * s4 + j + 1]};
+            const h2 ph = __builtin_convertvector(pr, h2);
+            pb16[s4][j] = ph[0];
+            pb16[s4][j + 1] = ph[1];
+            rs = __builtin_amdgcn_fdot2(ph, ones2, rs, false);
+          }
+        dsum += rs;
+        v4i t[4][NDT];
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+          const uint32_t a_ = va16 ^ (uint32_t)(16 * st);
+          if constexpr (NDT == 4) { lds_read_4x128<0, 4096, 8192, 12288>(t[st][0], t[st][1], t[st][2], t[st][3], a_); lds_wait4(t[st][0], t[st][1], t[st][2], t[st][3]); }
+          else { lds_read_2x128<0, 4096>(t[st][0], t[st][1], a_); lds_wait2(t[st][0], t[st][1]); }
+#pragma unroll
+          for (int dt = 0; dt < NDT; dt++)
+            O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, t[st][dt]), pb16[st], O[dt], 0, 0, 0);
+        }
+        if (more) load_v(blk1);
+      } else {
+        float ps = x[0];
+        if constexpr (D == 64) {
+          // (the sums of block_sparse_attn_kernel)
+          float pc[4] = {x[0], x[1], x[2], x[3]};
+#pragma unroll
+          for (int e = 4; e < 32; e++) pc[e % 4] += x[e];
+          ps = (pc[0] + pc[1]) + (pc[2] + pc[3]);
+        } else {
+#pragma unroll
+          for (int e = 1; e < 32; e++) ps += x[e];
+        }
+        dsum += ps;
+        v8i pb;
+#pragma unroll
+        for (int u = 0; u < 8; u++) pb[u] = pack4_e4m3(x[4 * u], x[4 * u + 1], x[4 * u + 2], x[4 * u + 3]);
+        v4i lo[NDT], hi[NDT];
+        if constexpr (NDT == 4) {
+          lds_read_4x128_wait<0, 2048>(lo[0], lo[1], hi[0], hi[1], va_lo, va_hi);
+          lds_read_4x128_wait<4096, 6144>(lo[2], lo[3], hi[2], hi[3], va_lo, va_hi);
+        } else {
+          lds_read_4x128_wait<0, 2048>(lo[0], lo[1], hi[0], hi[1], va_lo, va_hi);
+        }
+        if (more) load_v(blk1);
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++) {
+          const v8i av = {lo[dt][0], lo[dt][1], lo[dt][2], lo[dt][3], hi[dt][0], hi[dt][1], hi[dt][2], hi[dt][3]};
+          O[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, pb, O[dt], 0, 0, 0, 0, 0, 0);
+        }
+      }
+    }
+    blk = blk1;
+    ksc = ksc1;
+  }
+  // the groups' sums, relative to the row's maximum, through their own tiles; group g then adds up float4s g, g + G, ... of the lanes
+  const float f = __builtin_amdgcn_exp2f(m_own - m), d_own = half_swap_sum_f32(dsum) * f;
+  if (hh == 0) s_d[grp][qw * 32 + r] = d_own;
+  constexpr int SLOT = (TILE + VTILE) / 16;
+  float4 *const so = (float4 *)smem + qw * (G * SLOT) + lane;
+#pragma unroll
+  for (int i = 0; i < NI; i++)
+    so[grp * SLOT + i * 64] = make_float4(O[i / 4][4 * (i % 4)] * f, O[i / 4][4 * (i % 4) + 1] * f, O[i / 4][4 * (i % 4) + 2] * f, O[i / 4][4 * (i % 4) + 3] * f);
+  float4 vsc[(NI + G - 1) / G];                              // V scales of the channels that this thread stores
+#pragma unroll
+  for (int u = 0; u < (NI + G - 1) / G; u++) {
+    const int i = grp + u * G, d0 = 32 * (i / 4) + 8 * (i % 4) + 4 * hh;
+    vsc[u] = make_float4(1.f, 1.f, 1.f, 1.f);
+    if constexpr (!PV16) vsc[u] = *(const float4 *)(p.v_scale + (size_t)bhk * D + min(d0, D - 4));
+  }
+  __syncthreads();
+  float d = s_d[0][qw * 32 + r];
+#pragma unroll
+  for (int g = 1; g < G; g++) d += s_d[g][qw * 32 + r];
+  const float inv = __builtin_amdgcn_rcpf(d);
+  uint16_t *const out = (uint16_t *)p.out + (size_t)batch * p.os.sb + (size_t)head * p.os.sh + (size_t)(row0 + r) * p.os.sn;
+#pragma unroll
+  for (int u = 0; u < (NI + G - 1) / G; u++) {
+    const int i = grp + u * G, d0 = 32 * (i / 4) + 8 * (i % 4) + 4 * hh;
+    if (i >= NI) continue;
+    float4 s = so[i * 64];
+#pragma unroll
+    for (int g = 1; g < G; g++) {
+      const float4 t = so[g * SLOT + i * 64];
+      s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+    }
+    const uint16_t o0 = f32_to_elem<ODT>(s.x * inv * vsc[u].x), o1 = f32_to_elem<ODT>(s.y * inv * vsc[u].y);
+    const uint16_t o2 = f32_to_elem<ODT>(s.z * inv * vsc[u].z), o3 = f32_to_elem<ODT>(s.w * inv * vsc[u].w);
+    if (row0 + r < p.N) *(uint2 *)(out + d0) = make_uint2((uint32_t)o0 | ((uint32_t)o1 << 16), (uint32_t)o2 | ((uint32_t)o3 << 16));
+  }
+}
+
 // ---- rows in chunks ------------------------------------------------------------------------------------------------
 // Maxima of the chunks of a row but the last, per query, over the scores as block_sparse_attn_kernel sees them: its running maximum
 // in front of a chunk is the largest of those before it, to the bit, since it takes the same products in binary32.
@@ -1467,6 +1798,24 @@ static hipError_t launch_attn(AttnParams &p, int D, int out_dtype, bool causal_r
   p.rows_first = (causal_rows && p.wg_per_xcd <= SPG_ROW_MAJOR_MAX) ? p.nq : (p.N % 128 != 0 || causal_rows) ? 1 : 0;
   p.by_nq = FastDiv::of(p.nq); p.by_rest = FastDiv::of(p.nq > p.rows_first ? p.nq - p.rows_first : 1);
   p.by_H = FastDiv::of(p.H); p.by_group = FastDiv::of(p.H / p.Hkv);
+  if constexpr (FQ == 0) {
+    if (p.few > 0) {
+      p.queue = nullptr;
+#define SPG_FEW_(D_, PV16_, QW_, G_)                                                                                        \
+  {                                                                                                                         \
+    const int wgs = 8 * (4 / QW_) * p.wg_per_xcd;                                                                           \
+    if (out_dtype == 0) few_rows_attn_kernel<D_, 0, PV16_, SEL, QW_, G_><<<wgs, 64 * QW_ * G_, 0, st>>>(p);                    \
+    else few_rows_attn_kernel<D_, 1, PV16_, SEL, QW_, G_><<<wgs, 64 * QW_ * G_, 0, st>>>(p);                                   \
+  }
+#define SPG_FEW(D_, PV16_, NW_) { if (p.few == 4) SPG_FEW_(D_, PV16_, 1, NW_) else SPG_FEW_(D_, PV16_, 2, NW_ / 2) }
+      // (the FP16 tiles of eight wavefronts at D = 128 would not fit the LDS)
+      if (p.v_scale != nullptr) { if (D == 64) SPG_FEW(64, false, 8) else SPG_FEW(128, false, 8) }
+      else { if (D == 64) SPG_FEW(64, true, 8) else SPG_FEW_(128, true, 1, 6) }
+#undef SPG_FEW
+#undef SPG_FEW_
+      return hipGetLastError();
+    }
+  }
   if constexpr (SEL == 0 && FQ == 0) {
     if (p.split.chunks > 1) {
       p.queue = nullptr;
@@ -1504,10 +1853,11 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
                                       int out_dtype, const int32_t *lut, const int32_t *valid, const RowSelect *sel, const RawQ *q,
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
-                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue, const RowSplit *split,
+                                      int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue, const RowSplit *split, int few,
                                       hipStream_t st) {
   AttnParams p = {};
   p.queue = queue;
+  p.few = few;
   if (split != nullptr) p.split = *split;
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.out = out; p.os = os; p.lut = lut; p.valid = valid; p.pvthr = pvthreshd;
   p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.pv_count = pv_count;
@@ -1530,7 +1880,7 @@ hipError_t launch_block_sparse_attn(const int8_t *q8, const int8_t *k8, const ui
                                     int Hkv, int N, int Nk, int D, float sm_scale, int is_causal, int q_per_warp,
                                     int pv_mode, int32_t *pv_count, hipStream_t st) {
   return launch_block_sparse_attn_h(q8, k8, v8, out, os, out_dtype, lut, valid, nullptr, nullptr, Hyper{pvthreshd, 0.f}, q_scale, k_scale,
-                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, false, nullptr, nullptr, st);
+                                    v_scale, B, H, Hkv, N, Nk, D, sm_scale, is_causal, q_per_warp, pv_mode, pv_count, false, nullptr, nullptr, 0, st);
 }
 
 }  // namespace spg

@@ -5,6 +5,7 @@
 #include "forward_plan.h"
 
 #include <chrono>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 
@@ -195,35 +196,46 @@ int spg_block_sparse_attn_f16v(const int8_t *q8, const int8_t *k8, const void *v
                                                         pv_threshold_mode, pv_count, (hipStream_t)stream));
 }
 
-size_t spg_block_sparse_attn_chunks_bytes(int B, int H, int N, int N_kv, int D, int selection, float share, int is_causal) {
-  const char *fn = "spg_block_sparse_attn_chunks_bytes";
-  if (check_shape(fn, B, H, N, D) != SPG_OK || check_shape(fn, B, H, N_kv, D) != SPG_OK) return 0;
-  return rows_in_chunks(B, H, N, N_kv, D, selection, share, is_causal != 0) ? chunk_plan(B, H, N, N_kv, D).bytes : 0;
+int spg_few_rows_route(int B, int H, int N, int N_kv, int D, int pv_f16, int selection, float share, int is_causal, float pvthreshd,
+                       uint64_t *workspace_bytes) {
+  const char *fn = "spg_few_rows_route";
+  if (workspace_bytes != nullptr) *workspace_bytes = 0;
+  if (check_shape(fn, B, H, N, D) != SPG_OK || check_shape(fn, B, H, N_kv, D) != SPG_OK) return SPG_ROWS_ONE_WORKGROUP;
+  if (few_rows(B, H, N, N_kv, D, pv_f16 != 0, pvthreshd) > 0) return SPG_ROWS_BY_QUERIES;
+  if (!rows_in_chunks(B, H, N, N_kv, D, selection, share, is_causal != 0)) return SPG_ROWS_ONE_WORKGROUP;
+  if (workspace_bytes != nullptr) *workspace_bytes = chunk_plan(B, H, N, N_kv, D).bytes;
+  return SPG_ROWS_BY_BLOCKS;
 }
 
-int spg_block_sparse_attn_chunks(const int8_t *q8, const int8_t *k8, const void *v, void *out, const int64_t *out_strides, int out_dtype,
-                                 const int32_t *lut, const int32_t *valid_block_num, const float *pvthreshd, const float *q_scale,
-                                 const float *k_scale, const float *v_scale, int B, int H, int Hkv, int N, int N_kv, int D, float sm_scale,
-                                 int is_causal, int qk_quant_gran, void *workspace, uint64_t workspace_bytes, void *stream) {
-  const char *fn = "spg_block_sparse_attn_chunks";
+int spg_block_sparse_attn_few_rows(const int8_t *q8, const int8_t *k8, const void *v, void *out, const int64_t *out_strides, int out_dtype,
+                                   const int32_t *lut, const int32_t *valid_block_num, const float *pvthreshd, const float *q_scale,
+                                   const float *k_scale, const float *v_scale, int B, int H, int Hkv, int N, int N_kv, int D, float sm_scale,
+                                   int is_causal, int qk_quant_gran, int route, void *workspace, uint64_t workspace_bytes, void *stream) {
+  const char *fn = "spg_block_sparse_attn_few_rows";
   SPG_TRY(check_shape(fn, B, H, N, D));
   SPG_TRY(check_shape(fn, B, Hkv > 0 ? Hkv : 1, N_kv, D));
   SPG_TRY(check_kv_heads(fn, H, Hkv));
   SPG_TRY(check_quant_gran(fn, qk_quant_gran));
   SPG_TRY(check_dtype(fn, out_dtype));
   SPG_NONNULL(fn, q8); SPG_NONNULL(fn, k8); SPG_NONNULL(fn, v); SPG_NONNULL(fn, out); SPG_NONNULL(fn, lut);
-  SPG_NONNULL(fn, valid_block_num); SPG_NONNULL(fn, pvthreshd); SPG_NONNULL(fn, q_scale); SPG_NONNULL(fn, k_scale); SPG_NONNULL(fn, workspace);
+  SPG_NONNULL(fn, valid_block_num); SPG_NONNULL(fn, pvthreshd); SPG_NONNULL(fn, q_scale); SPG_NONNULL(fn, k_scale);
   spg::Strides os;
   SPG_TRY(get_strides(fn, "out_strides", out_strides, H, N, D, &os));
   const ChunkPlan c = chunk_plan(B, H, N, N_kv, D);
-  if (c.chunks == 1) return fail(SPG_ERR_UNSUPPORTED, "%s: rows of this call are not taken in chunks", fn);
-  if (workspace_bytes < c.bytes) return fail(SPG_ERR_INVALID, "%s: workspace of %zu bytes, %zu needed", fn, (size_t)workspace_bytes, c.bytes);
-  if ((uintptr_t)workspace % 256 != 0) return fail(SPG_ERR_INVALID, "%s: workspace must be 256-byte aligned (got %p)", fn, workspace);
-  const RowSplit split = row_split(c, workspace);
+  const int few = few_rows(B, H, N, N_kv, D, v_scale == nullptr, INFINITY);
+  if (route != SPG_ROWS_BY_QUERIES && route != SPG_ROWS_BY_BLOCKS) return fail(SPG_ERR_INVALID, "%s: bad route %d", fn, route);
+  if (route == SPG_ROWS_BY_QUERIES ? few == 0 : c.chunks == 1) return fail(SPG_ERR_UNSUPPORTED, "%s: the rows of this call have one workgroup each", fn);
+  RowSplit split = {};
+  if (route == SPG_ROWS_BY_BLOCKS) {
+    SPG_NONNULL(fn, workspace);
+    if (workspace_bytes < c.bytes) return fail(SPG_ERR_INVALID, "%s: workspace of %zu bytes, %zu needed", fn, (size_t)workspace_bytes, c.bytes);
+    if ((uintptr_t)workspace % 256 != 0) return fail(SPG_ERR_INVALID, "%s: workspace must be 256-byte aligned (got %p)", fn, workspace);
+    split = row_split(c, workspace);
+  }
   return check_launch(fn, spg::launch_block_sparse_attn_h(q8, k8, (const uint8_t *)v, out, os, out_dtype, lut, valid_block_num, nullptr, nullptr,
                                                           Hyper{pvthreshd, 0.f}, q_scale, k_scale, v_scale, B, H, Hkv, N, N_kv, D, sm_scale,
                                                           is_causal ? 1 : 0, qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0, SPG_PV_PER_BLOCK,
-                                                          nullptr, false, nullptr, &split, (hipStream_t)stream));
+                                                          nullptr, false, nullptr, &split, route == SPG_ROWS_BY_QUERIES ? few : 0, (hipStream_t)stream));
 }
 
 static int check_forward(const char *fn, const spg_attn_args *a) {

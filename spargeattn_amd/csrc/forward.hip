@@ -11,7 +11,7 @@
 //            of the next launch to add them up for itself)
 //   back     pooling + quantisation of K | V -> e4m3 tiles and scales (FP16 PV, many blocks: V^T tiles)
 //   select   block_select_* of maskpred.hip (rows of more than 128 blocks; shorter ones are selected inside the next launch)
-//   attn     block_sparse_attn_kernel (few long rows: in chunks, with a launch in front for their maxima and one behind)
+//   attn     block_sparse_attn_kernel (few short rows: few_rows_attn_kernel, several workgroups to a row; few long rows: in chunks, with a launch in front for their maxima and one behind)
 // Every body is the one the stage-by-stage entry points launch (stage_bodies.h): results are the same bits.
 // The extern "C" entry points and their argument checks are in capi.hip, the workspace layout in forward_plan.h.
 // Compile with -ffp-contract=off.
@@ -379,7 +379,8 @@ hipError_t run_forward(const spg_attn_args *a, const Strides &qs, const Strides 
                                     Hyper{a->pvthreshd, a->pvthreshd_value},
                                     f.q_scale, b.k_scale, a->pv_f16 ? nullptr : b.v_scale, a->B, a->H, a->Hkv, a->N, a->N_kv, a->D,
                                     a->sm_scale, a->kernel_causal ? 1 : 0, a->qk_quant_gran == SPG_QUANT_PER_WARP ? 1 : 0,
-                                    SPG_PV_PER_BLOCK, nullptr, pool && a->is_causal, f.queue, &split, st);
+                                    SPG_PV_PER_BLOCK, nullptr, pool && a->is_causal, f.queue, &split,
+                                    front_q ? few_rows(a) : 0, st);
 }
 
 }  // namespace spg

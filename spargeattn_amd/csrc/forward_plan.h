@@ -177,6 +177,27 @@ inline bool rows_in_chunks(const spg_attn_args *a) {
   return rows_in_chunks(a->B, a->H, a->N, a->N_kv, a->D, a->selection, share, a->is_causal != 0);
 }
 
+// Few short rows: workgroups to a row (few_rows_attn_kernel), or 0 where it has one.  Four while each has a CU to itself, two up to 128 rows; the
+// workgroup with all four quarters (attn_groups) beyond, and where a row has no more blocks than it has groups.  us per call with one /
+// four workgroups to a row, top-k 0.2, 0.5 and 1.0, rows x nk: D64 16 x 8 14.3 / 13.7, 14.9 / 14.0, 17.0 / 13.8; 64 x 16 16.4 / 14.4, 19.0 / 15.3, 22.3 / 16.0, 64 x 64 26.5 / 22.0,
+// 37.1 / 26.9, 53.4 / 32.8, 64 x 128 44.0 / 34.5, 61.9 / 43.5, 90.4 / 57.0; 96 x 16 16.5 / 19.5, 19.2 / 21.5, 22.6 / 23.1.  D128 16 x 4 14.5 / 14.8, 15.5 / 14.6, 16.6 /
+// 14.2; 64 x 16 22.5 / 19.9, 26.3 / 21.6, 30.6 / 23.4, 64 x 128 54.2 / 42.7, 78.6 / 55.5, 116.8 / 73.7; FP16 PV 64 x 64 36.4 / 30.6, 52.7 / 41.7, 76.4 / 54.5.  One /
+// two: D64 128 x 8 13.6 / 13.7, 15.2 / 14.5, 17.3 / 14.8; 128 x 16 16.6 / 15.8, 19.3 / 17.2, 22.6 / 19.5, 128 x 128 45.2 / 40.2, 62.5 / 55.3, 91.6 / 78.5, 160 x 32 21.5 / 27.9,
+// 27.5 / 34.5, 34.5 / 45.7; D128 128 x 8 16.7 / 17.6, 19.7 / 18.6, 22.3 / 20.0, 128 x 16 23.1 / 22.2, 26.7 / 24.7, 31.5 / 28.3, 128 x 128 54.3 / 49.5, 78.8 / 68.2, 116.5 /
+// 99.0; FP16 PV at D128, whose tiles leave room for three groups, 128 x 64 38.0 / 37.5, 53.9 / 54.1, 77.4 / 77.6.
+// The workgroups of a row do not see each other's votes on the PV threshold, so it has to be one that no vote can change a bit by: a block is skipped
+// when all its scores are `pvthreshd` below the running maxima in the exponent of 2, so from 45 on its P are zero in e4m3 and in fp16, and
+// what they add to the denominator is below 2^-40 of it.  (A per-head threshold is not known here: 0.)
+inline int few_rows(int B, int H, int N, int N_kv, int D, bool pv_f16, float pvthreshd) {
+  const long long rows = (long long)B * H * ((N + 127) / 128), nk = (N_kv + 63) / 64;
+  if (!(pvthreshd >= 45.f) || nk > 128) return 0;
+  if (rows <= 64) return nk >= 6 ? 4 : 0;
+  return rows <= 128 && nk >= 12 && !(pv_f16 && D == 128) ? 2 : 0;
+}
+inline int few_rows(const spg_attn_args *a) {
+  return few_rows(a->B, a->H, a->N, a->N_kv, a->D, a->pv_f16 != 0, a->pvthreshd == nullptr ? a->pvthreshd_value : 0.f);
+}
+
 struct Layout {
   size_t km_part, v_part, km, v_amax, pool_q, pool_k, sim_q, sim_k, q8, k8, q_scale, k_scale, v, v_scale, lut, valid, queue, split, total;
 };

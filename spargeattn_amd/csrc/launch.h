@@ -102,6 +102,7 @@ struct RowSplit {
   float *md;                        // [rows][chunks][2][128]    running maximum at its end, denominator
   float *o;                         // [rows][chunks][128 x D]   sums, as the lanes hold them
 };
+// few: workgroups to a row as few_rows (forward_plan.h) has them, with q == NULL and pv_count == NULL, or 0.
 // split: with sel == NULL, q == NULL, pv_count == NULL and the per-block PV threshold only.
 // sel == NULL: blocks come from lut / valid; otherwise they are selected in place and lut / valid are not read.
 // q == NULL: Q comes as q8 / q_scale (and pooled in sel); otherwise from the caller's tensor, and those are not read.
@@ -112,7 +113,7 @@ hipError_t launch_block_sparse_attn_h(const int8_t *q8, const int8_t *k8, const 
                                       Hyper pvthreshd, const float *q_scale, const float *k_scale, const float *v_scale,
                                       int B, int H, int Hkv, int N, int Nk, int D, float sm_scale, int is_causal,
                                       int q_per_warp, int pv_mode, int32_t *pv_count, bool causal_rows, int *queue,
-                                      const RowSplit *split, hipStream_t st);
+                                      const RowSplit *split, int few, hipStream_t st);
 void launch_fp8_pack_selftest(const float *x, uint8_t *codes, int n, int saturate, hipStream_t st);
 
 hipError_t launch_dense_attn_f16(const void *q, const void *k, const void *v, void *out, int B, int H, int N, int D,

@@ -58,6 +58,37 @@ __device__ __forceinline__ void lds_read_4x128(v4i &a, v4i &b, v4i &c, v4i &d, u
                : "v"(addr), "n"(O0), "n"(O1), "n"(O2), "n"(O3)
                : "memory");
 }
+// v[g] <- addr + 4 STRIDE g: one value of every group
+template <int STRIDE, int G>
+__device__ __forceinline__ void lds_read_column(float (&v)[G], uint32_t addr) {
+  static_assert((G - 1) * STRIDE * 4 < 65536, "immediate offsets");
+  if constexpr (G == 8)
+    asm volatile("ds_read_b32 %0, %8\n\tds_read_b32 %1, %8 offset:%9\n\tds_read_b32 %2, %8 offset:%10\n\tds_read_b32 %3, %8 offset:%11\n\t"
+                 "ds_read_b32 %4, %8 offset:%12\n\tds_read_b32 %5, %8 offset:%13\n\tds_read_b32 %6, %8 offset:%14\n\t"
+                 "ds_read_b32 %7, %8 offset:%15\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+                 : "v"(addr), "n"(4 * STRIDE), "n"(8 * STRIDE), "n"(12 * STRIDE), "n"(16 * STRIDE), "n"(20 * STRIDE), "n"(24 * STRIDE), "n"(28 * STRIDE)
+                 : "memory");
+  else if constexpr (G == 6)
+    asm volatile("ds_read_b32 %0, %6\n\tds_read_b32 %1, %6 offset:%7\n\tds_read_b32 %2, %6 offset:%8\n\tds_read_b32 %3, %6 offset:%9\n\t"
+                 "ds_read_b32 %4, %6 offset:%10\n\tds_read_b32 %5, %6 offset:%11\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5])
+                 : "v"(addr), "n"(4 * STRIDE), "n"(8 * STRIDE), "n"(12 * STRIDE), "n"(16 * STRIDE), "n"(20 * STRIDE)
+                 : "memory");
+  else if constexpr (G == 4)
+    asm volatile("ds_read_b32 %0, %4\n\tds_read_b32 %1, %4 offset:%5\n\tds_read_b32 %2, %4 offset:%6\n\tds_read_b32 %3, %4 offset:%7\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+                 : "v"(addr), "n"(4 * STRIDE), "n"(8 * STRIDE), "n"(12 * STRIDE)
+                 : "memory");
+  else {
+    static_assert(G == 3, "number of groups");
+    asm volatile("ds_read_b32 %0, %3\n\tds_read_b32 %1, %3 offset:%4\n\tds_read_b32 %2, %3 offset:%5\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2])
+                 : "v"(addr), "n"(4 * STRIDE), "n"(8 * STRIDE)
+                 : "memory");
+  }
+}
 // wait for all LDS reads but the last N (they return in order; a scalar load still under way only makes the wait longer)
 template <int N> __device__ __forceinline__ void lds_wait_but(v4i &a, v4i &b) {
   asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "n"(N));

@@ -24,7 +24,7 @@ hipError_t launch_block_sparse_attn(const int8_t *, const int8_t *, const uint8_
                                     int, int, int, int, float, int, int, int, int32_t *, hipStream_t) { g_launches++; return hipSuccess; }
 hipError_t launch_block_sparse_attn_h(const int8_t *, const int8_t *, const uint8_t *, void *, Strides, int, const int32_t *, const int32_t *,
                                       const RowSelect *, const RawQ *, Hyper, const float *, const float *, const float *, int, int, int, int,
-                                      int, int, float, int, int, int, int32_t *, bool, int *, const RowSplit *, hipStream_t) { g_launches++; return hipSuccess; }
+                                      int, int, float, int, int, int, int32_t *, bool, int *, const RowSplit *, int, hipStream_t) { g_launches++; return hipSuccess; }
 void launch_fp8_pack_selftest(const float *, uint8_t *, int, int, hipStream_t) { g_launches++; }
 hipError_t launch_dense_attn_f16(const void *, const void *, const void *, void *, int, int, int, int, float, int,
                                  hipStream_t) { g_launches++; return hipSuccess; }

@@ -20,8 +20,8 @@ def routes(tmp_path_factory):
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-4000:]
 
-    def route(B=1, H=1, Hkv=0, N=128, Nk=0, D=128, selection=TOPK, pv_f16=0, sim=-0.1, level=0.5, causal=0):
-        line = f"{B} {H} {Hkv or H} {N} {Nk or N} {D} {selection} {pv_f16} {sim} {level} {causal}\n"
+    def route(B=1, H=1, Hkv=0, N=128, Nk=0, D=128, selection=TOPK, pv_f16=0, sim=-0.1, level=0.5, causal=0, pv=50):
+        line = f"{B} {H} {Hkv or H} {N} {Nk or N} {D} {selection} {pv_f16} {sim} {level} {causal} {pv}\n"
         out = subprocess.run([exe], input=line, capture_output=True, text=True, timeout=60)
         assert out.returncode == 0
         return [int(x) for x in out.stdout.split()]
@@ -93,3 +93,12 @@ def test_chunks_of_a_row_are_bounded(routes, D, most):
         rows, n = H * -(-N // 128), routes(H=H, N=N, Nk=64 * nk, D=D, selection=MASK)[6]
         assert 1 < n <= 64 and n <= -(-nk // 16) and rows * (n - 1) <= most
     assert routes(H=2, N=16385, Nk=64 * 512, D=D)[6] == 1
+
+
+@pytest.mark.parametrize("kw,wgs", [
+    (dict(H=4, N=128, Nk=64 * 5), 0), (dict(H=4, N=128, Nk=64 * 6), 4), (dict(H=8, N=1024, Nk=64 * 128), 4), (dict(H=8, N=1024, Nk=64 * 129), 0),
+    (dict(H=13, N=640, Nk=64 * 12), 2), (dict(H=13, N=640, Nk=64 * 11), 0), (dict(H=8, N=2048, Nk=64 * 100), 2), (dict(H=8, N=2049, Nk=64 * 100), 0),
+    (dict(H=8, N=2048, Nk=64 * 100, pv_f16=1), 0), (dict(H=8, N=2048, Nk=64 * 100, D=64, pv_f16=1), 2), (dict(H=8, N=1024, Nk=64 * 100, pv_f16=1), 4),
+    (dict(H=8, N=1024, pv=44.9), 0), (dict(H=8, N=1024, pv=45), 4), (dict(H=8, N=1024, pv=0), 0), (dict(H=8, N=1024, pv="nan"), 0)])
+def test_few_short_rows_have_several_workgroups(routes, kw, wgs):
+    assert routes(**kw)[8] == wgs

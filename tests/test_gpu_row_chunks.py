@@ -40,8 +40,8 @@ def test_chunks_equal_the_sequential_walk(D, dtype, f16v, gran, causal, H, nq, n
     lut, valid = lists(B, H, nq, nk, [0, 1, 2, 3, 15, 16, 17, 18, 31, 32, 33, 34, 47, 48, 49, 64, 65, 97, nk - 1, nk], g)
     thr = torch.tensor([50.0, 2.0, 0.5, 0.0] * 2, device="cuda")[:H].contiguous()
     v = torch.randn((B, Hkv, Nk, D), generator=g).to(torch.float16).cuda()
-    selected = (_lib.SELECT_TOPK, share, False)
-    assert _lib.load().spg_block_sparse_attn_chunks_bytes(B, H, N, Nk, D, selected[0], share, 0) > 0
+    selected = (_lib.SELECT_TOPK, share, False, None)
+    assert _lib.few_rows_route(q8.shape, Nk, f16v, selected)[0] == _lib.ROWS_BY_BLOCKS
 
     def run(count):
         o = torch.full((B, H, N, D), 7.0, dtype=dtype, device="cuda")
