@@ -272,6 +272,47 @@ __global__ __launch_bounds__(256) void block_select_kernel(
   }
 }
 
+// A probability e / total as a 16-bit pattern, from e * (1 / total), which is within two units in the last place of the quotient:
+// through binary32, the two agree unless the product lands exactly on a rounding tie of the 16-bit format or outside its normal
+// range, and those elements take the division and the exact conversion.
+template <int DT> __device__ __forceinline__ uint32_t probability_bits(double e, double total, double rtotal) {
+  const float pr = (float)(e * rtotal);
+  const uint32_t pb = __builtin_bit_cast(uint32_t, pr);    // probabilities are non-negative
+  constexpr uint32_t DROP = DT == 1 ? 16u : 13u, LOWM = (1u << DROP) - 1u, TIE = 1u << (DROP - 1u);
+  constexpr uint32_t LO = DT == 1 ? 0x00800000u : 0x38800000u;     // smallest normal of the format
+  const bool safe = pb == 0u || (pb >= LO && pb <= 0x3f800000u && (pb & LOWM) != TIE);
+  if (safe) return f32_to_elem<DT>(pr);
+  double p = e / total;
+  if (!__builtin_isfinite(p)) p = 0.0;
+  return f64_to_elem<DT>(p);
+}
+
+// Top-k needs the n-th largest key only, not the order: build it bit by bit, the largest T with #{key >= T} >= n.  Keys are
+// distinct, probabilities are <= 1 (bits 31 and 30 of a key are clear) and bits 15 .. log2(64 EPL) are set in every real key (they
+// hold 0xFFFF - column).  A candidate that exactly n keys reach selects the same set as the n-th largest key itself, so the
+// search stops there.
+template <int EPL> __device__ __forceinline__ uint32_t nth_largest_key(const uint32_t (&okey)[EPL], int n) {
+  constexpr int LOW = 31 - __builtin_clz((unsigned)(64 * EPL));
+  uint32_t T = 0u;
+  bool exact = false;                                      // wavefront-uniform
+  auto try_bit = [&](int bit) {
+    const uint32_t cand = T | (1u << bit);
+    int cnt = 0;
+#pragma unroll
+    for (int tt = 0; tt < EPL; tt++) cnt += __builtin_popcountll(__ballot(okey[tt] >= cand));
+    if (cnt >= n) T = cand;
+    exact = cnt == n;
+  };
+#pragma unroll 1
+  for (int bit = 29; bit >= 16 && !exact; bit--) try_bit(bit);
+  if (!exact) {
+    T |= 0xffffu & ~((1u << LOW) - 1u);
+#pragma unroll 1
+    for (int bit = LOW - 1; bit >= 0 && !exact; bit--) try_bit(bit);
+  }
+  return T;
+}
+
 // =============================================================================================
 // block_select, wavefront-per-row variant (nk <= 2048).
 // Phase 1 computes the scores of 16 pooled-Q rows against all pooled-K rows on the matrix unit in binary64
@@ -432,29 +473,13 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
     part = wave_tree_sum_f64(part);
     const double total = part;
 
-    // probabilities -> sortable keys (value bits, then lower column first).  The 16-bit pattern of e / total is taken
-    // from e * (1 / total), which is within two units in the last place of the quotient: through binary32, the two
-    // agree unless the product lands exactly on a rounding tie of the 16-bit format or outside its normal range, and
-    // those elements take the division and the exact conversion.
+    // probabilities -> sortable keys (value bits, then lower column first)
     const double rtotal = total > 0.0 ? 1.0 / total : 0.0;     // a row without a live column has e = 0 everywhere
     uint32_t okey[EPL], key[EPL];
 #pragma unroll
     for (int t = 0; t < EPL; t++) {
       const int j = t * 64 + lane;
-      const float pr = (float)(ev[t] * rtotal);
-      const uint32_t pb = __builtin_bit_cast(uint32_t, pr);    // probabilities are non-negative
-      constexpr uint32_t DROP = DT == 1 ? 16u : 13u, LOWM = (1u << DROP) - 1u, TIE = 1u << (DROP - 1u);
-      constexpr uint32_t LO = DT == 1 ? 0x00800000u : 0x38800000u;     // smallest normal of the format
-      const bool safe = pb == 0u || (pb >= LO && pb <= 0x3f800000u && (pb & LOWM) != TIE);
-      uint32_t bits;
-      if (safe) {
-        bits = f32_to_elem<DT>(pr);
-      } else {
-        double p = ev[t] / total;
-        if (!__builtin_isfinite(p)) p = 0.0;
-        bits = f64_to_elem<DT>(p);
-      }
-      okey[t] = j < nk ? ((bits << 16) | (0xffffu - (uint32_t)j)) : 0u;
+      okey[t] = j < nk ? ((probability_bits<DT>(ev[t], total, rtotal) << 16) | (0xffffu - (uint32_t)j)) : 0u;
       key[t] = okey[t];
     }
     // how many to keep, and the key of the last one kept
@@ -464,31 +489,7 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
       const float t = level.at(h) * (float)nk;            // binary32 product, truncated (utils.py:405)
       n = (long long)t;
       if (n <= 0) n = 1;                              // utils.py:289
-      if (n < nk) {
-        // top-k needs the n-th largest key only, not the order: build it bit by bit, the largest T with
-        // #{key >= T} >= n.  Keys are distinct, probabilities are <= 1 (bits 31 and 30 of a key are clear) and
-        // bits 15 .. log2(NKP) are set in every real key (they hold 0xFFFF - column).  A candidate that exactly n keys
-        // reach selects the same set as the n-th largest key itself, so the search stops there.
-        constexpr int LOW = 31 - __builtin_clz((unsigned)NKP);   // log2(NKP)
-        uint32_t T = 0u;
-        bool exact = false;                                      // wavefront-uniform
-        auto try_bit = [&](int bit) {
-          const uint32_t cand = T | (1u << bit);
-          int cnt = 0;
-#pragma unroll
-          for (int tt = 0; tt < EPL; tt++) cnt += __builtin_popcountll(__ballot(okey[tt] >= cand));
-          if (cnt >= (int)n) T = cand;
-          exact = cnt == (int)n;
-        };
-#pragma unroll 1
-        for (int bit = 29; bit >= 16 && !exact; bit--) try_bit(bit);
-        if (!exact) {
-          T |= 0xffffu & ~((1u << LOW) - 1u);
-#pragma unroll 1
-          for (int bit = LOW - 1; bit >= 0 && !exact; bit--) try_bit(bit);
-        }
-        kth = T;
-      }
+      if (n < nk) kth = nth_largest_key<EPL>(okey, (int)n);
     } else {
       bitonic_sort_desc<EPL, 2>(key, lane);           // sorted position of key[t] is lane * EPL + t
       // cdf[v] = T(sum_{u<=v} p_sorted[u]);  n = #{v < nk : cdf[v] <= threshold}  (utils.py:398-403)
@@ -505,7 +506,7 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
 #pragma unroll
       for (int t = 0; t < EPL; t++) {
         run += (double)elem_to_f32<DT>((uint16_t)(key[t] >> 16));
-        const float cdfv = elem_to_f32<DT>(f64_to_elem<DT>(run));
+        const float cdfv = elem_to_f32<DT>(f64_to_elem_fast<DT>(run));
         if (lane * EPL + t < nk && (double)cdfv <= thr) cnt++;
       }
       n = wave_sum_i32(cnt);
@@ -556,6 +557,229 @@ __global__ __launch_bounds__(64 * NW, (!DUAL && NW == 8) ? 2 : 1) void block_sel
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();                  // the index list is reused by this wavefront's next row
+  }
+}
+
+// =============================================================================================
+// block_select, workgroup-per-row variant (nk <= 2048), for grids that leave most of the chip idle.
+// A row alone is a chain of steps that wait for each other, so what counts is the length of that chain: of 14.9 us in the
+// kernel above (one head, nk 278, CDF) the scores took 5.3 (three tiles behind one another on the matrix unit, half of each
+// tile for rows that are not there), the sort of 512 keys in one wavefront 2.6, the running sums and their conversion 2.2.
+// Launch of 139 such rows: 16.2 us there, 8.8 here; 64 rows of nk 1875, D=128, top-k: the call 210 -> 167.
+// Here the eight (nk <= 256: four) wavefronts of a workgroup share every step that can be shared: four lanes to a score, P = EPL / NW
+// columns per lane for exponentials and keys, a sort of 64 P keys per wavefront and the merge by rank (a binary search in each of
+// the other sorted runs).  Only the running sums are one wavefront's, since their order is part of the result.
+// =============================================================================================
+template <int D, int DT, int EPL>
+__global__ __launch_bounds__(EPL == 4 ? 256 : 512) void block_select_row_kernel(
+    const uint16_t *__restrict__ pool_q, const uint8_t *__restrict__ sim_q, const uint16_t *__restrict__ pool_k,
+    const uint8_t *__restrict__ sim_k, const bool by_topk, const Hyper level, int is_causal,
+    int sink, int32_t *__restrict__ lut, int32_t *__restrict__ valid, int32_t *__restrict__ valid_out, uint8_t *__restrict__ bmap, int H, int Hkv, int nq,
+    int nk) {
+  constexpr int NKP = 64 * EPL, NW = EPL == 4 ? 4 : 8, NT = 64 * NW, P = EPL / NW, RUN = 64 * P;
+  __shared__ uint16_t s_score[NKP];                     // scores as 16-bit patterns
+  __shared__ double s_ev[NKP];                          // exponentials
+  __shared__ __align__(16) uint32_t s_run[NKP];         // keys (top-k) or NW sorted runs of RUN keys (CDF)
+  __shared__ __align__(16) uint32_t s_sorted[NKP];
+  __shared__ double s_lsum[128];                        // 64 zeros, then the lane sums
+  __shared__ uint64_t s_map[EPL];
+  __shared__ uint32_t s_kth;
+
+  const int i = blockIdx.x, bh = blockIdx.y, h = bh % H, tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const float sm_scale = (D == 64) ? 0.125f : 0.088388347648318447f;  // fp32(D^-0.5)
+  const int bhk = (bh / H) * Hkv + h / (H / Hkv);
+  const uint16_t *pk_base = pool_k + (size_t)bhk * nk * D;
+  const uint8_t *simk = sim_k + (size_t)bhk * nk;
+  const int causal_lim = is_causal ? min(nk, 2 * (i + 1)) : nk;
+  constexpr uint16_t NEG_INF = DT == 1 ? 0xff80u : 0xfc00u;
+
+  // ---- scores: lane `part` of a group of four takes the 16-byte pieces part, part + 4, ...; products of two 16-bit floats and
+  // their sums are exact in binary64, so the order of the additions is free
+  {
+    constexpr int NL = D / 32, COLS = NT / 4;           // columns per trip
+    const int part = tid & 3, c = tid >> 2;
+    auto load_k = [&](int j, uint4 (&raw)[NL]) __attribute__((always_inline)) {
+      const uint16_t *krow = pk_base + (size_t)min(j, nk - 1) * D + 8 * part;    // (beyond nk: the last one, masked below)
+#pragma unroll
+      for (int t = 0; t < NL; t++) raw[t] = *(const uint4 *)(krow + 32 * t);
+    };
+    uint4 next[NL];
+    load_k(c, next);
+    double qd[D / 4];
+    const uint16_t *qrow = pool_q + ((size_t)bh * nq + i) * D + 8 * part;
+#pragma unroll
+    for (int t = 0; t < NL; t++) {
+      const uint4 v = *(const uint4 *)(qrow + 32 * t);
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 8; e++) qd[8 * t + e] = (double)elem_to_f32<DT>((uint16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu)));
+    }
+#pragma unroll 1
+    for (int j = c; j < NKP; j += COLS) {
+      if (j - c >= causal_lim) {                        // uniform: no live column in this trip
+        if (part == 0) s_score[j] = NEG_INF;
+        continue;
+      }
+      uint4 kv[NL];
+#pragma unroll
+      for (int t = 0; t < NL; t++) kv[t] = next[t];
+      load_k(j + COLS, next);
+      const bool dead = j >= causal_lim || simk[min(j, nk - 1)] == 0;
+      double acc = 0.0;
+#pragma unroll
+      for (int t = 0; t < NL; t++) {
+        const uint32_t w[4] = {kv[t].x, kv[t].y, kv[t].z, kv[t].w};
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          acc = __builtin_fma(qd[8 * t + e], (double)elem_to_f32<DT>((uint16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu))), acc);
+      }
+      acc = group_sum_f64<4>(acc);
+      const float a1 = elem_to_f32<DT>(f64_to_elem_fast<DT>(acc));
+      const uint16_t a2 = f64_to_elem_fast<DT>((double)a1 * (double)sm_scale);
+      if (part == 0) s_score[j] = dead ? NEG_INF : a2;
+    }
+  }
+  if (tid < 64) s_lsum[tid] = 0.0;
+  __syncthreads();
+
+  // ---- exponentials: wavefront w holds columns 64 (w + NW p) + lane; the maximum is taken by every wavefront for itself
+  float lmax = -INFINITY;
+#pragma unroll
+  for (int t = 0; t < EPL; t++) lmax = fmaxf(lmax, elem_to_f32<DT>(s_score[64 * t + lane]));
+  const float mx = wave_max_f32(lmax);
+  double ev[P];
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    const int j = 64 * (wave + NW * p) + lane;
+    const float sc = elem_to_f32<DT>(s_score[j]);
+    ev[p] = (sc == -INFINITY) ? 0.0 : cexp((double)sc - (double)mx);
+    s_ev[j] = ev[p];
+  }
+  __syncthreads();
+  // the fixed summation tree: lane l adds e[l], e[l+64], ... in order, then an xor butterfly (32 .. 1)
+  double part = 0.0;
+#pragma unroll
+  for (int t = 0; t < EPL; t++) part = part + s_ev[64 * t + lane];
+  const double total = wave_tree_sum_f64(part);
+
+  // ---- probabilities -> sortable keys (the comment on the kernel above says why the product will do)
+  const double rtotal = total > 0.0 ? 1.0 / total : 0.0;
+  uint32_t okey[P], key[P];
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    const int j = 64 * (wave + NW * p) + lane;
+    okey[p] = j < nk ? ((probability_bits<DT>(ev[p], total, rtotal) << 16) | (0xffffu - (uint32_t)j)) : 0u;
+    key[p] = okey[p];
+  }
+  long long n;
+  uint32_t kth = 0u;
+  if (by_topk) {
+#pragma unroll
+    for (int p = 0; p < P; p++) s_run[64 * (wave + NW * p) + lane] = okey[p];
+    __syncthreads();
+    const float t = level.at(h) * (float)nk;            // binary32 product, truncated (utils.py:405)
+    n = (long long)t;
+    if (n <= 0) n = 1;                                  // utils.py:289
+    if (n < nk) {
+      uint32_t all[EPL];
+#pragma unroll
+      for (int t2 = 0; t2 < EPL; t2++) all[t2] = s_run[64 * t2 + lane];
+      kth = nth_largest_key<EPL>(all, (int)n);
+    }
+  } else {
+    bitonic_sort_desc<P, 2>(key, lane);                 // sorted position of key[p] is lane * P + p
+    uint32_t *run_w = s_run + RUN * wave;
+#pragma unroll
+    for (int p = 0; p < P; p++) run_w[lane * P + p] = key[p];
+    for (int x = tid; x < NKP; x += NT)                 // the keys fill the first nk places
+      if (x >= nk) s_sorted[x] = 0u;
+    __syncthreads();
+    // place of a key: its own in its run, plus the larger ones of every other run (keys below nk are distinct)
+    int pos[P];
+#pragma unroll
+    for (int p = 0; p < P; p++) pos[p] = lane * P + p;
+#pragma unroll
+    for (int o = 1; o < NW; o++) {
+      const uint32_t *r = s_run + RUN * ((wave + o) & (NW - 1));
+#pragma unroll
+      for (int p = 0; p < P; p++) {
+        int cnt = 0;
+#pragma unroll
+        for (int s = RUN / 2; s >= 1; s >>= 1) cnt += r[cnt + s - 1] > key[p] ? s : 0;
+        pos[p] += cnt + (r[cnt] > key[p] ? 1 : 0);      // cnt <= RUN - 1 here
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < P; p++)
+      if (key[p] != 0u) s_sorted[pos[p]] = key[p];
+    __syncthreads();
+    if (wave == 0) {
+      uint32_t sk[EPL];
+#pragma unroll
+      for (int t = 0; t < EPL; t++) sk[t] = s_sorted[lane * EPL + t];
+      // cdf[v] = T(sum_{u<=v} p_sorted[u]);  n = #{v < nk : cdf[v] <= threshold}  (utils.py:398-403)
+      double lsum = 0.0;
+#pragma unroll
+      for (int t = 0; t < EPL; t++) lsum += (double)elem_to_f32<DT>((uint16_t)(sk[t] >> 16));
+      s_lsum[64 + lane] = lsum;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      // the sums of the lanes before this one, in their order: the window of 64 that ends there, zeros first
+      double run = 0.0;
+#pragma unroll 16
+      for (int u = 0; u < 64; u++) run += s_lsum[lane + u];
+      const double thr = (double)level.at(h);
+      int cnt = 0;
+#pragma unroll
+      for (int t = 0; t < EPL; t++) {
+        run += (double)elem_to_f32<DT>((uint16_t)(sk[t] >> 16));
+        const float cdfv = elem_to_f32<DT>(f64_to_elem_fast<DT>(run));
+        cnt += __builtin_popcountll(__ballot(lane * EPL + t < nk && (double)cdfv <= thr));
+      }
+      if (cnt <= 0) cnt = 1;                            // utils.py:289
+      if (lane == 0) s_kth = cnt < nk ? s_sorted[cnt - 1] : 0u;
+    }
+    __syncthreads();
+    kth = s_kth;
+  }
+
+  // ---- block map row, delta LUT: a kept column's place is the number of kept ones before it, its step the distance to the last of them
+  const bool row_forced = sim_q[(size_t)bh * nq + i] == 0;
+  const size_t row_off = ((size_t)bh * nq + i) * nk;
+  uint64_t mine[P];
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    const int j = 64 * (wave + NW * p) + lane;
+    bool f = false;
+    if (j < nk) {
+      f = row_forced || (okey[p] >= kth) || (simk[j] == 0);
+      if (j >= causal_lim) f = false;
+      if (sink && j == 0) f = true;
+      if (bmap != nullptr) bmap[row_off + j] = f ? 1 : 0;
+    }
+    mine[p] = __ballot(f);
+    if (lane == 0) s_map[wave + NW * p] = mine[p];
+  }
+  __syncthreads();
+  int base = 0, last = 0;                               // kept columns so far, the last of them
+#pragma unroll
+  for (int t = 0; t < EPL; t++) {
+    const uint64_t m = s_map[t];
+    if ((t & (NW - 1)) == wave) {                       // columns of this wavefront
+      const uint64_t below = m & ((1ull << lane) - 1ull);
+      if ((m >> lane) & 1ull)
+        lut[row_off + base + __builtin_popcountll(below)] = 64 * t + lane - (below ? 64 * t + 63 - __builtin_clzll(below) : last);
+    }
+    base += __builtin_popcountll(m);
+    if (m) last = 64 * t + 63 - __builtin_clzll(m);
+  }
+  for (int x = tid; x < nk; x += NT)
+    if (x >= base) lut[row_off + x] = 0;
+  if (tid == 0) {
+    valid[(size_t)bh * nq + i] = base;
+    if (valid_out != nullptr) valid_out[(size_t)bh * nq + i] = base;
   }
 }
 
@@ -723,6 +947,21 @@ static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, 
   const int nkp = next_pow2_ge(nk, 256);
   if (nkp <= 2048) {
     // a whole row fits the registers of one wavefront
+    // A workgroup to a row where two of them per CU hold all rows; a whole call in us with the kernels below / with this (top-k 0.05,
+    // D=64): 256 rows nk 256 37.5 / 34.3, nk 512 57.2 / 49.8, nk 1875 145.1 / 118.9; 512 rows nk 141 44.5 / 42.8, nk 278 60.7 / 58.8, nk 1875
+    // 217.1 / 199.3; CDF, D=128: 64 rows nk 141 69.5 / 64.8, 512 rows nk 278 317.1 / 312.6.  With 640 rows it is down to +-1 %, with
+    // 1112 rows nk 278 (top-k, D=128) 321.6 / 334.2: a wavefront to a row does less in all.
+    if ((long long)nq * B * H <= 512) {
+#define SPG_BSR(EPL_)                                                                                                        \
+      block_select_row_kernel<D, DT, EPL_><<<dim3(nq, B * H), EPL_ == 4 ? 256 : 512, 0, st>>>(                               \
+          (const uint16_t *)pq, sq, (const uint16_t *)pk, sk, by_topk, level, causal, sink, lut, valid, valid_out, bmap, H, Hkv, nq, nk)
+      if (nkp == 256) SPG_BSR(4);
+      else if (nkp == 512) SPG_BSR(8);
+      else if (nkp == 1024) SPG_BSR(16);
+      else SPG_BSR(32);
+#undef SPG_BSR
+      return hipSuccess;
+    }
 #define SPG_BSW(NW_, EPL_, DUAL_, R_)                                                                                    \
     {                                                                                                           \
       const size_t lds = (size_t)R_ * nkp * 2 + (size_t)NW_ * nkp * 2 + NW_ * 64 * 8;                           \
@@ -737,8 +976,8 @@ static hipError_t launch_bs2(const void *pq, const uint8_t *sq, const void *pk, 
     }
     // Eight rows instead of sixteen per workgroup, one per wavefront, where sixteen leave a CU with little more than one
     // workgroup: the time is then that of one wavefront's rows, and the half-empty score tiles cost less than the second row.
-    // us with 16 / 8: 9 workgroups D=64 nk=278 CDF 28.0 / 18.1, 96 D=128 nk=128 15.3 / 10.4, 128 D=128 nk=256 25.4 / 16.9, 192 D=64
-    // nk=256 21.5 / 18.2, 270 D=64 nk=278 44.0 / 35.7, 49 D=128 nk=1563 130 / 85; 512 D=128 nk=512 46.6 / 64.1.
+    // us with 16 / 8: 96 workgroups D=128 nk=128 15.3 / 10.4, 128 D=128 nk=256 25.4 / 16.9, 192 D=64 nk=256 21.5 / 18.2, 270 D=64
+    // nk=278 44.0 / 35.7, 49 D=128 nk=1563 130 / 85; 512 D=128 nk=512 46.6 / 64.1.
     const bool few = (nq + 15) / 16 * B * H <= (D == 64 ? 384 : 256);
     if (nkp == 256) { if (few) SPG_BSW(8, 4, false, 8) else SPG_BSW(8, 4, false, 16) }
     if (nkp == 512) { if (few) SPG_BSW(8, 8, false, 8) else SPG_BSW(8, 8, false, 16) }
