@@ -468,17 +468,21 @@ class ForwardPlan:
             a.pvthreshd = pvthreshd.data_ptr()
         else:
             a.pvthreshd_value = pvthreshd
-        rc = self._lib.spg_sparse_attn(ctypes.addressof(a), torch._C._cuda_getCurrentRawStream(self.device_index))
-        if rc != SPG_OK:
-            _check(rc)
-        if not return_valid:
-            return None
         if early:
-            kept = self._lib.spg_wait_counts(valid.data_ptr(), valid.numel(), 2e-3)
+            try:
+                _check(self._lib.spg_sparse_attn(ctypes.addressof(a), torch._C._cuda_getCurrentRawStream(self.device_index)))
+                kept = self._lib.spg_wait_counts(valid.data_ptr(), valid.numel(), 2e-3)
+            except BaseException:          # (an interrupt from the keyboard, too: the kernel's stores must not outlive `valid`)
+                torch.cuda.current_stream(self.device).synchronize()
+                raise
             if kept >= 0:
                 return kept
             torch.cuda.current_stream(self.device).synchronize()
-        return int(valid.cpu().sum())
+            return int(valid.sum())
+        rc = self._lib.spg_sparse_attn(ctypes.addressof(a), torch._C._cuda_getCurrentRawStream(self.device_index))
+        if rc != SPG_OK:
+            _check(rc)
+        return int(valid.cpu().sum()) if return_valid else None
 
 
 def v_tiles_f16_swizzled(v, stream=None):

@@ -123,8 +123,6 @@ inline bool q_overwritten(const spg_attn_args *a, const Strides &qs, const Strid
   return q < out + bytes(os) && out < q + bytes(qs);
 }
 
-
-inline int split_env(const char *n, int d) { const char *e = getenv(n); return e ? atoi(e) : d; }
 // ---- rows in chunks (RowSplit) --------------------------------------------------------------------------------------
 // Blocks of a chunk, and where the scratch for it lies.  About two rounds of workgroups if every block is kept (D = 64 fits four to a CU, D =
 // 128 three), so that one round or more is left with half of them.  us per call with 512 / 768 / 1024 / 1536 / 2048 workgroups in all: one head

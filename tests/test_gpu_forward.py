@@ -242,3 +242,26 @@ def test_fp16_tiles_beside_the_blocks_of_k(H, N, Nk, D, vdtype):
     plan = _lib.ForwardPlan(q, k, v, got, mask, _lib.SELECT_MASK, True, False, False, False, 1, D ** -0.5)
     plan.run(q, k, v, got, mask, 0.0, 0.0, 50.0)
     assert torch.equal(_bits(got), _bits(o))
+
+
+def test_interrupted_wait_for_counts(monkeypatch):
+    """A call that is interrupted while it waits for its counts ends only after the kernels that store them."""
+    q, k, v = (rand_T((1, 8, 8192, 128), torch.bfloat16, s) for s in (1, 2, 3))
+    call = lambda: sa.spas_sage2_attn_meansim_topk_cuda(q, k, v, return_sparsity=True)  # noqa: E731
+    out, sparsity = call()
+
+    class Interrupted:
+        def __getattr__(self, name):
+            return getattr(_lib.load(), name)
+
+        def spg_wait_counts(self, *args):
+            raise KeyboardInterrupt
+    for plan in core._plans.values():
+        monkeypatch.setattr(plan, "_lib", Interrupted())
+    torch.cuda.synchronize()
+    with pytest.raises(KeyboardInterrupt):
+        call()
+    assert torch.cuda.current_stream().query()
+    monkeypatch.undo()
+    again, sparsity2 = call()
+    assert torch.equal(_bits(out), _bits(again)) and sparsity == sparsity2
