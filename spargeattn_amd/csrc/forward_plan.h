@@ -135,8 +135,12 @@ struct ChunkPlan {
 inline ChunkPlan chunk_plan(int B, int H, int N, int N_kv, int D) {
   ChunkPlan c = {1, 0, 0, 0, 0, 0, 0};
   const long long rows = (long long)B * H * ((N + 127) / 128), nk = (N_kv + 63) / 64;
-  if (rows > 256 || nk <= 36 || nk > 32768) return c;
-  const long long wgs = D == 64 ? 1536 : 1024, spread = (rows * nk + wgs - 1) / wgs, most = (nk + 63) / 64;   // (64 chunks: those of a row are added up one by one)
+  // (beyond 256 rows only for the sake of a partial last Q block, whose rows keep everything; beyond 1200 they would have two chunks: H12 N17776
+  // top-k 0.15, 1668 rows, D64 263 / 275, D128 351 / 391)
+  if (rows > (N % 128 != 0 ? 1200 : 256) || nk <= 36 || nk > 32768) return c;
+  // beyond 256 rows, us with 1536 / 3072 / 4608 workgroups, N17776: D64 H2 0.5 141 / 144 / 149, H4 0.15 143 / 129 / 132, 0.3 167 / 180 / 171, 0.5 247 / 223 / 233, H8 0.15 218 /
+  // 185 / 171; D128 H2 0.5 216 / 205 / 214, H4 0.15 179 / 149 / 176, 0.3 215 / 235 / 249, H6 0.15 283 / 222 / 205; N30001 H4 0.15 430 / 340 / 324
+  const long long wgs = rows > 256 ? 3072 : D == 64 ? 1536 : 1024, spread = (rows * nk + wgs - 1) / wgs, most = (nk + 63) / 64;   // (64 chunks: those of a row are added up one by one)
   c.per = (int)(spread > most ? spread : most);
   if (c.per < 16) c.per = 16;
   c.chunks = (int)((nk + c.per - 1) / c.per);
@@ -163,11 +167,20 @@ inline RowSplit row_split(const ChunkPlan &c, void *scratch) {
 inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, int selection, float share, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
   if (chunk_plan(B, H, N, N_kv, D).chunks == 1 || (selection != SPG_SELECT_MASK && nk <= SPG_SELECT_IN_ATTN_NK)) return false;
-  share = share < 0.f ? 0.5f : share < 1.f ? share : 1.f;
+  const bool many = B * H * nq > 256;
+  share = share < 0.f ? (many ? (D == 64 ? 0.75f : 0.65f) : 0.5f) : share < 1.f ? share : 1.f;
   const float kept = share * nk;
   const bool partial = N % 128 != 0 && selection != SPG_SELECT_MASK;
   const float longest = partial ? (float)nk : kept;
   const float all = (float)(B * H) * (nq * kept * (causal ? 1.f - 0.5f * share : 1.f) + (partial ? nk - kept : 0.f));
+  // Beyond 256 rows a row walks its blocks in one group, 0.7 us per block at D = 64 and 0.9 at D = 128, beside others or alone at the end.  us per
+  // call, workgroup per row / chunks, a partial last Q block.  N17776 D64: H2 top-k 0.15 231 / 96, 0.5 230 / 147, 0.7 243 / 180; H4 0.3 237 / 181, 0.5 254 / 227, 0.7 296 / 299; H6 0.3 243 /
+  // 229, 0.5 303 / 307; H8 0.15 246 / 186, 0.3 249 / 236; causal H2 0.5 230 / 138, H4 250 / 218, H8 293 / 317.  D128: H2 0.15 276 / 113, 0.5 279 / 207; H3 0.3 283 / 200, 0.7 301 / 347;
+  // H4 0.3 303 / 239, 0.5 323 / 337; H8 0.15 326 / 278, 0.3 354 / 366; causal H2 276 / 196, H4 308 / 322; FP16 PV H2 0.5 326 / 241, D64 243 / 152.  N8300 H6 0.15 D64 125 / 80, D128
+  // 154 / 107, 0.5 127 / 117 and 156 / 161; 2 heads of 30000 over 8400 0.15 119 / 66 and 145 / 84.  Where nothing says how much is kept it is often more than half (CDF
+  // 0.9 on N(0, 1) data, D64: H2 N17776 268 / 208, H4 338 / 342, H6 N8300 146 / 157), so more is taken for granted than in
+  // shorter grids.
+  if (many) return longest - all / (D == 64 ? 350.f : 220.f) > 45.f;
   return longest - all / 180.f > 36.f;
 }
 inline bool rows_in_chunks(const spg_attn_args *a) {

@@ -76,14 +76,19 @@ def test_grids_beyond_one_row_per_cu_have_no_groups(routes):
     (dict(H=8, N=128, Nk=64 * 132, level=0.2), 0), (dict(H=8, N=128, Nk=64 * 132, level=0.35), 1), (dict(H=8, N=1024, Nk=64 * 132, level=0.5), 1),
     (dict(H=8, N=2048, Nk=64 * 288, level=0.2), 0), (dict(H=8, N=2048, Nk=64 * 288, level=0.5), 1), (dict(H=8, N=22 * 128, Nk=64 * 512, level=1.0), 0),
     (dict(H=8, N=32 * 128, Nk=64 * 512, level=0.5), 0), (dict(N=17776, D=64, selection=CDF), 1), (dict(N=17776, level=0.5), 1), (dict(N=24000, causal=1), 1),
-    (dict(N=64 * 257, Nk=64 * 600, level=0.3), 1), (dict(N=8192 * 4, level=0.5), 0), (dict(N=128 * 256 + 1, level=0.5), 0),
+    (dict(N=64 * 257, Nk=64 * 600, level=0.3), 1), (dict(N=8192 * 4, level=0.5), 0), (dict(N=128 * 256 + 1, level=0.5), 1), (dict(N=128 * 257, level=0.5), 0),
+    # beyond 256 rows: a partial last Q block only, and not where the rest takes as long
+    (dict(H=4, N=17776, D=64, level=0.5), 1), (dict(H=4, N=17776, D=64, level=0.7), 0), (dict(H=4, N=17776, level=0.3), 1), (dict(H=4, N=17776, level=0.5), 0),
+    (dict(H=4, N=17792, D=64, level=0.5), 0), (dict(H=8, N=17776, D=64, level=0.15), 1), (dict(H=9, N=17776, D=64, level=0.15), 0), (dict(H=3, N=17776, D=64, selection=MASK), 0),
+    (dict(H=2, N=17776, selection=CDF), 1), (dict(H=2, N=17776, D=64, selection=CDF), 1), (dict(H=3, N=17776, D=64, selection=CDF), 0),
+   
     (dict(H=8, N=128, Nk=64 * 128, level=1.0), 0), (dict(H=8, N=128, Nk=64 * 128, selection=MASK), 1), (dict(H=2, N=128, Nk=64 * 36, selection=MASK), 0)])
 def test_few_long_rows_go_over_several_workgroups(routes, kw, chunks):
     assert routes(**kw)[7] == chunks
 
 
 def test_workspace_does_not_depend_on_the_level(routes):
-    for kw in (dict(H=8, N=128, Nk=64 * 132), dict(N=17776, D=64), dict(H=8, N=2048, Nk=64 * 288, pv_f16=1)):
+    for kw in (dict(H=8, N=128, Nk=64 * 132), dict(N=17776, D=64), dict(H=8, N=2048, Nk=64 * 288, pv_f16=1), dict(H=4, N=17776)):
         assert len({routes(level=level, **kw)[5] for level in (0.05, 0.5, 1.0)}) == 1
 
 
@@ -92,7 +97,10 @@ def test_chunks_of_a_row_are_bounded(routes, D, most):
     for H, N, nk in ((1, 1, 8192), (1, 128, 37), (8, 128, 2048), (1, 17776, 278), (2, 16384, 8192)):
         rows, n = H * -(-N // 128), routes(H=H, N=N, Nk=64 * nk, D=D, selection=MASK)[6]
         assert 1 < n <= 64 and n <= -(-nk // 16) and rows * (n - 1) <= most
-    assert routes(H=2, N=16385, Nk=64 * 512, D=D)[6] == 1
+    assert routes(H=2, N=128 * 129, Nk=64 * 512, D=D)[6] == routes(H=8, N=128 * 150 + 1, Nk=64 * 512, D=D)[6] == 1
+    for H, N, nk in ((2, 16385, 512), (8, 128 * 150 - 1, 8192), (8, 128 * 150 - 1, 129)):
+        rows, n = H * -(-N // 128), routes(H=H, N=N, Nk=64 * nk, D=D)[6]
+        assert 2 < n <= 64 and n <= -(-nk // 16) and rows * (n - 1) <= 3072
 
 
 @pytest.mark.parametrize("kw,wgs", [

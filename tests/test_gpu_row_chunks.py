@@ -24,8 +24,8 @@ def lists(B, H, nq, nk, lengths, g):
     return lut.cuda(), valid.cuda()
 
 
-# heads, Q blocks, K blocks, what is said of the lists: chunks of 16 blocks, and of more where rows are many or long
-@pytest.mark.parametrize("H,nq,nk,share", [(4, 9, 129, 1.0), (4, 9, 300, 1.0), (8, 27, 150, 0.05), (1, 2, 1100, 0.9)])
+# heads, Q blocks, K blocks, what is said of the lists: chunks of 16 blocks, and of more where rows are many or long (beyond 256 rows, and at their most)
+@pytest.mark.parametrize("H,nq,nk,share", [(4, 9, 129, 1.0), (4, 9, 300, 1.0), (8, 27, 150, 0.05), (1, 2, 1100, 0.9), (8, 33, 150, 0.05), (8, 150, 141, 0.05)])
 @pytest.mark.parametrize("D,dtype,f16v,gran,causal", [(64, torch.float16, False, 1, True), (128, torch.bfloat16, False, 2, False), (64, torch.bfloat16, True, 2, False),
                                                       (128, torch.float16, True, 1, True)])
 def test_chunks_equal_the_sequential_walk(D, dtype, f16v, gran, causal, H, nq, nk, share):
