@@ -38,7 +38,7 @@ RESOURCE_REMARKS = "-Rpass-analysis=kernel-resource-usage"
 # under matrix instructions).  In between, the compiler believes the destination registers are already written; the
 # generated code has to be free of copies or live-range splits inside those windows.  tests/test_lds_read_windows.py
 # disassembles the built kernels and follows every path through them: no instruction names a register of an LDS read
-# before the wait that covers it, in any of the 80 attention kernels or the two dense ones.  Another compiler
+# before the wait that covers it, in any of the attention kernels or the two dense ones.  Another compiler
 # may schedule differently: the build then says so, loudly, and asks for that test
 # (SPARGEATTN_AMD_ALLOW_UNVALIDATED_COMPILER=1 silences the failure, not the warning).
 VALIDATED_COMPILERS = ("roc-7.2.0",)

@@ -139,7 +139,8 @@ inline ChunkPlan chunk_plan(int B, int H, int N, int N_kv, int D) {
   // top-k 0.15, 1668 rows, D64 263 / 275, D128 351 / 391)
   if (rows > (N % 128 != 0 ? 1200 : 256) || nk <= 36 || nk > 32768) return c;
   // beyond 256 rows, us with 1536 / 3072 / 4608 workgroups, N17776: D64 H2 0.5 141 / 144 / 149, H4 0.15 143 / 129 / 132, 0.3 167 / 180 / 171, 0.5 247 / 223 / 233, H8 0.15 218 /
-  // 185 / 171; D128 H2 0.5 216 / 205 / 214, H4 0.15 179 / 149 / 176, 0.3 215 / 235 / 249, H6 0.15 283 / 222 / 205; N30001 H4 0.15 430 / 340 / 324
+  // 185 / 171; D128 H2 0.5 216 / 205 / 214, H4 0.15 179 / 149 / 176, 0.3 215 / 235 / 249, H6 0.15 283 / 222 / 205; N30001 H4 0.15 430 / 340 / 324.
+  // The sums of a chunk are 128 x D floats: at most 4300 of them, 280 MB at D = 128, whatever the lengths.
   const long long wgs = rows > 256 ? 3072 : D == 64 ? 1536 : 1024, spread = (rows * nk + wgs - 1) / wgs, most = (nk + 63) / 64;   // (64 chunks: those of a row are added up one by one)
   c.per = (int)(spread > most ? spread : most);
   if (c.per < 16) c.per = 16;
