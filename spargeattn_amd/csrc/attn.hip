@@ -1248,8 +1248,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
 // turn, place rd G + grp of the list in round rd: several CUs to a row instead of one, and a row of up to G blocks in one round.  Each wavefront has tiles of its own and the next ones
 // are requested as soon as the operands of the present ones are in registers; it meets the others once per round, to learn the
 // running maximum in front of its block (P is rounded against it), and at the end, where O and the denominators are added up in the order
-// of the groups.  No wavefront sees the votes of the row's other workgroups: for thresholds at which a skipped block leaves
-// every bit as it is (few_rows).  Arithmetic and masks are those of block_sparse_attn_kernel; at most 128 blocks to a row.
+// of the groups.  No wavefront sees the votes of the row's other workgroups, so each skips a block on the vote of its own 32 queries: it skips whatever
+// the whole row skips, whose V it then leaves alone, and at the thresholds of this route the rest as well adds nothing (few_rows).
+// Arithmetic and masks are those of block_sparse_attn_kernel; at most 128 blocks to a row.
 template <int D, int ODT, bool PV16, int SEL, int QW, int G>
 __global__ __launch_bounds__(64 * QW * G, 2) void few_rows_attn_kernel(const AttnParams p) {
   constexpr int KS = D / 32, NDT = D / 32, TILE = 64 * D, VTILE = PV16 ? 2 * TILE : TILE, NKL = TILE / 1024, NVL = VTILE / 1024, W = SEL > 0 ? SEL : 1;
@@ -1365,6 +1366,7 @@ __global__ __launch_bounds__(64 * QW * G, 2) void few_rows_attn_kernel(const Att
   for (int ks = 0; ks < KS; ks++) kaddr[ks] = lds_k + (uint32_t)(krow0 * D + ((hh ^ ksw) & 1) * 16) + ((uint32_t)(32 * ks) ^ (uint32_t)((ksw & 6) * 16));
   const uint32_t va_lo = lds_v + (uint32_t)(r * 64 + (((2 * hh) ^ v_swz(r)) * 16)), va_hi = va_lo ^ 16u;
   const uint32_t va16 = lds_v + (uint32_t)(r * 128 + (((4 * hh) ^ ((r >> 1) & 7)) * 16));
+  const float thr = p.pvthr.p != nullptr ? ((c_f32_t)p.pvthr.p)[head] : p.pvthr.v;
   const float c = p.sm_scale_log2, cq26 = c * qs * SPG_ACC_SCALE, acc_c = __builtin_bit_cast(float, (int)SPG_ACC_C_BITS);
   const int kscale_precise_bits = __builtin_bit_cast(int, 16384.0f / (acc_c * cq26));
   float m = SPG_NEG_BIG, m_own = SPG_NEG_BIG, dsum = hh == 0 && grp == 0 ? 1.0f : 0.0f;
@@ -1452,6 +1454,9 @@ __global__ __launch_bounds__(64 * QW * G, 2) void few_rows_attn_kernel(const Att
 #pragma unroll
           for (int e = 0; e < 16; e++) O[dt][e] *= osc;
       }
+      // (All scores not a number: skipped, as in block_sparse_attn_kernel.  Only what V and P enter is left out: a branch in front of the exponentials
+      // waits for the vote, one head N8192 D64 30.8 us per call without, 31.1 so, 32.0 with it there.)
+      const bool skip = place < nv - 2 && !__any(fm - before + thr > 0.f);
       const float neg0 = PV16 ? -m_new : -m_new + SPG_FP8_OFFSET;
       float x[32];
       if (!masked) {
@@ -1490,16 +1495,18 @@ __global__ __launch_bounds__(64 * QW * G, 2) void few_rows_attn_kernel(const Att
             pb16[s4][j + 1] = ph[1];
             rs = __builtin_amdgcn_fdot2(ph, ones2, rs, false);
           }
-        dsum += rs;
-        v4i t[4][NDT];
+        if (!skip) {
+          dsum += rs;
+          v4i t[4][NDT];
 #pragma unroll
-        for (int st = 0; st < 4; st++) {
-          const uint32_t a_ = va16 ^ (uint32_t)(16 * st);
-          if constexpr (NDT == 4) { lds_read_4x128<0, 4096, 8192, 12288>(t[st][0], t[st][1], t[st][2], t[st][3], a_); lds_wait4(t[st][0], t[st][1], t[st][2], t[st][3]); }
-          else { lds_read_2x128<0, 4096>(t[st][0], t[st][1], a_); lds_wait2(t[st][0], t[st][1]); }
+          for (int st = 0; st < 4; st++) {
+            const uint32_t a_ = va16 ^ (uint32_t)(16 * st);
+            if constexpr (NDT == 4) { lds_read_4x128<0, 4096, 8192, 12288>(t[st][0], t[st][1], t[st][2], t[st][3], a_); lds_wait4(t[st][0], t[st][1], t[st][2], t[st][3]); }
+            else { lds_read_2x128<0, 4096>(t[st][0], t[st][1], a_); lds_wait2(t[st][0], t[st][1]); }
 #pragma unroll
-          for (int dt = 0; dt < NDT; dt++)
-            O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, t[st][dt]), pb16[st], O[dt], 0, 0, 0);
+            for (int dt = 0; dt < NDT; dt++)
+              O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, t[st][dt]), pb16[st], O[dt], 0, 0, 0);
+          }
         }
         if (more) load_v(blk1);
       } else {
@@ -1514,7 +1521,6 @@ __global__ __launch_bounds__(64 * QW * G, 2) void few_rows_attn_kernel(const Att
 #pragma unroll
           for (int e = 1; e < 32; e++) ps += x[e];
         }
-        dsum += ps;
         v8i pb;
 #pragma unroll
         for (int u = 0; u < 8; u++) pb[u] = pack4_e4m3(x[4 * u], x[4 * u + 1], x[4 * u + 2], x[4 * u + 3]);
@@ -1526,10 +1532,13 @@ __global__ __launch_bounds__(64 * QW * G, 2) void few_rows_attn_kernel(const Att
           lds_read_4x128_wait<0, 2048>(lo[0], lo[1], hi[0], hi[1], va_lo, va_hi);
         }
         if (more) load_v(blk1);
+        if (!skip) {
+          dsum += ps;
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) {
-          const v8i av = {lo[dt][0], lo[dt][1], lo[dt][2], lo[dt][3], hi[dt][0], hi[dt][1], hi[dt][2], hi[dt][3]};
-          O[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, pb, O[dt], 0, 0, 0, 0, 0, 0);
+          for (int dt = 0; dt < NDT; dt++) {
+            const v8i av = {lo[dt][0], lo[dt][1], lo[dt][2], lo[dt][3], hi[dt][0], hi[dt][1], hi[dt][2], hi[dt][3]};
+            O[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, pb, O[dt], 0, 0, 0, 0, 0, 0);
+          }
         }
       }
     }

@@ -197,9 +197,11 @@ inline bool rows_in_chunks(const spg_attn_args *a) {
 // two: D64 128 x 8 13.6 / 13.7, 15.2 / 14.5, 17.3 / 14.8; 128 x 16 16.6 / 15.8, 19.3 / 17.2, 22.6 / 19.5, 128 x 128 45.2 / 40.2, 62.5 / 55.3, 91.6 / 78.5, 160 x 32 21.5 / 27.9,
 // 27.5 / 34.5, 34.5 / 45.7; D128 128 x 8 16.7 / 17.6, 19.7 / 18.6, 22.3 / 20.0, 128 x 16 23.1 / 22.2, 26.7 / 24.7, 31.5 / 28.3, 128 x 128 54.3 / 49.5, 78.8 / 68.2, 116.5 /
 // 99.0; FP16 PV at D128, whose tiles leave room for three groups, 128 x 64 38.0 / 37.5, 53.9 / 54.1, 77.4 / 77.6.
-// The workgroups of a row do not see each other's votes on the PV threshold, so it has to be one that no vote can change a bit by: a block is skipped
-// when all its scores are `pvthreshd` below the running maxima in the exponent of 2, so from 45 on its P are zero in e4m3 and in fp16, and
-// what they add to the denominator is below 2^-40 of it.  (A per-head threshold is not known here: 0.)
+// The workgroups of a row do not see each other's votes on the PV threshold.  A block is skipped when all scores of the Q block are `pvthreshd`
+// below the running maxima in the exponent of 2; the quarter (half) of a workgroup alone may be that far below where the others are not, and then skips a
+// block that the row keeps.  So the threshold has to be one at which that changes next to nothing: from 45 on, P of such a block is zero in e4m3
+// and in fp16, so O stays as it is, and what is left out of a query's denominator is at most 64 x 2^-45 = 2^-39 of it per block, 2^-32
+// for 126 of them, below the rounding of its sum in binary32.  (A per-head threshold is not known here: 0.)
 inline int few_rows(int B, int H, int N, int N_kv, int D, bool pv_f16, float pvthreshd) {
   const long long rows = (long long)B * H * ((N + 127) / 128), nk = (N_kv + 63) / 64;
   if (!(pvthreshd >= 45.f) || nk > 128) return 0;

@@ -59,6 +59,51 @@ def test_equal_the_sequential_walk(D, dtype, f16v, gran, causal, H, N, nk):
     assert (o - w).norm() <= 3e-4 * w.norm() * (1 if dtype == torch.float16 else 8)
 
 
+# four workgroups to a row and two; the smallest threshold of the route and the usual one
+@pytest.mark.parametrize("H,N,nk", [(2, 256, 9), (8, 1920, 30)])
+@pytest.mark.parametrize("D,f16v", [(64, False), (128, False), (64, True), (128, True)])
+@pytest.mark.parametrize("thr", [45.0, 50.0])
+def test_a_skipped_block_is_not_touched(D, f16v, thr, H, N, nk):
+    """What stands in V of a block that the PV threshold skips for every query, or a K scale that is not finite, changes nothing, as in the walk."""
+    g = torch.Generator().manual_seed(nk)
+    B, nq, Nk = 1, (N + 127) // 128, 64 * nk
+    selected = (_lib.SELECT_MASK, None, False, thr)
+    if _lib.few_rows_route((B, H, N, D), Nk, f16v, selected)[0] != _lib.ROWS_BY_QUERIES:
+        assert f16v and D == 128 and H * nq > 64
+        pytest.skip("FP16 PV at D = 128: up to 64 rows")
+    # scores of blocks 0, 4, 8, ... are 0.002 * 64 * 60^2 * 0.125 * log2(e) = 83 (D = 128: 117) to 5 % more, those of the others minus as much
+    q8 = torch.randint(60, 62, (B, H, N, D), generator=g, dtype=torch.int8)
+    k8 = torch.randint(60, 62, (B, H, Nk, D), generator=g, dtype=torch.int8)
+    sign = torch.where(torch.arange(nk) % 4 == 0, 1, -1).to(torch.int8).repeat_interleave(64)
+    k8 *= sign[None, None, :, None]
+    qs, ks = torch.full((B, H, nq), 0.1), torch.full((B, H, nk), 0.02)
+    v = torch.randn((B, H, Nk, D), generator=g).to(torch.float16)
+    v[:, :, 64 * 1 + 3, 5] = float("nan")
+    if f16v:                                            # (with FP8 PV an infinity is the scale of its channel)
+        v[:, :, 64 * 2 + 60, 1] = float("inf")
+        v[:, 0, 64 * 5] = float("-inf")
+    ks[:, :, 6], k8[:, :, 64 * 6:64 * 7] = float("inf"), 0            # (what a block with an infinity in it is quantised to)
+    q8, k8, qs, ks, v = (t.cuda() for t in (q8, k8, qs, ks, v))
+    lut, valid = torch.ones((B, H, nq, nk), dtype=torch.int32), torch.full((B, H, nq), nk, dtype=torch.int32)
+    lut[..., 0] = 0
+    lut, valid, pv = lut.cuda(), valid.cuda(), torch.full((H,), thr, device="cuda")
+
+    def run(count):
+        o = torch.empty((B, H, N, D), dtype=torch.float16, device="cuda")
+        if f16v:
+            return o, _lib.block_sparse_attn_f16v(q8, k8, _lib.v_tiles_f16_swizzled(v), o, lut, valid, pv, qs, ks, D ** -0.5,
+                                                  return_pv_count=count, selected=selected)
+        v8, vs = _lib.v_quant_fp8(v)
+        return o, _lib.block_sparse_attn(q8, k8, v8, o, lut, valid, pv, qs, ks, vs, D ** -0.5, return_pv_count=count, selected=selected)
+
+    want, count = run(True)
+    got, _ = run(False)
+    # blocks 0, 4, 8, ... and the last two of the row
+    assert (count == len({b for b in range(nk) if b % 4 == 0} | {nk - 2, nk - 1})).all() and want.isfinite().all()
+    w, o = want.double(), got.double()
+    assert ((o - w).abs() <= 2.0 ** -10 * w.abs() + 1e-5 * w.abs().max()).all()
+
+
 @pytest.mark.parametrize("H,N,Nk", [(3, 129, 64 * 6), (3, 700, 64 * 64 - 3), (2, 1025, 64 * 65), (9, 1025, 64 * 128 - 1), (2, 128, 64 * 100)])
 @pytest.mark.parametrize("D,f16v", [(64, False), (128, False), (64, True), (128, True)])
 def test_selection_in_place_equals_the_stages(D, f16v, H, N, Nk):
