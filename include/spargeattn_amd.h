@@ -174,15 +174,16 @@ int spg_block_sparse_attn_f16v(const int8_t *q8, const int8_t *k8, const void *v
 /* ---- the two above for few rows (up to 256 Q blocks in all), whose work is spread over several workgroups to a row.
  * spg_few_rows_route says how the whole-operator call below takes such a call: every row in one workgroup (the functions above), by its
  * queries (short rows), or by its blocks (long ones; *workspace_bytes of device scratch).  selection as in spg_attn_args, share the top-k
- * fraction or a negative number if there is none, is_causal the selection's, pvthreshd the threshold if it is one number for all heads, else 0.
+ * fraction or a negative number if there is none, is_causal the selection's, simthreshd1 and pvthreshd the thresholds where they are one number for
+ * all heads, else 0.
  * spg_block_sparse_attn_few_rows: v and v_scale as for spg_block_sparse_attn, or, with v_scale == NULL, v as for spg_block_sparse_attn_f16v;
  * the PV threshold is per block, and by queries it is taken to be 45 or more: the 32 queries of a wavefront skip a block for themselves, whatever the
  * others of the Q block vote, and what that leaves out is P that rounds to zero, at most 2^-32 of the denominator in all.  The running maxima that P
  * is rounded against are those of the block-by-block walk, by blocks the skipped blocks, too; O and the denominator are summed in another order.  Results
  * are those of the whole-operator call, bit for bit.  workspace 256-byte aligned. */
 enum spg_rows { SPG_ROWS_ONE_WORKGROUP = 0, SPG_ROWS_BY_QUERIES = 1, SPG_ROWS_BY_BLOCKS = 2 };
-int spg_few_rows_route(int B, int H, int N, int N_kv, int D, int pv_f16, int selection, float share, int is_causal, float pvthreshd,
-                       uint64_t *workspace_bytes);
+int spg_few_rows_route(int B, int H, int N, int N_kv, int D, int pv_f16, int selection, float share, float simthreshd1, int is_causal,
+                       float pvthreshd, uint64_t *workspace_bytes);
 int spg_block_sparse_attn_few_rows(const int8_t *q8, const int8_t *k8, const void *v, void *out, const int64_t *out_strides,
                                    int out_dtype, const int32_t *lut, const int32_t *valid_block_num, const float *pvthreshd,
                                    const float *q_scale, const float *k_scale, const float *v_scale,

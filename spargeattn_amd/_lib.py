@@ -41,7 +41,7 @@ SIGNATURES = {
     "spg_block_sparse_attn": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _vp, _vp]),
     "spg_v_tiles_f16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "spg_block_sparse_attn_f16v": (_i, [_vp] * 5 + [_i] + [_vp] * 5 + [_i] * 6 + [_f, _i, _i, _i, _vp, _vp]),
-    "spg_few_rows_route": (_i, [_i] * 7 + [_f, _i, _f, _vp]),
+    "spg_few_rows_route": (_i, [_i] * 7 + [_f, _f, _i, _f, _vp]),
     "spg_block_sparse_attn_few_rows": (_i, [_vp] * 5 + [_i] + [_vp] * 6 + [_i] * 6 + [_f, _i, _i, _i, _vp, _c.c_uint64, _vp]),
     "spg_wait_counts": (_c.c_int64, [_vp, _c.c_int64, _c.c_double]),
     "spg_sparse_attn_workspace_bytes": (_sz, [_vp]),
@@ -344,12 +344,14 @@ def _check_attn_shapes(q8, k8, vt, lut, valid, q_scale, k_scale, v_scale=None, q
 
 
 def few_rows_route(shape, Nk, pv_f16, selected):
-    """(route, scratch bytes) of spg_few_rows_route.  selected: (selection, top-k fraction or None, causal, PV threshold or None)."""
+    """(route, scratch bytes) of spg_few_rows_route.  selected: (selection, top-k fraction or None, causal, PV threshold or None) and, with a similarity
+    threshold of 0 or more or one per head, that threshold or None."""
     B, H, N, D = shape
-    selection, share, causal, pvthreshd = selected
+    selection, share, causal, pvthreshd, simthreshd1 = selected if len(selected) == 5 else (*selected, -1.0)
     size = ctypes.c_uint64(0)
     # (a negative share means that nothing is known, so 0 stays 0)
-    route = load().spg_few_rows_route(B, H, N, Nk, D, int(pv_f16), selection, -1.0 if share is None else max(float(share), 0.0), int(bool(causal)),
+    route = load().spg_few_rows_route(B, H, N, Nk, D, int(pv_f16), selection, -1.0 if share is None else max(float(share), 0.0),
+                                      0.0 if simthreshd1 is None else float(simthreshd1), int(bool(causal)),
                                       0.0 if pvthreshd is None else float(pvthreshd), ctypes.addressof(size))
     return route, size.value
 

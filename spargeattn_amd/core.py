@@ -119,9 +119,10 @@ def _number(value):
     return float(value) if type(value) in (float, int) or (isinstance(value, torch.Tensor) and value.dim() == 0) else None
 
 
-def _selected(cdfthreshd, topk, is_causal, pvthreshd):
+def _selected(cdfthreshd, topk, is_causal, simthreshd1, pvthreshd):
     """What _lib.block_sparse_attn wants to know of the call to take its rows as the whole-operator call does."""
-    return (_lib.SELECT_CDF, None, is_causal, _number(pvthreshd)) if topk is None else (_lib.SELECT_TOPK, _number(topk), is_causal, _number(pvthreshd))
+    selection, share = (_lib.SELECT_CDF, None) if topk is None else (_lib.SELECT_TOPK, _number(topk))
+    return selection, share, is_causal, _number(pvthreshd), _number(simthreshd1)
 
 
 def _staged_meansim(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, topk, pvthreshd, attention_sink,
@@ -134,7 +135,7 @@ def _staged_meansim(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, topk, pv
         q, k, km, is_causal=is_causal, simthreshd1=simthreshd1, cdfthreshd=cdfthreshd, topk=topk, return_lut=True,
         attention_sink=attention_sink, BLKQ=128, BLKK=64, qk_quant_gran=qk_quant_gran)
     o, _ = _attention(q, k, v, q_int8, q_scale, k_int8, k_scale, lut, valid_block_num, scale, pvthreshd, kernel_causal,
-                      qk_quant_gran=qk_quant_gran, selected=_selected(cdfthreshd, topk, is_causal, pvthreshd))
+                      qk_quant_gran=qk_quant_gran, selected=_selected(cdfthreshd, topk, is_causal, simthreshd1, pvthreshd))
     return _finish(o, tensor_layout, return_sparsity, valid_block_num, lut, causal_denominator=is_causal is not False)
 
 
@@ -153,7 +154,7 @@ def _staged_meansim_sage1(q, k, v, is_causal, scale, simthreshd1, cdfthreshd, to
     if scale is None:
         scale = 1.0 / (headdim ** 0.5)
     assert headdim in [64, 128], "headdim should be in [64, 128]. For other headdim, you can use padding and specify the softmax scale."
-    selected = _selected(cdfthreshd, topk, is_causal, pvthreshd)
+    selected = _selected(cdfthreshd, topk, is_causal, simthreshd1, pvthreshd)
     pvthreshd = hyperparameter_check(pvthreshd, q.size(-3), q.device)
     o = _empty_out(q)
     _mark("vquant")

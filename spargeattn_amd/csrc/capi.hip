@@ -196,13 +196,13 @@ int spg_block_sparse_attn_f16v(const int8_t *q8, const int8_t *k8, const void *v
                                                         pv_threshold_mode, pv_count, (hipStream_t)stream));
 }
 
-int spg_few_rows_route(int B, int H, int N, int N_kv, int D, int pv_f16, int selection, float share, int is_causal, float pvthreshd,
-                       uint64_t *workspace_bytes) {
+int spg_few_rows_route(int B, int H, int N, int N_kv, int D, int pv_f16, int selection, float share, float simthreshd1, int is_causal,
+                       float pvthreshd, uint64_t *workspace_bytes) {
   const char *fn = "spg_few_rows_route";
   if (workspace_bytes != nullptr) *workspace_bytes = 0;
   if (check_shape(fn, B, H, N, D) != SPG_OK || check_shape(fn, B, H, N_kv, D) != SPG_OK) return SPG_ROWS_ONE_WORKGROUP;
   if (few_rows(B, H, N, N_kv, D, pv_f16 != 0, pvthreshd) > 0) return SPG_ROWS_BY_QUERIES;
-  if (!rows_in_chunks(B, H, N, N_kv, D, selection, share, is_causal != 0)) return SPG_ROWS_ONE_WORKGROUP;
+  if (!rows_in_chunks(B, H, N, N_kv, D, pv_f16 != 0, selection, share, simthreshd1, is_causal != 0)) return SPG_ROWS_ONE_WORKGROUP;
   if (workspace_bytes != nullptr) *workspace_bytes = chunk_plan(B, H, N, N_kv, D).bytes;
   return SPG_ROWS_BY_BLOCKS;
 }

@@ -165,13 +165,33 @@ inline RowSplit row_split(const ChunkPlan &c, void *scratch) {
 // 1.0 182 / 175; 224 x 512 1.0 321 / 332.  D128 8 x 132 0.2 58.5 / 63.6, 0.35 72.3 / 66.8; 64 x 512 0.1 128.7 / 133.4, 0.5 251 / 169; 128 x 288 0.35 134 /
 // 132, 0.5 161 / 143; 176 x 512 1.0 405 / 423; FP16 PV 64 x 288 0.2 107.5 / 95.3, 160 x 288 0.5 184 / 175, 256 x 288 0.5 198 / 217.  With a partial last
 // block: N24000, 188 rows, top-k 0.5 D64 207 / 145, D128 265 / 190, causal 207 / 140; N28000 D128 310 / 231; one head N17776 CDF 171 / 136.
-inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, int selection, float share, bool causal) {
+// Everything kept, with a partial last Q block: the longest row is as long as ever and the chunks have the most to do, so they pay nowhere less.  A
+// workgroup per row takes 0.48 (D = 64), 0.62 (D = 128) and 0.74 us (FP16 PV) per block of a row in groups, and 0.9 and 1.1 us in one group beyond 256
+// rows; causal rows, half as many blocks, save a tenth of the chunks' time only, since a chunk is as long as in a full row.  us per call, workgroup
+// per row / chunks, on both sides of the line, rows x nk:
+//            up to 256 rows                                              beyond
+// D64        188 x 376 215 / 192, 204 x 407 231 / 222, 252 x 251 156 / 185   376 x 376 375 / 339, 417 x 278 291 / 297, 390 x 130 157 / 166
+// causal     219 x 438 241 / 231, 235 x 469 257 / 260, 252 x 251 154 / 160   417 x 278 256 / 236, 556 x 278 283 / 283, 469 x 938 819 / 830
+// D128       157 x 313 242 / 218, 172 x 344 262 / 262, 204 x 407 300 / 348   278 x 278 359 / 336, 298 x 297 380 / 374, 376 x 376 465 / 518
+// causal     172 x 344 258 / 237, 188 x 376 274 / 269, 204 x 407 293 / 317   298 x 297 338 / 312, 330 x 329 372 / 358, 417 x 278 320 / 346
+// FP16 D64   172 x 344 206 / 190, 188 x 376 224 / 219, 204 x 407 238 / 245   376 x 376 396 / 379, 417 x 278 307 / 333, 470 x 469 487 / 574
+// FP16 D128  157 x 313 288 / 252, 172 x 344 314 / 303, 204 x 407 362 / 405   266 x 532 712 / 651, 278 x 278 400 / 398, 298 x 297 425 / 440
+inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool causal) {
+  const float all = (float)rows * nk * (causal ? 0.9f : 1.f);
+  if (rows > 256) return nk - all / (D == 64 ? 420.f : pv_f16 ? 290.f : 320.f) > 27.f;
+  return nk - all / (D == 128 ? 185.f : pv_f16 ? 200.f : 220.f) > 36.f;
+}
+// simthreshd1: blocks of Q and K whose similarity is below it keep everything.  A similarity is not negative, so below 0 it changes nothing and
+// a row keeps what top-k names; from 0 on a row may keep all of its blocks, and nothing on the host says how many do (H8 N17776 top-k 0.15 at 0.6, no block
+// similar: workgroup per row / chunks D64 578 / 661 us, D128 831 / 1041).
+inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, int selection, float share, float simthreshd1, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
   if (chunk_plan(B, H, N, N_kv, D).chunks == 1 || (selection != SPG_SELECT_MASK && nk <= SPG_SELECT_IN_ATTN_NK)) return false;
   const bool many = B * H * nq > 256;
   share = share < 0.f ? (many ? (D == 64 ? 0.75f : 0.65f) : 0.5f) : share < 1.f ? share : 1.f;
   const float kept = share * nk;
   const bool partial = N % 128 != 0 && selection != SPG_SELECT_MASK;
+  if (partial && selection == SPG_SELECT_TOPK && !(simthreshd1 < 0.f) && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
   const float longest = partial ? (float)nk : kept;
   const float all = (float)(B * H) * (nq * kept * (causal ? 1.f - 0.5f * share : 1.f) + (partial ? nk - kept : 0.f));
   // Beyond 256 rows a row walks its blocks in one group, 0.7 us per block at D = 64 and 0.9 at D = 128, beside others or alone at the end.  us per
@@ -186,7 +206,7 @@ inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, int selection, 
 }
 inline bool rows_in_chunks(const spg_attn_args *a) {
   const float share = a->selection == SPG_SELECT_TOPK && a->level == nullptr ? (a->level_value > 0.f ? a->level_value : 0.f) : -1.f;
-  return rows_in_chunks(a->B, a->H, a->N, a->N_kv, a->D, a->selection, share, a->is_causal != 0);
+  return rows_in_chunks(a->B, a->H, a->N, a->N_kv, a->D, a->pv_f16 != 0, a->selection, share, a->simthreshd1 == nullptr ? a->simthreshd1_value : 0.f, a->is_causal != 0);
 }
 
 // Few short rows: workgroups to a row (few_rows_attn_kernel), or 0 where it has one.  Four while each has a CU to itself, two up to 128 rows; the

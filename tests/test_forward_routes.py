@@ -5,6 +5,9 @@ import os
 import subprocess
 
 import pytest
+import torch
+
+from spargeattn_amd import _lib, core
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -85,6 +88,22 @@ def test_grids_beyond_one_row_per_cu_have_no_groups(routes):
     (dict(H=8, N=128, Nk=64 * 128, level=1.0), 0), (dict(H=8, N=128, Nk=64 * 128, selection=MASK), 1), (dict(H=2, N=128, Nk=64 * 36, selection=MASK), 0)])
 def test_few_long_rows_go_over_several_workgroups(routes, kw, chunks):
     assert routes(**kw)[7] == chunks
+
+
+# Top-k with a similarity threshold of 0 or more may keep every block: in chunks only where that pays with all of them, too.
+@pytest.mark.parametrize("kw,chunks", [
+    (dict(H=8, N=17776, D=64, level=0.15), 0), (dict(H=4, N=17776, D=64, level=0.3), 0), (dict(H=6, N=8300, D=64, level=0.15), 0), (dict(H=2, N=17776, D=64, level=0.15), 1),
+    (dict(H=8, N=17776, level=0.15), 0), (dict(H=2, N=17776, level=0.15), 1), (dict(N=17776, level=0.15), 1), (dict(N=30000, level=0.15), 0), (dict(N=30000, D=64, level=0.15), 0),
+    (dict(N=24001, D=64, level=0.5), 1), (dict(N=24001, D=64, level=0.5, pv_f16=1), 0), (dict(N=24001, level=0.5), 0), (dict(N=28001, D=64, level=0.5, causal=1), 1),
+    (dict(H=2, N=17776, level=0.15, pv_f16=1), 0), (dict(H=8, N=1024, Nk=64 * 288, level=0.5), 1)])
+def test_a_similarity_threshold_may_keep_everything(routes, kw, chunks):
+    assert routes(sim=0.0, **kw)[7] == chunks == routes(sim=0.6, **kw)[7] == routes(sim="nan", **kw)[7]
+    assert routes(sim=-0.1, **kw)[7] == 1
+    if os.path.exists(_lib.LIB_PATH):           # the stage-by-stage path takes the same route
+        shape, causal, pv_f16 = (1, kw.get("H", 1), kw["N"], kw.get("D", 128)), bool(kw.get("causal")), bool(kw.get("pv_f16"))
+        for sim, want in ((0.0, chunks), (None, chunks), (-0.1, 1)):
+            got = _lib.few_rows_route(shape, kw.get("Nk", kw["N"]), pv_f16, core._selected(None, kw["level"], causal, torch.zeros(2) if sim is None else sim, 50.0))
+            assert got[0] == (_lib.ROWS_BY_BLOCKS if want else _lib.ROWS_ONE_WORKGROUP)
 
 
 def test_workspace_does_not_depend_on_the_level(routes):
