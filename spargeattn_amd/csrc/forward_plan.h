@@ -183,15 +183,17 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 }
 // simthreshd1: blocks of Q and K whose similarity is below it keep everything.  A similarity is not negative, so below 0 it changes nothing and
 // a row keeps what top-k names; from 0 on a row may keep all of its blocks, and nothing on the host says how many do (H8 N17776 top-k 0.15 at 0.6, no block
-// similar: workgroup per row / chunks D64 578 / 661 us, D128 831 / 1041).
+// similar: workgroup per row / chunks D64 578 / 661 us, D128 831 / 1041).  Nor does it for a CDF threshold or a level per head (CDF 0.93 at 0.3,
+// causal, one head N31595 D128 342 / 438; 0.82 at 0.6 N31887 with FP16 PV 457 / 531).
 inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, int selection, float share, float simthreshd1, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
   if (chunk_plan(B, H, N, N_kv, D).chunks == 1 || (selection != SPG_SELECT_MASK && nk <= SPG_SELECT_IN_ATTN_NK)) return false;
   const bool many = B * H * nq > 256;
+  const bool exact = selection == SPG_SELECT_TOPK && share >= 0.f && simthreshd1 < 0.f;
   share = share < 0.f ? (many ? (D == 64 ? 0.75f : 0.65f) : 0.5f) : share < 1.f ? share : 1.f;
   const float kept = share * nk;
   const bool partial = N % 128 != 0 && selection != SPG_SELECT_MASK;
-  if (partial && selection == SPG_SELECT_TOPK && !(simthreshd1 < 0.f) && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
+  if (partial && !exact && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
   const float longest = partial ? (float)nk : kept;
   const float all = (float)(B * H) * (nq * kept * (causal ? 1.f - 0.5f * share : 1.f) + (partial ? nk - kept : 0.f));
   // Beyond 256 rows a row walks its blocks in one group, 0.7 us per block at D = 64 and 0.9 at D = 128, beside others or alone at the end.  us per

@@ -106,6 +106,15 @@ def test_a_similarity_threshold_may_keep_everything(routes, kw, chunks):
             assert got[0] == (_lib.ROWS_BY_BLOCKS if want else _lib.ROWS_ONE_WORKGROUP)
 
 
+# So may a CDF threshold.  (A level per head is a negative share to the rule, as a CDF threshold is.)
+@pytest.mark.parametrize("kw,chunks", [
+    (dict(N=31595, causal=1), 0), (dict(N=31887, causal=1, pv_f16=1), 0), (dict(N=30000, D=64), 0), (dict(N=24001, D=64), 1), (dict(N=17776), 1), (dict(N=24001), 0),
+    (dict(H=2, N=40573, D=64, causal=1), 0), (dict(H=2, N=24001, D=64), 1), (dict(H=2, N=17776, pv_f16=1), 0), (dict(N=24064), 0), (dict(N=12800), 1), (dict(H=8, N=1024, Nk=64 * 288), 1)])
+def test_a_cdf_threshold_may_keep_everything(routes, kw, chunks):
+    for sim in (-0.1, 0.6):
+        assert routes(selection=CDF, sim=sim, **kw)[7] == chunks
+
+
 def test_workspace_does_not_depend_on_the_level(routes):
     for kw in (dict(H=8, N=128, Nk=64 * 132), dict(N=17776, D=64), dict(H=8, N=2048, Nk=64 * 288, pv_f16=1), dict(H=4, N=17776)):
         assert len({routes(level=level, **kw)[5] for level in (0.05, 0.5, 1.0)}) == 1
