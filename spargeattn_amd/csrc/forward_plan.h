@@ -187,12 +187,19 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 // causal, one head N31595 D128 342 / 438; 0.82 at 0.6 N31887 with FP16 PV 457 / 531).
 inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, int selection, float share, float simthreshd1, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
-  if (chunk_plan(B, H, N, N_kv, D).chunks == 1 || (selection != SPG_SELECT_MASK && nk <= SPG_SELECT_IN_ATTN_NK)) return false;
+  if (chunk_plan(B, H, N, N_kv, D).chunks == 1 || nk <= SPG_SELECT_IN_ATTN_NK) return false;
   const bool many = B * H * nq > 256;
+  // A mask: its density is known on the device only, and a sparse one leaves a row one or two chunks, which the two launches more then cost for
+  // nothing.  So the line is where a density of 0.1 loses next to nothing.  us per call, workgroup per row / chunks, at 0.1, 0.15 and 0.6: D64 71 x 141 30.3 / 34.5, 30.7
+  // / 35.9 and 61.6 / 43.9, 125 x 250 39.7 / 45.5, 46.3 / 47.8 and 99.0 / 78.2, 64 x 192 43.6 / 48.3, 50.0 / 49.3 and 90.9 / 60.1, 64 x 256 50.9 / 51.6, 56.9 / 52.5 and 112.3 /
+  // 69.2, 96 x 938 98.3 / 99.1, 126 x 938 92.1 / 103.2; D128 71 x 141 36.4 / 45.5 and 85.3 / 58.4, 8 x 256 66.3 / 68.8, 73.2 / 68.1 and 145.2 / 72.2, 64 x 256 70.8 / 71.3, 79.8 / 72.4
+  // and 152.7 / 100.4, 96 x 938 142.1 / 165.7; at 0.1 the ratio over 256 / 400 / 1024 K blocks D64 8 rows 0.97 / 1.05 / 1.41, 64 rows 0.98 / 1.08 / 1.19, D128 8 rows 0.96 /
+  // 1.17 / 1.30, 64 rows 0.97 / 1.02 / 1.02, 75 rows 0.97 / 0.98 / 1.01.
+  if (selection == SPG_SELECT_MASK) return B * H * nq <= 64 && nk >= 256;
   const bool exact = selection == SPG_SELECT_TOPK && share >= 0.f && simthreshd1 < 0.f;
   share = share < 0.f ? (many ? (D == 64 ? 0.75f : 0.65f) : 0.5f) : share < 1.f ? share : 1.f;
   const float kept = share * nk;
-  const bool partial = N % 128 != 0 && selection != SPG_SELECT_MASK;
+  const bool partial = N % 128 != 0;
   if (partial && !exact && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
   const float longest = partial ? (float)nk : kept;
   const float all = (float)(B * H) * (nq * kept * (causal ? 1.f - 0.5f * share : 1.f) + (partial ? nk - kept : 0.f));
@@ -264,7 +271,7 @@ inline Layout layout_for(const spg_attn_args *a) {
   l.lut = take(bh * nq * nk * 4);
   l.valid = take(bh * nq * 4);
   l.queue = take(8 * sizeof(int));
-  l.split = take(!pool || nk > SPG_SELECT_IN_ATTN_NK ? chunk_plan(a->B, a->H, a->N, a->N_kv, a->D).bytes : 0);
+  l.split = take(nk > SPG_SELECT_IN_ATTN_NK ? chunk_plan(a->B, a->H, a->N, a->N_kv, a->D).bytes : 0);
   l.total = at;
   return l;
 }

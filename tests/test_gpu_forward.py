@@ -241,7 +241,14 @@ def test_fp16_tiles_beside_the_blocks_of_k(H, N, Nk, D, vdtype):
     got = torch.empty_like(q)
     plan = _lib.ForwardPlan(q, k, v, got, mask, _lib.SELECT_MASK, True, False, False, False, 1, D ** -0.5)
     plan.run(q, k, v, got, mask, 0.0, 0.0, 50.0)
-    assert torch.equal(_bits(got), _bits(o))
+    if _lib.few_rows_route(q.shape, Nk, True, (_lib.SELECT_TOPK, 1.0, False, 50.0)) == _lib.few_rows_route(q.shape, Nk, True, (_lib.SELECT_MASK, None, False, 50.0)):
+        assert torch.equal(_bits(got), _bits(o))
+    else:
+        # few long rows: cut into chunks where top-k names the share, not with a mask, whose density is not known.  The same P are summed in another order: a
+        # few binary32 roundings, 1e-5 of the largest output with margin, and one rounding to the output type that may fall on the other side
+        assert (H, N, Nk) == (4, 300, 8321)
+        a, b = got.double(), o.double()
+        assert ((a - b).abs() <= (2.0 ** -10 if vdtype == torch.float16 else 2.0 ** -7) * b.abs() + 1e-5 * b.abs().max()).all()
 
 
 def test_interrupted_wait_for_counts(monkeypatch):
