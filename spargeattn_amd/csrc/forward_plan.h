@@ -213,9 +213,19 @@ inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, in
   if (many) return longest - all / (D == 64 ? 350.f : 220.f) > 45.f;
   return longest - all / 180.f > 36.f;
 }
+inline bool rows_in_chunks(const spg_attn_args *a, float share, float simthreshd1) {
+  return rows_in_chunks(a->B, a->H, a->N, a->N_kv, a->D, a->pv_f16 != 0, a->selection, share, simthreshd1, a->is_causal != 0);
+}
+// Whether some call of this shape with these options is cut.  The workspace has the scratch then, whatever hyper-parameters the call brings, and not
+// otherwise: up to 280 MB beside some 50 (H8 N17776 D128).  For top-k the difference at the rule is linear in the share, or convex where it is
+// causal, so it is largest at an end; a similarity threshold only takes calls out.
+inline bool may_have_rows_in_chunks(const spg_attn_args *a) {
+  return a->selection == SPG_SELECT_TOPK ? rows_in_chunks(a, 0.f, -1.f) || rows_in_chunks(a, 1.f, -1.f) : rows_in_chunks(a, -1.f, 0.f);
+}
 inline bool rows_in_chunks(const spg_attn_args *a) {
   const float share = a->selection == SPG_SELECT_TOPK && a->level == nullptr ? (a->level_value > 0.f ? a->level_value : 0.f) : -1.f;
-  return rows_in_chunks(a->B, a->H, a->N, a->N_kv, a->D, a->pv_f16 != 0, a->selection, share, a->simthreshd1 == nullptr ? a->simthreshd1_value : 0.f, a->is_causal != 0);
+  // (without scratch never, however the sums at the line are rounded)
+  return may_have_rows_in_chunks(a) && rows_in_chunks(a, share, a->simthreshd1 == nullptr ? a->simthreshd1_value : 0.f);
 }
 
 // Few short rows: workgroups to a row (few_rows_attn_kernel), or 0 where it has one.  Four while each has a CU to itself, two up to 128 rows; the
@@ -271,7 +281,7 @@ inline Layout layout_for(const spg_attn_args *a) {
   l.lut = take(bh * nq * nk * 4);
   l.valid = take(bh * nq * 4);
   l.queue = take(8 * sizeof(int));
-  l.split = take(nk > SPG_SELECT_IN_ATTN_NK ? chunk_plan(a->B, a->H, a->N, a->N_kv, a->D).bytes : 0);
+  l.split = take(may_have_rows_in_chunks(a) ? chunk_plan(a->B, a->H, a->N, a->N_kv, a->D).bytes : 0);
   l.total = at;
   return l;
 }

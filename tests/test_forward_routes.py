@@ -124,6 +124,26 @@ def test_workspace_does_not_depend_on_the_level(routes):
         assert len({routes(level=level, **kw)[5] for level in (0.05, 0.5, 1.0)}) == 1
 
 
+# N17776 has a partial last Q block and N17792 has not, which makes 16 queries of difference where there are no chunks
+@pytest.mark.parametrize("kw", [dict(H=8, selection=CDF), dict(H=8, selection=MASK), dict(H=4, selection=MASK, D=64), dict(H=3, selection=CDF, D=64, pv_f16=1),
+                                dict(H=5, selection=CDF, causal=1)])
+def test_no_scratch_where_no_call_is_cut(routes, kw):
+    a, b = routes(N=17776, **kw), routes(N=17792, **kw)
+    assert a[6] > 1 and a[9] == 0 and a[5] <= b[5]
+    a, b = routes(H=2, N=16384), routes(H=2, N=16385)            # whole rows, as many as there are CUs: whatever top-k keeps
+    assert a[6] > 1 and a[9] == 0 and a[5] < b[5] - (20 << 20)
+
+
+def test_scratch_wherever_a_call_is_cut(routes):
+    for sel, H, N, Nk, D, causal, pv_f16 in ((TOPK, 8, 17776, 0, 64, 0, 0), (TOPK, 4, 17776, 0, 128, 1, 0), (TOPK, 1, 12800, 0, 64, 1, 0), (TOPK, 1, 26000, 0, 128, 1, 1),
+                                             (TOPK, 8, 1024, 64 * 288, 64, 0, 0), (TOPK, 24, 1024, 64 * 288, 128, 0, 0), (TOPK, 3, 30001, 0, 64, 1, 0), (TOPK, 16, 9000, 0, 128, 0, 0),
+                                             (TOPK, 12, 12001, 0, 64, 0, 1), (CDF, 1, 17776, 0, 64, 0, 0), (CDF, 2, 17776, 0, 128, 0, 1), (MASK, 8, 1024, 64 * 256, 64, 0, 0),
+                                             (MASK, 8, 1024, 64 * 255, 64, 0, 0), (MASK, 1, 17777, 0, 128, 0, 0)):
+        cut = {routes(selection=sel, H=H, N=N, Nk=Nk, D=D, causal=causal, pv_f16=pv_f16, level=level, sim=sim)[7]
+               for level in (0.0, 0.05, 0.15, 0.3, 0.5, 0.7, 0.9, 1.0, 1.5) for sim in (-0.1, 0.0)}
+        assert max(cut) == routes(selection=sel, H=H, N=N, Nk=Nk, D=D, causal=causal, pv_f16=pv_f16)[9], (sel, H, N, Nk, D)
+
+
 @pytest.mark.parametrize("D,most", [(64, 1536), (128, 1024)])
 def test_chunks_of_a_row_are_bounded(routes, D, most):
     for H, N, nk in ((1, 1, 8192), (1, 128, 37), (8, 128, 2048), (1, 17776, 278), (2, 16384, 8192)):
