@@ -1133,6 +1133,11 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     // 1851 / 1915), and what else runs gains nothing by it: three wavefronts of 168 registers leave no room on a SIMD, and beside D64 48 x 16384
     // small kernels of another stream take as long either way (an addition over a million floats 54.6, 51.5 with priority and 50.5, 51.4
     // without, 4.5 us alone).
+    // Rows in chunks: `item` counts chunks, wg_per_xcd rows, so up to 768 rows every chunk lowers its priority, also one that others wait for: the chunks of a
+    // round end together and the next ones start together.  us per call so / without lower priorities / over the last 96 chunks of an XCD only, top-k: N17776
+    // D64 H1 0.5 90.0 / 92.7 / 92.6, H4 0.15 127.1 / 135.9 / 135.6, H1 N30001 0.3 136.4 / 147.3 / 147.3; D128 H1 0.5 124.8 / 129.5 / 129.1, H2 0.5 205.6 / 202.6 / 202.0, H1
+    // N30001 0.3 193.1 / 209.9 / 206.6; FP16 PV H2 0.5 238.5 / 232.5 / 232.7.  Beyond 768 rows the first of an XCD do not: so / all of them, H8 0.15 D64 185.8 / 202.7, D128
+    // 279.5 / 269.8.
     int drop_at = 0x7fffffff;
     if constexpr (G == 1) {
       __builtin_amdgcn_s_setprio(3);
