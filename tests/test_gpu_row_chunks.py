@@ -63,6 +63,40 @@ def test_chunks_equal_the_sequential_walk(D, dtype, f16v, gran, causal, H, nq, n
     assert (o - w).norm() <= 3e-4 * w.norm() * (1 if dtype == torch.float16 else 8)
 
 
+@pytest.mark.parametrize("D,dtype,f16v", [(64, torch.bfloat16, False), (128, torch.float16, False), (64, torch.float16, True), (128, torch.bfloat16, True)])
+def test_chunks_of_batches_write_by_strides(D, dtype, f16v):
+    """Two batches, grouped heads, an output laid out (B, N, heads, D) with a head more than the call has: the walk's values, and nothing beside them."""
+    g = torch.Generator().manual_seed(D)
+    B, H, Hkv, nq, nk = 2, 4, 2, 5, 200
+    N, Nk = 128 * nq - 100, 64 * nk - 1
+    q8 = torch.randint(-127, 128, (B, H, N, D), generator=g, dtype=torch.int8).cuda()
+    k8 = torch.randint(-127, 128, (B, Hkv, Nk, D), generator=g, dtype=torch.int8).cuda()
+    qs, ks = (0.01 + 0.03 * torch.rand((B, H, nq), generator=g)).cuda(), (0.04 * 10 ** (-2 * torch.rand((B, Hkv, nk), generator=g))).cuda()
+    per_batch = [lists(1, H, nq, nk, [17, nk, 0, 33, 64, 16, 97, 150, 1], g) for _ in range(B)]
+    lut, valid = (torch.cat(t) for t in zip(*per_batch))
+    thr, v = torch.full((H,), 50.0, device="cuda"), torch.randn((B, Hkv, Nk, D), generator=g).to(torch.float16).cuda()
+    selected = (_lib.SELECT_TOPK, 1.0, False, None)
+    assert _lib.few_rows_route(q8.shape, Nk, f16v, selected)[0] == _lib.ROWS_BY_BLOCKS
+
+    def run(count, o):
+        if f16v:
+            return _lib.block_sparse_attn_f16v(q8, k8, _lib.v_tiles_f16_swizzled(v), o, lut, valid, thr, qs, ks, D ** -0.5, return_pv_count=count, selected=selected)
+        v8, vs = _lib.v_quant_fp8(v)
+        return _lib.block_sparse_attn(q8, k8, v8, o, lut, valid, thr, qs, ks, vs, D ** -0.5, return_pv_count=count, selected=selected)
+
+    want = torch.full((B, H, N, D), 7.0, dtype=dtype, device="cuda")
+    run(True, want)
+    whole = torch.full((B, N, H + 1, D), 7.0, dtype=dtype, device="cuda")
+    got = whole[:, :, :H].transpose(1, 2)
+    run(False, got)
+    assert (whole[:, :, H] == 7.0).all()
+    empty = (valid == 0).repeat_interleave(128, 2)[:, :, :N]
+    assert empty.any() and (got[empty] == 7.0).all()
+    w, o = want.double(), got.double()
+    ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
+    assert ((o - w).abs() <= ulp * w.abs() + 1e-5 * w.abs().max()).all()
+
+
 @pytest.mark.parametrize("level", [0.2, 0.9])
 def test_a_captured_call_replays(level):
     """Scratch of the chunks is written anew by every replay."""
