@@ -8,6 +8,8 @@ import pytest
 import torch
 
 import spargeattn_amd as sa
+from gpu_common import tag_of, to_np
+from oracle import api as oapi, attention as oat
 from spargeattn_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -95,6 +97,27 @@ def test_chunks_of_batches_write_by_strides(D, dtype, f16v):
     w, o = want.double(), got.double()
     ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
     assert ((o - w).abs() <= ulp * w.abs() + 1e-5 * w.abs().max()).all()
+
+
+@pytest.mark.parametrize("D,dtype,sage1,gran", [(64, torch.bfloat16, False, 2), (128, torch.float16, False, 1), (64, torch.float16, True, 1), (128, torch.bfloat16, True, 2)])
+@pytest.mark.parametrize("mode", ["topk", "cdf"])
+def test_cut_rows_against_the_oracle(D, dtype, sage1, gran, mode):
+    """The operator on a call whose rows are cut, from selection to output, two batches and an (B, N, H, D) layout."""
+    g = torch.Generator().manual_seed(D + gran)
+    B, H, Hkv, Nq, Nk = 2, 2, 1, 200, 64 * 150 - 7
+    q, k, v = (torch.randn((B, h, n, D), generator=g).to(dtype) for h, n in ((H, Nq), (Hkv, Nk), (Hkv, Nk)))
+    level, sim = (0.6, -0.1) if mode == "topk" else (0.7, 0.3)
+    assert _lib.few_rows_route(q.shape, Nk, sage1, (_lib.SELECT_TOPK if mode == "topk" else _lib.SELECT_CDF, level if mode == "topk" else None, False, 20.0, sim))[0] == _lib.ROWS_BY_BLOCKS
+    want = (oapi.spas_sage_attn_meansim_topk if sage1 else oapi.spas_sage2_attn_meansim_topk)(
+        to_np(q), to_np(k), to_np(v), tag_of(dtype), simthreshd1=sim, pvthreshd=20.0, qk_quant_gran=gran,
+        **(dict(topk=level, cdfthreshd=None) if mode == "topk" else dict(topk=None, cdfthreshd=level)))
+    op = {("topk", False): sa.spas_sage2_attn_meansim_topk_cuda, ("cdf", False): sa.spas_sage2_attn_meansim_cuda,
+          ("topk", True): sa.spas_sage_attn_meansim_topk_cuda, ("cdf", True): sa.spas_sage_attn_meansim_cuda}[mode, sage1]
+    o, sparsity = op(*(t.transpose(1, 2).contiguous().cuda() for t in (q, k, v)), simthreshd1=sim, pvthreshd=20.0, qk_quant_gran=gran, tensor_layout="NHD",
+                     return_sparsity=True, **{"topk" if mode == "topk" else "cdfthreshd": level})
+    assert abs(sparsity - want["sparsity"]) < 1e-6
+    met = oat.precision_metric(to_np(o.transpose(1, 2)), want["out"])
+    assert met["Cossim"] >= 0.999 and met["L1"] <= 1e-2, met
 
 
 @pytest.mark.parametrize("level", [0.2, 0.9])
