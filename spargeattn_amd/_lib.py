@@ -451,7 +451,7 @@ class ForwardPlan:
         early = return_valid and mask is None and not torch.cuda.is_current_stream_capturing()
         if return_valid:
             if early:
-                valid = torch.full(self.valid_shape, -1, dtype=torch.int32, pin_memory=True)
+                valid = torch.full(self.valid_shape, -1, dtype=torch.int32, device="cpu", pin_memory=True)
             else:
                 valid = torch.empty(self.valid_shape, dtype=torch.int32, device=self.device)
             a.valid_block_num = valid.data_ptr()

@@ -247,8 +247,8 @@ def _run(q, k, v, mask, selection, level, simthreshd1, pvthreshd, is_causal, att
     B, H, nq = plan.valid_shape
     cols = (plan.nk + 2) // 2 if causal_denominator else plan.nk
     # bit for bit what _finish computes on the GPU, where a division by a number is a product with its binary32 reciprocal
-    per_block = torch.tensor(cols * nq * B * H, dtype=torch.float32).reciprocal()
-    qk_sparsity = 1 - torch.tensor(kept).float() * per_block
+    per_block = torch.tensor(cols * nq * B * H, dtype=torch.float32, device="cpu").reciprocal()
+    qk_sparsity = 1 - torch.tensor(kept, device="cpu").float() * per_block
     return o, qk_sparsity.item()
 
 

@@ -272,3 +272,13 @@ def test_interrupted_wait_for_counts(monkeypatch):
     monkeypatch.undo()
     again, sparsity2 = call()
     assert torch.equal(_bits(out), _bits(again)) and sparsity == sparsity2
+
+
+@pytest.mark.parametrize("op,kw", [(sa.spas_sage2_attn_meansim_topk_cuda, dict(topk=0.4)), (sa.spas_sage2_attn_meansim_cuda, dict(cdfthreshd=0.9, simthreshd1=0.2))])
+def test_counts_under_a_default_device(op, kw):
+    """A program that makes its tensors on the GPU by default (torch.set_default_device) gets its sparsity as any other."""
+    q, k, v = (rand_T((1, 3, 1000, 64), torch.float16, s) for s in (1, 2, 3))
+    o, sparsity = op(q, k, v, return_sparsity=True, **kw)
+    with torch.device("cuda"):
+        o2, sparsity2 = op(q, k, v, return_sparsity=True, **kw)
+    assert torch.equal(_bits(o), _bits(o2)) and sparsity == sparsity2
