@@ -187,7 +187,7 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 // causal, one head N31595 D128 342 / 438; 0.82 at 0.6 N31887 with FP16 PV 457 / 531).
 inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, int selection, float share, float simthreshd1, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
-  if (chunk_plan(B, H, N, N_kv, D).chunks == 1 || nk <= SPG_SELECT_IN_ATTN_NK) return false;
+  if (nk <= SPG_SELECT_IN_ATTN_NK || chunk_plan(B, H, N, N_kv, D).chunks == 1) return false;
   const bool many = B * H * nq > 256;
   // A mask: its density is known on the device only, and a sparse one leaves a row one or two chunks, which the two launches more then cost for
   // nothing.  So the line is where a density of 0.1 loses next to nothing.  us per call, workgroup per row / chunks, at 0.1, 0.15 and 0.6: D64 71 x 141 30.3 / 34.5, 30.7
