@@ -219,8 +219,9 @@ typedef struct spg_attn_args {
   uint64_t workspace_bytes;
 } spg_attn_args;
 
-/* Host only.  Waits until none of n counts is negative any more and returns their sum, or -1 after `seconds`: for counts in pinned host
- * memory, filled with -1 before the call.  They arrive with the selection, before the attention has run. */
+/* Host only.  Waits until none of n counts is negative any more and returns their sum, or -1 after `seconds`: for counts in coherent pinned
+ * host memory (hipHostMalloc's default), filled with -1 before the call.  They arrive with the selection, before the attention has
+ * run.  The wait looks without a pause for half a millisecond, from then on every 50 us. */
 int64_t spg_wait_counts(const int32_t *counts, int64_t n, double seconds);
 size_t spg_sparse_attn_workspace_bytes(const spg_attn_args *args);
 int spg_sparse_attn(const spg_attn_args *args, void *stream);

@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
+#include <thread>
 
 static thread_local char g_err[512] = "";
 
@@ -257,14 +258,23 @@ static int check_forward(const char *fn, const spg_attn_args *a) {
   return SPG_OK;
 }
 
+// The counts of a call on its own are there after 20 to 40 us, behind an earlier call of the same kind after 100 to 200: they are looked
+// for without a pause.  After half a millisecond the call stands behind other work (or the memory is not coherent, and the counts come
+// with the end of the kernel): the core is given back, and looking every 50 us adds little to a wait of that length.
 int64_t spg_wait_counts(const int32_t *counts, int64_t n, double seconds) {
   if (counts == nullptr || n < 0) return -1;
   const auto start = std::chrono::steady_clock::now();
   int64_t sum = 0, i = 0;
-  for (unsigned spin = 0;; spin++) {
+  for (unsigned spin = 1;; spin++) {
     for (int v; i < n && (v = __atomic_load_n(counts + i, __ATOMIC_ACQUIRE)) >= 0; i++) sum += v;
     if (i == n) return sum;
-    if (spin % 64 == 63 && std::chrono::duration<double>(std::chrono::steady_clock::now() - start).count() > seconds) return -1;
+    if (spin % 64 != 0) continue;
+    const double waited = std::chrono::duration<double>(std::chrono::steady_clock::now() - start).count();
+    if (waited > seconds) return -1;
+    if (waited > 5e-4) {
+      std::this_thread::sleep_for(std::chrono::microseconds(50));
+      spin = 63;                                     // look once, then at the clock again
+    }
   }
 }
 

@@ -25,6 +25,13 @@ def test_gives_up_in_time():
     assert _lib.load().spg_wait_counts(None, 3, 0.02) == -1
 
 
+def test_a_long_wait_gives_the_core_back():
+    counts = np.array([-1], np.int32)
+    t = time.process_time()
+    assert _lib.load().spg_wait_counts(counts.ctypes.data, 1, 0.2) == -1
+    assert time.process_time() - t < 0.1                    # (half a millisecond, and a few microseconds in every 50)
+
+
 def test_waits_for_counts_in_any_order():
     counts = np.full(64, -1, np.int32)
 
