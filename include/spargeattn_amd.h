@@ -148,7 +148,8 @@ int spg_v_quant_fp8(const void *v, const int64_t *v_strides, uint8_t *v8, float 
  * Row blocks with valid_block_num == 0 are left unwritten, as in the reference (sm89.cuh:232-235).
  * Asking for counts can change the last bits of out: on small grids (up to 256 Q blocks in all, nk >= 12, mode
  * SPG_PV_PER_BLOCK) a call with pv_count == NULL splits a row over groups of wavefronts, which sum O and the denominator in
- * another order than the block-by-block walk that counts.  P, its rounding and the skipped blocks are the same. */
+ * another order than the block-by-block walk that counts.  P, its rounding and the skipped blocks are the same.  (The whole-operator
+ * call also splits rows of up to 1200 Q blocks, and from nk = 6: spg_block_sparse_attn_few_rows below.) */
 int spg_block_sparse_attn(const int8_t *q8, const int8_t *k8, const uint8_t *v8, void *out, const int64_t *out_strides,
                           int out_dtype, const int32_t *lut, const int32_t *valid_block_num, const float *pvthreshd,
                           const float *q_scale, const float *k_scale, const float *v_scale,
@@ -171,16 +172,18 @@ int spg_block_sparse_attn_f16v(const int8_t *q8, const int8_t *k8, const void *v
                                int B, int H, int Hkv, int N, int N_kv, int D, float sm_scale, int is_causal,
                                int qk_quant_gran, int pv_threshold_mode, int32_t *pv_count, void *stream);
 
-/* ---- the two above for few rows (up to 256 Q blocks in all), whose work is spread over several workgroups to a row.
+/* ---- the two above for few rows, whose work is spread over several workgroups to a row.
  * spg_few_rows_route says how the whole-operator call below takes such a call: every row in one workgroup (the functions above), by its
- * queries (short rows), or by its blocks (long ones; *workspace_bytes of device scratch).  selection as in spg_attn_args, share the top-k
- * fraction or a negative number if there is none, is_causal the selection's, simthreshd1 and pvthreshd the thresholds where they are one number for
- * all heads, else 0.
- * spg_block_sparse_attn_few_rows: v and v_scale as for spg_block_sparse_attn, or, with v_scale == NULL, v as for spg_block_sparse_attn_f16v;
- * the PV threshold is per block, and by queries it is taken to be 45 or more: the 32 queries of a wavefront skip a block for themselves, whatever the
- * others of the Q block vote, and what that leaves out is P that rounds to zero, at most 2^-32 of the denominator in all.  The running maxima that P
- * is rounded against are those of the block-by-block walk, by blocks the skipped blocks, too; O and the denominator are summed in another order.  Results
- * are those of the whole-operator call, bit for bit.  workspace 256-byte aligned. */
+ * queries (short rows: at most 128 Q blocks in all, 6 to 128 K blocks), or by its blocks (long ones: at most 256 Q blocks in all, or 1200
+ * where N is no multiple of 128; *workspace_bytes of device scratch, up to 275 MB).  selection as in spg_attn_args, share the top-k
+ * fraction or a negative number if there is none, is_causal the selection's, simthreshd1 and pvthreshd the thresholds where they are
+ * one number for all heads, else 0.
+ * spg_block_sparse_attn_few_rows: v and v_scale as for spg_block_sparse_attn, or, with v_scale == NULL, v as for
+ * spg_block_sparse_attn_f16v; the PV threshold is per block, and by queries it is taken to be 45 or more: the 32 queries of a wavefront
+ * skip a block for themselves, whatever the others of the Q block vote, and what that leaves out is P that rounds to zero, at most 2^-32
+ * of the denominator in all.  The running maxima that P is rounded against are those of the block-by-block walk, by blocks the skipped
+ * blocks, too; O and the denominator are summed in another order.  Results are those of the whole-operator call, bit for bit, on the
+ * route that spg_few_rows_route names.  workspace 256-byte aligned. */
 enum spg_rows { SPG_ROWS_ONE_WORKGROUP = 0, SPG_ROWS_BY_QUERIES = 1, SPG_ROWS_BY_BLOCKS = 2 };
 int spg_few_rows_route(int B, int H, int N, int N_kv, int D, int pv_f16, int selection, float share, float simthreshd1, int is_causal,
                        float pvthreshd, uint64_t *workspace_bytes);

@@ -1133,11 +1133,13 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
     // 1851 / 1915), and what else runs gains nothing by it: three wavefronts of 168 registers leave no room on a SIMD, and beside D64 48 x 16384
     // small kernels of another stream take as long either way (an addition over a million floats 54.6, 51.5 with priority and 50.5, 51.4
     // without, 4.5 us alone).
-    // Rows in chunks: `item` counts chunks, wg_per_xcd rows, so up to 768 rows every chunk lowers its priority, also one that others wait for: the chunks of a
-    // round end together and the next ones start together.  us per call so / without lower priorities / over the last 96 chunks of an XCD only, top-k: N17776
-    // D64 H1 0.5 90.0 / 92.7 / 92.6, H4 0.15 127.1 / 135.9 / 135.6, H1 N30001 0.3 136.4 / 147.3 / 147.3; D128 H1 0.5 124.8 / 129.5 / 129.1, H2 0.5 205.6 / 202.6 / 202.0, H1
-    // N30001 0.3 193.1 / 209.9 / 206.6; FP16 PV H2 0.5 238.5 / 232.5 / 232.7.  Beyond 768 rows the first of an XCD do not: so / all of them, H8 0.15 D64 185.8 / 202.7, D128
-    // 279.5 / 269.8.
+    // Rows in chunks: `item` counts chunks, wg_per_xcd rows, so up to 768 rows every chunk lowers its priority, also one that others wait for:
+    // the chunks of a round end together and the next ones start together.  Beyond 768 rows the first of an XCD do not.  us per call so /
+    // without lower priorities / over the last 96 chunks of an XCD only, top-k:
+    //   D64   H1 N17776 0.5 90.0 / 92.7 / 92.6, H4 N17776 0.15 127.1 / 135.9 / 135.6, H1 N30001 0.3 136.4 / 147.3 / 147.3
+    //   D128  H1 N17776 0.5 124.8 / 129.5 / 129.1, H2 N17776 0.5 205.6 / 202.6 / 202.0, H1 N30001 0.3 193.1 / 209.9 / 206.6
+    //   FP16 PV, D128  H2 N17776 0.5 238.5 / 232.5 / 232.7
+    // and so / all of them, H8 N17776 0.15, 1112 rows: D64 185.8 / 202.7, D128 279.5 / 269.8.
     int drop_at = 0x7fffffff;
     if constexpr (G == 1) {
       __builtin_amdgcn_s_setprio(3);
@@ -1250,11 +1252,12 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_ker
 
 // ---- few short rows -------------------------------------------------------------------------------------------------
 // A workgroup takes 32 QW queries of a row, a quarter or a half of it, and G wavefronts for each 32 of them, which take the row's blocks in
-// turn, place rd G + grp of the list in round rd: several CUs to a row instead of one, and a row of up to G blocks in one round.  Each wavefront has tiles of its own and the next ones
-// are requested as soon as the operands of the present ones are in registers; it meets the others once per round, to learn the
-// running maximum in front of its block (P is rounded against it), and at the end, where O and the denominators are added up in the order
-// of the groups.  No wavefront sees the votes of the row's other workgroups, so each skips a block on the vote of its own 32 queries: it skips whatever
-// the whole row skips, whose V it then leaves alone, and at the thresholds of this route the rest as well adds nothing (few_rows).
+// turn, place rd G + grp of the list in round rd: several CUs to a row instead of one, and a row of up to G blocks in one round.
+// Each wavefront has tiles of its own, and the next ones are requested as soon as the operands of the present ones are in registers;
+// it meets the others once per round, to learn the running maximum in front of its block (P is rounded against it), and at the
+// end, where O and the denominators are added up in the order of the groups.  No wavefront sees the votes of the row's other
+// workgroups, so each skips a block on the vote of its own 32 queries: it skips whatever the whole row skips, whose V it then leaves
+// alone, and at the thresholds of this route the rest as well adds nothing (few_rows).
 // Arithmetic and masks are those of block_sparse_attn_kernel; at most 128 blocks to a row.
 template <int D, int ODT, bool PV16, int SEL, int QW, int G>
 __global__ __launch_bounds__(64 * QW * G, 2) void few_rows_attn_kernel(const AttnParams p) {

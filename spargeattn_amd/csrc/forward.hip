@@ -11,7 +11,8 @@
 //            of the next launch to add them up for itself)
 //   back     pooling + quantisation of K | V -> e4m3 tiles and scales (FP16 PV, many blocks: V^T tiles)
 //   select   block_select_* of maskpred.hip (rows of more than 128 blocks; shorter ones are selected inside the next launch)
-//   attn     block_sparse_attn_kernel (few short rows: few_rows_attn_kernel, several workgroups to a row; few long rows: in chunks, with a launch in front for their maxima and one behind)
+//   attn     block_sparse_attn_kernel (few short rows: few_rows_attn_kernel, several workgroups to a row; few long rows: in chunks,
+//            with a launch in front for their maxima and one behind)
 // Every body is the one the stage-by-stage entry points launch (stage_bodies.h): results are the same bits.
 // The extern "C" entry points and their argument checks are in capi.hip, the workspace layout in forward_plan.h.
 // Compile with -ffp-contract=off.

@@ -124,10 +124,26 @@ inline bool q_overwritten(const spg_attn_args *a, const Strides &qs, const Strid
 }
 
 // ---- rows in chunks (RowSplit) --------------------------------------------------------------------------------------
-// Blocks of a chunk, and where the scratch for it lies.  About two rounds of workgroups if every block is kept (D = 64 fits four to a CU, D =
-// 128 three), so that one round or more is left with half of them.  us per call with 512 / 768 / 1024 / 1536 / 2048 workgroups in all: one head
-// N17776 D64 top-k 0.5 117 / 109 / 98 / 97 / 105, 2 x 10000 80 / 79 / 81 / 75 / 83; D128 160 / 140 / 133 / 140 / 143, 2 x 10000 106 / 101 / 96 / 103 / 108, with
-// every block kept 186 / 194 / 191 / 194 / 197.  (8 and 24 blocks instead of 16 at least: 8300 x 8300 D64 55.5 / 53.4 / 57.6, D128 68.5 / 67.7 / 74.5.)
+// Blocks of a chunk, and where the scratch for it lies.
+//
+// Up to 256 rows: about two rounds of workgroups if every block is kept (D = 64 fits four to a CU, D = 128 three), so that one
+// round or more is left with half of them.  us per call by workgroups in all:
+//                                       512   768  1024  1536  2048
+//   D64   one head N17776, top-k 0.5    117   109    98    97   105
+//         10000 x 10000, two heads       80    79    81    75    83
+//   D128  one head N17776, top-k 0.5    160   140   133   140   143
+//         the same, all blocks kept     186   194   191   194   197
+//         10000 x 10000, two heads      106   101    96   103   108
+// At least 16 blocks: 8300 x 8300 with 8 / 16 / 24 of them D64 55.5 / 53.4 / 57.6, D128 68.5 / 67.7 / 74.5.
+//
+// Beyond 256 rows: only for the sake of a partial last Q block, whose rows keep everything.  Beyond 1200 they would have two chunks
+// (H12 N17776 top-k 0.15, 1668 rows, workgroup per row / chunks: D64 263 / 275, D128 351 / 391).  us by workgroups in all, N17776:
+//                      1536  3072  4608                           1536  3072  4608
+//   D64  H2 0.5         141   144   149      D128  H2 0.5          216   205   214
+//        H4 0.15        143   129   132            H4 0.15         179   149   176
+//        H4 0.3         167   180   171            H4 0.3          215   235   249
+//        H4 0.5         247   223   233            H6 0.15         283   222   205
+//        H8 0.15        218   185   171            N30001 H4 0.15  430   340   324
 struct ChunkPlan {
   int chunks, per;                  // 1, 0: a row has one workgroup, whatever it keeps
   size_t first, maxima, md, o, bytes;
@@ -135,18 +151,14 @@ struct ChunkPlan {
 inline ChunkPlan chunk_plan(int B, int H, int N, int N_kv, int D) {
   ChunkPlan c = {1, 0, 0, 0, 0, 0, 0};
   const long long rows = (long long)B * H * ((N + 127) / 128), nk = (N_kv + 63) / 64;
-  // (beyond 256 rows only for the sake of a partial last Q block, whose rows keep everything; beyond 1200 they would have two chunks: H12 N17776
-  // top-k 0.15, 1668 rows, D64 263 / 275, D128 351 / 391)
   if (rows > (N % 128 != 0 ? 1200 : 256) || nk <= 36 || nk > 32768) return c;
-  // beyond 256 rows, us with 1536 / 3072 / 4608 workgroups, N17776: D64 H2 0.5 141 / 144 / 149, H4 0.15 143 / 129 / 132, 0.3 167 / 180 / 171, 0.5 247 / 223 / 233, H8 0.15 218 /
-  // 185 / 171; D128 H2 0.5 216 / 205 / 214, H4 0.15 179 / 149 / 176, 0.3 215 / 235 / 249, H6 0.15 283 / 222 / 205; N30001 H4 0.15 430 / 340 / 324.
-  // The sums of a chunk are 128 x D floats: at most 4300 of them, 280 MB at D = 128, whatever the lengths.
-  const long long wgs = rows > 256 ? 3072 : D == 64 ? 1536 : 1024, spread = (rows * nk + wgs - 1) / wgs, most = (nk + 63) / 64;   // (64 chunks: those of a row are added up one by one)
+  const long long wgs = rows > 256 ? 3072 : D == 64 ? 1536 : 1024, spread = (rows * nk + wgs - 1) / wgs;
+  const long long most = (nk + 63) / 64;                          // 64 chunks: those of a row are added up one by one
   c.per = (int)(spread > most ? spread : most);
   if (c.per < 16) c.per = 16;
   c.chunks = (int)((nk + c.per - 1) / c.per);
   auto take = [&](size_t bytes) { const size_t r = c.bytes; c.bytes += (bytes + 255) / 256 * 256; return r; };
-  const size_t all = (size_t)rows * c.chunks;
+  const size_t all = (size_t)rows * c.chunks;                     // at most 4092, 275 MB at D = 128, whatever the lengths
   c.first = take(all * 4);
   c.maxima = take(all * 128 * 4);
   c.md = take(all * 256 * 4);
@@ -157,18 +169,11 @@ inline RowSplit row_split(const ChunkPlan &c, void *scratch) {
   unsigned char *const at = (unsigned char *)scratch;
   return {c.chunks, c.per, 0, (int *)(at + c.first), (float *)(at + c.maxima), (float *)(at + c.md), (float *)(at + c.o)};
 }
-// Whether they pay: with a workgroup per row the call takes as long as its longest row, 0.45 us per block at D = 64 and 0.6 at D = 128 (0.76
-// with FP16 PV); in chunks all blocks count, 2.05, 3.25 and 4.2 ns each, and the two launches more take 16 us.  A row is expected to keep the
-// blocks that top-k names (share; below 0: nothing on the host says, and half is taken); a partial last Q block is never similar and keeps all.
-// us per call, workgroup per row / chunks, 8 to 176 whole rows, nk, top-k: D64 8 x 132 0.2 46.5 / 48.9, 0.35 56.0 / 51.9, 1.0 95.8 / 54.4; 64 x 132 0.35 59.9
-// / 57.8, 64 x 288 0.2 80.5 / 72.1, 1.0 183 / 111; 128 x 192 0.35 76.2 / 74.6, 0.5 90.4 / 82.0, 128 x 512 0.2 115.5 / 113.5, 1.0 303 / 218; 176 x 288 0.35 100 / 105,
-// 1.0 182 / 175; 224 x 512 1.0 321 / 332.  D128 8 x 132 0.2 58.5 / 63.6, 0.35 72.3 / 66.8; 64 x 512 0.1 128.7 / 133.4, 0.5 251 / 169; 128 x 288 0.35 134 /
-// 132, 0.5 161 / 143; 176 x 512 1.0 405 / 423; FP16 PV 64 x 288 0.2 107.5 / 95.3, 160 x 288 0.5 184 / 175, 256 x 288 0.5 198 / 217.  With a partial last
-// block: N24000, 188 rows, top-k 0.5 D64 207 / 145, D128 265 / 190, causal 207 / 140; N28000 D128 310 / 231; one head N17776 CDF 171 / 136.
-// Everything kept, with a partial last Q block: the longest row is as long as ever and the chunks have the most to do, so they pay nowhere less.  A
-// workgroup per row takes 0.48 (D = 64), 0.62 (D = 128) and 0.74 us (FP16 PV) per block of a row in groups, and 0.9 and 1.1 us in one group beyond 256
-// rows; causal rows, half as many blocks, save a tenth of the chunks' time only, since a chunk is as long as in a full row.  us per call, workgroup
-// per row / chunks, on both sides of the line, rows x nk:
+
+// Everything kept, with a partial last Q block: the longest row is as long as ever and the chunks have the most to do, so they pay nowhere
+// less.  A workgroup per row takes 0.48 (D = 64), 0.62 (D = 128) and 0.74 us (FP16 PV) per block of a row in groups, and 0.9 and 1.1 us in one
+// group beyond 256 rows; causal rows, half as many blocks, save a tenth of the chunks' time only, since a chunk is as long as in a full
+// row.  us per call, workgroup per row / chunks, on both sides of the line, rows x nk:
 //            up to 256 rows                                              beyond
 // D64        188 x 376 215 / 192, 204 x 407 231 / 222, 252 x 251 156 / 185   376 x 376 375 / 339, 417 x 278 291 / 297, 390 x 130 157 / 166
 // causal     219 x 438 241 / 231, 235 x 469 257 / 260, 252 x 251 154 / 160   417 x 278 256 / 236, 556 x 278 283 / 283, 469 x 938 819 / 830
@@ -181,35 +186,61 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
   if (rows > 256) return nk - all / (D == 64 ? 420.f : pv_f16 ? 290.f : 320.f) > 27.f;
   return nk - all / (D == 128 ? 185.f : pv_f16 ? 200.f : 220.f) > 36.f;
 }
-// simthreshd1: blocks of Q and K whose similarity is below it keep everything.  A similarity is not negative, so below 0 it changes nothing and
-// a row keeps what top-k names; from 0 on a row may keep all of its blocks, and nothing on the host says how many do (H8 N17776 top-k 0.15 at 0.6, no block
-// similar: workgroup per row / chunks D64 578 / 661 us, D128 831 / 1041).  Nor does it for a CDF threshold or a level per head (CDF 0.93 at 0.3,
-// causal, one head N31595 D128 342 / 438; 0.82 at 0.6 N31887 with FP16 PV 457 / 531).
+
+// Whether chunks pay: with a workgroup per row the call takes as long as its longest row, 0.45 us per block at D = 64 and 0.6 at D = 128
+// (0.76 with FP16 PV); in chunks all blocks count, 2.05, 3.25 and 4.2 ns each, and the two launches more take 16 us.
+//
+// What a row keeps:
+// * top-k without similar blocks to look for: what top-k names (share), and all of it in a partial last Q block, which is never similar.
+//   simthreshd1: blocks of Q and K whose similarity is below it keep everything.  A similarity is not negative, so below 0 it changes nothing.
+// * a similarity threshold of 0 or more, a CDF threshold or a level per head (share below 0): nothing on the host says, and it is often
+//   everything.  Half of it is taken, beyond 256 rows 0.65 to 0.75, and with a partial last Q block it has to pay with everything kept, too.
+//   us per call, workgroup per row / chunks: H8 N17776 top-k 0.15 with simthreshd1 0.6, no block similar, D64 578 / 661, D128 831 / 1041; CDF 0.93
+//   at 0.3, causal, one head N31595 D128 342 / 438; 0.82 at 0.6 N31887 with FP16 PV 457 / 531.
+// * a mask: its density is known on the device only, and a sparse one leaves a row one or two chunks, which the two launches more then
+//   cost for nothing.  So the line is where a density of 0.1 loses next to nothing:
+//     rows x nk        D64 0.1          0.15           0.6            D128 0.1         0.15           0.6
+//     71 x 141         30.3 / 34.5    30.7 / 35.9    61.6 / 43.9      36.4 / 45.5                   85.3 / 58.4
+//     125 x 250        39.7 / 45.5    46.3 / 47.8    99.0 / 78.2
+//     64 x 192         43.6 / 48.3    50.0 / 49.3    90.9 / 60.1
+//     8 x 256                                                         66.3 / 68.8    73.2 / 68.1   145.2 / 72.2
+//     64 x 256         50.9 / 51.6    56.9 / 52.5   112.3 / 69.2      70.8 / 71.3    79.8 / 72.4   152.7 / 100.4
+//     96 x 938         98.3 / 99.1                                   142.1 / 165.7
+//     126 x 938        92.1 / 103.2
+//   at 0.1 the ratio over 256 / 400 / 1024 K blocks D64 8 rows 0.97 / 1.05 / 1.41, 64 rows 0.98 / 1.08 / 1.19, D128 8 rows 0.96 / 1.17 / 1.30, 64 rows
+//   0.97 / 1.02 / 1.02, 75 rows 0.97 / 0.98 / 1.01.
+//
+// Up to 256 rows, top-k, us per call, workgroup per row / chunks, whole rows x nk:
+//   D64   8 x 132    0.2  46.5 / 48.9, 0.35  56.0 / 51.9, 1.0  95.8 / 54.4    128 x 192  0.35 76.2 / 74.6, 0.5  90.4 / 82.0
+//         64 x 132  0.35  59.9 / 57.8                                         128 x 512  0.2 115.5 / 113.5, 1.0 303 / 218
+//         64 x 288   0.2  80.5 / 72.1, 1.0 183 / 111                          176 x 288  0.35 100 / 105, 1.0 182 / 175
+//                                                                             224 x 512  1.0 321 / 332
+//   D128  8 x 132    0.2  58.5 / 63.6, 0.35  72.3 / 66.8                      128 x 288  0.35 134 / 132, 0.5 161 / 143
+//         64 x 512   0.1 128.7 / 133.4, 0.5 251 / 169                         176 x 512  1.0 405 / 423
+//   FP16 PV, D128  64 x 288 0.2 107.5 / 95.3, 160 x 288 0.5 184 / 175, 256 x 288 0.5 198 / 217
+// and with a partial last Q block, top-k 0.5: N24000, 188 rows, D64 207 / 145, causal 207 / 140, D128 265 / 190; N28000 D128 310 / 231; one head
+// N17776 D64 CDF 171 / 136.
+//
+// Beyond 256 rows, where a row walks its blocks in one group, 0.7 us per block at D = 64 and 0.9 at D = 128, beside others or alone at the
+// end; a partial last Q block, top-k:
+//   N17776 D64   H2 0.15 231 / 96, 0.5 230 / 147, 0.7 243 / 180    H4 0.3 237 / 181, 0.5 254 / 227, 0.7 296 / 299    H6 0.3 243 / 229, 0.5 303 / 307
+//                H8 0.15 246 / 186, 0.3 249 / 236    causal 0.5 H2 230 / 138, H4 250 / 218, H8 293 / 317    FP16 PV H2 0.5 243 / 152
+//   N17776 D128  H2 0.15 276 / 113, 0.5 279 / 207    H3 0.3 283 / 200, 0.7 301 / 347    H4 0.3 303 / 239, 0.5 323 / 337    H8 0.15 326 / 278, 0.3 354 / 366
+//                causal 0.5 H2 276 / 196, H4 308 / 322    FP16 PV H2 0.5 326 / 241
+//   N8300 H6     0.15 D64 125 / 80, D128 154 / 107    0.5 D64 127 / 117, D128 156 / 161
+//   30000 queries over 8400, two heads, 0.15  D64 119 / 66, D128 145 / 84
+//   CDF 0.9 on N(0, 1) data, D64  H2 N17776 268 / 208, H4 338 / 342, H6 N8300 146 / 157
 inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, int selection, float share, float simthreshd1, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
   if (nk <= SPG_SELECT_IN_ATTN_NK || chunk_plan(B, H, N, N_kv, D).chunks == 1) return false;
-  const bool many = B * H * nq > 256;
-  // A mask: its density is known on the device only, and a sparse one leaves a row one or two chunks, which the two launches more then cost for
-  // nothing.  So the line is where a density of 0.1 loses next to nothing.  us per call, workgroup per row / chunks, at 0.1, 0.15 and 0.6: D64 71 x 141 30.3 / 34.5, 30.7
-  // / 35.9 and 61.6 / 43.9, 125 x 250 39.7 / 45.5, 46.3 / 47.8 and 99.0 / 78.2, 64 x 192 43.6 / 48.3, 50.0 / 49.3 and 90.9 / 60.1, 64 x 256 50.9 / 51.6, 56.9 / 52.5 and 112.3 /
-  // 69.2, 96 x 938 98.3 / 99.1, 126 x 938 92.1 / 103.2; D128 71 x 141 36.4 / 45.5 and 85.3 / 58.4, 8 x 256 66.3 / 68.8, 73.2 / 68.1 and 145.2 / 72.2, 64 x 256 70.8 / 71.3, 79.8 / 72.4
-  // and 152.7 / 100.4, 96 x 938 142.1 / 165.7; at 0.1 the ratio over 256 / 400 / 1024 K blocks D64 8 rows 0.97 / 1.05 / 1.41, 64 rows 0.98 / 1.08 / 1.19, D128 8 rows 0.96 /
-  // 1.17 / 1.30, 64 rows 0.97 / 1.02 / 1.02, 75 rows 0.97 / 0.98 / 1.01.
   if (selection == SPG_SELECT_MASK) return B * H * nq <= 64 && nk >= 256;
-  const bool exact = selection == SPG_SELECT_TOPK && share >= 0.f && simthreshd1 < 0.f;
+  const bool many = B * H * nq > 256, partial = N % 128 != 0;
+  const bool known = selection == SPG_SELECT_TOPK && share >= 0.f && simthreshd1 < 0.f;
+  if (partial && !known && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
   share = share < 0.f ? (many ? (D == 64 ? 0.75f : 0.65f) : 0.5f) : share < 1.f ? share : 1.f;
   const float kept = share * nk;
-  const bool partial = N % 128 != 0;
-  if (partial && !exact && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
   const float longest = partial ? (float)nk : kept;
   const float all = (float)(B * H) * (nq * kept * (causal ? 1.f - 0.5f * share : 1.f) + (partial ? nk - kept : 0.f));
-  // Beyond 256 rows a row walks its blocks in one group, 0.7 us per block at D = 64 and 0.9 at D = 128, beside others or alone at the end.  us per
-  // call, workgroup per row / chunks, a partial last Q block.  N17776 D64: H2 top-k 0.15 231 / 96, 0.5 230 / 147, 0.7 243 / 180; H4 0.3 237 / 181, 0.5 254 / 227, 0.7 296 / 299; H6 0.3 243 /
-  // 229, 0.5 303 / 307; H8 0.15 246 / 186, 0.3 249 / 236; causal H2 0.5 230 / 138, H4 250 / 218, H8 293 / 317.  D128: H2 0.15 276 / 113, 0.5 279 / 207; H3 0.3 283 / 200, 0.7 301 / 347;
-  // H4 0.3 303 / 239, 0.5 323 / 337; H8 0.15 326 / 278, 0.3 354 / 366; causal H2 276 / 196, H4 308 / 322; FP16 PV H2 0.5 326 / 241, D64 243 / 152.  N8300 H6 0.15 D64 125 / 80, D128
-  // 154 / 107, 0.5 127 / 117 and 156 / 161; 2 heads of 30000 over 8400 0.15 119 / 66 and 145 / 84.  Where nothing says how much is kept it is often more than half (CDF
-  // 0.9 on N(0, 1) data, D64: H2 N17776 268 / 208, H4 338 / 342, H6 N8300 146 / 157), so more is taken for granted than in
-  // shorter grids.
   if (many) return longest - all / (D == 64 ? 350.f : 220.f) > 45.f;
   return longest - all / 180.f > 36.f;
 }
@@ -217,7 +248,7 @@ inline bool rows_in_chunks(const spg_attn_args *a, float share, float simthreshd
   return rows_in_chunks(a->B, a->H, a->N, a->N_kv, a->D, a->pv_f16 != 0, a->selection, share, simthreshd1, a->is_causal != 0);
 }
 // Whether some call of this shape with these options is cut.  The workspace has the scratch then, whatever hyper-parameters the call brings, and not
-// otherwise: up to 280 MB beside some 50 (H8 N17776 D128).  For top-k the difference at the rule is linear in the share, or convex where it is
+// otherwise: up to 275 MB beside some 50 (H8 N17776 D128).  For top-k the difference at the rule is linear in the share, or convex where it is
 // causal, so it is largest at an end; a similarity threshold only takes calls out.
 inline bool may_have_rows_in_chunks(const spg_attn_args *a) {
   return a->selection == SPG_SELECT_TOPK ? rows_in_chunks(a, 0.f, -1.f) || rows_in_chunks(a, 1.f, -1.f) : rows_in_chunks(a, -1.f, 0.f);
@@ -228,19 +259,27 @@ inline bool rows_in_chunks(const spg_attn_args *a) {
   return may_have_rows_in_chunks(a) && rows_in_chunks(a, share, a->simthreshd1 == nullptr ? a->simthreshd1_value : 0.f);
 }
 
-// Few short rows: workgroups to a row (few_rows_attn_kernel), or 0 where it has one.  Four while each has a CU to itself, two up to 128 rows; the
-// workgroup with all four quarters (attn_groups) beyond, and where a row has no more blocks than it has groups.  us per call with one /
-// four workgroups to a row, top-k 0.2, 0.5 and 1.0, rows x nk: D64 16 x 8 14.3 / 13.7, 14.9 / 14.0, 17.0 / 13.8; 64 x 16 16.4 / 14.4, 19.0 / 15.3, 22.3 / 16.0, 64 x 64 26.5 / 22.0,
-// 37.1 / 26.9, 53.4 / 32.8, 64 x 128 44.0 / 34.5, 61.9 / 43.5, 90.4 / 57.0; 96 x 16 16.5 / 19.5, 19.2 / 21.5, 22.6 / 23.1.  D128 16 x 4 14.5 / 14.8, 15.5 / 14.6, 16.6 /
-// 14.2; 64 x 16 22.5 / 19.9, 26.3 / 21.6, 30.6 / 23.4, 64 x 128 54.2 / 42.7, 78.6 / 55.5, 116.8 / 73.7; FP16 PV 64 x 64 36.4 / 30.6, 52.7 / 41.7, 76.4 / 54.5.  One /
-// two: D64 128 x 8 13.6 / 13.7, 15.2 / 14.5, 17.3 / 14.8; 128 x 16 16.6 / 15.8, 19.3 / 17.2, 22.6 / 19.5, 128 x 128 45.2 / 40.2, 62.5 / 55.3, 91.6 / 78.5, 160 x 32 21.5 / 27.9,
-// 27.5 / 34.5, 34.5 / 45.7; D128 128 x 8 16.7 / 17.6, 19.7 / 18.6, 22.3 / 20.0, 128 x 16 23.1 / 22.2, 26.7 / 24.7, 31.5 / 28.3, 128 x 128 54.3 / 49.5, 78.8 / 68.2, 116.5 /
-// 99.0; FP16 PV at D128, whose tiles leave room for three groups, 128 x 64 38.0 / 37.5, 53.9 / 54.1, 77.4 / 77.6.
+// Few short rows: workgroups to a row (few_rows_attn_kernel), or 0 where it has one.  Four while each has a CU to itself, two up to 128
+// rows; the workgroup with all four quarters (attn_groups) beyond, and where a row has no more blocks than it has groups.  us per call, top-k
+// 0.2, 0.5 and 1.0, rows x nk, one / four workgroups to a row:
+//   D64   16 x 8    14.3 / 13.7   14.9 / 14.0   17.0 / 13.8       D128  16 x 4    14.5 / 14.8   15.5 / 14.6   16.6 / 14.2
+//         64 x 16   16.4 / 14.4   19.0 / 15.3   22.3 / 16.0             64 x 16   22.5 / 19.9   26.3 / 21.6   30.6 / 23.4
+//         64 x 64   26.5 / 22.0   37.1 / 26.9   53.4 / 32.8             64 x 128  54.2 / 42.7   78.6 / 55.5  116.8 / 73.7
+//         64 x 128  44.0 / 34.5   61.9 / 43.5   90.4 / 57.0       FP16  64 x 64   36.4 / 30.6   52.7 / 41.7   76.4 / 54.5
+//         96 x 16   16.5 / 19.5   19.2 / 21.5   22.6 / 23.1       (at D128)
+// one / two:
+//   D64   128 x 8   13.6 / 13.7   15.2 / 14.5   17.3 / 14.8       D128  128 x 8   16.7 / 17.6   19.7 / 18.6   22.3 / 20.0
+//         128 x 16  16.6 / 15.8   19.3 / 17.2   22.6 / 19.5             128 x 16  23.1 / 22.2   26.7 / 24.7   31.5 / 28.3
+//         128 x 128 45.2 / 40.2   62.5 / 55.3   91.6 / 78.5             128 x 128 54.3 / 49.5   78.8 / 68.2  116.5 / 99.0
+//         160 x 32  21.5 / 27.9   27.5 / 34.5   34.5 / 45.7       FP16  128 x 64  38.0 / 37.5   53.9 / 54.1   77.4 / 77.6
+// (FP16 PV at D128: its tiles leave room for three groups.)
+//
 // The workgroups of a row do not see each other's votes on the PV threshold.  A block is skipped when all scores of the Q block are `pvthreshd`
-// below the running maxima in the exponent of 2; the quarter (half) of a workgroup alone may be that far below where the others are not, and then skips a
-// block that the row keeps.  So the threshold has to be one at which that changes next to nothing: from 45 on, P of such a block is zero in e4m3
-// and in fp16, so O stays as it is, and what is left out of a query's denominator is at most 64 x 2^-45 = 2^-39 of it per block, 2^-32
-// for 126 of them, below the rounding of its sum in binary32.  (A per-head threshold is not known here: 0.)
+// below the running maxima in the exponent of 2; the quarter (half) of a workgroup alone may be that far below where the others are not, and
+// then skips a block that the row keeps.  So the threshold has to be one at which that changes next to nothing: from 45 on, P of such a
+// block is zero in e4m3 and in fp16, so O stays as it is (a product with an infinity or a NaN in V apart), and what is left out of a query's
+// denominator is at most 64 x 2^-45 = 2^-39 of it per block, 2^-32 for 126 of them, below the rounding of its sum in binary32.
+// (A per-head threshold is not known here: 0.)
 inline int few_rows(int B, int H, int N, int N_kv, int D, bool pv_f16, float pvthreshd) {
   const long long rows = (long long)B * H * ((N + 127) / 128), nk = (N_kv + 63) / 64;
   if (!(pvthreshd >= 45.f) || nk > 128) return 0;
