@@ -328,7 +328,7 @@ __device__ __forceinline__ int v_swz(int row) { return (row >> 2) & 3; }
 // FQ: 0 Q comes as INT8 codes and scales; 1 the workgroup quantises its Q block itself; 2 it pools it, too, and works out its similarity
 // flag, for a selection in place (SEL).  Codes, pooled row and flag stay in LDS: what a kernel in front would write (half of Q's bytes
 // and more) and this one read again.
-// SPLIT: a row's blocks go over several workgroups, each with a stretch of its list (launch_row_maxima has the why).
+// SPLIT: a row's blocks go over several workgroups, each with a stretch of its list (launch_split has the why).
 template <int D, int ODT, bool PV16, int SEL, int G, int FQ, bool SPLIT>
 __global__ __launch_bounds__(256 * G, G == 1 ? 3 : G) void block_sparse_attn_kernel(const AttnParams p) {
   constexpr int KS = D / 32;        // k-steps of the int8 MFMA
