@@ -109,13 +109,13 @@ def kernels():
         if b"block_sparse_attn_kernel" in obj or b"dense_attn_f16_kernel" in obj:
             r = subprocess.run([OBJDUMP, "-d", "-"], input=obj, capture_output=True)
             assert r.returncode == 0, r.stderr[-500:]
-            out.update({k: v for k, v in functions(r.stdout.decode()).items() if "attn" in k})
+            out.update({k: v for k, v in functions(r.stdout.decode()).items() if "attn" in k or "row_maxima" in k})
     return out
 
 
 def test_every_read_is_waited_for_first(kernels):
     attn = [k for k in kernels if "block_sparse_attn_kernel" in k]
-    assert len(attn) >= 60 and any("dense_attn_f16_kernel" in k for k in kernels)
+    assert len(attn) >= 60 and all(any(name in k for k in kernels) for name in ("few_rows_attn_kernel", "row_maxima_kernel", "dense_attn_f16_kernel"))
     for name, code in kernels.items():
         assert sum(op == "ds_read_b128" for _, op, _, _ in code) > 0, name
         assert not violations(code), name
