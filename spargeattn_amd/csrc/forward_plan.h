@@ -197,18 +197,12 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 //   everything.  Half of it is taken, beyond 256 rows 0.65 to 0.75, and with a partial last Q block it has to pay with everything kept, too.
 //   us per call, workgroup per row / chunks: H8 N17776 top-k 0.15 with simthreshd1 0.6, no block similar, D64 578 / 661, D128 831 / 1041; CDF 0.93
 //   at 0.3, causal, one head N31595 D128 342 / 438; 0.82 at 0.6 N31887 with FP16 PV 457 / 531.
-// * a mask: its density is known on the device only, and a sparse one leaves a row one or two chunks, which the two launches more then
-//   cost for nothing.  So the line is where a density of 0.1 loses next to nothing:
-//     rows x nk        D64 0.1          0.15           0.6            D128 0.1         0.15           0.6
-//     71 x 141         30.3 / 34.5    30.7 / 35.9    61.6 / 43.9      36.4 / 45.5                   85.3 / 58.4
-//     125 x 250        39.7 / 45.5    46.3 / 47.8    99.0 / 78.2
-//     64 x 192         43.6 / 48.3    50.0 / 49.3    90.9 / 60.1
-//     8 x 256                                                         66.3 / 68.8    73.2 / 68.1   145.2 / 72.2
-//     64 x 256         50.9 / 51.6    56.9 / 52.5   112.3 / 69.2      70.8 / 71.3    79.8 / 72.4   152.7 / 100.4
-//     96 x 938         98.3 / 99.1                                   142.1 / 165.7
-//     126 x 938        92.1 / 103.2
-//   at 0.1 the ratio over 256 / 400 / 1024 K blocks D64 8 rows 0.97 / 1.05 / 1.41, 64 rows 0.98 / 1.08 / 1.19, D128 8 rows 0.96 / 1.17 / 1.30, 64 rows
-//   0.97 / 1.02 / 1.02, 75 rows 0.97 / 0.98 / 1.01.
+// * a mask: never in chunks.  Its density is known on the device only, and the rows of a sparse one are one or two chunks each, for which the
+//   launches more cost up to a fifth of the call.  rows x nk, density:
+//                  0.03          0.06          0.1           0.2                        0.03          0.06          0.1           0.2
+//     D64  8 x 512   31.4 / 38.4   41.5 / 39.1   53.2 / 41.0   84.9 / 43.0    D128  8 x 512   41.6 / 49.0   54.9 / 49.8   70.5 / 52.2  112.4 / 55.0
+//          64 x 256  31.6 / 36.2   38.1 / 43.2   45.5 / 44.8   60.1 / 50.0          64 x 256  45.0 / 50.2   54.3 / 59.5   62.9 / 60.4   81.5 / 65.3
+//          64 x 288  39.8 / 43.8   48.0 / 52.8   58.2 / 53.7   74.1 / 58.3          64 x 288  59.5 / 63.9   68.4 / 76.4   80.9 / 78.1  100.6 / 82.4
 //
 // Up to 256 rows, top-k, us per call, workgroup per row / chunks, whole rows x nk:
 //   D64   8 x 132    0.2  46.5 / 48.9, 0.35  56.0 / 51.9, 1.0  95.8 / 54.4    128 x 192  0.35 76.2 / 74.6, 0.5  90.4 / 82.0
@@ -232,8 +226,7 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 //   CDF 0.9 on N(0, 1) data, D64  H2 N17776 268 / 208, H4 338 / 342, H6 N8300 146 / 157
 inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, int selection, float share, float simthreshd1, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
-  if (nk <= SPG_SELECT_IN_ATTN_NK || chunk_plan(B, H, N, N_kv, D).chunks == 1) return false;
-  if (selection == SPG_SELECT_MASK) return B * H * nq <= 64 && nk >= 256;
+  if (selection == SPG_SELECT_MASK || nk <= SPG_SELECT_IN_ATTN_NK || chunk_plan(B, H, N, N_kv, D).chunks == 1) return false;
   const bool many = B * H * nq > 256, partial = N % 128 != 0;
   const bool known = selection == SPG_SELECT_TOPK && share >= 0.f && simthreshd1 < 0.f;
   if (partial && !known && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
