@@ -224,18 +224,41 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 //   N8300 H6     0.15 D64 125 / 80, D128 154 / 107    0.5 D64 127 / 117, D128 156 / 161
 //   30000 queries over 8400, two heads, 0.15  D64 119 / 66, D128 145 / 84
 //   CDF 0.9 on N(0, 1) data, D64  H2 N17776 268 / 208, H4 338 / 342, H6 N8300 146 / 157
+//
+// Causal, us per call, workgroup per row / chunks, rows x nk, top-k 0.35, 0.6 and 1.0 (* the rule takes chunks):
+//                    D64                                    D128                                   FP16 PV, D128
+//   125 x 250         72 / 67   101 / 82*  143 / 100*         92 / 88   130 / 107* 187 / 146*       104 / 91   151 / 119* 223 / 165*
+//   175 x 350         93 / 94   132 / 130  191 / 158*        118 / 129  170 / 171  247 / 234*       135 / 145  200 / 196  300 / 274*
+//   200 x 400        103 / 109  147 / 138  214 / 191*        130 / 145  189 / 236  276 / 298        150 / 162  224 / 274  337 / 347
+//   256 x 512        122 / 137  179 / 186  264 / 294         156 / 187  233 / 266  342 / 439        192 / 213  295 / 322  438 / 515
+//   2 heads, 250     77 / 87    107 / 112  149 / 161          97 / 115  136 / 153  193 / 237        113 / 125  162 / 178  232 / 279
+//   and with a partial last Q block
+//   250 x 500        263 / 174* 263 / 230* 260 / 289         334 / 249* 334 / 345  335 / 442        418 / 282* 425 / 404* 431 / 516
+//   H4 N17776        238 / 189* 266 / 251* 279 / 286         299 / 257* 328 / 347  346 / 427        357 / 298* 386 / 415  410 / 514
+// Of 1800 calls, up to 1200 rows and 1000 K blocks, the rule is 0.3 % on average behind the better side; the worst that it cuts loses 2.2 %.
+// The share of a head's blocks that the chunks' time goes by.  A causal row keeps the smaller of `share` and what lies in front of the diagonal; an
+// XCD works on an eighth of all rows, one behind the other, so with few heads the one with the last, longest rows of a head ends last.
+inline float blocks_that_count(long long heads, float share, bool causal) {
+  if (!causal) return share;
+  const float mean = share - 0.5f * share * share, part = heads < 8 ? heads / 8.f : 1.f, from = 1.f - part;      // rows from .. 1 of a head
+  const float last = share <= from ? share : (0.5f * (share * share - from * from) + share * (1.f - share)) / part;
+  return 0.3f * mean + 0.7f * last;
+}
 inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, int selection, float share, float simthreshd1, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
-  if (selection == SPG_SELECT_MASK || nk <= SPG_SELECT_IN_ATTN_NK || chunk_plan(B, H, N, N_kv, D).chunks == 1) return false;
+  if (selection == SPG_SELECT_MASK || nk <= SPG_SELECT_IN_ATTN_NK) return false;
+  const ChunkPlan plan = chunk_plan(B, H, N, N_kv, D);
+  if (plan.chunks == 1) return false;
   const bool many = B * H * nq > 256, partial = N % 128 != 0;
   const bool known = selection == SPG_SELECT_TOPK && share >= 0.f && simthreshd1 < 0.f;
   if (partial && !known && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
   share = share < 0.f ? (many ? (D == 64 ? 0.75f : 0.65f) : 0.5f) : share < 1.f ? share : 1.f;
   const float kept = share * nk;
   const float longest = partial ? (float)nk : kept;
-  const float all = (float)(B * H) * (nq * kept * (causal ? 1.f - 0.5f * share : 1.f) + (partial ? nk - kept : 0.f));
-  if (many) return longest - all / (D == 64 ? 350.f : 220.f) > 45.f;
-  return longest - all / 180.f > 36.f;
+  if (longest <= plan.per) return false;                            // no row has two chunks
+  const float all = (float)(B * H) * (nq * nk * blocks_that_count((long long)B * H, share, causal) + (partial ? nk - kept : 0.f));
+  if (many) return longest - all / (D == 64 ? 380.f : 250.f) > (D == 64 ? 56.f : 34.f);
+  return longest - all / (D == 64 ? 190.f : partial && !pv_f16 ? 145.f : 170.f) > (D == 64 ? 34.f : 30.f);
 }
 inline bool rows_in_chunks(const spg_attn_args *a, float share, float simthreshd1) {
   return rows_in_chunks(a->B, a->H, a->N, a->N_kv, a->D, a->pv_f16 != 0, a->selection, share, simthreshd1, a->is_causal != 0);

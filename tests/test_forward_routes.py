@@ -94,6 +94,20 @@ def test_few_long_rows_go_over_several_workgroups(routes, kw, chunks):
     assert routes(**kw)[7] == chunks
 
 
+# A causal selection: the XCD with the last rows of a head has more than its share of the blocks, so chunks pay less than the number of blocks says.
+@pytest.mark.parametrize("kw,chunks", [
+    (dict(N=16000, level=0.6), 1), (dict(N=22400, level=1.0), 1), (dict(N=25600, level=0.6), 0), (dict(N=25600, level=1.0), 0), (dict(N=25600, D=64, level=1.0), 1),
+    (dict(N=32768, level=1.0), 0), (dict(N=32768, D=64, level=1.0), 0), (dict(H=2, N=12800, D=64, level=1.0), 1), (dict(H=2, N=16000, D=64, level=1.0), 0),
+    (dict(H=2, N=16000, level=1.0), 0), (dict(N=31950, level=0.35), 1), (dict(N=31950, level=1.0), 0), (dict(N=31950, D=64, level=0.6), 1), (dict(N=31950, D=64, level=1.0), 0),
+    (dict(H=4, N=17776, D=64, level=0.6), 1), (dict(H=4, N=17776, D=64, level=1.0), 0), (dict(N=60001, D=64, level=1.0), 0)])
+def test_causal_chunks_end_with_the_longest_rows(routes, kw, chunks):
+    assert routes(causal=1, **kw)[7] == chunks == routes(causal=1, pv_f16=1, **kw)[7]
+
+
+def test_rows_of_one_chunk_are_not_cut(routes):
+    assert [routes(N=12800, Nk=64 * 1000, level=level)[7] for level in (0.097, 0.1)] == [0, 1]         # 98 blocks to a chunk
+
+
 # Top-k with a similarity threshold of 0 or more may keep every block: in chunks only where that pays with all of them, too.
 @pytest.mark.parametrize("kw,chunks", [
     (dict(H=8, N=17776, D=64, level=0.15), 0), (dict(H=4, N=17776, D=64, level=0.3), 0), (dict(H=6, N=8300, D=64, level=0.15), 0), (dict(H=2, N=17776, D=64, level=0.15), 1),
