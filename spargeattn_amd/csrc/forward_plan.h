@@ -193,10 +193,21 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 // What a row keeps:
 // * top-k without similar blocks to look for: what top-k names (share), and all of it in a partial last Q block, which is never similar.
 //   simthreshd1: blocks of Q and K whose similarity is below it keep everything.  A similarity is not negative, so below 0 it changes nothing.
-// * a similarity threshold of 0 or more, a CDF threshold or a level per head (share below 0): nothing on the host says, and it is often
-//   everything.  Half of it is taken, beyond 256 rows 0.65 to 0.75, and with a partial last Q block it has to pay with everything kept, too.
-//   us per call, workgroup per row / chunks: H8 N17776 top-k 0.15 with simthreshd1 0.6, no block similar, D64 578 / 661, D128 831 / 1041; CDF 0.93
-//   at 0.3, causal, one head N31595 D128 342 / 438; 0.82 at 0.6 N31887 with FP16 PV 457 / 531.
+// * a similarity threshold of 0 or more, a CDF threshold or a level per head (share below 0): nothing on the host says.
+//   With a partial last Q block the longest row keeps everything, and the chunks have the less to do the less the others keep: they have to pay with
+//   everything kept.  us per call, workgroup per row / chunks, where they do not: H8 N17776 top-k 0.15 with simthreshd1 0.6, no block similar, D64 578 /
+//   661, D128 831 / 1041; CDF 0.93 at 0.3, causal, one head N31595 D128 342 / 438; 0.82 at 0.6 N31887 with FP16 PV 457 / 531.
+//   Whole rows with a top-k level keep that or more, and the more they keep the better for chunks, so it has to pay at the level (causal: without
+//   the diagonal).
+//   Whole rows without one keep anything, and a few of their blocks are one or two chunks: up to 64 rows of 288 K blocks or more, where what
+//   is lost at low CDF thresholds is a tenth, and from 0.13 to 0.2 on there is a gain up to threefold.  One head, CDF threshold (no similarity test):
+//                          0.02       0.06       0.09       0.13       0.2        0.35                   0.02       0.06       0.09       0.13       0.2        0.35
+//     D64  8 x 288         31 / 33    36 / 41    41 / 44    46 / 44    55 / 48    76 / 49   D128         38 / 40    45 / 51    51 / 55    58 / 55    71 / 58    98 / 60
+//          64 x 288        36 / 38    42 / 47    47 / 51    52 / 52    61 / 55    81 / 62                43 / 46    52 / 58    59 / 63    65 / 69    78 / 66   103 / 78
+//          8 x 1000        59 / 63    77 / 69    91 / 69   110 / 71   142 / 73   211 / 80                69 / 74    94 / 80   113 / 81   138 / 84   180 / 86   267 / 89
+//          64 x 200        32 / 33    36 / 40    40 / 44    44 / 48    50 / 49    64 / 56                37 / 39    44 / 47    48 / 53    54 / 58    62 / 60    81 / 68
+//          100 x 256       34 / 36    40 / 44    43 / 48    48 / 52    57 / 59    74 / 65                40 / 42    48 / 54    54 / 61    60 / 64    71 / 74    94 / 83
+//     one head causal at 0.13 and 0.2, N9088 D128 42 / 52, 48 / 53; N16000 D64 46 / 53, N24064 D128 78 / 86, 94 / 116
 // * a mask: never in chunks.  Its density is known on the device only, and the rows of a sparse one are one or two chunks each, for which the
 //   launches more cost up to a fifth of the call.  rows x nk, density:
 //                  0.03          0.06          0.1           0.2                        0.03          0.06          0.1           0.2
@@ -251,8 +262,12 @@ inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, in
   if (plan.chunks == 1) return false;
   const bool many = B * H * nq > 256, partial = N % 128 != 0;
   const bool known = selection == SPG_SELECT_TOPK && share >= 0.f && simthreshd1 < 0.f;
-  if (partial && !known && !chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal)) return false;
-  share = share < 0.f ? (many ? (D == 64 ? 0.75f : 0.65f) : 0.5f) : share < 1.f ? share : 1.f;
+  if (!known) {
+    if (partial) return chunks_pay_with_all_kept(B * H * nq, nk, D, pv_f16, causal);
+    if (share < 0.f) return B * H * nq <= 64 && nk >= 288;
+    causal = false;
+  }
+  if (share > 1.f) share = 1.f;
   const float kept = share * nk;
   const float longest = partial ? (float)nk : kept;
   if (longest <= plan.per) return false;                            // no row has two chunks

@@ -113,7 +113,8 @@ def test_rows_of_one_chunk_are_not_cut(routes):
     (dict(H=8, N=17776, D=64, level=0.15), 0), (dict(H=4, N=17776, D=64, level=0.3), 0), (dict(H=6, N=8300, D=64, level=0.15), 0), (dict(H=2, N=17776, D=64, level=0.15), 1),
     (dict(H=8, N=17776, level=0.15), 0), (dict(H=2, N=17776, level=0.15), 1), (dict(N=17776, level=0.15), 1), (dict(N=30000, level=0.15), 0), (dict(N=30000, D=64, level=0.15), 0),
     (dict(N=24001, D=64, level=0.5), 1), (dict(N=24001, D=64, level=0.5, pv_f16=1), 0), (dict(N=24001, level=0.5), 0), (dict(N=28001, D=64, level=0.5, causal=1), 1),
-    (dict(H=2, N=17776, level=0.15, pv_f16=1), 0), (dict(H=8, N=1024, Nk=64 * 288, level=0.5), 1)])
+    (dict(H=2, N=17776, level=0.15, pv_f16=1), 0), (dict(H=8, N=1024, Nk=64 * 288, level=0.5), 1), (dict(N=16000, level=0.6, causal=1), 1),
+    (dict(N=22400, level=1.0, causal=1), 0)])
 def test_a_similarity_threshold_may_keep_everything(routes, kw, chunks):
     assert routes(sim=0.0, **kw)[7] == chunks == routes(sim=0.6, **kw)[7] == routes(sim="nan", **kw)[7]
     assert routes(sim=-0.1, **kw)[7] == 1
@@ -127,7 +128,10 @@ def test_a_similarity_threshold_may_keep_everything(routes, kw, chunks):
 # So may a CDF threshold.  (A level per head is a negative share to the rule, as a CDF threshold is.)
 @pytest.mark.parametrize("kw,chunks", [
     (dict(N=31595, causal=1), 0), (dict(N=31887, causal=1, pv_f16=1), 0), (dict(N=30000, D=64), 0), (dict(N=24001, D=64), 1), (dict(N=17776), 1), (dict(N=24001), 0),
-    (dict(H=2, N=40573, D=64, causal=1), 0), (dict(H=2, N=24001, D=64), 1), (dict(H=2, N=17776, pv_f16=1), 0), (dict(N=24064), 0), (dict(N=12800), 1), (dict(H=8, N=1024, Nk=64 * 288), 1)])
+    (dict(H=2, N=40573, D=64, causal=1), 0), (dict(H=2, N=24001, D=64), 1), (dict(H=2, N=17776, pv_f16=1), 0), (dict(N=24064), 0),
+    # whole rows may keep next to nothing
+    (dict(N=12800), 0), (dict(N=12800, D=64), 0), (dict(N=9088, causal=1), 0), (dict(N=16000, D=64, causal=1), 0), (dict(H=8, N=1024, Nk=64 * 288), 1),
+    (dict(H=8, N=1024, Nk=64 * 287), 0), (dict(H=65, N=128, Nk=64 * 400, D=64), 0), (dict(H=64, N=128, Nk=64 * 400, D=64), 1), (dict(H=2, N=128, Nk=64 * 140, D=64), 0)])
 def test_a_cdf_threshold_may_keep_everything(routes, kw, chunks):
     for sim in (-0.1, 0.6):
         assert routes(selection=CDF, sim=sim, **kw)[7] == chunks
