@@ -170,10 +170,21 @@ inline RowSplit row_split(const ChunkPlan &c, void *scratch) {
   return {c.chunks, c.per, 0, (int *)(at + c.first), (float *)(at + c.maxima), (float *)(at + c.md), (float *)(at + c.o)};
 }
 
+// The share of a head's blocks that the chunks' time goes by.  A causal row keeps the smaller of `share` and what lies in front of the diagonal; an
+// XCD works on an eighth of all rows, one behind the other, so with few heads the one with the last, longest rows of a head ends
+// last: everything kept, a causal call takes 0.95, 0.83, 0.76 and 0.59 of the time that it takes without the diagonal with 1, 2, 4 and 8 heads (D64, 31950 and
+// 17776 queries).
+inline float blocks_that_count(long long heads, float share, bool causal) {
+  if (!causal) return share;
+  const float mean = share - 0.5f * share * share, part = heads < 8 ? heads / 8.f : 1.f, from = 1.f - part;      // rows from .. 1 of a head
+  const float last = share <= from ? share : (0.5f * (share * share - from * from) + share * (1.f - share)) / part;
+  return 0.3f * mean + 0.7f * last;
+}
+
 // Everything kept, with a partial last Q block: the longest row is as long as ever and the chunks have the most to do, so they pay nowhere
 // less.  A workgroup per row takes 0.48 (D = 64), 0.62 (D = 128) and 0.74 us (FP16 PV) per block of a row in groups, and 0.9 and 1.1 us in one
-// group beyond 256 rows; causal rows, half as many blocks, save a tenth of the chunks' time only, since a chunk is as long as in a full
-// row.  us per call, workgroup per row / chunks, on both sides of the line, rows x nk:
+// group beyond 256 rows; causal rows, half as many blocks, save a tenth of the chunks' time only (blocks_that_count).  us per call, workgroup per
+// row / chunks, on both sides of the line, rows x nk:
 //            up to 256 rows                                              beyond
 // D64        188 x 376 215 / 192, 204 x 407 231 / 222, 252 x 251 156 / 185   376 x 376 375 / 339, 417 x 278 291 / 297, 390 x 130 157 / 166
 // causal     219 x 438 241 / 231, 235 x 469 257 / 260, 252 x 251 154 / 160   417 x 278 256 / 236, 556 x 278 283 / 283, 469 x 938 819 / 830
@@ -207,7 +218,7 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 //          8 x 1000        59 / 63    77 / 69    91 / 69   110 / 71   142 / 73   211 / 80                69 / 74    94 / 80   113 / 81   138 / 84   180 / 86   267 / 89
 //          64 x 200        32 / 33    36 / 40    40 / 44    44 / 48    50 / 49    64 / 56                37 / 39    44 / 47    48 / 53    54 / 58    62 / 60    81 / 68
 //          100 x 256       34 / 36    40 / 44    43 / 48    48 / 52    57 / 59    74 / 65                40 / 42    48 / 54    54 / 61    60 / 64    71 / 74    94 / 83
-//     one head causal at 0.13 and 0.2, N9088 D128 42 / 52, 48 / 53; N16000 D64 46 / 53, N24064 D128 78 / 86, 94 / 116
+//     one head, causal: N9088 D128 0.13 40 / 52, 0.2 46 / 53; N24064 D128 0.13 72 / 86, 0.2 88 / 116; not causal: N16000 D64 0.09 41 / 53
 // * a mask: never in chunks.  Its density is known on the device only, and the rows of a sparse one are one or two chunks each, for which the
 //   launches more cost up to a fifth of the call.  rows x nk, density:
 //                  0.03          0.06          0.1           0.2                        0.03          0.06          0.1           0.2
@@ -247,14 +258,6 @@ inline bool chunks_pay_with_all_kept(int rows, int nk, int D, bool pv_f16, bool 
 //   250 x 500        263 / 174* 263 / 230* 260 / 289         334 / 249* 334 / 345  335 / 442        418 / 282* 425 / 404* 431 / 516
 //   H4 N17776        238 / 189* 266 / 251* 279 / 286         299 / 257* 328 / 347  346 / 427        357 / 298* 386 / 415  410 / 514
 // Of 1800 calls, up to 1200 rows and 1000 K blocks, the rule is 0.3 % on average behind the better side; the worst that it cuts loses 2.2 %.
-// The share of a head's blocks that the chunks' time goes by.  A causal row keeps the smaller of `share` and what lies in front of the diagonal; an
-// XCD works on an eighth of all rows, one behind the other, so with few heads the one with the last, longest rows of a head ends last.
-inline float blocks_that_count(long long heads, float share, bool causal) {
-  if (!causal) return share;
-  const float mean = share - 0.5f * share * share, part = heads < 8 ? heads / 8.f : 1.f, from = 1.f - part;      // rows from .. 1 of a head
-  const float last = share <= from ? share : (0.5f * (share * share - from * from) + share * (1.f - share)) / part;
-  return 0.3f * mean + 0.7f * last;
-}
 inline bool rows_in_chunks(int B, int H, int N, int N_kv, int D, bool pv_f16, int selection, float share, float simthreshd1, bool causal) {
   const int nk = (N_kv + 63) / 64, nq = (N + 127) / 128;
   if (selection == SPG_SELECT_MASK || nk <= SPG_SELECT_IN_ATTN_NK) return false;
@@ -280,7 +283,7 @@ inline bool rows_in_chunks(const spg_attn_args *a, float share, float simthreshd
 }
 // Whether some call of this shape with these options is cut.  The workspace has the scratch then, whatever hyper-parameters the call brings, and not
 // otherwise: up to 275 MB beside some 50 (H8 N17776 D128).  For top-k the difference at the rule is linear in the share, or convex where it is
-// causal, so it is largest at an end; a similarity threshold only takes calls out.
+// causal, so it is largest at an end; a similarity threshold or a level per head only takes calls out.
 inline bool may_have_rows_in_chunks(const spg_attn_args *a) {
   return a->selection == SPG_SELECT_TOPK ? rows_in_chunks(a, 0.f, -1.f) || rows_in_chunks(a, 1.f, -1.f) : rows_in_chunks(a, -1.f, 0.f);
 }
