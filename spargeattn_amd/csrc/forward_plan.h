@@ -172,7 +172,7 @@ inline RowSplit row_split(const ChunkPlan &c, void *scratch) {
 
 // The share of a head's blocks that the chunks' time goes by.  A causal row keeps the smaller of `share` and what lies in front of the diagonal; an
 // XCD works on an eighth of all rows, one behind the other, so with few heads the one with the last, longest rows of a head ends
-// last: everything kept, a causal call takes 0.95, 0.83, 0.76 and 0.59 of the time that it takes without the diagonal with 1, 2, 4 and 8 heads (D64, 31950 and
+// last: everything kept, a causal call takes 0.93, 0.83, 0.76 and 0.59 of the time that it takes without the diagonal with 1, 2, 4 and 8 heads (D64, 31950 and
 // 17776 queries).
 inline float blocks_that_count(long long heads, float share, bool causal) {
   if (!causal) return share;
